@@ -3,7 +3,9 @@
 // `linear_tiled` is the plain path: float32 multiply-add on 64x64 output tiles staged through LDS, for any
 // mix of float32 / bfloat16 operands and any sizes.  Every output element is one sum over k in ascending order
 // inside fixed k-tiles, so a row's result does not depend on how many other rows the call carries.  It is the
-// whole of the float32 path and the fallback for operand mixes the MFMA kernels do not take.
+// fallback for operand mixes and widths that no matrix-core kernel takes.
+//
+// `linear_f32_few` and `linear_f32_wide` are the float32 path on the matrix cores (see below).
 
 #include "common.h"
 #include "api.h"
@@ -67,6 +69,243 @@ int launch_tiled(const void* x, const void* w, void* y, int rows, int outs, int 
   return AKV_LAUNCH_STATUS();
 }
 
+// ---- float32 on the matrix cores -----------------------------------------------------------------------------------------
+// v_mfma_f32_16x16x4_f32 multiplies and adds in float32 at twice the vector units' rate (157 TFLOP/s), with no rounding
+// of an operand.  A lane's operands of four such instructions are 16 consecutive bytes of a matrix row: lane (r, g) holds
+// elements 16 b + 4 g .. + 3 of row r, and instruction j takes element j of every group g.  Both kernels sum every output
+// the same way, so that a row's result depends neither on how many rows a call carries nor on which kernel takes it:
+// k is cut into segments of 128, a segment is one chain of instructions in the order (b, j), and the segments' sums are
+// added in their order.  (Rows and outputs beyond the matrices repeat the last one and are not stored; elements beyond k are
+// zeros and change no sum.)
+typedef float floats4 __attribute__((ext_vector_type(4)));
+constexpr int kSegment = 128;        // k of one chain
+constexpr int kSegmentBlocks = kSegment / 16;
+
+__device__ __forceinline__ floats4 mfma4(const floats4 a, const floats4 b, floats4 sums) {
+#pragma unroll
+  for (int j = 0; j < 4; ++j) sums = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], b[j], sums, 0, 0, 0);
+  return sums;
+}
+
+// The sums of 16 outputs (4 g .. 4 g + 3 of them in this lane) for row `row`, with their bias, to y.
+__device__ __forceinline__ void store_f32(float* __restrict__ y, long row, int out, int outs, floats4 sums,
+                                          const float* __restrict__ bias, bool wide_stores) {
+  if (bias != nullptr) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) sums[j] += bias[min(out + j, outs - 1)];
+  }
+  float* at = y + row * outs + out;
+  if (wide_stores && out + 4 <= outs) {
+    *reinterpret_cast<floats4*>(at) = sums;
+    return;
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    if (out + j < outs) at[j] = sums[j];
+}
+
+// Up to 64 rows: the matrix is read once and its reads are what the product waits for.  A block owns 16 outputs and all of
+// k; its waves take a segment each (a second round where k has more than 16), with the whole segment's loads in flight - 8 KB
+// a wave, 128 KB a block -, and leave their sums in LDS, where the first waves add them in order.  Rows lie in cache and
+// are read by every wave in operand order, without LDS: NT tiles of 16 rows.
+template <int NT>
+__global__ __launch_bounds__(1024) void linear_f32_few_kernel(const float* __restrict__ x, const float* __restrict__ w,
+                                                             float* __restrict__ y, int rows, int outs, int k, int segments,
+                                                             const float* __restrict__ bias, bool wide_stores) {
+  extern __shared__ floats4 pieces[];                      // [waves][NT][64]
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
+  const int r = lane & 15, g = lane >> 4;
+  const int out0 = blockIdx.x * 16;
+  const float* wp = w + static_cast<long>(min(out0 + r, outs - 1)) * k + 4 * g;
+  const float* xp[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) xp[t] = x + static_cast<long>(min(16 * t + r, rows - 1)) * k + 4 * g;
+  constexpr int kGroup = NT <= 2 ? 8 : 4;    // blocks of 16 k whose rows are asked for together (registers)
+  const floats4 zero = {0.f, 0.f, 0.f, 0.f};
+  floats4 total = zero;
+  for (int first = 0; first < segments; first += waves) {
+    const int segment = first + wave;
+    if (segment < segments) {
+      const int k0 = segment * kSegment;
+      floats4 sums[NT];
+#pragma unroll
+      for (int t = 0; t < NT; ++t) sums[t] = zero;
+      if (k0 + kSegment <= k) {
+        floats4 a[kSegmentBlocks];
+#pragma unroll
+        for (int b = 0; b < kSegmentBlocks; ++b) a[b] = *reinterpret_cast<const floats4*>(wp + k0 + 16 * b);
+        __builtin_amdgcn_sched_barrier(0);                 // (else the loads are moved down to where they are used)
+#pragma unroll
+        for (int b0 = 0; b0 < kSegmentBlocks; b0 += kGroup) {
+          floats4 v[kGroup][NT];
+#pragma unroll
+          for (int b = 0; b < kGroup; ++b)
+#pragma unroll
+            for (int t = 0; t < NT; ++t) v[b][t] = *reinterpret_cast<const floats4*>(xp[t] + k0 + 16 * (b0 + b));
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int b = 0; b < kGroup; ++b)
+#pragma unroll
+            for (int t = 0; t < NT; ++t) sums[t] = mfma4(a[b0 + b], v[b][t], sums[t]);
+        }
+      } else {
+        for (int b = 0; k0 + 16 * b < k; ++b) {
+          const int at = k0 + 16 * b;
+          const bool inside = at + 4 * g < k;              // (k is a multiple of 4: a group of four is whole or absent)
+          const floats4 a = inside ? *reinterpret_cast<const floats4*>(wp + at) : zero;
+#pragma unroll
+          for (int t = 0; t < NT; ++t) {
+            const floats4 v = inside ? *reinterpret_cast<const floats4*>(xp[t] + at) : zero;
+            sums[t] = mfma4(a, v, sums[t]);
+          }
+        }
+      }
+#pragma unroll
+      for (int t = 0; t < NT; ++t) pieces[(wave * NT + t) * 64 + lane] = sums[t];
+    }
+    __syncthreads();
+    if (wave < NT) {
+      const int there = min(waves, segments - first);
+      for (int s = 0; s < there; ++s) total += pieces[(s * NT + wave) * 64 + lane];
+    }
+    __syncthreads();
+  }
+  // (a block has at least NT waves: the launch sees to it)
+  if (wave < NT && 16 * wave + r < rows) store_f32(y, 16 * wave + r, out0 + 4 * g, outs, total, bias, wide_stores);
+}
+
+// More rows: tiles of 32 TM outputs by 32 TN rows, four waves of TM x TN tiles of 16 each, operands through two LDS buffers
+// of 32 k (row stride 36 floats: 16-byte reads of eight rows meet no bank twice), the next 32 k on their way in registers.
+// Bound by the matrix cores: 8 TM TN instructions of 32 cycles a step and wave for 2 (TM + TN) reads of 1 KB.
+template <int TM, int TN>
+__global__ __launch_bounds__(256) void linear_f32_wide_kernel(const float* __restrict__ x, const float* __restrict__ w,
+                                                              float* __restrict__ y, int rows, int outs, int k,
+                                                              const float* __restrict__ bias, bool wide_stores) {
+  constexpr int kStride = 36, kDeep = 32, kOuts = 32 * TM, kRows = 32 * TN;
+  __shared__ float ws[2][kOuts * kStride];
+  __shared__ float xs[2][kRows * kStride];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int r = lane & 15, g = lane >> 4;
+  const int out0 = blockIdx.x * kOuts, row0 = blockIdx.y * kRows;
+  const int file_row = threadIdx.x >> 3, file_k = (threadIdx.x & 7) * 4;   // thread t fetches 16 bytes of rows t / 8 + 32 i
+  const float* wp[TM];
+  const float* xp[TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i) wp[i] = w + static_cast<long>(min(out0 + file_row + 32 * i, outs - 1)) * k;
+#pragma unroll
+  for (int i = 0; i < TN; ++i) xp[i] = x + static_cast<long>(min(row0 + file_row + 32 * i, rows - 1)) * k;
+  const floats4 zero = {0.f, 0.f, 0.f, 0.f};
+  floats4 sums[TM][TN], total[TM][TN], next_w[TM], next_x[TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) sums[i][j] = total[i][j] = zero;
+  auto fetch = [&](int k0) {
+    const int at = min(k0 + file_k, k - 4);
+#pragma unroll
+    for (int i = 0; i < TM; ++i) next_w[i] = *reinterpret_cast<const floats4*>(wp[i] + at);
+#pragma unroll
+    for (int i = 0; i < TN; ++i) next_x[i] = *reinterpret_cast<const floats4*>(xp[i] + at);
+  };
+  auto file = [&](int buffer, int k0) {
+    const bool inside = k0 + file_k < k;
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+      *reinterpret_cast<floats4*>(&ws[buffer][(file_row + 32 * i) * kStride + file_k]) = inside ? next_w[i] : zero;
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+      *reinterpret_cast<floats4*>(&xs[buffer][(file_row + 32 * i) * kStride + file_k]) = inside ? next_x[i] : zero;
+  };
+  const int w_at = ((wave >> 1) * 16 * TM + r) * kStride + 4 * g, x_at = ((wave & 1) * 16 * TN + r) * kStride + 4 * g;
+  const int steps = (k + kDeep - 1) / kDeep;
+  fetch(0);
+  file(0, 0);
+  __syncthreads();
+  for (int step = 0; step < steps; ++step) {
+    const int buffer = step & 1;
+    if (step + 1 < steps) fetch((step + 1) * kDeep);
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      floats4 a[TM], v[TN];
+#pragma unroll
+      for (int i = 0; i < TM; ++i) a[i] = *reinterpret_cast<const floats4*>(&ws[buffer][w_at + 16 * i * kStride + 16 * b]);
+#pragma unroll
+      for (int j = 0; j < TN; ++j) v[j] = *reinterpret_cast<const floats4*>(&xs[buffer][x_at + 16 * j * kStride + 16 * b]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int j = 0; j < TN; ++j)
+            sums[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i][e], v[j][e], sums[i][j], 0, 0, 0);
+    }
+    if ((step & 3) == 3 || step + 1 == steps) {            // the end of a segment of 128
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          total[i][j] += sums[i][j];
+          sums[i][j] = zero;
+        }
+    }
+    if (step + 1 < steps) file(buffer ^ 1, (step + 1) * kDeep);   // (read last before the barrier of the step before)
+    __syncthreads();
+  }
+#pragma unroll
+  for (int j = 0; j < TN; ++j) {
+    const int row = row0 + (wave & 1) * 16 * TN + 16 * j + r;
+    if (row >= rows) continue;
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+      store_f32(y, row, out0 + (wave >> 1) * 16 * TM + 16 * i + 4 * g, outs, total[i][j], bias, wide_stores);
+  }
+}
+
+template <int NT>
+int launch_f32_few(const float* x, const float* w, float* y, int rows, int outs, int k, const float* bias, bool wide_stores,
+                   hipStream_t stream) {
+  const int segments = (k + kSegment - 1) / kSegment, rounds = (segments + 15) / 16;
+  const int waves = max((segments + rounds - 1) / rounds, NT);
+  const size_t lds = static_cast<size_t>(waves) * NT * 64 * sizeof(floats4);     // 64 KB at most
+  linear_f32_few_kernel<NT><<<(outs + 15) / 16, waves * 64, lds, stream>>>(x, w, y, rows, outs, k, segments, bias, wide_stores);
+  return AKV_LAUNCH_STATUS();
+}
+
+template <int TM, int TN>
+int launch_f32_wide(const float* x, const float* w, float* y, int rows, int outs, int k, const float* bias, bool wide_stores,
+                    hipStream_t stream) {
+  dim3 grid((outs + 32 * TM - 1) / (32 * TM), (rows + 32 * TN - 1) / (32 * TN));
+  linear_f32_wide_kernel<TM, TN><<<grid, 256, 0, stream>>>(x, w, y, rows, outs, k, bias, wide_stores);
+  return AKV_LAUNCH_STATUS();
+}
+
+// float32 operands whose rows are 16-byte aligned.  Which kernel takes a product is a matter of time alone (the bits are the
+// same).  Measured, us, on weights that no cache holds (outs x k = 2048 x 2048 / 6144 x 2048 / 4096 x 12288 / 32768 x 2048;
+// tiles of 64 x 64, 32 x 64 and 32 x 32 outputs x rows):
+//     17 rows: few 12.5 / 25 / 74 / 97    64 x 64 58 / 59 / 340 / 99    32 x 32 36 / 46 / 273 / 71
+//     64 rows: few 23 / 46 / 137 / 174    64 x 64 58 / 59 / 340 / 103   32 x 32 37 / 50 / 271 / 112
+//    200 rows:                            64 x 64 59 / 97 / 339 / 321   32 x 64 40 / 81 / 320 / 360   32 x 32 38 / 88 / 370 / 379
+//    300 rows:                            64 x 64 60 / 97 / 519 / 402   32 x 64 56 / 102 / 418 / 446  32 x 32 49 / 113 / 458 / 542
+//    999 rows:                            64 x 64 99 / 253 / 948 / 1244 32 x 64 103 / 280 / 1027 / 1381  (111 TFLOP/s at best;
+// the vector kernel above: 511 us on average over 2048 x 2048 and 2048 x 3072).  So: few rows stay with the kernel that reads
+// the matrix once unless tiles alone give every unit two blocks; otherwise the largest tile that still gives the units about
+// two blocks each (tiles of 128 are slower everywhere: the matrix cores wait for nothing that larger tiles would spare).
+int launch_f32(const float* x, const float* w, float* y, int rows, int outs, int k, const float* bias, hipStream_t stream) {
+  const bool wide_stores = outs % 4 == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0;
+  const long units = device_facts().compute_units;
+  const auto blocks = [&](int out_tile, int row_tile) {
+    return static_cast<long>((outs + out_tile - 1) / out_tile) * ((rows + row_tile - 1) / row_tile);
+  };
+  if (rows <= 16) return launch_f32_few<1>(x, w, y, rows, outs, k, bias, wide_stores, stream);
+  if (blocks(64, 64) < 2 * units) {
+    if (rows <= 32) return launch_f32_few<2>(x, w, y, rows, outs, k, bias, wide_stores, stream);
+    if (rows <= 64) return launch_f32_few<4>(x, w, y, rows, outs, k, bias, wide_stores, stream);
+  }
+  if (4 * blocks(64, 64) >= 7 * units) return launch_f32_wide<2, 2>(x, w, y, rows, outs, k, bias, wide_stores, stream);
+  if (blocks(32, 64) >= 2 * units) return launch_f32_wide<1, 2>(x, w, y, rows, outs, k, bias, wide_stores, stream);
+  return launch_f32_wide<1, 1>(x, w, y, rows, outs, k, bias, wide_stores, stream);
+}
+
 }  // namespace
 
 // `bias` [outs] float32 or null: added to a sum after its last product, before it is rounded to y's type.
@@ -76,7 +315,11 @@ extern "C" int akv_linear_tiled(const void* x, int x_dtype, const void* w, int w
   if (((rows + kTile - 1) / kTile) > 65535) return -2;
   const int code = x_dtype * 4 + w_dtype * 2 + y_dtype;
   switch (code) {
-    case 0: return launch_tiled<float, float, float>(x, w, y, rows, outs, k, bias, stream);
+    case 0:
+      if (k > 0 && k % 4 == 0 && (reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w)) % 16 == 0)
+        return launch_f32(static_cast<const float*>(x), static_cast<const float*>(w), static_cast<float*>(y), rows, outs, k,
+                          bias, stream);
+      return launch_tiled<float, float, float>(x, w, y, rows, outs, k, bias, stream);
     case 2: return launch_tiled<float, bf16_t, float>(x, w, y, rows, outs, k, bias, stream);
     case 4: return launch_tiled<bf16_t, float, float>(x, w, y, rows, outs, k, bias, stream);
     case 5: return launch_tiled<bf16_t, float, bf16_t>(x, w, y, rows, outs, k, bias, stream);

@@ -1025,6 +1025,36 @@ def test_linear_rows_do_not_depend_on_the_batch(hip):
         assert torch.equal(alone[0], whole[row])
 
 
+@pytest.mark.parametrize("outs,k", [(16, 4), (150, 300), (100, 128), (2051, 260), (64, 2052), (3072, 2048)])
+def test_float32_products_on_the_matrix_cores(hip, outs, k):
+    """Rows on both sides of every kernel's range (16 / 32 / 64 rows a launch, then tiles), widths that end inside a chain
+    of 128 and inside a group of 16, outputs that end inside a tile; with and without a bias.  Against float64: a
+    term passes at most min(k, 128) additions of its chain and one per chain, and its own product; every rounding is at most
+    2^-24 of a partial sum, which is at most the sum of the terms' magnitudes: |error| <= (min(k, 128) + chains + 1) 2^-24
+    sum |x w|.  A row's bits do not depend on the rows beside it."""
+    w, bias = rand(outs, k, seed=31).cuda(), rand(outs, seed=32).cuda()
+    x = rand(1000, k, seed=33).cuda()
+    alone = torch.empty(1, outs, device="cuda")
+    hip.linear(x[:1].contiguous(), w, alone)
+    for rows in (1, 15, 16, 17, 32, 33, 64, 65, 130, 257, 1000):
+        y, biased = torch.full((rows, outs), float("nan"), device="cuda"), torch.empty(rows, outs, device="cuda")
+        hip.linear(x[:rows].contiguous(), w, y)
+        hip.linear(x[:rows].contiguous(), w, biased, bias=bias)
+        want = x[:rows].double() @ w.double().T
+        reach = (min(k, 128) + (k + 127) // 128 + 1) * 2.0 ** -24 * (x[:rows].double().abs() @ w.double().abs().T)
+        assert ((y - want).abs() <= reach).all(), rows
+        assert torch.equal(biased, y + bias), rows
+        assert torch.equal(y[0], alone[0]), rows
+
+
+def test_float32_product_of_rows_that_are_not_aligned(hip, ref):
+    """A matrix that begins between 16-byte boundaries goes to the plain kernel."""
+    x, w = rand(20, 64, seed=34).cuda(), rand(40 * 64 + 1, seed=35).cuda()[1:].view(40, 64)
+    y = torch.empty(20, 40, device="cuda")
+    hip.linear(x, w, y)
+    torch.testing.assert_close(y.cpu(), x.cpu() @ w.cpu().T, rtol=2e-5, atol=2e-5)
+
+
 @pytest.mark.parametrize("inter", [200, 204, 203, 4096])     # widths in steps of 8, of 4 and of 1
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_swiglu(hip, ref, dtype, inter):
