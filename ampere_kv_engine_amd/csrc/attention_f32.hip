@@ -1,0 +1,369 @@
+// Attention over the paged cache in float32, on the matrix cores.
+//
+// v_mfma_f32_16x16x4_f32 takes float32 operands as they are and adds in float32.  A wave works on a tile of 16 query rows -
+// consecutive (token, head) pairs of one request whose heads read the same kv head - and 16 keys at a time:
+//   scores  S^T [keys x rows]  = K [keys x dim] Q^T:   a lane's operand of four instructions is 16 bytes of a key's record;
+//   sums    O^T [dim x rows]   = V^T [dim x keys] P^T: 16 bytes of a value row (pages hold values [dim, page]); what a lane
+//           has of S^T - keys 4 g .. 4 g + 3 of row lane & 15 - is its operand P^T as it stands, no exchange between lanes.
+// The order of every sum depends on the token's own position only - not on how a request was cut into steps, on what else
+// is in the batch, or on which blocks did the work: keys are cut at absolute positions into segments of 256; the four waves
+// of a block take tiles w, w + 4, w + 8, w + 12 of a segment's sixteen under ONE maximum per wave (no running rescaling
+// inside a segment), the waves' sums are folded in their order, then the segments' in theirs, always by `Fold`.  A tile or
+// segment that a row does not see folds as the identity, bit for bit.  Where a step has fewer tiles than would fill the
+// device, blocks take (tile, segment) items, leave the segments' sums in memory and a second kernel folds them - the same
+// folds, the same bits.
+//
+// Rows of one tile have different positions: a key that one row sees and another does not gets weight zero for the
+// other, and zero times an infinity is not zero.  So where a tile of keys is masked for some rows and its values are not
+// all finite, the sums are taken key by key and kept only for the rows that see the key.
+//
+// What bounds it: single tokens wait for their keys - a trip to the block table, one to the records, one to the values, then
+// the fold's launch; prompts run at the matrix cores' rate (64 instructions of 32 cycles per 16 x 16 scores at dim 128) where
+// their tiles fill the device.  Measured, us a layer, 16 heads over 4 of 128, against one wave per (token, head) in plain
+// float32 (`attention_rows`): 3 single tokens after 64 to 700 keys 298 -> 16.1 + 4.6 for the fold; 3 prompts of 333 tokens
+// 811 -> 62.
+
+#include "common.h"
+#include "api.h"
+
+using namespace akv;
+
+namespace {
+
+typedef float floats4 __attribute__((ext_vector_type(4)));
+
+constexpr int kRows = 16;         // query rows of a tile
+constexpr int kSegment = 256;     // keys of a segment
+constexpr int kTiles = 4;         // tiles of 16 keys a wave takes of a segment
+
+struct Args {
+  const float* q;
+  const float* k_pages;
+  const float* v_pages;
+  float* out;
+  float* partial;                 // [tokens * q_heads][segments][dim + 4], or null: a block folds all segments of its tile
+  const int* q_start;
+  const int* seq_lens;
+  const int* block_table;
+  const int* table_rows;
+  int table_width, seqs, q_heads, kv_heads, page_size, window, segments, splits;
+  long num_pages;
+  float scale;
+};
+
+// What a running (maximum, sum of weights, weighted sums) and a later part of it are multiplied by when they are added; the
+// maximum becomes that of both.  A part of no keys has maximum -inf and sums of zero.
+struct Fold {
+  float kept, added;
+  __device__ __forceinline__ Fold(float& maximum, float other) {
+    const float m = fmaxf(maximum, other);
+    kept = maximum == -INFINITY ? 0.f : expf(maximum - m);
+    added = other == -INFINITY ? 0.f : expf(other - m);
+    maximum = m;
+  }
+  // (written as one fused operation: left to the compiler, two kernels could fuse the two products differently)
+  __device__ __forceinline__ float operator()(float total, float part) const { return fmaf(total, kept, part * added); }
+};
+
+__device__ __forceinline__ bool all_finite(const floats4 v) {
+  bool fine = true;              // (an exponent of all ones: infinity or NaN)
+#pragma unroll
+  for (int j = 0; j < 4; ++j) fine = fine && (__float_as_uint(v[j]) & 0x7f800000u) != 0x7f800000u;
+  return fine;
+}
+
+template <int NT>
+__global__ __launch_bounds__(256, NT <= 8 ? 2 : 1) void attention_f32_kernel(const Args a) {
+  constexpr int kDim = 16 * NT;
+  constexpr int kOwn = (NT + 3) / 4;             // tiles of 16 dims whose totals a wave keeps: w, w + 4, ...
+  constexpr int kGroup = NT <= 6 ? kTiles : 2;   // tiles of keys whose records are asked for together (registers)
+  __shared__ floats4 sums_of[4][NT][64];
+  __shared__ float top_of[4][kRows], weight_of[4][kRows];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int c = lane & 15, g = lane >> 4;        // the row (or key, or dim) of a tile, and the lane's group of four
+  const int share = a.q_heads / a.kv_heads, kvh = blockIdx.y;
+
+  // whose tile this is: tiles are numbered request by request
+  int request = -1, tile = blockIdx.x;
+  for (int first = 0; first < a.seqs && request < 0; first += kWave) {
+    const int r = first + lane;
+    const int count = r < a.seqs ? ((a.q_start[r + 1] - a.q_start[r]) * share + kRows - 1) / kRows : 0;
+    int upto = count;
+#pragma unroll
+    for (int step = 1; step < kWave; step <<= 1) {
+      const int other = __shfl_up(upto, step, kWave);
+      if (lane >= step) upto += other;
+    }
+    const unsigned long long here = __ballot(tile < upto);
+    if (here != 0) {
+      const int at = __ffsll(here) - 1;
+      request = first + at;
+      tile -= __shfl(upto - count, at, kWave);
+    } else {
+      tile -= __shfl(upto, kWave - 1, kWave);
+    }
+  }
+  if (request < 0) return;
+  const int token0 = a.q_start[request], tokens = a.q_start[request + 1] - token0;
+  const int rows = tokens * share, row0 = tile * kRows;
+  const int history = a.seq_lens[request] - tokens;
+  const int* table = a.block_table + static_cast<long>(a.table_rows != nullptr ? a.table_rows[request] : request) * a.table_width;
+  const int row = min(row0 + c, rows - 1);       // (rows beyond the request's repeat its last and are not stored)
+  const int token = token0 + row / share, head = kvh * share + row % share;
+  const int pos = history + row / share;
+  const int low = a.window > 0 ? max(0, pos - a.window + 1) : 0;
+  // keys that some row of the tile sees: lowest .. pos_max; that every row sees: low_max .. pos_min
+  const int pos_min = history + row0 / share, pos_max = history + min(row0 + kRows - 1, rows - 1) / share;
+  const int lowest = a.window > 0 ? max(0, pos_min - a.window + 1) : 0;
+  const int low_max = a.window > 0 ? max(0, pos_max - a.window + 1) : 0;
+  const int first_segment = lowest / kSegment, last_segment = pos_max / kSegment;
+
+  const bool split = a.partial != nullptr;
+  const int stride = split ? a.splits : 1, first_own = first_segment + (split ? static_cast<int>(blockIdx.z) : 0);
+  if (first_own > last_segment) return;
+
+  floats4 q[NT];
+  {
+    const float* qp = a.q + (static_cast<long>(token) * a.q_heads + head) * kDim + 4 * g;
+#pragma unroll
+    for (int b = 0; b < NT; ++b) q[b] = *reinterpret_cast<const floats4*>(qp + 16 * b);
+  }
+  const floats4 zero = {0.f, 0.f, 0.f, 0.f};
+  float total_top = -INFINITY, total_weight = 0.f;
+  floats4 total[kOwn];
+#pragma unroll
+  for (int i = 0; i < kOwn; ++i) total[i] = zero;
+
+  for (int segment = first_own; segment <= last_segment; segment += stride) {
+    const int base = segment * kSegment + wave * 16;
+    // ---- scores of the wave's tiles
+    floats4 s[kTiles];
+    const float* vp[kTiles];                     // the lane's four keys in their page's first value row
+    bool there[kTiles];
+#pragma unroll
+    for (int t0 = 0; t0 < kTiles; t0 += kGroup) {
+      floats4 k[kGroup][NT];
+      bool known[kGroup];
+#pragma unroll
+      for (int t = 0; t < kGroup; ++t) {
+        const int key = base + 64 * (t0 + t) + c;
+        const int page = key >= lowest && key <= pos_max ? table[key / a.page_size] : 0;
+        known[t] = page >= 0 && page < a.num_pages;      // (a page that is not the request's is never read: its scores are NaN)
+        const long record = ((known[t] ? page : 0) * static_cast<long>(a.kv_heads) + kvh) * a.page_size + key % a.page_size;
+        const float* kp = a.k_pages + record * kDim + 4 * g;
+#pragma unroll
+        for (int b = 0; b < NT; ++b) k[t][b] = *reinterpret_cast<const floats4*>(kp + 16 * b);
+        // the page of the lane's four keys of the second product (pages hold a multiple of four)
+        const int four = base + 64 * (t0 + t) + 4 * g;
+        const int vpage = four + 3 >= lowest && four <= pos_max ? table[four / a.page_size] : -1;
+        there[t0 + t] = vpage >= 0 && vpage < a.num_pages;
+        vp[t0 + t] = a.v_pages + ((there[t0 + t] ? vpage : 0) * static_cast<long>(a.kv_heads) + kvh) * kDim * a.page_size +
+                     four % a.page_size;
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int t = 0; t < kGroup; ++t) {
+        floats4 sums = zero;
+#pragma unroll
+        for (int b = 0; b < NT; ++b)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) sums = __builtin_amdgcn_mfma_f32_16x16x4f32(k[t][b][e], q[b][e], sums, 0, 0, 0);
+        // lane (c, g) now has row c's scores of keys 4 g .. 4 g + 3
+        const unsigned unknown = static_cast<unsigned>(__ballot(!known[t]) & 0xffffu);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int key = base + 64 * (t0 + t) + 4 * g + j;
+          const float score = (unknown >> (4 * g + j)) & 1u ? __uint_as_float(0x7fc00000u) : sums[j] * a.scale;
+          s[t0 + t][j] = key >= low && key <= pos ? score : -INFINITY;
+        }
+      }
+    }
+    // ---- one maximum for the wave's tiles, weights, their sum
+    float top = -INFINITY;
+#pragma unroll
+    for (int t = 0; t < kTiles; ++t)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) top = fmaxf(top, s[t][j]);
+    top = fmaxf(top, __shfl_xor(top, 16, kWave));
+    top = fmaxf(top, __shfl_xor(top, 32, kWave));
+    const float shift = top == -INFINITY ? 0.f : top;
+    float weight = 0.f;
+#pragma unroll
+    for (int t = 0; t < kTiles; ++t)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int key = base + 64 * t + 4 * g + j;
+        s[t][j] = key >= low && key <= pos ? expf(s[t][j] - shift) : 0.f;
+        weight += s[t][j];
+      }
+    weight += __shfl_xor(weight, 16, kWave);
+    weight += __shfl_xor(weight, 32, kWave);
+    // ---- weighted sums
+    floats4 sums[NT];
+#pragma unroll
+    for (int n = 0; n < NT; ++n) sums[n] = zero;
+#pragma unroll
+    for (int t = 0; t < kTiles; ++t) {
+      const int first_key = base + 64 * t;
+      if (first_key > pos_max || first_key + 15 < lowest) continue;        // (the same for the whole wave)
+      floats4 v[NT];
+#pragma unroll
+      for (int n = 0; n < NT; ++n) v[n] = *reinterpret_cast<const floats4*>(vp[t] + static_cast<long>(16 * n + c) * a.page_size);
+      bool fine = true;
+      if (first_key < low_max || first_key + 15 > pos_min || !__all(there[t])) {
+        // some row does not see some key of the tile.  Slots that nobody has written, or that are not the request's, hold
+        // anything: no row sees them, and they count as zero
+#pragma unroll
+        for (int n = 0; n < NT; ++n) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const int key = first_key + 4 * g + j;
+            if (!there[t] || key < lowest || key > pos_max) v[n][j] = 0.f;
+          }
+          fine = fine && all_finite(v[n]);
+        }
+      }
+      if (__all(fine)) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int n = 0; n < NT; ++n) sums[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[n][e], s[t][e], sums[n], 0, 0, 0);
+      } else {                                   // key by key, for the rows that see it
+#pragma unroll 1
+        for (int four = 0; four < 4; ++four)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int key = first_key + 4 * four + e;
+            const bool seen = key >= low && key <= pos, mine = four == g;
+#pragma unroll
+            for (int n = 0; n < NT; ++n) {
+              const floats4 with = __builtin_amdgcn_mfma_f32_16x16x4f32(mine ? v[n][e] : 0.f, mine ? s[t][e] : 0.f, sums[n], 0, 0, 0);
+              if (seen) sums[n] = with;
+            }
+          }
+      }
+    }
+    // ---- the four waves' parts, in their order
+#pragma unroll
+    for (int n = 0; n < NT; ++n) sums_of[wave][n][lane] = sums[n];
+    if (g == 0) {
+      top_of[wave][c] = top;
+      weight_of[wave][c] = weight;
+    }
+    __syncthreads();
+    float segment_top = -INFINITY, segment_weight = 0.f;
+    floats4 segment_sums[kOwn];
+#pragma unroll
+    for (int i = 0; i < kOwn; ++i) segment_sums[i] = zero;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const Fold f(segment_top, top_of[w][c]);
+      segment_weight = f(segment_weight, weight_of[w][c]);
+#pragma unroll
+      for (int i = 0; i < kOwn; ++i) {
+        if (wave + 4 * i >= NT) continue;
+        const floats4 part = sums_of[w][wave + 4 * i][lane];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) segment_sums[i][j] = f(segment_sums[i][j], part[j]);
+      }
+    }
+    __syncthreads();                             // (the next segment writes LDS again)
+    if (split) {
+      if (row0 + c < rows) {
+        float* at = a.partial + ((static_cast<long>(token) * a.q_heads + head) * a.segments + segment) * (kDim + 4);
+#pragma unroll
+        for (int i = 0; i < kOwn; ++i)
+          if (wave + 4 * i < NT) *reinterpret_cast<floats4*>(at + 16 * (wave + 4 * i) + 4 * g) = segment_sums[i];
+        if (wave == 0 && g == 0) {
+          at[kDim] = segment_top;
+          at[kDim + 1] = segment_weight;
+        }
+      }
+      continue;
+    }
+    const Fold f(total_top, segment_top);
+    total_weight = f(total_weight, segment_weight);
+#pragma unroll
+    for (int i = 0; i < kOwn; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) total[i][j] = f(total[i][j], segment_sums[i][j]);
+  }
+  if (split || row0 + c >= rows) return;
+  float* at = a.out + (static_cast<long>(token) * a.q_heads + head) * kDim + 4 * g;
+#pragma unroll
+  for (int i = 0; i < kOwn; ++i) {
+    if (wave + 4 * i >= NT) continue;
+    floats4 o;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) o[j] = total[i][j] / total_weight;
+    *reinterpret_cast<floats4*>(at + 16 * (wave + 4 * i)) = o;
+  }
+}
+
+// The segments' sums of one (token, head), in their order: a wave a row, four values of dim a lane.
+__global__ __launch_bounds__(256) void attention_f32_fold_kernel(const Args a, const int* __restrict__ positions, int dim, long rows) {
+  const int lane = threadIdx.x & 63;
+  const long row = static_cast<long>(blockIdx.x) * 4 + (threadIdx.x >> 6);
+  if (row >= rows) return;
+  const int pos = positions[row / a.q_heads];
+  const int low = a.window > 0 ? max(0, pos - a.window + 1) : 0;
+  const int d = min(4 * lane, dim - 4);
+  const float* at = a.partial + row * a.segments * (dim + 4);
+  float total_top = -INFINITY, total_weight = 0.f;
+  floats4 total = {0.f, 0.f, 0.f, 0.f};
+  const int last = min(pos / kSegment, a.segments - 1);
+#pragma unroll 4
+  for (int segment = low / kSegment; segment <= last; ++segment) {
+    const float* part = at + static_cast<long>(segment) * (dim + 4);
+    const floats4 sums = *reinterpret_cast<const floats4*>(part + d);
+    const float top = part[dim], weight = part[dim + 1];
+    const Fold f(total_top, top);
+    total_weight = f(total_weight, weight);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) total[j] = f(total[j], sums[j]);
+  }
+  if (4 * lane >= dim) return;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) total[j] /= total_weight;
+  *reinterpret_cast<floats4*>(a.out + row * dim + d) = total;
+}
+
+}  // namespace
+
+extern "C" int akv_attention_f32_fits(int dim, int page_size) {
+  const int nt = dim / 16;
+  return dim % 16 == 0 && page_size > 0 && page_size % 4 == 0 &&
+         ((nt >= 1 && nt <= 6) || nt == 8 || nt == 12 || nt == 16);
+}
+
+extern "C" int akv_attention_f32_segments(long tiles, int longest, int kv_heads) {
+  const int segments = (longest + kSegment - 1) / kSegment;
+  return segments <= 1 || tiles * kv_heads >= device_facts().compute_units ? 1 : segments;
+}
+
+extern "C" int akv_attention_f32(const float* q, const float* k_pages, const float* v_pages, const int* q_start, const int* seq_lens,
+                                 const int* positions, const int* block_table, const int* table_rows, int table_width, float* out,
+                                 float* partial, long tokens, int seqs, long tiles, int segments, int q_heads, int kv_heads,
+                                 int dim, int page_size, long num_pages, float scale, int window, hipStream_t stream) {
+  if (tokens <= 0 || seqs <= 0 || tiles <= 0) return 0;
+  if (!akv_attention_f32_fits(dim, page_size) || tiles > 0x7fffffffL || kv_heads > 65535 || segments < 1 ||
+      (partial == nullptr) != (segments == 1))
+    return -2;
+  Args a{q, k_pages, v_pages, out, partial, q_start, seq_lens, block_table, table_rows, table_width, seqs, q_heads, kv_heads,
+         page_size, window, segments, 1, num_pages, scale};
+  if (partial != nullptr) {
+    const long blocks = tiles * kv_heads, wanted = (2L * device_facts().compute_units + blocks - 1) / blocks;
+    a.splits = static_cast<int>(wanted < segments ? wanted : segments);
+  }
+  const dim3 grid(static_cast<unsigned>(tiles), kv_heads, a.splits);
+  switch (dim / 16) {
+#define AKV_CASE(n) case n: attention_f32_kernel<n><<<grid, 256, 0, stream>>>(a); break
+    AKV_CASE(1); AKV_CASE(2); AKV_CASE(3); AKV_CASE(4); AKV_CASE(5); AKV_CASE(6); AKV_CASE(8); AKV_CASE(12); AKV_CASE(16);
+#undef AKV_CASE
+  }
+  if (partial != nullptr) {
+    const long rows = tokens * q_heads;
+    attention_f32_fold_kernel<<<static_cast<unsigned>((rows + 3) / 4), 256, 0, stream>>>(a, positions, dim, rows);
+  }
+  return AKV_LAUNCH_STATUS();
+}

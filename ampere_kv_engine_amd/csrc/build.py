@@ -19,7 +19,7 @@ import time
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
-SOURCES = ("elementwise.hip", "gemm.hip", "gemm_mfma.hip", "gemm_mid.hip", "gemm_decode.hip", "attention.hip", "sampling.hip")
+SOURCES = ("elementwise.hip", "gemm.hip", "gemm_mfma.hip", "gemm_mid.hip", "gemm_decode.hip", "attention.hip", "attention_f32.hip", "sampling.hip")
 HEADERS = ("common.h", "mfma_tiles.h", "api.h")
 LIBRARY = "libakv_kernels.so"
 # a second library, compiled when a model first needs it: token-wise kernels, mixers and the routed feed-forward of

@@ -151,7 +151,7 @@ class HipKernels(PartsKernels, KernelSet):
                      "akv_linear_mid_adds", "akv_linear_mid_rowscaled", "akv_linear_mid_bands", "akv_linear_mid_most_groups",
                      "akv_linear_adds", "akv_linear_scaled", "akv_linear_adds_rows", "akv_linear_rowscaled",
                      "akv_linear_decode_plan", "akv_read_probe",
-                     "akv_attention_rows", "akv_decode_plan", "akv_sample", "akv_sample_slots", "akv_sample_parts",
+                     "akv_attention_rows", "akv_attention_f32", "akv_attention_f32_fits", "akv_attention_f32_segments", "akv_decode_plan", "akv_sample", "akv_sample_slots", "akv_sample_parts",
                      "akv_step_prologue"):
             getattr(self.lib, name).restype = ctypes.c_int
         self._check_slot_layout()
@@ -1243,13 +1243,42 @@ class HipKernels(PartsKernels, KernelSet):
             return
         if encode_portions is not None:
             encode_portions()
-        self._dense(ctx.seq_of_token, "seq_of_token", torch.int32, (tokens,))
         self._dense(ctx.positions, "positions", torch.int32, (tokens,))
+        if (q.dtype == torch.float32 and not self.one_wave_per_head
+                and self.lib.akv_attention_f32_fits(head_dim, page_size)):
+            self._attention_f32(q, k_pages, v_pages, ctx, meta, q_heads, kv_heads, head_dim, scale, window, out, page_size, num_pages)
+            return
+        self._dense(ctx.seq_of_token, "seq_of_token", torch.int32, (tokens,))
         self._check(self.lib.akv_attention_rows(
             _ptr(q), _ptr(k_pages), _ptr(v_pages), _ptr(ctx.seq_of_token), _ptr(ctx.positions),
             _ptr(meta.block_table), _ptr(rows), meta.width, _ptr(out), _code(q), ctypes.c_long(tokens), q_heads, kv_heads,
             head_dim, page_size, ctypes.c_long(num_pages), ctypes.c_float(scale),
             int(window) if window is not None else 0, self._stream()), "attention")
+
+    def _attention_f32(self, q, k_pages, v_pages, ctx, meta, q_heads, kv_heads, head_dim, scale, window, out, page_size, num_pages):
+        """float32 attention on the matrix cores (`csrc/attention_f32.hip`), single tokens and portions alike; what it does
+        not take - heads or pages of other sizes - goes to the plain kernel, a wave per (token, head).  Both give a token
+        the same bits whatever step it comes in."""
+        tokens = q.shape[0]
+        self._dense(ctx.q_start, "q_start", torch.int32, (ctx.num_seqs + 1,))
+        self._dense(ctx.seq_lens, "seq_lens", torch.int32, (ctx.num_seqs,))
+        starts = ctx.host_q_start
+        if starts[ctx.num_seqs] != tokens or len(ctx.host_seq_lens) != ctx.num_seqs:
+            raise KernelError("the step's request boundaries do not match its tokens")
+        share = q_heads // kv_heads
+        tiles = sum(((starts[r + 1] - starts[r]) * share + 15) // 16 for r in range(ctx.num_seqs))
+        segments = self.lib.akv_attention_f32_segments(ctypes.c_long(tiles), max(ctx.host_seq_lens), kv_heads)
+        partial = None
+        if segments > 1:
+            arena = getattr(ctx, "arena", None)
+            count = tokens * q_heads * segments * (head_dim + 4)
+            partial = (arena.take((count,), torch.float32) if arena is not None
+                       else torch.empty(count, dtype=torch.float32, device=self.device))
+        self._check(self.lib.akv_attention_f32(
+            _ptr(q), _ptr(k_pages), _ptr(v_pages), _ptr(ctx.q_start), _ptr(ctx.seq_lens), _ptr(ctx.positions),
+            _ptr(meta.block_table), _ptr(getattr(meta, "rows", None)), meta.width, _ptr(out), _ptr(partial),
+            ctypes.c_long(tokens), ctx.num_seqs, ctypes.c_long(tiles), segments, q_heads, kv_heads, head_dim, page_size,
+            ctypes.c_long(num_pages), ctypes.c_float(scale), int(window) if window is not None else 0, self._stream()), "attention")
 
     # ---- sampling ----------------------------------------------------------------------------------------
     # A row of logits is cut over several blocks where the rows are few (one block on one compute unit takes 18 us

@@ -1249,6 +1249,54 @@ def test_attention(hip, ref, dtype, q_heads, kv_heads, dim, page_size, portions,
     torch.testing.assert_close(got.cpu().float(), want.float(), **attention_tol(dtype))
 
 
+F32_ATTENTION_SIZES = [(4, 2, 16, 16), (6, 1, 32, 8), (24, 1, 48, 12), (8, 2, 128, 16), (5, 5, 80, 4), (12, 2, 192, 20), (3, 1, 256, 32)]
+
+
+@pytest.mark.parametrize("q_heads,kv_heads,dim,page_size", F32_ATTENTION_SIZES)
+@pytest.mark.parametrize("window", [None, 5, 300])
+def test_float32_attention_gives_the_same_bits_however_a_request_is_cut(hip, ref, q_heads, kv_heads, dim, page_size, window):
+    """A request of 700 tokens fed whole beside others, in portions, and its last tokens alone: segments of keys are folded in
+    a block or by the second kernel, tiles hold other rows - the plain result, and a token's bits are the same everywhere."""
+    q, k_pages, v_pages, ctx, meta, _, _ = _attention_case(torch.float32, q_heads, kv_heads, dim, page_size, [(0, 700), (0, 33), (0, 1)],
+                                                           None, seed=41)
+    c, m = _to_cuda(ctx, meta)
+    whole, want = torch.empty_like(q).cuda(), torch.empty_like(q)
+    args = (q_heads, kv_heads, dim, dim ** -0.5, window)
+    hip.attention(q.cuda(), k_pages.cuda(), v_pages.cuda(), c, m, *args, whole)
+    ref.attention(q, k_pages, v_pages, ctx, meta, *args, want)
+    torch.testing.assert_close(whole.cpu(), want, **tol(torch.float32))
+    for start, stop in ((0, 1), (0, 5), (255, 256), (256, 300), (511, 530), (699, 700)):
+        part = SimpleNamespace(**vars(ctx))
+        part.num_seqs, part.num_tokens, part.host_q_start, part.host_seq_lens = 1, stop - start, [0, stop - start], [stop]
+        part.positions, part.seq_of_token = ctx.positions[start:stop], torch.zeros(stop - start, dtype=torch.int32)
+        part.max_seq_len, part.max_new_tokens = stop, stop - start
+        table = SimpleNamespace(**vars(meta))
+        table.block_table = meta.block_table[:1].contiguous()
+        c, m = _to_cuda(part, table)
+        out = torch.empty(stop - start, q_heads * dim, device="cuda")
+        hip.attention(q[start:stop].cuda(), k_pages.cuda(), v_pages.cuda(), c, m, *args, out)
+        assert torch.equal(out, whole[start:stop]), (start, stop)
+
+
+@pytest.mark.parametrize("poison", [float("inf"), float("nan")])
+@pytest.mark.parametrize("window", [None, 9])
+def test_float32_attention_keeps_a_token_clear_of_keys_it_does_not_see(hip, ref, poison, window):
+    """The key and value of one position are infinite or NaN: tokens that do not see it - earlier ones, and those whose window
+    has passed it - have the plain result all the same, though they share tiles with tokens that see it."""
+    q, k_pages, v_pages, ctx, meta, _, _ = _attention_case(torch.float32, 8, 2, 64, 16, [(0, 60)], None, seed=42)
+    out, want = torch.empty_like(q).cuda(), torch.empty_like(q)
+    ref.attention(q, k_pages, v_pages, ctx, meta, 8, 2, 64, 0.125, window, want)      # (without the poison)
+    page = int(meta.block_table[0, 2])
+    k_pages[page, :, 5], v_pages[page, :, :, 5] = poison, poison            # position 37
+    c, m = _to_cuda(ctx, meta)
+    hip.attention(q.cuda(), k_pages.cuda(), v_pages.cuda(), c, m, 8, 2, 64, 0.125, window, out)
+    clear = [t for t in range(60) if t < 37 or (window is not None and t - 37 >= window)]
+    assert torch.isfinite(out[clear]).all()
+    torch.testing.assert_close(out.cpu()[clear], want[clear], **tol(torch.float32))
+    hit = [t for t in range(60) if t not in clear]
+    assert not torch.isfinite(out[hit]).all(dim=1).any()
+
+
 @pytest.mark.parametrize("shared", ["narrow", "wide", False, "cut"])
 @pytest.mark.parametrize("q_heads,kv_heads,dim,page_size", [(8, 2, 128, 16), (6, 1, 32, 8), (8, 4, 64, 64), (3, 1, 256, 32),
                                                             (5, 5, 80, 16), (40, 2, 64, 8), (4, 2, 16, 128)])
