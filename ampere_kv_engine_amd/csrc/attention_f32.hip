@@ -57,8 +57,9 @@ struct Fold {
   float kept, added;
   __device__ __forceinline__ Fold(float& maximum, float other) {
     const float m = fmaxf(maximum, other);
-    kept = maximum == -INFINITY ? 0.f : expf(maximum - m);
-    added = other == -INFINITY ? 0.f : expf(other - m);
+    const float shift = m == -INFINITY ? 0.f : m;          // (of a part of no keys the factor is exp(-inf))
+    kept = expf(maximum - shift);
+    added = expf(other - shift);
     maximum = m;
   }
   // (written as one fused operation: left to the compiler, two kernels could fuse the two products differently)
@@ -68,12 +69,14 @@ struct Fold {
 __device__ __forceinline__ bool all_finite(const floats4 v) {
   bool fine = true;              // (an exponent of all ones: infinity or NaN)
 #pragma unroll
-  for (int j = 0; j < 4; ++j) fine = fine && (__float_as_uint(v[j]) & 0x7f800000u) != 0x7f800000u;
+  for (int j = 0; j < 4; ++j) fine = fine & ((__float_as_uint(v[j]) & 0x7f800000u) != 0x7f800000u);
   return fine;
 }
 
-template <int NT>
-__global__ __launch_bounds__(256, NT <= 8 ? 2 : 1) void attention_f32_kernel(const Args a) {
+// FEW: there are fewer blocks than compute units, and a block waits for its loads: a tile's values are asked for a tile ahead,
+// with the registers of one wave a SIMD.  Otherwise two waves a SIMD hide each other's waits.
+template <int NT, bool FEW>
+__global__ __launch_bounds__(256, FEW || NT > 8 ? 1 : 2) void attention_f32_kernel(const Args a) {
   constexpr int kDim = 16 * NT;
   constexpr int kOwn = (NT + 3) / 4;             // tiles of 16 dims whose totals a wave keeps: w, w + 4, ...
   constexpr int kGroup = NT <= 6 ? kTiles : 2;   // tiles of keys whose records are asked for together (registers)
@@ -137,6 +140,8 @@ __global__ __launch_bounds__(256, NT <= 8 ? 2 : 1) void attention_f32_kernel(con
   for (int segment = first_own; segment <= last_segment; segment += stride) {
     const int base = segment * kSegment + wave * 16;
     // ---- scores of the wave's tiles
+    // (no load stands behind a test: the compiler would wait for it before the next.  A key that no row sees asks for the
+    // nearest that one does)
     floats4 s[kTiles];
     const float* vp[kTiles];                     // the lane's four keys in their page's first value row
     bool there[kTiles];
@@ -144,21 +149,24 @@ __global__ __launch_bounds__(256, NT <= 8 ? 2 : 1) void attention_f32_kernel(con
     for (int t0 = 0; t0 < kTiles; t0 += kGroup) {
       floats4 k[kGroup][NT];
       bool known[kGroup];
+      int key[kGroup], four[kGroup], page[kGroup], vpage[kGroup];
 #pragma unroll
       for (int t = 0; t < kGroup; ++t) {
-        const int key = base + 64 * (t0 + t) + c;
-        const int page = key >= lowest && key <= pos_max ? table[key / a.page_size] : 0;
-        known[t] = page >= 0 && page < a.num_pages;      // (a page that is not the request's is never read: its scores are NaN)
-        const long record = ((known[t] ? page : 0) * static_cast<long>(a.kv_heads) + kvh) * a.page_size + key % a.page_size;
+        key[t] = min(max(base + 64 * (t0 + t) + c, lowest), pos_max);
+        four[t] = min(max(base + 64 * (t0 + t) + 4 * g, lowest & ~3), pos_max & ~3);      // (pages hold a multiple of four)
+        page[t] = table[key[t] / a.page_size];
+        vpage[t] = table[four[t] / a.page_size];
+      }
+#pragma unroll
+      for (int t = 0; t < kGroup; ++t) {
+        known[t] = (page[t] >= 0) & (page[t] < a.num_pages);       // (a page that is not the request's is never read: its scores
+        there[t0 + t] = (vpage[t] >= 0) & (vpage[t] < a.num_pages);                                              // are NaN)
+        const long record = ((known[t] ? page[t] : 0) * static_cast<long>(a.kv_heads) + kvh) * a.page_size + key[t] % a.page_size;
         const float* kp = a.k_pages + record * kDim + 4 * g;
 #pragma unroll
         for (int b = 0; b < NT; ++b) k[t][b] = *reinterpret_cast<const floats4*>(kp + 16 * b);
-        // the page of the lane's four keys of the second product (pages hold a multiple of four)
-        const int four = base + 64 * (t0 + t) + 4 * g;
-        const int vpage = four + 3 >= lowest && four <= pos_max ? table[four / a.page_size] : -1;
-        there[t0 + t] = vpage >= 0 && vpage < a.num_pages;
-        vp[t0 + t] = a.v_pages + ((there[t0 + t] ? vpage : 0) * static_cast<long>(a.kv_heads) + kvh) * kDim * a.page_size +
-                     four % a.page_size;
+        vp[t0 + t] = a.v_pages + ((there[t0 + t] ? vpage[t] : 0) * static_cast<long>(a.kv_heads) + kvh) * kDim * a.page_size +
+                     four[t] % a.page_size;
       }
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -174,7 +182,7 @@ __global__ __launch_bounds__(256, NT <= 8 ? 2 : 1) void attention_f32_kernel(con
         for (int j = 0; j < 4; ++j) {
           const int key = base + 64 * (t0 + t) + 4 * g + j;
           const float score = (unknown >> (4 * g + j)) & 1u ? __uint_as_float(0x7fc00000u) : sums[j] * a.scale;
-          s[t0 + t][j] = key >= low && key <= pos ? score : -INFINITY;
+          s[t0 + t][j] = (key >= low) & (key <= pos) ? score : -INFINITY;
         }
       }
     }
@@ -192,23 +200,32 @@ __global__ __launch_bounds__(256, NT <= 8 ? 2 : 1) void attention_f32_kernel(con
     for (int t = 0; t < kTiles; ++t)
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const int key = base + 64 * t + 4 * g + j;
-        s[t][j] = key >= low && key <= pos ? expf(s[t][j] - shift) : 0.f;
+        s[t][j] = expf(s[t][j] - shift);         // (exp(-inf) of a key that the row does not see)
         weight += s[t][j];
       }
     weight += __shfl_xor(weight, 16, kWave);
     weight += __shfl_xor(weight, 32, kWave);
     // ---- weighted sums
-    floats4 sums[NT];
+    constexpr bool kAhead = FEW && NT <= 8;
+    floats4 sums[NT], v[NT], next[kAhead ? NT : 1];
+    const auto values = [&](int t, floats4* to) {
+#pragma unroll
+      for (int n = 0; n < NT; ++n) to[n] = *reinterpret_cast<const floats4*>(vp[t] + static_cast<long>(16 * n + c) * a.page_size);
+    };
 #pragma unroll
     for (int n = 0; n < NT; ++n) sums[n] = zero;
+    if constexpr (kAhead) values(0, next);
 #pragma unroll
     for (int t = 0; t < kTiles; ++t) {
       const int first_key = base + 64 * t;
-      if (first_key > pos_max || first_key + 15 < lowest) continue;        // (the same for the whole wave)
-      floats4 v[NT];
+      if constexpr (kAhead) {
 #pragma unroll
-      for (int n = 0; n < NT; ++n) v[n] = *reinterpret_cast<const floats4*>(vp[t] + static_cast<long>(16 * n + c) * a.page_size);
+        for (int n = 0; n < NT; ++n) v[n] = next[n];
+        if (t + 1 < kTiles) values(t + 1, next);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if (first_key > pos_max || first_key + 15 < lowest) continue;        // (the same for the whole wave)
+      if constexpr (!kAhead) values(t, v);
       bool fine = true;
       if (first_key < low_max || first_key + 15 > pos_min || !__all(there[t])) {
         // some row does not see some key of the tile.  Slots that nobody has written, or that are not the request's, hold
@@ -218,9 +235,9 @@ __global__ __launch_bounds__(256, NT <= 8 ? 2 : 1) void attention_f32_kernel(con
 #pragma unroll
           for (int j = 0; j < 4; ++j) {
             const int key = first_key + 4 * g + j;
-            if (!there[t] || key < lowest || key > pos_max) v[n][j] = 0.f;
+            v[n][j] = there[t] & (key >= lowest) & (key <= pos_max) ? v[n][j] : 0.f;
           }
-          fine = fine && all_finite(v[n]);
+          fine = fine & all_finite(v[n]);
         }
       }
       if (__all(fine)) {
@@ -356,8 +373,13 @@ extern "C" int akv_attention_f32(const float* q, const float* k_pages, const flo
     a.splits = static_cast<int>(wanted < segments ? wanted : segments);
   }
   const dim3 grid(static_cast<unsigned>(tiles), kv_heads, a.splits);
+  const bool few = tiles * kv_heads < device_facts().compute_units;
   switch (dim / 16) {
-#define AKV_CASE(n) case n: attention_f32_kernel<n><<<grid, 256, 0, stream>>>(a); break
+#define AKV_CASE(n)                                                       \
+  case n:                                                                 \
+    if (few) attention_f32_kernel<n, true><<<grid, 256, 0, stream>>>(a);  \
+    else attention_f32_kernel<n, false><<<grid, 256, 0, stream>>>(a);     \
+    break
     AKV_CASE(1); AKV_CASE(2); AKV_CASE(3); AKV_CASE(4); AKV_CASE(5); AKV_CASE(6); AKV_CASE(8); AKV_CASE(12); AKV_CASE(16);
 #undef AKV_CASE
   }

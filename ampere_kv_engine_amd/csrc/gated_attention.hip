@@ -732,3 +732,360 @@ int akv_gated_attention_rows(const void* q, const void* k_pages, const void* v_p
   return AKV_LAUNCH_STATUS();
 }
 }
+
+namespace {
+
+// ---- single tokens on the matrix cores ---------------------------------------------------------------------------------
+// bfloat16, the sizes of the tiles above.  What a single token waits for is its keys and values: a block that walks them all
+// for one query head asks for them a tile after the other, and the heads of a group ask for the same ones again.  Here a
+// block is a token, a vector of a key head with all query vectors that read it as the columns of a tile, and ONE segment of 16
+// steps of 16 keys at absolute positions; its four waves take four steps each and ask for all of their keys and values
+// before the first score: one trip to the block table, one to the pages.  A wave's 64 keys have one maximum; waves and
+// segments are folded in their order.  A token of one segment is finished by its block; of more, the segments' sums are left
+// in `partial` ([token][query vector][segment][vdim + 4]) and added by `gated_attention_fold_kernel`.  How a token's keys are
+// cut depends on its position alone.  Scores, maxima, weights and sums are float32; a weight enters the second product as
+// three bfloat16 numbers that add up to it.
+// What bounds it: trips to memory in a row (positions, table, keys and values, then the fold's launch).  8 tokens of 2,048 keys
+// (34 MB), 16 query and 4 key heads of 128, us: 39 with a block of sixteen waves per (token, query head) in `rows`, 14 + 7 for
+// the fold here; two maps of 64 over a window of 1,024: 26.5 -> 12 + 5.  (With the loads behind tests, which the compiler
+// waits for one by one, and the softcap's and the bias's code in every kernel: 33.)
+struct Steps {
+  int lowest, first, kept, all;      // the window's first key; its step, the steps of the kept first keys, all steps
+  __device__ __forceinline__ Steps(int pos, int window, int chunk, int keep_first) {
+    lowest = window > 0 ? max(0, pos - window + 1) : 0;
+    if (chunk > 0) lowest = max(lowest, pos / chunk * chunk);
+    first = lowest >> 4;
+    kept = min((keep_first + 15) >> 4, first);
+    all = kept + (pos >> 4) - first + 1;
+  }
+  __device__ __forceinline__ int key(int turn) const { return (turn < kept ? turn : first + turn - kept) << 4; }
+};
+constexpr int kSegmentSteps = 16;
+
+// What a running (maximum, sum of weights, weighted sums) and a later part of it are multiplied by when they are added.
+struct Fold {
+  float kept, added;
+  __device__ __forceinline__ Fold(float& maximum, float other) {
+    const float m = fmaxf(maximum, other);
+    const float shift = m == -INFINITY ? 0.f : m;          // (of a part of no keys the factor is exp(-inf))
+    kept = expf(maximum - shift);
+    added = expf(other - shift);
+    maximum = m;
+  }
+  __device__ __forceinline__ float operator()(float total, float part) const { return fmaf(total, kept, part * added); }
+};
+
+struct SingleArgs {
+  const bf16_t *q, *k_pages, *v_pages, *gates;
+  const int *seq_of_token, *positions, *block_table, *table_rows;
+  const float *sink_logits, *distance_bias;
+  bf16_t* out;
+  float* partial;
+  long gate_stride, num_pages, out_stride;
+  float scale, softcap, out_scale;
+  int gate_at, table_width, q_heads, kv_heads, page_size, chunk, window, sink, maps, keep_first, segments;
+};
+
+__device__ __forceinline__ float gate_of(const SingleArgs& a, long n, int vector) {
+  if (a.gates == nullptr) return a.out_scale;
+  return a.out_scale / (1.f + expf(-to_float(a.gates[n * a.gate_stride + a.gate_at + vector])));
+}
+__device__ __forceinline__ float sink_of(const SingleArgs& a, int vector) {
+  return !a.sink ? -INFINITY : a.sink_logits != nullptr ? a.sink_logits[vector] : 0.f;
+}
+
+// SHAPED: scores have a softcap or a distance bias (their code, in every kernel, would be most of what a block fetches).
+template <int DT, int VT, bool SHAPED>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) void gated_attention_singles_kernel(const SingleArgs a) {
+  constexpr int DIM = 32 * DT, VDIM = 16 * VT, kOwn = (VT + 3) / 4;      // tiles of values whose totals a wave keeps
+  __shared__ float4_t sums_of[4][VT][kWave];
+  __shared__ float top_of[4][16], weight_of[4][16];
+  const int wave = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
+  const int col = lane & 15, grp = lane >> 4;
+  const long n = blockIdx.x / a.segments;
+  const int segment = blockIdx.x % a.segments;
+  const int share = a.q_heads / a.kv_heads / a.maps, groups = (share + 15) / 16;      // query vectors of a key vector
+  const int kvh = blockIdx.y / (a.maps * groups), map = blockIdx.y / groups % a.maps, of_group = blockIdx.y % groups * 16 + col;
+  const int vector = (kvh * share + min(of_group, share - 1)) * a.maps + map;
+  const int r = a.table_rows != nullptr ? a.table_rows[a.seq_of_token[n]] : a.seq_of_token[n];
+  const int pos = a.positions[n];
+  const Steps steps(pos, a.window, a.chunk, a.keep_first);
+  const int first = segment * kSegmentSteps;
+  if (first >= steps.all) return;
+
+  uint4 q[DT], keys[4][DT];
+  uint2 values[4][VT];
+  int at_key[4], offset[4];
+  long page[4];
+  bool foreign[4];
+  const int* table = a.block_table + static_cast<long>(r) * a.table_width;
+  // (no load stands behind a test: the compiler would wait for it before the next; a step beyond the last asks for the last)
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int turn = first + wave + 4 * i;
+    const int key = steps.key(min(turn, steps.all - 1));
+    page[i] = table[key / a.page_size];
+    offset[i] = key % a.page_size;
+    at_key[i] = turn < steps.all ? key : pos + 1;                  // (none of a step beyond the last counts)
+  }
+  const bf16_t* qp = a.q + (n * a.q_heads + vector) * DIM + grp * 8;
+#pragma unroll
+  for (int d = 0; d < DT; ++d) q[d] = load_bf16x8(qp + d * 32);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    foreign[i] = page[i] < 0 || page[i] >= a.num_pages;            // (a page that is not the request's is never read: its
+    const long from = (foreign[i] ? 0 : page[i]) * a.kv_heads + kvh;                                 // scores are NaN)
+    const bf16_t* kp = a.k_pages + ((from * a.page_size + offset[i] + col) * a.maps + map) * DIM + grp * 8;
+#pragma unroll
+    for (int d = 0; d < DT; ++d) keys[i][d] = load_bf16x8(kp + d * 32);
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const long from = (foreign[i] ? 0 : page[i]) * a.kv_heads + kvh;
+    const bf16_t* vp = a.v_pages + (from * VDIM + col) * a.page_size + offset[i] + grp * 4;
+#pragma unroll
+    for (int v = 0; v < VT; ++v) values[i][v] = *reinterpret_cast<const uint2*>(vp + static_cast<long>(v) * 16 * a.page_size);
+  }
+  __builtin_amdgcn_sched_barrier(0);             // (else the loads are moved down to where they are used)
+
+  const auto counts = [&](int i, int e) {
+    const int j = at_key[i] + 4 * grp + e;
+    return ((j >= steps.lowest) | (j < a.keep_first)) & (j <= pos);
+  };
+  const float bias_size = SHAPED && a.distance_bias != nullptr ? a.distance_bias[vector] : 0.f;
+  const float bias_rate = SHAPED && a.distance_bias != nullptr ? a.distance_bias[a.q_heads + vector] : 0.f;
+  float s[4][4], top = -INFINITY;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    float4_t acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int d = 0; d < DT; ++d)
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, keys[i][d]), __builtin_bit_cast(bf16x8_t, q[d]),
+                                                    acc, 0, 0, 0);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      float v = acc[e] * a.scale;
+      if constexpr (SHAPED) {
+        if (a.softcap > 0.f) v = a.softcap * tanhf(v / a.softcap);
+        if (a.distance_bias != nullptr)
+          v -= bias_size * log1pf(bias_rate * static_cast<float>(max(pos - at_key[i] - 4 * grp - e, 0)));
+      }
+      if (foreign[i]) v = __uint_as_float(0x7fc00000u);
+      s[i][e] = counts(i, e) ? v : -INFINITY;
+      top = fmaxf(top, s[i][e]);
+    }
+  }
+  top = fmaxf(top, __shfl_xor(top, 16, kWave));
+  top = fmaxf(top, __shfl_xor(top, 32, kWave));
+  const float shift = top == -INFINITY ? 0.f : top;
+  float weight = 0.f;
+  bool fine = true;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    uint32_t kept[2] = {0u, 0u};                 // slots that nobody has written hold anything: what does not count is zero
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const bool counted = counts(i, e);
+      s[i][e] = expf(s[i][e] - shift);           // (exp(-inf) where the key does not count)
+      weight += s[i][e];
+      kept[e >> 1] |= counted & !foreign[i] ? 0xffffu << (16 * (e & 1)) : 0u;
+    }
+#pragma unroll
+    for (int v = 0; v < VT; ++v) {
+      values[i][v].x &= kept[0];
+      values[i][v].y &= kept[1];
+      fine = fine & ((values[i][v].x & 0x7f80u) != 0x7f80u) & ((values[i][v].x & 0x7f800000u) != 0x7f800000u) &
+             ((values[i][v].y & 0x7f80u) != 0x7f80u) & ((values[i][v].y & 0x7f800000u) != 0x7f800000u);
+    }
+  }
+  weight += __shfl_xor(weight, 16, kWave);
+  weight += __shfl_xor(weight, 32, kWave);
+
+  float4_t sums[VT];
+#pragma unroll
+  for (int v = 0; v < VT; ++v) sums[v] = float4_t{0.f, 0.f, 0.f, 0.f};
+  if (__builtin_expect(__all(fine), 1)) {
+    // two steps of 16 keys are one product over 32: a lane's eight are keys 4 grp .. + 3 of the one and of the other
+#pragma unroll
+    for (int i = 0; i < 4; i += 2) {
+      float left[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) left[e] = s[i + (e >> 2)][e & 3];
+#pragma unroll
+      for (int part = 0; part < 3; ++part) {
+        uint32_t words[4];
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+          words[w] = bf16_pair(left[2 * w], left[2 * w + 1]);
+          left[2 * w] -= __uint_as_float(words[w] << 16);
+          left[2 * w + 1] -= __uint_as_float(words[w] & 0xffff0000u);
+        }
+        const bf16x8_t weights = __builtin_bit_cast(bf16x8_t, make_uint4(words[0], words[1], words[2], words[3]));
+#pragma unroll
+        for (int v = 0; v < VT; ++v)
+          sums[v] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              __builtin_bit_cast(bf16x8_t, make_uint4(values[i][v].x, values[i][v].y, values[i + 1][v].x, values[i + 1][v].y)),
+              weights, sums[v], 0, 0, 0);
+      }
+    }
+  } else {
+    // an infinite or undefined value: a weight of zero takes nothing from it (zero times infinity is not zero), so the keys
+    // are added one by one - of step i the one that lies in element e of group `four` - where their weight is not zero
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll 1
+      for (int one = 0; one < 16; ++one) {
+        const int four = one >> 2, e = one & 3;
+        const float own = e == 0 ? s[i][0] : e == 1 ? s[i][1] : e == 2 ? s[i][2] : s[i][3];
+        const bool taken = __shfl(own, 16 * four + col, kWave) != 0.f;
+        const uint32_t place = grp == four ? 0xffffu << (16 * (e & 1)) : 0u;
+        const uint2 only = make_uint2(e < 2 ? place : 0u, e < 2 ? 0u : place);
+        short4_t part[3];
+        float left = own;
+#pragma unroll
+        for (int t = 0; t < 3; ++t) {
+          const uint32_t bits = bf16_bits(left);
+          left -= __uint_as_float(bits << 16);
+          part[t] = __builtin_bit_cast(short4_t, make_uint2((bits | bits << 16) & only.x, (bits | bits << 16) & only.y));
+        }
+#pragma unroll
+        for (int v = 0; v < VT; ++v) {
+          const short4_t value = __builtin_bit_cast(short4_t, make_uint2(values[i][v].x & only.x, values[i][v].y & only.y));
+          float4_t with = sums[v];
+#pragma unroll
+          for (int t = 0; t < 3; ++t) with = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(value, part[t], with, 0, 0, 0);
+          if (taken) sums[v] = with;
+        }
+      }
+  }
+
+  // the four waves' parts, in their order; a token of one segment starts from its sink
+#pragma unroll
+  for (int v = 0; v < VT; ++v) sums_of[wave][v][lane] = sums[v];
+  if (grp == 0) {
+    top_of[wave][col] = top;
+    weight_of[wave][col] = weight;
+  }
+  __syncthreads();
+  const bool whole = steps.all <= kSegmentSteps;
+  float total_top = whole ? sink_of(a, vector) : -INFINITY, total_weight = total_top == -INFINITY ? 0.f : 1.f;
+  float4_t total[kOwn];
+#pragma unroll
+  for (int i = 0; i < kOwn; ++i) total[i] = float4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    const Fold f(total_top, top_of[w][col]);
+    total_weight = f(total_weight, weight_of[w][col]);
+#pragma unroll
+    for (int i = 0; i < kOwn; ++i) {
+      if (wave + 4 * i >= VT) continue;
+      const float4_t part = sums_of[w][wave + 4 * i][lane];
+#pragma unroll
+      for (int d = 0; d < 4; ++d) total[i][d] = f(total[i][d], part[d]);
+    }
+  }
+  if (of_group >= share) return;
+  if (!whole) {
+    float* at = a.partial + ((n * a.q_heads + vector) * a.segments + segment) * (VDIM + 4);
+#pragma unroll
+    for (int i = 0; i < kOwn; ++i)
+      if (wave + 4 * i < VT) *reinterpret_cast<float4_t*>(at + 16 * (wave + 4 * i) + 4 * grp) = total[i];
+    if (wave == 0 && grp == 0) {
+      at[VDIM] = total_top;
+      at[VDIM + 1] = total_weight;
+    }
+    return;
+  }
+  const float factor = gate_of(a, n, vector) / total_weight;
+  bf16_t* at = a.out + n * a.out_stride + static_cast<long>(vector) * VDIM + 4 * grp;
+#pragma unroll
+  for (int i = 0; i < kOwn; ++i) {
+    if (wave + 4 * i >= VT) continue;
+    uint2 packed;
+    packed.x = bf16_pair(total[i][0] * factor, total[i][1] * factor);
+    packed.y = bf16_pair(total[i][2] * factor, total[i][3] * factor);
+    *reinterpret_cast<uint2*>(at + 16 * (wave + 4 * i)) = packed;
+  }
+}
+
+// The segments of every (token, query vector) that has more than one, in their order: a wave a row, four values a lane.
+__global__ __launch_bounds__(256) void gated_attention_fold_kernel(const SingleArgs a, int vdim, long rows) {
+  const int lane = threadIdx.x & (kWave - 1);
+  const long row = static_cast<long>(blockIdx.x) * 4 + threadIdx.x / kWave;
+  if (row >= rows) return;
+  const long n = row / a.q_heads;
+  const int vector = static_cast<int>(row % a.q_heads);
+  const Steps steps(a.positions[n], a.window, a.chunk, a.keep_first);
+  if (steps.all <= kSegmentSteps || 4 * lane >= vdim) return;
+  const int count = min((steps.all + kSegmentSteps - 1) / kSegmentSteps, a.segments);
+  const float* at = a.partial + row * a.segments * (vdim + 4);
+  float total_top = sink_of(a, vector), total_weight = total_top == -INFINITY ? 0.f : 1.f;
+  float4_t total = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 8
+  for (int segment = 0; segment < count; ++segment) {
+    const float* part = at + static_cast<long>(segment) * (vdim + 4);
+    const float4_t sums = *reinterpret_cast<const float4_t*>(part + 4 * lane);
+    const Fold f(total_top, part[vdim]);
+    total_weight = f(total_weight, part[vdim + 1]);
+#pragma unroll
+    for (int d = 0; d < 4; ++d) total[d] = f(total[d], sums[d]);
+  }
+  const float factor = gate_of(a, n, vector) / total_weight;
+  uint2 packed;
+  packed.x = bf16_pair(total[0] * factor, total[1] * factor);
+  packed.y = bf16_pair(total[2] * factor, total[3] * factor);
+  *reinterpret_cast<uint2*>(a.out + n * a.out_stride + static_cast<long>(vector) * vdim + 4 * lane) = packed;
+}
+
+}  // namespace
+
+extern "C" {
+
+int akv_gated_attention_singles(const void* q, const void* k_pages, const void* v_pages, const void* gates, long gate_stride,
+                                int gate_at, const int* seq_of_token, const int* positions, const int* block_table,
+                                const int* table_rows, int table_width, void* out, float* partial, int segments, int tokens,
+                                int q_heads, int kv_heads, int dim, int vdim, int page_size, long num_pages, float scale,
+                                float softcap, int chunk, int window, int sink, long out_stride, float out_scale,
+                                const float* sink_logits, int maps, int keep_first, const float* distance_bias,
+                                hipStream_t stream) {
+  if (tokens <= 0) return 0;
+  if (page_size % 16 != 0 || maps < 1 || kv_heads <= 0 || q_heads % (kv_heads * maps) != 0 || segments < 1 || static_cast<long>(tokens) * segments > 0x7fffffffL ||
+      (segments > 1 && partial == nullptr))
+    return -2;
+  const SingleArgs a{static_cast<const bf16_t*>(q), static_cast<const bf16_t*>(k_pages), static_cast<const bf16_t*>(v_pages),
+                     static_cast<const bf16_t*>(gates), seq_of_token, positions, block_table, table_rows, sink_logits,
+                     distance_bias, static_cast<bf16_t*>(out), partial, gate_stride, num_pages, out_stride, scale, softcap,
+                     out_scale, gate_at, table_width, q_heads, kv_heads, page_size, chunk, window, sink, maps, keep_first, segments};
+  const long columns = static_cast<long>(kv_heads) * maps * ((q_heads / kv_heads / maps + 15) / 16);
+  if (columns > 65535) return -2;
+  const dim3 grid(static_cast<unsigned>(static_cast<long>(tokens) * segments), static_cast<unsigned>(columns));
+#define AKV_SINGLES(DT, VT)                                                                        \
+  if (softcap > 0.f || distance_bias != nullptr)                                                   \
+    gated_attention_singles_kernel<DT, VT, true><<<grid, 256, 0, stream>>>(a);                      \
+  else                                                                                             \
+    gated_attention_singles_kernel<DT, VT, false><<<grid, 256, 0, stream>>>(a)
+#define AKV_SINGLES_V(DT)                  \
+  switch (vdim) {                          \
+    case 32: AKV_SINGLES(DT, 2); break;    \
+    case 64: AKV_SINGLES(DT, 4); break;    \
+    case 128: AKV_SINGLES(DT, 8); break;   \
+    case 256: AKV_SINGLES(DT, 16); break;  \
+    default: return -2;                    \
+  }
+  switch (dim) {
+    case 32: AKV_SINGLES_V(1); break;
+    case 64: AKV_SINGLES_V(2); break;
+    case 128: AKV_SINGLES_V(4); break;
+    case 256: AKV_SINGLES_V(8); break;
+    default: return -2;
+  }
+#undef AKV_SINGLES_V
+#undef AKV_SINGLES
+  if (segments > 1) {
+    const long rows = static_cast<long>(tokens) * q_heads;
+    gated_attention_fold_kernel<<<static_cast<unsigned>((rows + 3) / 4), 256, 0, stream>>>(a, vdim, rows);
+  }
+  return AKV_LAUNCH_STATUS();
+}
+
+}

@@ -45,7 +45,7 @@ class PartsKernels:
                          "akv_rotate_queries", "akv_heads_linear", "akv_latent_attend", "akv_latent_attend_mfma", "akv_conv_silu",
                          "akv_conv_state_update", "akv_selective_scan", "akv_route", "akv_gate_relu_squared",
                          "akv_parts_slot_layout", "akv_conv_taps", "akv_scaled_sum", "akv_unit_norm_write",
-                         "akv_gated_attention_rows", "akv_gated_attention_tiles", "akv_retention", "akv_retention_chunked", "akv_gated_linear_scan", "akv_route_chosen",
+                         "akv_gated_attention_rows", "akv_gated_attention_tiles", "akv_gated_attention_singles", "akv_retention", "akv_retention_chunked", "akv_gated_linear_scan", "akv_route_chosen",
                          "akv_gate_pair_mul", "akv_route_corrected", "akv_add_weighted_rows", "akv_embed_normed", "akv_gated_activation", "akv_difference_norm_gate",
                          "akv_delta_rule", "akv_embed_rows", "akv_norm_gate_rows", "akv_gate_activation", "akv_softcap",
                          "akv_token_shift", "akv_tanh_rows", "akv_time_mixing", "akv_matrix_memory"):
@@ -792,7 +792,8 @@ class PartsKernels:
 
     # ---- attention with unit-normed queries and keys, a softcap, chunks, a sink and a gate per head ----------------------
     MAX_VALUE_DIM = 256
-    MATRIX_CORE_HEAD_DIMS = (32, 64, 128, 256)      # widths of keys and of values that the portions' kernel is built for
+    MATRIX_CORE_HEAD_DIMS = (32, 64, 128, 256)      # widths of keys and of values that the matrix-core kernels are built for
+    SEGMENT_STEPS = 16      # steps of 16 keys in a segment of a single token's keys (`kSegmentSteps` of the kernel)
 
     def check_gated_attention_sizes(self, q_heads: int, kv_heads: int, dim: int, vdim: int, page_size: int) -> None:
         if q_heads % kv_heads:
@@ -909,26 +910,42 @@ class PartsKernels:
         tail = (ctypes.c_float(scale), ctypes.c_float(softcap if softcap is not None else 0.0),
                 int(chunk) if chunk is not None else 0, int(window) if window is not None else 0, 1 if sink else 0,
                 _long(out.shape[1]), ctypes.c_float(out_scale), _ptr(sink_logits), maps, int(keep_first), _ptr(distance_bias), self._stream())
-        singles = tokens
+        # keys a row can see at most (a bound that a recorded step keeps)
+        span = min(x for x in (chunk, window, ctx.max_seq_len) if x is not None)
         if (q.dtype == torch.bfloat16 and dim in self.MATRIX_CORE_HEAD_DIMS and vdim in self.MATRIX_CORE_HEAD_DIMS
                 and page_size % 16 == 0 and out.shape[1] % 4 == 0 and out_at % 4 == 0):
-            # single tokens: a wave per token and head; the portions' rows, which follow them, go to the matrix cores
+            # on the matrix cores: single tokens with the query heads of a key head as a tile's columns, the portions' rows,
+            # which follow them, with sixteen tokens of a head
             singles = ctx.num_decode_seqs
+            if singles:
+                # steps of 16 keys that a token's keys can touch: where the first of them need not be a step's first, one more
+                steps = ((span + 15) // 16 + (0 if window is None and (chunk is None or chunk % 16 == 0) else 1)
+                         + (keep_first + 15) // 16)
+                segments = (steps + self.SEGMENT_STEPS - 1) // self.SEGMENT_STEPS
+                partial = None
+                if segments > 1:
+                    arena = getattr(ctx, "arena", None)
+                    count = singles * q_heads * segments * (vdim + 4)
+                    partial = (arena.take((count,), torch.float32) if arena is not None
+                               else torch.empty(count, dtype=torch.float32, device=self.device))
+                self._check(self._parts().akv_gated_attention_singles(
+                    _ptr(q), _ptr(k_pages), _ptr(v_pages), _ptr(gates), _long(gate_stride), gate_at, _ptr(ctx.seq_of_token),
+                    _ptr(ctx.positions), _ptr(meta.block_table), _ptr(meta.rows), meta.width, _ptr_at(out, out_at), _ptr(partial),
+                    segments, singles, q_heads, kv_heads, dim, vdim, page_size, _long(num_pages), *tail),
+                    "gated_attention of single tokens")
             self._check(self._parts().akv_gated_attention_tiles(
                 _ptr(q), _ptr(k_pages), _ptr(v_pages), _ptr(gates), _long(gate_stride), gate_at, _ptr(ctx.seq_of_token),
                 _ptr(ctx.q_start), _ptr(ctx.positions), _ptr(meta.block_table), _ptr(meta.rows), meta.width,
                 _ptr_at(out, out_at), singles, tokens, q_heads, kv_heads, dim, vdim, page_size, _long(num_pages), *tail),
                 "gated_attention on the matrix cores")
-        if singles:
-            # waves that share a token's head: by the most keys a row can see (a bound that a recorded step keeps), fewer
-            # where the rows alone fill the device
-            span = min(x for x in (chunk, window, ctx.max_seq_len) if x is not None)
-            row_waves = max(1, min(16 if singles * q_heads <= 4096 else 4, span // 128))
-            self._check(self._parts().akv_gated_attention_rows(
-                _ptr(q), _ptr(k_pages), _ptr(v_pages), _ptr(gates), _long(gate_stride), gate_at, _ptr(ctx.seq_of_token),
-                _ptr(ctx.positions), _ptr(meta.block_table), _ptr(meta.rows), meta.width, _ptr_at(out, out_at),
-                self._code_of(q), _long(singles), q_heads, kv_heads, dim, vdim, page_size, _long(num_pages), *tail[:-5], row_waves,
-                *tail[-5:]), "gated_attention")
+            return
+        # waves that share a token's head: by the most keys a row can see, fewer where the rows alone fill the device
+        row_waves = max(1, min(16 if tokens * q_heads <= 4096 else 4, span // 128))
+        self._check(self._parts().akv_gated_attention_rows(
+            _ptr(q), _ptr(k_pages), _ptr(v_pages), _ptr(gates), _long(gate_stride), gate_at, _ptr(ctx.seq_of_token),
+            _ptr(ctx.positions), _ptr(meta.block_table), _ptr(meta.rows), meta.width, _ptr_at(out, out_at),
+            self._code_of(q), _long(tokens), q_heads, kv_heads, dim, vdim, page_size, _long(num_pages), *tail[:-5], row_waves,
+            *tail[-5:]), "gated_attention")
 
     # ---- mixers with a state of fixed size -----------------------------------------------------------------------------
     def check_retention_sizes(self, heads: int, dim: int, vdim: int) -> None:

@@ -282,6 +282,72 @@ def test_attention_kernel_alone(hip, dtype, heads, kv_heads, dim, vdim, chunk, p
         assert error < limit, f"request {r}: {error:.2e}"
 
 
+SINGLES = [     # heads, kv heads, dim, vdim, page, maps, options
+    (4, 2, 32, 32, 16, 1, dict(softcap=9.0, chunk=48, sink="zero", gates=True)), (16, 4, 128, 128, 16, 1, dict(sink="learned")),
+    (8, 8, 64, 256, 32, 1, dict(window=700)), (6, 2, 64, 128, 16, 2, dict(window=33)), (20, 1, 128, 64, 48, 1, dict(chunk=300)),
+    (8, 2, 256, 128, 16, 1, dict(window=40, keep_first=20)), (36, 2, 32, 64, 16, 1, dict(bias=True, sink="zero")), (2, 1, 256, 256, 16, 1, dict())]
+
+
+@pytest.mark.parametrize("heads,kv_heads,dim,vdim,page,maps,options", SINGLES)
+def test_single_tokens_on_the_matrix_cores(hip, heads, kv_heads, dim, vdim, page, maps, options):
+    """Single tokens whose keys end at every edge of a step, of a wave's share and of a segment, and the same in the kernel that
+    takes a wave's tiles in turn: both against the double.  Weights are exact in float32 in all of them, so what is left is one
+    rounding of an output - two results on either side of a rounding's edge lie one unit in the last of eight bits apart, at
+    most 2^-7 of them - and float32 sums (1e-4).  Slots beyond a request's tokens
+    hold NaN; one key of weight zero has an infinite value, which nobody takes."""
+    from torch_kernels import TorchKernels
+    torch.manual_seed(dim + heads)
+    befores = [0, 1, 15, 16, 62, 63, 64, 255, 256, 257, 300, 511, 512, 1037]
+    counts = [1] * len(befores)
+    ctx = _ctx(befores, counts)
+    need = [(b + page) // page for b in befores]
+    order = torch.randperm(sum(need) + 2).tolist()
+    table = torch.full((len(befores), max(need)), -1, dtype=torch.int32)
+    k_pages = torch.full((sum(need) + 2, kv_heads, page, maps * dim), float("nan"))
+    v_pages = torch.full((sum(need) + 2, kv_heads, vdim, page), float("nan"))
+    for r, before in enumerate(befores):
+        for p in range(before + 1):
+            if p % page == 0:
+                table[r, p // page] = order.pop()
+            at = int(table[r, p // page])
+            k_pages[at, :, p % page], v_pages[at, :, :, p % page] = torch.randn(kv_heads, maps * dim), torch.randn(kv_heads, vdim)
+    vectors = heads * maps
+    q = torch.randn(len(befores), vectors * dim).bfloat16()
+    k_pages, v_pages = k_pages.bfloat16(), v_pages.bfloat16()
+    width = vectors * vdim + 12
+    gates = torch.randn(len(befores), vectors + 3).bfloat16() if options.get("gates") else None
+    sinks = torch.randn(vectors) * 3 if options.get("sink") == "learned" else None
+    bias = torch.rand(2, vectors) if options.get("bias") else None
+    meta = SimpleNamespace(block_table=table.to(DEVICE), rows=None, width=table.shape[1])
+
+    def through(kernels, device, v, c, m):
+        out = torch.zeros(len(befores), width, dtype=torch.bfloat16, device=device)
+        move = lambda t: t.to(device) if t is not None else None
+        kernels.gated_attention(move(q), move(k_pages), move(v), move(gates), 2, c, m, heads, kv_heads, dim, vdim, 1.7 * dim ** -0.5,
+                                options.get("softcap"), options.get("chunk"), options.get("window"), "sink" in options, out,
+                                out_at=4, out_scale=0.7, sink_logits=move(sinks), maps=maps,
+                                keep_first=options.get("keep_first", 0), distance_bias=move(bias))
+        return out.float().cpu()
+
+    host = SimpleNamespace(**{k: (v.cpu() if isinstance(v, torch.Tensor) else v) for k, v in vars(ctx).items()})
+    want = through(TorchKernels(), "cpu", v_pages, host, SimpleNamespace(block_table=table, rows=None, width=table.shape[1]))
+    got = through(hip, DEVICE, v_pages, ctx, meta)
+    portion = SimpleNamespace(**dict(vars(ctx), num_decode_seqs=0))          # (the same rows through the portions' kernel)
+    assert ((got - want).abs() <= want.abs() * 2.0 ** -7 + 1e-4).all(), (got - want).abs().max()
+    assert ((through(hip, DEVICE, v_pages, portion, meta) - want).abs() <= want.abs() * 2.0 ** -7 + 5e-3).all()
+    if options or maps > 1:
+        return
+    # the last request's key 700 points away from every query by so much that its weight is zero; its value is infinite
+    at, place = int(table[-1, 700 // page]), 700 % page
+    k_pages[at, :, place] = -q[-1].view(heads, dim).float().sum(0).bfloat16() * 1000
+    clean = through(hip, DEVICE, v_pages, ctx, meta)
+    v_pages[at, :, :, place] = float("inf")
+    assert torch.equal(through(hip, DEVICE, v_pages, ctx, meta)[:-1], clean[:-1])
+    last = through(hip, DEVICE, v_pages, ctx, meta)[-1]
+    assert torch.isfinite(last).all()
+    assert ((last - clean[-1]).abs() <= clean[-1].abs() * 2.0 ** -7 + 1e-4).all()
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("heads,dim,vdim,rot", [(2, 16, 12, 8), (1, 64, 32, 64), (3, 24, 40, 0), (2, 128, 128, 32), (1, 256, 256, 2)])
 def test_retention_kernel_alone(hip, dtype, heads, dim, vdim, rot):
