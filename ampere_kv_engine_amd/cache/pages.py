@@ -45,6 +45,28 @@ class PageAllocator:
         self._held[page] = False
         self._free.append(page)
 
+    def allocate_run(self, count: int) -> list[int]:
+        """`count` pages in the order in which `allocate` would hand them out, all or none."""
+        if count > len(self._free):
+            raise PagePoolExhausted("the page pool is exhausted")
+        if count <= 0:
+            return []
+        pages = self._free[:-count - 1:-1]
+        del self._free[-count:]
+        held = self._held
+        for page in pages:
+            held[page] = True
+        return pages
+
+    def free_run(self, pages: list[int]) -> None:
+        """`free` for every one of `pages`, in their order."""
+        held = self._held
+        for page in pages:
+            if not (0 <= page < self.num_pages) or not held[page]:
+                raise ValueError(f"page {page} is not allocated (double free or foreign id)")
+            held[page] = False
+            self._free.append(page)
+
     def is_held(self, page: int) -> bool:
         return self._held[page]
 
@@ -67,9 +89,18 @@ class BlockTable:
 
     def take_changes(self) -> list[tuple[int, int]]:
         """(index, page id or RELEASED) of every entry that was appended or given back since the last call."""
-        changes = [(index, int(self._mirror[index])) for index in self._changed]
+        index, pages = self.take_changed()
+        return list(zip(index.tolist(), pages.tolist()))
+
+    def take_changed(self) -> tuple[np.ndarray, np.ndarray]:
+        """The same as two arrays: the entries' indices and what they hold now."""
+        index = np.array(self._changed, dtype=np.int64)
         self._changed.clear()
-        return changes
+        return index, self._mirror[index]
+
+    @property
+    def has_changed(self) -> bool:
+        return bool(self._changed)
 
     @property
     def length(self) -> int:
@@ -126,11 +157,11 @@ class BlockTable:
             grown = np.empty(max(required, 2 * len(self._mirror)), dtype=np.int32)
             grown[:len(self._pages)] = self._mirror[:len(self._pages)]
             self._mirror = grown
-        for _ in range(additional):
-            page = self._allocator.allocate()
-            self._mirror[len(self._pages)] = page
-            self._changed.append(len(self._pages))
-            self._pages.append(page)
+        if additional:
+            held = len(self._pages)
+            self._pages += self._allocator.allocate_run(additional)
+            self._mirror[held:required] = self._pages[held:]
+            self._changed.extend(range(held, required))
         self._length = start + num_tokens
         return start
 
@@ -147,8 +178,7 @@ class BlockTable:
         return page, offset
 
     def release(self) -> None:
-        for page in self._pages[:self.kept_pages] + self._pages[max(self._first_live, self.kept_pages):]:
-            self._allocator.free(page)
+        self._allocator.free_run(self._pages[:self.kept_pages] + self._pages[max(self._first_live, self.kept_pages):])
         self._pages.clear()
         self._changed.clear()
         self._length = 0

@@ -170,11 +170,12 @@ class BatchBuilder:
         page = self.cache.page_size
         return len(self.cache.groups) * sum(2 * ((count + page - 1) // page + 1) for count in counts)
 
-    def build(self, entries: list[StepEntry], width_multiple: int = 1) -> tuple[StepContext, list[int]]:
+    def build(self, entries: list[StepEntry], width_multiple: int = 1, token_arrays=None) -> tuple[StepContext, list[int]]:
         """Returns the context and, for every entry in the caller's order, the offset of its first wanted
         row in the logits the step returns.  `ctx.table_pages` is the longest request's page count rounded up to
         `width_multiple` pages: a bound that sizes launches and is the same for all steps under it (what a recorded
-        graph needs)."""
+        graph needs).  `token_arrays`: the entries' tokens as arrays of integers, where the caller has them (None for an
+        entry of a single token)."""
         if not entries:
             raise ValueError("a step needs at least one entry")
         if len(entries) > self.max_seqs:
@@ -247,7 +248,8 @@ class BatchBuilder:
                 positions[row] = start
                 seq_of_token[row] = index
             else:
-                token_ids[row:row + count] = np.asarray(e.tokens, dtype=np.int64)
+                ids = token_arrays[order[index]] if token_arrays is not None else None
+                token_ids[row:row + count] = np.asarray(e.tokens, dtype=np.int64) if ids is None else ids
                 positions[row:row + count] = np.arange(start, start + count)
                 seq_of_token[row:row + count] = index
             for name, (view, _, width_of) in extra_spans.items():
@@ -259,21 +261,23 @@ class BatchBuilder:
             for g, (slot_map, _) in zip(self.cache.groups, group_spans):
                 table = e.seq.tables[g.index]
                 pages = table.page_array
-                if arrays is not None:      # what this step changed in the request's row of the device's table
-                    changes = table.take_changes()
-                    if len(changes) > 2 * ((count + page_size - 1) // page_size + 1):
+                if arrays is not None and table.has_changed:     # what this step changed in the request's row of the device's table
+                    at, held = table.take_changed()
+                    if len(at) > 2 * ((count + page_size - 1) // page_size + 1):
                         # (tokens were registered outside a step: the row goes to the device as a whole)
                         arrays.write_row(g.index, e.seq.slot, pages)
-                        changes = ()
-                    for entry, page in changes:
-                        patches[2 * changed] = arrays.table_offset(g.index, e.seq.slot, entry)
-                        patches[2 * changed + 1] = page
-                        changed += 1
+                    else:
+                        upto = changed + len(at)
+                        patches[2 * changed:2 * upto:2] = arrays.table_offset(g.index, e.seq.slot, 0) + at
+                        patches[2 * changed + 1:2 * upto:2] = held
+                        changed = upto
                 if count == 1:
                     slot_map[row] = int(pages[start // page_size]) * page_size + start % page_size
                 else:
-                    pos = np.arange(start, start + count)
-                    slot_map[row:row + count] = pages[pos // page_size].astype(np.int64) * page_size + pos % page_size
+                    # a run of slots per page, the first and the last cut to the tokens
+                    first, last = start // page_size, (start + count - 1) // page_size
+                    slots = pages[first:last + 1, None] * page_size + np.arange(page_size, dtype=np.int32)
+                    slot_map[row:row + count] = slots.reshape(-1)[start - first * page_size:][:count]
             row += count
         # wanted rows in the caller's order of entries and places, whatever the layout above
         want_cursor = 0

@@ -114,7 +114,7 @@ class Engine:
         `step` and spares a copy (the scheduler and `generate_tokens` sample from it at once)."""
         if not self.loaded:
             raise RuntimeError("the engine has no weights yet")
-        self._check_token_ids(entries)
+        token_arrays = self._check_token_ids(entries)
         reach = self.model.embedding.position_rows
         if reach is not None:
             for e in entries:
@@ -124,9 +124,9 @@ class Engine:
         if self._recordable:
             shape = self._recordable_shape(entries)
             if shape is not None:
-                logits = self._step_recorded(entries, shape)
+                logits = self._step_recorded(entries, shape, token_arrays)
                 return logits if borrow_logits else logits.clone()
-        ctx, _ = self.builder.build(entries)
+        ctx, _ = self.builder.build(entries, token_arrays=token_arrays)
         ctx.stream_buffer, ctx.spare_buffer = self.stream_buffer, self.spare_buffer
         self._last_step = ctx
         return self.model.forward(ctx, self.cache.layer_cache)
@@ -159,15 +159,17 @@ class Engine:
             self._chooser = SlotSampler(self.kernels, self.device, self.config.max_seqs)
         return self._chooser.choose_later(logits, ctx)
 
-    def _check_token_ids(self, entries: list[StepEntry]) -> None:
-        """Every token id must name a row of the embedding table; one comparison per entry, not one per token."""
+    def _check_token_ids(self, entries: list[StepEntry]) -> list:
+        """Every token id must name a row of the embedding table; one comparison per entry, not one per token.  Returns
+        the entries' tokens as arrays (None for single ones): a long prompt is turned into an array once a step."""
         vocab = self.spec.vocab_size
-        for e in entries:
+        arrays = [None] * len(entries)
+        for index, e in enumerate(entries):
             if len(e.tokens) == 1:
                 # (-1 alone: the token chosen last for the request, which its slot on the device holds)
                 bad = not 0 <= int(e.tokens[0]) < vocab and not (int(e.tokens[0]) == -1 and e.seq.length > 0)
             else:
-                ids = np.asarray(e.tokens)
+                ids = arrays[index] = np.asarray(e.tokens)
                 if ids.dtype.kind not in "iu":
                     raise ValueError(f"the token ids of request {e.seq.request_id!r} are not integers")
                 bad = ids.size and (int(ids.min()) < 0 or int(ids.max()) >= vocab)
@@ -175,6 +177,7 @@ class Engine:
                 token = next(t for t in e.tokens if not 0 <= int(t) < vocab)
                 raise ValueError(f"token id {token} of request {e.seq.request_id!r} is outside the vocabulary "
                                  f"of {vocab}")
+        return arrays
 
     # ---- steps as recorded graphs -----------------------------------------------------------------------------
     PORTION_BOUND = 2048          # recorded steps: the smallest bound on the length of a request that brings a portion
@@ -194,7 +197,7 @@ class Engine:
             return None
         return counts, wanted
 
-    def _step_recorded(self, entries: list[StepEntry], shape) -> torch.Tensor:
+    def _step_recorded(self, entries: list[StepEntry], shape, token_arrays) -> torch.Tensor:
         """A step launches the same kernels with the same arguments every time, as long as the requests bring the
         same numbers of tokens, as many rows are wanted and the width of the block tables stays: only the metadata in
         the step's device buffer differs.  A step of such a shape is run once as it is, then recorded into a HIP
@@ -203,7 +206,7 @@ class Engine:
         serves all lengths under it.  The logits are written to a buffer that all recordings share: the next
         recorded step overwrites them (`step` hands out a copy unless the caller asked to borrow the buffer)."""
         counts, wanted = shape
-        ctx, _ = self.builder.build(entries, width_multiple=self.config.graph_width_multiple)
+        ctx, _ = self.builder.build(entries, width_multiple=self.config.graph_width_multiple, token_arrays=token_arrays)
         ctx.stream_buffer, ctx.spare_buffer = self.stream_buffer, self.spare_buffer
         self._last_step = ctx
         width = ctx.table_pages        # the longest request's pages, rounded up: a bound the recording is made for
