@@ -121,6 +121,15 @@ int akv_gated_attention_tiles(const void* q, const void* k_pages, const void* v_
                               const float* sink_logits, int maps, int keep_first, const float* distance_bias,
                               hipStream_t stream);
 
+// The same for requests first_seq .. seqs - 1, keys and values shared by blocks of 64 (token, query vector) columns; keys and
+// values 32, 64 or 128 wide.  `tiles`: columns of 64 over all of these requests, each request's rounded up.
+int akv_gated_attention_shared(const void* q, const void* k_pages, const void* v_pages, const void* gates, long gate_stride,
+                               int gate_at, const int* q_start, const int* seq_lens, const int* block_table,
+                               const int* table_rows, int table_width, void* out, int first_seq, int seqs, int tiles, int q_heads,
+                               int kv_heads, int dim, int vdim, int page_size, long num_pages, float scale, float softcap,
+                               int chunk, int window, int sink, long out_stride, float out_scale, const float* sink_logits,
+                               int maps, int keep_first, const float* distance_bias, hipStream_t stream);
+
 // ---- mixers with a state of fixed size (recurrent_mixers.hip) ----------------------------------------------------------
 // projected [tokens, stride]: rows [q | k (heads x dim each) | v | g (heads x vdim each)].  q and k are rotated over their
 // first rot_dims dimensions (pairs i, i + rot_dims / 2; `table` [positions, rot_dims / 2, 2] holds cos and sin), k times

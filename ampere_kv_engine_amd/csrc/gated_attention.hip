@@ -1089,3 +1089,325 @@ int akv_gated_attention_singles(const void* q, const void* k_pages, const void* 
 }
 
 }
+
+namespace {
+
+// ---- prompt portions, keys and values shared through LDS ------------------------------------------------------------------
+// bfloat16, keys and values of 32, 64 or 128, where the portions make enough blocks to fill the device.  The tiles above
+// have every wave fetch its own keys and values: 2,000 tokens of 16 heads ask the L2 for a gigabyte, and a step of 16 keys
+// pays the softmax's bookkeeping for four scores a lane.  Here a block is 64 columns - consecutive (token, query vector)
+// pairs of one request whose vectors read one vector of one key head -, a wave 16 of them; a step is 32 keys at absolute
+// positions, fetched once by the block two steps ahead and filed in two LDS buffers in turn (one barrier a step): keys by rows of the
+// head's width, values by rows of 32 keys in the order of the second product's operand (a lane's eight are keys 4 g .. 4 g + 3
+// of the step's two sixteens, where the first product leaves their scores).  Rows are padded by 16 bytes, so that a 16-byte
+// read of sixteen rows meets no bank twice.  A wave passes over steps that none of its columns sees.  Scores, maxima,
+// weights and sums are float32 (base 2); a weight enters the second product as two bfloat16; the exponentials' reference
+// point trails the maximum by at most 2^8, so that sums are rescaled a few times a prompt and not once a step.
+// What bounds it: a step's chain of dependent instructions (products, maximum, exponentials, products: 1.2 us with one wave a
+// SIMD), as often as the longest block has steps; two blocks a unit fill each other's gaps.  2,000 tokens of 16 / 4 heads of
+// 128, us: 116 with the tiles above, 102 here with pages and keys asked for a step ahead, 85 two steps ahead, 77 with the
+// place in the page moved on by additions (a division a page and sixteen: 40 instructions of a step's 500).
+constexpr int kSharedColumns = 64;
+
+// The maximum over the four lanes c, c + 16, c + 32 and c + 48, in all four: lane swaps inside the vector unit.
+__device__ __forceinline__ float max_over_groups(float v) {
+  const auto halves = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = fmaxf(__uint_as_float(halves[0]), __uint_as_float(halves[1]));
+  const auto rows = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fmaxf(__uint_as_float(rows[0]), __uint_as_float(rows[1]));
+}
+constexpr float kTrail = 8.f;
+
+struct SharedArgs {
+  const bf16_t *q, *k_pages, *v_pages, *gates;
+  const int *q_start, *seq_lens, *block_table, *table_rows;
+  const float *sink_logits, *distance_bias;
+  bf16_t* out;
+  long gate_stride, num_pages, out_stride;
+  float scale, softcap, out_scale;
+  int first_seq, seqs, tiles, gate_at, table_width, q_heads, kv_heads, page_size, chunk, window, sink, maps, keep_first;
+};
+
+template <int DT, int VT, bool SHAPED>
+__global__ __launch_bounds__(256, 2) void gated_attention_shared_kernel(const SharedArgs a) {
+  constexpr int DIM = 32 * DT, VDIM = 16 * VT, kKeyRow = DIM + 8, kValueRow = 32 + 8;
+  constexpr int kKeyLoads = (32 * DIM / 8 + 255) / 256, kValueLoads = (VDIM * 4 + 255) / 256;     // 16 bytes a thread each
+  __shared__ __attribute__((aligned(16))) bf16_t filed_keys[2][32 * kKeyRow];
+  __shared__ __attribute__((aligned(16))) bf16_t filed_values[2][VDIM * kValueRow];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x & (kWave - 1);
+  const int col = lane & 15, grp = lane >> 4;
+  const int share = a.q_heads / a.kv_heads / a.maps, columns = a.kv_heads * a.maps;
+  const int kvh = blockIdx.x % columns / a.maps, map = blockIdx.x % a.maps;
+  // whose tile this is: numbered request by request; the last ones - those with the most keys before them - start first
+  int request = -1, tile = a.tiles - 1 - static_cast<int>(blockIdx.x) / columns;
+  for (int first = a.first_seq; first < a.seqs && request < 0; first += kWave) {
+    const int r = first + lane;
+    const int count = r < a.seqs ? ((a.q_start[r + 1] - a.q_start[r]) * share + kSharedColumns - 1) / kSharedColumns : 0;
+    int upto = count;
+#pragma unroll
+    for (int step = 1; step < kWave; step <<= 1) {
+      const int other = __shfl_up(upto, step, kWave);
+      if (lane >= step) upto += other;
+    }
+    const unsigned long long here = __ballot(tile < upto);
+    if (here != 0) {
+      const int at = __ffsll(here) - 1;
+      request = first + at;
+      tile -= __shfl(upto - count, at, kWave);
+    } else {
+      tile -= __shfl(upto, kWave - 1, kWave);
+    }
+  }
+  if (request < 0) return;
+  request = __builtin_amdgcn_readfirstlane(request);             // (the same in every lane: what follows is scalar)
+  tile = __builtin_amdgcn_readfirstlane(tile);
+  const int token0 = a.q_start[request], tokens = a.q_start[request + 1] - token0, history = a.seq_lens[request] - tokens;
+  const int rows = tokens * share, row0 = tile * kSharedColumns, row_end = min(row0 + kSharedColumns, rows);
+  const auto low_of = [&](int pos) {
+    int low = a.window > 0 ? max(0, pos - a.window + 1) : 0;
+    if (a.chunk > 0) low = max(low, pos / a.chunk * a.chunk);
+    return low;
+  };
+  const int my_row = min(row0 + wave * 16 + col, rows - 1);      // (columns beyond the request's repeat its last, unstored)
+  const int token = token0 + my_row / share, vector = (kvh * share + my_row % share) * a.maps + map;
+  const int pos = history + my_row / share, low = low_of(pos);
+  // what the block's and the wave's columns see: positions first .. last
+  const int block_low = low_of(history + row0 / share), block_last = history + (row_end - 1) / share;
+  const int wave_first = history + min(row0 + wave * 16, rows - 1) / share, wave_last = history + min(row0 + wave * 16 + 15, rows - 1) / share;
+  const int wave_low = low_of(wave_first), wave_low_last = low_of(wave_last);
+
+  uint4 q[DT];
+  const bf16_t* qp = a.q + (static_cast<long>(token) * a.q_heads + vector) * DIM + grp * 8;
+#pragma unroll
+  for (int d = 0; d < DT; ++d) q[d] = load_bf16x8(qp + d * 32);
+  constexpr float kLog2e = 1.4426950408889634f;
+  const float scale = SHAPED ? a.scale : a.scale * kLog2e;
+  const float cap = SHAPED ? a.softcap : 0.f, inverse_cap = SHAPED && a.softcap > 0.f ? 1.f / a.softcap : 0.f;
+  const float bias_size = SHAPED && a.distance_bias != nullptr ? a.distance_bias[vector] : 0.f;
+  const float bias_rate = SHAPED && a.distance_bias != nullptr ? a.distance_bias[a.q_heads + vector] : 0.f;
+  float m = !a.sink ? -INFINITY : a.sink_logits != nullptr ? a.sink_logits[vector] * kLog2e : 0.f;
+  float l = a.sink && grp == 0 ? 1.f : 0.f;                      // (a lane's own keys; added over the groups at the end)
+  float4_t o[VT];
+#pragma unroll
+  for (int v = 0; v < VT; ++v) o[v] = float4_t{0.f, 0.f, 0.f, 0.f};
+
+  // steps of 32 keys: those of the request's first `keep_first` that lie before the window's, then the window's
+  const int first_step = block_low >> 5, kept_steps = min((a.keep_first + 31) >> 5, first_step);
+  const int steps = kept_steps + (block_last >> 5) - first_step + 1;
+  const auto key_of = [&](int turn) { return (turn < kept_steps ? turn : first_step + turn - kept_steps) << 5; };
+  const int* table = a.block_table + static_cast<long>(a.table_rows != nullptr ? a.table_rows[request] : request) * a.table_width;
+  const auto known = [&](int page) -> bool { return (page >= 0) & (page < a.num_pages); };
+  // Where the step to fetch next lies: the table entry and the place in the page of each of its two sixteens (a page holds a
+  // multiple of sixteen).  It moves on with additions: a division a step and sixteen cost more than the step's products.
+  int entry[2], place[2], pages[2];
+  const int last_entry = block_last / a.page_size;
+  const auto stand_at = [&](int key) {
+    entry[0] = key / a.page_size;
+    place[0] = key - entry[0] * a.page_size;
+  };
+  const auto ask_pages = [&]() {
+    entry[1] = entry[0];
+    place[1] = place[0] + 16;
+    if (place[1] >= a.page_size) {
+      place[1] -= a.page_size;
+      ++entry[1];
+    }
+#pragma unroll
+    for (int half = 0; half < 2; ++half) pages[half] = table[min(entry[half], last_entry)];    // (beyond the last: the last)
+  };
+  // what a step's keys and values come through: two sets in turn, asked for two steps ahead; their pages three steps ahead
+  struct Ahead {
+    uint4 keys[kKeyLoads], values[kValueLoads];
+    bool there[2];
+  } even, odd;
+  // thread t fetches 16 bytes of key t / (DIM / 8) and, for values, keys 8 (t & 3) .. + 7 of dimension t / 4, and so on;
+  // then the pages of the step after are asked for
+  const auto fetch = [&](int turn, Ahead& to) {
+    const bf16_t* key_half[2];
+    const bf16_t* value_half[2];
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      to.there[half] = known(pages[half]);
+      const long head = (to.there[half] ? pages[half] : 0) * static_cast<long>(a.kv_heads) + kvh;
+      key_half[half] = a.k_pages + ((head * a.page_size + place[half]) * a.maps + map) * DIM;
+      value_half[half] = a.v_pages + head * VDIM * a.page_size + place[half];
+    }
+#pragma unroll
+    for (int i = 0; i < kKeyLoads; ++i) {
+      const int at = min(i * 256 + static_cast<int>(threadIdx.x), 32 * DIM / 8 - 1), key = at / (DIM / 8);
+      to.keys[i] = load_bf16x8((key < 16 ? key_half[0] : key_half[1]) + (key & 15) * a.maps * DIM + at % (DIM / 8) * 8);
+    }
+#pragma unroll
+    for (int i = 0; i < kValueLoads; ++i) {
+      const int at = min(i * 256 + static_cast<int>(threadIdx.x), VDIM * 4 - 1), eight = at & 3;
+      to.values[i] = load_bf16x8((eight < 2 ? value_half[0] : value_half[1]) + at / 4 * a.page_size + 8 * (eight & 1));
+    }
+    if (turn + 1 == kept_steps) {
+      stand_at(first_step << 5);
+    } else {
+      place[0] += 32;
+      while (place[0] >= a.page_size) {
+        place[0] -= a.page_size;
+        ++entry[0];
+      }
+    }
+    ask_pages();
+  };
+  stand_at(key_of(0));
+  ask_pages();
+  const auto work = [&](int turn, Ahead& from, bf16_t* keys, bf16_t* values) {
+    const int j0 = key_of(turn);
+    const bool here0 = from.there[0], here1 = from.there[1];
+#pragma unroll
+    for (int i = 0; i < kKeyLoads; ++i) {
+      const int at = i * 256 + threadIdx.x;
+      if (32 * DIM / 8 % 256 == 0 || at < 32 * DIM / 8)
+        *reinterpret_cast<uint4*>(keys + at / (DIM / 8) * kKeyRow + at % (DIM / 8) * 8) = from.keys[i];
+    }
+    const bool ragged = j0 + 31 > block_last || !here0 || !here1;
+#pragma unroll
+    for (int i = 0; i < kValueLoads; ++i) {
+      const int at = i * 256 + threadIdx.x, eight = at & 3;
+      uint4 v = from.values[i];
+      if (ragged) {        // slots that nobody has written, or of a page that is not the request's, hold anything: zeros
+        const int left = (eight < 2 ? here0 : here1) ? block_last - (j0 + 8 * eight) + 1 : 0;
+        uint32_t words[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int w = 0; w < 4; ++w) words[w] &= (2 * w < left ? 0xffffu : 0u) | (2 * w + 1 < left ? 0xffff0000u : 0u);
+        v = make_uint4(words[0], words[1], words[2], words[3]);
+      }
+      if (VDIM * 4 % 256 == 0 || at < VDIM * 4) {
+        // keys 8 eight .. + 3 are group 2 (eight & 1)'s of sixteen number eight / 2, the next four the group after's
+        bf16_t* to = values + at / 4 * kValueRow + (eight & 1) * 16 + (eight >> 1) * 4;
+        *reinterpret_cast<uint2*>(to) = make_uint2(v.x, v.y);
+        *reinterpret_cast<uint2*>(to + 8) = make_uint2(v.z, v.w);
+      }
+    }
+    __syncthreads();
+    fetch(turn + 2, from);
+    // (the same for the whole wave: none of its columns sees a key of the step)
+    if (j0 > wave_last || (j0 + 31 < wave_low && j0 >= a.keep_first)) return;
+    float4_t acc[2] = {float4_t{0.f, 0.f, 0.f, 0.f}, float4_t{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+    for (int d = 0; d < DT; ++d)
+#pragma unroll
+      for (int half = 0; half < 2; ++half)
+        acc[half] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+            __builtin_bit_cast(bf16x8_t, load_bf16x8(keys + (16 * half + col) * kKeyRow + d * 32 + grp * 8)),
+            __builtin_bit_cast(bf16x8_t, q[d]), acc[half], 0, 0, 0);
+    float s[8], top = -INFINITY;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      s[e] = acc[e >> 2][e & 3] * scale;
+      if constexpr (SHAPED) {
+        if (cap > 0.f) {      // tanh(x) = 1 - 2 / (exp(2 x) + 1), with the hardware's exponential and reciprocal
+          const float x = __expf(2.f * fabsf(s[e]) * inverse_cap);
+          s[e] = copysignf(cap * (1.f - 2.f * __frcp_rn(x + 1.f)), s[e]);
+        }
+        s[e] *= kLog2e;
+        if (a.distance_bias != nullptr) {        // (keys behind the query are masked below: their logarithm is taken of 1)
+          const int j = j0 + 16 * (e >> 2) + 4 * grp + (e & 3);
+          s[e] -= bias_size * __builtin_amdgcn_logf(fmaf(bias_rate, static_cast<float>(max(pos - j, 0)), 1.f));
+        }
+      }
+    }
+    if (j0 + 31 > wave_first || (j0 < wave_low_last && j0 + 31 >= a.keep_first) || !here0 || !here1) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const int j = j0 + 16 * (e >> 2) + 4 * grp + (e & 3);
+        const bool seen = ((j >= low) | (j < a.keep_first)) & (j <= pos) & (e < 4 ? here0 : here1);
+        s[e] = seen ? s[e] : -INFINITY;
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) top = fmaxf(top, s[e]);
+    top = max_over_groups(top);
+    if (__any(top > m + kTrail)) {
+      const float moved = fmaxf(m, top), shift = moved == -INFINITY ? 0.f : moved;
+      const float correction = __builtin_amdgcn_exp2f(m - shift);
+      l *= correction;
+#pragma unroll
+      for (int v = 0; v < VT; ++v)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[v][i] *= correction;
+      m = moved;
+    }
+    const float reference = m == -INFINITY ? 0.f : m;
+    uint32_t high[4], rest[4];
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const float p0 = __builtin_amdgcn_exp2f(s[2 * w] - reference), p1 = __builtin_amdgcn_exp2f(s[2 * w + 1] - reference);
+      l += p0 + p1;
+      high[w] = bf16_pair(p0, p1);
+      rest[w] = bf16_pair(p0 - __uint_as_float(high[w] << 16), p1 - __uint_as_float(high[w] & 0xffff0000u));
+    }
+    const bf16x8_t p_high = __builtin_bit_cast(bf16x8_t, make_uint4(high[0], high[1], high[2], high[3]));
+    const bf16x8_t p_rest = __builtin_bit_cast(bf16x8_t, make_uint4(rest[0], rest[1], rest[2], rest[3]));
+#pragma unroll
+    for (int v = 0; v < VT; ++v) {
+      const bf16x8_t operand = __builtin_bit_cast(bf16x8_t, load_bf16x8(values + (16 * v + col) * kValueRow + grp * 8));
+      o[v] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(operand, p_high, o[v], 0, 0, 0);
+      o[v] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(operand, p_rest, o[v], 0, 0, 0);
+    }
+  };
+  fetch(0, even);
+  fetch(1, odd);
+  for (int turn = 0; turn < steps; turn += 2) {
+    work(turn, even, filed_keys[0], filed_values[0]);
+    if (turn + 1 < steps) work(turn + 1, odd, filed_keys[1], filed_values[1]);
+  }
+  l += __shfl_xor(l, 16, kWave);
+  l += __shfl_xor(l, 32, kWave);
+  if (row0 + wave * 16 + col >= rows) return;
+  float gate = a.out_scale;
+  if (a.gates != nullptr) gate = a.out_scale / (1.f + expf(-to_float(a.gates[static_cast<long>(token) * a.gate_stride + a.gate_at + vector])));
+  const float factor = gate / l;
+  bf16_t* to = a.out + static_cast<long>(token) * a.out_stride + static_cast<long>(vector) * VDIM + grp * 4;
+#pragma unroll
+  for (int v = 0; v < VT; ++v) {
+    uint2 packed;
+    packed.x = bf16_pair(o[v][0] * factor, o[v][1] * factor);
+    packed.y = bf16_pair(o[v][2] * factor, o[v][3] * factor);
+    *reinterpret_cast<uint2*>(to + v * 16) = packed;
+  }
+}
+
+}  // namespace
+
+extern "C" int akv_gated_attention_shared(const void* q, const void* k_pages, const void* v_pages, const void* gates,
+                                          long gate_stride, int gate_at, const int* q_start, const int* seq_lens,
+                                          const int* block_table, const int* table_rows, int table_width, void* out, int first_seq,
+                                          int seqs, int tiles, int q_heads, int kv_heads, int dim, int vdim, int page_size,
+                                          long num_pages, float scale, float softcap, int chunk, int window, int sink,
+                                          long out_stride, float out_scale, const float* sink_logits, int maps, int keep_first,
+                                          const float* distance_bias, hipStream_t stream) {
+  if (seqs <= first_seq || tiles <= 0) return 0;
+  if (page_size % 16 != 0 || maps < 1 || kv_heads <= 0 || q_heads % (kv_heads * maps) != 0) return -2;
+  const long blocks = static_cast<long>(tiles) * kv_heads * maps;
+  if (blocks > 0x7fffffffL) return -2;
+  const SharedArgs a{static_cast<const bf16_t*>(q), static_cast<const bf16_t*>(k_pages), static_cast<const bf16_t*>(v_pages),
+                     static_cast<const bf16_t*>(gates), q_start, seq_lens, block_table, table_rows, sink_logits, distance_bias,
+                     static_cast<bf16_t*>(out), gate_stride, num_pages, out_stride, scale, softcap, out_scale, first_seq, seqs,
+                     tiles, gate_at, table_width, q_heads, kv_heads, page_size, chunk, window, sink, maps, keep_first};
+#define AKV_SHARED(DT, VT)                                                                                                  \
+  if (softcap > 0.f || distance_bias != nullptr)                                                                            \
+    gated_attention_shared_kernel<DT, VT, true><<<static_cast<unsigned>(blocks), 256, 0, stream>>>(a);                      \
+  else                                                                                                                      \
+    gated_attention_shared_kernel<DT, VT, false><<<static_cast<unsigned>(blocks), 256, 0, stream>>>(a)
+#define AKV_SHARED_V(DT)                  \
+  switch (vdim) {                         \
+    case 32: AKV_SHARED(DT, 2); break;    \
+    case 64: AKV_SHARED(DT, 4); break;    \
+    case 128: AKV_SHARED(DT, 8); break;   \
+    default: return -2;                   \
+  }
+  switch (dim) {
+    case 32: AKV_SHARED_V(1); break;
+    case 64: AKV_SHARED_V(2); break;
+    case 128: AKV_SHARED_V(4); break;
+    default: return -2;
+  }
+#undef AKV_SHARED_V
+#undef AKV_SHARED
+  return AKV_LAUNCH_STATUS();
+}

@@ -45,7 +45,7 @@ class PartsKernels:
                          "akv_rotate_queries", "akv_heads_linear", "akv_latent_attend", "akv_latent_attend_mfma", "akv_conv_silu",
                          "akv_conv_state_update", "akv_selective_scan", "akv_route", "akv_gate_relu_squared",
                          "akv_parts_slot_layout", "akv_conv_taps", "akv_scaled_sum", "akv_unit_norm_write",
-                         "akv_gated_attention_rows", "akv_gated_attention_tiles", "akv_gated_attention_singles", "akv_retention", "akv_retention_chunked", "akv_gated_linear_scan", "akv_route_chosen",
+                         "akv_gated_attention_rows", "akv_gated_attention_tiles", "akv_gated_attention_singles", "akv_gated_attention_shared", "akv_retention", "akv_retention_chunked", "akv_gated_linear_scan", "akv_route_chosen",
                          "akv_gate_pair_mul", "akv_route_corrected", "akv_add_weighted_rows", "akv_embed_normed", "akv_gated_activation", "akv_difference_norm_gate",
                          "akv_delta_rule", "akv_embed_rows", "akv_norm_gate_rows", "akv_gate_activation", "akv_softcap",
                          "akv_token_shift", "akv_tanh_rows", "akv_time_mixing", "akv_matrix_memory"):
@@ -793,6 +793,25 @@ class PartsKernels:
     # ---- attention with unit-normed queries and keys, a softcap, chunks, a sink and a gate per head ----------------------
     MAX_VALUE_DIM = 256
     MATRIX_CORE_HEAD_DIMS = (32, 64, 128, 256)      # widths of keys and of values that the matrix-core kernels are built for
+    shared_attention_blocks = None      # prompt portions of this many blocks share their keys through LDS; None: by the rule below
+
+    def _shares_attention_keys(self, blocks: int, ctx, first: int) -> bool:
+        """Whether prompt portions of `blocks` blocks of 64 (token, query vector) columns go to the kernel that shares keys
+        through LDS.  Each of its blocks walks all of its columns' keys alone, where a tile of the other kernel has four waves
+        for them; it pays where there are more blocks than compute units, or as many and mostly history to read.  Measured, us,
+        shared / tiles: 16 query and 4 key heads of 128, 2,048 tokens (512 blocks) 77 / 116 inside a step, 500 x 4 (512) 29 / 46,
+        1,024 after 6,000 (256) 242 / 403, 512 after 6,000 (128) 223 / 199; 32 / 8 heads, 2,048 tokens (1,024) 89 / 227, 800 (400)
+        34 / 50, 512 after 2,048 (256) 93 / 155, 512 (256) 23 / 25, 400 (200) 20 / 19; 16 heads of 64 of their own, 1,024 (256)
+        31 / 28, 2,048 (512) 59 / 81; two maps of 64 over a window of 1,024, 512 (256) 22 / 20, 800 (400) 31 / 41."""
+        if self.shared_attention_blocks is not None:
+            return blocks >= self.shared_attention_blocks
+        units = self.compute_units
+        if 4 * blocks >= 5 * units:
+            return True
+        starts = ctx.host_q_start
+        longest_portion = max((starts[r + 1] - starts[r] for r in range(first, ctx.num_seqs)), default=0)
+        return blocks >= units and max(ctx.host_seq_lens[first:], default=0) >= 5 * longest_portion
+
     SEGMENT_STEPS = 16      # steps of 16 keys in a segment of a single token's keys (`kSegmentSteps` of the kernel)
 
     def check_gated_attention_sizes(self, q_heads: int, kv_heads: int, dim: int, vdim: int, page_size: int) -> None:
@@ -933,6 +952,15 @@ class PartsKernels:
                     _ptr(ctx.positions), _ptr(meta.block_table), _ptr(meta.rows), meta.width, _ptr_at(out, out_at), _ptr(partial),
                     segments, singles, q_heads, kv_heads, dim, vdim, page_size, _long(num_pages), *tail),
                     "gated_attention of single tokens")
+            starts, columns = ctx.host_q_start, q_heads // kv_heads // maps
+            tiles = sum(((starts[r + 1] - starts[r]) * columns + 63) // 64 for r in range(singles, ctx.num_seqs))
+            if dim <= 128 and vdim <= 128 and self._shares_attention_keys(tiles * kv_heads * maps, ctx, singles):
+                self._dense(ctx.seq_lens, "seq_lens", torch.int32, (ctx.num_seqs,))
+                self._check(self._parts().akv_gated_attention_shared(
+                    _ptr(q), _ptr(k_pages), _ptr(v_pages), _ptr(gates), _long(gate_stride), gate_at, _ptr(ctx.q_start),
+                    _ptr(ctx.seq_lens), _ptr(meta.block_table), _ptr(meta.rows), meta.width, _ptr_at(out, out_at), singles, ctx.num_seqs,
+                    tiles, q_heads, kv_heads, dim, vdim, page_size, _long(num_pages), *tail), "gated_attention of shared keys")
+                return
             self._check(self._parts().akv_gated_attention_tiles(
                 _ptr(q), _ptr(k_pages), _ptr(v_pages), _ptr(gates), _long(gate_stride), gate_at, _ptr(ctx.seq_of_token),
                 _ptr(ctx.q_start), _ptr(ctx.positions), _ptr(meta.block_table), _ptr(meta.rows), meta.width,

@@ -348,6 +348,56 @@ def test_single_tokens_on_the_matrix_cores(hip, heads, kv_heads, dim, vdim, page
     assert ((last - clean[-1]).abs() <= clean[-1].abs() * 2.0 ** -7 + 1e-4).all()
 
 
+@pytest.mark.parametrize("heads,kv_heads,dim,vdim,page,maps,options", [c for c in SINGLES if c[2] <= 128 and c[3] <= 128] + [
+    (12, 4, 128, 128, 16, 1, dict(sink="learned", gates=True)), (3, 3, 64, 64, 64, 1, dict(window=70, keep_first=40)),
+    (4, 2, 64, 128, 16, 2, dict(window=50, sink="zero"))])
+def test_portions_that_share_their_keys_through_lds(hip, monkeypatch, heads, kv_heads, dim, vdim, page, maps, options):
+    """Portions whose first and last columns fall inside tiles of 64, with and without history, beside single tokens - in the
+    kernel that shares keys through LDS, whatever the number of blocks, and in the one in which every wave fetches its own: both
+    against the double.  A weight is two bfloat16 (2^-17 of it is left out: times values of up to 5 sigma, below 1e-4 of the
+    largest), an output is rounded once (an ulp apart at a rounding's edge: 2^-7 of it), exponentials are the hardware's (a
+    few 2^-23 of scores of up to 60 in base 2): 2^-7 |out| + 2e-3.  Slots beyond a request's tokens hold NaN."""
+    from torch_kernels import TorchKernels
+    torch.manual_seed(dim + heads + vdim)
+    befores, counts = [7, 0, 33, 300, 16, 0], [1, 1, 3, 90, 64, 331]
+    ctx = _ctx(befores, counts)
+    ctx.seq_lens = torch.tensor(ctx.host_seq_lens, dtype=torch.int32, device=DEVICE)
+    need = [(n + page - 1) // page for n in ctx.host_seq_lens]
+    order = torch.randperm(sum(need) + 2).tolist()
+    table = torch.full((len(befores), max(need)), -1, dtype=torch.int32)
+    k_pages = torch.full((sum(need) + 2, kv_heads, page, maps * dim), float("nan"))
+    v_pages = torch.full((sum(need) + 2, kv_heads, vdim, page), float("nan"))
+    for r, length in enumerate(ctx.host_seq_lens):
+        for p in range(length):
+            if p % page == 0:
+                table[r, p // page] = order.pop()
+            at = int(table[r, p // page])
+            k_pages[at, :, p % page], v_pages[at, :, :, p % page] = torch.randn(kv_heads, maps * dim), torch.randn(kv_heads, vdim)
+    vectors, tokens = heads * maps, ctx.num_tokens
+    q = torch.randn(tokens, vectors * dim).bfloat16()
+    k_pages, v_pages = k_pages.bfloat16(), v_pages.bfloat16()
+    gates = torch.randn(tokens, vectors + 3).bfloat16() if options.get("gates") else None
+    sinks = torch.randn(vectors) * 3 if options.get("sink") == "learned" else None
+    bias = torch.rand(2, vectors) if options.get("bias") else None
+
+    def through(kernels, device, c):
+        out = torch.zeros(tokens, vectors * vdim + 12, dtype=torch.bfloat16, device=device)
+        move = lambda t: t.to(device) if t is not None else None
+        meta = SimpleNamespace(block_table=move(table), rows=None, width=table.shape[1])
+        kernels.gated_attention(move(q), move(k_pages), move(v_pages), move(gates), 2, c, meta, heads, kv_heads, dim, vdim, 1.7 * dim ** -0.5,
+                                options.get("softcap"), options.get("chunk"), options.get("window"), "sink" in options, out,
+                                out_at=4, out_scale=0.7, sink_logits=move(sinks), maps=maps,
+                                keep_first=options.get("keep_first", 0), distance_bias=move(bias))
+        return out.float().cpu()
+
+    host = SimpleNamespace(**{k: (v.cpu() if isinstance(v, torch.Tensor) else v) for k, v in vars(ctx).items()})
+    want = through(TorchKernels(), "cpu", host)
+    for blocks in (1, 1 << 30):
+        monkeypatch.setattr(hip, "shared_attention_blocks", blocks, raising=False)
+        got = through(hip, DEVICE, ctx)
+        assert ((got - want).abs() <= want.abs() * 2.0 ** -7 + 2e-3).all(), (blocks, (got - want).abs().max())
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("heads,dim,vdim,rot", [(2, 16, 12, 8), (1, 64, 32, 64), (3, 24, 40, 0), (2, 128, 128, 32), (1, 256, 256, 2)])
 def test_retention_kernel_alone(hip, dtype, heads, dim, vdim, rot):
