@@ -138,6 +138,12 @@ class StepContext:
     slot_words: torch.Tensor | None = None      # int32 [slots, SLOT_WORDS]: its first part
     extra: dict = field(default_factory=dict)   # name -> int32 [tokens, width]: what the entries brought per token
 
+    @property
+    def wants_every_row(self) -> bool:
+        """Every request brings one token and wants its logits: the wanted rows are all rows, in their order (single tokens
+        keep the caller's order)."""
+        return self.logit_rows.shape[0] == self.num_tokens == self.num_decode_seqs and self.most_wanted == 1
+
 
 class BatchBuilder:
     """Turns entries into a `StepContext`: registers the new tokens with the cache manager (which hands out

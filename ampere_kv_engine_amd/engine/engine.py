@@ -57,7 +57,7 @@ class Engine:
                                         device=self.device)
         self.loaded = False
         self._chooser = None
-        self._graphs: dict[tuple, object] = {}               # (tokens per request, wanted rows, table width, portions' bound) -> graph
+        self._graphs: dict[tuple, object] = {}               # (tokens per request, wanted rows, table width, portions' bound, whether every row is wanted) -> graph
         self._graph_logits = None                            # [max_seqs, vocab] float32, where recorded steps write
         self._recordable = (engine_config.decode_graphs and self.device.type == "cuda" and all(
             part.graph_safe for block in self.model.blocks for part in (block, block.mixer, block.feed_forward)))
@@ -222,7 +222,7 @@ class Engine:
             while portion_bound < max(ctx.host_seq_lens[decodes:]):
                 portion_bound *= 2
             portion_bound = min(portion_bound, bound)
-        key = (counts, wanted, width, portion_bound)
+        key = (counts, wanted, width, portion_bound, ctx.wants_every_row)     # (the last: such a step picks no rows)
         ctx.max_seq_len = bound
         ctx.host_seq_lens = [bound] * decodes + [portion_bound] * (ctx.num_seqs - decodes)
         if self._graph_logits is None:  # one buffer for every recording: a recorded step's logits are its first rows

@@ -124,19 +124,30 @@ class Model:
         wanted = ctx.logit_rows.shape[0]
         if wanted == 0:
             return None
+        ctx.arena = arenas[len(self.spec.run_order) & 1]
+        ctx.arena.reset()
+        if ctx.wants_every_row:
+            # nothing is picked, and the last branch is added inside the final norm's kernel (a decode step: one launch
+            # instead of two or three)
+            normed = ctx.arena.take((wanted, hidden), rt.dtype)
+            if isinstance(pending, Unsettled):
+                self.final_norm.after(stream, pending, normed)
+            else:
+                self.final_norm.forward_residual(stream, pending, normed)
+            return self._logits(normed, wanted, logits_out)
         if isinstance(pending, Unsettled):     # the last branch is normed and added before the rows are picked
             pending.settle(stream)
             pending = None
-        ctx.arena = arenas[len(self.spec.run_order) & 1]
-        ctx.arena.reset()
         picked = ctx.arena.take((wanted, hidden), torch.float32)
         k.gather_rows(stream, pending, ctx.logit_rows, picked)
         normed = ctx.arena.take((wanted, hidden), rt.dtype)
         self.final_norm.forward_residual(picked, None, normed)
-        if logits_out is None:
-            logits_out = torch.empty((wanted, self.spec.vocab_size), dtype=torch.float32, device=rt.device)
-        return self.head.forward(normed, logits_out)
+        return self._logits(normed, wanted, logits_out)
 
+    def _logits(self, normed, wanted: int, logits_out):
+        if logits_out is None:
+            logits_out = torch.empty((wanted, self.spec.vocab_size), dtype=torch.float32, device=self.rt.device)
+        return self.head.forward(normed, logits_out)
 
     def _with_vector(self, pending, vector, ctx):
         """`pending` with `vector` still to be added to every row of the residual sum after it: a branch that is added

@@ -325,3 +325,27 @@ def test_two_fresh_processes_give_the_same_bits_in_bfloat16(case, tmp_path):
     assert names == sorted(os.listdir(outs[1])) and len(names) == len(schedule)
     for name in names:
         assert (outs[0] / name).read_bytes() == (outs[1] / name).read_bytes(), f"{name} differs between the two runs"
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_recorded_steps_that_want_every_row_and_steps_that_pick_rows(case, dtype):
+    """Two requests that bring one token each and want both logits - nothing is picked, the last branch meets the final norm in its
+    kernel - in turn with steps of the same numbers of tokens and wanted rows in which one request wants its place twice
+    and the other nothing, each kind run as it is, recorded and replayed: the rows of an engine that records nothing."""
+    from ampere_kv_engine_amd.engine import StepEntry
+    ids = case["requests"][sorted(case["requests"])[0]] if "requests" in case else list(range(3, 60))
+    ids = [int(t) for t in ids][:40]
+    got = {}
+    for graphs in (True, False):
+        engine = cases.make_engine(case, dtype, "cuda:0", decode_graphs=graphs)
+        seqs = [engine.open("a"), engine.open("b")]
+        engine.step([StepEntry(seqs[0], ids[:5], []), StepEntry(seqs[1], ids[3:10], [])])
+        got[graphs] = []
+        for step in range(12):
+            places = [[0], [0]] if step % 2 == 0 else ([[0, 0], []] if step % 4 == 1 else [[], [0, 0]])
+            entries = [StepEntry(seq, [ids[10 + step]], want) for seq, want in zip(seqs, places)]
+            got[graphs].append(engine.step(entries[::-1] if step % 3 == 2 else entries).cpu())
+        if graphs:
+            assert sum(graph is not None for graph in engine._graphs.values()) == 2
+    for step, (recorded, eager) in enumerate(zip(got[True], got[False])):
+        assert torch.equal(recorded, eager), step
