@@ -104,7 +104,7 @@ __device__ __forceinline__ void store_f32(float* __restrict__ y, long row, int o
     if (out + j < outs) at[j] = sums[j];
 }
 
-// Up to 64 rows: the matrix is read once and its reads are what the product waits for.  A block owns 16 outputs and all of
+// Up to 32 rows: the matrix is read once and its reads are what the product waits for.  A block owns 16 outputs and all of
 // k; its waves take a segment each (a second round where k has more than 16), with the whole segment's loads in flight - 8 KB
 // a wave, 128 KB a block -, and leave their sums in LDS, where the first waves add them in order.  Rows lie in cache and
 // are read by every wave in operand order, without LDS: NT tiles of 16 rows.
@@ -120,7 +120,6 @@ __global__ __launch_bounds__(1024) void linear_f32_few_kernel(const float* __res
   const float* xp[NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t) xp[t] = x + static_cast<long>(min(16 * t + r, rows - 1)) * k + 4 * g;
-  constexpr int kGroup = NT <= 2 ? 8 : 4;    // blocks of 16 k whose rows are asked for together (registers)
   const floats4 zero = {0.f, 0.f, 0.f, 0.f};
   floats4 total = zero;
   for (int first = 0; first < segments; first += waves) {
@@ -135,19 +134,16 @@ __global__ __launch_bounds__(1024) void linear_f32_few_kernel(const float* __res
 #pragma unroll
         for (int b = 0; b < kSegmentBlocks; ++b) a[b] = *reinterpret_cast<const floats4*>(wp + k0 + 16 * b);
         __builtin_amdgcn_sched_barrier(0);                 // (else the loads are moved down to where they are used)
+        floats4 v[kSegmentBlocks][NT];
 #pragma unroll
-        for (int b0 = 0; b0 < kSegmentBlocks; b0 += kGroup) {
-          floats4 v[kGroup][NT];
+        for (int b = 0; b < kSegmentBlocks; ++b)
 #pragma unroll
-          for (int b = 0; b < kGroup; ++b)
+          for (int t = 0; t < NT; ++t) v[b][t] = *reinterpret_cast<const floats4*>(xp[t] + k0 + 16 * b);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int t = 0; t < NT; ++t) v[b][t] = *reinterpret_cast<const floats4*>(xp[t] + k0 + 16 * (b0 + b));
-          __builtin_amdgcn_sched_barrier(0);
+        for (int b = 0; b < kSegmentBlocks; ++b)
 #pragma unroll
-          for (int b = 0; b < kGroup; ++b)
-#pragma unroll
-            for (int t = 0; t < NT; ++t) sums[t] = mfma4(a[b0 + b], v[b][t], sums[t]);
-        }
+          for (int t = 0; t < NT; ++t) sums[t] = mfma4(a[b], v[b][t], sums[t]);
       } else {
         for (int b = 0; k0 + 16 * b < k; ++b) {
           const int at = k0 + 16 * b;
@@ -175,9 +171,13 @@ __global__ __launch_bounds__(1024) void linear_f32_few_kernel(const float* __res
 }
 
 // More rows: tiles of 32 TM outputs by 32 TN rows, four waves of TM x TN tiles of 16 each, operands through two LDS buffers
-// of 32 k (row stride 36 floats: 16-byte reads of eight rows meet no bank twice), the next 32 k on their way in registers.
-// Bound by the matrix cores: 8 TM TN instructions of 32 cycles a step and wave for 2 (TM + TN) reads of 1 KB.
-template <int TM, int TN>
+// of 32 k (row stride 36 floats: 16-byte reads of eight rows meet no bank twice), the next AHEAD steps of 32 k on their way in
+// registers.  Bound by the matrix cores where tiles fill the chip (8 TM TN instructions of 32 cycles a step and wave for
+// 2 (TM + TN) reads of 1 KB), and by the time a read takes where a unit holds one or two blocks, which is longer than a step:
+// 2048 outputs, k 2048 with 128 rows take 36.5 / 22.0 / 20.1 us with 1 / 2 / 4 steps on their way, k 6144 136 / 73 / 54, and
+// with 999 rows (tiles of 64 x 64) 85.5 / 85.1 / 83.9 and 251 / 244 / 242; 2048 rows of 12288 x 2048 949 / 916 / 918 (113
+// TFLOP/s).  Steps are a multiple of AHEAD, so that no register is copied at a loop's end: steps beyond k add zeros.
+template <int TM, int TN, int AHEAD>
 __global__ __launch_bounds__(256) void linear_f32_wide_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                               float* __restrict__ y, int rows, int outs, int k,
                                                               const float* __restrict__ bias, bool wide_stores) {
@@ -195,61 +195,68 @@ __global__ __launch_bounds__(256) void linear_f32_wide_kernel(const float* __res
 #pragma unroll
   for (int i = 0; i < TN; ++i) xp[i] = x + static_cast<long>(min(row0 + file_row + 32 * i, rows - 1)) * k;
   const floats4 zero = {0.f, 0.f, 0.f, 0.f};
-  floats4 sums[TM][TN], total[TM][TN], next_w[TM], next_x[TN];
+  floats4 sums[TM][TN], total[TM][TN], next_w[AHEAD][TM], next_x[AHEAD][TN];
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
     for (int j = 0; j < TN; ++j) sums[i][j] = total[i][j] = zero;
-  auto fetch = [&](int k0) {
+  auto fetch = [&](int slot, int k0) {
     const int at = min(k0 + file_k, k - 4);
 #pragma unroll
-    for (int i = 0; i < TM; ++i) next_w[i] = *reinterpret_cast<const floats4*>(wp[i] + at);
+    for (int i = 0; i < TM; ++i) next_w[slot][i] = *reinterpret_cast<const floats4*>(wp[i] + at);
 #pragma unroll
-    for (int i = 0; i < TN; ++i) next_x[i] = *reinterpret_cast<const floats4*>(xp[i] + at);
+    for (int i = 0; i < TN; ++i) next_x[slot][i] = *reinterpret_cast<const floats4*>(xp[i] + at);
   };
-  auto file = [&](int buffer, int k0) {
+  auto file = [&](int slot, int buffer, int k0) {
     const bool inside = k0 + file_k < k;
 #pragma unroll
     for (int i = 0; i < TM; ++i)
-      *reinterpret_cast<floats4*>(&ws[buffer][(file_row + 32 * i) * kStride + file_k]) = inside ? next_w[i] : zero;
+      *reinterpret_cast<floats4*>(&ws[buffer][(file_row + 32 * i) * kStride + file_k]) = inside ? next_w[slot][i] : zero;
 #pragma unroll
     for (int i = 0; i < TN; ++i)
-      *reinterpret_cast<floats4*>(&xs[buffer][(file_row + 32 * i) * kStride + file_k]) = inside ? next_x[i] : zero;
+      *reinterpret_cast<floats4*>(&xs[buffer][(file_row + 32 * i) * kStride + file_k]) = inside ? next_x[slot][i] : zero;
   };
   const int w_at = ((wave >> 1) * 16 * TM + r) * kStride + 4 * g, x_at = ((wave & 1) * 16 * TN + r) * kStride + 4 * g;
-  const int steps = (k + kDeep - 1) / kDeep;
-  fetch(0);
-  file(0, 0);
+  const int steps = (k + AHEAD * kDeep - 1) / (AHEAD * kDeep) * AHEAD;
+  fetch(0, 0);
+#pragma unroll
+  for (int i = 1; i < AHEAD; ++i) fetch(i, i * kDeep);
+  file(0, 0, 0);
   __syncthreads();
-  for (int step = 0; step < steps; ++step) {
-    const int buffer = step & 1;
-    if (step + 1 < steps) fetch((step + 1) * kDeep);
+  for (int first = 0; first < steps; first += AHEAD) {
 #pragma unroll
-    for (int b = 0; b < 2; ++b) {
-      floats4 a[TM], v[TN];
+    for (int turn = 0; turn < AHEAD; ++turn) {
+      const int step = first + turn;
+      const int buffer = step & 1;
+      fetch(turn, (step + AHEAD) * kDeep);                 // (beyond k the last elements once more; they are filed as zeros)
+      __builtin_amdgcn_sched_barrier(0);                   // (else the loads are moved down to where they are filed)
 #pragma unroll
-      for (int i = 0; i < TM; ++i) a[i] = *reinterpret_cast<const floats4*>(&ws[buffer][w_at + 16 * i * kStride + 16 * b]);
+      for (int b = 0; b < 2; ++b) {
+        floats4 a[TM], v[TN];
 #pragma unroll
-      for (int j = 0; j < TN; ++j) v[j] = *reinterpret_cast<const floats4*>(&xs[buffer][x_at + 16 * j * kStride + 16 * b]);
+        for (int i = 0; i < TM; ++i) a[i] = *reinterpret_cast<const floats4*>(&ws[buffer][w_at + 16 * i * kStride + 16 * b]);
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
+        for (int j = 0; j < TN; ++j) v[j] = *reinterpret_cast<const floats4*>(&xs[buffer][x_at + 16 * j * kStride + 16 * b]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+              sums[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i][e], v[j][e], sums[i][j], 0, 0, 0);
+      }
+      if ((step & 3) == 3 || step + 1 == steps) {          // the end of a segment of 128
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
-          for (int j = 0; j < TN; ++j)
-            sums[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i][e], v[j][e], sums[i][j], 0, 0, 0);
+          for (int j = 0; j < TN; ++j) {
+            total[i][j] += sums[i][j];
+            sums[i][j] = zero;
+          }
+      }
+      file((turn + 1) % AHEAD, buffer ^ 1, (step + 1) * kDeep);   // (read last before the barrier of the step before)
+      __syncthreads();
     }
-    if ((step & 3) == 3 || step + 1 == steps) {            // the end of a segment of 128
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) {
-          total[i][j] += sums[i][j];
-          sums[i][j] = zero;
-        }
-    }
-    if (step + 1 < steps) file(buffer ^ 1, (step + 1) * kDeep);   // (read last before the barrier of the step before)
-    __syncthreads();
   }
 #pragma unroll
   for (int j = 0; j < TN; ++j) {
@@ -266,7 +273,7 @@ int launch_f32_few(const float* x, const float* w, float* y, int rows, int outs,
                    hipStream_t stream) {
   const int segments = (k + kSegment - 1) / kSegment, rounds = (segments + 15) / 16;
   const int waves = max((segments + rounds - 1) / rounds, NT);
-  const size_t lds = static_cast<size_t>(waves) * NT * 64 * sizeof(floats4);     // 64 KB at most
+  const size_t lds = static_cast<size_t>(waves) * NT * 64 * sizeof(floats4);     // 32 KB at most
   linear_f32_few_kernel<NT><<<(outs + 15) / 16, waves * 64, lds, stream>>>(x, w, y, rows, outs, k, segments, bias, wide_stores);
   return AKV_LAUNCH_STATUS();
 }
@@ -275,34 +282,36 @@ template <int TM, int TN>
 int launch_f32_wide(const float* x, const float* w, float* y, int rows, int outs, int k, const float* bias, bool wide_stores,
                     hipStream_t stream) {
   dim3 grid((outs + 32 * TM - 1) / (32 * TM), (rows + 32 * TN - 1) / (32 * TN));
-  linear_f32_wide_kernel<TM, TN><<<grid, 256, 0, stream>>>(x, w, y, rows, outs, k, bias, wide_stores);
+  linear_f32_wide_kernel<TM, TN, TM * TN == 4 ? 2 : 4><<<grid, 256, 0, stream>>>(x, w, y, rows, outs, k, bias, wide_stores);
   return AKV_LAUNCH_STATUS();
 }
 
 // float32 operands whose rows are 16-byte aligned.  Which kernel takes a product is a matter of time alone (the bits are the
 // same).  Measured, us, on weights that no cache holds (outs x k = 2048 x 2048 / 6144 x 2048 / 4096 x 12288 / 32768 x 2048;
-// tiles of 64 x 64, 32 x 64 and 32 x 32 outputs x rows):
-//     17 rows: few 12.5 / 25 / 74 / 97    64 x 64 58 / 59 / 340 / 99    32 x 32 36 / 46 / 273 / 71
-//     64 rows: few 23 / 46 / 137 / 174    64 x 64 58 / 59 / 340 / 103   32 x 32 37 / 50 / 271 / 112
-//    200 rows:                            64 x 64 59 / 97 / 339 / 321   32 x 64 40 / 81 / 320 / 360   32 x 32 38 / 88 / 370 / 379
-//    300 rows:                            64 x 64 60 / 97 / 519 / 402   32 x 64 56 / 102 / 418 / 446  32 x 32 49 / 113 / 458 / 542
-//    999 rows:                            64 x 64 99 / 253 / 948 / 1244 32 x 64 103 / 280 / 1027 / 1381  (111 TFLOP/s at best;
-// the vector kernel above: 511 us on average over 2048 x 2048 and 2048 x 3072).  So: few rows stay with the kernel that reads
-// the matrix once unless tiles alone give every unit two blocks; otherwise the largest tile that still gives the units about
-// two blocks each (tiles of 128 are slower everywhere: the matrix cores wait for nothing that larger tiles would spare).
+// tiles of outputs x rows):
+//     16 rows: few 9.8 / 20 / 59 / 74     32 x 32 19 / 20 / 102 / 90
+//     17 rows: few 12.4 / 26 / 73 / 86    32 x 32 19 / 20 / 101 / 87   (64 x 64 at 32768)
+//     64 rows: few 22 / 45 / 129 / -      32 x 32 20 / 28 / 101 / 114  32 x 64 30 / 30 / 160 / 92    64 x 64 48 / 48 / 273 / 92
+//    300 rows:                            32 x 32 39 / 90 / 338 / 498  32 x 64 47 / 84 / 362 / 409   64 x 64 48 / 84 / 478 / 390
+//    700 rows:                            32 x 32 68 / 184 / 708 / 1046  32 x 64 64 / 178 / 709 / 892  64 x 64 82 / 196 / 698 / 849
+//    999 rows:                            32 x 32 89 / 264 / 1025 / 1496 32 x 64 86 / 244 / 932 / 1291 64 x 64 85 / 237 / 920 / 1224
+// (110 TFLOP/s at best; the vector kernel above: 511 us on average over 999 rows of 2048 x 2048 and 2048 x 3072).  So: few
+// rows stay with the kernel that reads the matrix once, from 17 on only where its blocks of 16 outputs are one a unit; tiles
+// are the kind whose busiest unit has the least to do - the blocks it gets times their area, a block of 32 x 64 taking 5 % and
+// one of 32 x 32 15 % longer for its area than one of 64 x 64.  (Tiles of 128 are slower everywhere: the matrix cores wait for
+// nothing that larger tiles would spare.)
 int launch_f32(const float* x, const float* w, float* y, int rows, int outs, int k, const float* bias, hipStream_t stream) {
   const bool wide_stores = outs % 4 == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0;
   const long units = device_facts().compute_units;
-  const auto blocks = [&](int out_tile, int row_tile) {
-    return static_cast<long>((outs + out_tile - 1) / out_tile) * ((rows + row_tile - 1) / row_tile);
+  const auto rounds = [&](int out_tile, int row_tile) {
+    const long blocks = static_cast<long>((outs + out_tile - 1) / out_tile) * ((rows + row_tile - 1) / row_tile);
+    return (blocks + units - 1) / units;
   };
   if (rows <= 16) return launch_f32_few<1>(x, w, y, rows, outs, k, bias, wide_stores, stream);
-  if (blocks(64, 64) < 2 * units) {
-    if (rows <= 32) return launch_f32_few<2>(x, w, y, rows, outs, k, bias, wide_stores, stream);
-    if (rows <= 64) return launch_f32_few<4>(x, w, y, rows, outs, k, bias, wide_stores, stream);
-  }
-  if (4 * blocks(64, 64) >= 7 * units) return launch_f32_wide<2, 2>(x, w, y, rows, outs, k, bias, wide_stores, stream);
-  if (blocks(32, 64) >= 2 * units) return launch_f32_wide<1, 2>(x, w, y, rows, outs, k, bias, wide_stores, stream);
+  if (rows <= 32 && (outs + 15) / 16 <= units) return launch_f32_few<2>(x, w, y, rows, outs, k, bias, wide_stores, stream);
+  const long large = 400 * rounds(64, 64), middle = 210 * rounds(32, 64), small = 115 * rounds(32, 32);
+  if (large <= middle && large <= small) return launch_f32_wide<2, 2>(x, w, y, rows, outs, k, bias, wide_stores, stream);
+  if (middle <= small) return launch_f32_wide<1, 2>(x, w, y, rows, outs, k, bias, wide_stores, stream);
   return launch_f32_wide<1, 1>(x, w, y, rows, outs, k, bias, wide_stores, stream);
 }
 

@@ -1025,9 +1025,9 @@ def test_linear_rows_do_not_depend_on_the_batch(hip):
         assert torch.equal(alone[0], whole[row])
 
 
-@pytest.mark.parametrize("outs,k", [(16, 4), (150, 300), (100, 128), (2051, 260), (64, 2052), (3072, 2048)])
+@pytest.mark.parametrize("outs,k", [(16, 4), (150, 300), (100, 128), (2051, 260), (64, 2052), (3072, 2048), (4200, 160)])
 def test_float32_products_on_the_matrix_cores(hip, outs, k):
-    """Rows on both sides of every kernel's range (16 / 32 / 64 rows a launch, then tiles), widths that end inside a chain
+    """Rows on both sides of every kernel's range (16 / 32 rows a launch where outputs are few, then tiles), widths that end inside a chain
     of 128 and inside a group of 16, outputs that end inside a tile; with and without a bias.  Against float64: a
     term passes at most min(k, 128) additions of its chain and one per chain, and its own product; every rounding is at most
     2^-24 of a partial sum, which is at most the sum of the terms' magnitudes: |error| <= (min(k, 128) + chains + 1) 2^-24
