@@ -138,6 +138,119 @@ __global__ __launch_bounds__(256) void unit_norm_write_kernel(const T* __restric
                     positions, q_weight, k_weight, interleaved, value_eps, temp_coef, temp_every, values_at);
 }
 
+// Eight bfloat16 (or float32) values from 16-byte aligned memory, widened.
+__device__ __forceinline__ void load8(const bf16_t* p, float (&v)[8]) {
+  const uint4 raw = *reinterpret_cast<const uint4*>(p);
+  const uint32_t words[4] = {raw.x, raw.y, raw.z, raw.w};
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    v[2 * k] = __uint_as_float(words[k] << 16);
+    v[2 * k + 1] = __uint_as_float(words[k] & 0xffff0000u);
+  }
+}
+__device__ __forceinline__ void load8(const float* p, float (&v)[8]) {
+  const float4 a = *reinterpret_cast<const float4*>(p), b = *reinterpret_cast<const float4*>(p + 4);
+  v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w, v[4] = b.x, v[5] = b.y, v[6] = b.z, v[7] = b.w;
+}
+
+// bfloat16 vectors whose widths come in eights, unscaled but for the norm: a thread takes eight neighbouring elements of a
+// vector with 16-byte reads and writes (a norm's sum meets over the dim / 8 lanes of its vector, a power of two), and a wave
+// takes 64 dimensions of a value head for eight tokens, which it turns through LDS: where the eight slots are a run of one
+// page from a multiple of eight on - a prompt's are -, every lane writes its dimension's eight tokens as 16 bytes.  Bound by
+// memory; what is not is the reads of single elements and the writes of two bytes each that the kernel above makes (a wave a
+// vector).  2,000 tokens of 16 query, 4 key and 4 value heads of 128 (25 MB): 18.9 us there, of 32 query and 8 key vectors of 64
+// and 4 values of 128 27.8; here 10.1 both (2.5 TB/s: a thread has one 16-byte group or two on their way).  8 tokens 4 us both.
+template <bool NORMED>
+__global__ __launch_bounds__(256) void unit_norm_write_eights_kernel(const bf16_t* __restrict__ projected, long stride, int tokens,
+                                                                     int q_vectors, int kv_heads, int dim, int vdim, float eps,
+                                                                     const int* __restrict__ slot_map,
+                                                                     bf16_t* __restrict__ k_pages, bf16_t* __restrict__ v_pages,
+                                                                     int page_size, long num_pages, bf16_t* __restrict__ q_out,
+                                                                     int maps, const float* __restrict__ table,
+                                                                     int table_positions, int rot_dims,
+                                                                     const int* __restrict__ positions, int values_at,
+                                                                     unsigned vector_blocks) {
+  __shared__ __align__(16) bf16_t turned[4][8][72];        // (a row of 144 bytes: 16-byte writes, reads along a column)
+  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+  if (blockIdx.x < vector_blocks) {
+    const unsigned eights = dim / 8, per_token = (q_vectors + (slot_map != nullptr ? kv_heads * maps : 0)) * eights;
+    const unsigned index = blockIdx.x * 256 + threadIdx.x, token = index / per_token, at = index % per_token;
+    if (token >= static_cast<unsigned>(tokens)) return;    // (whole vectors: a vector's lanes leave together)
+    const int which = at / eights, i = (at % eights) * 8;
+    const bf16_t* x = projected + token * stride + static_cast<long>(which) * dim;
+    float v[8];
+    load8(x + i, v);
+    float scale = 1.f;
+    if constexpr (NORMED) {
+      float squares = 0.f;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) squares += v[j] * v[j];
+      for (unsigned reach = 1; reach < eights; reach *= 2) squares += __shfl_xor(squares, reach);
+      scale = rsqrtf(squares / static_cast<float>(dim) + eps);
+    }
+    bf16_t* y = q_out + (static_cast<long>(token) * q_vectors + which) * dim;
+    if (which >= q_vectors) {
+      const int slot = slot_map[token], page = slot / page_size, vector = which - q_vectors;
+      if (slot < 0 || page >= num_pages) return;
+      y = k_pages + (((static_cast<long>(page) * kv_heads + vector / maps) * page_size + slot % page_size) * maps + vector % maps) * dim;
+    }
+    if (NORMED) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[j] *= scale;
+    }
+    if (i < rot_dims) {
+      const int half = rot_dims / 2;
+      const bool low = i < half;
+      const int pos = positions[token];
+      const bool known = pos >= 0 && pos < table_positions;      // (a position beyond the table poisons the vector)
+      const float* angles = table + (static_cast<long>(known ? pos : 0) * half + (low ? i : i - half)) * 2;
+      float other[8];
+      load8(x + (low ? i + half : i - half), other);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float c = angles[2 * j], s = angles[2 * j + 1], o = other[j] * scale;
+        v[j] = low ? v[j] * c - o * s : v[j] * c + o * s;
+        if (!known) v[j] = __uint_as_float(0x7fc00000u);
+      }
+    }
+    alignas(16) bf16_t packed[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) packed[j] = from_float<bf16_t>(v[j]);
+    *reinterpret_cast<uint4*>(y + i) = *reinterpret_cast<const uint4*>(packed);
+    return;
+  }
+  // values: a wave's item is eight tokens, a head and 64 of its dimensions
+  const int pieces = (vdim + 63) / 64, per_group = kv_heads * pieces;
+  const unsigned item = (blockIdx.x - vector_blocks) * 4 + wave;
+  const int first = item / per_group * 8, h = item % per_group / pieces, d0 = item % pieces * 64;
+  const int token = first + lane / 8, d = d0 + lane % 8 * 8;
+  const bool there = token < tokens && d < vdim;
+  const int slot = token < tokens ? slot_map[token] : -1;
+  uint4 raw = make_uint4(0, 0, 0, 0);
+  if (there) raw = *reinterpret_cast<const uint4*>(projected + token * stride + values_at + static_cast<long>(h) * vdim + d);
+  const int start = __shfl(slot, 0);
+  const bool run = first + 8 <= tokens && start >= 0 && start % 8 == 0;
+  // (page_size is a multiple of eight: a run from a multiple of eight on stays in its page)
+  if (__all(run && slot == start + lane / 8)) {
+    *reinterpret_cast<uint4*>(&turned[wave][lane / 8][lane % 8 * 8]) = raw;
+    wave_sync_lds();
+    alignas(16) bf16_t packed[8];
+#pragma unroll
+    for (int t = 0; t < 8; ++t) packed[t] = turned[wave][t][lane];
+    const long page = start / page_size;
+    if (page < num_pages && d0 + lane < vdim)
+      *reinterpret_cast<uint4*>(v_pages + ((page * kv_heads + h) * vdim + d0 + lane) * page_size + start % page_size) =
+          *reinterpret_cast<const uint4*>(packed);
+    return;
+  }
+  if (!there || slot < 0 || slot / page_size >= num_pages) return;
+  alignas(16) bf16_t own[8];
+  *reinterpret_cast<uint4*>(own) = raw;
+  bf16_t* y = v_pages + ((static_cast<long>(slot / page_size) * kv_heads + h) * vdim + d) * page_size + slot % page_size;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) y[static_cast<long>(j) * page_size] = own[j];
+}
+
 // The same with the root mean square taken over all of a token's query vectors at once, and over all its key vectors: a
 // block is a token, sums both sides' squares once, and its waves then take the token's items in turn.
 template <typename T>
@@ -173,21 +286,6 @@ __global__ __launch_bounds__(1024) void unit_norm_write_whole_kernel(const T* __
 
 constexpr int kMaxValueRegs = 4;  // value widths up to 256: each lane owns dims lane, lane + 64, ...
 constexpr int kMaxRowWaves = 16;  // the most waves that share a (token, head): wave w of W takes the key tiles w, w + W, ...
-
-// Eight bfloat16 (or float32) values from 16-byte aligned memory, widened.
-__device__ __forceinline__ void load8(const bf16_t* p, float (&v)[8]) {
-  const uint4 raw = *reinterpret_cast<const uint4*>(p);
-  const uint32_t words[4] = {raw.x, raw.y, raw.z, raw.w};
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    v[2 * k] = __uint_as_float(words[k] << 16);
-    v[2 * k + 1] = __uint_as_float(words[k] & 0xffff0000u);
-  }
-}
-__device__ __forceinline__ void load8(const float* p, float (&v)[8]) {
-  const float4 a = *reinterpret_cast<const float4*>(p), b = *reinterpret_cast<const float4*>(p + 4);
-  v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w, v[4] = b.x, v[5] = b.y, v[6] = b.z, v[7] = b.w;
-}
 
 // A block is a token and G query heads that read the same key head (G = 1: a single head); its waves (1 to 16, the
 // caller's choice) take the row's tiles of 64 keys in turn and their shares - maximum, sum of weights, weighted values,
@@ -670,6 +768,28 @@ int akv_unit_norm_write(const void* projected, long stride, int dtype, long toke
                                static_cast<T*>(k_pages), static_cast<T*>(v_pages), page_size, num_pages, static_cast<T*>(q_out),
                                maps, table, table_positions, rot_dims, positions, q_weight, k_weight, interleaved, value_eps,
                                temp_coef, temp_every, values_at));
+    return AKV_LAUNCH_STATUS();
+  }
+  // Eights: nothing but a norm and a rotation of halves, and every 16-byte group of a vector, a rotated half or a page row is
+  // whole and aligned - of all numbers of tokens, so that a token's bits do not depend on how its request was cut (2,000
+  // tokens 10 us against 19 to 28, 8 tokens 4 us either way).
+  const auto aligned = [](const void* at) { return reinterpret_cast<uintptr_t>(at) % 16 == 0; };
+  const int eights = dim / 8;
+  const bool rotates = table != nullptr && rot_dims > 0;
+  if (dtype == 1 && dim % 8 == 0 && vdim % 8 == 0 && stride % 8 == 0 && page_size % 8 == 0 &&
+      (q_heads + kv_heads) * static_cast<long>(maps) * eights * tokens < (1L << 31) && q_weight == nullptr &&
+      k_weight == nullptr && value_eps < 0.f && temp_every <= 0 &&
+      (!rotates || (rot_dims % 16 == 0 && !interleaved)) && (!normed || ((eights & (eights - 1)) == 0 && eights <= kWave)) &&
+      aligned(projected) && aligned(q_out) && aligned(k_pages) && aligned(v_pages)) {
+    const long vectors = (q_heads + (slot_map != nullptr ? kv_heads : 0)) * static_cast<long>(maps);
+    const long value_items = slot_map != nullptr ? (tokens + 7) / 8 * kv_heads * ((vdim + 63) / 64) : 0;
+    const unsigned vector_blocks = static_cast<unsigned>((vectors * eights * tokens + 255) / 256);
+    const unsigned blocks = vector_blocks + static_cast<unsigned>((value_items + 3) / 4);
+    const auto kernel = normed ? unit_norm_write_eights_kernel<true> : unit_norm_write_eights_kernel<false>;
+    kernel<<<blocks, 256, 0, stream>>>(static_cast<const bf16_t*>(projected), stride, static_cast<int>(tokens), q_heads * maps,
+                                       kv_heads, dim, vdim, eps, slot_map, static_cast<bf16_t*>(k_pages),
+                                       static_cast<bf16_t*>(v_pages), page_size, num_pages, static_cast<bf16_t*>(q_out), maps,
+                                       table, table_positions, rotates ? rot_dims : 0, positions, values_at, vector_blocks);
     return AKV_LAUNCH_STATUS();
   }
   AKV_DISPATCH(dtype, T, unit_norm_write_kernel<T><<<static_cast<unsigned>((items + 3) / 4), 256, 0, stream>>>(

@@ -348,6 +348,51 @@ def test_single_tokens_on_the_matrix_cores(hip, heads, kv_heads, dim, vdim, page
     assert ((last - clean[-1]).abs() <= clean[-1].abs() * 2.0 ** -7 + 1e-4).all()
 
 
+@pytest.mark.parametrize("heads,kv_heads,dim,vdim,page,maps,eps,rot,keyed", [
+    (4, 2, 64, 64, 16, 1, 1e-6, 0, False), (16, 4, 128, 128, 16, 1, None, 64, False), (2, 1, 40, 72, 8, 2, None, 16, False),
+    (3, 3, 8, 8, 64, 1, 1e-5, 0, True), (1, 1, 512, 256, 32, 1, 1e-6, 512, False), (6, 2, 24, 200, 24, 1, None, 0, False)])
+@pytest.mark.parametrize("lead", [0, 3, 8])
+def test_norm_and_rotation_in_eights(hip, heads, kv_heads, dim, vdim, page, maps, eps, rot, keyed, lead):
+    """Vectors whose widths come in eights, against the oracle on the same rows in float32: `lead` tokens of other requests and
+    a portion of 29 - so that eight tokens are a run of a page, cross into one, or lie askew -, some tokens without a
+    slot or beyond the pages, with and without the cache write.  Queries and keys: a rounding to bfloat16 is at most 2^-8 of the value, and float32's
+    own roundings (a norm of at most 512 terms, a turn of two) at most 2^-16 of the magnitudes that meet; values the same bits;
+    nothing else in the pages changes."""
+    from torch_kernels import TorchKernels
+    generator = torch.Generator().manual_seed(heads * 1000 + dim + lead)
+    tokens, num_pages = lead + 29, 29 // page + 12
+    columns = (heads + kv_heads) * maps * dim + (0 if keyed else kv_heads * vdim)
+    rows = torch.randn(tokens, 16 + columns, generator=generator).bfloat16()
+    positions = torch.randint(0, 300, (tokens,), generator=generator, dtype=torch.int32)
+    slots = torch.cat([torch.arange(lead) * (page + 1) + 5 * page, torch.arange(29) + page]).int()
+    slots[[lead + 9, tokens - 1]] = torch.tensor([-1, num_pages * page + 3], dtype=torch.int32)
+    slots[:lead] += 29 // page * page + page * 2 - 5 * page + page
+    slots[:lead] = torch.where(slots[:lead] < num_pages * page, slots[:lead], -1)
+    angles = torch.rand(300, max(rot, 2) // 2, generator=generator) * 6
+    table = torch.stack([angles.cos(), angles.sin()], -1).float() if rot else None
+    more = dict(at=16, maps=maps, rot_dims=rot, keyed_values=keyed)
+    k_pages = torch.full((num_pages, kv_heads, page, maps * dim), 7.0)
+    v_pages = torch.full((num_pages, kv_heads, vdim, page), 7.0)
+    want_q, oracle = torch.empty(tokens, heads * maps * dim), TorchKernels()
+    oracle.unit_norm_write(rows.float(), heads, kv_heads, dim, vdim, eps, None, k_pages, v_pages, want_q, table=table,
+                           positions=positions, **more)
+    kept = (slots >= 0) & (slots < num_pages * page)
+    got_k, got_v = k_pages.bfloat16().to(DEVICE), v_pages.bfloat16().to(DEVICE)
+    oracle.unit_norm_write(rows[kept].float(), heads, kv_heads, dim, vdim, eps, slots[kept], k_pages, v_pages,
+                           want_q[kept], table=table, positions=positions[kept], **more)
+    for slot_map in (None, slots.to(DEVICE)):
+        if slot_map is not None:
+            assert (got_k == 7).all() and (got_v == 7).all()
+        q = torch.empty(tokens, heads * maps * dim, dtype=torch.bfloat16, device=DEVICE)
+        hip.unit_norm_write(rows.to(DEVICE), heads, kv_heads, dim, vdim, eps, slot_map, got_k, got_v, q,
+                            table=table.to(DEVICE) if rot else None, positions=positions.to(DEVICE), **more)
+        reach = 2.0 ** -16 * 2 * (want_q.abs().max())
+        assert ((q.cpu().float() - want_q).abs() <= want_q.abs() * 2.0 ** -8 + reach).all()
+    reach = 2.0 ** -16 * 2 * k_pages.abs().max()
+    assert ((got_k.cpu().float() - k_pages).abs() <= k_pages.abs() * 2.0 ** -8 + reach).all()
+    assert torch.equal(got_v.cpu().float(), v_pages)
+
+
 @pytest.mark.parametrize("heads,kv_heads,dim,vdim,page,maps,options", [c for c in SINGLES if c[2] <= 128 and c[3] <= 128] + [
     (12, 4, 128, 128, 16, 1, dict(sink="learned", gates=True)), (3, 3, 64, 64, 64, 1, dict(window=70, keep_first=40)),
     (4, 2, 64, 128, 16, 2, dict(window=50, sink="zero"))])
