@@ -67,6 +67,49 @@ __global__ __launch_bounds__(256) void delta_prepare_kernel(const T* __restrict_
   }
 }
 
+// The same for vectors of 4 L elements, L a power of two up to 64: L lanes take a q / k pair, four elements of each a lane, and
+// behind the pairs (from a multiple of a wave on) a lane takes four decays.  Memory and the exponentials bound it: 2,000 tokens
+// of 16 heads of 128 with decays per channel, 82 MB: 24.4 us, 33.5 with single elements; 8 tokens 4.2 and 5.1.
+template <typename T, typename TD, bool HEAD_DECAY>
+__global__ __launch_bounds__(256) void delta_prepare_fours_kernel(const T* __restrict__ conv, long conv_stride,
+                                                                  const T* __restrict__ beta_logits, long beta_stride,
+                                                                  const TD* __restrict__ decay_logits, long decay_stride,
+                                                                  const float* __restrict__ decay_bias,
+                                                                  const float* __restrict__ rate, float unit_eps, float q_scale,
+                                                                  float* __restrict__ prepared, int heads, int groups, int dim) {
+  const long n = blockIdx.x;
+  const int lanes = dim / 4, pairs = groups * lanes, at = blockIdx.y * 256 + threadIdx.x;
+  const long width = prepared_width(heads, groups, dim, HEAD_DECAY);
+  float* row = prepared + n * width;
+  float* beta = row + prepared_scalars_at(heads, groups, dim, HEAD_DECAY);
+  const TD* logits = decay_logits + n * decay_stride;
+  if (at < pairs) {                                        // (a pair's lanes come together)
+    const T* from = conv + n * conv_stride + at * 4;
+    const float4 q = four_of(from), k = four_of(from + static_cast<long>(groups) * dim);
+    const float qq = lanes_sum(four_squares(q), lanes), kk = lanes_sum(four_squares(k), lanes);
+    const float q_unit = q_scale / sqrtf(qq + unit_eps), k_unit = 1.f / sqrtf(kk + unit_eps);
+    const float dot = lanes_sum(fmaf(q.z, k.z, q.x * k.x) + fmaf(q.w, k.w, q.y * k.y), lanes) * q_unit * k_unit;
+    put_four(row + at * 4, make_float4(q.x * q_unit, q.y * q_unit, q.z * q_unit, q.w * q_unit));
+    put_four(row + static_cast<long>(groups) * dim + at * 4, make_float4(k.x * k_unit, k.y * k_unit, k.z * k_unit, k.w * k_unit));
+    const int unit = at / lanes, share = heads / groups;
+    for (int j = at % lanes; j < share; j += lanes) {
+      const int h = unit * share + j;
+      beta[h] = sigmoid_of(to_float(beta_logits[n * beta_stride + h]));
+      beta[heads + h] = dot;
+      if constexpr (HEAD_DECAY) beta[2 * heads + h] = expf(-rate[h] * softplus_of(to_float(logits[h]) + decay_bias[h]));
+    }
+    return;
+  }
+  if constexpr (!HEAD_DECAY) {
+    const int i = (at - (pairs + kWave - 1) / kWave * kWave) * 4;
+    if (i < 0 || i >= heads * dim) return;
+    const float4 z = four_of(logits + i), bias = four_of(decay_bias + i);
+    const float fall = -rate[i / dim];
+    put_four(row + 2L * groups * dim + i, make_float4(expf(fall * softplus_of(z.x + bias.x)), expf(fall * softplus_of(z.y + bias.y)),
+                                                      expf(fall * softplus_of(z.z + bias.z)), expf(fall * softplus_of(z.w + bias.w))));
+  }
+}
+
 template <typename T, typename TD, typename TG, bool HEAD_DECAY>
 int delta_rule(const T* conv, long conv_stride, const T* beta_logits, long beta_stride, const TD* decay_logits,
                long decay_stride, const float* decay_bias, const float* rate, const TG* gates, long gate_stride, int gate_act,
@@ -75,18 +118,24 @@ int delta_rule(const T* conv, long conv_stride, const T* beta_logits, long beta_
                int dim, int vdim, int longest, hipStream_t stream) {
   float* prepared = workspace;
   float* raw = workspace + (static_cast<long>(tokens) + kRowsBehind) * prepared_width(heads, groups, dim, HEAD_DECAY);
-  const int units = groups + (HEAD_DECAY ? 0 : (heads * dim + 255) / 256);
-  const dim3 prepare_grid(static_cast<unsigned>(tokens), static_cast<unsigned>((units + 3) / 4));
-  delta_prepare_kernel<T, TD, HEAD_DECAY><<<prepare_grid, 256, 0, stream>>>(conv, conv_stride, beta_logits, beta_stride,
-                                                                            decay_logits, decay_stride, decay_bias, rate,
-                                                                            unit_eps, q_scale, prepared, heads, groups, dim);
+  if (lanes_of_fours(dim) && conv_stride % 4 == 0 && in_fours(conv) && in_fours(prepared) &&
+      (HEAD_DECAY || (decay_stride % 4 == 0 && in_fours(decay_logits) && in_fours(decay_bias)))) {
+    const int pairs = (groups * dim / 4 + kWave - 1) / kWave * kWave, threads = pairs + (HEAD_DECAY ? 0 : heads * dim / 4);
+    delta_prepare_fours_kernel<T, TD, HEAD_DECAY><<<dim3(tokens, (threads + 255) / 256), 256, 0, stream>>>(
+        conv, conv_stride, beta_logits, beta_stride, decay_logits, decay_stride, decay_bias, rate, unit_eps, q_scale, prepared,
+        heads, groups, dim);
+  } else {
+    const int units = groups + (HEAD_DECAY ? 0 : (heads * dim + 255) / 256);
+    delta_prepare_kernel<T, TD, HEAD_DECAY><<<dim3(tokens, (units + 3) / 4), 256, 0, stream>>>(
+        conv, conv_stride, beta_logits, beta_stride, decay_logits, decay_stride, decay_bias, rate, unit_eps, q_scale, prepared,
+        heads, groups, dim);
+  }
   const int status = launch_state_walk<T, kDelta, HEAD_DECAY>(prepared, conv + 2L * groups * dim, conv_stride, state,
                                                               state_stride, q_start, seq_slots, raw, seqs, heads, groups, dim,
                                                               vdim, 0, longest, stream);
   if (status != 0) return status;
-  const long items = static_cast<long>(tokens) * heads;
-  state_finish_kernel<T, TG><<<static_cast<unsigned>((items + 3) / 4), 256, 0, stream>>>(
-      raw, nullptr, 0.f, norm_weight, 0, gates, gate_stride, gate_act, norm_eps, out, items, heads, vdim, 0);
+  launch_state_finish<T, TG>(raw, nullptr, 0.f, norm_weight, 0, gates, gate_stride, gate_act, norm_eps, out, tokens, heads, vdim,
+                             0, stream);
   return 0;
 }
 

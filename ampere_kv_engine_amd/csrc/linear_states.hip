@@ -192,9 +192,7 @@ int time_mixing(const T* r, const T* k, const T* v, const T* gates, long row_str
   const int status = launch_state_walk<T, kAddAfter, false>(prepared, v, row_stride, state, state_stride, q_start, seq_slots, raw,
                                                             seqs, heads, heads, dim, dim, 0, longest, stream);
   if (status != 0) return status;
-  const long items = static_cast<long>(tokens) * heads;
-  state_finish_kernel<T, T><<<static_cast<unsigned>((items + 3) / 4), 256, 0, stream>>>(
-      raw, nullptr, 0.f, norm_weight, 1, gates, row_stride, 2, eps, out, items, heads, dim, 0);
+  launch_state_finish<T, T>(raw, nullptr, 0.f, norm_weight, 1, gates, row_stride, 2, eps, out, tokens, heads, dim, 0, stream);
   return 0;
 }
 
@@ -216,9 +214,7 @@ int matrix_memory(const T* q, const T* k, const T* v, const T* gates, const T* i
   const int status = launch_state_walk<T, kAdd, true>(prepared, v, row_stride, state, state_stride, q_start, seq_slots, raw, seqs,
                                                       heads, heads, dim, vdim, 1, longest, stream);
   if (status != 0) return status;
-  const long items = static_cast<long>(tokens) * heads;
-  state_finish_kernel<T, T><<<static_cast<unsigned>((items + 3) / 4), 256, 0, stream>>>(
-      raw, tops, read_eps, norm_weight, 1, gates, row_stride, 1, eps, out, items, heads, vdim, 1);
+  launch_state_finish<T, T>(raw, tops, read_eps, norm_weight, 1, gates, row_stride, 1, eps, out, tokens, heads, vdim, 1, stream);
   return 0;
 }
 

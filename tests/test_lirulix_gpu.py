@@ -349,6 +349,33 @@ def test_delta_rule_kernels_alone(hip, dtype, heads, groups, dim, vdim, taps):
         error = (got[r] - want).abs().max() / want.abs().max()
         assert error < (3e-5 if dtype == torch.float32 else 0.02), f"request {r}: {error:.2e}"
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("sizes", [(2, 2, 4, 4, 2), (3, 1, 256, 256, 2), (5, 5, 16, 8, 3), (1, 1, 32, 6, 2), (2, 1, 12, 32, 2)])
+def test_delta_rule_at_the_edges_of_its_fours(hip, dtype, sizes):
+    """Widths of 4 to 256 in powers of two, on either side alone and on both, pairs that fill no wave."""
+    test_delta_rule_kernels_alone(hip, dtype, *sizes)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("tokens,heads,vdim,lead", [(1, 1, 4, 0), (3, 5, 8, 4), (7, 3, 256, 8), (70, 2, 64, 0), (5, 2, 64, 2), (4, 3, 12, 0),
+                                                    (2, 1, 512, 0)])
+def test_difference_norm_gate_at_the_edges_of_its_fours(hip, dtype, tokens, heads, vdim, lead):
+    """Heads of four values to beyond 256, items that fill no block, gates that begin askew: against float64.  Float32's
+    roundings: a norm of at most 512 terms and a dozen operations, within 2^-16 of the value; bfloat16 rounds once more, 2^-8."""
+    generator = torch.Generator().manual_seed(tokens * 100 + vdim)
+    maps = torch.randn(tokens, heads * 2 * vdim, generator=generator).to(dtype)
+    gates = torch.randn(tokens, lead + heads * vdim + (-lead - heads * vdim) % 4, generator=generator).to(dtype)
+    lam, eps, after = torch.tensor([0.4]), 1e-5, 0.7
+    out = torch.empty(tokens, heads * vdim, dtype=dtype, device=DEVICE)
+    hip.difference_norm_gate(maps.to(DEVICE), lam.to(DEVICE), eps, after, gates.to(DEVICE), lead, heads, vdim, out)
+    first, second = maps.double().view(tokens, heads, 2, vdim).unbind(2)
+    o = first - lam.double() * second
+    want = o / torch.sqrt((o * o).mean(-1, keepdim=True) + eps) * after
+    want = (want * torch.sigmoid(gates[:, lead:lead + heads * vdim].double().view(tokens, heads, vdim))).reshape(tokens, -1)
+    reach = 2.0 ** -16 if dtype == torch.float32 else 2.0 ** -8 + 2.0 ** -16
+    # (a difference of two nearly equal values keeps its absolute error: 2^-23 of what was subtracted, times the norm's factor)
+    assert ((out.cpu().double() - want).abs() <= want.abs() * reach + 1e-5).all()
+
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("channels,extra,taps", [(64, 0, 4), (264, 8, 2), (40, 16, 3), (512, 24, 5), (48, 4, 4), (36, 4, 3), (16, 0, 6)])
