@@ -5,7 +5,7 @@
 // inside fixed k-tiles, so a row's result does not depend on how many other rows the call carries.  It is the
 // fallback for operand mixes and widths that no matrix-core kernel takes.
 //
-// `linear_f32_few` and `linear_f32_wide` are the float32 path on the matrix cores (see below).
+// `linear_f32_pairs`, `linear_f32_few` and `linear_f32_wide` are the float32 path on the matrix cores (see below).
 
 #include "common.h"
 #include "api.h"
@@ -170,6 +170,54 @@ __global__ __launch_bounds__(1024) void linear_f32_few_kernel(const float* __res
   if (wave < NT && 16 * wave + r < rows) store_f32(y, 16 * wave + r, out0 + 4 * g, outs, total, bias, wide_stores);
 }
 
+// Up to 8 rows: bound by what the units have on their way from memory; a block a tile of 16 outputs leaves half of them without
+// one at 2,048 outputs, and its sixteen waves share a unit with no other block at more.  Here a block owns 8 outputs,
+// and an instruction carries two segments of k - its rows 0 .. 7 the outputs' first and its rows 8 .. 15 their second, its
+// columns likewise the rows of x, so that two quarters of its sums are the two segments' and the others mean nothing (the matrix
+// cores have nothing else to do).  Each sum is the chain that the other kernels form, and the segments are added in their order.
+__global__ __launch_bounds__(1024) void linear_f32_pairs_kernel(const float* __restrict__ x, const float* __restrict__ w,
+                                                               float* __restrict__ y, int rows, int outs, int k, int segments,
+                                                               const float* __restrict__ bias, bool wide_stores) {
+  extern __shared__ floats4 pieces[];                      // [2 waves][16]
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
+  const int r = lane & 7, second = lane >> 3 & 1, g = lane >> 4;
+  const int out0 = blockIdx.x * 8;
+  const float* wp = w + static_cast<long>(min(out0 + r, outs - 1)) * k;
+  const float* xp = x + static_cast<long>(min(r, rows - 1)) * k;
+  const floats4 zero = {0.f, 0.f, 0.f, 0.f};
+  floats4 total = zero;
+  for (int first = 0; first < segments; first += 2 * waves) {
+    const int segment = first + 2 * wave + second, at = segment * kSegment + 4 * g;
+    floats4 a[kSegmentBlocks], v[kSegmentBlocks];
+    // (beyond k - a multiple of 4: a group of four is whole or absent - the last elements once more, which count as zeros)
+#pragma unroll
+    for (int b = 0; b < kSegmentBlocks; ++b) a[b] = *reinterpret_cast<const floats4*>(wp + min(at + 16 * b, k - 4));
+#pragma unroll
+    for (int b = 0; b < kSegmentBlocks; ++b) v[b] = *reinterpret_cast<const floats4*>(xp + min(at + 16 * b, k - 4));
+    __builtin_amdgcn_sched_barrier(0);                     // (else the loads are moved down to where they are used)
+    floats4 sums = zero;
+    if ((first + 2 * wave + 2) * kSegment <= k) {          // (the same for the wave)
+#pragma unroll
+      for (int b = 0; b < kSegmentBlocks; ++b) sums = mfma4(a[b], v[b], sums);
+    } else {
+#pragma unroll
+      for (int b = 0; b < kSegmentBlocks; ++b) {
+        const bool inside = at + 16 * b < k;
+        sums = mfma4(inside ? a[b] : zero, inside ? v[b] : zero, sums);
+      }
+    }
+    // lane (column, g) holds the sums of instruction rows 4 g .. 4 g + 3: of outputs 4 (g & 1) .. + 3 and segment g / 2
+    if (second == g >> 1) pieces[(2 * wave + second) * 16 + (g & 1) * 8 + r] = sums;
+    __syncthreads();
+    if (threadIdx.x < 16) {
+      const int there = min(2 * waves, segments - first);
+      for (int s = 0; s < there; ++s) total += pieces[s * 16 + threadIdx.x];
+    }
+    __syncthreads();
+  }
+  if (threadIdx.x < 16 && r < rows) store_f32(y, r, out0 + 4 * static_cast<int>(threadIdx.x >> 3), outs, total, bias, wide_stores && out0 + 8 <= outs);
+}
+
 // More rows: tiles of 32 TM outputs by 32 TN rows, four waves of TM x TN tiles of 16 each, operands through two LDS buffers
 // of 32 k (row stride 36 floats: 16-byte reads of eight rows meet no bank twice), the next AHEAD steps of 32 k on their way in
 // registers.  Bound by the matrix cores where tiles fill the chip (8 TM TN instructions of 32 cycles a step and wave for
@@ -278,6 +326,15 @@ int launch_f32_few(const float* x, const float* w, float* y, int rows, int outs,
   return AKV_LAUNCH_STATUS();
 }
 
+int launch_f32_pairs(const float* x, const float* w, float* y, int rows, int outs, int k, const float* bias, bool wide_stores,
+                     hipStream_t stream) {
+  const int segments = (k + kSegment - 1) / kSegment, pairs = (segments + 1) / 2, rounds = (pairs + 15) / 16;
+  const int waves = (pairs + rounds - 1) / rounds;
+  linear_f32_pairs_kernel<<<(outs + 7) / 8, waves * 64, 2 * waves * 16 * sizeof(floats4), stream>>>(x, w, y, rows, outs, k, segments,
+                                                                                                    bias, wide_stores);
+  return AKV_LAUNCH_STATUS();
+}
+
 template <int TM, int TN>
 int launch_f32_wide(const float* x, const float* w, float* y, int rows, int outs, int k, const float* bias, bool wide_stores,
                     hipStream_t stream) {
@@ -296,10 +353,16 @@ int launch_f32_wide(const float* x, const float* w, float* y, int rows, int outs
 //    700 rows:                            32 x 32 68 / 184 / 708 / 1046  32 x 64 64 / 178 / 709 / 892  64 x 64 82 / 196 / 698 / 849
 //    999 rows:                            32 x 32 89 / 264 / 1025 / 1496 32 x 64 86 / 244 / 932 / 1291 64 x 64 85 / 237 / 920 / 1224
 // (110 TFLOP/s at best; the vector kernel above: 511 us on average over 999 rows of 2048 x 2048 and 2048 x 3072).  So: few
-// rows stay with the kernel that reads the matrix once, from 17 on only where its blocks of 16 outputs are one a unit; tiles
+// rows stay with the kernels that read the matrix once, from 17 on only where blocks of 16 outputs are one a unit; tiles
 // are the kind whose busiest unit has the least to do - the blocks it gets times their area, a block of 32 x 64 taking 5 % and
 // one of 32 x 32 15 % longer for its area than one of 64 x 64.  (Tiles of 128 are slower everywhere: the matrix cores wait for
 // nothing that larger tiles would spare.)
+// Up to 8 rows, blocks of 8 outputs (pairs) against blocks of 16 (few), outs x k = 2048 x 2048 / 2048 x 6144 / 3072 x 2048 /
+// 4096 x 2048 / 6144 x 2048 / 12288 x 2048 / 32768 x 2048:
+//      1 row:  pairs 5.5 / 12.7 / 7.7 / 7.9 / 11.7 / 20.1 / 48     few 7.5 / 20.3 / 8.0 / 9.2 / 15.5 / 23.7 / 55
+//      8 rows: pairs 6.5 / 16.0 / 9.9 / 10.1 / 14.6 / 26.0 / 64    few 8.6 / 22.6 / 8.9 / 9.8 / 16.9 / 26.2 / 62
+// So: pairs up to 4 rows (also with 3: 2048 x 6144 13.4 against 20.6); from 5 on where they are one block a unit, or where
+// blocks of 16 are several a unit, but not many (100,000 x 1024 with 8 rows: 96 against 87).
 int launch_f32(const float* x, const float* w, float* y, int rows, int outs, int k, const float* bias, hipStream_t stream) {
   const bool wide_stores = outs % 4 == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0;
   const long units = device_facts().compute_units;
@@ -307,8 +370,11 @@ int launch_f32(const float* x, const float* w, float* y, int rows, int outs, int
     const long blocks = static_cast<long>((outs + out_tile - 1) / out_tile) * ((rows + row_tile - 1) / row_tile);
     return (blocks + units - 1) / units;
   };
+  const long tiles = (outs + 15) / 16;
+  if (rows <= 4 || (rows <= 8 && ((outs + 7) / 8 <= units || (tiles > units && tiles <= 4 * units))))
+    return launch_f32_pairs(x, w, y, rows, outs, k, bias, wide_stores, stream);
   if (rows <= 16) return launch_f32_few<1>(x, w, y, rows, outs, k, bias, wide_stores, stream);
-  if (rows <= 32 && (outs + 15) / 16 <= units) return launch_f32_few<2>(x, w, y, rows, outs, k, bias, wide_stores, stream);
+  if (rows <= 32 && tiles <= units) return launch_f32_few<2>(x, w, y, rows, outs, k, bias, wide_stores, stream);
   const long large = 400 * rounds(64, 64), middle = 210 * rounds(32, 64), small = 115 * rounds(32, 32);
   if (large <= middle && large <= small) return launch_f32_wide<2, 2>(x, w, y, rows, outs, k, bias, wide_stores, stream);
   if (middle <= small) return launch_f32_wide<1, 2>(x, w, y, rows, outs, k, bias, wide_stores, stream);

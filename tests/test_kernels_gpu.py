@@ -1025,10 +1025,11 @@ def test_linear_rows_do_not_depend_on_the_batch(hip):
         assert torch.equal(alone[0], whole[row])
 
 
-@pytest.mark.parametrize("outs,k", [(16, 4), (150, 300), (100, 128), (2051, 260), (64, 2052), (3072, 2048), (4200, 160)])
+@pytest.mark.parametrize("outs,k", [(16, 4), (150, 300), (100, 128), (2051, 260), (64, 2052), (3072, 2048), (4200, 160), (17000, 384)])
 def test_float32_products_on_the_matrix_cores(hip, outs, k):
-    """Rows on both sides of every kernel's range (16 / 32 rows a launch where outputs are few, then tiles), widths that end inside a chain
-    of 128 and inside a group of 16, outputs that end inside a tile; with and without a bias.  Against float64: a
+    """Rows on both sides of every kernel's range (4 / 8 / 16 / 32 rows a launch by the outputs' number, then tiles), widths that
+    end inside a chain of 128, after an odd number of chains and inside a group of 16, outputs that end inside a tile; with and
+    without a bias.  Against float64: a
     term passes at most min(k, 128) additions of its chain and one per chain, and its own product; every rounding is at most
     2^-24 of a partial sum, which is at most the sum of the terms' magnitudes: |error| <= (min(k, 128) + chains + 1) 2^-24
     sum |x w|.  A row's bits do not depend on the rows beside it."""
@@ -1036,7 +1037,7 @@ def test_float32_products_on_the_matrix_cores(hip, outs, k):
     x = rand(1000, k, seed=33).cuda()
     alone = torch.empty(1, outs, device="cuda")
     hip.linear(x[:1].contiguous(), w, alone)
-    for rows in (1, 15, 16, 17, 32, 33, 64, 65, 130, 257, 1000):
+    for rows in (1, 4, 5, 8, 9, 15, 16, 17, 32, 33, 64, 65, 130, 257, 1000):
         y, biased = torch.full((rows, outs), float("nan"), device="cuda"), torch.empty(rows, outs, device="cuda")
         hip.linear(x[:rows].contiguous(), w, y)
         hip.linear(x[:rows].contiguous(), w, biased, bias=bias)
