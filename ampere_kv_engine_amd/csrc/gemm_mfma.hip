@@ -666,7 +666,7 @@ extern "C" int akv_linear_packed_static(const void* x, const void* wp, void* y, 
 }
 
 // The gated pair in one pass: wp holds 2 * inter / 16 row tiles, gate tile t at 2t and up tile t at 2t + 1;
-// y [rows, inter] = silu(x Wgate^T) * (x Wup^T), or with `clamp` (three numbers on the device, else null) the clamped gate
+// y [rows, inter] = silu(x Wgate^T) * (x Wup^T), or with `clamp` (four numbers on the device, else null) the other gates
 // of `gate_times`.  inter must be a multiple of 16.
 extern "C" int akv_linear_packed_swiglu(const void* x, const void* wp, void* y, int y_dtype, int rows, int inter,
                                         int k, int n_tiles, int k_tiles, int x_packed, const float* clamp,

@@ -65,14 +65,21 @@ __device__ __forceinline__ floatx4 plus_bias(floatx4 acc, const float* __restric
   return acc;
 }
 
-// What a gated product stores.  `clamp` null: silu(gate) * up.  Otherwise its three numbers are a limit, a slope and a
-// shift: with g = min(gate, limit) and u = the up value held to [-limit, limit], g * sigmoid(slope g) * (u + shift).
+// What a gated product stores.  `clamp` null: silu(gate) * up.  Otherwise its four numbers are a limit, a slope, a shift and
+// a cubic: with g = min(gate, limit) and u = the up value held to [-limit, limit], g * sigmoid(slope g) * (u + shift) - or,
+// where the cubic is not 0, gate * sigmoid(slope (gate + cubic gate^3)) * up, the tanh form of gelu.
 __device__ __forceinline__ floatx4 gate_times(floatx4 gate, floatx4 up, const float* __restrict__ clamp) {
   floatx4 v;
   float slope = 1.f;
   if (clamp != nullptr) {
-    const float limit = clamp[0], shift = clamp[2];
+    const float limit = clamp[0], shift = clamp[2], cubic = clamp[3];
     slope = clamp[1];
+    if (cubic != 0.f) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        v[i] = gate[i] / (1.f + expf(-slope * (gate[i] + cubic * gate[i] * gate[i] * gate[i]))) * up[i];
+      return v;
+    }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       gate[i] = fminf(gate[i], limit);

@@ -346,6 +346,8 @@ class KernelSet:
     then launch the norm's and the product's own kernels.  (The operations every kernel set must have - `linear`,
     `add_rmsnorm`, `attention`, ... - are those `kernels/hip.py` defines.)"""
 
+    gated_gelu = False      # `prepare_gated_linear` takes gelu=True: the tanh form of gelu in the one-pass gated product
+
     def folds_norm(self, rows: int, hidden: int, dtype) -> bool:
         """A step of `rows` rows may let branches add themselves to the residual sum (`linear_adds`) and the next
         product norm its rows from the sums left there (`linear_scaled`)."""

@@ -958,6 +958,29 @@ def test_gated_product_with_a_clamped_gate(hip_own, hip_library, rows, inter, k)
             torch.testing.assert_close(got.cpu().float(), want, **tol(torch.bfloat16))
 
 
+@pytest.mark.parametrize("rows", [1, 8, 16, 17, 64, 130, 600])
+@pytest.mark.parametrize("inter,k", [(208, 264), (512, 1032)])
+def test_gated_product_with_a_gelu_gate(hip_own, hip_library, rows, inter, k):
+    """Every kernel that may take the product, against float64; gates from deep in gelu's left tail to far right of it.  One
+    rounding of the result to bfloat16 (2^-8 of it) - where the library takes the product also of gate and up, the gate's
+    times gelu's steepest slope (1.13) - and float32 sums of k terms."""
+    gate, up = (rand(inter, k, dtype=torch.bfloat16, seed=621 + i, scale=0.05 + 0.25 * (1 - i)) for i in range(2))
+    x = rand(rows, k, dtype=torch.bfloat16, seed=623)
+    x64, g64, u64 = x.double(), gate.double(), up.double()
+    g, u = x64 @ g64.T, x64 @ u64.T
+    gelu = torch.nn.functional.gelu(g, approximate="tanh")
+    want = gelu * u
+    sums = k * 2.0 ** -24 * (1.13 * (x64.abs() @ g64.abs().T) * u.abs() + gelu.abs() * (x64.abs() @ u64.abs().T))
+    for kernels in (hip_own, hip_library):
+        weight = kernels.prepare_gated_linear(gate.cuda(), up.cuda(), gelu=True)
+        shape = kernels.gated_scratch(weight, rows, torch.bfloat16)
+        scratch = torch.empty(shape, dtype=torch.bfloat16, device="cuda") if shape else None
+        got = torch.full((rows, inter), float("nan"), dtype=torch.bfloat16, device="cuda")
+        kernels.gated_linear(x.cuda(), weight, got, scratch)
+        rounded = 2.0 ** -8 * 1.01 * (want.abs() + ((1.13 * g.abs() + gelu.abs()) * u.abs() if shape else 0.0))
+        assert ((got.cpu().double() - want).abs() <= rounded + sums + 1e-6).all(), (kernels is hip_library, rows)
+
+
 @pytest.mark.parametrize("rows", [1, 3, 16, 40])
 def test_products_with_a_clamped_gate_that_norm_or_scale_their_rows(hip_own, ref, rows, monkeypatch):
     monkeypatch.setattr(hip_own, "fold_norms", True)
