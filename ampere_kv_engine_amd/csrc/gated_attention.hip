@@ -1223,9 +1223,13 @@ namespace {
 // read of sixteen rows meets no bank twice.  A wave passes over steps that none of its columns sees.  Scores, maxima,
 // weights and sums are float32 (base 2); a weight enters the second product as two bfloat16; the exponentials' reference
 // point trails the maximum by at most 2^8, so that sums are rescaled a few times a prompt and not once a step.
+// A key that one column sees and another does not has weight zero for the other, and zero times an infinity is not zero: where a
+// step is masked for some column of the block, the threads that file its values file zeros for what is not finite and say so,
+// and the waves then add it, one value at a time, to the columns that see its key (finite values pay for the look in a few
+// steps a block: 2,048 tokens of 16 heads of 64 of their own 56.5 -> 59.0 us, of 16 / 4 heads of 128 76.7 -> 74.6).
 // What bounds it: a step's chain of dependent instructions (products, maximum, exponentials, products: 1.2 us with one wave a
 // SIMD), as often as the longest block has steps; two blocks a unit fill each other's gaps.  2,000 tokens of 16 / 4 heads of
-// 128, us: 116 with the tiles above, 102 here with pages and keys asked for a step ahead, 85 two steps ahead, 77 with the
+// 128, us: 116 with the tiles above, 102 here with pages and keys asked for a step ahead, 85 two steps ahead, 75 with the
 // place in the page moved on by additions (a division a page and sixteen: 40 instructions of a step's 500).
 constexpr int kSharedColumns = 64;
 
@@ -1254,6 +1258,7 @@ __global__ __launch_bounds__(256, 2) void gated_attention_shared_kernel(const Sh
   constexpr int kKeyLoads = (32 * DIM / 8 + 255) / 256, kValueLoads = (VDIM * 4 + 255) / 256;     // 16 bytes a thread each
   __shared__ __attribute__((aligned(16))) bf16_t filed_keys[2][32 * kKeyRow];
   __shared__ __attribute__((aligned(16))) bf16_t filed_values[2][VDIM * kValueRow];
+  __shared__ __attribute__((aligned(4))) unsigned char filed_infinite[2][4];     // by wave: what it was to file is not all finite
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x & (kWave - 1);
   const int col = lane & 15, grp = lane >> 4;
   const int share = a.q_heads / a.kv_heads / a.maps, columns = a.kv_heads * a.maps;
@@ -1292,9 +1297,10 @@ __global__ __launch_bounds__(256, 2) void gated_attention_shared_kernel(const Sh
   const int token = token0 + my_row / share, vector = (kvh * share + my_row % share) * a.maps + map;
   const int pos = history + my_row / share, low = low_of(pos);
   // what the block's and the wave's columns see: positions first .. last
-  const int block_low = low_of(history + row0 / share), block_last = history + (row_end - 1) / share;
+  const int block_first = history + row0 / share, block_last = history + (row_end - 1) / share;
+  const int block_low = low_of(block_first), block_low_last = low_of(block_last);
   const int wave_first = history + min(row0 + wave * 16, rows - 1) / share, wave_last = history + min(row0 + wave * 16 + 15, rows - 1) / share;
-  const int wave_low = low_of(wave_first), wave_low_last = low_of(wave_last);
+  const int wave_low = low_of(wave_first);
 
   uint4 q[DT];
   const bf16_t* qp = a.q + (static_cast<long>(token) * a.q_heads + vector) * DIM + grp * 8;
@@ -1375,7 +1381,8 @@ __global__ __launch_bounds__(256, 2) void gated_attention_shared_kernel(const Sh
   };
   stand_at(key_of(0));
   ask_pages();
-  const auto work = [&](int turn, Ahead& from, bf16_t* keys, bf16_t* values) {
+  const auto work = [&](int turn, Ahead& from, int buffer) {
+    bf16_t *keys = filed_keys[buffer], *values = filed_values[buffer];
     const int j0 = key_of(turn);
     const bool here0 = from.there[0], here1 = from.there[1];
 #pragma unroll
@@ -1384,18 +1391,34 @@ __global__ __launch_bounds__(256, 2) void gated_attention_shared_kernel(const Sh
       if (32 * DIM / 8 % 256 == 0 || at < 32 * DIM / 8)
         *reinterpret_cast<uint4*>(keys + at / (DIM / 8) * kKeyRow + at % (DIM / 8) * 8) = from.keys[i];
     }
-    const bool ragged = j0 + 31 > block_last || !here0 || !here1;
+    // (the same for the whole block: some column does not see some key of the step)
+    const bool partly = j0 + 31 > block_first || (j0 < block_low_last && j0 + 31 >= a.keep_first) || !here0 || !here1;
+    if (partly) {
+      // slots that nobody has written, or of a page that is not the request's, hold anything: zeros - and zeros for what is not
+      // finite (an exponent of all ones), which is said to the waves
+      bool finite = true;
+#pragma unroll
+      for (int i = 0; i < kValueLoads; ++i) {
+        const int eight = (i * 256 + static_cast<int>(threadIdx.x)) & 3;
+        const int left = (eight < 2 ? here0 : here1) ? block_last - (j0 + 8 * eight) + 1 : 0;
+        uint32_t words[4] = {from.values[i].x, from.values[i].y, from.values[i].z, from.values[i].w};
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+          words[w] &= (2 * w < left ? 0xffffu : 0u) | (2 * w + 1 < left ? 0xffff0000u : 0u);
+          const uint32_t kept = ((words[w] & 0x7f80u) != 0x7f80u ? 0xffffu : 0u) |
+                                ((words[w] & 0x7f800000u) != 0x7f800000u ? 0xffff0000u : 0u);
+          finite = finite & (kept == 0xffffffffu);
+          words[w] &= kept;
+        }
+        from.values[i] = make_uint4(words[0], words[1], words[2], words[3]);
+      }
+      const bool any = __any(!finite);
+      if (lane == 0) filed_infinite[buffer][wave] = any;
+    }
 #pragma unroll
     for (int i = 0; i < kValueLoads; ++i) {
       const int at = i * 256 + threadIdx.x, eight = at & 3;
-      uint4 v = from.values[i];
-      if (ragged) {        // slots that nobody has written, or of a page that is not the request's, hold anything: zeros
-        const int left = (eight < 2 ? here0 : here1) ? block_last - (j0 + 8 * eight) + 1 : 0;
-        uint32_t words[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-        for (int w = 0; w < 4; ++w) words[w] &= (2 * w < left ? 0xffffu : 0u) | (2 * w + 1 < left ? 0xffff0000u : 0u);
-        v = make_uint4(words[0], words[1], words[2], words[3]);
-      }
+      const uint4 v = from.values[i];
       if (VDIM * 4 % 256 == 0 || at < VDIM * 4) {
         // keys 8 eight .. + 3 are group 2 (eight & 1)'s of sixteen number eight / 2, the next four the group after's
         bf16_t* to = values + at / 4 * kValueRow + (eight & 1) * 16 + (eight >> 1) * 4;
@@ -1431,18 +1454,18 @@ __global__ __launch_bounds__(256, 2) void gated_attention_shared_kernel(const Sh
         }
       }
     }
-    if (j0 + 31 > wave_first || (j0 < wave_low_last && j0 + 31 >= a.keep_first) || !here0 || !here1) {
+    const auto sees = [&](int j, bool here) -> bool { return ((j >= low) | (j < a.keep_first)) & (j <= pos) & here; };
+    int infinite = 0;
+    if (partly) {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int j = j0 + 16 * (e >> 2) + 4 * grp + (e & 3);
-        const bool seen = ((j >= low) | (j < a.keep_first)) & (j <= pos) & (e < 4 ? here0 : here1);
-        s[e] = seen ? s[e] : -INFINITY;
-      }
+      for (int e = 0; e < 8; ++e)
+        s[e] = sees(j0 + 16 * (e >> 2) + 4 * grp + (e & 3), e < 4 ? here0 : here1) ? s[e] : -INFINITY;
+      infinite = __builtin_amdgcn_readfirstlane(*reinterpret_cast<const int*>(filed_infinite[buffer]));
     }
 #pragma unroll
     for (int e = 0; e < 8; ++e) top = fmaxf(top, s[e]);
     top = max_over_groups(top);
-    if (__any(top > m + kTrail)) {
+    if (__any(top > m + kTrail) || infinite != 0) {
       const float moved = fmaxf(m, top), shift = moved == -INFINITY ? 0.f : moved;
       const float correction = __builtin_amdgcn_exp2f(m - shift);
       l *= correction;
@@ -1451,6 +1474,26 @@ __global__ __launch_bounds__(256, 2) void gated_attention_shared_kernel(const Sh
 #pragma unroll
         for (int i = 0; i < 4; ++i) o[v][i] *= correction;
       m = moved;
+      if (infinite != 0) {       // the values that were filed as zeros
+#pragma unroll 1
+        for (int one = 0; one < 32; ++one) {
+          const int j = j0 + one, page = table[min(j / a.page_size, last_entry)];
+          float own = s[0];      // the key's score lies in element 4 (one / 16) + one % 4 of group one / 4 % 4
+#pragma unroll
+          for (int e = 1; e < 8; ++e) own = e == (one >> 4) * 4 + (one & 3) ? s[e] : own;
+          const float weight = __builtin_amdgcn_exp2f(__shfl(own, (one & 12) * 4 + col, kWave) - shift);
+          if (!sees(j, known(page))) continue;
+          const bf16_t* at = a.v_pages + ((page * static_cast<long>(a.kv_heads) + kvh) * VDIM + grp * 4) * a.page_size + j % a.page_size;
+#pragma unroll
+          for (int v = 0; v < VT; ++v)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              const float value = to_float(at[static_cast<long>(16 * v + i) * a.page_size]);
+              if (!(fabsf(value) < INFINITY)) o[v][i] = fmaf(weight, value, o[v][i]);
+              __builtin_amdgcn_sched_barrier(0); // (else all loads are asked for first: a third more registers in the kernel)
+            }
+        }
+      }
     }
     const float reference = m == -INFINITY ? 0.f : m;
     uint32_t high[4], rest[4];
@@ -1473,8 +1516,8 @@ __global__ __launch_bounds__(256, 2) void gated_attention_shared_kernel(const Sh
   fetch(0, even);
   fetch(1, odd);
   for (int turn = 0; turn < steps; turn += 2) {
-    work(turn, even, filed_keys[0], filed_values[0]);
-    if (turn + 1 < steps) work(turn + 1, odd, filed_keys[1], filed_values[1]);
+    work(turn, even, 0);
+    if (turn + 1 < steps) work(turn + 1, odd, 1);
   }
   l += __shfl_xor(l, 16, kWave);
   l += __shfl_xor(l, 32, kWave);

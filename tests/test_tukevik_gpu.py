@@ -443,6 +443,58 @@ def test_portions_that_share_their_keys_through_lds(hip, monkeypatch, heads, kv_
         assert ((got - want).abs() <= want.abs() * 2.0 ** -7 + 2e-3).all(), (blocks, (got - want).abs().max())
 
 
+@pytest.mark.parametrize("poison", [float("inf"), float("-inf"), float("nan")])
+@pytest.mark.parametrize("heads,kv_heads,dim,vdim,maps,options", [
+    (4, 4, 64, 64, 1, {}), (16, 4, 128, 128, 1, dict(sink=True)), (8, 2, 32, 64, 1, dict(softcap=9.0)), (4, 2, 64, 128, 2, dict(window=40)),
+    (6, 2, 64, 32, 1, dict(chunk=48)), (2, 1, 128, 64, 1, dict(window=33, keep_first=20))])
+def test_portions_that_share_their_keys_keep_clear_of_values_they_do_not_see(hip, monkeypatch, poison, heads, kv_heads, dim, vdim, maps,
+                                                                             options):
+    """One dimension of a position's value is infinite or NaN - a position inside a portion, one in its history, one among the
+    kept first keys.  Tokens that do not see it share steps and tiles with tokens that do: they have the result without
+    it in every dimension, as those that see it have in all dimensions but that one, which is not finite.  (2^-7 |out| + 2e-3 as
+    for `test_portions_that_share_their_keys_through_lds`.)"""
+    from torch_kernels import TorchKernels
+    torch.manual_seed(dim + heads)
+    page, befores, counts = 16, [0, 70], [131, 90]
+    ctx = _ctx(befores, counts)
+    ctx.seq_lens = torch.tensor(ctx.host_seq_lens, dtype=torch.int32, device=DEVICE)
+    need = [(n + page - 1) // page for n in ctx.host_seq_lens]
+    order, table = torch.randperm(sum(need)).tolist(), torch.full((2, max(need)), -1, dtype=torch.int32)
+    for r, pages in enumerate(need):
+        table[r, :pages] = torch.tensor([order.pop() for _ in range(pages)])
+    k_pages = torch.randn(sum(need), kv_heads, page, maps * dim).bfloat16()
+    v_pages = torch.randn(sum(need), kv_heads, vdim, page).bfloat16()
+    vectors, tokens = heads * maps, ctx.num_tokens
+    q = torch.randn(tokens, vectors * dim).bfloat16()
+    window, chunk, kept = options.get("window"), options.get("chunk"), options.get("keep_first", 0)
+
+    def through(kernels, device, values, c):
+        out = torch.zeros(tokens, vectors * vdim, dtype=torch.bfloat16, device=device)
+        meta = SimpleNamespace(block_table=table.to(device), rows=None, width=table.shape[1])
+        kernels.gated_attention(q.to(device), k_pages.to(device), values.to(device), None, 0, c, meta, heads, kv_heads, dim, vdim, dim ** -0.5,
+                                options.get("softcap"), chunk, window, options.get("sink", False), out, maps=maps, keep_first=kept)
+        return out.float().cpu().view(tokens, vectors, vdim)
+
+    host = SimpleNamespace(**{k: (v.cpu() if isinstance(v, torch.Tensor) else v) for k, v in vars(ctx).items()})
+    want = through(TorchKernels(), "cpu", v_pages, host)
+    reach = want.abs() * 2.0 ** -7 + 2e-3
+    monkeypatch.setattr(hip, "shared_attention_blocks", 1, raising=False)
+    for request, at in ((0, 37), (0, 100), (1, 9), (1, 64), (1, 120)):
+        values = v_pages.clone()
+        values[int(table[request, at // page]), :, 3, at % page] = poison
+        got = through(hip, DEVICE, values, ctx)
+        pos = ctx.positions.cpu()
+        sees = (ctx.seq_of_token.cpu() == request) & (pos >= at)
+        inside = torch.ones_like(sees) if window is None else pos - at < window
+        if chunk is not None:
+            inside &= pos // chunk == at // chunk
+        sees &= inside | (at < kept)
+        assert not torch.isfinite(got[sees][:, :, 3]).any(), (request, at)
+        got[sees, :, 3] = want[sees, :, 3]
+        assert torch.isfinite(got).all(), (request, at)
+        assert ((got - want).abs() <= reach).all(), (request, at)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("heads,dim,vdim,rot", [(2, 16, 12, 8), (1, 64, 32, 64), (3, 24, 40, 0), (2, 128, 128, 32), (1, 256, 256, 2)])
 def test_retention_kernel_alone(hip, dtype, heads, dim, vdim, rot):
