@@ -102,11 +102,11 @@ int akv_gated_attention_rows(const void* q, const void* k_pages, const void* v_p
 
 // The same for the first `tokens` rows of a bfloat16 step, each the only token of its request, on the matrix cores: widths and
 // pages as below.  `segments`: a bound on the segments of 16 steps of 16 keys that a token's keys touch; with more than one
-// `partial` holds tokens * q_heads * segments * (vdim + 4) floats.
+// the tokens are taken `at_once` at a time and `partial` holds at_once * q_heads * segments * (vdim + 4) floats.
 int akv_gated_attention_singles(const void* q, const void* k_pages, const void* v_pages, const void* gates, long gate_stride,
                                 int gate_at, const int* seq_of_token, const int* positions, const int* block_table,
-                                const int* table_rows, int table_width, void* out, float* partial, int segments, int tokens,
-                                int q_heads, int kv_heads, int dim, int vdim, int page_size, long num_pages, float scale,
+                                const int* table_rows, int table_width, void* out, float* partial, int segments, int at_once,
+                                int tokens, int q_heads, int kv_heads, int dim, int vdim, int page_size, long num_pages, float scale,
                                 float softcap, int chunk, int window, int sink, long out_stride, float out_scale,
                                 const float* sink_logits, int maps, int keep_first, const float* distance_bias,
                                 hipStream_t stream);

@@ -862,8 +862,8 @@ namespace {
 // steps of 16 keys at absolute positions; its four waves take four steps each and ask for all of their keys and values
 // before the first score: one trip to the block table, one to the pages.  A wave's 64 keys have one maximum; waves and
 // segments are folded in their order.  A token of one segment is finished by its block; of more, the segments' sums are left
-// in `partial` ([token][query vector][segment][vdim + 4]) and added by `gated_attention_fold_kernel`.  How a token's keys are
-// cut depends on its position alone.  Scores, maxima, weights and sums are float32; a weight enters the second product as
+// in `partial` ([token][query vector][segment][vdim + 4], as many of the step's tokens at once as the caller has room for) and
+// added by `gated_attention_fold_kernel`.  How a token's keys are cut depends on its position alone.  Scores, maxima, weights and sums are float32; a weight enters the second product as
 // three bfloat16 numbers that add up to it.
 // What bounds it: trips to memory in a row (positions, table, keys and values, then the fold's launch).  8 tokens of 2,048 keys
 // (34 MB), 16 query and 4 key heads of 128, us: 39 with a block of sixteen waves per (token, query head) in `rows`, 14 + 7 for
@@ -1163,22 +1163,25 @@ extern "C" {
 
 int akv_gated_attention_singles(const void* q, const void* k_pages, const void* v_pages, const void* gates, long gate_stride,
                                 int gate_at, const int* seq_of_token, const int* positions, const int* block_table,
-                                const int* table_rows, int table_width, void* out, float* partial, int segments, int tokens,
-                                int q_heads, int kv_heads, int dim, int vdim, int page_size, long num_pages, float scale,
+                                const int* table_rows, int table_width, void* out, float* partial, int segments, int at_once,
+                                int tokens, int q_heads, int kv_heads, int dim, int vdim, int page_size, long num_pages, float scale,
                                 float softcap, int chunk, int window, int sink, long out_stride, float out_scale,
                                 const float* sink_logits, int maps, int keep_first, const float* distance_bias,
                                 hipStream_t stream) {
   if (tokens <= 0) return 0;
-  if (page_size % 16 != 0 || maps < 1 || kv_heads <= 0 || q_heads % (kv_heads * maps) != 0 || segments < 1 || static_cast<long>(tokens) * segments > 0x7fffffffL ||
-      (segments > 1 && partial == nullptr))
+  if (page_size % 16 != 0 || maps < 1 || kv_heads <= 0 || q_heads % (kv_heads * maps) != 0 || segments < 1 || at_once < 1 ||
+      static_cast<long>(at_once) * segments > 0x7fffffffL || (segments > 1 && partial == nullptr))
     return -2;
-  const SingleArgs a{static_cast<const bf16_t*>(q), static_cast<const bf16_t*>(k_pages), static_cast<const bf16_t*>(v_pages),
+  SingleArgs a{static_cast<const bf16_t*>(q), static_cast<const bf16_t*>(k_pages), static_cast<const bf16_t*>(v_pages),
                      static_cast<const bf16_t*>(gates), seq_of_token, positions, block_table, table_rows, sink_logits,
                      distance_bias, static_cast<bf16_t*>(out), partial, gate_stride, num_pages, out_stride, scale, softcap,
                      out_scale, gate_at, table_width, q_heads, kv_heads, page_size, chunk, window, sink, maps, keep_first, segments};
   const long columns = static_cast<long>(kv_heads) * maps * ((q_heads / kv_heads / maps + 15) / 16);
   if (columns > 65535) return -2;
-  const dim3 grid(static_cast<unsigned>(static_cast<long>(tokens) * segments), static_cast<unsigned>(columns));
+  // (a launch's partial sums are folded before the next one, on the same stream, writes its own)
+  for (int first = 0; first < tokens; first += at_once) {
+    const int count = min(at_once, tokens - first);
+    const dim3 grid(static_cast<unsigned>(static_cast<long>(count) * segments), static_cast<unsigned>(columns));
 #define AKV_SINGLES(DT, VT)                                                                        \
   if (softcap > 0.f || distance_bias != nullptr)                                                   \
     gated_attention_singles_kernel<DT, VT, true><<<grid, 256, 0, stream>>>(a);                      \
@@ -1192,18 +1195,24 @@ int akv_gated_attention_singles(const void* q, const void* k_pages, const void* 
     case 256: AKV_SINGLES(DT, 16); break;  \
     default: return -2;                    \
   }
-  switch (dim) {
-    case 32: AKV_SINGLES_V(1); break;
-    case 64: AKV_SINGLES_V(2); break;
-    case 128: AKV_SINGLES_V(4); break;
-    case 256: AKV_SINGLES_V(8); break;
-    default: return -2;
-  }
+    switch (dim) {
+      case 32: AKV_SINGLES_V(1); break;
+      case 64: AKV_SINGLES_V(2); break;
+      case 128: AKV_SINGLES_V(4); break;
+      case 256: AKV_SINGLES_V(8); break;
+      default: return -2;
+    }
 #undef AKV_SINGLES_V
 #undef AKV_SINGLES
-  if (segments > 1) {
-    const long rows = static_cast<long>(tokens) * q_heads;
-    gated_attention_fold_kernel<<<static_cast<unsigned>((rows + 3) / 4), 256, 0, stream>>>(a, vdim, rows);
+    if (segments > 1) {
+      const long rows = static_cast<long>(count) * q_heads;
+      gated_attention_fold_kernel<<<static_cast<unsigned>((rows + 3) / 4), 256, 0, stream>>>(a, vdim, rows);
+    }
+    a.q += static_cast<long>(count) * q_heads * dim;
+    a.out += count * out_stride;
+    a.seq_of_token += count;
+    a.positions += count;
+    if (a.gates != nullptr) a.gates += count * gate_stride;
   }
   return AKV_LAUNCH_STATUS();
 }

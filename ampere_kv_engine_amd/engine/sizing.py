@@ -55,6 +55,7 @@ def plan_memory(spec: ModelSpec, engine_config: EngineConfig, memory_bytes: int)
              + engine_config.max_seqs * spec.vocab_size * 4 * 2                       # logits, eager and recorded
              + engine_config.max_batched_tokens * widest * element * 18               # activations of a step, two arenas
              + 2 * largest                                                            # a matrix in flight while it is packed
+             + partial_sum_bytes(model, engine_config)
              + model.rt.shared_bytes()                                                # position tables, one per kind and size
              + (512 << 20))                                                           # timing spacer, library workspaces
     left = memory_bytes - weight_bytes - second - fixed
@@ -64,6 +65,11 @@ def plan_memory(spec: ModelSpec, engine_config: EngineConfig, memory_bytes: int)
                          f"engine's buffers ({fixed / 2**30:.1f} GiB) but not a page for each of {engine_config.max_seqs} "
                          "requests")
     return MemoryPlan(weight_bytes, second, page_bytes, fixed, int(num_pages), engine_config.page_size)
+
+
+def partial_sum_bytes(model: Model, engine_config: EngineConfig) -> int:
+    """Partial results of attention whose keys are cut over blocks: they lie in a layer's arena, and a step has two arenas."""
+    return 2 * max((block.mixer.partial_sum_bytes(engine_config) for block in model.blocks), default=0)
 
 
 def page_bytes(spec: ModelSpec, dtype: str, page_size: int) -> int:

@@ -10,6 +10,7 @@ import ctypes
 import torch
 
 from ..csrc.build import ensure_parts
+from . import partial_sums
 
 _DTYPE_CODE = {torch.float32: 0, torch.bfloat16: 1}
 
@@ -792,7 +793,6 @@ class PartsKernels:
 
     # ---- attention with unit-normed queries and keys, a softcap, chunks, a sink and a gate per head ----------------------
     MAX_VALUE_DIM = 256
-    MATRIX_CORE_HEAD_DIMS = (32, 64, 128, 256)      # widths of keys and of values that the matrix-core kernels are built for
     shared_attention_blocks = None      # prompt portions of this many blocks share their keys through LDS; None: by the rule below
 
     def _shares_attention_keys(self, blocks: int, ctx, first: int) -> bool:
@@ -811,8 +811,6 @@ class PartsKernels:
         starts = ctx.host_q_start
         longest_portion = max((starts[r + 1] - starts[r] for r in range(first, ctx.num_seqs)), default=0)
         return blocks >= units and max(ctx.host_seq_lens[first:], default=0) >= 5 * longest_portion
-
-    SEGMENT_STEPS = 16      # steps of 16 keys in a segment of a single token's keys (`kSegmentSteps` of the kernel)
 
     def check_gated_attention_sizes(self, q_heads: int, kv_heads: int, dim: int, vdim: int, page_size: int) -> None:
         if q_heads % kv_heads:
@@ -931,26 +929,18 @@ class PartsKernels:
                 _long(out.shape[1]), ctypes.c_float(out_scale), _ptr(sink_logits), maps, int(keep_first), _ptr(distance_bias), self._stream())
         # keys a row can see at most (a bound that a recorded step keeps)
         span = min(x for x in (chunk, window, ctx.max_seq_len) if x is not None)
-        if (q.dtype == torch.bfloat16 and dim in self.MATRIX_CORE_HEAD_DIMS and vdim in self.MATRIX_CORE_HEAD_DIMS
-                and page_size % 16 == 0 and out.shape[1] % 4 == 0 and out_at % 4 == 0):
+        if (q.dtype == torch.bfloat16 and partial_sums.gated_on_matrix_cores(dim, vdim, page_size) and out.shape[1] % 4 == 0
+                and out_at % 4 == 0):
             # on the matrix cores: single tokens with the query heads of a key head as a tile's columns, the portions' rows,
             # which follow them, with sixteen tokens of a head
             singles = ctx.num_decode_seqs
             if singles:
-                # steps of 16 keys that a token's keys can touch: where the first of them need not be a step's first, one more
-                steps = ((span + 15) // 16 + (0 if window is None and (chunk is None or chunk % 16 == 0) else 1)
-                         + (keep_first + 15) // 16)
-                segments = (steps + self.SEGMENT_STEPS - 1) // self.SEGMENT_STEPS
-                partial = None
-                if segments > 1:
-                    arena = getattr(ctx, "arena", None)
-                    count = singles * q_heads * segments * (vdim + 4)
-                    partial = (arena.take((count,), torch.float32) if arena is not None
-                               else torch.empty(count, dtype=torch.float32, device=self.device))
+                segments, at_once, floats = partial_sums.gated_cut(singles, q_heads, vdim, span, window, chunk, keep_first)
+                partial = partial_sums.take(ctx, floats, self.device) if floats else None
                 self._check(self._parts().akv_gated_attention_singles(
                     _ptr(q), _ptr(k_pages), _ptr(v_pages), _ptr(gates), _long(gate_stride), gate_at, _ptr(ctx.seq_of_token),
                     _ptr(ctx.positions), _ptr(meta.block_table), _ptr(meta.rows), meta.width, _ptr_at(out, out_at), _ptr(partial),
-                    segments, singles, q_heads, kv_heads, dim, vdim, page_size, _long(num_pages), *tail),
+                    segments, at_once, singles, q_heads, kv_heads, dim, vdim, page_size, _long(num_pages), *tail),
                     "gated_attention of single tokens")
             starts, columns = ctx.host_q_start, q_heads // kv_heads // maps
             tiles = sum(((starts[r + 1] - starts[r]) * columns + 63) // 64 for r in range(singles, ctx.num_seqs))

@@ -179,6 +179,11 @@ class Part:
         """Bytes of weights one step reads (for roofline accounting)."""
         return 0
 
+    def partial_sum_bytes(self, engine_config) -> int:
+        """(mixers) What a step's arena holds at most for the partial results that lie between two kernels of the mixer, where
+        their size grows with the requests' lengths (what the memory plan counts beside the activations)."""
+        return 0
+
 
 class SharesProducts:
     """A mixer whose first step is one product over the layer's input (`inputs`, a `Linear` whose names are relative to

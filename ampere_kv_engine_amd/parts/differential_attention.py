@@ -17,6 +17,7 @@ from __future__ import annotations
 
 import torch
 
+from ..kernels import partial_sums
 from ..weights.spec import BIAS, TensorSpec
 from .base import PagedKV, Part, build_part, register_part
 from .linear import Linear
@@ -68,6 +69,9 @@ class DifferentialAttention(Part):
 
     def weight_bytes(self):
         return self.qkvg.weight_bytes() + self.out.weight_bytes()
+
+    def partial_sum_bytes(self, engine_config):
+        return partial_sums.gated_bytes(engine_config, self.q_heads * MAPS, self.dim, self.vdim, self.window, None, 0)
 
     def cache_request(self):
         return PagedKV(self.kv_heads, MAPS * self.dim, self.window, value_dim=self.vdim)

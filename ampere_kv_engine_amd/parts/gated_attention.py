@@ -30,6 +30,7 @@ from __future__ import annotations
 
 import torch
 
+from ..kernels import partial_sums
 from ..weights.random import register_init_law
 from ..weights.spec import BIAS, NORM, TensorSpec
 from .base import PagedKV, Part, SharesProducts, build_part, register_part
@@ -145,6 +146,9 @@ class GatedAttention(Part, SharesProducts):
 
     def weight_bytes(self):
         return self.qkvg.weight_bytes() + self.out.weight_bytes()
+
+    def partial_sum_bytes(self, engine_config):
+        return partial_sums.gated_bytes(engine_config, self.q_heads, self.dim, self.vdim, self.window, self.chunk, self.keep_first)
 
     def cache_request(self):
         return PagedKV(self.kv_heads, self.dim, self.window, value_dim=self.vdim, chunk=self.chunk,

@@ -74,6 +74,9 @@ class ParallelMixers(Part):
         if self.out_eps is not None:
             self.out_weights = [fetch(spec).to(torch.float32).contiguous() for spec in self._out_norms(prefix)]
 
+    def partial_sum_bytes(self, engine_config):
+        return sum(mixer.partial_sum_bytes(engine_config) for mixer in self.mixers)
+
     def weight_bytes(self):
         if self.shared:
             return self.inputs.weight_bytes() + self.outputs.weight_bytes()

@@ -152,6 +152,54 @@ def test_layers_share_one_position_table_and_the_memory_plan_counts_it():
     assert long.fixed_bytes - short.fixed_bytes == 4096 * 8 * 2 * 4
 
 
+@pytest.mark.parametrize("vectors,vdim,seqs", [(16, 128, 64), (64, 128, 64), (128, 256, 3), (16, 64, 1)])
+@pytest.mark.parametrize("step", [1111, 64])
+def test_partial_sums_of_growing_contexts_are_bounded_and_in_the_memory_plan(vectors, vdim, seqs, step):
+    """Single tokens of gated attention leave a segment's sums per 256 keys.  Contexts that grow to 131,072 tokens, with exact
+    lengths as eager steps have them, other activations before and behind: what the arena holds beside the first step's
+    stays within what the plan counts."""
+    from types import SimpleNamespace
+    import torch
+    from ampere_kv_engine_amd.config import EngineConfig
+    from ampere_kv_engine_amd.engine.batch import Arena
+    from ampere_kv_engine_amd.kernels import partial_sums
+    config = EngineConfig(max_seqs=seqs, max_seq_len=131072, page_size=16)
+    ctx = SimpleNamespace(arena=Arena("meta"))
+    assert ctx.arena.chunk_bytes == partial_sums.ARENA_CHUNK
+    held = None
+    for length in list(range(200, 131072, step)) + [131072]:
+        ctx.arena.reset()
+        ctx.arena.take((seqs, 40000), torch.bfloat16)
+        segments, at_once, floats = partial_sums.gated_cut(seqs, vectors, vdim, length, None, None, 0)
+        assert segments * 256 >= length > (segments - 1) * 256 and floats == (at_once * vectors * segments * (vdim + 4) if segments > 1 else 0)
+        assert at_once == 1 or floats * 4 <= partial_sums.BYTES
+        if floats:
+            assert partial_sums.take(ctx, floats, "meta").numel() >= floats
+        ctx.arena.take((seqs, 40000), torch.bfloat16)
+        now = sum(chunk.numel() for chunk in ctx.arena.chunks)
+        held = held or now
+    assert now - held <= partial_sums.gated_bytes(config, vectors, 128, vdim, None, None, 0) <= 1 << 30
+
+
+def test_plan_memory_counts_the_partial_sums_of_cut_attention():
+    """Once per arena, by the mixer with the largest; none where every key a token sees lies in one segment, or in float32, whose
+    gated attention is one kernel."""
+    from ampere_kv_engine_amd.config import EngineConfig
+    from ampere_kv_engine_amd.engine.sizing import partial_sum_bytes
+    from ampere_kv_engine_amd.engine.dry import dry_runtime
+    from ampere_kv_engine_amd.engine.model import Model
+    from ampere_kv_engine_amd.config.lirulix import LirulixConfig
+    raw = dict(architecture="Lirulix", vocab=256, width=64, norm=dict(eps=1e-6), loop=dict(start=0, stop=1, times=1), layers=[
+        dict(type="attention", mixer=dict(heads=4, kv_heads=2, dim=32, vdim=32, scale=0.2, rot=dict(
+            dims=16, base=1e4, scaling=dict(factor=4.0, original=64, fast=32.0, slow=1.0))), mlp=dict(kind="dense", ff=64))])
+    model = Model(LirulixConfig.from_dict(raw).to_model_spec(), dry_runtime(8192, 16))
+    sizes = dict(page_size=16, max_seqs=2, max_seq_len=8192)
+    assert partial_sum_bytes(model, EngineConfig(**sizes)) == 2 * (64 << 20)
+    assert partial_sum_bytes(model, EngineConfig(dtype="float32", **sizes)) == 0
+    assert partial_sum_bytes(model, EngineConfig(page_size=8, max_seqs=2, max_seq_len=8192)) == 0
+    assert partial_sum_bytes(model, EngineConfig(page_size=16, max_seqs=2, max_seq_len=128, graph_width_multiple=1)) == 0
+
+
 def test_attention_bias_adds_the_four_bias_vectors_to_every_layer():
     """`attention_bias: true` (ampere_kv/runner.py:64-66, :165 hand each projection's bias to F.linear): every layer
     expects q/k/v/o biases beside the 11 tensors, 15 L + 3 in all; the key reads back from `to_dict`."""

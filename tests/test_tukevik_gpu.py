@@ -348,6 +348,40 @@ def test_single_tokens_on_the_matrix_cores(hip, heads, kv_heads, dim, vdim, page
     assert ((last - clean[-1]).abs() <= clean[-1].abs() * 2.0 ** -7 + 1e-4).all()
 
 
+@pytest.mark.parametrize("tokens_at_once", [1, 2, 5, 9])
+@pytest.mark.parametrize("dim,vdim,window,keep_first", [(64, 128, None, 0), (128, 32, 6000, 40), (256, 256, None, 0)])
+def test_single_tokens_whose_partial_sums_do_not_fit(hip, monkeypatch, tokens_at_once, dim, vdim, window, keep_first):
+    """Nine single tokens of one to 33 segments whose partial sums would be more than a launch may leave: they are taken so many at
+    a time through one buffer, and have the bits they have in one launch."""
+    from ampere_kv_engine_amd.kernels import partial_sums
+    torch.manual_seed(3)
+    heads, kv_heads, page = 6, 2, 16
+    befores = [8300, 0, 300, 255, 256, 4095, 17, 4096, 7000]
+    ctx = _ctx(befores, [1] * 9)
+    pages = max(befores) // page + 1
+    table = torch.randperm(9 * pages, dtype=torch.int32).view(9, pages).to(DEVICE)
+    meta = SimpleNamespace(block_table=table, rows=None, width=pages)
+    k_pages = torch.randn(9 * pages, kv_heads, page, dim, device=DEVICE).bfloat16()
+    v_pages = torch.randn(9 * pages, kv_heads, vdim, page, device=DEVICE).bfloat16()
+    q, gates = torch.randn(9, heads * dim, device=DEVICE).bfloat16(), torch.randn(9, heads + 5, device=DEVICE).bfloat16()
+    cuts, cut = [], partial_sums.gated_cut
+    monkeypatch.setattr(partial_sums, "gated_cut", lambda *args: cuts.append(cut(*args)) or cuts[-1])
+
+    def attend():
+        out = torch.full((9, heads * vdim + 8), 7.0, dtype=torch.bfloat16, device=DEVICE)
+        hip.gated_attention(q, k_pages, v_pages, gates, 3, ctx, meta, heads, kv_heads, dim, vdim, 0.1, None, None, window, True, out, out_at=4,
+                            keep_first=keep_first)
+        return out
+
+    want = attend()
+    floats = heads * cuts[0][0] * (vdim + 4)
+    monkeypatch.setattr(partial_sums, "BYTES", 4 * floats * tokens_at_once)
+    asked = []
+    monkeypatch.setattr(partial_sums, "take", lambda ctx, count, device: asked.append(count) or torch.empty(count, device=device))
+    assert torch.equal(attend(), want)
+    assert [c[1] for c in cuts] == [9, tokens_at_once] and asked == [tokens_at_once * floats]
+
+
 @pytest.mark.parametrize("heads,kv_heads,dim,vdim,page,maps,eps,rot,keyed", [
     (4, 2, 64, 64, 16, 1, 1e-6, 0, False), (16, 4, 128, 128, 16, 1, None, 64, False), (2, 1, 40, 72, 8, 2, None, 16, False),
     (3, 3, 8, 8, 64, 1, 1e-5, 0, True), (1, 1, 512, 256, 32, 1, 1e-6, 512, False), (6, 2, 24, 200, 24, 1, None, 0, False)])
