@@ -36,15 +36,17 @@ int akv_qk_norm_rope_write(const void* qkv, const float* q_weight, const float* 
                            void* k_pages, void* v_pages, void* q_out, int dtype, long tokens, int q_heads,
                            int kv_heads, int dim, int page_size, long num_pages, hipStream_t stream);
 // float32 attention on the matrix cores: whether heads of `dim` and pages of `page_size` tokens are taken; into how many
-// segments of keys a step's work is cut over blocks (1: a block folds its tile's segments itself and `partial` is null; else
-// `partial` holds tokens * q_heads * segments * (dim + 4) floats) - cut where the tiles of 16 (token, head) rows, `tiles` over
-// all requests, leave compute units without a block.
+// segments of keys a row's work is cut over blocks at most (1: a block folds its tile's segments itself and `partial` is null) -
+// cut where the tiles of 16 (token, head) rows, `tiles` over all requests, leave compute units without a block.  A launch
+// takes the tokens first_token .. token_end - 1, whose tiles, numbered request by request, are first_tile .. + tiles - 1 (without
+// `partial` all of the step's); `partial` holds its tokens * q_heads * segments * (dim + 4) floats.
 int akv_attention_f32_fits(int dim, int page_size);
-int akv_attention_f32_segments(long tiles, int longest, int kv_heads);
+int akv_attention_f32_segments(long tiles, int longest, int window, int kv_heads);
 int akv_attention_f32(const float* q, const float* k_pages, const float* v_pages, const int* q_start, const int* seq_lens,
                       const int* positions, const int* block_table, const int* table_rows, int table_width, float* out,
-                      float* partial, long tokens, int seqs, long tiles, int segments, int q_heads, int kv_heads, int dim,
-                      int page_size, long num_pages, float scale, int window, hipStream_t stream);
+                      float* partial, int first_token, int token_end, int seqs, int first_tile, long tiles, int segments,
+                      int q_heads, int kv_heads, int dim, int page_size, long num_pages, float scale, int window,
+                      hipStream_t stream);
 // Products y = x W^T (+ bias): `bias` [outs] float32 or null, added to the float32 sums before they are rounded.
 int akv_linear_tiled(const void* x, int x_dtype, const void* w, int w_dtype, void* y, int y_dtype, int rows, int outs,
                      int k, const float* bias, hipStream_t stream);

@@ -10,8 +10,9 @@
 // of a block take tiles w, w + 4, w + 8, w + 12 of a segment's sixteen under ONE maximum per wave (no running rescaling
 // inside a segment), the waves' sums are folded in their order, then the segments' in theirs, always by `Fold`.  A tile or
 // segment that a row does not see folds as the identity, bit for bit.  Where a step has fewer tiles than would fill the
-// device, blocks take (tile, segment) items, leave the segments' sums in memory and a second kernel folds them - the same
-// folds, the same bits.
+// device, blocks take (tile, segment) items, leave the segments' sums in memory - counted from the first segment that a row sees,
+// so that a window bounds them - and a second kernel folds them: the same folds, the same bits.  Such a launch may take a part
+// of the step's tokens, as many as the caller has room for.
 //
 // Rows of one tile have different positions: a key that one row sees and another does not gets weight zero for the
 // other, and zero times an infinity is not zero.  So where a tile of keys is masked for some rows and its values are not
@@ -41,12 +42,13 @@ struct Args {
   const float* k_pages;
   const float* v_pages;
   float* out;
-  float* partial;                 // [tokens * q_heads][segments][dim + 4], or null: a block folds all segments of its tile
+  float* partial;                 // [(token_end - first_token) * q_heads][segments][dim + 4], or null: a block folds all of its tile's
   const int* q_start;
   const int* seq_lens;
   const int* block_table;
   const int* table_rows;
   int table_width, seqs, q_heads, kv_heads, page_size, window, segments, splits;
+  int first_tile, first_token, token_end;      // what the launch takes of the step's tokens (all of them where `partial` is null)
   long num_pages;
   float scale;
 };
@@ -87,7 +89,7 @@ __global__ __launch_bounds__(256, FEW || NT > 8 ? 1 : 2) void attention_f32_kern
   const int share = a.q_heads / a.kv_heads, kvh = blockIdx.y;
 
   // whose tile this is: tiles are numbered request by request
-  int request = -1, tile = blockIdx.x;
+  int request = -1, tile = a.first_tile + static_cast<int>(blockIdx.x);
   for (int first = 0; first < a.seqs && request < 0; first += kWave) {
     const int r = first + lane;
     const int count = r < a.seqs ? ((a.q_start[r + 1] - a.q_start[r]) * share + kRows - 1) / kRows : 0;
@@ -286,8 +288,9 @@ __global__ __launch_bounds__(256, FEW || NT > 8 ? 1 : 2) void attention_f32_kern
     }
     __syncthreads();                             // (the next segment writes LDS again)
     if (split) {
-      if (row0 + c < rows) {
-        float* at = a.partial + ((static_cast<long>(token) * a.q_heads + head) * a.segments + segment) * (kDim + 4);
+      const int of_row = segment - low / kSegment;         // (segments that the row does not see are nobody's to fold)
+      if (row0 + c < rows && token >= a.first_token && token < a.token_end && of_row >= 0 && of_row < a.segments) {
+        float* at = a.partial + ((static_cast<long>(token - a.first_token) * a.q_heads + head) * a.segments + of_row) * (kDim + 4);
 #pragma unroll
         for (int i = 0; i < kOwn; ++i)
           if (wave + 4 * i < NT) *reinterpret_cast<floats4*>(at + 16 * (wave + 4 * i) + 4 * g) = segment_sums[i];
@@ -322,15 +325,15 @@ __global__ __launch_bounds__(256) void attention_f32_fold_kernel(const Args a, c
   const int lane = threadIdx.x & 63;
   const long row = static_cast<long>(blockIdx.x) * 4 + (threadIdx.x >> 6);
   if (row >= rows) return;
-  const int pos = positions[row / a.q_heads];
+  const int pos = positions[a.first_token + row / a.q_heads];
   const int low = a.window > 0 ? max(0, pos - a.window + 1) : 0;
   const int d = min(4 * lane, dim - 4);
   const float* at = a.partial + row * a.segments * (dim + 4);
   float total_top = -INFINITY, total_weight = 0.f;
   floats4 total = {0.f, 0.f, 0.f, 0.f};
-  const int last = min(pos / kSegment, a.segments - 1);
+  const int last = min(pos / kSegment - low / kSegment, a.segments - 1);
 #pragma unroll 4
-  for (int segment = low / kSegment; segment <= last; ++segment) {
+  for (int segment = 0; segment <= last; ++segment) {
     const float* part = at + static_cast<long>(segment) * (dim + 4);
     const floats4 sums = *reinterpret_cast<const floats4*>(part + d);
     const float top = part[dim], weight = part[dim + 1];
@@ -342,7 +345,7 @@ __global__ __launch_bounds__(256) void attention_f32_fold_kernel(const Args a, c
   if (4 * lane >= dim) return;
 #pragma unroll
   for (int j = 0; j < 4; ++j) total[j] /= total_weight;
-  *reinterpret_cast<floats4*>(a.out + row * dim + d) = total;
+  *reinterpret_cast<floats4*>(a.out + (static_cast<long>(a.first_token) * a.q_heads + row) * dim + d) = total;
 }
 
 }  // namespace
@@ -353,21 +356,24 @@ extern "C" int akv_attention_f32_fits(int dim, int page_size) {
          ((nt >= 1 && nt <= 6) || nt == 8 || nt == 12 || nt == 16);
 }
 
-extern "C" int akv_attention_f32_segments(long tiles, int longest, int kv_heads) {
-  const int segments = (longest + kSegment - 1) / kSegment;
+extern "C" int akv_attention_f32_segments(long tiles, int longest, int window, int kv_heads) {
+  int segments = (longest + kSegment - 1) / kSegment;
+  // (a row's keys are `window` in a row: they touch one segment more than they fill where they begin inside one)
+  if (window > 0) segments = min(segments, (window + kSegment - 2) / kSegment + 1);
   return segments <= 1 || tiles * kv_heads >= device_facts().compute_units ? 1 : segments;
 }
 
 extern "C" int akv_attention_f32(const float* q, const float* k_pages, const float* v_pages, const int* q_start, const int* seq_lens,
                                  const int* positions, const int* block_table, const int* table_rows, int table_width, float* out,
-                                 float* partial, long tokens, int seqs, long tiles, int segments, int q_heads, int kv_heads,
-                                 int dim, int page_size, long num_pages, float scale, int window, hipStream_t stream) {
-  if (tokens <= 0 || seqs <= 0 || tiles <= 0) return 0;
-  if (!akv_attention_f32_fits(dim, page_size) || tiles > 0x7fffffffL || kv_heads > 65535 || segments < 1 ||
+                                 float* partial, int first_token, int token_end, int seqs, int first_tile, long tiles, int segments,
+                                 int q_heads, int kv_heads, int dim, int page_size, long num_pages, float scale, int window,
+                                 hipStream_t stream) {
+  if (token_end <= first_token || seqs <= 0 || tiles <= 0) return 0;
+  if (!akv_attention_f32_fits(dim, page_size) || first_token < 0 || first_tile < 0 || first_tile + tiles > 0x7fffffffL || kv_heads > 65535 || segments < 1 ||
       (partial == nullptr) != (segments == 1))
     return -2;
   Args a{q, k_pages, v_pages, out, partial, q_start, seq_lens, block_table, table_rows, table_width, seqs, q_heads, kv_heads,
-         page_size, window, segments, 1, num_pages, scale};
+         page_size, window, segments, 1, first_tile, first_token, token_end, num_pages, scale};
   if (partial != nullptr) {
     const long blocks = tiles * kv_heads, wanted = (2L * device_facts().compute_units + blocks - 1) / blocks;
     a.splits = static_cast<int>(wanted < segments ? wanted : segments);
@@ -384,7 +390,7 @@ extern "C" int akv_attention_f32(const float* q, const float* k_pages, const flo
 #undef AKV_CASE
   }
   if (partial != nullptr) {
-    const long rows = tokens * q_heads;
+    const long rows = static_cast<long>(token_end - first_token) * q_heads;
     attention_f32_fold_kernel<<<static_cast<unsigned>((rows + 3) / 4), 256, 0, stream>>>(a, positions, dim, rows);
   }
   return AKV_LAUNCH_STATUS();

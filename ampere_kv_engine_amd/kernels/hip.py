@@ -14,6 +14,7 @@ import torch
 
 from ..csrc.build import ensure_attention, ensure_built
 from ..parts.base import KernelSet
+from . import partial_sums
 from .hip_parts import PartsKernels
 
 _DTYPE_CODE = {torch.float32: 0, torch.bfloat16: 1}
@@ -1277,20 +1278,20 @@ class HipKernels(PartsKernels, KernelSet):
         starts = ctx.host_q_start
         if starts[ctx.num_seqs] != tokens or len(ctx.host_seq_lens) != ctx.num_seqs:
             raise KernelError("the step's request boundaries do not match its tokens")
-        share = q_heads // kv_heads
-        tiles = sum(((starts[r + 1] - starts[r]) * share + 15) // 16 for r in range(ctx.num_seqs))
-        segments = self.lib.akv_attention_f32_segments(ctypes.c_long(tiles), max(ctx.host_seq_lens), kv_heads)
-        partial = None
+        share, window = q_heads // kv_heads, int(window) if window is not None else 0
+        tiles = partial_sums.tiles_before(starts, ctx.num_seqs, share, tokens)
+        segments = self.lib.akv_attention_f32_segments(ctypes.c_long(tiles), max(ctx.host_seq_lens), window, kv_heads)
+        launches, partial = [(0, tokens, 0, tiles)], None
         if segments > 1:
-            arena = getattr(ctx, "arena", None)
-            count = tokens * q_heads * segments * (head_dim + 4)
-            partial = (arena.take((count,), torch.float32) if arena is not None
-                       else torch.empty(count, dtype=torch.float32, device=self.device))
-        self._check(self.lib.akv_attention_f32(
-            _ptr(q), _ptr(k_pages), _ptr(v_pages), _ptr(ctx.q_start), _ptr(ctx.seq_lens), _ptr(ctx.positions),
-            _ptr(meta.block_table), _ptr(getattr(meta, "rows", None)), meta.width, _ptr(out), _ptr(partial),
-            ctypes.c_long(tokens), ctx.num_seqs, ctypes.c_long(tiles), segments, q_heads, kv_heads, head_dim, page_size,
-            ctypes.c_long(num_pages), ctypes.c_float(scale), int(window) if window is not None else 0, self._stream()), "attention")
+            floats = q_heads * segments * (head_dim + 4)
+            launches = partial_sums.launches_of_tiles(starts, ctx.num_seqs, share, partial_sums.at_once(tokens, floats))
+            partial = partial_sums.take(ctx, max(end - first for first, end, _, _ in launches) * floats, self.device)
+        for first, end, first_tile, count in launches:     # (each folds its partial sums before the next writes its own)
+            self._check(self.lib.akv_attention_f32(
+                _ptr(q), _ptr(k_pages), _ptr(v_pages), _ptr(ctx.q_start), _ptr(ctx.seq_lens), _ptr(ctx.positions),
+                _ptr(meta.block_table), _ptr(getattr(meta, "rows", None)), meta.width, _ptr(out), _ptr(partial),
+                first, end, ctx.num_seqs, first_tile, ctypes.c_long(count), segments, q_heads, kv_heads, head_dim, page_size,
+                ctypes.c_long(num_pages), ctypes.c_float(scale), window, self._stream()), "attention")
 
     # ---- sampling ----------------------------------------------------------------------------------------
     # A row of logits is cut over several blocks where the rows are few (one block on one compute unit takes 18 us

@@ -8,11 +8,13 @@ and take 2,173.)"""
 
 from __future__ import annotations
 
+import math
+
 import torch
 
 BYTES = 256 << 20           # of one launch's sums
 ARENA_CHUNK = 64 << 20      # what an arena grows by
-SEGMENT_KEYS = 256          # `kSegmentSteps` steps of 16 keys of gated_attention.hip
+SEGMENT_KEYS = 256          # `kSegment` of attention_f32.hip, `kSegmentSteps` steps of 16 keys of gated_attention.hip
 
 
 def at_once(tokens: int, floats_a_token: int) -> int:
@@ -83,3 +85,51 @@ def gated_bytes(config, vectors: int, dim: int, vdim: int, window: int | None, c
         return 0
     span = min(x for x in (chunk, window, longest_bound(config)) if x is not None)
     return held_bytes(gated_cut(config.max_seqs, vectors, vdim, span, window, chunk, keep_first)[2])
+
+
+# ---- float32 attention (attention_f32.hip) ------------------------------------------------------------------------------
+def tile_tokens(share: int) -> int:
+    """The fewest tokens after which a tile of 16 (token, head) rows ends where a token's does (`share` query heads a key head)."""
+    return 16 // math.gcd(16, share)
+
+
+def tiles_before(starts, seqs: int, share: int, token: int) -> int:
+    """The tiles of the tokens before `token`, request by request (inside a request: a multiple of `tile_tokens`)."""
+    return sum((max(0, min(starts[r + 1], token) - starts[r]) * share + 15) // 16 for r in range(seqs))
+
+
+def launches_of_tiles(starts, seqs: int, share: int, tokens_at_once: int) -> list[tuple[int, int, int, int]]:
+    """A step's tokens as launches of about so many: (first token, token end, first tile, tiles).  A launch ends where a request
+    does or a tile of its does - after `tile_tokens` at least."""
+    whole = tile_tokens(share)
+    limit, tokens = max(tokens_at_once, whole), starts[seqs]
+    launches, first, tile = [], 0, 0
+    request = 0
+    while first < tokens:
+        end = min(first + limit, tokens)
+        while starts[request + 1] <= end and request + 1 < seqs:
+            request += 1
+        if end < tokens:        # (inside `request`, or where it starts)
+            end = starts[request] + (end - starts[request]) // whole * whole
+        upto = tiles_before(starts, seqs, share, end)
+        launches.append((first, end, tile, upto - tile))
+        first, tile = end, upto
+    return launches
+
+
+def f32_segments(longest: int, window: int | None) -> int:
+    """Segments that a token's keys touch at most (`akv_attention_f32_segments`, of steps that it cuts)."""
+    segments = (longest + SEGMENT_KEYS - 1) // SEGMENT_KEYS
+    return min(segments, (window + SEGMENT_KEYS - 2) // SEGMENT_KEYS + 1) if window else segments
+
+
+def f32_bytes(config, q_heads: int, dim: int, window: int | None) -> int:
+    """What an arena of an engine of this configuration holds at most: keys are cut only in steps whose tiles of 16 (token, head)
+    rows leave some of 256 units without a block, which is up to 4,096 rows."""
+    if config.dtype != "float32":
+        return 0
+    segments = f32_segments(longest_bound(config), window)
+    if segments <= 1:
+        return 0
+    tokens, floats = min(config.max_batched_tokens, 4096 // q_heads + 1), q_heads * segments * (dim + 4)
+    return held_bytes(min(tokens, max(at_once(tokens, floats), 16)) * floats)

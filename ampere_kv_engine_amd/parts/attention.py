@@ -9,6 +9,7 @@ Order per token: stacked q/k/v projection (with biases where the specification's
 
 from __future__ import annotations
 
+from ..kernels import partial_sums
 from .base import PagedKV, Part, build_part, register_part
 from .linear import Linear
 from .norm import RMSNorm
@@ -68,6 +69,9 @@ class Attention(Part):
 
     def weight_bytes(self):
         return self.qkv.weight_bytes() + self.out.weight_bytes()
+
+    def partial_sum_bytes(self, engine_config):
+        return partial_sums.f32_bytes(engine_config, self.q_heads, self.head_dim, self.window)
 
     # ---- cache ------------------------------------------------------------------------------------
     def cache_request(self):

@@ -181,9 +181,57 @@ def test_partial_sums_of_growing_contexts_are_bounded_and_in_the_memory_plan(vec
     assert now - held <= partial_sums.gated_bytes(config, vectors, 128, vdim, None, None, 0) <= 1 << 30
 
 
+@pytest.mark.parametrize("window", [None, 1000])
+def test_partial_sums_of_float32_portions_are_bounded_and_in_the_memory_plan(window):
+    """Float32 attention leaves a segment's sums per 256 keys where tiles of 16 (token, head) rows are few.  Portions of 200
+    tokens (16 heads over 4: 200 blocks) of a prompt of 32,768, and single tokens at every length: with a window the sums stop
+    growing at its segments, without one what the arena holds stays within what the plan counts."""
+    from types import SimpleNamespace
+    import torch
+    from ampere_kv_engine_amd.config import EngineConfig
+    from ampere_kv_engine_amd.engine.batch import Arena
+    from ampere_kv_engine_amd.kernels import partial_sums
+    config = EngineConfig(dtype="float32", max_seqs=64, max_seq_len=32768, page_size=16)
+    ctx = SimpleNamespace(arena=Arena("meta"))
+    asked = 0
+    for tokens, lengths in ((200, range(200, 32769, 200)), (1, range(1, 32769, 61))):
+        for length in lengths:
+            ctx.arena.reset()
+            segments = partial_sums.f32_segments(length, window)
+            assert window is None or segments <= 5
+            if segments > 1:
+                floats = 16 * segments * 132
+                launches = partial_sums.launches_of_tiles([0, tokens], 1, 4, partial_sums.at_once(tokens, floats))
+                largest = max(end - first for first, end, _, _ in launches) * floats
+                assert 4 * largest <= partial_sums.BYTES
+                asked = max(asked, partial_sums.take(ctx, largest, "meta").numel())
+    held = sum(chunk.numel() for chunk in ctx.arena.chunks)
+    assert 4 * asked <= held <= partial_sums.f32_bytes(config, 16, 128, window)
+    assert held <= (512 << 20 if window is None else 64 << 20)
+
+
+@pytest.mark.parametrize("share", [1, 2, 3, 4, 6, 16, 20])
+def test_launches_of_tiles_hold_whole_tiles(share):
+    """Requests of all sizes, launches of every size: the launches' tokens and tiles follow each other, and a launch's tiles are those
+    of its tokens."""
+    from ampere_kv_engine_amd.kernels import partial_sums
+    starts = [0, 1, 2, 19, 20, 100, 116, 117, 150]
+    tiles = [(first + row // share, first + min(row + 15, (end - first) * share - 1) // share)      # a tile's first and last token
+             for first, end in zip(starts, starts[1:]) for row in range(0, (end - first) * share, 16)]
+    for at_once in range(1, 160):
+        launches = partial_sums.launches_of_tiles(starts, len(starts) - 1, share, at_once)
+        token = tile = 0
+        for first, end, first_tile, count in launches:
+            assert (first, first_tile) == (token, tile) and 0 < end - first <= max(at_once, partial_sums.tile_tokens(share))
+            assert [t for t in tiles if first <= t[0] < end] == tiles[tile:tile + count]
+            assert all(t[1] < end for t in tiles[tile:tile + count])
+            token, tile = end, tile + count
+        assert (token, tile) == (150, len(tiles))
+
+
 def test_plan_memory_counts_the_partial_sums_of_cut_attention():
-    """Once per arena, by the mixer with the largest; none where every key a token sees lies in one segment, or in float32, whose
-    gated attention is one kernel."""
+    """Once per arena, by the mixer with the largest; none where every key a token sees lies in one segment, nor for float32's gated
+    attention, which is one kernel, or bfloat16's plain one, whose cut is sized by the device."""
     from ampere_kv_engine_amd.config import EngineConfig
     from ampere_kv_engine_amd.engine.sizing import partial_sum_bytes
     from ampere_kv_engine_amd.engine.dry import dry_runtime
@@ -198,6 +246,9 @@ def test_plan_memory_counts_the_partial_sums_of_cut_attention():
     assert partial_sum_bytes(model, EngineConfig(dtype="float32", **sizes)) == 0
     assert partial_sum_bytes(model, EngineConfig(page_size=8, max_seqs=2, max_seq_len=8192)) == 0
     assert partial_sum_bytes(model, EngineConfig(page_size=16, max_seqs=2, max_seq_len=128, graph_width_multiple=1)) == 0
+    qwen3 = Model(Qwen3Config.from_dict(TINY_A).to_model_spec(), dry_runtime(8192, 16))
+    assert partial_sum_bytes(qwen3, EngineConfig(**sizes)) == 0
+    assert partial_sum_bytes(qwen3, EngineConfig(dtype="float32", **sizes)) >= 2 * (64 << 20)
 
 
 def test_attention_bias_adds_the_four_bias_vectors_to_every_layer():

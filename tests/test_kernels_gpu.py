@@ -1302,6 +1302,28 @@ def test_float32_attention_gives_the_same_bits_however_a_request_is_cut(hip, ref
         assert torch.equal(out, whole[start:stop]), (start, stop)
 
 
+@pytest.mark.parametrize("q_heads,kv_heads,dim,page_size", [(8, 2, 64, 16), (6, 1, 32, 8), (5, 5, 80, 4)])
+@pytest.mark.parametrize("window", [None, 300])
+def test_float32_attention_in_several_launches(hip, monkeypatch, q_heads, kv_heads, dim, page_size, window):
+    """A step whose partial sums do not fit the bound on a launch's, in launches that end inside a portion, between requests and
+    after several of them: the bits of one launch."""
+    from ampere_kv_engine_amd.kernels import partial_sums
+    q, k_pages, v_pages, ctx, meta, _, _ = _attention_case(torch.float32, q_heads, kv_heads, dim, page_size,
+                                                           [(600, 1), (299, 1), (0, 1), (513, 40), (0, 33), (255, 3)], None, seed=43)
+    c, m = _to_cuda(ctx, meta)
+    whole = torch.empty_like(q).cuda()
+    args = (q_heads, kv_heads, dim, dim ** -0.5, window)
+    hip.attention(q.cuda(), k_pages.cuda(), v_pages.cuda(), c, m, *args, whole)
+    cuts, cut = [], partial_sums.launches_of_tiles
+    monkeypatch.setattr(partial_sums, "launches_of_tiles", lambda *a: cuts.append(cut(*a)) or cuts[-1])
+    for at_once in (1, 17, 50):
+        monkeypatch.setattr(partial_sums, "BYTES", 4 * at_once * q_heads * partial_sums.f32_segments(ctx.max_seq_len, window) * (dim + 4))
+        out = torch.full_like(whole, float("nan"))
+        hip.attention(q.cuda(), k_pages.cuda(), v_pages.cuda(), c, m, *args, out)
+        assert torch.equal(out, whole), at_once
+    assert len(cuts) == 3 and len(cuts[0]) >= len(cuts[1]) > len(cuts[2]) > 1
+
+
 @pytest.mark.parametrize("poison", [float("inf"), float("nan")])
 @pytest.mark.parametrize("window", [None, 9])
 def test_float32_attention_keeps_a_token_clear_of_keys_it_does_not_see(hip, ref, poison, window):
