@@ -35,7 +35,8 @@ int akv_qk_norm_rope_write(const void* qkv, const float* q_weight, const float* 
                            const float* table, int table_positions, const int* positions, const int* slot_map,
                            void* k_pages, void* v_pages, void* q_out, int dtype, long tokens, int q_heads,
                            int kv_heads, int dim, int page_size, long num_pages, hipStream_t stream);
-// float32 attention on the matrix cores: whether heads of `dim` and pages of `page_size` tokens are taken; into how many
+// float32 attention on the matrix cores (q, pages, out and `partial` on 16-byte boundaries, else -2): whether heads of `dim` and
+// pages of `page_size` tokens are taken; into how many
 // segments of keys a row's work is cut over blocks at most (1: a block folds its tile's segments itself and `partial` is null) -
 // cut where the tiles of 16 (token, head) rows, `tiles` over all requests, leave compute units without a block.  A launch
 // takes the tokens first_token .. token_end - 1, whose tiles, numbered request by request, are first_tile .. + tiles - 1 (without

@@ -369,8 +369,11 @@ extern "C" int akv_attention_f32(const float* q, const float* k_pages, const flo
                                  int q_heads, int kv_heads, int dim, int page_size, long num_pages, float scale, int window,
                                  hipStream_t stream) {
   if (token_end <= first_token || seqs <= 0 || tiles <= 0) return 0;
-  if (!akv_attention_f32_fits(dim, page_size) || first_token < 0 || first_tile < 0 || first_tile + tiles > 0x7fffffffL || kv_heads > 65535 || segments < 1 ||
-      (partial == nullptr) != (segments == 1))
+  if (!akv_attention_f32_fits(dim, page_size) || first_token < 0 || first_tile < 0 || first_tile + tiles > 0x7fffffffL ||
+      kv_heads > 65535 || segments < 1 ||
+      (partial == nullptr) != (segments == 1) ||
+      (reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k_pages) | reinterpret_cast<uintptr_t>(v_pages) |
+       reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(partial)) % 16 != 0)      // (what is read and written 16 bytes at a time)
     return -2;
   Args a{q, k_pages, v_pages, out, partial, q_start, seq_lens, block_table, table_rows, table_width, seqs, q_heads, kv_heads,
          page_size, window, segments, 1, first_tile, first_token, token_end, num_pages, scale};

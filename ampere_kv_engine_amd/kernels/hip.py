@@ -1257,8 +1257,8 @@ class HipKernels(PartsKernels, KernelSet):
         if encode_portions is not None:
             encode_portions()
         self._dense(ctx.positions, "positions", torch.int32, (tokens,))
-        if (q.dtype == torch.float32 and not self.one_wave_per_head
-                and self.lib.akv_attention_f32_fits(head_dim, page_size)):
+        if (q.dtype == torch.float32 and not self.one_wave_per_head and self.lib.akv_attention_f32_fits(head_dim, page_size)
+                and (q.data_ptr() | k_pages.data_ptr() | v_pages.data_ptr() | out.data_ptr()) % 16 == 0):
             self._attention_f32(q, k_pages, v_pages, ctx, meta, q_heads, kv_heads, head_dim, scale, window, out, page_size, num_pages)
             return
         self._dense(ctx.seq_of_token, "seq_of_token", torch.int32, (tokens,))
@@ -1270,7 +1270,7 @@ class HipKernels(PartsKernels, KernelSet):
 
     def _attention_f32(self, q, k_pages, v_pages, ctx, meta, q_heads, kv_heads, head_dim, scale, window, out, page_size, num_pages):
         """float32 attention on the matrix cores (`csrc/attention_f32.hip`), single tokens and portions alike; what it does
-        not take - heads or pages of other sizes - goes to the plain kernel, a wave per (token, head).  Both give a token
+        not take - heads or pages of other sizes, operands off a 16-byte boundary - goes to the plain kernel, a wave per (token, head).  Both give a token
         the same bits whatever step it comes in."""
         tokens = q.shape[0]
         self._dense(ctx.q_start, "q_start", torch.int32, (ctx.num_seqs + 1,))

@@ -1324,6 +1324,22 @@ def test_float32_attention_in_several_launches(hip, monkeypatch, q_heads, kv_hea
     assert len(cuts) == 3 and len(cuts[0]) >= len(cuts[1]) > len(cuts[2]) > 1
 
 
+@pytest.mark.parametrize("askew", ["q", "k_pages", "v_pages", "out"])
+@pytest.mark.parametrize("portions", [[(40, 1), (3, 1)], [(0, 33), (9, 5)]])
+def test_float32_attention_of_operands_that_are_not_aligned(hip, ref, askew, portions):
+    """A tensor that begins one element behind a 16-byte boundary, as a view into a larger one may, goes to the plain kernel."""
+    q, k_pages, v_pages, ctx, meta, _, _ = _attention_case(torch.float32, 8, 2, 64, 16, portions, None, seed=44)
+    want = torch.empty_like(q)
+    ref.attention(q, k_pages, v_pages, ctx, meta, 8, 2, 64, 0.125, None, want)
+    given = dict(q=q.cuda(), k_pages=k_pages.cuda(), v_pages=v_pages.cuda(), out=torch.empty_like(q).cuda())
+    room = torch.empty(given[askew].numel() + 1, device="cuda")
+    given[askew] = room[1:].view(given[askew].shape).copy_(given[askew])
+    assert given[askew].data_ptr() % 16 == 4
+    c, m = _to_cuda(ctx, meta)
+    hip.attention(given["q"], given["k_pages"], given["v_pages"], c, m, 8, 2, 64, 0.125, None, given["out"])
+    torch.testing.assert_close(given["out"].cpu(), want, **tol(torch.float32))
+
+
 @pytest.mark.parametrize("poison", [float("inf"), float("nan")])
 @pytest.mark.parametrize("window", [None, 9])
 def test_float32_attention_keeps_a_token_clear_of_keys_it_does_not_see(hip, ref, poison, window):
