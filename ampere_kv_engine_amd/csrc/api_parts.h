@@ -100,8 +100,8 @@ int akv_gated_attention_rows(const void* q, const void* k_pages, const void* v_p
                              const float* sink_logits, int maps, int keep_first, const float* distance_bias,
                              hipStream_t stream);
 
-// The same for the first `tokens` rows of a bfloat16 step, each the only token of its request, on the matrix cores: widths and
-// pages as below.  `segments`: a bound on the segments of 16 steps of 16 keys that a token's keys touch; with more than one
+// The same for the first `tokens` rows of a bfloat16 step, each the only token of its request, on the matrix cores: widths, pages
+// and alignment as below.  `segments`: a bound on the segments of 16 steps of 16 keys that a token's keys touch; with more than one
 // the tokens are taken `at_once` at a time and `partial` holds at_once * q_heads * segments * (vdim + 4) floats.
 int akv_gated_attention_singles(const void* q, const void* k_pages, const void* v_pages, const void* gates, long gate_stride,
                                 int gate_at, const int* seq_of_token, const int* positions, const int* block_table,
@@ -112,7 +112,7 @@ int akv_gated_attention_singles(const void* q, const void* k_pages, const void* 
                                 hipStream_t stream);
 
 // The same for rows first_row .. tokens - 1 of a bfloat16 step, on the matrix cores: keys and values 32, 64, 128 or 256
-// wide, pages of a multiple of 16 tokens (-2 otherwise); a request's rows follow each other in the order of their positions.
+// wide, pages of a multiple of 16 tokens, q and pages on 16-byte boundaries, out on 8-byte ones (-2 otherwise); a request's rows follow each other in the order of their positions.
 int akv_gated_attention_tiles(const void* q, const void* k_pages, const void* v_pages, const void* gates, long gate_stride,
                               int gate_at, const int* seq_of_token, const int* q_start, const int* positions,
                               const int* block_table, const int* table_rows, int table_width, void* out, int first_row,

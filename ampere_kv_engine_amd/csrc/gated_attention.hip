@@ -510,6 +510,12 @@ __device__ __forceinline__ short4_t load_bf16x4(const bf16_t* p) {
   return __builtin_bit_cast(short4_t, *reinterpret_cast<const uint2*>(p));
 }
 
+// What the matrix-core kernels read 16 bytes and write 8 bytes at a time.
+inline bool aligned_for_tiles(const void* q, const void* k_pages, const void* v_pages, const void* out, long out_stride) {
+  return ((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k_pages) | reinterpret_cast<uintptr_t>(v_pages)) % 16 == 0) &&
+         reinterpret_cast<uintptr_t>(out) % 8 == 0 && out_stride % 4 == 0;
+}
+
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
 
 __device__ __forceinline__ uint4 load_bf16x8(const bf16_t* p) { return *reinterpret_cast<const uint4*>(p); }
@@ -718,6 +724,7 @@ int akv_gated_attention_tiles(const void* q, const void* k_pages, const void* v_
                               hipStream_t stream) {
   if (tokens <= first_row) return 0;
   if (page_size % 16 != 0 || q_heads % kv_heads != 0 || maps < 1) return -2;
+  if (!aligned_for_tiles(q, k_pages, v_pages, out, out_stride)) return -2;
   const long items = static_cast<long>((tokens - first_row + 15) / 16) * q_heads;
   const unsigned grid = static_cast<unsigned>(((tokens - first_row + 15) / 16 + kXcds - 1) / kXcds * kXcds * q_heads);
   const int waves = vdim > 128 ? 2 : 4;       // (their shares must fit into 64 KB of LDS)
@@ -1177,6 +1184,7 @@ int akv_gated_attention_singles(const void* q, const void* k_pages, const void* 
                      distance_bias, static_cast<bf16_t*>(out), partial, gate_stride, num_pages, out_stride, scale, softcap,
                      out_scale, gate_at, table_width, q_heads, kv_heads, page_size, chunk, window, sink, maps, keep_first, segments};
   const long columns = static_cast<long>(kv_heads) * maps * ((q_heads / kv_heads / maps + 15) / 16);
+  if (!aligned_for_tiles(q, k_pages, v_pages, out, out_stride)) return -2;
   if (columns > 65535) return -2;
   // (a launch's partial sums are folded before the next one, on the same stream, writes its own)
   for (int first = 0; first < tokens; first += at_once) {
@@ -1555,6 +1563,7 @@ extern "C" int akv_gated_attention_shared(const void* q, const void* k_pages, co
                                           const float* distance_bias, hipStream_t stream) {
   if (seqs <= first_seq || tiles <= 0) return 0;
   if (page_size % 16 != 0 || maps < 1 || kv_heads <= 0 || q_heads % (kv_heads * maps) != 0) return -2;
+  if (!aligned_for_tiles(q, k_pages, v_pages, out, out_stride)) return -2;
   const long blocks = static_cast<long>(tiles) * kv_heads * maps;
   if (blocks > 0x7fffffffL) return -2;
   const SharedArgs a{static_cast<const bf16_t*>(q), static_cast<const bf16_t*>(k_pages), static_cast<const bf16_t*>(v_pages),

@@ -929,8 +929,10 @@ class PartsKernels:
                 _long(out.shape[1]), ctypes.c_float(out_scale), _ptr(sink_logits), maps, int(keep_first), _ptr(distance_bias), self._stream())
         # keys a row can see at most (a bound that a recorded step keeps)
         span = min(x for x in (chunk, window, ctx.max_seq_len) if x is not None)
-        if (q.dtype == torch.bfloat16 and partial_sums.gated_on_matrix_cores(dim, vdim, page_size) and out.shape[1] % 4 == 0
-                and out_at % 4 == 0):
+        # (the matrix-core kernels read queries and pages 16 bytes at a time and write 8)
+        aligned = ((q.data_ptr() | k_pages.data_ptr() | v_pages.data_ptr()) % 16 == 0 and out.data_ptr() % 8 == 0
+                   and out.shape[1] % 4 == 0 and out_at % 4 == 0)
+        if q.dtype == torch.bfloat16 and aligned and partial_sums.gated_on_matrix_cores(dim, vdim, page_size):
             # on the matrix cores: single tokens with the query heads of a key head as a tile's columns, the portions' rows,
             # which follow them, with sixteen tokens of a head
             singles = ctx.num_decode_seqs

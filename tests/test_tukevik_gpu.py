@@ -348,6 +348,39 @@ def test_single_tokens_on_the_matrix_cores(hip, heads, kv_heads, dim, vdim, page
     assert ((last - clean[-1]).abs() <= clean[-1].abs() * 2.0 ** -7 + 1e-4).all()
 
 
+@pytest.mark.parametrize("askew", ["q", "k_pages", "v_pages", "out"])
+@pytest.mark.parametrize("counts", [[1, 1], [70, 3]])
+def test_gated_attention_of_operands_that_are_not_aligned(hip, monkeypatch, askew, counts):
+    """A tensor that begins one element behind the boundary that wide accesses need, as a view into a larger one may, goes to the
+    plain kernel - single tokens and portions, whichever matrix-core kernel they would go to.  (2^-7 |out| + 2e-3 as above.)"""
+    from torch_kernels import TorchKernels
+    torch.manual_seed(9)
+    heads, kv_heads, dim, vdim, page = 4, 2, 64, 32, 16
+    ctx = _ctx([300, 17], counts)
+    ctx.seq_lens = torch.tensor(ctx.host_seq_lens, dtype=torch.int32, device=DEVICE)
+    pages = max(ctx.host_seq_lens) // page + 1
+    table = torch.randperm(2 * pages, dtype=torch.int32).view(2, pages)
+    given = dict(q=torch.randn(ctx.num_tokens, heads * dim), k_pages=torch.randn(2 * pages, kv_heads, page, dim),
+                 v_pages=torch.randn(2 * pages, kv_heads, vdim, page), out=torch.zeros(ctx.num_tokens, heads * vdim))
+    given = {name: t.bfloat16() for name, t in given.items()}
+
+    def attend(kernels, device, c, q, k_pages, v_pages, out):
+        meta = SimpleNamespace(block_table=table.to(device), rows=None, width=pages)
+        kernels.gated_attention(q, k_pages, v_pages, None, 0, c, meta, heads, kv_heads, dim, vdim, 0.1, None, None, None, True, out)
+        return out.float().cpu()
+
+    host = SimpleNamespace(**{k: (v.cpu() if isinstance(v, torch.Tensor) else v) for k, v in vars(ctx).items()})
+    want = attend(TorchKernels(), "cpu", host, **given)
+    given = {name: t.to(DEVICE) for name, t in given.items()}
+    room = torch.empty(given[askew].numel() + 1, dtype=torch.bfloat16, device=DEVICE)
+    given[askew] = room[1:].view(given[askew].shape).copy_(given[askew])
+    assert given[askew].data_ptr() % 16 == 2
+    for blocks in (1, 1 << 30):
+        monkeypatch.setattr(hip, "shared_attention_blocks", blocks, raising=False)
+        given["out"].zero_()
+        assert ((attend(hip, DEVICE, ctx, **given) - want).abs() <= want.abs() * 2.0 ** -7 + 2e-3).all()
+
+
 @pytest.mark.parametrize("tokens_at_once", [1, 2, 5, 9])
 @pytest.mark.parametrize("dim,vdim,window,keep_first", [(64, 128, None, 0), (128, 32, 6000, 40), (256, 256, None, 0)])
 def test_single_tokens_whose_partial_sums_do_not_fit(hip, monkeypatch, tokens_at_once, dim, vdim, window, keep_first):
