@@ -28,6 +28,40 @@ def _ptr_at(t, column: int):
     return ctypes.c_void_p(t.data_ptr() + int(column) * t.element_size())
 
 
+def shared_blocks(portions, vectors: int, kv_heads: int, maps: int) -> int:
+    """Blocks of 64 (token, query vector) columns that prompt portions of (tokens, tokens held after the step) make."""
+    share = vectors // kv_heads // maps
+    return sum((count * share + 63) // 64 for count, _ in portions) * kv_heads * maps
+
+
+def shares_keys(units: int, portions, vectors: int, kv_heads: int, maps: int, dim: int, vdim: int, window, chunk) -> bool:
+    """Whether prompt portions are faster where blocks of 64 columns share their keys through LDS (`gated_attention_shared`) than
+    where a block is a tile of 16 tokens of a vector whose four waves take the keys in turn (`gated_attention_tiles`).  A
+    shared block takes steps of 32 keys in a chain of its own, `step` us each; two blocks a unit fill each other's gaps, so
+    the longest block counts, or all steps over two blocks a unit.  Tiles are bound by their number of steps of 16 keys, `tile`
+    ns each over 256 units, and by the longest one's chain.  Fitted to and checked against, us, shared / tiles, 256 units:
+      heads of 128 / 128: 16 over 4, 1,024 tokens 39 / 38, 2,048 75 / 116, 1,024 after 6,000 233 / 403, after 8,000 with a window of
+        1,024 41 / 74, 8 x 128 10 / 15, 900 beside 124 after 6,000 205 / 175; 32 over 8, 512 22 / 25, after 2,048 89 / 153;
+      64 / 64: 16 over 16, 1,024 31 / 28, after 3,000 109 / 117; 16 over 4, 1,280 38 / 32, 2,048 59 / 68, 1,024 after 4,000 134 / 142;
+      64 / 128 in two maps, 16 over 8, a window of 1,024: 512 21 / 19, 512 after 6,000 40 / 50;
+      32 / 32: 16 over 4, 1,024 30 / 17, 1,280 36 / 25, 2,048 55 / 49, 1,024 after 4,000 129 / 111; 32 over 8, 2,048 55 / 95."""
+    reach = min((x for x in (window, chunk) if x is not None), default=1 << 30)
+    share = vectors // kv_heads // maps
+    tile, step = 0.21 + 0.0024 * dim + 0.0022 * vdim, 0.72 + 0.0018 * dim + 0.0017 * vdim
+    longest = tiles = tile_steps = steps = 0.0
+    for count, length in portions:
+        before = length - count
+        growing = min(max(reach - before, 0), count)       # tokens that see more keys than the one before them
+        keys = (growing * (before + growing / 2) + (count - growing) * reach) / count
+        longest = max(longest, min(length, reach))
+        of_tile = count / 16 * vectors
+        tiles += of_tile
+        tile_steps += of_tile * (keys / 16 + 1)
+        steps += (count * share + 63) // 64 * kv_heads * maps * (keys / 32 + 1)
+    by_tiles = 6 + max((6 * tiles + tile_steps) * tile / 1000 * 256 / units, longest / 64 * 2.2 * tile)
+    return 5 + step * max(longest / 32, steps / (2 * units)) < by_tiles
+
+
 class PartsKernels:
     """Mixed into `HipKernels` (which provides `_dense`, `_check`, `_stream`, `device`)."""
 
@@ -793,24 +827,28 @@ class PartsKernels:
 
     # ---- attention with unit-normed queries and keys, a softcap, chunks, a sink and a gate per head ----------------------
     MAX_VALUE_DIM = 256
-    shared_attention_blocks = None      # prompt portions of this many blocks share their keys through LDS; None: by the rule below
+    shared_attention_blocks = None      # prompt portions of this many blocks share their keys through LDS; None: by `shares_keys`
+    FEW_TOKENS = 512                    # (what `EngineConfig.record_max_tokens` allows a recorded step by default)
 
-    def _shares_attention_keys(self, blocks: int, ctx, first: int) -> bool:
-        """Whether prompt portions of `blocks` blocks of 64 (token, query vector) columns go to the kernel that shares keys
-        through LDS.  Each of its blocks walks all of its columns' keys alone, where a tile of the other kernel has four waves
-        for them; it pays where there are more blocks than compute units, or as many and mostly history to read.  Measured, us,
-        shared / tiles: 16 query and 4 key heads of 128, 2,048 tokens (512 blocks) 77 / 116 inside a step, 500 x 4 (512) 29 / 46,
-        1,024 after 6,000 (256) 242 / 403, 512 after 6,000 (128) 223 / 199; 32 / 8 heads, 2,048 tokens (1,024) 89 / 227, 800 (400)
-        34 / 50, 512 after 2,048 (256) 93 / 155, 512 (256) 23 / 25, 400 (200) 20 / 19; 16 heads of 64 of their own, 1,024 (256)
-        31 / 28, 2,048 (512) 59 / 81; two maps of 64 over a window of 1,024, 512 (256) 22 / 20, 800 (400) 31 / 41."""
-        if self.shared_attention_blocks is not None:
-            return blocks >= self.shared_attention_blocks
-        units = self.compute_units
-        if 4 * blocks >= 5 * units:
-            return True
-        starts = ctx.host_q_start
-        longest_portion = max((starts[r + 1] - starts[r] for r in range(first, ctx.num_seqs)), default=0)
-        return blocks >= units and max(ctx.host_seq_lens[first:], default=0) >= 5 * longest_portion
+    def _shares_attention_keys(self, ctx, first: int, heads: tuple[int, int, int, int, int], window, chunk) -> tuple[int, bool]:
+        """The blocks that the portions of a step, requests `first` on, make in the kernel that shares keys, and whether they go
+        there.  It takes enough blocks for every unit, and then what `shares_keys` says.  In steps of few tokens - those that may be
+        recorded, where a request's length is only a bound - portions count as having as much before them as they bring,
+        recorded or not, so that a step goes the same way either time.  (Kept with the step for its other layers.)"""
+        starts, lengths = ctx.host_q_start[first:ctx.num_seqs + 1], ctx.host_seq_lens[first:ctx.num_seqs]
+        choices = ctx.__dict__.setdefault("shared_attention", {})
+        key = (tuple(starts), tuple(lengths), heads, window, chunk, self.shared_attention_blocks)
+        if key not in choices:
+            few = starts[-1] <= self.FEW_TOKENS
+            portions = [(end - start, 2 * (end - start) if few else length)
+                        for start, end, length in zip(starts, starts[1:], lengths)]
+            blocks = shared_blocks(portions, *heads[:3])
+            if self.shared_attention_blocks is not None:
+                shared = blocks >= self.shared_attention_blocks
+            else:
+                shared = blocks >= self.compute_units and shares_keys(self.compute_units, portions, *heads, window, chunk)
+            choices[key] = blocks, shared
+        return choices[key]
 
     def check_gated_attention_sizes(self, q_heads: int, kv_heads: int, dim: int, vdim: int, page_size: int) -> None:
         if q_heads % kv_heads:
@@ -944,14 +982,15 @@ class PartsKernels:
                     _ptr(ctx.positions), _ptr(meta.block_table), _ptr(meta.rows), meta.width, _ptr_at(out, out_at), _ptr(partial),
                     segments, at_once, singles, q_heads, kv_heads, dim, vdim, page_size, _long(num_pages), *tail),
                     "gated_attention of single tokens")
-            starts, columns = ctx.host_q_start, q_heads // kv_heads // maps
-            tiles = sum(((starts[r + 1] - starts[r]) * columns + 63) // 64 for r in range(singles, ctx.num_seqs))
-            if dim <= 128 and vdim <= 128 and self._shares_attention_keys(tiles * kv_heads * maps, ctx, singles):
+            if singles == ctx.num_seqs:
+                return
+            blocks, shared = self._shares_attention_keys(ctx, singles, (q_heads, kv_heads, maps, dim, vdim), window, chunk)
+            if shared and dim <= 128 and vdim <= 128:
                 self._dense(ctx.seq_lens, "seq_lens", torch.int32, (ctx.num_seqs,))
                 self._check(self._parts().akv_gated_attention_shared(
                     _ptr(q), _ptr(k_pages), _ptr(v_pages), _ptr(gates), _long(gate_stride), gate_at, _ptr(ctx.q_start),
                     _ptr(ctx.seq_lens), _ptr(meta.block_table), _ptr(meta.rows), meta.width, _ptr_at(out, out_at), singles, ctx.num_seqs,
-                    tiles, q_heads, kv_heads, dim, vdim, page_size, _long(num_pages), *tail), "gated_attention of shared keys")
+                    blocks // (kv_heads * maps), q_heads, kv_heads, dim, vdim, page_size, _long(num_pages), *tail), "gated_attention of shared keys")
                 return
             self._check(self._parts().akv_gated_attention_tiles(
                 _ptr(q), _ptr(k_pages), _ptr(v_pages), _ptr(gates), _long(gate_stride), gate_at, _ptr(ctx.seq_of_token),

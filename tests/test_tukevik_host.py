@@ -172,3 +172,62 @@ def test_a_far_key_at_the_chunks_edges_decides_the_output():
     out = plain.chunked_attention(h, w, m, 1e-6)
     assert out[15, 0] > 0.9 and out[9, 0] > 0.9           # seen from the chunk's own last position, and from nearby
     assert out[16, 0].abs() < 1e-6 and out[7, 0].abs() < 1e-6      # not from the next chunk, nor from before
+
+
+# us in the kernel that shares keys through LDS and in the one whose waves fetch their own, on 256 compute units:
+# (heads, kv heads, maps, key width, value width, window), [(tokens, tokens before them)], shared, tiles
+PORTIONS_MEASURED = [
+    ((16, 4, 1, 128, 128, None), [(1024, 0)], 39, 38), ((16, 4, 1, 128, 128, None), [(2048, 0)], 75, 116),
+    ((16, 4, 1, 128, 128, None), [(1024, 6000)], 233, 403), ((16, 4, 1, 128, 128, 1024), [(1024, 8000)], 41, 74),
+    ((16, 4, 1, 128, 128, None), [(128, 0)] * 8, 10, 15), ((16, 4, 1, 128, 128, None), [(900, 0), (124, 6000)], 205, 175),
+    ((32, 8, 1, 128, 128, None), [(512, 0)], 22, 25), ((32, 8, 1, 128, 128, None), [(512, 2048)], 89, 153),
+    ((64, 8, 1, 128, 128, None), [(280, 0)], 16, 22), ((16, 16, 1, 64, 64, None), [(1024, 0)], 31, 28),
+    ((16, 16, 1, 64, 64, None), [(256, 0)] * 4, 12, 14), ((16, 4, 1, 64, 64, None), [(1280, 0)], 38, 32),
+    ((16, 4, 1, 64, 64, None), [(2048, 0)], 59, 68), ((16, 4, 1, 64, 64, None), [(1024, 4000)], 134, 142),
+    ((16, 8, 2, 64, 128, 1024), [(512, 6000)], 40, 50), ((16, 4, 1, 32, 32, None), [(1024, 0)], 30, 17),
+    ((16, 4, 1, 32, 32, None), [(1280, 0)], 36, 25), ((16, 4, 1, 32, 32, None), [(2048, 0)], 55, 49),
+    ((16, 4, 1, 32, 32, None), [(1024, 4000)], 129, 111), ((32, 8, 1, 32, 32, None), [(2048, 0)], 55, 95),
+    ((16, 4, 1, 32, 128, None), [(1280, 0)], 43, 39), ((16, 16, 1, 128, 64, None), [(1280, 0)], 42.6, 44.5)]
+
+
+@pytest.mark.parametrize("sizes,portions,shared,tiles", PORTIONS_MEASURED)
+def test_portions_go_to_the_faster_attention_kernel(sizes, portions, shared, tiles):
+    """Whichever kernel the rule takes is within a twentieth of the faster one's measured time."""
+    from ampere_kv_engine_amd.kernels.hip_parts import shared_blocks, shares_keys
+    heads, kv_heads, maps, dim, vdim, window = sizes
+    held = [(count, before + count) for count, before in portions]
+    assert shared_blocks(held, heads * maps, kv_heads, maps) >= 256
+    chosen = shared if shares_keys(256, held, heads * maps, kv_heads, maps, dim, vdim, window, None) else tiles
+    assert chosen <= 1.05 * min(shared, tiles)
+
+
+@pytest.mark.parametrize("vectors,kv_heads,maps,dim,vdim", [(64, 8, 1, 128, 128), (32, 8, 1, 128, 128), (64, 64, 1, 32, 32), (32, 8, 2, 64, 128)])
+@pytest.mark.parametrize("window", [None, 40, 1024])
+def test_a_recorded_step_goes_where_the_same_step_goes_unrecorded(vectors, kv_heads, maps, dim, vdim, window):
+    """Steps of the sizes that may be recorded: their requests' lengths - as they are, or bounds - do not turn the choice.  Larger
+    steps go by their lengths."""
+    from types import SimpleNamespace
+    from ampere_kv_engine_amd.config import EngineConfig
+    from ampere_kv_engine_amd.kernels.hip_parts import PartsKernels
+    kernels = PartsKernels.__new__(PartsKernels)
+    kernels.compute_units = 256
+    assert kernels.FEW_TOKENS == EngineConfig().record_max_tokens
+    heads, seen = (vectors, kv_heads, maps, dim, vdim), set()
+    for singles, counts in ((0, [512]), (0, [280]), (3, [300]), (1, [200, 311]), (2, [64] * 7)):
+        starts = [0]
+        for count in [1] * singles + counts:
+            starts.append(starts[-1] + count)
+        choices = set()
+        for before in (0, 37, 2048, 30000):
+            lengths = [before + 1] * singles + [before + count for count in counts]
+            for bound in (None, 2048, 65536):
+                ctx = SimpleNamespace(num_seqs=len(lengths), host_q_start=starts,
+                                      host_seq_lens=lengths if bound is None else [65536] * singles + [bound] * len(counts))
+                choices.add(kernels._shares_attention_keys(ctx, singles, heads, window, None))
+                assert kernels._shares_attention_keys(ctx, singles, heads, window, None) in choices
+        assert len(choices) == 1
+        seen |= choices
+    assert all(blocks >= 256 for blocks, shared in seen if shared)
+    fresh, late = (kernels._shares_attention_keys(SimpleNamespace(num_seqs=1, host_q_start=[0, 1024], host_seq_lens=[length]), 0,
+                                                  (16, 4, 1, 128, 128), None, None) for length in (1024, 7024))
+    assert fresh == (256, False) and late == (256, True)
