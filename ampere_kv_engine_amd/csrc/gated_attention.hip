@@ -875,7 +875,9 @@ namespace {
 // What bounds it: trips to memory in a row (positions, table, keys and values, then the fold's launch).  8 tokens of 2,048 keys
 // (34 MB), 16 query and 4 key heads of 128, us: 39 with a block of sixteen waves per (token, query head) in `rows`, 14 + 7 for
 // the fold here; two maps of 64 over a window of 1,024: 26.5 -> 12 + 5.  (With the loads behind tests, which the compiler
-// waits for one by one, and the softcap's and the bias's code in every kernel: 33.)
+// waits for one by one, and the softcap's and the bias's code in every kernel: 33.)  Where tokens and key heads are many, blocks
+// beside each other on a unit hide the trips: up to four, where registers allow them (64 tokens of 2,048 keys, 16 heads of 64 of
+// their own: 119 us, 139 with two at most).
 struct Steps {
   int lowest, first, kept, all;      // the window's first key; its step, the steps of the kept first keys, all steps
   __device__ __forceinline__ Steps(int pos, int window, int chunk, int keep_first) {
@@ -923,7 +925,7 @@ __device__ __forceinline__ float sink_of(const SingleArgs& a, int vector) {
 
 // SHAPED: scores have a softcap or a distance bias (their code, in every kernel, would be most of what a block fetches).
 template <int DT, int VT, bool SHAPED>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) void gated_attention_singles_kernel(const SingleArgs a) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 4))) void gated_attention_singles_kernel(const SingleArgs a) {
   constexpr int DIM = 32 * DT, VDIM = 16 * VT, kOwn = (VT + 3) / 4;      // tiles of values whose totals a wave keeps
   __shared__ float4_t sums_of[4][VT][kWave];
   __shared__ float top_of[4][16], weight_of[4][16];
