@@ -970,11 +970,18 @@ class PartsKernels:
         # (the matrix-core kernels read queries and pages 16 bytes at a time and write 8)
         aligned = ((q.data_ptr() | k_pages.data_ptr() | v_pages.data_ptr()) % 16 == 0 and out.data_ptr() % 8 == 0
                    and out.shape[1] % 4 == 0 and out_at % 4 == 0)
+        singles = tokens
         if q.dtype == torch.bfloat16 and aligned and partial_sums.gated_on_matrix_cores(dim, vdim, page_size):
             # on the matrix cores: single tokens with the query heads of a key head as a tile's columns, the portions' rows,
             # which follow them, with sixteen tokens of a head
             singles = ctx.num_decode_seqs
-            if singles:
+            # Many single tokens whose heads have keys of their own, values of 256: a tile has one column, a block a unit nearly to
+            # itself, and the waves of the plain kernel are faster.  (tokens x vectors = 512, matrix cores / plain, us: 128 / 256
+            # wide, 256 keys 30 / 38, 300 53 / 49, 600 79 / 59, 2,048 240 / 198; 2,048 of them: 256 117 / 100, 300 212 / 122, 2,048
+            # 880 / 755.  256 of 256 / 256: 256 20 / 37, 600 52 / 56, 2,048 165 / 145.  128 / 128, 1,024 of them: 300 43 / 41,
+            # 2,048 207 / 274.)
+            plain = vdim == 256 and q_heads == kv_heads * maps and singles * q_heads >= 2 * self.compute_units
+            if singles and not plain:
                 segments, at_once, floats = partial_sums.gated_cut(singles, q_heads, vdim, span, window, chunk, keep_first)
                 partial = partial_sums.take(ctx, floats, self.device) if floats else None
                 self._check(self._parts().akv_gated_attention_singles(
@@ -982,29 +989,37 @@ class PartsKernels:
                     _ptr(ctx.positions), _ptr(meta.block_table), _ptr(meta.rows), meta.width, _ptr_at(out, out_at), _ptr(partial),
                     segments, at_once, singles, q_heads, kv_heads, dim, vdim, page_size, _long(num_pages), *tail),
                     "gated_attention of single tokens")
-            if singles == ctx.num_seqs:
-                return
-            blocks, shared = self._shares_attention_keys(ctx, singles, (q_heads, kv_heads, maps, dim, vdim), window, chunk)
-            if shared and dim <= 128 and vdim <= 128:
-                self._dense(ctx.seq_lens, "seq_lens", torch.int32, (ctx.num_seqs,))
-                self._check(self._parts().akv_gated_attention_shared(
-                    _ptr(q), _ptr(k_pages), _ptr(v_pages), _ptr(gates), _long(gate_stride), gate_at, _ptr(ctx.q_start),
-                    _ptr(ctx.seq_lens), _ptr(meta.block_table), _ptr(meta.rows), meta.width, _ptr_at(out, out_at), singles, ctx.num_seqs,
-                    blocks // (kv_heads * maps), q_heads, kv_heads, dim, vdim, page_size, _long(num_pages), *tail), "gated_attention of shared keys")
-                return
-            self._check(self._parts().akv_gated_attention_tiles(
-                _ptr(q), _ptr(k_pages), _ptr(v_pages), _ptr(gates), _long(gate_stride), gate_at, _ptr(ctx.seq_of_token),
-                _ptr(ctx.q_start), _ptr(ctx.positions), _ptr(meta.block_table), _ptr(meta.rows), meta.width,
-                _ptr_at(out, out_at), singles, tokens, q_heads, kv_heads, dim, vdim, page_size, _long(num_pages), *tail),
-                "gated_attention on the matrix cores")
+            portions = singles < ctx.num_seqs
+            singles = singles if plain else 0
+            if portions:
+                self._attend_portions(ctx, meta, (q, k_pages, v_pages, gates), gate_stride, gate_at, out, out_at, tail,
+                                      (q_heads, kv_heads, maps, dim, vdim), window, chunk, page_size, num_pages)
+        if not singles:
             return
         # waves that share a token's head: by the most keys a row can see, fewer where the rows alone fill the device
-        row_waves = max(1, min(16 if tokens * q_heads <= 4096 else 4, span // 128))
+        row_waves = max(1, min(16 if singles * q_heads <= 4096 else 4, span // 128))
         self._check(self._parts().akv_gated_attention_rows(
             _ptr(q), _ptr(k_pages), _ptr(v_pages), _ptr(gates), _long(gate_stride), gate_at, _ptr(ctx.seq_of_token),
             _ptr(ctx.positions), _ptr(meta.block_table), _ptr(meta.rows), meta.width, _ptr_at(out, out_at),
-            self._code_of(q), _long(tokens), q_heads, kv_heads, dim, vdim, page_size, _long(num_pages), *tail[:-5], row_waves,
+            self._code_of(q), _long(singles), q_heads, kv_heads, dim, vdim, page_size, _long(num_pages), *tail[:-5], row_waves,
             *tail[-5:]), "gated_attention")
+
+    def _attend_portions(self, ctx, meta, operands, gate_stride, gate_at, out, out_at, tail, heads, window, chunk, page_size, num_pages):
+        """The prompt portions of a step, which follow its single tokens, on the matrix cores."""
+        first, (vectors, kv_heads, maps, dim, vdim) = ctx.num_decode_seqs, heads
+        q, k_pages, v_pages, gates = map(_ptr, operands)
+        blocks, shared = self._shares_attention_keys(ctx, first, heads, window, chunk)
+        if shared and dim <= 128 and vdim <= 128:
+            self._dense(ctx.seq_lens, "seq_lens", torch.int32, (ctx.num_seqs,))
+            self._check(self._parts().akv_gated_attention_shared(
+                q, k_pages, v_pages, gates, _long(gate_stride), gate_at, _ptr(ctx.q_start), _ptr(ctx.seq_lens), _ptr(meta.block_table),
+                _ptr(meta.rows), meta.width, _ptr_at(out, out_at), first, ctx.num_seqs, blocks // (kv_heads * maps), vectors, kv_heads,
+                dim, vdim, page_size, _long(num_pages), *tail), "gated_attention of shared keys")
+            return
+        self._check(self._parts().akv_gated_attention_tiles(
+            q, k_pages, v_pages, gates, _long(gate_stride), gate_at, _ptr(ctx.seq_of_token), _ptr(ctx.q_start), _ptr(ctx.positions),
+            _ptr(meta.block_table), _ptr(meta.rows), meta.width, _ptr_at(out, out_at), first, out.shape[0], vectors, kv_heads, dim,
+            vdim, page_size, _long(num_pages), *tail), "gated_attention on the matrix cores")
 
     # ---- mixers with a state of fixed size -----------------------------------------------------------------------------
     def check_retention_sizes(self, heads: int, dim: int, vdim: int) -> None:

@@ -381,6 +381,33 @@ def test_gated_attention_of_operands_that_are_not_aligned(hip, monkeypatch, aske
         assert ((attend(hip, DEVICE, ctx, **given) - want).abs() <= want.abs() * 2.0 ** -7 + 2e-3).all()
 
 
+@pytest.mark.parametrize("singles,portions", [(63, []), (64, []), (65, [40, 2])])
+def test_many_single_tokens_of_wide_heads_of_their_own(hip, singles, portions):
+    """On both sides of the line from which single tokens whose heads have keys of their own and values of 256 go to the plain kernel
+    (512 rows on 256 units), with portions behind them: against the double.  (2^-7 |out| + 2e-3 as above.)"""
+    from torch_kernels import TorchKernels
+    torch.manual_seed(singles)
+    heads, dim, vdim, page = 8, 32, 256, 16
+    ctx = _ctx([(37 * r) % 300 for r in range(singles)] + [20] * len(portions), [1] * singles + portions)
+    ctx.seq_lens = torch.tensor(ctx.host_seq_lens, dtype=torch.int32, device=DEVICE)
+    seqs, pages = ctx.num_seqs, max(ctx.host_seq_lens) // page + 1
+    table = torch.randperm(seqs * pages, dtype=torch.int32).view(seqs, pages)
+    k_pages = torch.randn(seqs * pages, heads, page, dim).bfloat16()
+    v_pages = torch.randn(seqs * pages, heads, vdim, page).bfloat16()
+    q, gates = torch.randn(ctx.num_tokens, heads * dim).bfloat16(), torch.randn(ctx.num_tokens, heads).bfloat16()
+
+    def attend(kernels, device, c):
+        out = torch.full((ctx.num_tokens, heads * vdim), float("nan"), dtype=torch.bfloat16, device=device)
+        meta = SimpleNamespace(block_table=table.to(device), rows=None, width=pages)
+        kernels.gated_attention(q.to(device), k_pages.to(device), v_pages.to(device), gates.to(device), 0, c, meta, heads, heads, dim, vdim,
+                                0.2, None, None, None, True, out)
+        return out.float().cpu()
+
+    host = SimpleNamespace(**{k: (v.cpu() if isinstance(v, torch.Tensor) else v) for k, v in vars(ctx).items()})
+    want = attend(TorchKernels(), "cpu", host)
+    assert ((attend(hip, DEVICE, ctx) - want).abs() <= want.abs() * 2.0 ** -7 + 2e-3).all()
+
+
 @pytest.mark.parametrize("tokens_at_once", [1, 2, 5, 9])
 @pytest.mark.parametrize("dim,vdim,window,keep_first", [(64, 128, None, 0), (128, 32, 6000, 40), (256, 256, None, 0)])
 def test_single_tokens_whose_partial_sums_do_not_fit(hip, monkeypatch, tokens_at_once, dim, vdim, window, keep_first):
