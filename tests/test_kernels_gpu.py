@@ -1324,6 +1324,20 @@ def test_float32_attention_in_several_launches(hip, monkeypatch, q_heads, kv_hea
     assert len(cuts) == 3 and len(cuts[0]) >= len(cuts[1]) > len(cuts[2]) > 1
 
 
+@pytest.mark.parametrize("requests", [64, 65, 150])
+@pytest.mark.parametrize("q_heads,kv_heads", [(6, 2), (4, 4)])
+def test_float32_attention_of_many_requests(hip, ref, requests, q_heads, kv_heads):
+    """A block finds its tile's request by adding up 64 requests' tiles at a time: more of them than that, of uneven portions - on one
+    tile and on several - and histories of one segment and of two."""
+    portions = [((37 * r) % 300, 1 + (7 * r) % 23) for r in range(requests)]
+    q, k_pages, v_pages, ctx, meta, _, _ = _attention_case(torch.float32, q_heads, kv_heads, 32, 8, portions, None, seed=45)
+    want, out = torch.empty_like(q), torch.full_like(q, float("nan")).cuda()
+    ref.attention(q, k_pages, v_pages, ctx, meta, q_heads, kv_heads, 32, 0.2, None, want)
+    c, m = _to_cuda(ctx, meta)
+    hip.attention(q.cuda(), k_pages.cuda(), v_pages.cuda(), c, m, q_heads, kv_heads, 32, 0.2, None, out)
+    torch.testing.assert_close(out.cpu(), want, **tol(torch.float32))
+
+
 @pytest.mark.parametrize("askew", ["q", "k_pages", "v_pages", "out"])
 @pytest.mark.parametrize("portions", [[(40, 1), (3, 1)], [(0, 33), (9, 5)]])
 def test_float32_attention_of_operands_that_are_not_aligned(hip, ref, askew, portions):

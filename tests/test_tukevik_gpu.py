@@ -537,6 +537,36 @@ def test_portions_that_share_their_keys_through_lds(hip, monkeypatch, heads, kv_
         assert ((got - want).abs() <= want.abs() * 2.0 ** -7 + 2e-3).all(), (blocks, (got - want).abs().max())
 
 
+@pytest.mark.parametrize("singles,portions", [(0, 65), (3, 64), (5, 140)])
+def test_portions_that_share_their_keys_of_many_requests(hip, monkeypatch, singles, portions):
+    """A block finds its tile's request by adding up 64 requests' tiles at a time, from the first portion on: more of them than that,
+    of uneven lengths, behind single tokens.  (2^-7 |out| + 2e-3 as above.)"""
+    from torch_kernels import TorchKernels
+    torch.manual_seed(portions)
+    heads, kv_heads, dim, vdim, page = 6, 2, 32, 64, 16
+    counts = [1] * singles + [2 + (7 * r) % 41 for r in range(portions)]
+    ctx = _ctx([(29 * r) % 90 for r in range(len(counts))], counts)
+    ctx.seq_lens = torch.tensor(ctx.host_seq_lens, dtype=torch.int32, device=DEVICE)
+    seqs, pages = ctx.num_seqs, max(ctx.host_seq_lens) // page + 1
+    table = torch.randperm(seqs * pages, dtype=torch.int32).view(seqs, pages)
+    k_pages = torch.randn(seqs * pages, kv_heads, page, dim).bfloat16()
+    v_pages = torch.randn(seqs * pages, kv_heads, vdim, page).bfloat16()
+    q = torch.randn(ctx.num_tokens, heads * dim).bfloat16()
+
+    def attend(kernels, device, c):
+        out = torch.full((ctx.num_tokens, heads * vdim), float("nan"), dtype=torch.bfloat16, device=device)
+        meta = SimpleNamespace(block_table=table.to(device), rows=None, width=pages)
+        kernels.gated_attention(q.to(device), k_pages.to(device), v_pages.to(device), None, 0, c, meta, heads, kv_heads, dim, vdim, 0.2,
+                                None, None, None, False, out)
+        return out.float().cpu()
+
+    host = SimpleNamespace(**{k: (v.cpu() if isinstance(v, torch.Tensor) else v) for k, v in vars(ctx).items()})
+    want = attend(TorchKernels(), "cpu", host)
+    for blocks in (1, 1 << 30):
+        monkeypatch.setattr(hip, "shared_attention_blocks", blocks, raising=False)
+        assert ((attend(hip, DEVICE, ctx) - want).abs() <= want.abs() * 2.0 ** -7 + 2e-3).all(), blocks
+
+
 @pytest.mark.parametrize("poison", [float("inf"), float("-inf"), float("nan")])
 @pytest.mark.parametrize("heads,kv_heads,dim,vdim,maps,options", [
     (4, 4, 64, 64, 1, {}), (16, 4, 128, 128, 1, dict(sink=True)), (8, 2, 32, 64, 1, dict(softcap=9.0)), (4, 2, 64, 128, 2, dict(window=40)),
