@@ -72,7 +72,7 @@ int launch_tiled(const void* x, const void* w, void* y, int rows, int outs, int 
 // ---- float32 on the matrix cores -----------------------------------------------------------------------------------------
 // v_mfma_f32_16x16x4_f32 multiplies and adds in float32 at twice the vector units' rate (157 TFLOP/s), with no rounding
 // of an operand.  A lane's operands of four such instructions are 16 consecutive bytes of a matrix row: lane (r, g) holds
-// elements 16 b + 4 g .. + 3 of row r, and instruction j takes element j of every group g.  Both kernels sum every output
+// elements 16 b + 4 g .. + 3 of row r, and instruction j takes element j of every group g.  All three kernels sum every output
 // the same way, so that a row's result depends neither on how many rows a call carries nor on which kernel takes it:
 // k is cut into segments of 128, a segment is one chain of instructions in the order (b, j), and the segments' sums are
 // added in their order.  (Rows and outputs beyond the matrices repeat the last one and are not stored; elements beyond k are
@@ -375,6 +375,8 @@ int launch_f32(const float* x, const float* w, float* y, int rows, int outs, int
     return launch_f32_pairs(x, w, y, rows, outs, k, bias, wide_stores, stream);
   if (rows <= 16) return launch_f32_few<1>(x, w, y, rows, outs, k, bias, wide_stores, stream);
   if (rows <= 32 && tiles <= units) return launch_f32_few<2>(x, w, y, rows, outs, k, bias, wide_stores, stream);
+  // (The caller counts the grid's limit in tiles of 64 rows.  Where tiles of 32 would pass it they are not taken: by then tiles of 64
+  // are more than a hundred rounds, and from eleven on twice the tiles at 115 cost more than 210.)
   const long large = 400 * rounds(64, 64), middle = 210 * rounds(32, 64), small = 115 * rounds(32, 32);
   if (large <= middle && large <= small) return launch_f32_wide<2, 2>(x, w, y, rows, outs, k, bias, wide_stores, stream);
   if (middle <= small) return launch_f32_wide<1, 2>(x, w, y, rows, outs, k, bias, wide_stores, stream);
