@@ -50,6 +50,8 @@ def shares_keys(units: int, portions, vectors: int, kv_heads: int, maps: int, di
     tile, step = 0.21 + 0.0024 * dim + 0.0022 * vdim, 0.72 + 0.0018 * dim + 0.0017 * vdim
     longest = tiles = tile_steps = steps = 0.0
     for count, length in portions:
+        if count == 0:
+            continue
         before = length - count
         growing = min(max(reach - before, 0), count)       # tokens that see more keys than the one before them
         keys = (growing * (before + growing / 2) + (count - growing) * reach) / count

@@ -231,3 +231,15 @@ def test_a_recorded_step_goes_where_the_same_step_goes_unrecorded(vectors, kv_he
     fresh, late = (kernels._shares_attention_keys(SimpleNamespace(num_seqs=1, host_q_start=[0, 1024], host_seq_lens=[length]), 0,
                                                   (16, 4, 1, 128, 128), None, None) for length in (1024, 7024))
     assert fresh == (256, False) and late == (256, True)
+
+
+def test_requests_without_tokens_add_nothing_to_the_choice():
+    """A request of a step may bring no token (a caller of the kernels alone): it makes no block and takes no time."""
+    from ampere_kv_engine_amd.kernels.hip_parts import shared_blocks, shares_keys
+    heads = (16, 4, 1, 128, 128)
+    for portions in ([(2048, 2048)], [(1024, 7024)], [(900, 900), (124, 6124)]):
+        for empty in ((0, 0), (0, 5000)):
+            assert shared_blocks(portions + [empty], *heads[:3]) == shared_blocks(portions, *heads[:3])
+            for window in (None, 1024):
+                for order in (portions + [empty], [empty] + portions):
+                    assert shares_keys(256, order, *heads, window, None) == shares_keys(256, portions, *heads, window, None)
