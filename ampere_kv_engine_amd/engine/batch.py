@@ -116,6 +116,7 @@ class StepContext:
     max_seq_len: int = 0           # longest request of the step, after the step
     max_new_tokens: int = 0        # longest portion of the step
     most_wanted: int = 0           # the most places any one request wants logits at
+    recordable_tokens: int = 0     # steps with portions of up to so many tokens may be recorded: lengths are then bounds
     arenas: tuple = ()             # two arenas used by alternate layers (a layer's output outlives its own arena's reset)
     stream_buffer: torch.Tensor | None = None   # float32 [max tokens, hidden]: the residual sum
     spare_buffer: torch.Tensor | None = None    # float32 [a few rows, hidden]: where a small step may move it

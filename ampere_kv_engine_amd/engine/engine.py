@@ -128,6 +128,7 @@ class Engine:
                 return logits if borrow_logits else logits.clone()
         ctx, _ = self.builder.build(entries, token_arrays=token_arrays)
         ctx.stream_buffer, ctx.spare_buffer = self.stream_buffer, self.spare_buffer
+        ctx.recordable_tokens = self.config.record_max_tokens
         self._last_step = ctx
         return self.model.forward(ctx, self.cache.layer_cache)
 
@@ -208,6 +209,7 @@ class Engine:
         counts, wanted = shape
         ctx, _ = self.builder.build(entries, width_multiple=self.config.graph_width_multiple, token_arrays=token_arrays)
         ctx.stream_buffer, ctx.spare_buffer = self.stream_buffer, self.spare_buffer
+        ctx.recordable_tokens = self.config.record_max_tokens
         self._last_step = ctx
         width = ctx.table_pages        # the longest request's pages, rounded up: a bound the recording is made for
         # sizes of launches come from bounds, not from this step's lengths: single tokens from the longest request's

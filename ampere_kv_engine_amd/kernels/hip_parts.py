@@ -830,7 +830,7 @@ class PartsKernels:
     # ---- attention with unit-normed queries and keys, a softcap, chunks, a sink and a gate per head ----------------------
     MAX_VALUE_DIM = 256
     shared_attention_blocks = None      # prompt portions of this many blocks share their keys through LDS; None: by `shares_keys`
-    FEW_TOKENS = 512                    # (what `EngineConfig.record_max_tokens` allows a recorded step by default)
+    FEW_TOKENS = 512                    # (what `EngineConfig.record_max_tokens` allows a recorded step by default; more where it does)
 
     def _shares_attention_keys(self, ctx, first: int, heads: tuple[int, int, int, int, int], window, chunk) -> tuple[int, bool]:
         """The blocks that the portions of a step, requests `first` on, make in the kernel that shares keys, and whether they go
@@ -841,7 +841,7 @@ class PartsKernels:
         choices = ctx.__dict__.setdefault("shared_attention", {})
         key = (tuple(starts), tuple(lengths), heads, window, chunk, self.shared_attention_blocks)
         if key not in choices:
-            few = starts[-1] <= self.FEW_TOKENS
+            few = starts[-1] <= max(self.FEW_TOKENS, getattr(ctx, "recordable_tokens", 0))
             portions = [(end - start, 2 * (end - start) if few else length)
                         for start, end, length in zip(starts, starts[1:], lengths)]
             blocks = shared_blocks(portions, *heads[:3])

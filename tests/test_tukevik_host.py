@@ -243,3 +243,25 @@ def test_requests_without_tokens_add_nothing_to_the_choice():
             for window in (None, 1024):
                 for order in (portions + [empty], [empty] + portions):
                     assert shares_keys(256, order, *heads, window, None) == shares_keys(256, portions, *heads, window, None)
+
+
+@pytest.mark.parametrize("allowed", [64, 512, 513, 1024, 4096])
+def test_an_engine_that_records_longer_portions_sends_them_the_same_way(allowed):
+    """The line between steps that look at lengths and steps that do not follows what their engine may record."""
+    from types import SimpleNamespace
+    from ampere_kv_engine_amd.kernels.hip_parts import PartsKernels
+    kernels = PartsKernels.__new__(PartsKernels)
+    kernels.compute_units, turned = 256, False
+    for heads in ((16, 4, 1, 128, 128), (64, 8, 1, 128, 128), (32, 8, 2, 64, 128)):
+        for tokens in (280, 512, 513, 900, 1024, 1025):
+            choices = {kernels._shares_attention_keys(
+                SimpleNamespace(num_seqs=1, host_q_start=[0, tokens], host_seq_lens=[length], recordable_tokens=allowed),
+                0, heads, None, None) for length in (tokens, tokens + 300, 2048, 7000, 65536)}
+            turned |= len(choices) > 1
+            assert len(choices) == 1 or tokens > max(allowed, 512)
+    assert turned == (allowed < 1025)
+
+
+def test_every_step_says_what_its_engine_may_record(engine, case):
+    T.case_whole(engine, case)
+    assert engine._last_step.recordable_tokens == engine.config.record_max_tokens
