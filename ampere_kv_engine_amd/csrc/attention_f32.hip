@@ -24,6 +24,8 @@
 // float32 (`attention_rows`): 3 single tokens after 64 to 700 keys 298 -> 16.1 + 4.6 for the fold; 3 prompts of 333 tokens
 // 811 -> 62.
 
+#include <type_traits>
+
 #include "common.h"
 #include "api.h"
 
@@ -76,39 +78,52 @@ __device__ __forceinline__ bool all_finite(const floats4 v) {
 }
 
 // FEW: there are fewer blocks than compute units, and a block waits for its loads: a tile's values are asked for a tile ahead,
-// with the registers of one wave a SIMD.  Otherwise two waves a SIMD hide each other's waits.
+// with the registers of one wave a SIMD.  Otherwise two waves a SIMD hide each other's waits, three or four of narrow heads.
+// A wave that has one tile of a segment - short contexts, windows, a request's last segment - takes that one alone, with its
+// values asked for beside its records, and one that has none goes straight to the fold: 256 tokens of 30 keys, 16 heads of
+// 64 of their own, 73 us with four tiles always and 34 now (31 in `attention_rows`), a window of 100 of 300 keys 130 -> 65 (79),
+// 5 tokens of 16 / 4 heads of 128 12.4 -> 8.6 (11.1); where every wave has four, 0 to 0.5 us of code to fetch more.
 template <int NT, bool FEW>
-__global__ __launch_bounds__(256, FEW || NT > 8 ? 1 : 2) void attention_f32_kernel(const Args a) {
+__global__ __launch_bounds__(256, FEW || NT > 8 ? 1 : NT > 4 ? 2 : NT > 2 ? 3 : 4) void attention_f32_kernel(const Args a) {
   constexpr int kDim = 16 * NT;
   constexpr int kOwn = (NT + 3) / 4;             // tiles of 16 dims whose totals a wave keeps: w, w + 4, ...
   constexpr int kGroup = NT <= 6 ? kTiles : 2;   // tiles of keys whose records are asked for together (registers)
   __shared__ floats4 sums_of[4][NT][64];
   __shared__ float top_of[4][kRows], weight_of[4][kRows];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int c = lane & 15, g = lane >> 4;        // the row (or key, or dim) of a tile, and the lane's group of four
   const int share = a.q_heads / a.kv_heads, kvh = blockIdx.y;
 
-  // whose tile this is: tiles are numbered request by request
+  // whose tile this is: tiles are numbered request by request, a lane counts those of four requests in a row (one
+  // turn for 256)
   int request = -1, tile = a.first_tile + static_cast<int>(blockIdx.x);
-  for (int first = 0; first < a.seqs && request < 0; first += kWave) {
-    const int r = first + lane;
-    const int count = r < a.seqs ? ((a.q_start[r + 1] - a.q_start[r]) * share + kRows - 1) / kRows : 0;
-    int upto = count;
+  for (int first = 0; first < a.seqs && request < 0; first += 4 * kWave) {
+    int upto[4], count = 0, start = a.q_start[min(first + 4 * lane, a.seqs)];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int end = a.q_start[min(first + 4 * lane + i + 1, a.seqs)];
+      upto[i] = count += ((end - start) * share + kRows - 1) / kRows;
+      start = end;
+    }
+    int all = count;
 #pragma unroll
     for (int step = 1; step < kWave; step <<= 1) {
-      const int other = __shfl_up(upto, step, kWave);
-      if (lane >= step) upto += other;
+      const int other = __shfl_up(all, step, kWave);
+      if (lane >= step) all += other;
     }
-    const unsigned long long here = __ballot(tile < upto);
+    const unsigned long long here = __ballot(tile < all);
     if (here != 0) {
-      const int at = __ffsll(here) - 1;
-      request = first + at;
-      tile -= __shfl(upto - count, at, kWave);
+      const int at = __ffsll(here) - 1, own = tile - (all - count);
+      const int of_lane = (own >= upto[0]) + (own >= upto[1]) + (own >= upto[2]);
+      const int before = of_lane == 0 ? 0 : of_lane == 1 ? upto[0] : of_lane == 2 ? upto[1] : upto[2];
+      request = first + 4 * at + __builtin_amdgcn_readlane(of_lane, at);
+      tile = __builtin_amdgcn_readlane(own - before, at);
     } else {
-      tile -= __shfl(upto, kWave - 1, kWave);
+      tile -= __builtin_amdgcn_readlane(all, kWave - 1);
     }
   }
   if (request < 0) return;
+  request = __builtin_amdgcn_readfirstlane(request), tile = __builtin_amdgcn_readfirstlane(tile);      // (the same for all lanes)
   const int token0 = a.q_start[request], tokens = a.q_start[request + 1] - token0;
   const int rows = tokens * share, row0 = tile * kRows;
   const int history = a.seq_lens[request] - tokens;
@@ -140,134 +155,152 @@ __global__ __launch_bounds__(256, FEW || NT > 8 ? 1 : 2) void attention_f32_kern
   for (int i = 0; i < kOwn; ++i) total[i] = zero;
 
   for (int segment = first_own; segment <= last_segment; segment += stride) {
-    const int base = segment * kSegment + wave * 16;
-    // ---- scores of the wave's tiles
-    // (no load stands behind a test: the compiler would wait for it before the next.  A key that no row sees asks for the
-    // nearest that one does)
-    floats4 s[kTiles];
-    const float* vp[kTiles];                     // the lane's four keys in their page's first value row
-    bool there[kTiles];
-#pragma unroll
-    for (int t0 = 0; t0 < kTiles; t0 += kGroup) {
-      floats4 k[kGroup][NT];
-      bool known[kGroup];
-      int key[kGroup], four[kGroup], page[kGroup], vpage[kGroup];
-#pragma unroll
-      for (int t = 0; t < kGroup; ++t) {
-        key[t] = min(max(base + 64 * (t0 + t) + c, lowest), pos_max);
-        four[t] = min(max(base + 64 * (t0 + t) + 4 * g, lowest & ~3), pos_max & ~3);      // (pages hold a multiple of four)
-        page[t] = table[key[t] / a.page_size];
-        vpage[t] = table[four[t] / a.page_size];
-      }
-#pragma unroll
-      for (int t = 0; t < kGroup; ++t) {
-        known[t] = (page[t] >= 0) & (page[t] < a.num_pages);       // (a page that is not the request's is never read: its scores
-        there[t0 + t] = (vpage[t] >= 0) & (vpage[t] < a.num_pages);                                              // are NaN)
-        const long record = ((known[t] ? page[t] : 0) * static_cast<long>(a.kv_heads) + kvh) * a.page_size + key[t] % a.page_size;
-        const float* kp = a.k_pages + record * kDim + 4 * g;
-#pragma unroll
-        for (int b = 0; b < NT; ++b) k[t][b] = *reinterpret_cast<const floats4*>(kp + 16 * b);
-        vp[t0 + t] = a.v_pages + ((there[t0 + t] ? vpage[t] : 0) * static_cast<long>(a.kv_heads) + kvh) * kDim * a.page_size +
-                     four[t] % a.page_size;
-      }
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int t = 0; t < kGroup; ++t) {
-        floats4 sums = zero;
-#pragma unroll
-        for (int b = 0; b < NT; ++b)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) sums = __builtin_amdgcn_mfma_f32_16x16x4f32(k[t][b][e], q[b][e], sums, 0, 0, 0);
-        // lane (c, g) now has row c's scores of keys 4 g .. 4 g + 3
-        const unsigned unknown = static_cast<unsigned>(__ballot(!known[t]) & 0xffffu);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int key = base + 64 * (t0 + t) + 4 * g + j;
-          const float score = (unknown >> (4 * g + j)) & 1u ? __uint_as_float(0x7fc00000u) : sums[j] * a.scale;
-          s[t0 + t][j] = (key >= low) & (key <= pos) ? score : -INFINITY;
-        }
-      }
-    }
-    // ---- one maximum for the wave's tiles, weights, their sum
-    float top = -INFINITY;
-#pragma unroll
-    for (int t = 0; t < kTiles; ++t)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) top = fmaxf(top, s[t][j]);
-    top = fmaxf(top, __shfl_xor(top, 16, kWave));
-    top = fmaxf(top, __shfl_xor(top, 32, kWave));
-    const float shift = top == -INFINITY ? 0.f : top;
-    float weight = 0.f;
-#pragma unroll
-    for (int t = 0; t < kTiles; ++t)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        s[t][j] = expf(s[t][j] - shift);         // (exp(-inf) of a key that the row does not see)
-        weight += s[t][j];
-      }
-    weight += __shfl_xor(weight, 16, kWave);
-    weight += __shfl_xor(weight, 32, kWave);
-    // ---- weighted sums
-    constexpr bool kAhead = FEW && NT <= 8;
-    floats4 sums[NT], v[NT], next[kAhead ? NT : 1];
-    const auto values = [&](int t, floats4* to) {
-#pragma unroll
-      for (int n = 0; n < NT; ++n) to[n] = *reinterpret_cast<const floats4*>(vp[t] + static_cast<long>(16 * n + c) * a.page_size);
+    // A wave's tiles that some row sees lie side by side: the first and how many (the same for the whole wave)
+    const auto first_tile_of = [&](int w) { return max(0, (lowest - 15 - (segment * kSegment + 16 * w) + 63) >> 6); };
+    const auto tiles_of = [&](int w) {
+      return min(kTiles - 1, (pos_max - (segment * kSegment + 16 * w)) >> 6) - first_tile_of(w) + 1;
     };
+    floats4 sums[NT];
 #pragma unroll
     for (int n = 0; n < NT; ++n) sums[n] = zero;
-    if constexpr (kAhead) values(0, next);
+    float top = -INFINITY, weight = 0.f;
+    // The scores of a wave's TILES tiles from `base` on, their maximum, weights and weighted sums.
+    const auto take = [&](auto count, const int base) {
+      constexpr int TILES = decltype(count)::value;
+      constexpr int kTogether = TILES < kGroup ? TILES : kGroup;
+      constexpr bool kAtOnce = TILES == 1;       // the values are asked for with the records
+      // ---- scores of the wave's tiles
+      // (no load stands behind a test: the compiler would wait for it before the next.  A key that no row sees asks for the
+      // nearest that one does)
+      floats4 s[TILES], v[NT];
+      const float* vp[TILES];                    // the lane's four keys in their page's first value row
+      bool there[TILES];
+      const auto values = [&](int t, floats4* to) {
 #pragma unroll
-    for (int t = 0; t < kTiles; ++t) {
-      const int first_key = base + 64 * t;
-      if constexpr (kAhead) {
+        for (int n = 0; n < NT; ++n) to[n] = *reinterpret_cast<const floats4*>(vp[t] + static_cast<long>(16 * n + c) * a.page_size);
+      };
 #pragma unroll
-        for (int n = 0; n < NT; ++n) v[n] = next[n];
-        if (t + 1 < kTiles) values(t + 1, next);
+      for (int t0 = 0; t0 < TILES; t0 += kTogether) {
+        floats4 k[kTogether][NT];
+        bool known[kTogether];
+        int key[kTogether], four[kTogether], page[kTogether], vpage[kTogether];
+#pragma unroll
+        for (int t = 0; t < kTogether; ++t) {
+          key[t] = min(max(base + 64 * (t0 + t) + c, lowest), pos_max);
+          four[t] = min(max(base + 64 * (t0 + t) + 4 * g, lowest & ~3), pos_max & ~3);      // (pages hold a multiple of four)
+          page[t] = table[key[t] / a.page_size];
+          vpage[t] = table[four[t] / a.page_size];
+        }
+#pragma unroll
+        for (int t = 0; t < kTogether; ++t) {
+          known[t] = (page[t] >= 0) & (page[t] < a.num_pages);       // (a page that is not the request's is never read: its scores
+          there[t0 + t] = (vpage[t] >= 0) & (vpage[t] < a.num_pages);                                              // are NaN)
+          const long record = ((known[t] ? page[t] : 0) * static_cast<long>(a.kv_heads) + kvh) * a.page_size + key[t] % a.page_size;
+          const float* kp = a.k_pages + record * kDim + 4 * g;
+#pragma unroll
+          for (int b = 0; b < NT; ++b) k[t][b] = *reinterpret_cast<const floats4*>(kp + 16 * b);
+          vp[t0 + t] = a.v_pages + ((there[t0 + t] ? vpage[t] : 0) * static_cast<long>(a.kv_heads) + kvh) * kDim * a.page_size +
+                       four[t] % a.page_size;
+        }
+        if constexpr (kAtOnce) values(0, v);
         __builtin_amdgcn_sched_barrier(0);
-      }
-      if (first_key > pos_max || first_key + 15 < lowest) continue;        // (the same for the whole wave)
-      if constexpr (!kAhead) values(t, v);
-      bool fine = true;
-      if (first_key < low_max || first_key + 15 > pos_min || !__all(there[t])) {
-        // some row does not see some key of the tile.  Slots that nobody has written, or that are not the request's, hold
-        // anything: no row sees them, and they count as zero
 #pragma unroll
-        for (int n = 0; n < NT; ++n) {
+        for (int t = 0; t < kTogether; ++t) {
+          floats4 scores = zero;
+#pragma unroll
+          for (int b = 0; b < NT; ++b)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) scores = __builtin_amdgcn_mfma_f32_16x16x4f32(k[t][b][e], q[b][e], scores, 0, 0, 0);
+          // lane (c, g) now has row c's scores of keys 4 g .. 4 g + 3
+          const unsigned unknown = static_cast<unsigned>(__ballot(!known[t]) & 0xffffu);
 #pragma unroll
           for (int j = 0; j < 4; ++j) {
-            const int key = first_key + 4 * g + j;
-            v[n][j] = there[t] & (key >= lowest) & (key <= pos_max) ? v[n][j] : 0.f;
+            const int key = base + 64 * (t0 + t) + 4 * g + j;
+            const float score = (unknown >> (4 * g + j)) & 1u ? __uint_as_float(0x7fc00000u) : scores[j] * a.scale;
+            s[t0 + t][j] = (key >= low) & (key <= pos) ? score : -INFINITY;
           }
-          fine = fine & all_finite(v[n]);
         }
       }
-      if (__all(fine)) {
+      // ---- one maximum for the wave's tiles, weights, their sum
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
+      for (int t = 0; t < TILES; ++t)
 #pragma unroll
-          for (int n = 0; n < NT; ++n) sums[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[n][e], s[t][e], sums[n], 0, 0, 0);
-      } else {                                   // key by key, for the rows that see it
-#pragma unroll 1
-        for (int four = 0; four < 4; ++four)
+        for (int j = 0; j < 4; ++j) top = fmaxf(top, s[t][j]);
+      top = fmaxf(top, __shfl_xor(top, 16, kWave));
+      top = fmaxf(top, __shfl_xor(top, 32, kWave));
+      const float shift = top == -INFINITY ? 0.f : top;
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const int key = first_key + 4 * four + e;
-            const bool seen = key >= low && key <= pos, mine = four == g;
+      for (int t = 0; t < TILES; ++t)
 #pragma unroll
-            for (int n = 0; n < NT; ++n) {
-              const floats4 with = __builtin_amdgcn_mfma_f32_16x16x4f32(mine ? v[n][e] : 0.f, mine ? s[t][e] : 0.f, sums[n], 0, 0, 0);
-              if (seen) sums[n] = with;
+        for (int j = 0; j < 4; ++j) {
+          s[t][j] = expf(s[t][j] - shift);         // (exp(-inf) of a key that the row does not see)
+          weight += s[t][j];
+        }
+      weight += __shfl_xor(weight, 16, kWave);
+      weight += __shfl_xor(weight, 32, kWave);
+      // ---- weighted sums
+      constexpr bool kAhead = FEW && NT <= 8 && !kAtOnce;
+      floats4 next[kAhead ? NT : 1];
+      if constexpr (kAhead) values(0, next);
+#pragma unroll
+      for (int t = 0; t < TILES; ++t) {
+        const int first_key = base + 64 * t;
+        if constexpr (kAhead) {
+#pragma unroll
+          for (int n = 0; n < NT; ++n) v[n] = next[n];
+          if (t + 1 < TILES) values(t + 1, next);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        if (first_key > pos_max || first_key + 15 < lowest) continue;        // (the same for the whole wave)
+        if constexpr (!kAhead && !kAtOnce) values(t, v);
+        bool fine = true;
+        if (first_key < low_max || first_key + 15 > pos_min || !__all(there[t])) {
+          // some row does not see some key of the tile.  Slots that nobody has written, or that are not the request's, hold
+          // anything: no row sees them, and they count as zero
+#pragma unroll
+          for (int n = 0; n < NT; ++n) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+              const int key = first_key + 4 * g + j;
+              v[n][j] = there[t] & (key >= lowest) & (key <= pos_max) ? v[n][j] : 0.f;
             }
+            fine = fine & all_finite(v[n]);
           }
-      }
-    }
-    // ---- the four waves' parts, in their order
+        }
+        if (__all(fine)) {
 #pragma unroll
-    for (int n = 0; n < NT; ++n) sums_of[wave][n][lane] = sums[n];
-    if (g == 0) {
-      top_of[wave][c] = top;
-      weight_of[wave][c] = weight;
+          for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int n = 0; n < NT; ++n) sums[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[n][e], s[t][e], sums[n], 0, 0, 0);
+        } else {                                   // key by key, for the rows that see it
+#pragma unroll 1
+          for (int four = 0; four < 4; ++four)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const int key = first_key + 4 * four + e;
+              const bool seen = key >= low && key <= pos, mine = four == g;
+#pragma unroll
+              for (int n = 0; n < NT; ++n) {
+                const floats4 with = __builtin_amdgcn_mfma_f32_16x16x4f32(mine ? v[n][e] : 0.f, mine ? s[t][e] : 0.f, sums[n], 0, 0, 0);
+                if (seen) sums[n] = with;
+              }
+            }
+        }
+      }
+    };
+    const int own_tiles = tiles_of(wave);
+    if (own_tiles == 1)
+      take(std::integral_constant<int, 1>(), segment * kSegment + wave * 16 + 64 * first_tile_of(wave));
+    else if (own_tiles > 1)
+      take(std::integral_constant<int, kTiles>(), segment * kSegment + wave * 16);
+    // ---- the four waves' parts, in their order; one of no keys changes nothing (and is passed over where no latency hangs on it)
+    if (FEW || own_tiles > 0) {
+#pragma unroll
+      for (int n = 0; n < NT; ++n) sums_of[wave][n][lane] = sums[n];
+      if (g == 0) {
+        top_of[wave][c] = top;
+        weight_of[wave][c] = weight;
+      }
     }
     __syncthreads();
     float segment_top = -INFINITY, segment_weight = 0.f;
@@ -276,6 +309,7 @@ __global__ __launch_bounds__(256, FEW || NT > 8 ? 1 : 2) void attention_f32_kern
     for (int i = 0; i < kOwn; ++i) segment_sums[i] = zero;
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
+      if (!FEW && tiles_of(w) <= 0) continue;
       const Fold f(segment_top, top_of[w][c]);
       segment_weight = f(segment_weight, weight_of[w][c]);
 #pragma unroll

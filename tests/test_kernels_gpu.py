@@ -1324,11 +1324,11 @@ def test_float32_attention_in_several_launches(hip, monkeypatch, q_heads, kv_hea
     assert len(cuts) == 3 and len(cuts[0]) >= len(cuts[1]) > len(cuts[2]) > 1
 
 
-@pytest.mark.parametrize("requests", [64, 65, 150])
+@pytest.mark.parametrize("requests", [64, 65, 150, 256, 257, 300])
 @pytest.mark.parametrize("q_heads,kv_heads", [(6, 2), (4, 4)])
 def test_float32_attention_of_many_requests(hip, ref, requests, q_heads, kv_heads):
-    """A block finds its tile's request by adding up 64 requests' tiles at a time: more of them than that, of uneven portions - on one
-    tile and on several - and histories of one segment and of two."""
+    """A block finds its tile's request by adding up 256 requests' tiles at a time, four a lane: fewer and more of them, of uneven
+    portions - on one tile and on several - and histories of one segment and of two."""
     portions = [((37 * r) % 300, 1 + (7 * r) % 23) for r in range(requests)]
     q, k_pages, v_pages, ctx, meta, _, _ = _attention_case(torch.float32, q_heads, kv_heads, 32, 8, portions, None, seed=45)
     want, out = torch.empty_like(q), torch.full_like(q, float("nan")).cuda()
@@ -1336,6 +1336,27 @@ def test_float32_attention_of_many_requests(hip, ref, requests, q_heads, kv_head
     c, m = _to_cuda(ctx, meta)
     hip.attention(q.cuda(), k_pages.cuda(), v_pages.cuda(), c, m, q_heads, kv_heads, 32, 0.2, None, out)
     torch.testing.assert_close(out.cpu(), want, **tol(torch.float32))
+
+
+@pytest.mark.parametrize("q_heads,kv_heads,dim", [(4, 4, 32), (16, 16, 16), (8, 2, 64), (4, 1, 128), (2, 2, 256)])
+@pytest.mark.parametrize("window", [None, 40, 64])
+@pytest.mark.parametrize("every", [1, 15])
+def test_float32_attention_of_a_token_among_others_and_alone(hip, q_heads, kv_heads, dim, window, every):
+    """A wave of a token alone may have no tile of a segment, or one, where beside the other rows of a portion it has one or more: the
+    same bits, in steps of blocks for every unit and of fewer."""
+    q, k_pages, v_pages, ctx, meta, _, _ = _attention_case(torch.float32, q_heads, kv_heads, dim, 16, [(0, 600)], None, seed=46)
+    k_pages, v_pages, scale = k_pages.cuda(), v_pages.cuda(), dim ** -0.5
+    whole = torch.full_like(q, float("nan")).cuda()
+    hip.attention(q.cuda(), k_pages, v_pages, *_to_cuda(ctx, meta), q_heads, kv_heads, dim, scale, window, whole)
+    taken = torch.arange(0, 600, every)
+    alone = SimpleNamespace(**dict(vars(ctx), num_seqs=len(taken), num_tokens=len(taken), host_q_start=list(range(len(taken) + 1)),
+                                   host_seq_lens=(taken + 1).tolist(), positions=taken.int(),
+                                   seq_of_token=torch.arange(len(taken), dtype=torch.int32), max_new_tokens=1))
+    out = torch.full((len(taken), q.shape[1]), float("nan"), device="cuda")
+    rows = SimpleNamespace(**dict(vars(meta), block_table=meta.block_table.expand(len(taken), -1).contiguous()))
+    hip.attention(q[taken].cuda(), k_pages, v_pages, *_to_cuda(alone, rows), q_heads, kv_heads, dim, scale, window, out)
+    assert torch.isfinite(out).all()
+    assert torch.equal(out, whole[taken])
 
 
 @pytest.mark.parametrize("askew", ["q", "k_pages", "v_pages", "out"])
