@@ -77,31 +77,18 @@ __device__ __forceinline__ bool all_finite(const floats4 v) {
   return fine;
 }
 
-// FEW: there are fewer blocks than compute units, and a block waits for its loads: a tile's values are asked for a tile ahead,
-// with the registers of one wave a SIMD.  Otherwise two waves a SIMD hide each other's waits, three or four of narrow heads.
-// A wave that has one tile of a segment - short contexts, windows, a request's last segment - takes that one alone, with its
-// values asked for beside its records, and one that has none goes straight to the fold: 256 tokens of 30 keys, 16 heads of
-// 64 of their own, 73 us with four tiles always and 34 now (31 in `attention_rows`), a window of 100 of 300 keys 130 -> 65 (79),
-// 5 tokens of 16 / 4 heads of 128 12.4 -> 8.6 (11.1); where every wave has four, 0 to 0.5 us of code to fetch more.
-template <int NT, bool FEW>
-__global__ __launch_bounds__(256, FEW || NT > 8 ? 1 : NT > 4 ? 2 : NT > 2 ? 3 : 4) void attention_f32_kernel(const Args a) {
-  constexpr int kDim = 16 * NT;
-  constexpr int kOwn = (NT + 3) / 4;             // tiles of 16 dims whose totals a wave keeps: w, w + 4, ...
-  constexpr int kGroup = NT <= 6 ? kTiles : 2;   // tiles of keys whose records are asked for together (registers)
-  __shared__ floats4 sums_of[4][NT][64];
-  __shared__ float top_of[4][kRows], weight_of[4][kRows];
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int c = lane & 15, g = lane >> 4;        // the row (or key, or dim) of a tile, and the lane's group of four
-  const int share = a.q_heads / a.kv_heads, kvh = blockIdx.y;
-
-  // whose tile this is: tiles are numbered request by request, a lane counts those of four requests in a row (one
-  // turn for 256)
-  int request = -1, tile = a.first_tile + static_cast<int>(blockIdx.x);
-  for (int first = 0; first < a.seqs && request < 0; first += 4 * kWave) {
-    int upto[4], count = 0, start = a.q_start[min(first + 4 * lane, a.seqs)];
+// Whose tile this is: tiles are numbered request by request, and a lane counts those of EACH requests in a row (four: one turn for
+// 256).  Sets `request`, which is -1 before, and leaves `tile` its number in the request; the same for all lanes of a wave.  With
+// four that is said to the compiler, which keeps what follows from it in scalar registers; a block of SPLIT, which waits for each
+// load in turn, finds the next numbers of the step sooner where the vector loads left them (a decode step of 3 requests and 8
+// layers: 632 us with scalar loads, 624 without).
+template <int EACH>
+__device__ __forceinline__ void find_request(const Args& a, int share, int lane, int& request, int& tile) {
+  for (int first = 0; first < a.seqs && request < 0; first += EACH * kWave) {
+    int upto[EACH], count = 0, start = a.q_start[min(first + EACH * lane, a.seqs)];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int end = a.q_start[min(first + 4 * lane + i + 1, a.seqs)];
+    for (int i = 0; i < EACH; ++i) {
+      const int end = a.q_start[min(first + EACH * lane + i + 1, a.seqs)];
       upto[i] = count += ((end - start) * share + kRows - 1) / kRows;
       start = end;
     }
@@ -114,16 +101,42 @@ __global__ __launch_bounds__(256, FEW || NT > 8 ? 1 : NT > 4 ? 2 : NT > 2 ? 3 : 
     const unsigned long long here = __ballot(tile < all);
     if (here != 0) {
       const int at = __ffsll(here) - 1, own = tile - (all - count);
-      const int of_lane = (own >= upto[0]) + (own >= upto[1]) + (own >= upto[2]);
-      const int before = of_lane == 0 ? 0 : of_lane == 1 ? upto[0] : of_lane == 2 ? upto[1] : upto[2];
-      request = first + 4 * at + __builtin_amdgcn_readlane(of_lane, at);
-      tile = __builtin_amdgcn_readlane(own - before, at);
+      int of_lane = 0, before = 0;
+#pragma unroll
+      for (int i = 0; i + 1 < EACH; ++i) {
+        of_lane += own >= upto[i];
+        before = own >= upto[i] ? upto[i] : before;
+      }
+      request = first + EACH * at + (EACH > 1 ? __builtin_amdgcn_readlane(of_lane, at) : 0);
+      tile = EACH > 1 ? __builtin_amdgcn_readlane(own - before, at) : __shfl(own, at, kWave);
     } else {
-      tile -= __builtin_amdgcn_readlane(all, kWave - 1);
+      tile -= __shfl(all, kWave - 1, kWave);
     }
   }
+}
+
+// FEW: there are fewer blocks than compute units, and a block waits for its loads: a tile's values are asked for a tile ahead,
+// with the registers of one wave a SIMD.  Otherwise two waves a SIMD hide each other's waits, three or four of narrow heads.
+// A wave that has one tile of a segment - short contexts, windows, a request's last segment - takes that one alone, with its
+// values asked for beside its records, and one that has none goes straight to the fold: 256 tokens of 30 keys, 16 heads of
+// 64 of their own, 73 us with four tiles always and 34 now (31 in `attention_rows`), a window of 100 of 300 keys 130 -> 65 (79),
+// 5 tokens of 16 / 4 heads of 128 12.4 -> 8.6 (11.1).  SPLIT: the segments are blocks of their own, most of them whole, and waves
+// take four tiles always.
+template <int NT, bool FEW, bool SPLIT>
+__global__ __launch_bounds__(256, FEW || NT > 8 ? 1 : NT > 4 ? 2 : NT > 2 ? 3 : 4) void attention_f32_kernel(const Args a) {
+  constexpr int kDim = 16 * NT;
+  constexpr int kOwn = (NT + 3) / 4;             // tiles of 16 dims whose totals a wave keeps: w, w + 4, ...
+  constexpr int kGroup = NT <= 6 ? kTiles : 2;   // tiles of keys whose records are asked for together (registers)
+  __shared__ floats4 sums_of[4][NT][64];
+  __shared__ float top_of[4][kRows], weight_of[4][kRows];
+  const int lane = threadIdx.x & 63, wave = SPLIT ? threadIdx.x >> 6 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int c = lane & 15, g = lane >> 4;        // the row (or key, or dim) of a tile, and the lane's group of four
+  const int share = a.q_heads / a.kv_heads, kvh = blockIdx.y;
+
+  int request = -1, tile = a.first_tile + static_cast<int>(blockIdx.x);
+  find_request<SPLIT ? 1 : 4>(a, share, lane, request, tile);
   if (request < 0) return;
-  request = __builtin_amdgcn_readfirstlane(request), tile = __builtin_amdgcn_readfirstlane(tile);      // (the same for all lanes)
+  if constexpr (!SPLIT) request = __builtin_amdgcn_readfirstlane(request), tile = __builtin_amdgcn_readfirstlane(tile);
   const int token0 = a.q_start[request], tokens = a.q_start[request + 1] - token0;
   const int rows = tokens * share, row0 = tile * kRows;
   const int history = a.seq_lens[request] - tokens;
@@ -138,8 +151,7 @@ __global__ __launch_bounds__(256, FEW || NT > 8 ? 1 : NT > 4 ? 2 : NT > 2 ? 3 : 
   const int low_max = a.window > 0 ? max(0, pos_max - a.window + 1) : 0;
   const int first_segment = lowest / kSegment, last_segment = pos_max / kSegment;
 
-  const bool split = a.partial != nullptr;
-  const int stride = split ? a.splits : 1, first_own = first_segment + (split ? static_cast<int>(blockIdx.z) : 0);
+  const int stride = SPLIT ? a.splits : 1, first_own = first_segment + (SPLIT ? static_cast<int>(blockIdx.z) : 0);
   if (first_own > last_segment) return;
 
   floats4 q[NT];
@@ -289,9 +301,9 @@ __global__ __launch_bounds__(256, FEW || NT > 8 ? 1 : NT > 4 ? 2 : NT > 2 ? 3 : 
       }
     };
     const int own_tiles = tiles_of(wave);
-    if (own_tiles == 1)
+    if (!SPLIT && own_tiles == 1)
       take(std::integral_constant<int, 1>(), segment * kSegment + wave * 16 + 64 * first_tile_of(wave));
-    else if (own_tiles > 1)
+    else if (SPLIT || own_tiles > 1)
       take(std::integral_constant<int, kTiles>(), segment * kSegment + wave * 16);
     // ---- the four waves' parts, in their order; one of no keys changes nothing (and is passed over where no latency hangs on it)
     if (FEW || own_tiles > 0) {
@@ -321,7 +333,7 @@ __global__ __launch_bounds__(256, FEW || NT > 8 ? 1 : NT > 4 ? 2 : NT > 2 ? 3 : 
       }
     }
     __syncthreads();                             // (the next segment writes LDS again)
-    if (split) {
+    if constexpr (SPLIT) {
       const int of_row = segment - low / kSegment;         // (segments that the row does not see are nobody's to fold)
       if (row0 + c < rows && token >= a.first_token && token < a.token_end && of_row >= 0 && of_row < a.segments) {
         float* at = a.partial + ((static_cast<long>(token - a.first_token) * a.q_heads + head) * a.segments + of_row) * (kDim + 4);
@@ -342,7 +354,7 @@ __global__ __launch_bounds__(256, FEW || NT > 8 ? 1 : NT > 4 ? 2 : NT > 2 ? 3 : 
 #pragma unroll
       for (int j = 0; j < 4; ++j) total[i][j] = f(total[i][j], segment_sums[i][j]);
   }
-  if (split || row0 + c >= rows) return;
+  if (SPLIT || row0 + c >= rows) return;
   float* at = a.out + (static_cast<long>(token) * a.q_heads + head) * kDim + 4 * g;
 #pragma unroll
   for (int i = 0; i < kOwn; ++i) {
@@ -418,10 +430,11 @@ extern "C" int akv_attention_f32(const float* q, const float* k_pages, const flo
   const dim3 grid(static_cast<unsigned>(tiles), kv_heads, a.splits);
   const bool few = tiles * kv_heads < device_facts().compute_units;
   switch (dim / 16) {
-#define AKV_CASE(n)                                                       \
-  case n:                                                                 \
-    if (few) attention_f32_kernel<n, true><<<grid, 256, 0, stream>>>(a);  \
-    else attention_f32_kernel<n, false><<<grid, 256, 0, stream>>>(a);     \
+#define AKV_CASE(n)                                                                            \
+  case n:                                                                                      \
+    if (partial != nullptr) attention_f32_kernel<n, true, true><<<grid, 256, 0, stream>>>(a); \
+    else if (few) attention_f32_kernel<n, true, false><<<grid, 256, 0, stream>>>(a);           \
+    else attention_f32_kernel<n, false, false><<<grid, 256, 0, stream>>>(a);                   \
     break
     AKV_CASE(1); AKV_CASE(2); AKV_CASE(3); AKV_CASE(4); AKV_CASE(5); AKV_CASE(6); AKV_CASE(8); AKV_CASE(12); AKV_CASE(16);
 #undef AKV_CASE
