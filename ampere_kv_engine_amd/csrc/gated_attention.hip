@@ -924,12 +924,16 @@ __device__ __forceinline__ float sink_of(const SingleArgs& a, int vector) {
 }
 
 // SHAPED: scores have a softcap or a distance bias (their code, in every kernel, would be most of what a block fetches).
-template <int DT, int VT, bool SHAPED>
+// SHORT: one segment holds all keys that a token can see.  A wave that has one step of 16 keys takes that one alone, and one that
+// has none leaves zeros for the fold: 256 tokens of 30 keys, 16 heads of 64 of their own, 52 -> 20 us, of 128 77 -> 37 (14 and 21 in
+// `gated_attention_rows`, a wave per token and head), 16 / 4 heads of 128 24.5 -> 16.  Of several segments most are whole, and
+// a look at the steps first would stand before their loads.
+template <int DT, int VT, bool SHAPED, bool SHORT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 4))) void gated_attention_singles_kernel(const SingleArgs a) {
   constexpr int DIM = 32 * DT, VDIM = 16 * VT, kOwn = (VT + 3) / 4;      // tiles of values whose totals a wave keeps
   __shared__ float4_t sums_of[4][VT][kWave];
   __shared__ float top_of[4][16], weight_of[4][16];
-  const int wave = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x & (kWave - 1);
   const int col = lane & 15, grp = lane >> 4;
   const long n = blockIdx.x / a.segments;
   const int segment = blockIdx.x % a.segments;
@@ -942,151 +946,161 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 4))) voi
   const int first = segment * kSegmentSteps;
   if (first >= steps.all) return;
 
-  uint4 q[DT], keys[4][DT];
-  uint2 values[4][VT];
-  int at_key[4], offset[4];
-  long page[4];
-  bool foreign[4];
   const int* table = a.block_table + static_cast<long>(r) * a.table_width;
-  // (no load stands behind a test: the compiler would wait for it before the next; a step beyond the last asks for the last)
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int turn = first + wave + 4 * i;
-    const int key = steps.key(min(turn, steps.all - 1));
-    page[i] = table[key / a.page_size];
-    offset[i] = key % a.page_size;
-    at_key[i] = turn < steps.all ? key : pos + 1;                  // (none of a step beyond the last counts)
-  }
-  const bf16_t* qp = a.q + (n * a.q_heads + vector) * DIM + grp * 8;
-#pragma unroll
-  for (int d = 0; d < DT; ++d) q[d] = load_bf16x8(qp + d * 32);
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    foreign[i] = page[i] < 0 || page[i] >= a.num_pages;            // (a page that is not the request's is never read: its
-    const long from = (foreign[i] ? 0 : page[i]) * a.kv_heads + kvh;                                 // scores are NaN)
-    const bf16_t* kp = a.k_pages + ((from * a.page_size + offset[i] + col) * a.maps + map) * DIM + grp * 8;
-#pragma unroll
-    for (int d = 0; d < DT; ++d) keys[i][d] = load_bf16x8(kp + d * 32);
-  }
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const long from = (foreign[i] ? 0 : page[i]) * a.kv_heads + kvh;
-    const bf16_t* vp = a.v_pages + (from * VDIM + col) * a.page_size + offset[i] + grp * 4;
-#pragma unroll
-    for (int v = 0; v < VT; ++v) values[i][v] = *reinterpret_cast<const uint2*>(vp + static_cast<long>(v) * 16 * a.page_size);
-  }
-  __builtin_amdgcn_sched_barrier(0);             // (else the loads are moved down to where they are used)
-
-  const auto counts = [&](int i, int e) {
-    const int j = at_key[i] + 4 * grp + e;
-    return ((j >= steps.lowest) | (j < a.keep_first)) & (j <= pos);
-  };
-  const float bias_size = SHAPED && a.distance_bias != nullptr ? a.distance_bias[vector] : 0.f;
-  const float bias_rate = SHAPED && a.distance_bias != nullptr ? a.distance_bias[a.q_heads + vector] : 0.f;
-  float s[4][4], top = -INFINITY;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    float4_t acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int d = 0; d < DT; ++d)
-      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, keys[i][d]), __builtin_bit_cast(bf16x8_t, q[d]),
-                                                    acc, 0, 0, 0);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      float v = acc[e] * a.scale;
-      if constexpr (SHAPED) {
-        if (a.softcap > 0.f) v = a.softcap * tanhf(v / a.softcap);
-        if (a.distance_bias != nullptr)
-          v -= bias_size * log1pf(bias_rate * static_cast<float>(max(pos - at_key[i] - 4 * grp - e, 0)));
-      }
-      if (foreign[i]) v = __uint_as_float(0x7fc00000u);
-      s[i][e] = counts(i, e) ? v : -INFINITY;
-      top = fmaxf(top, s[i][e]);
-    }
-  }
-  top = fmaxf(top, __shfl_xor(top, 16, kWave));
-  top = fmaxf(top, __shfl_xor(top, 32, kWave));
-  const float shift = top == -INFINITY ? 0.f : top;
-  float weight = 0.f;
-  bool fine = true;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    uint32_t kept[2] = {0u, 0u};                 // slots that nobody has written hold anything: what does not count is zero
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const bool counted = counts(i, e);
-      s[i][e] = expf(s[i][e] - shift);           // (exp(-inf) where the key does not count)
-      weight += s[i][e];
-      kept[e >> 1] |= counted & !foreign[i] ? 0xffffu << (16 * (e & 1)) : 0u;
-    }
-#pragma unroll
-    for (int v = 0; v < VT; ++v) {
-      values[i][v].x &= kept[0];
-      values[i][v].y &= kept[1];
-      fine = fine & ((values[i][v].x & 0x7f80u) != 0x7f80u) & ((values[i][v].x & 0x7f800000u) != 0x7f800000u) &
-             ((values[i][v].y & 0x7f80u) != 0x7f80u) & ((values[i][v].y & 0x7f800000u) != 0x7f800000u);
-    }
-  }
-  weight += __shfl_xor(weight, 16, kWave);
-  weight += __shfl_xor(weight, 32, kWave);
-
   float4_t sums[VT];
 #pragma unroll
   for (int v = 0; v < VT; ++v) sums[v] = float4_t{0.f, 0.f, 0.f, 0.f};
-  if (__builtin_expect(__all(fine), 1)) {
-    // two steps of 16 keys are one product over 32: a lane's eight are keys 4 grp .. + 3 of the one and of the other
+  float top = -INFINITY, weight = 0.f;
+  // a wave's first STEPS steps: scores, their maximum, weights and weighted sums
+  const auto take = [&](auto count) {
+    constexpr int STEPS = decltype(count)::value;
+    uint4 q[DT], keys[STEPS][DT];
+    uint2 values[STEPS][VT];
+    int at_key[STEPS], offset[STEPS];
+    long page[STEPS];
+    bool foreign[STEPS];
+    // (no load stands behind a test: the compiler would wait for it before the next; a step beyond the last asks for the last)
 #pragma unroll
-    for (int i = 0; i < 4; i += 2) {
-      float left[8];
+    for (int i = 0; i < STEPS; ++i) {
+      const int turn = first + wave + 4 * i;
+      const int key = steps.key(min(turn, steps.all - 1));
+      page[i] = table[key / a.page_size];
+      offset[i] = key % a.page_size;
+      at_key[i] = turn < steps.all ? key : pos + 1;                  // (none of a step beyond the last counts)
+    }
+    const bf16_t* qp = a.q + (n * a.q_heads + vector) * DIM + grp * 8;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) left[e] = s[i + (e >> 2)][e & 3];
+    for (int d = 0; d < DT; ++d) q[d] = load_bf16x8(qp + d * 32);
 #pragma unroll
-      for (int part = 0; part < 3; ++part) {
-        uint32_t words[4];
+    for (int i = 0; i < STEPS; ++i) {
+      foreign[i] = page[i] < 0 || page[i] >= a.num_pages;            // (a page that is not the request's is never read: its
+      const long from = (foreign[i] ? 0 : page[i]) * a.kv_heads + kvh;                                 // scores are NaN)
+      const bf16_t* kp = a.k_pages + ((from * a.page_size + offset[i] + col) * a.maps + map) * DIM + grp * 8;
 #pragma unroll
-        for (int w = 0; w < 4; ++w) {
-          words[w] = bf16_pair(left[2 * w], left[2 * w + 1]);
-          left[2 * w] -= __uint_as_float(words[w] << 16);
-          left[2 * w + 1] -= __uint_as_float(words[w] & 0xffff0000u);
+      for (int d = 0; d < DT; ++d) keys[i][d] = load_bf16x8(kp + d * 32);
+    }
+#pragma unroll
+    for (int i = 0; i < STEPS; ++i) {
+      const long from = (foreign[i] ? 0 : page[i]) * a.kv_heads + kvh;
+      const bf16_t* vp = a.v_pages + (from * VDIM + col) * a.page_size + offset[i] + grp * 4;
+#pragma unroll
+      for (int v = 0; v < VT; ++v) values[i][v] = *reinterpret_cast<const uint2*>(vp + static_cast<long>(v) * 16 * a.page_size);
+    }
+    __builtin_amdgcn_sched_barrier(0);             // (else the loads are moved down to where they are used)
+
+    const auto counts = [&](int i, int e) {
+      const int j = at_key[i] + 4 * grp + e;
+      return ((j >= steps.lowest) | (j < a.keep_first)) & (j <= pos);
+    };
+    const float bias_size = SHAPED && a.distance_bias != nullptr ? a.distance_bias[vector] : 0.f;
+    const float bias_rate = SHAPED && a.distance_bias != nullptr ? a.distance_bias[a.q_heads + vector] : 0.f;
+    float s[STEPS][4];
+#pragma unroll
+    for (int i = 0; i < STEPS; ++i) {
+      float4_t acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int d = 0; d < DT; ++d)
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, keys[i][d]), __builtin_bit_cast(bf16x8_t, q[d]),
+                                                      acc, 0, 0, 0);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        float v = acc[e] * a.scale;
+        if constexpr (SHAPED) {
+          if (a.softcap > 0.f) v = a.softcap * tanhf(v / a.softcap);
+          if (a.distance_bias != nullptr)
+            v -= bias_size * log1pf(bias_rate * static_cast<float>(max(pos - at_key[i] - 4 * grp - e, 0)));
         }
-        const bf16x8_t weights = __builtin_bit_cast(bf16x8_t, make_uint4(words[0], words[1], words[2], words[3]));
-#pragma unroll
-        for (int v = 0; v < VT; ++v)
-          sums[v] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-              __builtin_bit_cast(bf16x8_t, make_uint4(values[i][v].x, values[i][v].y, values[i + 1][v].x, values[i + 1][v].y)),
-              weights, sums[v], 0, 0, 0);
+        if (foreign[i]) v = __uint_as_float(0x7fc00000u);
+        s[i][e] = counts(i, e) ? v : -INFINITY;
+        top = fmaxf(top, s[i][e]);
       }
     }
-  } else {
-    // an infinite or undefined value: a weight of zero takes nothing from it (zero times infinity is not zero), so the keys
-    // are added one by one - of step i the one that lies in element e of group `four` - where their weight is not zero
+    top = fmaxf(top, __shfl_xor(top, 16, kWave));
+    top = fmaxf(top, __shfl_xor(top, 32, kWave));
+    const float shift = top == -INFINITY ? 0.f : top;
+    bool fine = true;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll 1
-      for (int one = 0; one < 16; ++one) {
-        const int four = one >> 2, e = one & 3;
-        const float own = e == 0 ? s[i][0] : e == 1 ? s[i][1] : e == 2 ? s[i][2] : s[i][3];
-        const bool taken = __shfl(own, 16 * four + col, kWave) != 0.f;
-        const uint32_t place = grp == four ? 0xffffu << (16 * (e & 1)) : 0u;
-        const uint2 only = make_uint2(e < 2 ? place : 0u, e < 2 ? 0u : place);
-        short4_t part[3];
-        float left = own;
+    for (int i = 0; i < STEPS; ++i) {
+      uint32_t kept[2] = {0u, 0u};                 // slots that nobody has written hold anything: what does not count is zero
 #pragma unroll
-        for (int t = 0; t < 3; ++t) {
-          const uint32_t bits = bf16_bits(left);
-          left -= __uint_as_float(bits << 16);
-          part[t] = __builtin_bit_cast(short4_t, make_uint2((bits | bits << 16) & only.x, (bits | bits << 16) & only.y));
-        }
+      for (int e = 0; e < 4; ++e) {
+        const bool counted = counts(i, e);
+        s[i][e] = expf(s[i][e] - shift);           // (exp(-inf) where the key does not count)
+        weight += s[i][e];
+        kept[e >> 1] |= counted & !foreign[i] ? 0xffffu << (16 * (e & 1)) : 0u;
+      }
 #pragma unroll
-        for (int v = 0; v < VT; ++v) {
-          const short4_t value = __builtin_bit_cast(short4_t, make_uint2(values[i][v].x & only.x, values[i][v].y & only.y));
-          float4_t with = sums[v];
+      for (int v = 0; v < VT; ++v) {
+        values[i][v].x &= kept[0];
+        values[i][v].y &= kept[1];
+        fine = fine & ((values[i][v].x & 0x7f80u) != 0x7f80u) & ((values[i][v].x & 0x7f800000u) != 0x7f800000u) &
+               ((values[i][v].y & 0x7f80u) != 0x7f80u) & ((values[i][v].y & 0x7f800000u) != 0x7f800000u);
+      }
+    }
+    weight += __shfl_xor(weight, 16, kWave);
+    weight += __shfl_xor(weight, 32, kWave);
+
+    if (__builtin_expect(__all(fine), 1)) {
+      // two steps of 16 keys are one product over 32: a lane's eight are keys 4 grp .. + 3 of the one and of the other
 #pragma unroll
-          for (int t = 0; t < 3; ++t) with = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(value, part[t], with, 0, 0, 0);
-          if (taken) sums[v] = with;
+      for (int i = 0; i < STEPS; i += 2) {
+        float left[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) left[e] = i + (e >> 2) < STEPS ? s[min(i + (e >> 2), STEPS - 1)][e & 3] : 0.f;
+#pragma unroll
+        for (int part = 0; part < 3; ++part) {
+          uint32_t words[4];
+#pragma unroll
+          for (int w = 0; w < 4; ++w) {
+            words[w] = bf16_pair(left[2 * w], left[2 * w + 1]);
+            left[2 * w] -= __uint_as_float(words[w] << 16);
+            left[2 * w + 1] -= __uint_as_float(words[w] & 0xffff0000u);
+          }
+          const bf16x8_t weights = __builtin_bit_cast(bf16x8_t, make_uint4(words[0], words[1], words[2], words[3]));
+#pragma unroll
+          for (int v = 0; v < VT; ++v)
+            sums[v] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                __builtin_bit_cast(bf16x8_t, make_uint4(values[i][v].x, values[i][v].y, i + 1 < STEPS ? values[min(i + 1, STEPS - 1)][v].x : 0u,
+                                                        i + 1 < STEPS ? values[min(i + 1, STEPS - 1)][v].y : 0u)),
+                weights, sums[v], 0, 0, 0);
         }
       }
-  }
+    } else {
+      // an infinite or undefined value: a weight of zero takes nothing from it (zero times infinity is not zero), so the keys
+      // are added one by one - of step i the one that lies in element e of group `four` - where their weight is not zero
+#pragma unroll
+      for (int i = 0; i < STEPS; ++i)
+#pragma unroll 1
+        for (int one = 0; one < 16; ++one) {
+          const int four = one >> 2, e = one & 3;
+          const float own = e == 0 ? s[i][0] : e == 1 ? s[i][1] : e == 2 ? s[i][2] : s[i][3];
+          const bool taken = __shfl(own, 16 * four + col, kWave) != 0.f;
+          const uint32_t place = grp == four ? 0xffffu << (16 * (e & 1)) : 0u;
+          const uint2 only = make_uint2(e < 2 ? place : 0u, e < 2 ? 0u : place);
+          short4_t part[3];
+          float left = own;
+#pragma unroll
+          for (int t = 0; t < 3; ++t) {
+            const uint32_t bits = bf16_bits(left);
+            left -= __uint_as_float(bits << 16);
+            part[t] = __builtin_bit_cast(short4_t, make_uint2((bits | bits << 16) & only.x, (bits | bits << 16) & only.y));
+          }
+#pragma unroll
+          for (int v = 0; v < VT; ++v) {
+            const short4_t value = __builtin_bit_cast(short4_t, make_uint2(values[i][v].x & only.x, values[i][v].y & only.y));
+            float4_t with = sums[v];
+#pragma unroll
+            for (int t = 0; t < 3; ++t) with = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(value, part[t], with, 0, 0, 0);
+            if (taken) sums[v] = with;
+          }
+        }
+    }
+  };
+  const int own = (steps.all - first - wave + 3) >> 2;               // (steps of the wave, four at most)
+  if (!SHORT || own > 1)
+    take(std::integral_constant<int, 4>());
+  else if (own == 1)
+    take(std::integral_constant<int, 1>());
 
   // the four waves' parts, in their order; a token of one segment starts from its sink
 #pragma unroll
@@ -1192,11 +1206,16 @@ int akv_gated_attention_singles(const void* q, const void* k_pages, const void* 
   for (int first = 0; first < tokens; first += at_once) {
     const int count = min(at_once, tokens - first);
     const dim3 grid(static_cast<unsigned>(static_cast<long>(count) * segments), static_cast<unsigned>(columns));
+    const bool shaped = softcap > 0.f || distance_bias != nullptr;
 #define AKV_SINGLES(DT, VT)                                                                        \
-  if (softcap > 0.f || distance_bias != nullptr)                                                   \
-    gated_attention_singles_kernel<DT, VT, true><<<grid, 256, 0, stream>>>(a);                      \
+  if (segments > 1 && shaped)                                                                      \
+    gated_attention_singles_kernel<DT, VT, true, false><<<grid, 256, 0, stream>>>(a);               \
+  else if (segments > 1)                                                                           \
+    gated_attention_singles_kernel<DT, VT, false, false><<<grid, 256, 0, stream>>>(a);              \
+  else if (shaped)                                                                                 \
+    gated_attention_singles_kernel<DT, VT, true, true><<<grid, 256, 0, stream>>>(a);                \
   else                                                                                             \
-    gated_attention_singles_kernel<DT, VT, false><<<grid, 256, 0, stream>>>(a)
+    gated_attention_singles_kernel<DT, VT, false, true><<<grid, 256, 0, stream>>>(a)
 #define AKV_SINGLES_V(DT)                  \
   switch (vdim) {                          \
     case 32: AKV_SINGLES(DT, 2); break;    \
