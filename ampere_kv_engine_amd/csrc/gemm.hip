@@ -339,7 +339,10 @@ template <int TM, int TN>
 int launch_f32_wide(const float* x, const float* w, float* y, int rows, int outs, int k, const float* bias, bool wide_stores,
                     hipStream_t stream) {
   dim3 grid((outs + 32 * TM - 1) / (32 * TM), (rows + 32 * TN - 1) / (32 * TN));
-  linear_f32_wide_kernel<TM, TN, TM * TN == 4 ? 2 : 4><<<grid, 256, 0, stream>>>(x, w, y, rows, outs, k, bias, wide_stores);
+  if (k <= 32)       // (one step: those that are asked for ahead would add zeros)
+    linear_f32_wide_kernel<TM, TN, 1><<<grid, 256, 0, stream>>>(x, w, y, rows, outs, k, bias, wide_stores);
+  else
+    linear_f32_wide_kernel<TM, TN, TM * TN == 4 ? 2 : 4><<<grid, 256, 0, stream>>>(x, w, y, rows, outs, k, bias, wide_stores);
   return AKV_LAUNCH_STATUS();
 }
 
@@ -363,6 +366,8 @@ int launch_f32_wide(const float* x, const float* w, float* y, int rows, int outs
 //      8 rows: pairs 6.5 / 16.0 / 9.9 / 10.1 / 14.6 / 26.0 / 64    few 8.6 / 22.6 / 8.9 / 9.8 / 16.9 / 26.2 / 62
 // So: pairs up to 4 rows (also with 3: 2048 x 6144 13.4 against 20.6); from 5 on where they are one block a unit, or where
 // blocks of 16 are several a unit, but not many (100,000 x 1024 with 8 rows: 96 against 87).
+// Never where k is one segment: an instruction's second would be empty (32768 x 16 with 1 row 6.7 against 4.0, 32768 x 128 8.2
+// against 5.6).
 int launch_f32(const float* x, const float* w, float* y, int rows, int outs, int k, const float* bias, hipStream_t stream) {
   const bool wide_stores = outs % 4 == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0;
   const long units = device_facts().compute_units;
@@ -371,7 +376,7 @@ int launch_f32(const float* x, const float* w, float* y, int rows, int outs, int
     return (blocks + units - 1) / units;
   };
   const long tiles = (outs + 15) / 16;
-  if (rows <= 4 || (rows <= 8 && ((outs + 7) / 8 <= units || (tiles > units && tiles <= 4 * units))))
+  if (k > kSegment && (rows <= 4 || (rows <= 8 && ((outs + 7) / 8 <= units || (tiles > units && tiles <= 4 * units)))))
     return launch_f32_pairs(x, w, y, rows, outs, k, bias, wide_stores, stream);
   if (rows <= 16) return launch_f32_few<1>(x, w, y, rows, outs, k, bias, wide_stores, stream);
   if (rows <= 32 && tiles <= units) return launch_f32_few<2>(x, w, y, rows, outs, k, bias, wide_stores, stream);
