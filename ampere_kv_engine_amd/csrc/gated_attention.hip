@@ -926,7 +926,7 @@ __device__ __forceinline__ float sink_of(const SingleArgs& a, int vector) {
 // SHAPED: scores have a softcap or a distance bias (their code, in every kernel, would be most of what a block fetches).
 // SHORT: one segment holds all keys that a token can see.  A wave that has one step of 16 keys takes that one alone, and one that
 // has none leaves zeros for the fold: 256 tokens of 30 keys, 16 heads of 64 of their own, 52 -> 20 us, of 128 77 -> 37 (14 and 21 in
-// `gated_attention_rows`, a wave per token and head), 16 / 4 heads of 128 24.5 -> 16.  Of several segments most are whole, and
+// `gated_attention_rows`, a wave per token and head), 16 / 4 heads of 128 24.5 -> 12.6 (17).  Of several segments most are whole, and
 // a look at the steps first would stand before their loads.
 template <int DT, int VT, bool SHAPED, bool SHORT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 4))) void gated_attention_singles_kernel(const SingleArgs a) {
