@@ -754,3 +754,37 @@ def test_scaled_residual_norm_and_scaled_sum(hip, dtype):
         total = torch.empty_like(a)
         hip.scaled_sum(a, 0.8, b, 1.1, total)
         torch.testing.assert_close(total.float(), (a.float() * 0.8 + b.float() * 1.1).to(dtype).float(), rtol=1e-2 if dtype == torch.bfloat16 else 1e-6, atol=1e-6)
+
+
+@pytest.mark.parametrize("heads,kv_heads,maps,dim,vdim", [(16, 4, 1, 128, 128), (4, 4, 1, 32, 256), (3, 1, 2, 64, 64), (20, 1, 1, 256, 32)])
+@pytest.mark.parametrize("softcap", [None, 9.0])
+@pytest.mark.parametrize("sink", [False, True])
+def test_single_tokens_of_short_contexts_beside_a_long_one(hip, heads, kv_heads, maps, dim, vdim, softcap, sink):
+    """Where one segment holds all keys, waves have no step of 16 keys, one or several, and take what they have; beside a longer request they
+    take four always: the same bits.  One value in a short request is infinite: it reaches its own request alone."""
+    torch.manual_seed(dim + heads)
+    page, befores = 16, [0, 1, 15, 16, 17, 40, 63, 64, 65, 100, 127, 128, 200, 255, 500]
+    need = [before // page + 1 for before in befores]
+    table = torch.full((len(befores), max(need)), -1, dtype=torch.int32)
+    order = torch.randperm(sum(need)).tolist()
+    for r, pages in enumerate(need):
+        table[r, :pages] = torch.tensor([order.pop() for _ in range(pages)])
+    k_pages = torch.randn(sum(need), kv_heads, page, maps * dim, device=DEVICE).bfloat16()
+    v_pages = torch.randn(sum(need), kv_heads, vdim, page, device=DEVICE).bfloat16()
+    q = torch.randn(len(befores), heads * maps * dim, device=DEVICE).bfloat16()
+
+    def of(count):
+        out = torch.full((count, heads * maps * vdim), float("nan"), dtype=torch.bfloat16, device=DEVICE)
+        meta = SimpleNamespace(block_table=table[:count].contiguous().to(DEVICE), rows=None, width=table.shape[1])
+        hip.gated_attention(q[:count].contiguous(), k_pages, v_pages, None, 0, _ctx(befores[:count], [1] * count), meta, heads, kv_heads, dim,
+                            vdim, dim ** -0.5, softcap, None, None, sink, out, maps=maps)
+        return out
+
+    short, beside = of(len(befores) - 1), of(len(befores))
+    assert torch.isfinite(beside).all()
+    assert torch.equal(short, beside[:-1])
+    v_pages[table[6, 2], :, 1, 3] = float("inf")           # position 35 of the request of 64 keys
+    poisoned = of(len(befores) - 1)
+    assert not torch.isfinite(poisoned[6]).all()
+    assert torch.equal(poisoned[:6], short[:6]) and torch.equal(poisoned[7:], short[7:])
+    assert torch.equal(poisoned.view(torch.int16), of(len(befores))[:-1].view(torch.int16))
