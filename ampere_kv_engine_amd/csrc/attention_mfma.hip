@@ -683,7 +683,7 @@ __global__ __launch_bounds__(64, (SPLIT && NQ == 1 && D <= 128) ? 2 : 1) void at
 // per tile this takes three quarters of the traffic off the vector memory pipe and the address arithmetic off the
 // waves.  With 16 columns per wave (NQ = 1) three blocks fit a compute unit; with 32 (NQ = 2) two, which do a step for
 // twice the columns with the same loads, barriers and bookkeeping - the host takes them where they still fill the
-// device.  In LDS a key row is stored at the MFMA row it feeds (tile j, row rho); a value row is one dim's 32 keys.
+// device.  (Heads of 64 and 128 on pages of 16 and more have a kernel of their own for 32 columns, below.)  In LDS a key row is stored at the MFMA row it feeds (tile j, row rho); a value row is one dim's 32 keys.
 // Pages must hold at least 8 tokens (an aligned run of 8 keys of a value row is one 16-byte piece).
 constexpr int kSharedWaves = 4;
 // Rows in LDS, in bfloat16.  16 lanes read 16 bytes each from 16 consecutive rows; such a read runs at full rate when
@@ -1137,6 +1137,362 @@ __global__ __launch_bounds__(64 * kSharedWaves, D <= 128 ? (NQ == 1 ? 3 : 2) : 1
   attention_shared_body<NQ, SP>(a, static_cast<int>(blockIdx.x), static_cast<int>(threadIdx.x));
 }
 
+// ---- prompt portions on tiles of 32 columns: both products on 32 x 32 tiles, three steps in the air ----------------------
+// Heads of 64 and 128 on pages of 16 and more.  A block of 4 waves works on 4 consecutive tiles of 32 columns of one
+// request and one kv head, as above; what differs is how a step of 32 keys passes through:
+// * Keys and values come into LDS by loads that write it directly (no register holds them), three steps before they are
+//   read, in rings of four steps.  A wave's load fills 1 KB in the order of its lanes, so there is no padding; rows are
+//   read without bank conflicts because the 16-byte pieces of a row are stored exchanged by the row's number.
+// * The matrix instruction is the one of 32 x 32 x 16: a wave reads a step's 2 x 32 * D * 2 bytes of operands for 32
+//   columns at half the instructions of the 16 x 16 form, and the vector unit has the slots that this frees.
+// * A turn of the loop multiplies the keys of step j, makes the weights of step j - 1 and sums the values of step j - 2:
+//   three pieces of work that do not wait for each other, so the matrix cores run while the vector unit computes weights -
+//   in one wave, and beside the other wave of its SIMD.
+// * Whether a reference point must move is read off the weights' sum, which is needed anyway: as long as no lane's 16
+//   weights add up to more than 2^8, no weight exceeds 2^8.  Else the maximum is searched, and a reference moves if the
+//   maximum passed it by 2^kSlack: a lane whose weights are all below that adds up to less than the 2^8 that ask.
+// What bounds it: the matrix instructions are busy 67 % of the cycles at the 1.87 GHz that the device holds under them (2 of
+// 3 of them are the weighted sum's, a third the second part of the weights), the vector unit 50 %; in the same run the
+// order of a turn, the distance of the loads and what stands between the matrix instructions move it by 1 to 3 % only.
+// Where the device has one block a unit (short prompts) a wave alone issues an instruction every 5 cycles, 195 a turn.
+// 32 heads of 8 key heads, against the kernel above at its better width: 2,048 tokens 87 -> 72 us, 1,000 tokens of 40 heads
+// 41 -> 37; 64 heads, 2,048 tokens after 6,144 768 -> 600 us (0.80 PFLOP/s, the weights' second part not counted).
+// Every address of a step is a page's address (scalar) plus a constant of the thread: pages are looked up at indices held
+// inside the range, keys beyond it (their slots hold anything) are hidden from the scores by position, values outside it are
+// blanked as they are read from LDS.
+#if AKV_HEAD_DIM == 64 || AKV_HEAD_DIM == 128
+#define AKV_PROMPT_TILES 1
+constexpr float kSlack = 4.f;
+
+typedef __attribute__((ext_vector_type(16))) float floatx16;
+__device__ __forceinline__ floatx16 mfma32(uintx4 a, uintx4 b, floatx16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+
+// SP: pages per step of 32 keys (2: pages of 16, 1: of 32 or more)
+template <int SP>
+__device__ __forceinline__ void attention_prompt_body(const Args& a, const int block, const int tid) {
+  constexpr int KP = D / 8;        // 16-byte pieces of a key's row
+  constexpr int QT = D / 16;       // 16-dim steps of the score product
+  constexpr int OT = D / 32;       // 32-dim tiles of the output
+  constexpr int kLoads = D / 64;   // pieces of a step's keys that a thread moves, and as many of its values
+  constexpr int kStep = 32 * D;    // elements of a step's keys, and of its values
+  __shared__ __align__(1024) bf16_t k_lds[4 * kStep];
+  __shared__ __align__(1024) bf16_t v_lds[4 * kStep];
+  const int page_shift = SP == 2 ? 4 : a.page_shift;
+  const int lane = tid & 63, c32 = lane & 31, h = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // the order of the blocks: as in attention_shared_body
+  const int heads = a.kv_heads * a.head_groups, round = 2 * a.units;
+  const int turn = block / round, within = block % round;
+  const int total = a.tiles * heads, in_round = min(round, total - turn * round);
+  const int rank = turn * round + (within < a.units ? within : in_round - 1 - (within - a.units));
+  Tile t = find_tile(a, a.tiles - 1 - rank / heads, kSharedWaves * a.tokens_per_tile);
+  if (!t.found) return;  // the same in every wave of the block
+  t.request = __builtin_amdgcn_readfirstlane(t.request);
+  t.first_row = __builtin_amdgcn_readfirstlane(t.first_row);
+  t.tokens = __builtin_amdgcn_readfirstlane(t.tokens);
+  t.first_pos = __builtin_amdgcn_readfirstlane(t.first_pos);
+  const int kvh = (rank % heads) / a.head_groups, hg = (rank % heads) % a.head_groups;
+  const uintx4 zero = uintx4{0u, 0u, 0u, 0u};
+
+  // this lane's column
+  const int wave_token0 = wave * a.tokens_per_tile;
+  const int token = wave_token0 + c32 / a.heads_per_tile, head_in_group = hg * a.heads_per_tile + c32 % a.heads_per_tile;
+  const bool col_valid = token < t.tokens && c32 / a.heads_per_tile < a.tokens_per_tile && head_in_group < a.group;
+  const int col_pos = col_valid ? t.first_pos + token : -1;   // (a column that is no (token, head) pair sees nothing)
+  const uint32_t span = a.window > 0 ? static_cast<uint32_t>(a.window) : 0x80000000u;   // keys a column sees: pos - key < span
+  const long col_at = (static_cast<long>(t.first_row + token) * a.q_heads + kvh * a.group + head_in_group) * D;
+  uintx4 qreg[QT];
+#pragma unroll
+  for (int kt = 0; kt < QT; ++kt) qreg[kt] = col_valid ? *reinterpret_cast<const uintx4*>(a.q + col_at + kt * 16 + h * 8) : zero;
+
+  // keys the block looks at, in steps of 32 from `first_base`; steps the wave's tokens see: wave_from .. wave_to - 1; steps
+  // all of whose keys all its tokens see: calm_from .. calm_to - 1
+  const int last_pos = t.first_pos + t.tokens - 1;
+  const int range_lo = a.window > 0 ? max(0, t.first_pos - a.window + 1) : 0;
+  const int range_hi = last_pos;
+  const int first_base = range_lo & ~31;
+  const int steps = ((range_hi - first_base) >> 5) + 1;
+  int wave_from = 0, wave_to = 0, calm_from = 0, calm_to = 0;
+  if (wave_token0 < t.tokens) {
+    const int wave_first = t.first_pos + wave_token0;
+    const int wave_last = t.first_pos + min(t.tokens, wave_token0 + a.tokens_per_tile) - 1;
+    wave_to = ((wave_last - first_base) >> 5) + 1;
+    calm_to = (wave_first + 1 - first_base) >> 5;
+    if (a.window > 0) {
+      wave_from = max(0, wave_first - a.window + 1 - first_base) >> 5;
+      calm_from = (max(range_lo, wave_last - a.window + 1) - first_base + 31) >> 5;
+    }
+  }
+
+  // ---- the block's loads: pieces of 16 bytes, piece p * 256 + tid of the step's keys and of its values ------------------
+  // Keys lie row by row in the order of the matrix instruction: its row 8a + 4h + i is key 16 (a / 2) + 8h + 4 (a % 2) + i
+  // of the step, so that a lane's scores 8t .. 8t + 7 are the consecutive keys 16t + 8h .. + 7 - one operand of the second
+  // product.  Values lie as two halves of 16 keys, a dim's half in 32 bytes.
+  typedef const __attribute__((address_space(4))) int* scalar_ints;
+  typedef __attribute__((address_space(3))) bf16_t* lds_rows;
+  const scalar_ints table = reinterpret_cast<scalar_ints>(reinterpret_cast<uintptr_t>(
+      a.block_table + static_cast<long>(a.table_rows != nullptr ? __builtin_amdgcn_readfirstlane(a.table_rows[t.request]) : t.request) * a.table_width));
+  const char* k_bytes = reinterpret_cast<const char*>(a.k_pages);
+  const char* v_bytes = reinterpret_cast<const char*>(a.v_pages);
+  const uint32_t page_bytes = static_cast<uint32_t>(a.kv_heads) * D * 2u << page_shift;
+  const uint32_t head_bytes = static_cast<uint32_t>(kvh) * D * 2u << page_shift;
+  const int page_mask = (1 << page_shift) - 1;
+  uint32_t k_from[kLoads], v_from[kLoads];   // byte offset inside the page, without what the step's first key adds
+  int k_sel[kLoads], v_sel[kLoads];          // which of the step's pages (the same in every lane of a wave)
+#pragma unroll
+  for (int p = 0; p < kLoads; ++p) {
+    const int c = p * 256 + tid, row = c / KP;
+    const int piece = (c % KP) ^ (D == 128 ? row & 15 : (row >> 1) & 7);
+    const int key = ((row >> 4) << 4) + (((row >> 2) & 1) << 3) + (((row >> 3) & 1) << 2) + (row & 3);
+    k_sel[p] = SP == 1 ? 0 : __builtin_amdgcn_readfirstlane(row >> 4);
+    k_from[p] = head_bytes + piece * 16u + static_cast<uint32_t>(SP == 2 ? key & 15 : key) * (D * 2u);
+    const int half = c / (2 * D), dim = (c % (2 * D)) >> 1, run = (c & 1) ^ ((dim >> 3) & 1);
+    v_sel[p] = SP == 1 ? 0 : __builtin_amdgcn_readfirstlane(half);
+    v_from[p] = head_bytes + (static_cast<uint32_t>(dim) << (page_shift + 1)) + (SP == 2 ? 0u : half * 32u) + run * 16u;
+  }
+  const int page_lo = range_lo >> page_shift, page_hi = range_hi >> page_shift;
+  const uint32_t page_count = static_cast<uint32_t>(min(a.num_pages, 0x7fffffffL));
+  bool bad = false;
+  auto lookup = [&](int step, int (&pages)[SP]) {
+    const int first = (first_base + step * 32) >> page_shift;
+#pragma unroll
+    for (int i = 0; i < SP; ++i) pages[i] = table[min(max(first + i, page_lo), page_hi)];
+  };
+  // Page addresses of four steps: a step's keys are asked for three turns before its own, its values one before.
+  size_t at[4][SP];
+  int pending[4][SP];   // pages of the four steps whose keys are asked for next
+  // One load of 16 bytes a lane into LDS, in the order of the lanes, from a scalar address and the lane's offset.  Written
+  // as text because the compiler, which does not see that rings keep such loads and the reads of LDS apart, waits for all
+  // of them before every read; the turns' own counted waits are what orders them.  Nothing is loaded into registers.
+  auto into_lds = [&](const char* from, uint32_t offset, uint32_t to) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                 :: "s"(to), "v"(offset), "s"(from));
+  };
+  const uint32_t k_base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_rows)(&k_lds[wave * 512])));
+  const uint32_t v_base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_rows)(&v_lds[wave * 512])));
+  auto keys_of = [&](int step, int u) {   // (u: the step modulo 4)
+    const uint32_t in = SP == 2 ? 0u : static_cast<uint32_t>((first_base + step * 32) & page_mask) * (D * 2u);
+#pragma unroll
+    for (int p = 0; p < kLoads; ++p)
+      into_lds(k_bytes + (k_sel[p] == 0 ? at[u][0] : at[u][SP - 1]) + in, k_from[p], k_base + u * (kStep * 2u) + p * 4096u);
+  };
+  auto values_of = [&](int step, int u) {
+    const uint32_t in = SP == 2 ? 0u : static_cast<uint32_t>((first_base + step * 32) & page_mask) * 2u;
+#pragma unroll
+    for (int p = 0; p < kLoads; ++p)
+      into_lds(v_bytes + (v_sel[p] == 0 ? at[u][0] : at[u][SP - 1]) + in, v_from[p], v_base + u * (kStep * 2u) + p * 4096u);
+  };
+  auto resolve = [&](int u, int which) {
+#pragma unroll
+    for (int i = 0; i < SP; ++i) {
+      uint32_t page = static_cast<uint32_t>(pending[which][i]);
+      if (page >= page_count) {
+        bad = true;
+        page = 0;
+      }
+      at[u][i] = static_cast<size_t>(page) * page_bytes;
+    }
+  };
+  // the loads of turn j (= u modulo 4): the keys of step j + 3, the values of step j + 1
+  auto ask = [&](int j, int u) {
+    resolve((u + 3) & 3, u);
+    keys_of(j + 3, (u + 3) & 3);
+    values_of(j + 1, (u + 1) & 3);
+    if (u == 3) {
+#pragma unroll
+      for (int v = 0; v < 4; ++v) lookup(j + 4 + v, pending[v]);
+    }
+  };
+  // where a lane reads its operands: key row c32, dims kt * 16 + 8h .. + 7; value dim dt * 32 + c32, keys 16t + 8h .. + 7
+  const uint32_t k_row = c32 * (D * 2u) + ((h ^ (D == 128 ? c32 & 15 : (c32 >> 1) & 7)) << 4);
+  const uint32_t v_row = c32 * 32u + ((h ^ ((c32 >> 3) & 1)) << 4);
+  auto key_piece = [&](int buffer, int kt) {
+    return *reinterpret_cast<const uintx4*>(reinterpret_cast<const char*>(k_lds) + (k_row ^ (kt * 32u)) + buffer * (kStep * 2u));
+  };
+  auto value_piece = [&](int buffer, int half, int dt) {
+    return *reinterpret_cast<const uintx4*>(reinterpret_cast<const char*>(v_lds) + v_row + (buffer * (kStep * 2u) + half * (D * 32u) + dt * 1024u));
+  };
+
+  // ---- the three pieces of work -------------------------------------------------------------------------------------------
+  floatx16 o[OT], s[2];      // sums; scores of two steps
+  uintx4 high[2][2], low[2][2];   // weights of two steps, each as two bfloat16 numbers (16 bits of mantissa together)
+  float away = col_valid ? INFINITY : -1e30f;   // minus the reference point; +inf: nothing seen yet
+  float l = 0.f;             // this lane's part of its column's sum of weights
+#pragma unroll
+  for (int dt = 0; dt < OT; ++dt)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) o[dt][r] = 0.f;
+  auto scores = [&](int buffer, floatx16& to) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) to[r] = 0.f;
+#pragma unroll
+    for (int kt = 0; kt < QT; ++kt) to = mfma32(key_piece(buffer, kt), qreg[kt], to);
+  };
+  auto hide = [&](int step, floatx16& of) {
+    const int reach = col_pos - (first_base + step * 32 + h * 8);
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+      if (static_cast<uint32_t>(reach - ((r >> 3) * 16 + (r & 7))) >= span) of[r] = -INFINITY;
+  };
+  // weights 2^(s * scale + away) of a step's scores; returns this lane's sum of them
+  auto weigh = [&](const floatx16& of, float shift, uintx4 (&hi)[2], uintx4 (&lo)[2]) {
+    float sum[4];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const floatx2 p = {__builtin_amdgcn_exp2f(fmaf(of[2 * e], a.scale_log2, shift)),
+                         __builtin_amdgcn_exp2f(fmaf(of[2 * e + 1], a.scale_log2, shift))};
+      sum[e & 1] = e < 2 ? p[0] : sum[e & 1] + p[0];
+      sum[2 + (e & 1)] = e < 2 ? p[1] : sum[2 + (e & 1)] + p[1];
+      const uint32_t bits = __builtin_bit_cast(uint32_t, __builtin_convertvector(p, bf16x2));
+      const floatx2 rest = {p[0] - __uint_as_float(bits << 16), p[1] - __uint_as_float(bits & 0xffff0000u)};
+      hi[e >> 2][e & 3] = bits;
+      lo[e >> 2][e & 3] = __builtin_bit_cast(uint32_t, __builtin_convertvector(rest, bf16x2));
+    }
+    return (sum[0] + sum[1]) + (sum[2] + sum[3]);
+  };
+  // some lane's weights add up to more than 2^8 (or to no number): the reference points follow the maximum
+  auto follow = [&](const floatx16& of, uintx4 (&hi)[2], uintx4 (&lo)[2]) {
+    float top = of[0];
+#pragma unroll
+    for (int r = 1; r < 16; ++r) top = fmaxf(top, of[r]);
+    const float scaled = max_over_halves(top) * a.scale_log2;   // the scale is positive: max commutes with it
+    const float m = -away;                                      // -inf: nothing seen yet
+    if (scaled > m + kSlack) {
+      const float correction = __builtin_amdgcn_exp2f(m - scaled);
+      away = -scaled;
+      l *= correction;
+#pragma unroll
+      for (int dt = 0; dt < OT; ++dt) o[dt] *= correction;
+    }
+    return weigh(of, away == INFINITY ? 0.f : away, hi, lo);    // (nothing seen: every weight is 0, no NaN)
+  };
+  auto gather = [&](int buffer, const uintx4 (&hi)[2], const uintx4 (&lo)[2]) {
+#pragma unroll
+    for (int half = 0; half < 2; ++half)
+#pragma unroll
+      for (int dt = 0; dt < OT; ++dt) {
+        const uintx4 values = value_piece(buffer, half, dt);
+        o[dt] = mfma32(values, lo[half], mfma32(values, hi[half], o[dt]));
+      }
+  };
+  // the same for the steps that hold the first and the last key: slots outside hold anything, NaN included (never written, or
+  // of a page that stands in for one that a window has passed)
+  auto gather_edge = [&](int step, int buffer, const uintx4 (&hi)[2], const uintx4 (&lo)[2]) {
+    const uint32_t keys = static_cast<uint32_t>(range_hi - range_lo);
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      const int key = first_base + step * 32 + half * 16 + h * 8 - range_lo;
+      uintx4 keep;
+#pragma unroll
+      for (int w = 0; w < 4; ++w)
+        keep[w] = (static_cast<uint32_t>(key + 2 * w) <= keys ? 0xffffu : 0u) | (static_cast<uint32_t>(key + 2 * w + 1) <= keys ? 0xffff0000u : 0u);
+#pragma unroll
+      for (int dt = 0; dt < OT; ++dt) {
+        const uintx4 values = value_piece(buffer, half, dt) & keep;
+        o[dt] = mfma32(values, lo[half], mfma32(values, hi[half], o[dt]));
+      }
+    }
+  };
+
+  // ---- the turns: scores of step j, weights of step j - 1, sums of step j - 2; the keys of step j + 3 and the values of
+  // step j + 1 are asked for (the loads of two later turns may still be on their way when a turn begins) ---------------------
+  auto begin = [&]() {
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"(4 * kLoads) : "memory");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+  };
+#pragma unroll
+  for (int i = 0; i < SP; ++i) at[2][i] = at[3][i] = 0;   // (steps -2 and -1 do not exist: what their loads bring is not read)
+#pragma unroll
+  for (int v = 1; v < 4; ++v) lookup(v - 1, pending[v]);
+#pragma unroll
+  for (int j = -3; j < 0; ++j) ask(j, j + 4);
+  const int turns = steps + 2;
+  // `count` turns from j0 = `from` (modulo 4) with a test for everything that may be missing or hidden
+  auto careful = [&](int j0, auto from, auto count) {
+#pragma unroll
+    for (int i = 0; i < decltype(count)::value; ++i) {
+      const int j = j0 + i, u = (decltype(from)::value + i) & 3;
+      if (j >= turns) break;
+      begin();
+      ask(j, u);
+      __builtin_amdgcn_sched_barrier(0);
+      if (j - 2 >= wave_from && j - 2 < wave_to) {
+        if (j - 2 == 0 || j - 2 == steps - 1) gather_edge(j - 2, (u + 2) & 3, high[i & 1], low[i & 1]);
+        else gather((u + 2) & 3, high[i & 1], low[i & 1]);
+      }
+      if (j - 1 >= wave_from && j - 1 < wave_to) {
+        floatx16& of = s[(i + 1) & 1];
+        if (j - 1 < calm_from || j - 1 >= calm_to) hide(j - 1, of);
+        float sum = weigh(of, away, high[(i + 1) & 1], low[(i + 1) & 1]);
+        if (__any(!(sum <= 256.f))) sum = follow(of, high[(i + 1) & 1], low[(i + 1) & 1]);
+        l += sum;
+      }
+      if (j >= wave_from && j < wave_to) scores(u, s[i & 1]);
+    }
+  };
+  // Three loops, one after the other (in a loop of its own a calm turn's sums stay in their registers): turns before the
+  // calm ones, the calm ones - all three pieces of work are there, nothing is hidden -, and those after.
+  const std::integral_constant<int, 0> zeroth{};
+  const std::integral_constant<int, 2> second{}, two{};
+  const std::integral_constant<int, 4> four{};
+  careful(0, zeroth, two);
+  int j0 = 2;
+  for (; j0 < turns && j0 < calm_from + 2; j0 += 4) careful(j0, second, four);
+  for (; j0 + 3 < min(calm_to + 1, wave_to); j0 += 4) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int u = (2 + i) & 3;
+      begin();
+      ask(j0 + i, u);
+      __builtin_amdgcn_sched_barrier(0);
+      scores(u, s[u & 1]);
+      float sum = weigh(s[(u + 1) & 1], away, high[(u + 1) & 1], low[(u + 1) & 1]);
+      gather((u + 2) & 3, high[u & 1], low[u & 1]);
+      // (the weights' two parts are made here, not behind the test that may make them anew)
+#pragma unroll
+      for (int half = 0; half < 2; ++half) asm volatile("" : "+v"(high[(u + 1) & 1][half]), "+v"(low[(u + 1) & 1][half]));
+      // The order of the turn: a step's keys are read ahead, and between two matrix instructions stand the vector
+      // instructions that fit beside one.
+      __builtin_amdgcn_sched_group_barrier(0x100, QT, 0);
+#pragma unroll
+      for (int x = 0; x < QT + 4 * OT; ++x) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, D == 128 ? 5 : 9, 0);
+        if (D == 64 || x % 3 != 2) __builtin_amdgcn_sched_group_barrier(0x400, D == 64 ? 2 : 1, 0);
+        if (x < 2 * OT) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+      }
+      if (__any(!(sum <= 256.f))) sum = follow(s[(u + 1) & 1], high[(u + 1) & 1], low[(u + 1) & 1]);
+      l += sum;
+    }
+  }
+  for (; j0 < turns; j0 += 4) careful(j0, second, four);
+
+  // ---- results: a lane holds, of its column, dims dt * 32 + 8 i + 4h .. + 3 ------------------------------------------------
+  const auto halves = __builtin_amdgcn_permlane32_swap(__float_as_uint(l), __float_as_uint(l), false, false);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (the last turns' loads still write this block's LDS)
+  const float inv = bad ? __uint_as_float(0x7fc00000u) : 1.f / (__uint_as_float(halves[0]) + __uint_as_float(halves[1]));
+  if (!col_valid) return;
+#pragma unroll
+  for (int dt = 0; dt < OT; ++dt)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      uintx2 packed;
+      packed.x = bf16_pair(o[dt][4 * i] * inv, o[dt][4 * i + 1] * inv);
+      packed.y = bf16_pair(o[dt][4 * i + 2] * inv, o[dt][4 * i + 3] * inv);
+      *reinterpret_cast<uintx2*>(a.out + col_at + dt * 32 + i * 8 + h * 4) = packed;
+    }
+}
+
+template <int SP>
+__global__ __launch_bounds__(64 * kSharedWaves, 2) void attention_prompt_kernel(const Args a) {
+  attention_prompt_body<SP>(a, static_cast<int>(blockIdx.x), static_cast<int>(threadIdx.x));
+}
+#endif
+
 // ---- single tokens and short prompt portions in one launch ---------------------------------------------------------------
 // A step that decodes some requests and feeds a short portion of another's prompt has two attention launches that do
 // not depend on each other and do not fill the device: the single tokens' keys stream from memory, the portion's few
@@ -1286,10 +1642,18 @@ int launch(const Args& a, int tiles, bool shared, hipStream_t stream) {
   dim3 grid(tiles, a.kv_heads * a.head_groups, a.num_splits);
   if (shared) {
     const dim3 blocks(tiles * a.kv_heads * a.head_groups);
-    if (a.page_shift >= 5) attention_shared_kernel<NQ, 1><<<blocks, 64 * kSharedWaves, 0, stream>>>(a);
-    else if (a.page_shift == 4) attention_shared_kernel<NQ, 2><<<blocks, 64 * kSharedWaves, 0, stream>>>(a);
-    else if (a.page_shift == 3) attention_shared_kernel<NQ, 4><<<blocks, 64 * kSharedWaves, 0, stream>>>(a);
-    else return -2;
+    if (a.page_shift < 3) return -2;
+    if (a.page_shift == 3) {
+      attention_shared_kernel<NQ, 4><<<blocks, 64 * kSharedWaves, 0, stream>>>(a);
+#ifdef AKV_PROMPT_TILES
+    } else if constexpr (NQ == 2) {
+      if (a.page_shift >= 5) attention_prompt_kernel<1><<<blocks, 64 * kSharedWaves, 0, stream>>>(a);
+      else attention_prompt_kernel<2><<<blocks, 64 * kSharedWaves, 0, stream>>>(a);
+#endif
+    } else {
+      if (a.page_shift >= 5) attention_shared_kernel<NQ, 1><<<blocks, 64 * kSharedWaves, 0, stream>>>(a);
+      else attention_shared_kernel<NQ, 2><<<blocks, 64 * kSharedWaves, 0, stream>>>(a);
+    }
     return AKV_LAUNCH_STATUS();
   }
   const bool items = a.plan != nullptr;  // single tokens whose keys were cut on the device: always with the merge

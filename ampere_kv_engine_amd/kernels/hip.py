@@ -1094,12 +1094,20 @@ class HipKernels(PartsKernels, KernelSet):
         blocks = sum((starts[r + 1] - starts[r] + per_block - 1) // per_block for r in range(first, ctx.num_seqs))
         return blocks * kv_heads * ((group + heads_per_tile - 1) // heads_per_tile)
 
-    def _wide_shared_tiles(self, ctx, first, q_heads, kv_heads) -> bool:
-        """Whether the prompt portions of the step go to blocks of 4 x 32 columns rather than 4 x 16.  The wide
-        blocks do a step of 32 keys for twice the columns with the same loads and bookkeeping (a fifth to a quarter
-        faster where they fill the device), but there are half as many of them, and two per compute unit instead of
-        three: they are taken when there are two or more per compute unit and the keys are many (measured on
+    def _wide_shared_tiles(self, ctx, first, q_heads, kv_heads, head_dim, page_size) -> bool:
+        """Whether the prompt portions of the step go to blocks of 4 x 32 columns rather than 4 x 16.
+        Heads of 64 and 128 on pages of 16 and more have a kernel of their own for 32 columns, whose turns overlap: it is
+        the faster one from some hundred keys on however few its blocks are, and pays for its longer start before
+        (heads of 128, narrow / wide us: 256 keys 15.3 / 16.9, 320 keys 17.3 / 17.4, 400 keys of 16 heads 19.3 / 18.5,
+        1,128 keys 39.7 / 33.1, 8,171 keys 233 / 181; heads of 64, half the work a key: 512 keys 14.1 / 15.9, 2,048 keys
+        45.0 / 46.1, 8,192 keys 234 / 201).
+        Elsewhere the wide blocks do a step of 32 keys for twice the columns with the same loads and bookkeeping (a fifth
+        to a quarter faster where they fill the device), but there are half as many of them, and two per compute unit
+        instead of three: they are taken when there are two or more per compute unit and the keys are many (measured on
         prompts of 512 to 8,192 tokens after histories of 0 to 15,360)."""
+        longest = max(ctx.host_seq_lens[first:ctx.num_seqs])
+        if head_dim in (64, 128) and page_size >= 16:
+            return longest >= (384 if head_dim == 128 else 4096)
         group = q_heads // kv_heads
         heads_per_tile = min(group, 32)
         per_block = 4 * (32 // heads_per_tile)
@@ -1107,7 +1115,7 @@ class HipKernels(PartsKernels, KernelSet):
         blocks = sum((starts[r + 1] - starts[r] + per_block - 1) // per_block for r in range(first, ctx.num_seqs))
         blocks *= kv_heads * ((group + heads_per_tile - 1) // heads_per_tile)
         units = self.compute_units
-        return blocks >= 2 * units and (max(ctx.host_seq_lens[first:ctx.num_seqs]) >= 4096 or 2 * blocks >= 5 * units)
+        return blocks >= 2 * units and (longest >= 4096 or 2 * blocks >= 5 * units)
 
     def _matrix_core_attention(self, dtype, page_size) -> bool:
         fits = page_size >= 4 and page_size & (page_size - 1) == 0
@@ -1227,7 +1235,7 @@ class HipKernels(PartsKernels, KernelSet):
                 if shared and nq == 2:
                     wide = self.wide_prompt_tiles
                     if wide is None:
-                        wide = self._wide_shared_tiles(ctx, decodes, q_heads, kv_heads)
+                        wide = self._wide_shared_tiles(ctx, decodes, q_heads, kv_heads, head_dim, page_size)
                     nq = 2 if wide else 1
                 self._attention_mfma(*common, decodes, ctx.num_seqs - decodes, nq, False, shared=shared)
 

@@ -1419,6 +1419,50 @@ def test_attention_prompt_portions(hip, ref, shared, q_heads, kv_heads, dim, pag
     torch.testing.assert_close(got.cpu().float(), want.float(), **attention_tol(torch.bfloat16))
 
 
+@pytest.mark.parametrize("q_heads,kv_heads,dim,page_size", [(8, 2, 128, 16), (3, 3, 128, 32), (40, 2, 64, 16), (8, 1, 64, 128)])
+@pytest.mark.parametrize("portions", [[(0, 1), (0, 31), (0, 32), (0, 33)], [(31, 2), (64, 97), (1, 128), (95, 1)], [(0, 257), (300, 129)]])
+@pytest.mark.parametrize("window", [None, 1, 33, 150])
+@pytest.mark.parametrize("spike", [None, (1, 20)])
+def test_attention_on_tiles_of_32_columns(hip, ref, q_heads, kv_heads, dim, page_size, portions, window, spike):
+    """The kernel of heads of 64 and 128 on pages of 16 and more: contexts around its steps of 32 keys, fewer steps than its turns
+    are deep, first and last steps that a window cuts, waves without tokens, groups that do not fill a tile or need several,
+    and a key that stands out of those before it (the reference point of the weights moves)."""
+    q, k_pages, v_pages, ctx, meta, _, _ = _attention_case(torch.bfloat16, q_heads, kv_heads, dim, page_size, portions, window, 61, spike)
+    want = torch.empty_like(q)
+    ref.attention(q, k_pages, v_pages, ctx, meta, q_heads, kv_heads, dim, dim ** -0.5, window, want)
+    cctx, cmeta = _to_cuda(ctx, meta)
+    got = torch.full_like(q, float("nan"), device="cuda")
+    hip.wide_prompt_tiles, hip.split_prompt_keys = True, False
+    try:
+        hip.attention(q.cuda(), k_pages.cuda(), v_pages.cuda(), cctx, cmeta, q_heads, kv_heads, dim, dim ** -0.5, window, got)
+    finally:
+        hip.wide_prompt_tiles, hip.split_prompt_keys = None, None
+    torch.testing.assert_close(got.cpu().float(), want.float(), **attention_tol(torch.bfloat16))
+
+
+@pytest.mark.parametrize("dim,page_size", [(128, 16), (64, 32)])
+def test_attention_on_tiles_of_32_columns_says_that_a_page_is_missing(hip, dim, page_size):
+    """A page that is not the request's, in the middle of what is seen: the tokens that walk over it are NaN, the others not."""
+    q, k_pages, v_pages, ctx, meta, _, _ = _attention_case(torch.bfloat16, 8, 2, dim, page_size, [(0, 200), (0, 70)], None, 62)
+    meta.block_table[0, 64 // page_size] = -1
+    cctx, cmeta = _to_cuda(ctx, meta)
+    got = torch.zeros_like(q, device="cuda")
+    hip.wide_prompt_tiles, hip.split_prompt_keys = True, False
+    try:
+        hip.attention(q.cuda(), k_pages.cuda(), v_pages.cuda(), cctx, cmeta, 8, 2, dim, dim ** -0.5, None, got)
+    finally:
+        hip.wide_prompt_tiles, hip.split_prompt_keys = None, None
+    assert torch.isnan(got[64:200]).all() and not torch.isnan(got[:64]).any() and not torch.isnan(got[200:]).any()
+
+
+def test_attention_takes_tiles_of_32_columns_from_some_hundred_keys_on(hip):
+    """The rule that chooses between 16 and 32 columns a wave asks for the longest context, by head size and page."""
+    ctx = lambda length: SimpleNamespace(num_seqs=1, host_q_start=[0, 60], host_seq_lens=[length])
+    wide = lambda length, dim, page: hip._wide_shared_tiles(ctx(length), 0, 8, 2, dim, page)
+    assert not wide(383, 128, 16) and wide(384, 128, 16) and not wide(4095, 64, 32) and wide(4096, 64, 32)
+    assert not wide(8000, 128, 8) and not wide(8000, 96, 16)
+
+
 @pytest.mark.parametrize("q_heads,kv_heads,dim,page_size", ATTENTION_SIZES + [(32, 8, 128, 16), (40, 2, 64, 8)])
 @pytest.mark.parametrize("histories", [[0], [64, 17, 0], [1500, 2, 700, 255], [4000] * 9])
 @pytest.mark.parametrize("window", [None, 100])
