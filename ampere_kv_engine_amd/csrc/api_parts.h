@@ -166,9 +166,9 @@ int akv_gated_linear_scan(const void* u, int dtype, const float* gates, const fl
 // Per request and head, S [dim, vdim] (in the slot as [heads, vdim, dim] float32): S <- g S; u = beta (v - S^T k);
 // S <- S + k u^T; o = S^T q.  out [tokens, heads x vdim] = o / rms(o) * norm_weight[i] * act(gates[t * gate_stride + h * vdim
 // + i]), gate_act 1: sigmoid, 2: silu.  Decay logits and gates are float32 where decays are per channel, else of `dtype`.
-// `workspace`: akv_delta_rule_workspace(...) floats.  `longest`: the most tokens a request brings (chooses the walk's tile;
-// the sums are the same either way).
-long akv_delta_rule_workspace(int tokens, int heads, int groups, int dim, int vdim, int decay_per_head);
+// `workspace`: akv_delta_rule_workspace(...) floats.  `longest`: the most tokens a request brings (chooses the walk: token by
+// token, its tile, or in chunks of 16 tokens).
+long akv_delta_rule_workspace(int tokens, int seqs, int heads, int groups, int dim, int vdim, int decay_per_head, int longest);
 int akv_delta_rule(const void* conv, long conv_stride, int dtype, const void* beta_logits, long beta_stride,
                    const void* decay_logits, int decay_dtype, long decay_stride, const float* decay_bias, const float* rate,
                    int decay_per_head, const void* gates, int gate_dtype, long gate_stride, int gate_act,

@@ -600,7 +600,9 @@ class PartsKernels:
         self.check_delta_rule_sizes(heads, groups, dim, vdim)
         self._step_arrays(ctx, tokens)
         lib = self._parts()
-        workspace = self._walk_workspace(int(lib.akv_delta_rule_workspace(tokens, heads, groups, dim, vdim, 1 if per_head else 0)))
+        longest = int(ctx.max_new_tokens) or tokens
+        workspace = self._walk_workspace(int(lib.akv_delta_rule_workspace(tokens, ctx.num_seqs, heads, groups, dim, vdim,
+                                                                          1 if per_head else 0, longest)))
         self._check(lib.akv_delta_rule(
             _ptr(conv), _long(width), self._code_of(conv), _ptr_at(beta_logits, beta_at), _long(beta_logits.shape[1]),
             _ptr_at(decay_logits, decay_at), self._code_of(decay_logits), _long(decay_logits.shape[1]), _ptr(decay_bias),
@@ -608,7 +610,7 @@ class PartsKernels:
             self.GATE_ACTS[gate], _ptr(norm_weight), ctypes.c_float(unit_eps),
             ctypes.c_float(norm_eps), ctypes.c_float(q_scale), _ptr(state), _long(state.shape[1]), _ptr(ctx.q_start),
             _ptr(ctx.seq_slots), _ptr(workspace), _ptr(out), tokens, ctx.num_seqs, heads, groups, dim, vdim,
-            int(ctx.max_new_tokens) or tokens, self._stream()),
+            longest, self._stream()),
             "delta_rule")
 
     def _state_of_slots(self, state, need: int, ctx) -> None:

@@ -356,6 +356,65 @@ def test_delta_rule_at_the_edges_of_its_fours(hip, dtype, sizes):
     test_delta_rule_kernels_alone(hip, dtype, *sizes)
 
 
+def _delta_step(hip, counts, heads, groups, dim, vdim, per_head, state, inputs):
+    conv, beta, decay_logits, decay_bias, rate, gates, weight = inputs
+    out = torch.empty(sum(counts), heads * vdim, device=DEVICE)
+    extra = dict(decay_at=0, gate_at=0, gate="sigmoid") if per_head else {}
+    hip.delta_rule(conv, beta, 0, decay_logits, decay_bias, rate, gates, weight, 1e-6, 1e-5, dim ** -0.5, heads, groups, dim, vdim,
+                   state, _ctx([0] * len(counts), counts), out, **extra)
+    return out
+
+
+def _delta_inputs(tokens, heads, groups, dim, vdim, per_head):
+    rand = lambda *shape: torch.randn(*shape).to(DEVICE)
+    decays = heads if per_head else heads * dim
+    return [rand(tokens, 2 * groups * dim + heads * vdim), rand(tokens, heads) * 2, rand(tokens, decays), rand(decays) * 0.5,
+            torch.exp(-4.0 + 4.0 * torch.rand(heads)).to(DEVICE), rand(tokens, heads * vdim), 1 + 0.2 * rand(vdim)]
+
+
+@pytest.mark.parametrize("per_head", [False, True])
+@pytest.mark.parametrize("heads,groups,dim,vdim", [(2, 1, 64, 20), (2, 2, 128, 16), (1, 1, 192, 33), (3, 1, 256, 7)])
+def test_delta_rule_in_chunks_is_the_walk_token_by_token(hip, per_head, heads, groups, dim, vdim):
+    """Requests of lengths around the chunks of 16 in one step, from a state that holds something: against the walk token by
+    token, which takes states whose stride is no multiple of four.  Both are float32 (2e-7 off 64 bits each): 1e-5 of the largest."""
+    torch.manual_seed(dim + vdim)
+    counts = (1, 15, 16, 17, 47, 48, 49, 100)
+    inputs = _delta_inputs(sum(counts), heads, groups, dim, vdim, per_head)
+    size = heads * dim * vdim
+    begun = torch.randn(len(counts), size).to(DEVICE)
+    apart = torch.zeros(len(counts), (size + 3) // 4 * 4 + 1, device=DEVICE)
+    together = torch.zeros(len(counts), (size + 3) // 4 * 4, device=DEVICE)
+    apart[:, :size], together[:, :size] = begun, begun
+    want, got = (_delta_step(hip, counts, heads, groups, dim, vdim, per_head, state, inputs) for state in (apart, together))
+    assert (got - want).abs().max() < 1e-5 * want.abs().max()
+    assert (together[:, :size] - apart[:, :size]).abs().max() < 1e-5 * apart[:, :size].abs().max()
+
+
+@pytest.mark.parametrize("where", ["value", "infinite value", "key", "query", "beta", "decay"])
+def test_delta_rule_in_chunks_keeps_what_is_not_finite_from_earlier_tokens(hip, where):
+    """One element of token 37 that is no number (or infinite): outputs before it are as the walk token by token leaves them, and
+    those that are no numbers are the same."""
+    torch.manual_seed(5)
+    heads, dim, vdim, counts, at = 2, 64, 32, (60,), 37
+    inputs = _delta_inputs(60, heads, heads, dim, vdim, False)
+    conv, beta, decay = inputs[:3]
+    bad = float("inf") if where == "infinite value" else float("nan")
+    if where.endswith("value"):
+        conv[at, 2 * heads * dim + 3] = bad
+    elif where in ("key", "query"):
+        conv[at, (heads * dim if where == "key" else 0) + 5] = bad
+    elif where == "beta":
+        beta[at, 0] = bad
+    else:
+        decay[at, 7] = bad
+    size = heads * dim * vdim
+    apart, together = torch.zeros(1, size + 1, device=DEVICE), torch.zeros(1, size, device=DEVICE)
+    want, got = (_delta_step(hip, counts, heads, heads, dim, vdim, False, state, inputs) for state in (apart, together))
+    assert not torch.isnan(want[:at]).any() and torch.isnan(want[at]).any()
+    assert torch.equal(torch.isnan(got), torch.isnan(want))
+    assert (got - want).nan_to_num(0.0).abs().max() < 1e-5 * want.nan_to_num(0.0).abs().max()
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("tokens,heads,vdim,lead", [(1, 1, 4, 0), (3, 5, 8, 4), (7, 3, 256, 8), (70, 2, 64, 0), (5, 2, 64, 2), (4, 3, 12, 0),
                                                     (2, 1, 512, 0)])
