@@ -105,12 +105,15 @@ __global__ __launch_bounds__(256) void attention_rows_kernel(
 // (at most 64).  A request's keys span from `first` (the start of its window, down to a multiple of 32) to its token's
 // position; the size is the sum of the spans over items_wanted, up to a multiple of 32, at least min_segment; items
 // are numbered request by request.  The cut depends on the lengths only, so one plan serves every layer of a step.
-//   plan[0] = items in all, plan[1] = keys per segment
+// With `share` the items are for blocks of four waves that share one: a quarter as many are wanted, a request's pieces are made
+// alike, and the requests with the most keys come first - blocks start in the order of the items, and the short ones then
+// fill what the long ones leave.
+//   plan[0] = items in all, plan[1] = keys per segment (at most)
 //   plan[4 + 2 r] = items before request r's, plan[5 + 2 r] = its items                          (r < 64)
 //   plan[132 + 4 i] = request of item i (counted from seq_first), its first key, the token's position, its last key
 namespace {
 __global__ __launch_bounds__(64) void decode_plan_kernel(const int* __restrict__ seq_lens, int seq_first, int seq_count,
-                                                        int window, int items_wanted, int min_segment, int items_grid,
+                                                        int window, int items_wanted, int min_segment, int items_grid, int share,
                                                         int* __restrict__ plan) {
   const int lane = threadIdx.x;
   int pos = -1, first = 0, span = 0;
@@ -122,17 +125,30 @@ __global__ __launch_bounds__(64) void decode_plan_kernel(const int* __restrict__
   int total_span = span;
 #pragma unroll
   for (int offset = 32; offset > 0; offset >>= 1) total_span += __shfl_xor(total_span, offset, kWave);
+  if (share) items_wanted = max(items_wanted / 4, 1);
   const int size = max(min_segment, ((total_span + items_wanted - 1) / items_wanted + 31) & ~31);
   const int count = (span + size - 1) / size;
-  int upto = count;  // inclusive prefix sum over the wave
+  int piece = size, before = 0;
+  if (share) {
+    if (count > 1) piece = ((span + count - 1) / count + 31) & ~31;   // (at most `size`: that is a multiple of 32)
+    for (int other = 0; other < seq_count; ++other) {
+      const int others_span = __shfl(span, other, kWave), others_count = __shfl(count, other, kWave);
+      if (others_span > span || (others_span == span && other < lane)) before += others_count;
+    }
+  } else {
+    int upto = count;  // inclusive prefix sum over the wave
 #pragma unroll
-  for (int step = 1; step < kWave; step <<= 1) {
-    const int other = __shfl_up(upto, step, kWave);
-    if (lane >= step) upto += other;
+    for (int step = 1; step < kWave; step <<= 1) {
+      const int other = __shfl_up(upto, step, kWave);
+      if (lane >= step) upto += other;
+    }
+    before = upto - count;
   }
-  const int before = upto - count;
-  if (lane == kWave - 1) {
-    plan[0] = min(upto, items_grid);
+  int items = count;
+#pragma unroll
+  for (int offset = 32; offset > 0; offset >>= 1) items += __shfl_xor(items, offset, kWave);
+  if (lane == 0) {
+    plan[0] = min(items, items_grid);
     plan[1] = size;
   }
   plan[4 + 2 * lane] = before;
@@ -140,18 +156,18 @@ __global__ __launch_bounds__(64) void decode_plan_kernel(const int* __restrict__
   for (int z = 0; z < count; ++z) {
     const int item = before + z;
     if (item >= items_grid) break;  // (cannot happen with the host's bound; never write beyond the buffer)
-    const int lo = first + z * size;
-    *reinterpret_cast<int4*>(plan + 132 + 4 * item) = make_int4(lane, lo, pos, min(pos, lo + size - 1));
+    const int lo = first + z * piece;
+    *reinterpret_cast<int4*>(plan + 132 + 4 * item) = make_int4(lane, lo, pos, min(pos, lo + piece - 1));
   }
 }
 }  // namespace
 
 extern "C" int akv_decode_plan(const int* seq_lens, int seq_first, int seq_count, int window, int items_wanted,
-                               int min_segment, int items_grid, int* plan, hipStream_t stream) {
+                               int min_segment, int items_grid, int share, int* plan, hipStream_t stream) {
   if (seq_count <= 0) return 0;
   if (seq_count > 64 || items_wanted < 1 || min_segment < 32 || (min_segment & 31) != 0 || items_grid < 1) return -2;
   decode_plan_kernel<<<1, 64, 0, stream>>>(seq_lens, seq_first, seq_count, window, items_wanted, min_segment, items_grid,
-                                           plan);
+                                           share, plan);
   return AKV_LAUNCH_STATUS();
 }
 

@@ -261,11 +261,22 @@ __device__ __forceinline__ void encode_head(uintx4 (&reg)[KT], bool normed, floa
 // prompt portions' blocks: see `attention_pair_kernel`.)
 struct Where {
   int bx, by, bz, gx, gy;   // the wave's block and the grid, as blockIdx and gridDim would name them
-  int lane;
+  int lane, wave;           // (wave: of the four that share an item)
 };
 
-template <int NQ, bool SPLIT, bool PIPE, bool FRESH, bool ONCE>
-__device__ __forceinline__ void attention_mfma_body(const Args& a, const Where at) {
+// Where requests are few, an item of a plan (single tokens) is worked on by a block of four waves: each takes a quarter of the
+// item's steps of 32 keys, and what the four have - maximum, sum and weighted sum per column - is merged through LDS into the
+// item's one partial result.  A wave's steps follow each other at the latency of a page's lookup and its keys, so a short
+// context's 128 keys cost one such step instead of four, and a long one's segments leave a quarter of the partial results to
+// the merge.  (A step of one request of 210 keys, 8 layers of 16 / 4 heads: 380 -> 365 us.)
+constexpr int kItemWaves = 4;
+struct ItemLds {
+  float parts[kItemWaves][16][PSTRIDE];
+};
+
+template <int NQ, bool SPLIT, bool PIPE, bool FRESH, bool ONCE, bool ITEMS>
+__device__ __forceinline__ void attention_mfma_body(const Args& a, const Where at, ItemLds* item_lds) {
+  static_assert(!ITEMS || (SPLIT && NQ == 1), "items are single tokens cut by a plan");
   const int lane = at.lane, r16 = lane & 15, g = lane >> 4;
   auto from_pages = [](const char* at) {
     const uintx4* p = reinterpret_cast<const uintx4*>(at);
@@ -293,6 +304,11 @@ __device__ __forceinline__ void attention_mfma_body(const Args& a, const Where a
     t.found = true;
     seg_lo = record.y;
     seg_hi = record.w;
+    if constexpr (ITEMS) {
+      const int steps = ((seg_hi - seg_lo) >> 5) + 1, share = (steps + kItemWaves - 1) / kItemWaves * 32;
+      seg_lo += at.wave * share;           // (a wave that gets no step has seg_hi < seg_lo)
+      seg_hi = min(seg_hi, seg_lo + share - 1);
+    }
     part = static_cast<long>(item) * at.gx + at.bx;
   } else {
     t = find_tile(a, slot, a.tokens_per_tile);
@@ -645,7 +661,16 @@ __device__ __forceinline__ void attention_mfma_body(const Args& a, const Where a
   for (int nq = 0; nq < NQ; ++nq) {
     l[nq] += __shfl_xor(l[nq], 16, 64);
     l[nq] += __shfl_xor(l[nq], 32, 64);
-    if (SPLIT) {
+    if constexpr (ITEMS) {
+      if (!col_valid[nq]) continue;
+      float* mine = item_lds->parts[at.wave][r16];
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) *reinterpret_cast<floatx4*>(mine + dt * 16 + g * 4) = o[nq][dt];
+      if (g == 0) {
+        mine[D] = poisoned ? nan : m[nq];
+        mine[D + 1] = l[nq];
+      }
+    } else if (SPLIT) {
       if (!col_valid[nq]) continue;  // (next column) the merge never reads columns that are no (token, head) pair
       const int c = nq * 16 + r16;
       float* dst = a.partial + (part * (16 * NQ) + c) * PSTRIDE;
@@ -666,14 +691,52 @@ __device__ __forceinline__ void attention_mfma_body(const Args& a, const Where a
       }
     }
   }
+  if constexpr (ITEMS) {   // the four waves' results into the item's: thread (column, four dims)
+    __syncthreads();
+    const int columns = min(a.heads_per_tile, a.group - hg * a.heads_per_tile);
+    for (int e = at.wave * 64 + lane; e < columns * (D / 4); e += 64 * kItemWaves) {
+      const int c = e / (D / 4), d = e % (D / 4) * 4;
+      float mw[kItemWaves], top = -INFINITY, sum = 0.f;
+      bool bad = false;
+#pragma unroll
+      for (int w = 0; w < kItemWaves; ++w) {
+        mw[w] = item_lds->parts[w][c][D];
+        bad = bad || mw[w] != mw[w];
+        top = fmaxf(top, mw[w]);
+      }
+      floatx4 all = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int w = 0; w < kItemWaves; ++w) {
+        const float by = mw[w] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mw[w] - top);
+        all += *reinterpret_cast<const floatx4*>(&item_lds->parts[w][c][d]) * by;
+        sum = fmaf(by, item_lds->parts[w][c][D + 1], sum);
+      }
+      float* dst = a.partial + (part * 16 + c) * PSTRIDE;
+      *reinterpret_cast<floatx4*>(dst + d) = all;
+      if (d == 0) {
+        dst[D] = bad ? nan : top;
+        dst[D + 1] = sum;
+      }
+    }
+  }
   }  // pass
 }
 
 template <int NQ, bool SPLIT, bool PIPE, bool FRESH, bool ONCE>
 __global__ __launch_bounds__(64, (SPLIT && NQ == 1 && D <= 128) ? 2 : 1) void attention_mfma_kernel(const Args a) {
-  attention_mfma_body<NQ, SPLIT, PIPE, FRESH, ONCE>(
+  attention_mfma_body<NQ, SPLIT, PIPE, FRESH, ONCE, false>(
       a, Where{static_cast<int>(blockIdx.x), static_cast<int>(blockIdx.y), static_cast<int>(blockIdx.z),
-               static_cast<int>(gridDim.x), static_cast<int>(gridDim.y), static_cast<int>(threadIdx.x)});
+               static_cast<int>(gridDim.x), static_cast<int>(gridDim.y), static_cast<int>(threadIdx.x), 0}, nullptr);
+}
+
+// Items of a plan: block (head block, item).
+template <bool FRESH, bool ONCE>
+__global__ __launch_bounds__(64 * kItemWaves, D <= 128 ? 2 : 1) void attention_items_kernel(const Args a) {
+  __shared__ __align__(16) ItemLds lds;
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+  attention_mfma_body<1, true, true, FRESH, ONCE, true>(
+      a, Where{static_cast<int>(blockIdx.x), static_cast<int>(blockIdx.y), 0, static_cast<int>(gridDim.x),
+               static_cast<int>(gridDim.y), static_cast<int>(threadIdx.x) & 63, wave}, &lds);
 }
 
 // ---- prompt portions: four waves share every key and value through LDS ------------------------------------------------
@@ -695,12 +758,16 @@ constexpr float kLazy = 8.f;  // the exponentials' reference point trails the ma
 
 // SP: pages per step of 32 keys (4: pages of 8 tokens, 2: of 16, 1: of 32 or more) - with it the page arithmetic of a
 // step is known when compiling.
+struct SharedLds {
+  bf16_t k[2][32 * KROW], v[2][D * VROW];
+  int bad_page;
+};
 template <int NQ, int SP>
-__device__ __forceinline__ void attention_shared_body(const Args& a, const int block, const int thread) {
+__device__ __forceinline__ void attention_shared_body(const Args& a, const int block, const int thread, SharedLds& lds) {
   const int page_shift = SP == 4 ? 3 : (SP == 2 ? 4 : a.page_shift);
-  __shared__ __align__(16) bf16_t k_lds[2][32 * KROW];
-  __shared__ __align__(16) bf16_t v_lds[2][D * VROW];
-  __shared__ int bad_page;
+  auto& k_lds = lds.k;
+  auto& v_lds = lds.v;
+  int& bad_page = lds.bad_page;
   const int tid = thread, lane = tid & 63, r16 = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   // Late tiles of a prompt see the most keys.  Blocks are ranked longest first, and the ranks are dealt out to the
@@ -1134,7 +1201,8 @@ __device__ __forceinline__ void attention_shared_body(const Args& a, const int b
 
 template <int NQ, int SP>
 __global__ __launch_bounds__(64 * kSharedWaves, D <= 128 ? (NQ == 1 ? 3 : 2) : 1) void attention_shared_kernel(const Args a) {
-  attention_shared_body<NQ, SP>(a, static_cast<int>(blockIdx.x), static_cast<int>(threadIdx.x));
+  __shared__ __align__(16) SharedLds lds;
+  attention_shared_body<NQ, SP>(a, static_cast<int>(blockIdx.x), static_cast<int>(threadIdx.x), lds);
 }
 
 // ---- prompt portions on tiles of 32 columns: both products on 32 x 32 tiles, three steps in the air ----------------------
@@ -1507,14 +1575,16 @@ template <bool ONCE, int SP>
 __global__ __launch_bounds__(64 * kSharedWaves, 2) void attention_pair_kernel(const Args single, const Args portion,
                                                                               const int portion_blocks) {
   if constexpr (D % 64 == 0) {
+    __shared__ __align__(16) SharedLds lds;
     if (static_cast<int>(blockIdx.x) < portion_blocks) {
-      attention_shared_body<1, SP>(portion, static_cast<int>(blockIdx.x), static_cast<int>(threadIdx.x));
+      attention_shared_body<1, SP>(portion, static_cast<int>(blockIdx.x), static_cast<int>(threadIdx.x), lds);
     } else {
       const int gx = single.kv_heads * single.head_groups, gy = single.items_grid;
       const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
       const int unit = (static_cast<int>(blockIdx.x) - portion_blocks) * kSharedWaves + wave;
       if (unit >= gx * gy) return;
-      attention_mfma_body<1, true, true, true, ONCE>(single, Where{unit % gx, unit / gx, 0, gx, gy, static_cast<int>(threadIdx.x) & 63});
+      attention_mfma_body<1, true, true, true, ONCE, false>(
+          single, Where{unit % gx, unit / gx, 0, gx, gy, static_cast<int>(threadIdx.x) & 63, 0}, nullptr);
     }
   }
 }
@@ -1638,7 +1708,7 @@ __global__ __launch_bounds__(64 * kMergeWaves) void attention_merge_kernel(const
 }
 
 template <int NQ>
-int launch(const Args& a, int tiles, bool shared, hipStream_t stream) {
+int launch(const Args& a, int tiles, bool shared, int waves_per_item, hipStream_t stream) {
   dim3 grid(tiles, a.kv_heads * a.head_groups, a.num_splits);
   if (shared) {
     const dim3 blocks(tiles * a.kv_heads * a.head_groups);
@@ -1668,7 +1738,11 @@ int launch(const Args& a, int tiles, bool shared, hipStream_t stream) {
   if (a.qkv != nullptr) {
     if constexpr (NQ == 1 && D % 64 == 0) {
       if (!a.single_tokens) return -2;
-      if (items || a.num_splits > 1) {
+      if (items && waves_per_item == kItemWaves) {
+        if (once) attention_items_kernel<true, true><<<grid, 64 * kItemWaves, 0, stream>>>(a);
+        else attention_items_kernel<true, false><<<grid, 64 * kItemWaves, 0, stream>>>(a);
+        merge();
+      } else if (items || a.num_splits > 1) {
         if (once) attention_mfma_kernel<NQ, true, true, true, true><<<grid, 64, 0, stream>>>(a);
         else attention_mfma_kernel<NQ, true, true, true, false><<<grid, 64, 0, stream>>>(a);
         merge();
@@ -1680,7 +1754,15 @@ int launch(const Args& a, int tiles, bool shared, hipStream_t stream) {
       return -2;
     }
   }
-  if (items || a.num_splits > 1) {
+  if (items && waves_per_item == kItemWaves) {
+    if constexpr (NQ == 1) {
+      if (once) attention_items_kernel<false, true><<<grid, 64 * kItemWaves, 0, stream>>>(a);
+      else attention_items_kernel<false, false><<<grid, 64 * kItemWaves, 0, stream>>>(a);
+      merge();
+    } else {
+      return -2;
+    }
+  } else if (items || a.num_splits > 1) {
     if (once) attention_mfma_kernel<NQ, true, true, false, true><<<grid, 64, 0, stream>>>(a);
     else attention_mfma_kernel<NQ, true, true, false, false><<<grid, 64, 0, stream>>>(a);
     merge();
@@ -1773,7 +1855,8 @@ int units_of_device() {
 // 4 * tokens_per_tile tokens, num_splits must be 1 and pages hold at least 8 tokens.
 // `plan` (not null: single tokens, at most 64 requests): seg_keys and num_splits are not used; the requests' keys were
 // cut into items by akv_decode_plan with the same seq_first, seq_count and window; `items_grid` is the bound given
-// there, and `partial` must hold items_grid * kv_heads * head_groups * 16 * nq * (D + 4) floats.
+// there, and `partial` must hold items_grid * kv_heads * head_groups * 16 * nq * (D + 4) floats.  `waves_per_item`: 1, or 4
+// that share an item (the plan was then made with `share`).
 // `qkv` (not null: single tokens, nq 1, head sizes that are multiples of 64): the tokens' stacked raw projections
 // [tokens, (q_heads + 2 * kv_heads) * D]; `q` is not read, the kernel norms (q_weight, k_weight, eps; both weights
 // null: no norm) and rotates (rope_table [table_positions, D / 2, 2], null: no rotation) queries and the new keys
@@ -1785,12 +1868,12 @@ extern "C" int AKV_CONCAT(akv_attention_mfma_d, AKV_HEAD_DIM)(
     int q_heads, int kv_heads, int heads_per_tile, int head_groups, int tokens_per_tile, int page_size, long num_pages,
     float scale, int window, int seg_keys, int num_splits, int single_tokens, int shared, const void* qkv,
     const float* q_weight, const float* k_weight, float eps, const float* rope_table, int table_positions,
-    const int* plan, int items_grid, hipStream_t stream) {
+    const int* plan, int items_grid, int waves_per_item, hipStream_t stream) {
   if (tiles <= 0 || seq_count <= 0) return 0;
   if (heads_per_tile * tokens_per_tile > 16 * nq || kv_heads * head_groups > 65535 || num_splits > 65535 ||
       num_splits < 1 || (single_tokens && tiles != seq_count) || (shared && (page_size < 8 || num_splits != 1)) ||
       (qkv != nullptr && (shared || !single_tokens || nq != 1 || D % 64 != 0 || (q_weight == nullptr) != (k_weight == nullptr))) ||
-      (plan != nullptr && (shared || !single_tokens || seq_count > 64 || items_grid < 1 || items_grid > 65535)))
+      (plan != nullptr && (shared || nq != 1 || (waves_per_item != 1 && waves_per_item != kItemWaves) || !single_tokens || seq_count > 64 || items_grid < 1 || items_grid > 65535)))
     return -2;
   Args a;
   const int status = common_args(a, q, k_pages, v_pages, out, q_start, seq_lens, block_table, table_rows, table_width,
@@ -1820,8 +1903,8 @@ extern "C" int AKV_CONCAT(akv_attention_mfma_d, AKV_HEAD_DIM)(
     if (static_cast<long>(tiles) * kv_heads * head_groups > 0x7fffffffL) return -2;
   }
   switch (nq) {
-    case 1: return launch<1>(a, tiles, shared != 0, stream);
-    case 2: return launch<2>(a, tiles, shared != 0, stream);
+    case 1: return launch<1>(a, tiles, shared != 0, waves_per_item, stream);
+    case 2: return launch<2>(a, tiles, shared != 0, waves_per_item, stream);
     default: return -2;
   }
 }
@@ -1864,7 +1947,7 @@ extern "C" int AKV_CONCAT(akv_attention_pair_d, AKV_HEAD_DIM)(
   single.num_splits = 1;
   single.plan = plan;
   single.items_grid = items_grid;
-  single.qkv = static_cast<const bf16_t*>(qkv);
+    single.qkv = static_cast<const bf16_t*>(qkv);
   single.q_weight = q_weight;
   single.k_weight = k_weight;
   single.rope_table = rope_table;

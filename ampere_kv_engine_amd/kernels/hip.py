@@ -1008,7 +1008,7 @@ class HipKernels(PartsKernels, KernelSet):
                 and max(ctx.host_seq_lens[seq_first:seq_first + seq_count]) > self.decode_min_segment):
             # single tokens: their keys are cut on the device, from the lengths there (requests of 128 keys or
             # fewer are not cut: then the kernel without merge)
-            plan, items_grid = self._decode_plan(ctx, seq_first, seq_count, window, kv_heads * head_groups)
+            plan, items_grid = self._decode_plan(ctx, seq_first, seq_count, window, kv_heads * head_groups, share=self._share_segments(seq_count, kv_heads * head_groups))
             partial = take(items_grid * kv_heads * head_groups * 16 * nq * (head_dim + 4))
         elif split:
             longest = max(ctx.host_seq_lens[seq_first:seq_first + seq_count])
@@ -1021,6 +1021,7 @@ class HipKernels(PartsKernels, KernelSet):
             if num_splits > 1:
                 partial = take(tiles * kv_heads * head_groups * num_splits * 16 * nq * (head_dim + 4))
         qkv, q_weight, k_weight, eps, table = fresh if fresh is not None else (None, None, None, 0.0, None)
+        waves_per_item = 4 if plan is not None and self._share_segments(seq_count, kv_heads * head_groups) else 1
         self._check(self._attention_mfma_entry(head_dim)(
             _ptr(q), _ptr(k_pages), _ptr(v_pages), _ptr(out), _ptr(partial), _ptr(ctx.q_start), _ptr(ctx.seq_lens),
             _ptr(meta.block_table), _ptr(getattr(meta, "rows", None)), meta.width, seq_first, seq_count, tiles, nq,
@@ -1028,19 +1029,30 @@ class HipKernels(PartsKernels, KernelSet):
             head_groups, tokens_per_tile, page_size, ctypes.c_long(num_pages), ctypes.c_float(scale),
             int(window) if window is not None else 0, seg_keys, num_splits, 1 if single else 0, 1 if shared else 0,
             _ptr(qkv), _ptr(q_weight), _ptr(k_weight), ctypes.c_float(eps), _ptr(table),
-            table.shape[0] if table is not None else 0, _ptr(plan), items_grid, self._stream()),
+            table.shape[0] if table is not None else 0, _ptr(plan), items_grid, waves_per_item, self._stream()),
             "attention")
 
     PLAN_ENTRIES = 132          # ints of a plan before its items (4 per item)
 
-    def _decode_plan(self, ctx, seq_first, seq_count, window, head_blocks, waves=None):
+    @staticmethod
+    def _share_segments(seq_count: int, head_blocks: int) -> bool:
+        """Whether four waves share a segment of a single token's keys (`attention_items_kernel`) rather than a wave alone
+        take it.  Shared segments end a short context's chain of steps sooner and leave a quarter of the partial results, but
+        there are at most two rounds of blocks for the device to even out: with up to 32 (request, head block) pairs a
+        request has 16 segments or more and their last pieces do not count.  It hangs on the number of requests only, so
+        that a recorded step and the same step run eagerly are cut alike.  Whole steps, alone / shared us: one request of
+        2,048 keys 941 / 928 (8 layers of the 8B sizes), of 16,000 1,017 / 985, four of 64 to 16,000 1,069 / 1,061; 8 heads and
+        8 requests of 64 to 12,000 1,115 / 1,141, 27 of 64 to 16,000 1,657 / 1,691 (6 layers of 14B)."""
+        return seq_count * head_blocks <= 32
+
+    def _decode_plan(self, ctx, seq_first, seq_count, window, head_blocks, waves=None, share=False):
         """The cut of the keys of requests seq_first .. + seq_count - 1 (single tokens) into (request, segment) items:
         segments of one size for all requests - about `decode_wave_target` waves in all, no segment shorter than
         `decode_min_segment` unless it is a request's only one - worked out by a one-wave kernel from the lengths on
-        the device.  The cut depends on the lengths alone, so the layers of a step share one plan: it is remembered on
-        the step's context.  Returns the plan and the bound on the number of items that sizes grids and buffers."""
+        the device.  With `share` four waves work on a segment: a quarter as many are wanted.  The cut depends on the lengths alone, so the layers of a step share one plan: it is
+        remembered on the step's context.  Returns the plan and the bound on the number of items that sizes grids and buffers."""
         items = max(1, (waves if waves is not None else self.decode_wave_target) // head_blocks)
-        key = (seq_first, seq_count, int(window) if window is not None else 0, items, self.decode_min_segment)
+        key = (seq_first, seq_count, int(window) if window is not None else 0, items, self.decode_min_segment, share)
         plans = getattr(ctx, "decode_plans", None)
         if plans is None:
             plans = {}
@@ -1051,7 +1063,7 @@ class HipKernels(PartsKernels, KernelSet):
         if key in plans:
             return plans[key]
         smallest = self.decode_min_segment
-        items_grid = min(items + seq_count, sum((length + smallest - 1) // smallest
+        items_grid = min((max(1, items // 4) if share else items) + seq_count, sum((length + smallest - 1) // smallest
                                                 for length in ctx.host_seq_lens[seq_first:seq_first + seq_count]))
         if items_grid > 65535:
             raise KernelError(f"{items_grid} segments of keys in one launch; the grid holds 65,535")
@@ -1070,7 +1082,7 @@ class HipKernels(PartsKernels, KernelSet):
         plan = self._plan_buffers[index]
         self._dense(ctx.seq_lens, "seq_lens", torch.int32, (ctx.num_seqs,))
         self._check(self.lib.akv_decode_plan(_ptr(ctx.seq_lens), seq_first, seq_count, key[2], items, smallest,
-                                             items_grid, _ptr(plan), self._stream()), "decode_plan")
+                                             items_grid, 1 if share else 0, _ptr(plan), self._stream()), "decode_plan")
         plans[key] = (plan, items_grid)
         return plans[key]
 

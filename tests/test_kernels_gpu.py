@@ -1514,6 +1514,49 @@ def test_decode_plan(hip, lengths, window):
             item += 1
 
 
+@pytest.mark.parametrize("lengths,window", [([9000, 130, 129, 4000], None), ([70000, 33, 512], None), ([5000, 200, 1000], 300),
+                                            ([1], None), ([300] * 8, None)])
+def test_decode_plan_of_shared_items(hip, lengths, window):
+    """The cut for items that four waves share: a quarter of the items, a request's pieces alike, the longest request first;
+    every key of a span in one item."""
+    items_wanted, smallest = 64, 128
+    ctx = SimpleNamespace(seq_lens=torch.tensor(lengths, dtype=torch.int32, device="cuda"), num_seqs=len(lengths), host_seq_lens=lengths)
+    plan, grid = hip._decode_plan(ctx, 0, len(lengths), window, 1, waves=4 * items_wanted, share=True)
+    plan = plan.cpu().tolist()
+    firsts = [(max(0, n - window) if window else 0) // 32 * 32 for n in lengths]
+    spans = [n - first for n, first in zip(lengths, firsts)]
+    size = max(smallest, (-(-sum(spans) // items_wanted) + 31) // 32 * 32)
+    assert plan[1] == size and plan[0] == sum(-(-span // size) for span in spans) <= grid
+    item = 0
+    for r in sorted(range(len(lengths)), key=lambda r: (-spans[r], r)):
+        count = -(-spans[r] // size)
+        piece = size if count == 1 else (-(-spans[r] // count) + 31) // 32 * 32
+        assert piece <= size and plan[4 + 2 * r:6 + 2 * r] == [item, count]
+        for z in range(count):
+            lo = firsts[r] + z * piece
+            assert plan[132 + 4 * item:136 + 4 * item] == [r, lo, lengths[r] - 1, min(lengths[r] - 1, lo + piece - 1)]
+            item += 1
+
+
+@pytest.mark.parametrize("q_heads,kv_heads,dim,page_size", [(8, 2, 128, 16), (3, 1, 256, 32), (40, 2, 64, 8), (6, 1, 32, 4), (5, 5, 80, 16)])
+@pytest.mark.parametrize("histories", [[128], [160, 31, 300], [2100], [700, 96, 0, 33]])
+@pytest.mark.parametrize("window", [None, 1, 150])
+def test_single_tokens_whose_items_are_shared_by_four_waves(hip, ref, monkeypatch, q_heads, kv_heads, dim, page_size, histories, window):
+    """Items of one step to several a wave, waves without a step, one item a request and many; the same items taken by a wave
+    alone give the same within the tolerance of either."""
+    portions = [(h, 1) for h in histories]
+    q, k_pages, v_pages, ctx, meta, _, _ = _attention_case(torch.bfloat16, q_heads, kv_heads, dim, page_size, portions, window, 63)
+    ctx.num_decode_seqs = len(portions)
+    want = torch.empty_like(q)
+    ref.attention(q, k_pages, v_pages, ctx, meta, q_heads, kv_heads, dim, dim ** -0.5, window, want)
+    for share in (True, False):
+        monkeypatch.setattr(type(hip), "_share_segments", staticmethod(lambda seq_count, head_blocks: share))
+        cctx, cmeta = _to_cuda(ctx, meta)
+        got = torch.full_like(q, float("nan"), device="cuda")
+        hip.attention(q.cuda(), k_pages.cuda(), v_pages.cuda(), cctx, cmeta, q_heads, kv_heads, dim, dim ** -0.5, window, got)
+        torch.testing.assert_close(got.cpu().float(), want.float(), **attention_tol(torch.bfloat16))
+
+
 def test_attention_of_many_single_tokens_of_very_different_lengths(hip, ref):
     """70 requests in one step (two launches of at most 64), one of them a hundred times longer than most: every
     request's keys are cut into segments of the same size."""
