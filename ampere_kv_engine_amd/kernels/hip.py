@@ -1004,11 +1004,14 @@ class HipKernels(PartsKernels, KernelSet):
         arena = getattr(ctx, "arena", None)
         take = lambda count: (arena.take((count,), torch.float32) if arena is not None
                               else torch.empty(count, dtype=torch.float32, device=self.device))
-        if (split and single and self.cut_keys_on_device and seq_count <= 64
-                and max(ctx.host_seq_lens[seq_first:seq_first + seq_count]) > self.decode_min_segment):
-            # single tokens: their keys are cut on the device, from the lengths there (requests of 128 keys or
-            # fewer are not cut: then the kernel without merge)
-            plan, items_grid = self._decode_plan(ctx, seq_first, seq_count, window, kv_heads * head_groups, share=self._share_segments(seq_count, kv_heads * head_groups))
+        by_plan = split and single and self.cut_keys_on_device and seq_count <= 64
+        # (a step that feeds portions too has its single tokens' segments taken by waves alone, in one launch with the portions
+        # or in two: which one hangs on bounds that are not the same recorded and not)
+        shared_items = by_plan and ctx.num_seqs == ctx.num_decode_seqs and self._share_segments(seq_count, kv_heads * head_groups)
+        if shared_items or (by_plan and max(ctx.host_seq_lens[seq_first:seq_first + seq_count]) > self.decode_min_segment):
+            # single tokens: their keys are cut on the device, from the lengths there (requests of 128 keys or fewer are not
+            # cut: where a wave alone takes a segment, the kernel without merge then gives the same bits)
+            plan, items_grid = self._decode_plan(ctx, seq_first, seq_count, window, kv_heads * head_groups, share=shared_items)
             partial = take(items_grid * kv_heads * head_groups * 16 * nq * (head_dim + 4))
         elif split:
             longest = max(ctx.host_seq_lens[seq_first:seq_first + seq_count])
@@ -1021,7 +1024,6 @@ class HipKernels(PartsKernels, KernelSet):
             if num_splits > 1:
                 partial = take(tiles * kv_heads * head_groups * num_splits * 16 * nq * (head_dim + 4))
         qkv, q_weight, k_weight, eps, table = fresh if fresh is not None else (None, None, None, 0.0, None)
-        waves_per_item = 4 if plan is not None and self._share_segments(seq_count, kv_heads * head_groups) else 1
         self._check(self._attention_mfma_entry(head_dim)(
             _ptr(q), _ptr(k_pages), _ptr(v_pages), _ptr(out), _ptr(partial), _ptr(ctx.q_start), _ptr(ctx.seq_lens),
             _ptr(meta.block_table), _ptr(getattr(meta, "rows", None)), meta.width, seq_first, seq_count, tiles, nq,
@@ -1029,7 +1031,7 @@ class HipKernels(PartsKernels, KernelSet):
             head_groups, tokens_per_tile, page_size, ctypes.c_long(num_pages), ctypes.c_float(scale),
             int(window) if window is not None else 0, seg_keys, num_splits, 1 if single else 0, 1 if shared else 0,
             _ptr(qkv), _ptr(q_weight), _ptr(k_weight), ctypes.c_float(eps), _ptr(table),
-            table.shape[0] if table is not None else 0, _ptr(plan), items_grid, waves_per_item, self._stream()),
+            table.shape[0] if table is not None else 0, _ptr(plan), items_grid, 4 if shared_items else 1, self._stream()),
             "attention")
 
     PLAN_ENTRIES = 132          # ints of a plan before its items (4 per item)
@@ -1040,7 +1042,7 @@ class HipKernels(PartsKernels, KernelSet):
         take it.  Shared segments end a short context's chain of steps sooner and leave a quarter of the partial results, but
         there are at most two rounds of blocks for the device to even out: with up to 32 (request, head block) pairs a
         request has 16 segments or more and their last pieces do not count.  It hangs on the number of requests only, so
-        that a recorded step and the same step run eagerly are cut alike.  Whole steps, alone / shared us: one request of
+        that a recorded step and the same step run eagerly are cut alike; short contexts, too, come by a plan then.  Whole steps, alone / shared us: one request of
         2,048 keys 941 / 928 (8 layers of the 8B sizes), of 16,000 1,017 / 985, four of 64 to 16,000 1,069 / 1,061; 8 heads and
         8 requests of 64 to 12,000 1,115 / 1,141, 27 of 64 to 16,000 1,657 / 1,691 (6 layers of 14B)."""
         return seq_count * head_blocks <= 32
