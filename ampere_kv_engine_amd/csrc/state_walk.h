@@ -1,7 +1,8 @@
 // Recurrences over a matrix state S [dim, columns] per head, walked token after token.  A column of S is spread over R
 // neighbouring lanes (RP rows each), so sums over the rows are sums over RP registers and a butterfly over R lanes inside the
 // vector unit, and columns need nothing of each other - a block takes 256 / R columns of one head.  The recurrence is a chain
-// through the tokens whose length nothing shortens, so what counts is a wave's instructions per token: with four rows a lane,
+// through the tokens (the delta rule of many tokens has a form in chunks, delta_rule.hip), so what counts is a wave's
+// instructions per token: with four rows a lane,
 // one request's heads of 128 x 128 are 1,024 waves - one on every vector unit of the device.  A tile of tokens' vectors passes
 // through LDS for all columns of the block; the next tile's values are asked for before this tile's tokens are walked; a
 // whole tile is walked without a loop (constant LDS addresses, a token's reads issued one token ahead) and its outputs are
