@@ -1114,14 +1114,17 @@ class HipKernels(PartsKernels, KernelSet):
         the faster one from some hundred keys on however few its blocks are, and pays for its longer start before
         (heads of 128, narrow / wide us: 256 keys 15.3 / 16.9, 320 keys 17.3 / 17.4, 400 keys of 16 heads 19.3 / 18.5,
         1,128 keys 39.7 / 33.1, 8,171 keys 233 / 181; heads of 64, half the work a key: 512 keys 14.1 / 15.9, 2,048 keys
-        45.0 / 46.1, 8,192 keys 234 / 201).
+        45.0 / 46.1, 8,192 keys 234 / 201).  A recorded step knows contexts as bounds, powers of two from 2,048 on: lengths are
+        asked for against such powers only, below them the portions' tokens decide, so that it takes the kernel that the
+        same step run eagerly takes.
         Elsewhere the wide blocks do a step of 32 keys for twice the columns with the same loads and bookkeeping (a fifth
         to a quarter faster where they fill the device), but there are half as many of them, and two per compute unit
         instead of three: they are taken when there are two or more per compute unit and the keys are many (measured on
         prompts of 512 to 8,192 tokens after histories of 0 to 15,360)."""
         longest = max(ctx.host_seq_lens[first:ctx.num_seqs])
         if head_dim in (64, 128) and page_size >= 16:
-            return longest >= (384 if head_dim == 128 else 4096)
+            most = max(ctx.host_q_start[r + 1] - ctx.host_q_start[r] for r in range(first, ctx.num_seqs))
+            return longest > 2048 or most >= 384 if head_dim == 128 else longest > 4096
         group = q_heads // kv_heads
         heads_per_tile = min(group, 32)
         per_block = 4 * (32 // heads_per_tile)

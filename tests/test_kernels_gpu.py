@@ -1456,11 +1456,17 @@ def test_attention_on_tiles_of_32_columns_says_that_a_page_is_missing(hip, dim, 
 
 
 def test_attention_takes_tiles_of_32_columns_from_some_hundred_keys_on(hip):
-    """The rule that chooses between 16 and 32 columns a wave asks for the longest context, by head size and page."""
-    ctx = lambda length: SimpleNamespace(num_seqs=1, host_q_start=[0, 60], host_seq_lens=[length])
-    wide = lambda length, dim, page: hip._wide_shared_tiles(ctx(length), 0, 8, 2, dim, page)
-    assert not wide(383, 128, 16) and wide(384, 128, 16) and not wide(4095, 64, 32) and wide(4096, 64, 32)
-    assert not wide(8000, 128, 8) and not wide(8000, 96, 16)
+    """The rule that chooses between 16 and 32 columns a wave asks for a portion's tokens and, against powers of two from 2,048 on
+    (which a recorded step's bounds are), for the longest context, by head size and page."""
+    def wide(tokens, length, dim, page):
+        ctx = SimpleNamespace(num_seqs=2, host_q_start=[0, 1, 1 + tokens], host_seq_lens=[9000, length])
+        return hip._wide_shared_tiles(ctx, 1, 8, 2, dim, page)
+    assert not wide(383, 383, 128, 16) and wide(384, 384, 128, 16) and not wide(60, 2048, 128, 16) and wide(60, 2049, 128, 16)
+    assert not wide(2000, 4096, 64, 32) and wide(60, 4097, 64, 32)
+    assert not wide(600, 600, 128, 8) and not wide(600, 600, 96, 16)
+    for length in (300, 2048, 2049, 4096, 5000):
+        bound = 2048 if length <= 2048 else 4096 if length <= 4096 else 8192
+        assert all(wide(170, length, dim, 16) == wide(170, bound, dim, 16) for dim in (64, 128))
 
 
 @pytest.mark.parametrize("q_heads,kv_heads,dim,page_size", ATTENTION_SIZES + [(32, 8, 128, 16), (40, 2, 64, 8)])
