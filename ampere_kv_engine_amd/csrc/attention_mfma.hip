@@ -1336,7 +1336,7 @@ __device__ __forceinline__ void attention_prompt_body(const Args& a, const int b
   // of them before every read; the turns' own counted waits are what orders them.  Nothing is loaded into registers.
   auto into_lds = [&](const char* from, uint32_t offset, uint32_t to) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-                 :: "s"(to), "v"(offset), "s"(from));
+                 :: "s"(to), "v"(offset), "s"(from) : "m0");
   };
   const uint32_t k_base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_rows)(&k_lds[wave * 512])));
   const uint32_t v_base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_rows)(&v_lds[wave * 512])));
