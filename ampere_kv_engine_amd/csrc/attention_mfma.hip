@@ -1476,6 +1476,11 @@ __device__ __forceinline__ void attention_prompt_body(const Args& a, const int b
   for (int i = 0; i < SP; ++i) at[2][i] = at[3][i] = 0;   // (steps -2 and -1 do not exist: what their loads bring is not read)
 #pragma unroll
   for (int v = 1; v < 4; ++v) lookup(v - 1, pending[v]);
+  // The queries' loads end here, beside the first lookups.  Registers that a loop carries and whose loads may still be on their way
+  // when it is entered are waited for inside it, and the compiler does not count the loads into LDS, which are younger: the first
+  // of four calm turns then waited for all but three of these (heads of 128), or for all (of 64).
+#pragma unroll
+  for (int kt = 0; kt < QT; ++kt) asm volatile("" : "+v"(qreg[kt]));
 #pragma unroll
   for (int j = -3; j < 0; ++j) ask(j, j + 4);
   const int turns = steps + 2;

@@ -1,10 +1,17 @@
-"""What the compiler is told where results cannot show a mistake: inline assembly that writes a register must say so."""
+"""What the compiler is told, and what it makes of it, where results cannot show a mistake: inline assembly that writes a register
+must say so, and loads that are meant to stay on their way must not be waited for."""
 
 import glob
 import os
 import re
+import shutil
+import subprocess
+
+import pytest
 
 from ampere_kv_engine_amd.csrc import build
+
+OBJDUMP = next((p for p in (shutil.which("llvm-objdump"), "/opt/rocm/llvm/bin/llvm-objdump") if p and os.path.exists(p)), None)
 
 
 def test_inline_assembly_that_writes_m0_says_so():
@@ -16,3 +23,35 @@ def test_inline_assembly_that_writes_m0_says_so():
     assert writers, "no block writes m0 any more: this test can go"
     for name, block in writers:
         assert block.count(":") == 3 and '"m0"' in block.split(":")[3], f"{name}: {block}"
+
+
+def _prompt_kernel(dim, pages_per_step, folder):
+    """(address, instruction) of `attention_prompt_kernel` in the built library."""
+    library = build.attention_library_path(dim)
+    if library is None or OBJDUMP is None:
+        pytest.skip("the attention library is not built, or there is nothing to list it with")
+    copied = shutil.copy(library, folder)
+    subprocess.run([OBJDUMP, "--offloading", copied], cwd=folder, check=True, capture_output=True)
+    code, = glob.glob(os.path.join(folder, "*gfx950"))
+    listing = subprocess.run([OBJDUMP, "-d", "--no-show-raw-insn", code], cwd=folder, check=True, capture_output=True, text=True).stdout
+    kernel = re.split(r"\n\n", listing[listing.index(f"attention_prompt_kernelILi{pages_per_step}E"):])[0]
+    lines = [re.match(r"\s+(\S.*?)\s*// ([0-9A-F]+):(?:.*<.*\+0x([0-9a-f]+)>)?", line) for line in kernel.splitlines()]
+    return [(int(m[2], 16), m[1], int(m[3], 16) if m[3] else None) for m in lines if m]
+
+
+@pytest.mark.parametrize("pages_per_step", [1, 2])
+@pytest.mark.parametrize("dim", [64, 128])
+def test_calm_turns_of_the_prompt_attention_wait_for_counted_loads_alone(dim, pages_per_step, tmp_path):
+    """The loop of four calm turns (a turn multiplies D / 16 times for the scores and D / 8 times for the sums) waits for memory four
+    times, and each time leaves the loads of two turns (2 * D / 64 of keys, as many of values) on their way."""
+    code = _prompt_kernel(dim, pages_per_step, str(tmp_path))
+    start = code[0][0]
+    loops = []
+    for index, (at, text, target) in enumerate(code):
+        if text.startswith(("s_cbranch", "s_branch")) and target is not None and start + target <= at:
+            body = [t for a, t, _ in code[:index + 1] if a >= start + target]
+            if sum("v_mfma" in t for t in body) == 4 * (dim // 16 + dim // 8):
+                loops.append(body)
+    assert len(loops) == 1
+    waits = [re.search(r"vmcnt\((\d+)\)", t) for t in loops[0] if t.startswith("s_waitcnt")]
+    assert [int(w[1]) for w in waits if w] == [4 * dim // 64] * 4
