@@ -1108,31 +1108,57 @@ class HipKernels(PartsKernels, KernelSet):
         blocks = sum((starts[r + 1] - starts[r] + per_block - 1) // per_block for r in range(first, ctx.num_seqs))
         return blocks * kv_heads * ((group + heads_per_tile - 1) // heads_per_tile)
 
-    def _wide_shared_tiles(self, ctx, first, q_heads, kv_heads, head_dim, page_size) -> bool:
+    def _wide_shared_tiles(self, ctx, first, q_heads, kv_heads, head_dim, page_size, window=None) -> bool:
         """Whether the prompt portions of the step go to blocks of 4 x 32 columns rather than 4 x 16.
-        Heads of 64 and 128 on pages of 16 and more have a kernel of their own for 32 columns, whose turns overlap: it is
-        the faster one from some hundred keys on however few its blocks are, and pays for its longer start before
-        (heads of 128, narrow / wide us: 256 keys 15.3 / 16.9, 320 keys 17.3 / 17.4, 400 keys of 16 heads 19.3 / 18.5,
-        1,128 keys 39.7 / 33.1, 8,171 keys 233 / 181; heads of 64, half the work a key: 512 keys 14.1 / 15.9, 2,048 keys
-        45.0 / 46.1, 8,192 keys 234 / 201).  A recorded step knows contexts as bounds, powers of two from 2,048 on: lengths are
-        asked for against such powers only, below them the portions' tokens decide, so that it takes the kernel that the
-        same step run eagerly takes.
+        Heads of 64 and 128 on pages of 16 and more have a kernel of their own for 32 columns, whose turns overlap: it does a
+        step of keys faster, pays for its longer start, and makes half as many blocks.  All figures narrow / wide us.
+        Heads of 128: from some hundred keys on (32 / 8 heads: 256 keys 14.3 / 15.7, 383 18.1 / 18.4, 2,048 82 / 66; 256 tokens after
+        14,000 380 / 300; 16 portions of 300 after 1,500 249 / 188).  Where a window shows a column fewer, only blocks that fill
+        most of the device's two places a unit make up for the start (window 128: 512 tokens of 16 / 4 heads 13.2 / 15.7, 668 of two
+        requests of 40 / 8 31.4 / 23.7; blocks of heads that share no keys hold 128 tokens: 300 after 5,000 of 16 / 16 heads, window 512,
+        26.4 / 29.3).
+        Heads of 64, half the work a key: where blocks fill those places (2,048 tokens of 32 / 8 heads after 4,096 159 / 140) - of
+        short contexts with some to spare, where a request fills them or blocks walk 700 keys and more (3,000 tokens 79 / 71, 24
+        portions of 375 after 1,000 196 / 173, but 2,048 43.0 / 43.6, four requests of 1,024 46 / 51) -; else after 4,096
+        keys, on pages of 16 where every unit has a block and few have a second (1,024 tokens of 32 / 8 heads after 4,000 87 / 82, but
+        512 72 / 74, 700 of three requests of 16 / 4 heads after 6,000 140 / 152), on larger ones always (512 tokens 74 / 71, 700
+        145 / 143) - unless a window shows fewer (512 tokens, window 1,024 23.3 / 25.0).
+        A recorded step knows contexts as bounds, powers of two from 2,048 on: in a step that may be recorded lengths are asked for
+        against such powers only and all else hangs on the portions' tokens, so that it takes the kernel that the same step run
+        eagerly takes.
         Elsewhere the wide blocks do a step of 32 keys for twice the columns with the same loads and bookkeeping (a fifth
         to a quarter faster where they fill the device), but there are half as many of them, and two per compute unit
         instead of three: they are taken when there are two or more per compute unit and the keys are many (measured on
         prompts of 512 to 8,192 tokens after histories of 0 to 15,360)."""
         longest = max(ctx.host_seq_lens[first:ctx.num_seqs])
-        if head_dim in (64, 128) and page_size >= 16:
-            most = max(ctx.host_q_start[r + 1] - ctx.host_q_start[r] for r in range(first, ctx.num_seqs))
-            return longest > 2048 or most >= 384 if head_dim == 128 else longest > 4096
         group = q_heads // kv_heads
         heads_per_tile = min(group, 32)
         per_block = 4 * (32 // heads_per_tile)
+        per_token_block = kv_heads * ((group + heads_per_tile - 1) // heads_per_tile)
         starts = ctx.host_q_start
-        blocks = sum((starts[r + 1] - starts[r] + per_block - 1) // per_block for r in range(first, ctx.num_seqs))
-        blocks *= kv_heads * ((group + heads_per_tile - 1) // heads_per_tile)
+        counts = [starts[r + 1] - starts[r] for r in range(first, ctx.num_seqs)]
+        most = max(counts)
+        blocks = sum((count + per_block - 1) // per_block for count in counts) * per_token_block
         units = self.compute_units
-        return blocks >= 2 * units and (longest >= 4096 or 2 * blocks >= 5 * units)
+        many = 2 * blocks >= 5 * units
+        if head_dim not in (64, 128) or page_size < 16:
+            return blocks >= 2 * units and (longest >= 4096 or many)
+        # (about the keys that a block walks, in steps of many blocks that are never recorded, whose lengths are what they are)
+        exact = starts[ctx.num_seqs] > max(self.FEW_TOKENS, getattr(ctx, "recordable_tokens", 0))
+        walked = longest - most // 2 if many and exact else 0
+        if head_dim == 128:
+            if window is not None and 2 * blocks < 3 * units and window < (512 if 4 * blocks >= 3 * units else 512 + 4 * per_block):
+                return False
+            return longest > 2048 or most >= 384 or walked >= 512
+        if longest <= 4096:
+            in_one = (most + per_block - 1) // per_block * per_token_block
+            return many and (window is None or window >= 1024) and (longest > 2048 or in_one >= 2 * units or walked >= 704)
+        if 2 * blocks >= 3 * units:
+            return True
+        even = 3 * units <= 4 * blocks <= 4 * units
+        if window is not None and window < (256 + 4 * per_block if even else 4096):
+            return False
+        return even or page_size >= 32
 
     def _matrix_core_attention(self, dtype, page_size) -> bool:
         fits = page_size >= 4 and page_size & (page_size - 1) == 0
@@ -1252,7 +1278,7 @@ class HipKernels(PartsKernels, KernelSet):
                 if shared and nq == 2:
                     wide = self.wide_prompt_tiles
                     if wide is None:
-                        wide = self._wide_shared_tiles(ctx, decodes, q_heads, kv_heads, head_dim, page_size)
+                        wide = self._wide_shared_tiles(ctx, decodes, q_heads, kv_heads, head_dim, page_size, window)
                     nq = 2 if wide else 1
                 self._attention_mfma(*common, decodes, ctx.num_seqs - decodes, nq, False, shared=shared)
 

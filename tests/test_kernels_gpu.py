@@ -1469,6 +1469,39 @@ def test_attention_takes_tiles_of_32_columns_from_some_hundred_keys_on(hip):
         assert all(wide(170, length, dim, 16) == wide(170, bound, dim, 16) for dim in (64, 128))
 
 
+def test_tiles_of_32_columns_are_chosen_by_what_a_column_sees_and_by_the_blocks(hip):
+    """Short windows, and heads of 64, take them only where the blocks fill the device; a recorded step's bounds change nothing."""
+    units = hip.compute_units
+
+    def wide(counts, longest, dim, page=16, window=None, q_heads=32, kv_heads=8):
+        starts = [0]
+        for count in counts:
+            starts.append(starts[-1] + count)
+        ctx = SimpleNamespace(num_seqs=len(counts), host_q_start=starts, host_seq_lens=[longest] * len(counts))
+        return hip._wide_shared_tiles(ctx, 0, q_heads, kv_heads, dim, page, window)
+
+    tokens = 32 * (units // 8)              # a block a unit, at 32 / 8 heads (a block holds 32 tokens of a key head)
+    for dim in (64, 128):
+        assert not wide([tokens], 5000, dim, window=128) and wide([3 * tokens // 2], 5000, dim, window=128)
+        assert not wide([300], 5000, dim, window=512, q_heads=16, kv_heads=16)
+    assert wide([tokens // 2], 5000, 128) and wide([tokens // 2], 5000, 128, window=1024)
+    # heads of 64 after a long history: one block a unit, or one and a half and more
+    assert [wide([count], 9000, 64) for count in (tokens // 2, tokens, tokens + 32, 2 * tokens - 32, 2 * tokens)] == [False, True, False, True, True]
+    assert all(wide([count], 9000, 64, page=32) for count in (tokens // 2, tokens, tokens + 32))
+    # and of a short one: more than two a unit, one request's or walking many keys
+    assert [wide([tokens * n], tokens * n, 64) for n in (1, 2, 3)] == [False, False, True]
+    assert wide([2 * tokens] * 2, 2 * tokens, 64) and not wide([tokens] * 4, tokens, 64) and wide([tokens] * 4, 2 * tokens, 64)
+    assert not wide([3 * tokens], 3 * tokens, 64, window=100)
+    # many portions behind histories, in steps that are never recorded
+    for dim in (64, 128):
+        assert wide([300] * 16, 1800, dim) and not wide([300] * 16, 300, dim)
+    for longest, bound in ((300, 2048), (2048, 2048), (2049, 4096), (4096, 4096), (5000, 8192)):
+        for dim in (64, 128):
+            for window in (None, 100, 1500, 3000, 6000):
+                assert all(wide(counts, longest, dim, page, window) == wide(counts, bound, dim, page, window)
+                           for counts in ([170], [300, 170], [512]) for page in (16, 32))
+
+
 @pytest.mark.parametrize("q_heads,kv_heads,dim,page_size", ATTENTION_SIZES + [(32, 8, 128, 16), (40, 2, 64, 8)])
 @pytest.mark.parametrize("histories", [[0], [64, 17, 0], [1500, 2, 700, 255], [4000] * 9])
 @pytest.mark.parametrize("window", [None, 100])
