@@ -758,16 +758,16 @@ constexpr float kLazy = 8.f;  // the exponentials' reference point trails the ma
 
 // SP: pages per step of 32 keys (4: pages of 8 tokens, 2: of 16, 1: of 32 or more) - with it the page arithmetic of a
 // step is known when compiling.
+typedef bf16_t SharedKeys[2][32 * KROW], SharedValues[2][D * VROW];
 struct SharedLds {
-  bf16_t k[2][32 * KROW], v[2][D * VROW];
+  SharedKeys k;
+  SharedValues v;
   int bad_page;
 };
 template <int NQ, int SP>
-__device__ __forceinline__ void attention_shared_body(const Args& a, const int block, const int thread, SharedLds& lds) {
+__device__ __forceinline__ void attention_shared_body(const Args& a, const int block, const int thread, SharedKeys& k_lds,
+                                                      SharedValues& v_lds, int& bad_page) {
   const int page_shift = SP == 4 ? 3 : (SP == 2 ? 4 : a.page_shift);
-  auto& k_lds = lds.k;
-  auto& v_lds = lds.v;
-  int& bad_page = lds.bad_page;
   const int tid = thread, lane = tid & 63, r16 = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   // Late tiles of a prompt see the most keys.  Blocks are ranked longest first, and the ranks are dealt out to the
@@ -1201,8 +1201,17 @@ __device__ __forceinline__ void attention_shared_body(const Args& a, const int b
 
 template <int NQ, int SP>
 __global__ __launch_bounds__(64 * kSharedWaves, D <= 128 ? (NQ == 1 ? 3 : 2) : 1) void attention_shared_kernel(const Args a) {
-  __shared__ __align__(16) SharedLds lds;
-  attention_shared_body<NQ, SP>(a, static_cast<int>(blockIdx.x), static_cast<int>(threadIdx.x), lds);
+  // (How the compiler orders a step hangs on whether it sees one array or three.  32 / 8 heads, 400 tokens after 4,500, one / three:
+  // heads of 64 on pages of 64 79.6 / 77.5 us, on pages of 16 75.1 / 76.5; heads of 128 on pages of 16 131.7 / 140.0.)
+  if constexpr (D == 64 && SP == 1) {
+    __shared__ __align__(16) SharedKeys k;
+    __shared__ __align__(16) SharedValues v;
+    __shared__ int bad_page;
+    attention_shared_body<NQ, SP>(a, static_cast<int>(blockIdx.x), static_cast<int>(threadIdx.x), k, v, bad_page);
+  } else {
+    __shared__ __align__(16) SharedLds lds;
+    attention_shared_body<NQ, SP>(a, static_cast<int>(blockIdx.x), static_cast<int>(threadIdx.x), lds.k, lds.v, lds.bad_page);
+  }
 }
 
 // ---- prompt portions on tiles of 32 columns: both products on 32 x 32 tiles, three steps in the air ----------------------
@@ -1582,7 +1591,7 @@ __global__ __launch_bounds__(64 * kSharedWaves, 2) void attention_pair_kernel(co
   if constexpr (D % 64 == 0) {
     __shared__ __align__(16) SharedLds lds;
     if (static_cast<int>(blockIdx.x) < portion_blocks) {
-      attention_shared_body<1, SP>(portion, static_cast<int>(blockIdx.x), static_cast<int>(threadIdx.x), lds);
+      attention_shared_body<1, SP>(portion, static_cast<int>(blockIdx.x), static_cast<int>(threadIdx.x), lds.k, lds.v, lds.bad_page);
     } else {
       const int gx = single.kv_heads * single.head_groups, gy = single.items_grid;
       const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
