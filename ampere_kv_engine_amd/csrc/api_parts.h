@@ -166,15 +166,20 @@ int akv_gated_linear_scan(const void* u, int dtype, const float* gates, const fl
 // Per request and head, S [dim, vdim] (in the slot as [heads, vdim, dim] float32): S <- g S; u = beta (v - S^T k);
 // S <- S + k u^T; o = S^T q.  out [tokens, heads x vdim] = o / rms(o) * norm_weight[i] * act(gates[t * gate_stride + h * vdim
 // + i]), gate_act 1: sigmoid, 2: silu.  Decay logits and gates are float32 where decays are per channel, else of `dtype`.
-// `workspace`: akv_delta_rule_workspace(...) floats.  `longest`: the most tokens a request brings (chooses the walk: token by
-// token, its tile, or in chunks of 16 tokens).
-long akv_delta_rule_workspace(int tokens, int seqs, int heads, int groups, int dim, int vdim, int decay_per_head, int longest);
+// akv_delta_rule_forms: a request of fewer than from[0] tokens walks token by token in small tiles, of from[1] and more it goes in
+// chunks of 16 tokens, between them it walks in large tiles - whatever else is in the step: a request's sums do not hang on it
+// (between the forms they differ by rounding).
+// `workspace`: akv_delta_rule_workspace(...) floats.  `longest`: the most tokens a request brings.  `walked_tokens`: the tokens up to
+// the end of the last request that walks (0: none does); `walked_forms`: 1 if some walk in small tiles, + 2 if some in large ones.
+void akv_delta_rule_forms(int dim, int* from);
+long akv_delta_rule_workspace(int tokens, int seqs, int heads, int groups, int dim, int vdim, int decay_per_head, int longest,
+                              int walked_tokens);
 int akv_delta_rule(const void* conv, long conv_stride, int dtype, const void* beta_logits, long beta_stride,
                    const void* decay_logits, int decay_dtype, long decay_stride, const float* decay_bias, const float* rate,
                    int decay_per_head, const void* gates, int gate_dtype, long gate_stride, int gate_act,
                    const float* norm_weight, float unit_eps, float norm_eps, float q_scale, float* state, long state_stride,
                    const int* q_start, const int* seq_slots, float* workspace, void* out, int tokens, int seqs, int heads,
-                   int groups, int dim, int vdim, int longest, hipStream_t stream);
+                   int groups, int dim, int vdim, int longest, int walked_tokens, int walked_forms, hipStream_t stream);
 
 // ---- time mixing and the matrix memory (linear_states.hip) ---------------------------------------------------------------
 // out [count, tokens, width] = x_t + (x_(t-1) - x_t) * mu[s]; the row before a portion's first token lies in the request's slot

@@ -4,8 +4,9 @@
 // Everything after the projections and the short convolutions is float32: the unit norms, sigmoid, softplus, the
 // exponentials, the state and its sums, the norm of the outputs.
 //
-// Three kernels (of many tokens: two others before the last, below).  `delta_prepare` is token-wise: the unit vectors, decays, betas and k . q of every token, float32, into a
-// workspace.  The walk over a request's tokens is state_walk.h's with the rule kDelta.
+// Three kernels.  `delta_prepare` is token-wise: the unit vectors, decays, betas and k . q of every token, float32, into a
+// workspace.  The walk over a request's tokens is state_walk.h's with the rule kDelta.  (For the requests that bring many
+// tokens two others stand in the place of these: below.)
 // `state_finish_kernel` is token-wise again: o / rms(o) times a weight per value channel and a gate.
 
 #include <type_traits>
@@ -126,17 +127,27 @@ __global__ __launch_bounds__(256) void delta_prepare_fours_kernel(const T* __res
 // Chunks count from a request's first token of the step; chunk c of request r has slot q_start[r] / 16 + r + c of the
 // workspace, which no other request's chunks reach.
 // Bound by the chain: per chunk (dim 128) 20 matrix instructions of 32 cycles that wait for each other, an exchange of sums
-// through LDS (160 ns alone) and their way between registers; 0.92 us as measured.  One request of 16 heads of 128 x 128, decays
-// per channel, whole rule (prepare, walk, finish), token by token / in chunks: 16 tokens 23.6 / 22.2 us, 171 34.0 / 29.8, 512 76.1 /
-// 56.4, 2,000 261 / 158; 16 requests of 16 49.9 / 47.7.  Against 64 bits both are 2e-7 off (relative, outputs and states, 64 to
-// 2,000 tokens).  With the outputs in the chain's own waves the walk of 2,000 tokens took 149 us, with them beside it 116.
-constexpr int kChunk = 16, kChunkFrom = 16;
+// through LDS (160 ns alone) and their way between registers; 0.92 us as measured.  One request of 16 heads of 128 x 128, whole
+// rule (prepare, walk, finish), token by token / in chunks: decays per channel 171 tokens 35.5 / 29.4 us, 512 78.8 / 55.8, 2,000 257 /
+// 154; a decay per head 32.3 / 26.7, 70.0 / 52.9, 229 / 146.  Against 64 bits both are 2e-7 off (relative, outputs and states, 64
+// to 2,000 tokens).  With the outputs in the chain's own waves the walk of 2,000 tokens took 149 us, with them beside it 116.
+constexpr int kChunk = 16;
 typedef __attribute__((ext_vector_type(4))) float floatx4;
 
 inline long chunk_slots(int tokens, int seqs) { return tokens / kChunk + static_cast<long>(seqs) + 1; }
 // [cum k | cum q | k for the next state] in the order the matrix instruction's lanes read them, [cum_15], [T], [B]
 __host__ __device__ inline long chunk_floats(int dim) { return 3L * kChunk * dim + dim + 2L * kChunk * kChunk; }
-inline bool chunks_fit(int dim, int longest) { return dim % 64 == 0 && dim <= 256 && longest >= kChunkFrom; }
+// The fewest tokens of a request that goes in chunks.  Which form a request takes hangs on its own tokens and the head's size
+// alone, so that its bits do not change with what else is in the step (fewer than kTilesFrom walk in small tiles, others in
+// large ones: a step of all three kinds has three launches).  32 single tokens beside 171, 16 heads of 128 x 128: 94 us, where
+// the single ones went in chunks too 113, where all walked in large tiles 162.  The lines lie
+// where one request alone breaks even; batches would from fewer on.  Whole rule, walk / chunks us, decays per channel: 16 heads of 64
+// x 64 64 tokens 14.9 / 15.5, 80 18.1 / 16.1; 16 heads of 128 x 128 96 tokens 21.6 / 24.2, 128 25.8 / 25.9, 160 30.4 / 28.4 (four
+// requests 80 tokens 43.0 / 36.6; a decay per head 96 21.2 / 21.5, 128 25.0 / 23.5); 8 heads of 256 x 256 32 tokens 21.8 / 27.5, 48
+// 32.2 / 29.6; 6 of 192 x 192 32 22.2 / 24.2, 48 32.2 / 26.0.
+__host__ __device__ inline int chunks_from(int dim) {
+  return dim == 64 ? 65 : dim == 128 ? 128 : dim == 192 || dim == 256 ? 33 : 0x7fffffff;
+}
 
 // Products over the 16 lanes of a row: of lanes up to this one (SHR), of this one and those behind it (SHL).
 template <int CTRL> __device__ __forceinline__ float times_lane(float v) {
@@ -164,7 +175,7 @@ __global__ __launch_bounds__(256) void delta_chunks_kernel(const T* __restrict__
     else high = middle - 1;
   }
   const int t0 = q_start[r] + (slot - (q_start[r] / kChunk + r)) * kChunk, count = min(kChunk, q_start[r + 1] - t0);
-  if (count <= 0) return;                                  // (the same in every thread)
+  if (count <= 0 || q_start[r + 1] - q_start[r] < chunks_from(dim)) return;   // (the same in every thread)
   float* to = chunks + (static_cast<long>(slot) * heads + h) * chunk_floats(dim);
 
   // unit vectors and decays, thread (token, 16 parts of four elements 64 apart); a token that does not exist changes nothing
@@ -297,7 +308,7 @@ __global__ __launch_bounds__(512) void delta_chunk_walk_kernel(const float* chun
   const int column_blocks = (vdim + 15) / 16;
   const int r = unit / (heads * column_blocks), h = unit / column_blocks % heads, col0 = unit % column_blocks * 16;
   const int first = q_start[r], last = q_start[r + 1];
-  if (first >= last) return;
+  if (last - first < chunks_from(dim)) return;             // (it walks)
   const int tid = threadIdx.x & 255, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = lane >> 4;
   const bool chain = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) == 0;
   const int total = (last - first + kChunk - 1) / kChunk;
@@ -514,30 +525,11 @@ void launch_chunks(const T* conv, long conv_stride, const T* beta_logits, long b
       chunks, conv + 2L * groups * 64 * TILES, conv_stride, state, state_stride, q_start, seq_slots, raw, units, heads, vdim);
 }
 
-template <typename T, typename TD, typename TG, bool HEAD_DECAY>
-int delta_rule(const T* conv, long conv_stride, const T* beta_logits, long beta_stride, const TD* decay_logits,
-               long decay_stride, const float* decay_bias, const float* rate, const TG* gates, long gate_stride, int gate_act,
-               const float* norm_weight, float unit_eps, float norm_eps, float q_scale, float* state, long state_stride,
-               const int* q_start, const int* seq_slots, float* workspace, T* out, int tokens, int seqs, int heads, int groups,
-               int dim, int vdim, int longest, hipStream_t stream) {
-  if (chunks_fit(dim, longest) && conv_stride % 4 == 0 && in_fours(conv) && in_fours(workspace) && state_stride % 4 == 0 &&
-      in_fours(state) && (HEAD_DECAY || (decay_stride % 4 == 0 && in_fours(decay_logits) && in_fours(decay_bias)))) {
-    float* raw = workspace + chunk_slots(tokens, seqs) * heads * chunk_floats(dim);
-#define AKV_CHUNKS(TILES)                                                                                                      \
-  launch_chunks<T, TD, HEAD_DECAY, TILES>(conv, conv_stride, beta_logits, beta_stride, decay_logits, decay_stride, decay_bias, \
-                                          rate, unit_eps, q_scale, state, state_stride, q_start, seq_slots, workspace, raw,    \
-                                          tokens, seqs, heads, groups, vdim, stream)
-    if (dim == 64) AKV_CHUNKS(1);
-    else if (dim == 128) AKV_CHUNKS(2);
-    else if (dim == 192) AKV_CHUNKS(3);
-    else AKV_CHUNKS(4);
-#undef AKV_CHUNKS
-    launch_state_finish<T, TG>(raw, nullptr, 0.f, norm_weight, 0, gates, gate_stride, gate_act, norm_eps, out, tokens, heads, vdim,
-                               0, stream);
-    return 0;
-  }
-  float* prepared = workspace;
-  float* raw = workspace + (static_cast<long>(tokens) + kRowsBehind) * prepared_width(heads, groups, dim, HEAD_DECAY);
+// Unit vectors, decays, betas and k . q of the first `tokens` tokens.
+template <typename T, typename TD, bool HEAD_DECAY>
+void launch_prepare(const T* conv, long conv_stride, const T* beta_logits, long beta_stride, const TD* decay_logits, long decay_stride,
+                    const float* decay_bias, const float* rate, float unit_eps, float q_scale, float* prepared, int tokens, int heads,
+                    int groups, int dim, hipStream_t stream) {
   if (lanes_of_fours(dim) && conv_stride % 4 == 0 && in_fours(conv) && in_fours(prepared) &&
       (HEAD_DECAY || (decay_stride % 4 == 0 && in_fours(decay_logits) && in_fours(decay_bias)))) {
     const int pairs = (groups * dim / 4 + kWave - 1) / kWave * kWave, threads = pairs + (HEAD_DECAY ? 0 : heads * dim / 4);
@@ -550,10 +542,55 @@ int delta_rule(const T* conv, long conv_stride, const T* beta_logits, long beta_
         conv, conv_stride, beta_logits, beta_stride, decay_logits, decay_stride, decay_bias, rate, unit_eps, q_scale, prepared,
         heads, groups, dim);
   }
-  const int status = launch_state_walk<T, kDelta, HEAD_DECAY>(prepared, conv + 2L * groups * dim, conv_stride, state,
-                                                              state_stride, q_start, seq_slots, raw, seqs, heads, groups, dim,
-                                                              vdim, 0, longest, stream);
-  if (status != 0) return status;
+}
+
+// The workspace: [chunks][rows of the tokens that walk][outputs], the first part only where some request goes in chunks.
+struct Parts {
+  long rows, raw, total;      // floats before the rows, before the outputs, in all
+};
+inline Parts parts_of(int tokens, int seqs, int heads, int groups, int dim, int vdim, bool head_decay, bool chunks, int walked_tokens) {
+  Parts p;
+  p.rows = chunks ? chunk_slots(tokens, seqs) * heads * chunk_floats(dim) : 0;
+  p.raw = p.rows + (walked_tokens > 0 ? (static_cast<long>(walked_tokens) + kRowsBehind) * prepared_width(heads, groups, dim, head_decay) : 0);
+  p.total = p.raw + (static_cast<long>(tokens) + kRowsBehind) * heads * vdim;
+  return p;
+}
+
+template <typename T, typename TD, typename TG, bool HEAD_DECAY>
+int delta_rule(const T* conv, long conv_stride, const T* beta_logits, long beta_stride, const TD* decay_logits,
+               long decay_stride, const float* decay_bias, const float* rate, const TG* gates, long gate_stride, int gate_act,
+               const float* norm_weight, float unit_eps, float norm_eps, float q_scale, float* state, long state_stride,
+               const int* q_start, const int* seq_slots, float* workspace, T* out, int tokens, int seqs, int heads, int groups,
+               int dim, int vdim, int longest, int walked_tokens, bool shorts, bool longer, hipStream_t stream) {
+  const bool chunks = longest >= chunks_from(dim) && conv_stride % 4 == 0 && in_fours(conv) && in_fours(workspace) &&
+                      state_stride % 4 == 0 && in_fours(state) &&
+                      (HEAD_DECAY || (decay_stride % 4 == 0 && in_fours(decay_logits) && in_fours(decay_bias)));
+  if (!chunks) walked_tokens = tokens, longer = longest >= kTilesFrom;
+  const Parts parts = parts_of(tokens, seqs, heads, groups, dim, vdim, HEAD_DECAY, chunks, walked_tokens);
+  float* raw = workspace + parts.raw;
+  if (chunks) {
+#define AKV_CHUNKS(TILES)                                                                                                      \
+  launch_chunks<T, TD, HEAD_DECAY, TILES>(conv, conv_stride, beta_logits, beta_stride, decay_logits, decay_stride, decay_bias, \
+                                          rate, unit_eps, q_scale, state, state_stride, q_start, seq_slots, workspace, raw,    \
+                                          tokens, seqs, heads, groups, vdim, stream)
+    if (dim == 64) AKV_CHUNKS(1);
+    else if (dim == 128) AKV_CHUNKS(2);
+    else if (dim == 192) AKV_CHUNKS(3);
+    else AKV_CHUNKS(4);
+#undef AKV_CHUNKS
+  }
+  if (walked_tokens > 0) {
+    float* prepared = workspace + parts.rows;
+    launch_prepare<T, TD, HEAD_DECAY>(conv, conv_stride, beta_logits, beta_stride, decay_logits, decay_stride, decay_bias, rate,
+                                      unit_eps, q_scale, prepared, walked_tokens, heads, groups, dim, stream);
+    auto walk = [&](int longest, int least, int most) {
+      return launch_state_walk<T, kDelta, HEAD_DECAY>(prepared, conv + 2L * groups * dim, conv_stride, state, state_stride, q_start,
+                                                      seq_slots, raw, seqs, heads, groups, dim, vdim, 0, longest, stream, least, most);
+    };
+    const int short_status = shorts ? walk(kTilesFrom - 1, 0, kTilesFrom - 1) : 0;
+    const int status = longer && short_status == 0 ? walk(longest, kTilesFrom, chunks ? chunks_from(dim) - 1 : 0x7fffffff) : short_status;
+    if (status != 0) return status;
+  }
   launch_state_finish<T, TG>(raw, nullptr, 0.f, norm_weight, 0, gates, gate_stride, gate_act, norm_eps, out, tokens, heads, vdim,
                              0, stream);
   return 0;
@@ -563,12 +600,15 @@ int delta_rule(const T* conv, long conv_stride, const T* beta_logits, long beta_
 
 extern "C" {
 
-long akv_delta_rule_workspace(int tokens, int seqs, int heads, int groups, int dim, int vdim, int decay_per_head, int longest) {
-  const long outputs = static_cast<long>(heads) * vdim;
-  const long rows = (static_cast<long>(tokens) + kRowsBehind) * (prepared_width(heads, groups, dim, decay_per_head != 0) + outputs);
-  if (!chunks_fit(dim, longest)) return rows;
-  const long in_chunks = chunk_slots(tokens, seqs) * heads * chunk_floats(dim) + tokens * outputs;
-  return in_chunks > rows ? in_chunks : rows;
+void akv_delta_rule_forms(int dim, int* from) { from[0] = kTilesFrom, from[1] = chunks_from(dim); }
+
+long akv_delta_rule_workspace(int tokens, int seqs, int heads, int groups, int dim, int vdim, int decay_per_head, int longest,
+                              int walked_tokens) {
+  const bool head_decay = decay_per_head != 0;
+  const long walked = parts_of(tokens, seqs, heads, groups, dim, vdim, head_decay, false, tokens).total;
+  if (longest < chunks_from(dim)) return walked;
+  const long in_chunks = parts_of(tokens, seqs, heads, groups, dim, vdim, head_decay, true, walked_tokens).total;
+  return in_chunks > walked ? in_chunks : walked;
 }
 
 int akv_delta_rule(const void* conv, long conv_stride, int dtype, const void* beta_logits, long beta_stride,
@@ -576,10 +616,11 @@ int akv_delta_rule(const void* conv, long conv_stride, int dtype, const void* be
                    int decay_per_head, const void* gates, int gate_dtype, long gate_stride, int gate_act,
                    const float* norm_weight, float unit_eps, float norm_eps, float q_scale, float* state, long state_stride,
                    const int* q_start, const int* seq_slots, float* workspace, void* out, int tokens, int seqs, int heads,
-                   int groups, int dim, int vdim, int longest, hipStream_t stream) {
+                   int groups, int dim, int vdim, int longest, int walked_tokens, int walked_forms, hipStream_t stream) {
   if (tokens <= 0 || seqs <= 0) return 0;
   if (heads <= 0 || groups <= 0 || heads % groups != 0 || dim <= 0 || vdim <= 0 || dim > 2048) return -2;
   if (gate_act != 1 && gate_act != 2) return -2;
+  if (walked_tokens < 0 || walked_tokens > tokens) return -2;
   // decays per channel come from a product of their own with float32 sums, as do their gates; decays per head and their
   // gates are columns of the layer's first product
   const int own = decay_per_head ? dtype : static_cast<int>(kF32);
@@ -590,7 +631,7 @@ int akv_delta_rule(const void* conv, long conv_stride, int dtype, const void* be
                                        static_cast<const TD*>(decay_logits), decay_stride, decay_bias, rate,                    \
                                        static_cast<const TD*>(gates), gate_stride, gate_act, norm_weight, unit_eps, norm_eps,   \
                                        q_scale, state, state_stride, q_start, seq_slots, workspace, static_cast<T*>(out), tokens, \
-                                       seqs, heads, groups, dim, vdim, longest, stream)
+                                       seqs, heads, groups, dim, vdim, longest, walked_tokens, walked_forms & 1, walked_forms & 2, stream)
   AKV_DISPATCH(dtype, T, {
     if (decay_per_head) AKV_DELTA(T, true);
     else AKV_DELTA(float, false);

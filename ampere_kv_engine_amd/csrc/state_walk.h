@@ -116,7 +116,7 @@ __global__ __launch_bounds__(256) void state_walk_kernel(const float* __restrict
                                                          long value_stride, float* __restrict__ state,
                                                          long state_stride, const int* __restrict__ q_start,
                                                          const int* __restrict__ seq_slots, float* __restrict__ raw_out,
-                                                         int heads, int groups, int dim, int vdim, int ones) {
+                                                         int heads, int groups, int dim, int vdim, int ones, int least, int most) {
   using Tile = StateTile<RP, R, CAP, HEAD_DECAY>;
   constexpr int SP = Tile::kSegment, kArray = Tile::kArray, kColumns = Tile::kColumns, kTile = Tile::kTokens;
   constexpr int kArrays = Tile::kArrays, kScalars = Tile::kScalars;
@@ -134,6 +134,7 @@ __global__ __launch_bounds__(256) void state_walk_kernel(const float* __restrict
   const int col = col0 + threadIdx.x / R;
   const bool works = col < columns;
   const int first = q_start[r], last = q_start[r + 1];
+  if (last - first < least || last - first > most) return;   // (another launch takes this request)
   const long width = prepared_width(heads, groups, dim, HEAD_DECAY);
   const int share = heads / groups;
   const long q_off = static_cast<long>(h / share) * dim, k_off = static_cast<long>(groups + h / share) * dim;
@@ -407,7 +408,8 @@ __global__ __launch_bounds__(THREADS) void tile_walk_kernel(const float* __restr
                                                                 long value_stride, float* __restrict__ state,
                                                                 long state_stride, const int* __restrict__ q_start,
                                                                 const int* __restrict__ seq_slots, float* __restrict__ raw_out,
-                                                                int units, int heads, int groups, int dim, int vdim, int ones) {
+                                                                int units, int heads, int groups, int dim, int vdim, int ones,
+                                                                int least, int most) {
   using Tile = SumTile<R, CP, THREADS, HEAD_DECAY>;
   constexpr int kTile = Tile::kTokens, kArrays = Tile::kArrays, kArray = Tile::kArray, kColumns = Tile::kColumns;
   constexpr int kScalars = Tile::kScalars, kGroups = THREADS / R, kAhead = 2;
@@ -423,6 +425,7 @@ __global__ __launch_bounds__(THREADS) void tile_walk_kernel(const float* __restr
   const int r = unit / (heads * column_blocks), h = unit / column_blocks % heads, col0 = unit % column_blocks * kColumns;
   const int part = threadIdx.x % R, group = threadIdx.x / R;
   const int first = q_start[r], last = q_start[r + 1];
+  if (last - first < least || last - first > most) return;   // (another launch takes this request)
   const long width = prepared_width(heads, groups, dim, HEAD_DECAY);
   const int share = heads / groups;
   const long q_off = static_cast<long>(h / share) * dim, k_off = static_cast<long>(groups + h / share) * dim;
@@ -627,16 +630,18 @@ __global__ __launch_bounds__(THREADS) void tile_walk_kernel(const float* __restr
 }
 
 // Launches the walk for heads of `dim` x (vdim + ones); dims beyond 2,048 are refused.  `longest`: the most tokens a request
-// of the step brings (short steps take small tiles; the sums are the same either way).
+// of the step brings (short steps take small tiles, long ones where they can `tile_walk_kernel`, whose sums differ by rounding).
+// Requests of fewer than `least` tokens and of more than `most` are passed by.
+constexpr int kTilesFrom = 16;
 template <typename T, int RULE, bool HEAD_DECAY>
 int launch_state_walk(const float* prepared, const T* values, long value_stride, float* state, long state_stride,
                       const int* q_start, const int* seq_slots, float* raw, int seqs, int heads, int groups, int dim, int vdim,
-                      int ones, int longest, hipStream_t stream) {
+                      int ones, int longest, hipStream_t stream, int least = 0, int most = 0x7fffffff) {
   if (dim <= 0 || dim > 2048) return -2;
   const int rp = dim <= 256 ? 4 : dim <= 512 ? 8 : dim <= 1024 ? 16 : 32;
   int R = 1;
   while (R * rp < dim) R *= 2;
-  if (longest >= 16 && dim % 4 == 0 && rp == 4 && R >= 8) {
+  if (longest >= kTilesFrom && dim % 4 == 0 && rp == 4 && R >= 8) {
 #define AKV_TILES(R_, CP, THREADS)                                                                                              \
   do {                                                                                                                          \
     using Tile = SumTile<R_, CP, THREADS, HEAD_DECAY>;                                                                          \
@@ -650,7 +655,8 @@ int launch_state_walk(const float* prepared, const T* values, long value_stride,
       allowed = true;                                                                                                           \
     }                                                                                                                           \
     kernel<<<(units + kXcds - 1) / kXcds * kXcds, THREADS, Tile::kBytes, stream>>>(                                             \
-        prepared, values, value_stride, state, state_stride, q_start, seq_slots, raw, units, heads, groups, dim, vdim, ones);   \
+        prepared, values, value_stride, state, state_stride, q_start, seq_slots, raw, units, heads, groups, dim, vdim, ones,    \
+        least, most);                                                                                                           \
   } while (0)
     if (R == 64) AKV_TILES(64, 1, 256);
     else if (R == 32) AKV_TILES(32, 1, 256);
@@ -663,12 +669,14 @@ int launch_state_walk(const float* prepared, const T* values, long value_stride,
   const unsigned grid = static_cast<unsigned>(static_cast<long>(seqs) * heads * column_blocks);
 #define AKV_WALK(RP, R_)                                                                                                        \
   do {                                                                                                                          \
-    if (longest < 16)                                                                                                           \
+    if (longest < kTilesFrom)                                                                                                        \
       state_walk_kernel<T, RP, R_, 4, RULE, HEAD_DECAY><<<grid, 256, 0, stream>>>(                                              \
-          prepared, values, value_stride, state, state_stride, q_start, seq_slots, raw, heads, groups, dim, vdim, ones);        \
+          prepared, values, value_stride, state, state_stride, q_start, seq_slots, raw, heads, groups, dim, vdim, ones,        \
+          least, most);                                                                                                         \
     else                                                                                                                        \
       state_walk_kernel<T, RP, R_, 8, RULE, HEAD_DECAY><<<grid, 256, 0, stream>>>(                                           \
-          prepared, values, value_stride, state, state_stride, q_start, seq_slots, raw, heads, groups, dim, vdim, ones);        \
+          prepared, values, value_stride, state, state_stride, q_start, seq_slots, raw, heads, groups, dim, vdim, ones,        \
+          least, most);                                                                                                         \
   } while (0)
   if (rp == 32) AKV_WALK(32, 64);
   else if (rp == 16) AKV_WALK(16, 64);

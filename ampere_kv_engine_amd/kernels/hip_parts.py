@@ -601,8 +601,9 @@ class PartsKernels:
         self._step_arrays(ctx, tokens)
         lib = self._parts()
         longest = int(ctx.max_new_tokens) or tokens
+        walked_tokens, walked_forms = self._delta_forms(ctx, tokens, longest, dim)
         workspace = self._walk_workspace(int(lib.akv_delta_rule_workspace(tokens, ctx.num_seqs, heads, groups, dim, vdim,
-                                                                          1 if per_head else 0, longest)))
+                                                                          1 if per_head else 0, longest, walked_tokens)))
         self._check(lib.akv_delta_rule(
             _ptr(conv), _long(width), self._code_of(conv), _ptr_at(beta_logits, beta_at), _long(beta_logits.shape[1]),
             _ptr_at(decay_logits, decay_at), self._code_of(decay_logits), _long(decay_logits.shape[1]), _ptr(decay_bias),
@@ -610,8 +611,25 @@ class PartsKernels:
             self.GATE_ACTS[gate], _ptr(norm_weight), ctypes.c_float(unit_eps),
             ctypes.c_float(norm_eps), ctypes.c_float(q_scale), _ptr(state), _long(state.shape[1]), _ptr(ctx.q_start),
             _ptr(ctx.seq_slots), _ptr(workspace), _ptr(out), tokens, ctx.num_seqs, heads, groups, dim, vdim,
-            longest, self._stream()),
+            longest, walked_tokens, walked_forms, self._stream()),
             "delta_rule")
+
+    def _delta_forms(self, ctx, tokens: int, longest: int, dim: int) -> tuple[int, int]:
+        """Each request's form follows from its own tokens (`akv_delta_rule_forms`).  Of those that walk: the step's tokens up to
+        the end of the last of them, and which forms they take (1: small tiles, 2: large ones)."""
+        lines = self.__dict__.setdefault("_delta_lines", {})
+        if dim not in lines:
+            found = (ctypes.c_int * 2)()
+            self._parts().akv_delta_rule_forms(dim, found)
+            lines[dim] = tuple(found)
+        large, chunks = lines[dim]
+        if longest < large:
+            return tokens, 1
+        upto = forms = 0
+        for first, last in zip(ctx.host_q_start, ctx.host_q_start[1:]):
+            if last - first < chunks:
+                upto, forms = last, forms | (1 if last - first < large else 2)
+        return upto, forms
 
     def _state_of_slots(self, state, need: int, ctx) -> None:
         self._dense(state, "state", torch.float32)

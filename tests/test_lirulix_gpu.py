@@ -3,6 +3,7 @@ the engine with the HIP kernels through the cuttings of `lirulix_cases` - float3
 it is served."""
 
 import json
+import ctypes
 import math
 import os
 import random
@@ -358,36 +359,77 @@ def test_delta_rule_at_the_edges_of_its_fours(hip, dtype, sizes):
 
 def _delta_step(hip, counts, heads, groups, dim, vdim, per_head, state, inputs):
     conv, beta, decay_logits, decay_bias, rate, gates, weight = inputs
-    out = torch.empty(sum(counts), heads * vdim, device=DEVICE)
+    out = torch.empty(sum(counts), heads * vdim, dtype=conv.dtype, device=DEVICE)
     extra = dict(decay_at=0, gate_at=0, gate="sigmoid") if per_head else {}
     hip.delta_rule(conv, beta, 0, decay_logits, decay_bias, rate, gates, weight, 1e-6, 1e-5, dim ** -0.5, heads, groups, dim, vdim,
                    state, _ctx([0] * len(counts), counts), out, **extra)
     return out
 
 
-def _delta_inputs(tokens, heads, groups, dim, vdim, per_head):
+def _delta_inputs(tokens, heads, groups, dim, vdim, per_head, dtype=torch.float32):
     rand = lambda *shape: torch.randn(*shape).to(DEVICE)
-    decays = heads if per_head else heads * dim
-    return [rand(tokens, 2 * groups * dim + heads * vdim), rand(tokens, heads) * 2, rand(tokens, decays), rand(decays) * 0.5,
-            torch.exp(-4.0 + 4.0 * torch.rand(heads)).to(DEVICE), rand(tokens, heads * vdim), 1 + 0.2 * rand(vdim)]
+    decays, own = (heads, dtype) if per_head else (heads * dim, torch.float32)
+    return [rand(tokens, 2 * groups * dim + heads * vdim).to(dtype), (rand(tokens, heads) * 2).to(dtype), rand(tokens, decays).to(own),
+            rand(decays) * 0.5, torch.exp(-4.0 + 4.0 * torch.rand(heads)).to(DEVICE), rand(tokens, heads * vdim).to(own),
+            1 + 0.2 * rand(vdim)]
 
 
+def _chunks_from(hip, dim):
+    found = (ctypes.c_int * 2)()
+    hip._parts().akv_delta_rule_forms(dim, found)
+    return found[1]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("per_head", [False, True])
-@pytest.mark.parametrize("heads,groups,dim,vdim", [(2, 1, 64, 20), (2, 2, 128, 16), (1, 1, 192, 33), (3, 1, 256, 7)])
-def test_delta_rule_in_chunks_is_the_walk_token_by_token(hip, per_head, heads, groups, dim, vdim):
+@pytest.mark.parametrize("heads,groups,dim,vdim", [(2, 1, 64, 20), (2, 2, 128, 16), (1, 1, 192, 36), (4, 1, 256, 7)])
+def test_delta_rule_in_chunks_is_the_walk_token_by_token(hip, dtype, per_head, heads, groups, dim, vdim):
     """Requests of lengths around the chunks of 16 in one step, from a state that holds something: against the walk token by
-    token, which takes states whose stride is no multiple of four.  Both are float32 (2e-7 off 64 bits each): 1e-5 of the largest."""
+    token, which takes states whose stride is no multiple of four.  Both are float32 (2e-7 off 64 bits each): 1e-5 of the largest;
+    outputs in bfloat16 are rounded behind that, to neighbours at most.  Requests of fewer tokens than chunks are for walk either
+    way and have the same bits; the others have not (else nothing was compared)."""
     torch.manual_seed(dim + vdim)
-    counts = (1, 15, 16, 17, 47, 48, 49, 100)
-    inputs = _delta_inputs(sum(counts), heads, groups, dim, vdim, per_head)
+    least = _chunks_from(hip, dim)
+    whole = (least + 15) // 16 * 16
+    counts = (1, least, 15, whole, whole + 1, least - 1, whole + 15, 17, whole + 48)
+    inputs = _delta_inputs(sum(counts), heads, groups, dim, vdim, per_head, dtype)
     size = heads * dim * vdim
     begun = torch.randn(len(counts), size).to(DEVICE)
     apart = torch.zeros(len(counts), (size + 3) // 4 * 4 + 1, device=DEVICE)
     together = torch.zeros(len(counts), (size + 3) // 4 * 4, device=DEVICE)
     apart[:, :size], together[:, :size] = begun, begun
     want, got = (_delta_step(hip, counts, heads, groups, dim, vdim, per_head, state, inputs) for state in (apart, together))
-    assert (got - want).abs().max() < 1e-5 * want.abs().max()
+    near = 1e-5 if dtype == torch.float32 else 2.0 ** -7
+    assert (got.float() - want.float()).abs().max() < near * want.float().abs().max()
     assert (together[:, :size] - apart[:, :size]).abs().max() < 1e-5 * apart[:, :size].abs().max()
+    at = 0
+    for r, count in enumerate(counts):
+        same = torch.equal(together[r, :size], apart[r, :size])
+        assert same == (count < least), f"{count} tokens"
+        assert not same or torch.equal(got[at:at + count], want[at:at + count])
+        at += count
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("per_head", [False, True])
+@pytest.mark.parametrize("heads,groups,dim,vdim", [(2, 1, 64, 64), (2, 2, 128, 128), (1, 1, 256, 32), (3, 3, 40, 24)])
+def test_delta_rule_of_a_request_does_not_hang_on_its_neighbours(hip, dtype, per_head, heads, groups, dim, vdim):
+    """Single tokens, short portions and long ones in one step: each request's outputs and state have the bits that they have
+    where the request is alone, whichever forms the others take."""
+    torch.manual_seed(dim)
+    least = min(_chunks_from(hip, dim), 128)
+    counts = (1, 1, 7, least, 20, 200, least - 1, 1)
+    inputs = _delta_inputs(sum(counts), heads, groups, dim, vdim, per_head, dtype)
+    begun = torch.randn(len(counts), heads * dim * vdim).to(DEVICE)
+    states = begun.clone()
+    together = _delta_step(hip, counts, heads, groups, dim, vdim, per_head, states, inputs)
+    at = 0
+    for r, count in enumerate(counts):
+        alone = begun[r:r + 1].clone()
+        rows = [x[at:at + count].contiguous() if x.dim() == 2 else x for x in inputs]
+        out = _delta_step(hip, (count,), heads, groups, dim, vdim, per_head, alone, rows)
+        assert torch.equal(out, together[at:at + count]) and torch.equal(alone[0], states[r]), f"request {r} of {count} tokens"
+        at += count
 
 
 @pytest.mark.parametrize("where", ["value", "infinite value", "key", "query", "beta", "decay"])
@@ -395,8 +437,9 @@ def test_delta_rule_in_chunks_keeps_what_is_not_finite_from_earlier_tokens(hip, 
     """One element of token 37 that is no number (or infinite): outputs before it are as the walk token by token leaves them, and
     those that are no numbers are the same."""
     torch.manual_seed(5)
-    heads, dim, vdim, counts, at = 2, 64, 32, (60,), 37
-    inputs = _delta_inputs(60, heads, heads, dim, vdim, False)
+    heads, dim, vdim, counts, at = 2, 64, 32, (90,), 37
+    assert counts[0] >= _chunks_from(hip, dim)
+    inputs = _delta_inputs(90, heads, heads, dim, vdim, False)
     conv, beta, decay = inputs[:3]
     bad = float("inf") if where == "infinite value" else float("nan")
     if where.endswith("value"):
