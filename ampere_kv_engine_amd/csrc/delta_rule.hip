@@ -139,7 +139,7 @@ inline long chunk_slots(int tokens, int seqs) { return tokens / kChunk + static_
 __host__ __device__ inline long chunk_floats(int dim) { return 3L * kChunk * dim + dim + 2L * kChunk * kChunk; }
 // The fewest tokens of a request that goes in chunks.  Which form a request takes hangs on its own tokens and the head's size
 // alone, so that its bits do not change with what else is in the step (fewer than kTilesFrom walk in small tiles, others in
-// large ones: a step of all three kinds has three launches).  32 single tokens beside 171, 16 heads of 128 x 128: 94 us, where
+// large ones: a step of all three kinds has three launches).  32 single tokens beside 171, 16 heads of 128 x 128: 60 us, where
 // the single ones went in chunks too 113, where all walked in large tiles 162.  The lines lie
 // where one request alone breaks even; batches would from fewer on.  Whole rule, walk / chunks us, decays per channel: 16 heads of 64
 // x 64 64 tokens 14.9 / 15.5, 80 18.1 / 16.1; 16 heads of 128 x 128 96 tokens 21.6 / 24.2, 128 25.8 / 25.9, 160 30.4 / 28.4 (four
@@ -300,13 +300,12 @@ template <typename T, int TILES>
 __global__ __launch_bounds__(512) void delta_chunk_walk_kernel(const float* chunks, const T* token_values,
                                                                long value_stride, float* __restrict__ state, long state_stride,
                                                                const int* __restrict__ q_start, const int* __restrict__ seq_slots,
-                                                               float* __restrict__ raw_out, int units, int heads, int vdim) {
+                                                               float* __restrict__ raw_out, int seqs, int heads, int vdim) {
   constexpr int dim = 64 * TILES;
   __shared__ __align__(16) float w_parts[2][4 * 256], o_parts[2][4 * 256], s_parts[2][4 * TILES * 256], u_whole[2][256], x_whole[2][256];
-  const int unit = static_cast<int>(blockIdx.x % kXcds * (gridDim.x / kXcds) + blockIdx.x / kXcds);
-  if (unit >= units) return;
-  const int column_blocks = (vdim + 15) / 16;
-  const int r = unit / (heads * column_blocks), h = unit / column_blocks % heads, col0 = unit % column_blocks * 16;
+  const WalkUnit unit = walk_unit(seqs, heads, (vdim + 15) / 16);
+  if (unit.request >= seqs) return;
+  const int r = unit.request, h = unit.head, col0 = unit.column_block * 16;
   const int first = q_start[r], last = q_start[r + 1];
   if (last - first < chunks_from(dim)) return;             // (it walks)
   const int tid = threadIdx.x & 255, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = lane >> 4;
@@ -520,9 +519,8 @@ void launch_chunks(const T* conv, long conv_stride, const T* beta_logits, long b
   delta_chunks_kernel<T, TD, HEAD_DECAY, TILES><<<dim3(static_cast<unsigned>(chunk_slots(tokens, seqs)), heads), 256, 0, stream>>>(
       conv, conv_stride, beta_logits, beta_stride, decay_logits, decay_stride, decay_bias, rate, unit_eps, q_scale, q_start, seqs,
       chunks, heads, groups);
-  const int units = seqs * heads * ((vdim + 15) / 16);
-  delta_chunk_walk_kernel<T, TILES><<<(units + kXcds - 1) / kXcds * kXcds, 512, 0, stream>>>(
-      chunks, conv + 2L * groups * 64 * TILES, conv_stride, state, state_stride, q_start, seq_slots, raw, units, heads, vdim);
+  delta_chunk_walk_kernel<T, TILES><<<walk_grid(seqs, heads, (vdim + 15) / 16), 512, 0, stream>>>(
+      chunks, conv + 2L * groups * 64 * TILES, conv_stride, state, state_stride, q_start, seq_slots, raw, seqs, heads, vdim);
 }
 
 // Unit vectors, decays, betas and k . q of the first `tokens` tokens.
