@@ -9,6 +9,7 @@ from dataclasses import dataclass
 from ..cache.manager import CacheManager
 from ..config.engine import EngineConfig
 from ..config.specs import ModelSpec
+from ..kernels import walk_room
 from ..weights.spec import MATRIX
 from .dry import dry_runtime
 from .model import Model
@@ -56,6 +57,7 @@ def plan_memory(spec: ModelSpec, engine_config: EngineConfig, memory_bytes: int)
              + engine_config.max_batched_tokens * widest * element * 18               # activations of a step, two arenas
              + 2 * largest                                                            # a matrix in flight while it is packed
              + partial_sum_bytes(model, engine_config)
+             + walk_bytes(model, engine_config)
              + model.rt.shared_bytes()                                                # position tables, one per kind and size
              + (512 << 20))                                                           # timing spacer, library workspaces
     left = memory_bytes - weight_bytes - second - fixed
@@ -70,6 +72,11 @@ def plan_memory(spec: ModelSpec, engine_config: EngineConfig, memory_bytes: int)
 def partial_sum_bytes(model: Model, engine_config: EngineConfig) -> int:
     """Partial results of attention whose keys are cut over blocks: they lie in a layer's arena, and a step has two arenas."""
     return 2 * max((block.mixer.partial_sum_bytes(engine_config) for block in model.blocks), default=0)
+
+
+def walk_bytes(model: Model, engine_config: EngineConfig) -> int:
+    """The buffer of matrix states that walk over a step's tokens, which all layers share, and what it outgrew."""
+    return walk_room.held_bytes(max((block.mixer.walk_floats(engine_config) for block in model.blocks), default=0))
 
 
 def page_bytes(spec: ModelSpec, dtype: str, page_size: int) -> int:

@@ -10,7 +10,7 @@ import ctypes
 import torch
 
 from ..csrc.build import ensure_parts
-from . import partial_sums
+from . import partial_sums, walk_room
 
 _DTYPE_CODE = {torch.float32: 0, torch.bfloat16: 1}
 
@@ -645,7 +645,7 @@ class PartsKernels:
             if torch.cuda.is_current_stream_capturing():
                 self._refuse("a recorded step needs more room for a recurrence's tokens than the steps before it")
             self.__dict__.setdefault("_walk_outgrown", []).append(held)
-            held = self.__dict__["_walk_buffer"] = torch.empty(max(need, 1 << 22), dtype=torch.float32, device=self.device)
+            held = self.__dict__["_walk_buffer"] = torch.empty(walk_room.room(need), dtype=torch.float32, device=self.device)
         return held
 
     # ---- time mixing -----------------------------------------------------------------------------------------------------

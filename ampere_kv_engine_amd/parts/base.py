@@ -184,6 +184,10 @@ class Part:
         their size grows with the requests' lengths (what the memory plan counts beside the activations)."""
         return 0
 
+    def walk_floats(self, engine_config) -> int:
+        """(mixers whose matrix state walks over the tokens) The floats a step needs at most in the kernel set's buffer for it."""
+        return 0
+
 
 class SharesProducts:
     """A mixer whose first step is one product over the layer's input (`inputs`, a `Linear` whose names are relative to

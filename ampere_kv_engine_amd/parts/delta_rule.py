@@ -21,6 +21,7 @@ from __future__ import annotations
 
 import torch
 
+from ..kernels import walk_room
 from ..weights.spec import BIAS, MATRIX, NORM, TensorSpec
 from .base import Part, SlotState, register_part
 from .linear import Linear
@@ -89,6 +90,10 @@ class GatedDeltaRule(Part):
 
     def weight_bytes(self):
         return sum(linear.weight_bytes() for linear in (self.into, *self.ups, self.out))
+
+    def walk_floats(self, engine_config):
+        return walk_room.delta_rule_floats(engine_config.max_batched_tokens, engine_config.max_seqs, self.heads, self.kv_heads,
+                                           self.dim, self.vdim, self.per_head)
 
     def cache_request(self):
         return SlotState((self.heads * self.dim * self.vdim + (self.taps - 1) * self.conv_channels,), torch.float32)

@@ -16,6 +16,7 @@ from __future__ import annotations
 
 import torch
 
+from ..kernels import walk_room
 from ..weights.spec import BIAS, NORM, TensorSpec
 from .base import Part, SlotState, register_part
 from .linear import Linear
@@ -61,6 +62,9 @@ class MatrixMemory(Part):
 
     def weight_bytes(self):
         return self.into.weight_bytes() + self.out.weight_bytes()
+
+    def walk_floats(self, engine_config):
+        return walk_room.matrix_memory_floats(engine_config.max_batched_tokens, self.heads, self.dim, self.vdim)
 
     def cache_request(self):
         return SlotState((self.state_size,), torch.float32)

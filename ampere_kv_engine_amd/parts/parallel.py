@@ -77,6 +77,9 @@ class ParallelMixers(Part):
     def partial_sum_bytes(self, engine_config):
         return sum(mixer.partial_sum_bytes(engine_config) for mixer in self.mixers)
 
+    def walk_floats(self, engine_config):
+        return max(mixer.walk_floats(engine_config) for mixer in self.mixers)      # (one after the other, in one buffer)
+
     def weight_bytes(self):
         if self.shared:
             return self.inputs.weight_bytes() + self.outputs.weight_bytes()

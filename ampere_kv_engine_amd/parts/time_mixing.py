@@ -16,6 +16,7 @@ from __future__ import annotations
 import torch
 
 from ..weights.random import register_init_law
+from ..kernels import walk_room
 from ..weights.spec import BIAS, NORM, TensorSpec
 from .base import Part, SlotState, register_part
 from .linear import Linear
@@ -68,6 +69,9 @@ class TimeMixing(Part):
 
     def weight_bytes(self):
         return sum(linear.weight_bytes() for linear in self._linears())
+
+    def walk_floats(self, engine_config):
+        return walk_room.time_mixing_floats(engine_config.max_batched_tokens, self.heads, self.dim)
 
     def cache_request(self):
         return SlotState((self.state_size + self.hidden,), torch.float32)

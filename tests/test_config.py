@@ -229,6 +229,64 @@ def test_launches_of_tiles_hold_whole_tiles(share):
         assert (token, tile) == (150, len(tiles))
 
 
+def test_the_room_of_walked_states_covers_what_the_kernels_ask_for():
+    """The memory plan's counts of floats against the kernel library's, over sizes, mixes of forms and of requests."""
+    import ctypes
+    import random
+    from ampere_kv_engine_amd.csrc.build import parts_library_path
+    from ampere_kv_engine_amd.kernels import walk_room
+    path = parts_library_path()
+    if path is None:
+        pytest.skip("the kernel library is not built")
+    lib = ctypes.CDLL(path)
+    asks = [getattr(lib, f"akv_{name}_workspace") for name in ("delta_rule", "time_mixing", "matrix_memory")]
+    for ask in asks:
+        ask.restype = ctypes.c_long
+    rng = random.Random(3)
+    for _ in range(300):
+        groups, dim, vdim = rng.choice((1, 2, 16)), rng.choice((24, 64, 128, 192, 256, 300)), rng.choice((16, 36, 128))
+        heads, per_head, tokens, seqs = groups * rng.choice((1, 3, 16)), rng.random() < 0.5, rng.randrange(1, 5000), rng.randrange(1, 65)
+        longest, walked = rng.randrange(1, tokens + 1), rng.randrange(0, tokens + 1)
+        need = asks[0](tokens, seqs, heads, groups, dim, vdim, int(per_head), longest, walked)
+        assert need <= walk_room.delta_rule_floats(tokens, seqs, heads, groups, dim, vdim, per_head)
+        assert asks[1](tokens, heads, dim) <= walk_room.time_mixing_floats(tokens, heads, dim)
+        assert asks[2](tokens, heads, dim, vdim) <= walk_room.matrix_memory_floats(tokens, heads, dim, vdim)
+
+
+def test_the_room_of_walked_states_is_bounded_and_in_the_memory_plan(monkeypatch):
+    """Steps that grow token by token: what is held - the buffer and what it outgrew - stays within the plan's count."""
+    from types import SimpleNamespace
+    import torch
+    from ampere_kv_engine_amd.config import EngineConfig
+    from ampere_kv_engine_amd.config.lirulix import LirulixConfig
+    from ampere_kv_engine_amd.engine import plan_memory
+    from ampere_kv_engine_amd.engine.dry import dry_runtime
+    from ampere_kv_engine_amd.engine.model import Model
+    from ampere_kv_engine_amd.engine.sizing import walk_bytes
+    from ampere_kv_engine_amd.kernels import walk_room
+    from ampere_kv_engine_amd.kernels.hip_parts import PartsKernels
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    kernels = SimpleNamespace(device="meta")
+    sizes = (16, 1, 128, 128)                       # one key head for 16 heads: what the chunks hold is most beside the rows
+    for tokens in range(1, 2049):
+        PartsKernels._walk_workspace(kernels, walk_room.delta_rule_floats(tokens, 8, *sizes, False))
+    held = 4 * sum(b.numel() for b in [kernels._walk_buffer, *kernels._walk_outgrown] if b is not None)
+    assert held <= walk_room.held_bytes(walk_room.delta_rule_floats(2048, 8, *sizes, False)) <= 1 << 28
+    raw = dict(architecture="Lirulix", vocab=256, width=64, norm=dict(eps=1e-6), loop=dict(start=0, stop=2, times=1), layers=[
+        dict(type="channel_delta", mixer=dict(heads=16, kv_heads=1, dim=128, vdim=128, conv=4, ranks=dict(decay=8, gate=8)),
+             mlp=dict(kind="dense", ff=64)),
+        dict(type="attention", mixer=dict(heads=4, kv_heads=2, dim=32, vdim=32, scale=0.2, rot=dict(
+            dims=16, base=1e4, scaling=dict(factor=4.0, original=64, fast=32.0, slow=1.0))), mlp=dict(kind="dense", ff=64))])
+    spec = LirulixConfig.from_dict(raw).to_model_spec()
+    config = EngineConfig(page_size=16, max_seqs=8, max_seq_len=4096, max_batched_tokens=2048, num_pages=8)
+    assert walk_bytes(Model(spec, dry_runtime(4096, 16)), config) >= held
+    small = EngineConfig(page_size=16, max_seqs=8, max_seq_len=4096, max_batched_tokens=64, num_pages=8)
+    plans = [plan_memory(spec, c, 1 << 33) for c in (config, small)]
+    assert plans[0].fixed_bytes - plans[1].fixed_bytes > held - walk_room.held_bytes(1)
+    qwen3 = Model(Qwen3Config.from_dict(TINY_A).to_model_spec(), dry_runtime(8192, 16))
+    assert walk_bytes(qwen3, config) == 0
+
+
 def test_plan_memory_counts_the_partial_sums_of_cut_attention():
     """Once per arena, by the mixer with the largest; none where every key a token sees lies in one segment, nor for float32's gated
     attention, which is one kernel, or bfloat16's plain one, whose cut is sized by the device."""
