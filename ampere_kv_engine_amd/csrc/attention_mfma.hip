@@ -268,7 +268,8 @@ struct Where {
 // item's steps of 32 keys, and what the four have - maximum, sum and weighted sum per column - is merged through LDS into the
 // item's one partial result.  A wave's steps follow each other at the latency of a page's lookup and its keys, so a short
 // context's 128 keys cost one such step instead of four, and a long one's segments leave a quarter of the partial results to
-// the merge.  (A step of one request of 210 keys, 8 layers of 16 / 4 heads: 380 -> 365 us.)
+// the merge.  (A step of one request of 210 keys, 8 layers of 16 / 4 heads: 380 -> 365 us.)  Without a plan - no request has more
+// keys than a segment holds at least - a request is one item, whose result is the output: what the merge would make of it.
 constexpr int kItemWaves = 4;
 struct ItemLds {
   float parts[kItemWaves][16][PSTRIDE];
@@ -276,7 +277,7 @@ struct ItemLds {
 
 template <int NQ, bool SPLIT, bool PIPE, bool FRESH, bool ONCE, bool ITEMS>
 __device__ __forceinline__ void attention_mfma_body(const Args& a, const Where at, ItemLds* item_lds) {
-  static_assert(!ITEMS || (SPLIT && NQ == 1), "items are single tokens cut by a plan");
+  static_assert(!ITEMS || (SPLIT && NQ == 1), "items are single tokens");
   const int lane = at.lane, r16 = lane & 15, g = lane >> 4;
   auto from_pages = [](const char* at) {
     const uintx4* p = reinterpret_cast<const uintx4*>(at);
@@ -293,10 +294,16 @@ __device__ __forceinline__ void attention_mfma_body(const Args& a, const Where a
   Tile t{};
   int seg_lo = 0, seg_hi = 0x7fffffff;     // SPLIT: the keys of this block's segment
   long part = 0;                           // SPLIT: index of its partial result's tile
-  if (SPLIT && a.plan != nullptr) {        // item `by` of the plan: a request and a segment of its keys
+  if (SPLIT && (ITEMS || a.plan != nullptr)) {   // item `by` of the plan: a request and a segment of its keys
     const int item = at.by;
-    if (item >= a.plan[0]) return;
-    const int4 record = *reinterpret_cast<const int4*>(a.plan + 132 + 4 * item);
+    int4 record;
+    if (ITEMS && a.plan == nullptr) {      // request `by`, all of its keys
+      const int pos = a.seq_lens[a.seq_first + item] - 1;
+      record = make_int4(item, a.window > 0 ? max(0, pos - a.window + 1) & ~31 : 0, pos, pos);
+    } else {
+      if (item >= a.plan[0]) return;
+      record = *reinterpret_cast<const int4*>(a.plan + 132 + 4 * item);
+    }
     t.request = a.seq_first + record.x;
     t.first_row = a.q_start[a.seq_first] + record.x;   // one row per request
     t.tokens = 1;
@@ -319,7 +326,7 @@ __device__ __forceinline__ void attention_mfma_body(const Args& a, const Where a
       part = (static_cast<long>(at.bx) * at.gy + at.by) * a.num_splits + at.bz;
     }
   }
-  const int head_block = (SPLIT && a.plan != nullptr) ? at.bx : at.by;  // (kv head, group of its query heads)
+  const int head_block = (SPLIT && (ITEMS || a.plan != nullptr)) ? at.bx : at.by;  // (kv head, group of its query heads)
   const int kvh = head_block / a.head_groups, hg = head_block % a.head_groups;
   const uintx4 zero = uintx4{0u, 0u, 0u, 0u};
   const int page_size = 1 << a.page_shift, page_mask = page_size - 1;
@@ -711,6 +718,13 @@ __device__ __forceinline__ void attention_mfma_body(const Args& a, const Where a
         all += *reinterpret_cast<const floatx4*>(&item_lds->parts[w][c][d]) * by;
         sum = fmaf(by, item_lds->parts[w][c][D + 1], sum);
       }
+      if (a.plan == nullptr) {
+        bf16_t* out = a.out + (static_cast<long>(t.first_row) * a.q_heads + kvh * a.group + hg * a.heads_per_tile + c) * D + d;
+        const float inv = bad ? nan : 1.f / sum;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) out[i] = from_float<bf16_t>(all[i] * inv);
+        continue;
+      }
       float* dst = a.partial + (part * 16 + c) * PSTRIDE;
       *reinterpret_cast<floatx4*>(dst + d) = all;
       if (d == 0) {
@@ -729,7 +743,7 @@ __global__ __launch_bounds__(64, (SPLIT && NQ == 1 && D <= 128) ? 2 : 1) void at
                static_cast<int>(gridDim.x), static_cast<int>(gridDim.y), static_cast<int>(threadIdx.x), 0}, nullptr);
 }
 
-// Items of a plan: block (head block, item).
+// Items of a plan, or requests: block (head block, item).
 template <bool FRESH, bool ONCE>
 __global__ __launch_bounds__(64 * kItemWaves, D <= 128 ? 2 : 1) void attention_items_kernel(const Args a) {
   __shared__ __align__(16) ItemLds lds;
@@ -1740,8 +1754,9 @@ int launch(const Args& a, int tiles, bool shared, int waves_per_item, hipStream_
     }
     return AKV_LAUNCH_STATUS();
   }
-  const bool items = a.plan != nullptr;  // single tokens whose keys were cut on the device: always with the merge
-  if (items) grid = dim3(a.kv_heads * a.head_groups, a.items_grid, 1);
+  const bool whole = a.plan == nullptr && waves_per_item == kItemWaves;   // single tokens, a request an item: without merge
+  const bool items = a.plan != nullptr || whole;  // single tokens whose keys were cut on the device: with the merge
+  if (items) grid = dim3(a.kv_heads * a.head_groups, whole ? a.seq_count : a.items_grid, 1);
   const int columns = a.heads_per_tile * (a.single_tokens ? 1 : a.tokens_per_tile);   // that can be a (token, head) pair
   const dim3 merge_grid(items ? a.seq_count : tiles, a.kv_heads * a.head_groups, columns);
   auto merge = [&]() { attention_merge_kernel<NQ><<<merge_grid, 64 * kMergeWaves, 0, stream>>>(a); };
@@ -1755,7 +1770,7 @@ int launch(const Args& a, int tiles, bool shared, int waves_per_item, hipStream_
       if (items && waves_per_item == kItemWaves) {
         if (once) attention_items_kernel<true, true><<<grid, 64 * kItemWaves, 0, stream>>>(a);
         else attention_items_kernel<true, false><<<grid, 64 * kItemWaves, 0, stream>>>(a);
-        merge();
+        if (!whole) merge();
       } else if (items || a.num_splits > 1) {
         if (once) attention_mfma_kernel<NQ, true, true, true, true><<<grid, 64, 0, stream>>>(a);
         else attention_mfma_kernel<NQ, true, true, true, false><<<grid, 64, 0, stream>>>(a);
@@ -1772,7 +1787,7 @@ int launch(const Args& a, int tiles, bool shared, int waves_per_item, hipStream_
     if constexpr (NQ == 1) {
       if (once) attention_items_kernel<false, true><<<grid, 64 * kItemWaves, 0, stream>>>(a);
       else attention_items_kernel<false, false><<<grid, 64 * kItemWaves, 0, stream>>>(a);
-      merge();
+      if (!whole) merge();
     } else {
       return -2;
     }
@@ -1870,7 +1885,8 @@ int units_of_device() {
 // `plan` (not null: single tokens, at most 64 requests): seg_keys and num_splits are not used; the requests' keys were
 // cut into items by akv_decode_plan with the same seq_first, seq_count and window; `items_grid` is the bound given
 // there, and `partial` must hold items_grid * kv_heads * head_groups * 16 * nq * (D + 4) floats.  `waves_per_item`: 1, or 4
-// that share an item (the plan was then made with `share`).
+// that share an item (the plan was then made with `share`); 4 without a plan (single tokens): four waves take all of a
+// request's keys, and there are no partial results.
 // `qkv` (not null: single tokens, nq 1, head sizes that are multiples of 64): the tokens' stacked raw projections
 // [tokens, (q_heads + 2 * kv_heads) * D]; `q` is not read, the kernel norms (q_weight, k_weight, eps; both weights
 // null: no norm) and rotates (rope_table [table_positions, D / 2, 2], null: no rotation) queries and the new keys
@@ -1887,7 +1903,10 @@ extern "C" int AKV_CONCAT(akv_attention_mfma_d, AKV_HEAD_DIM)(
   if (heads_per_tile * tokens_per_tile > 16 * nq || kv_heads * head_groups > 65535 || num_splits > 65535 ||
       num_splits < 1 || (single_tokens && tiles != seq_count) || (shared && (page_size < 8 || num_splits != 1)) ||
       (qkv != nullptr && (shared || !single_tokens || nq != 1 || D % 64 != 0 || (q_weight == nullptr) != (k_weight == nullptr))) ||
-      (plan != nullptr && (shared || nq != 1 || (waves_per_item != 1 && waves_per_item != kItemWaves) || !single_tokens || seq_count > 64 || items_grid < 1 || items_grid > 65535)))
+      (waves_per_item != 1 && waves_per_item != kItemWaves) ||
+      ((plan != nullptr || waves_per_item == kItemWaves) && (shared || nq != 1 || !single_tokens || seq_count > 64)) ||
+      (plan != nullptr && (items_grid < 1 || items_grid > 65535)) ||
+      (plan == nullptr && waves_per_item == kItemWaves && num_splits != 1))
     return -2;
   Args a;
   const int status = common_args(a, q, k_pages, v_pages, out, q_start, seq_lens, block_table, table_rows, table_width,

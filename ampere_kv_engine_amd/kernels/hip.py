@@ -1008,9 +1008,9 @@ class HipKernels(PartsKernels, KernelSet):
         # (a step that feeds portions too has its single tokens' segments taken by waves alone, in one launch with the portions
         # or in two: which one hangs on bounds that are not the same recorded and not)
         shared_items = by_plan and ctx.num_seqs == ctx.num_decode_seqs and self._share_segments(seq_count, kv_heads * head_groups)
-        if shared_items or (by_plan and max(ctx.host_seq_lens[seq_first:seq_first + seq_count]) > self.decode_min_segment):
+        if by_plan and max(ctx.host_seq_lens[seq_first:seq_first + seq_count]) > self.decode_min_segment:
             # single tokens: their keys are cut on the device, from the lengths there (requests of 128 keys or fewer are not
-            # cut: where a wave alone takes a segment, the kernel without merge then gives the same bits)
+            # cut: the kernels without plan and merge then give the same bits)
             plan, items_grid = self._decode_plan(ctx, seq_first, seq_count, window, kv_heads * head_groups, share=shared_items)
             partial = take(items_grid * kv_heads * head_groups * 16 * nq * (head_dim + 4))
         elif split:
@@ -1041,18 +1041,20 @@ class HipKernels(PartsKernels, KernelSet):
         """Whether four waves share a segment of a single token's keys (`attention_items_kernel`) rather than a wave alone
         take it.  Shared segments end a short context's chain of steps sooner and leave a quarter of the partial results, but
         there are at most two rounds of blocks for the device to even out: with up to 32 (request, head block) pairs a
-        request has 16 segments or more and their last pieces do not count.  It hangs on the number of requests only, so
-        that a recorded step and the same step run eagerly are cut alike; short contexts, too, come by a plan then.  Whole steps, alone / shared us: one request of
-        2,048 keys 941 / 928 (8 layers of the 8B sizes), of 16,000 1,017 / 985, four of 64 to 16,000 1,069 / 1,061; 8 heads and
-        8 requests of 64 to 12,000 1,115 / 1,141, 27 of 64 to 16,000 1,657 / 1,691 (6 layers of 14B)."""
+        request has 16 segments on average - fewer of short or uneven contexts -, and their last pieces count little.  That is
+        where the line was measured; it hangs on the number of requests only, so that a recorded step and the same step run
+        eagerly are cut alike.  Whole steps, alone / shared us: one request of 2,048 keys 941 / 928 (8 layers of the 8B sizes), of
+        16,000 1,017 / 985, four of 64 to 16,000 1,069 / 1,061; 8 heads and 8 requests of 64 to 12,000 1,115 / 1,141, 27 of 64 to
+        16,000 1,657 / 1,691 (6 layers of 14B)."""
         return seq_count * head_blocks <= 32
 
     def _decode_plan(self, ctx, seq_first, seq_count, window, head_blocks, waves=None, share=False):
         """The cut of the keys of requests seq_first .. + seq_count - 1 (single tokens) into (request, segment) items:
         segments of one size for all requests - about `decode_wave_target` waves in all, no segment shorter than
         `decode_min_segment` unless it is a request's only one - worked out by a one-wave kernel from the lengths on
-        the device.  With `share` four waves work on a segment: a quarter as many are wanted.  The cut depends on the lengths alone, so the layers of a step share one plan: it is
-        remembered on the step's context.  Returns the plan and the bound on the number of items that sizes grids and buffers."""
+        the device.  With `share` four waves work on a segment: a quarter as many are wanted.  The cut depends on the lengths
+        alone, so the layers of a step share one plan: it is remembered on the step's context.  Returns the plan and the bound on
+        the number of items that sizes grids and buffers."""
         items = max(1, (waves if waves is not None else self.decode_wave_target) // head_blocks)
         key = (seq_first, seq_count, int(window) if window is not None else 0, items, self.decode_min_segment, share)
         plans = getattr(ctx, "decode_plans", None)

@@ -1596,6 +1596,32 @@ def test_single_tokens_whose_items_are_shared_by_four_waves(hip, ref, monkeypatc
         torch.testing.assert_close(got.cpu().float(), want.float(), **attention_tol(torch.bfloat16))
 
 
+@pytest.mark.parametrize("q_heads,kv_heads,dim,page_size", [(8, 2, 128, 16), (16, 4, 64, 32), (3, 1, 256, 32), (40, 2, 64, 8), (6, 1, 32, 4), (5, 5, 80, 16)])
+@pytest.mark.parametrize("window", [None, 1, 100])
+@pytest.mark.parametrize("histories", [[0], [127], [0, 31, 32, 126], [64, 100, 5]])
+def test_single_tokens_of_few_short_requests_need_no_plan_and_no_merge(hip, ref, monkeypatch, q_heads, kv_heads, dim, page_size, window, histories):
+    """Contexts of up to 128 keys: one kernel, with the bits of the plan and the merge that a recorded step goes by, whose bound on
+    the lengths is larger."""
+    portions = [(h, 1) for h in histories]
+    q, k_pages, v_pages, ctx, meta, _, _ = _attention_case(torch.bfloat16, q_heads, kv_heads, dim, page_size, portions, window, 64)
+    ctx.num_decode_seqs = len(portions)
+    want = torch.empty_like(q)
+    ref.attention(q, k_pages, v_pages, ctx, meta, q_heads, kv_heads, dim, dim ** -0.5, window, want)
+    plans, make = [], hip._decode_plan
+    monkeypatch.setattr(hip, "_decode_plan", lambda *a, **k: plans.append(1) or make(*a, **k))
+    results = []
+    for bound in (None, 256):
+        cctx, cmeta = _to_cuda(ctx, meta)
+        if bound is not None:
+            cctx.host_seq_lens = [bound] * len(portions)
+        got = torch.full_like(q, float("nan"), device="cuda")
+        hip.attention(q.cuda(), k_pages.cuda(), v_pages.cuda(), cctx, cmeta, q_heads, kv_heads, dim, dim ** -0.5, window, got)
+        assert len(plans) == (0 if bound is None else 1)
+        torch.testing.assert_close(got.cpu().float(), want.float(), **attention_tol(torch.bfloat16))
+        results.append(got)
+    assert torch.equal(*results)
+
+
 def test_attention_of_many_single_tokens_of_very_different_lengths(hip, ref):
     """70 requests in one step (two launches of at most 64), one of them a hundred times longer than most: every
     request's keys are cut into segments of the same size."""
