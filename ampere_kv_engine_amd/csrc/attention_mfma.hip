@@ -1358,8 +1358,11 @@ __device__ __forceinline__ void attention_prompt_body(const Args& a, const int b
   // as text because the compiler, which does not see that rings keep such loads and the reads of LDS apart, waits for all
   // of them before every read; the turns' own counted waits are what orders them.  Nothing is loaded into registers.
   auto into_lds = [&](const char* from, uint32_t offset, uint32_t to) {
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"   // (the allocator never hands m0 out: the passes that merge its settings read this)
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
                  :: "s"(to), "v"(offset), "s"(from) : "m0");
+#pragma clang diagnostic pop
   };
   const uint32_t k_base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_rows)(&k_lds[wave * 512])));
   const uint32_t v_base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_rows)(&v_lds[wave * 512])));
@@ -1468,23 +1471,39 @@ __device__ __forceinline__ void attention_prompt_body(const Args& a, const int b
         o[dt] = mfma32(values, lo[half], mfma32(values, hi[half], o[dt]));
       }
   };
-  // the same for the steps that hold the first and the last key: slots outside hold anything, NaN included (never written, or
-  // of a page that stands in for one that a window has passed)
-  auto gather_edge = [&](int step, int buffer, const uintx4 (&hi)[2], const uintx4 (&lo)[2]) {
+  // The same for steps that some column does not see whole.  Slots outside the block's keys hold anything, NaN included (never
+  // written, or of a page that stands in for one that a window has passed): blanked.  And a hidden key's weight of zero times an
+  // infinite value is not zero: a step that holds values that are not finite is left out and noted; after the turns its values
+  // are added one by one to the columns that see their keys.  (Such steps lie within three of the wave's first or last.)
+  uint32_t left_first = 0u, left_last = 0u;   // steps left out: counted from the wave's first, or back from its last
+  auto gather_partly = [&](int step, int buffer, const uintx4 (&hi)[2], const uintx4 (&lo)[2]) {
     const uint32_t keys = static_cast<uint32_t>(range_hi - range_lo);
+    uintx4 keep[2];
+    uint32_t carries = 0u;     // (an exponent of all ones carries into the sign's place)
 #pragma unroll
     for (int half = 0; half < 2; ++half) {
       const int key = first_base + step * 32 + half * 16 + h * 8 - range_lo;
-      uintx4 keep;
 #pragma unroll
       for (int w = 0; w < 4; ++w)
-        keep[w] = (static_cast<uint32_t>(key + 2 * w) <= keys ? 0xffffu : 0u) | (static_cast<uint32_t>(key + 2 * w + 1) <= keys ? 0xffff0000u : 0u);
+        keep[half][w] = (static_cast<uint32_t>(key + 2 * w) <= keys ? 0xffffu : 0u) | (static_cast<uint32_t>(key + 2 * w + 1) <= keys ? 0xffff0000u : 0u);
 #pragma unroll
       for (int dt = 0; dt < OT; ++dt) {
-        const uintx4 values = value_piece(buffer, half, dt) & keep;
-        o[dt] = mfma32(values, lo[half], mfma32(values, hi[half], o[dt]));
+        const uintx4 c = (value_piece(buffer, half, dt) & keep[half] & 0x7fff7fffu) + 0x00800080u;
+        carries |= (c[0] | c[1]) | (c[2] | c[3]);
       }
     }
+    if (__any((carries & 0x80008000u) != 0u)) {
+      if (step - wave_from < 32) left_first |= 1u << (step - wave_from);
+      else left_last |= 1u << ((wave_to - 1 - step) & 31);
+      return;
+    }
+#pragma unroll
+    for (int half = 0; half < 2; ++half)
+#pragma unroll
+      for (int dt = 0; dt < OT; ++dt) {
+        const uintx4 values = value_piece(buffer, half, dt) & keep[half];
+        o[dt] = mfma32(values, lo[half], mfma32(values, hi[half], o[dt]));
+      }
   };
 
   // ---- the turns: scores of step j, weights of step j - 1, sums of step j - 2; the keys of step j + 3 and the values of
@@ -1499,11 +1518,15 @@ __device__ __forceinline__ void attention_prompt_body(const Args& a, const int b
   for (int i = 0; i < SP; ++i) at[2][i] = at[3][i] = 0;   // (steps -2 and -1 do not exist: what their loads bring is not read)
 #pragma unroll
   for (int v = 1; v < 4; ++v) lookup(v - 1, pending[v]);
-  // The queries' loads end here, beside the first lookups.  Registers that a loop carries and whose loads may still be on their way
-  // when it is entered are waited for inside it, and the compiler does not count the loads into LDS, which are younger: the first
-  // of four calm turns then waited for all but three of these (heads of 128), or for all (of 64).
+  // The queries' loads end here, beside the first lookups (and again before the calm turns, where they may have been put aside
+  // meanwhile).  Registers that a loop carries and whose loads may still be on their way when it is entered are waited for inside
+  // it, and the compiler does not count the loads into LDS, which are younger: the first of four calm turns then waited for all but
+  // three of these (heads of 128), or for all (of 64).
+  auto settle = [&]() {
 #pragma unroll
-  for (int kt = 0; kt < QT; ++kt) asm volatile("" : "+v"(qreg[kt]));
+    for (int kt = 0; kt < QT; ++kt) asm volatile("" : "+v"(qreg[kt]));
+  };
+  settle();
 #pragma unroll
   for (int j = -3; j < 0; ++j) ask(j, j + 4);
   const int turns = steps + 2;
@@ -1517,7 +1540,7 @@ __device__ __forceinline__ void attention_prompt_body(const Args& a, const int b
       ask(j, u);
       __builtin_amdgcn_sched_barrier(0);
       if (j - 2 >= wave_from && j - 2 < wave_to) {
-        if (j - 2 == 0 || j - 2 == steps - 1) gather_edge(j - 2, (u + 2) & 3, high[i & 1], low[i & 1]);
+        if (j - 2 < calm_from || j - 2 >= calm_to) gather_partly(j - 2, (u + 2) & 3, high[i & 1], low[i & 1]);
         else gather((u + 2) & 3, high[i & 1], low[i & 1]);
       }
       if (j - 1 >= wave_from && j - 1 < wave_to) {
@@ -1538,6 +1561,7 @@ __device__ __forceinline__ void attention_prompt_body(const Args& a, const int b
   careful(0, zeroth, two);
   int j0 = 2;
   for (; j0 < turns && j0 < calm_from + 2; j0 += 4) careful(j0, second, four);
+  settle();
   for (; j0 + 3 < min(calm_to + 1, wave_to); j0 += 4) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -1566,6 +1590,32 @@ __device__ __forceinline__ void attention_prompt_body(const Args& a, const int b
     }
   }
   for (; j0 < turns; j0 += 4) careful(j0, second, four);
+
+  // ---- steps left out (their weights are in the sums of weights): a lane makes half of its column's score of a key ------------
+  for (; !bad && (left_first | left_last) != 0u;) {
+    const bool at_first = left_first != 0u;
+    uint32_t& left = at_first ? left_first : left_last;
+    const int bit = __builtin_ctz(left), step = at_first ? wave_from + bit : wave_to - 1 - bit;
+    left &= left - 1u;
+    for (int key = max(range_lo, first_base + step * 32); key <= min(range_hi, first_base + step * 32 + 31); ++key) {
+      const long page = static_cast<long>(table[key >> page_shift]) * a.kv_heads + kvh;
+      const bf16_t* k = a.k_pages + (page * D << page_shift) + static_cast<long>(key & page_mask) * D + h * (D / 2);
+      const bf16_t* v = a.v_pages + (page * D << page_shift) + (key & page_mask);
+      const bool seen = static_cast<uint32_t>(col_pos - key) < span;
+      float score = 0.f;
+      if (seen)
+        for (int d = 0; d < D / 2; ++d) score = fmaf(to_float(a.q[col_at + h * (D / 2) + d]), to_float(k[d]), score);
+      score += __shfl_xor(score, 32, 64);
+      const float weight = __builtin_amdgcn_exp2f(fmaf(score, a.scale_log2, away));
+#pragma unroll
+      for (int dt = 0; dt < OT; ++dt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const float value = to_float(v[static_cast<long>(dt * 32 + (r >> 2) * 8 + h * 4 + (r & 3)) << page_shift]);
+          if (seen) o[dt][r] = fmaf(weight, value, o[dt][r]);
+        }
+    }
+  }
 
   // ---- results: a lane holds, of its column, dims dt * 32 + 8 i + 4h .. + 3 ------------------------------------------------
   const auto halves = __builtin_amdgcn_permlane32_swap(__float_as_uint(l), __float_as_uint(l), false, false);

@@ -1455,6 +1455,43 @@ def test_attention_on_tiles_of_32_columns_says_that_a_page_is_missing(hip, dim, 
     assert torch.isnan(got[64:200]).all() and not torch.isnan(got[:64]).any() and not torch.isnan(got[200:]).any()
 
 
+@pytest.mark.parametrize("q_heads,kv_heads,dim,page_size", [(8, 2, 128, 16), (3, 3, 128, 64), (40, 2, 64, 16), (8, 1, 64, 32)])
+@pytest.mark.parametrize("poison", [float("inf"), float("nan")])
+@pytest.mark.parametrize("window,at", [(None, 37), (None, 0), (None, 255), (9, 37), (40, 64), (150, 95)])
+def test_attention_on_tiles_of_32_columns_keeps_tokens_clear_of_keys_they_do_not_see(hip, ref, q_heads, kv_heads, dim, page_size, poison, window, at):
+    """Some dims of one position's value, or its key, are infinite or NaN: tokens that do not see it have the plain result; of those
+    that do the poisoned dims are not finite - of a poisoned value no others are."""
+    q, k_pages, v_pages, ctx, meta, _, _ = _attention_case(torch.bfloat16, q_heads, kv_heads, dim, page_size, [(0, 300)], None, 65)
+    want = torch.empty_like(q)
+    ref.attention(q, k_pages, v_pages, ctx, meta, q_heads, kv_heads, dim, dim ** -0.5, window, want)      # (without the poison)
+    page, slot = int(meta.block_table[0, at // page_size]), at % page_size
+    hit = [t for t in range(300) if t >= at and (window is None or t - at < window)]
+    clear = [t for t in range(300) if t not in hit]
+    poisoned = [3, dim // 2 + 1, dim - 1]
+    hip.wide_prompt_tiles, hip.split_prompt_keys = True, False
+    try:
+        for of_values in (True, False):
+            keys, values = k_pages.clone(), v_pages.clone()
+            if of_values:
+                values[page, :, poisoned, slot] = poison
+            else:
+                keys[page, :, slot, poisoned] = poison
+            out = torch.full_like(q, 7.0, device="cuda")
+            cctx, cmeta = _to_cuda(ctx, meta)
+            hip.attention(q.cuda(), keys.cuda(), values.cuda(), cctx, cmeta, q_heads, kv_heads, dim, dim ** -0.5, window, out)
+            out = out.cpu().float().view(300, q_heads, dim)
+            plain = want.float().view(300, q_heads, dim)
+            torch.testing.assert_close(out[clear], plain[clear], **attention_tol(torch.bfloat16))
+            if of_values:
+                assert not torch.isfinite(out[hit][:, :, poisoned]).any()
+                others = [d for d in range(dim) if d not in poisoned]
+                torch.testing.assert_close(out[hit][:, :, others], plain[hit][:, :, others], **attention_tol(torch.bfloat16))
+            elif poison != poison:
+                assert not torch.isfinite(out[hit]).any()
+    finally:
+        hip.wide_prompt_tiles, hip.split_prompt_keys = None, None
+
+
 def test_attention_takes_tiles_of_32_columns_from_some_hundred_keys_on(hip):
     """The rule that chooses between 16 and 32 columns a wave asks for a portion's tokens and, against powers of two from 2,048 on
     (which a recorded step's bounds are), for the longest context, by head size and page."""
