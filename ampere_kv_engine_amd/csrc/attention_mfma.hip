@@ -275,9 +275,10 @@ struct ItemLds {
   float parts[kItemWaves][16][PSTRIDE];
 };
 
-template <int NQ, bool SPLIT, bool PIPE, bool FRESH, bool ONCE, bool ITEMS>
+enum Items : int { kNoItems, kPlanned, kWhole };     // (kWhole: a request is an item, whose result is the output)
+template <int NQ, bool SPLIT, bool PIPE, bool FRESH, bool ONCE, Items ITEMS>
 __device__ __forceinline__ void attention_mfma_body(const Args& a, const Where at, ItemLds* item_lds) {
-  static_assert(!ITEMS || (SPLIT && NQ == 1), "items are single tokens");
+  static_assert(ITEMS == kNoItems || (SPLIT && NQ == 1), "items are single tokens");
   const int lane = at.lane, r16 = lane & 15, g = lane >> 4;
   auto from_pages = [](const char* at) {
     const uintx4* p = reinterpret_cast<const uintx4*>(at);
@@ -294,10 +295,10 @@ __device__ __forceinline__ void attention_mfma_body(const Args& a, const Where a
   Tile t{};
   int seg_lo = 0, seg_hi = 0x7fffffff;     // SPLIT: the keys of this block's segment
   long part = 0;                           // SPLIT: index of its partial result's tile
-  if (SPLIT && (ITEMS || a.plan != nullptr)) {   // item `by` of the plan: a request and a segment of its keys
+  if (SPLIT && (ITEMS == kWhole || a.plan != nullptr)) {   // item `by` of the plan: a request and a segment of its keys
     const int item = at.by;
     int4 record;
-    if (ITEMS && a.plan == nullptr) {      // request `by`, all of its keys
+    if constexpr (ITEMS == kWhole) {       // request `by`, all of its keys
       const int pos = a.seq_lens[a.seq_first + item] - 1;
       record = make_int4(item, a.window > 0 ? max(0, pos - a.window + 1) & ~31 : 0, pos, pos);
     } else {
@@ -311,7 +312,7 @@ __device__ __forceinline__ void attention_mfma_body(const Args& a, const Where a
     t.found = true;
     seg_lo = record.y;
     seg_hi = record.w;
-    if constexpr (ITEMS) {
+    if constexpr (ITEMS != kNoItems) {
       const int steps = ((seg_hi - seg_lo) >> 5) + 1, share = (steps + kItemWaves - 1) / kItemWaves * 32;
       seg_lo += at.wave * share;           // (a wave that gets no step has seg_hi < seg_lo)
       seg_hi = min(seg_hi, seg_lo + share - 1);
@@ -326,7 +327,7 @@ __device__ __forceinline__ void attention_mfma_body(const Args& a, const Where a
       part = (static_cast<long>(at.bx) * at.gy + at.by) * a.num_splits + at.bz;
     }
   }
-  const int head_block = (SPLIT && (ITEMS || a.plan != nullptr)) ? at.bx : at.by;  // (kv head, group of its query heads)
+  const int head_block = (SPLIT && (ITEMS == kWhole || a.plan != nullptr)) ? at.bx : at.by;  // (kv head, group of its query heads)
   const int kvh = head_block / a.head_groups, hg = head_block % a.head_groups;
   const uintx4 zero = uintx4{0u, 0u, 0u, 0u};
   const int page_size = 1 << a.page_shift, page_mask = page_size - 1;
@@ -668,7 +669,7 @@ __device__ __forceinline__ void attention_mfma_body(const Args& a, const Where a
   for (int nq = 0; nq < NQ; ++nq) {
     l[nq] += __shfl_xor(l[nq], 16, 64);
     l[nq] += __shfl_xor(l[nq], 32, 64);
-    if constexpr (ITEMS) {
+    if constexpr (ITEMS != kNoItems) {
       if (!col_valid[nq]) continue;
       float* mine = item_lds->parts[at.wave][r16];
 #pragma unroll
@@ -698,7 +699,7 @@ __device__ __forceinline__ void attention_mfma_body(const Args& a, const Where a
       }
     }
   }
-  if constexpr (ITEMS) {   // the four waves' results into the item's: thread (column, four dims)
+  if constexpr (ITEMS != kNoItems) {   // the four waves' results into the item's: thread (column, four dims)
     __syncthreads();
     const int columns = min(a.heads_per_tile, a.group - hg * a.heads_per_tile);
     for (int e = at.wave * 64 + lane; e < columns * (D / 4); e += 64 * kItemWaves) {
@@ -718,7 +719,7 @@ __device__ __forceinline__ void attention_mfma_body(const Args& a, const Where a
         all += *reinterpret_cast<const floatx4*>(&item_lds->parts[w][c][d]) * by;
         sum = fmaf(by, item_lds->parts[w][c][D + 1], sum);
       }
-      if (a.plan == nullptr) {
+      if constexpr (ITEMS == kWhole) {
         bf16_t* out = a.out + (static_cast<long>(t.first_row) * a.q_heads + kvh * a.group + hg * a.heads_per_tile + c) * D + d;
         const float inv = bad ? nan : 1.f / sum;
 #pragma unroll
@@ -738,17 +739,17 @@ __device__ __forceinline__ void attention_mfma_body(const Args& a, const Where a
 
 template <int NQ, bool SPLIT, bool PIPE, bool FRESH, bool ONCE>
 __global__ __launch_bounds__(64, (SPLIT && NQ == 1 && D <= 128) ? 2 : 1) void attention_mfma_kernel(const Args a) {
-  attention_mfma_body<NQ, SPLIT, PIPE, FRESH, ONCE, false>(
+  attention_mfma_body<NQ, SPLIT, PIPE, FRESH, ONCE, kNoItems>(
       a, Where{static_cast<int>(blockIdx.x), static_cast<int>(blockIdx.y), static_cast<int>(blockIdx.z),
                static_cast<int>(gridDim.x), static_cast<int>(gridDim.y), static_cast<int>(threadIdx.x), 0}, nullptr);
 }
 
 // Items of a plan, or requests: block (head block, item).
-template <bool FRESH, bool ONCE>
+template <bool FRESH, bool ONCE, Items ITEMS>
 __global__ __launch_bounds__(64 * kItemWaves, D <= 128 ? 2 : 1) void attention_items_kernel(const Args a) {
   __shared__ __align__(16) ItemLds lds;
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
-  attention_mfma_body<1, true, true, FRESH, ONCE, true>(
+  attention_mfma_body<1, true, true, FRESH, ONCE, ITEMS>(
       a, Where{static_cast<int>(blockIdx.x), static_cast<int>(blockIdx.y), 0, static_cast<int>(gridDim.x),
                static_cast<int>(gridDim.y), static_cast<int>(threadIdx.x) & 63, wave}, &lds);
 }
@@ -1661,7 +1662,7 @@ __global__ __launch_bounds__(64 * kSharedWaves, 2) void attention_pair_kernel(co
       const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
       const int unit = (static_cast<int>(blockIdx.x) - portion_blocks) * kSharedWaves + wave;
       if (unit >= gx * gy) return;
-      attention_mfma_body<1, true, true, true, ONCE, false>(
+      attention_mfma_body<1, true, true, true, ONCE, kNoItems>(
           single, Where{unit % gx, unit / gx, 0, gx, gy, static_cast<int>(threadIdx.x) & 63, 0}, nullptr);
     }
   }
@@ -1785,6 +1786,13 @@ __global__ __launch_bounds__(64 * kMergeWaves) void attention_merge_kernel(const
     if (lane + e * 64 < D) dst[lane + e * 64] = from_float<bf16_t>(acc[e] * inv);
 }
 
+template <bool FRESH>
+void launch_items(const Args& a, dim3 grid, bool once, bool whole, hipStream_t stream) {
+  if (whole) attention_items_kernel<FRESH, false, kWhole><<<grid, 64 * kItemWaves, 0, stream>>>(a);   // (few keys: not marked)
+  else if (once) attention_items_kernel<FRESH, true, kPlanned><<<grid, 64 * kItemWaves, 0, stream>>>(a);
+  else attention_items_kernel<FRESH, false, kPlanned><<<grid, 64 * kItemWaves, 0, stream>>>(a);
+}
+
 template <int NQ>
 int launch(const Args& a, int tiles, bool shared, int waves_per_item, hipStream_t stream) {
   dim3 grid(tiles, a.kv_heads * a.head_groups, a.num_splits);
@@ -1818,8 +1826,7 @@ int launch(const Args& a, int tiles, bool shared, int waves_per_item, hipStream_
     if constexpr (NQ == 1 && D % 64 == 0) {
       if (!a.single_tokens) return -2;
       if (items && waves_per_item == kItemWaves) {
-        if (once) attention_items_kernel<true, true><<<grid, 64 * kItemWaves, 0, stream>>>(a);
-        else attention_items_kernel<true, false><<<grid, 64 * kItemWaves, 0, stream>>>(a);
+        launch_items<true>(a, grid, once, whole, stream);
         if (!whole) merge();
       } else if (items || a.num_splits > 1) {
         if (once) attention_mfma_kernel<NQ, true, true, true, true><<<grid, 64, 0, stream>>>(a);
@@ -1835,8 +1842,7 @@ int launch(const Args& a, int tiles, bool shared, int waves_per_item, hipStream_
   }
   if (items && waves_per_item == kItemWaves) {
     if constexpr (NQ == 1) {
-      if (once) attention_items_kernel<false, true><<<grid, 64 * kItemWaves, 0, stream>>>(a);
-      else attention_items_kernel<false, false><<<grid, 64 * kItemWaves, 0, stream>>>(a);
+      launch_items<false>(a, grid, once, whole, stream);
       if (!whole) merge();
     } else {
       return -2;
