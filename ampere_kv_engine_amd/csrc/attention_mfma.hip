@@ -1475,12 +1475,16 @@ __device__ __forceinline__ void attention_prompt_body(const Args& a, const int b
   // The same for steps that some column does not see whole.  Slots outside the block's keys hold anything, NaN included (never
   // written, or of a page that stands in for one that a window has passed): blanked.  And a hidden key's weight of zero times an
   // infinite value is not zero: a step that holds values that are not finite is left out and noted; after the turns its values
-  // are added one by one to the columns that see their keys.  (Such steps lie within three of the wave's first or last.)
+  // are added one by one to the columns that see their keys.  (Such steps lie within three of the wave's first or last.)  What is
+  // not finite is found by the matrix instruction, as a product with zero (a window's launch of 25 us: 1.5 us less than by the
+  // vector unit, whose instructions a wave alone issues five cycles apart).
   uint32_t left_first = 0u, left_last = 0u;   // steps left out: counted from the wave's first, or back from its last
   auto gather_partly = [&](int step, int buffer, const uintx4 (&hi)[2], const uintx4 (&lo)[2]) {
     const uint32_t keys = static_cast<uint32_t>(range_hi - range_lo);
     uintx4 keep[2];
-    uint32_t carries = 0u;     // (an exponent of all ones carries into the sign's place)
+    floatx16 probe;            // zero times every value: a sum that is not zero is no number
+#pragma unroll
+    for (int r = 0; r < 16; ++r) probe[r] = 0.f;
 #pragma unroll
     for (int half = 0; half < 2; ++half) {
       const int key = first_base + step * 32 + half * 16 + h * 8 - range_lo;
@@ -1488,12 +1492,12 @@ __device__ __forceinline__ void attention_prompt_body(const Args& a, const int b
       for (int w = 0; w < 4; ++w)
         keep[half][w] = (static_cast<uint32_t>(key + 2 * w) <= keys ? 0xffffu : 0u) | (static_cast<uint32_t>(key + 2 * w + 1) <= keys ? 0xffff0000u : 0u);
 #pragma unroll
-      for (int dt = 0; dt < OT; ++dt) {
-        const uintx4 c = (value_piece(buffer, half, dt) & keep[half] & 0x7fff7fffu) + 0x00800080u;
-        carries |= (c[0] | c[1]) | (c[2] | c[3]);
-      }
+      for (int dt = 0; dt < OT; ++dt) probe = mfma32(value_piece(buffer, half, dt) & keep[half], zero, probe);
     }
-    if (__any((carries & 0x80008000u) != 0u)) {
+    float sum = probe[0];
+#pragma unroll
+    for (int r = 1; r < 16; ++r) sum += probe[r];
+    if (__any(sum != 0.f)) {
       if (step - wave_from < 32) left_first |= 1u << (step - wave_from);
       else left_last |= 1u << ((wave_to - 1 - step) & 31);
       return;

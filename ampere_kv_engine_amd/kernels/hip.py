@@ -1149,7 +1149,7 @@ class HipKernels(PartsKernels, KernelSet):
         exact = starts[ctx.num_seqs] > max(self.FEW_TOKENS, getattr(ctx, "recordable_tokens", 0))
         walked = longest - most // 2 if many and exact else 0
         if head_dim == 128:
-            if window is not None and 2 * blocks < 3 * units and window < (512 if 4 * blocks >= 3 * units else 512 + 4 * per_block):
+            if window is not None and 2 * blocks < 3 * units and window < (512 if 4 * blocks >= 3 * units else 576 + 4 * per_block):
                 return False
             return longest > 2048 or most >= 384 or walked >= 512
         if longest <= 4096:

@@ -42,15 +42,15 @@ def _prompt_kernel(dim, pages_per_step, folder):
 @pytest.mark.parametrize("pages_per_step", [1, 2])
 @pytest.mark.parametrize("dim", [64, 128])
 def test_calm_turns_of_the_prompt_attention_wait_for_counted_loads_alone(dim, pages_per_step, tmp_path):
-    """The loop of four calm turns (a turn multiplies D / 16 times for the scores and D / 8 times for the sums) waits for memory four
-    times, and each time leaves the loads of two turns (2 * D / 64 of keys, as many of values) on their way."""
+    """The loop of four calm turns (a turn multiplies D / 16 times for the scores and D / 8 times for the sums and asks for D / 64
+    pieces of keys and as many of values) waits for memory four times, and each time leaves the loads of two turns on their way."""
     code = _prompt_kernel(dim, pages_per_step, str(tmp_path))
     start = code[0][0]
     loops = []
     for index, (at, text, target) in enumerate(code):
         if text.startswith(("s_cbranch", "s_branch")) and target is not None and start + target <= at:
             body = [t for a, t, _ in code[:index + 1] if a >= start + target]
-            if sum("v_mfma" in t for t in body) == 4 * (dim // 16 + dim // 8):
+            if (sum("v_mfma" in t for t in body), sum("global_load_lds" in t for t in body)) == (4 * (dim // 16 + dim // 8), 4 * 2 * dim // 64):
                 loops.append(body)
     assert len(loops) == 1
     waits = [re.search(r"vmcnt\((\d+)\)", t) for t in loops[0] if t.startswith("s_waitcnt")]

@@ -1460,7 +1460,8 @@ def test_attention_on_tiles_of_32_columns_says_that_a_page_is_missing(hip, dim, 
 @pytest.mark.parametrize("window,at", [(None, 37), (None, 0), (None, 255), (9, 37), (40, 64), (150, 95)])
 def test_attention_on_tiles_of_32_columns_keeps_tokens_clear_of_keys_they_do_not_see(hip, ref, q_heads, kv_heads, dim, page_size, poison, window, at):
     """Some dims of one position's value, or its key, are infinite or NaN: tokens that do not see it have the plain result; of those
-    that do the poisoned dims are not finite - of a poisoned value no others are."""
+    that do the poisoned dims are not finite - of a poisoned value no others are, also where an earlier value has poisoned another
+    dim for everybody."""
     q, k_pages, v_pages, ctx, meta, _, _ = _attention_case(torch.bfloat16, q_heads, kv_heads, dim, page_size, [(0, 300)], None, 65)
     want = torch.empty_like(q)
     ref.attention(q, k_pages, v_pages, ctx, meta, q_heads, kv_heads, dim, dim ** -0.5, window, want)      # (without the poison)
@@ -1470,17 +1471,24 @@ def test_attention_on_tiles_of_32_columns_keeps_tokens_clear_of_keys_they_do_not
     poisoned = [3, dim // 2 + 1, dim - 1]
     hip.wide_prompt_tiles, hip.split_prompt_keys = True, False
     try:
-        for of_values in (True, False):
+        for of_values, earlier in ((True, False), (True, True), (False, False)):
+            if earlier and (window is not None or at < 30):
+                continue
             keys, values = k_pages.clone(), v_pages.clone()
             if of_values:
                 values[page, :, poisoned, slot] = poison
+                if earlier:
+                    values[int(meta.block_table[0, 0]), :, 9, 0] = poison
             else:
                 keys[page, :, slot, poisoned] = poison
             out = torch.full_like(q, 7.0, device="cuda")
             cctx, cmeta = _to_cuda(ctx, meta)
             hip.attention(q.cuda(), keys.cuda(), values.cuda(), cctx, cmeta, q_heads, kv_heads, dim, dim ** -0.5, window, out)
             out = out.cpu().float().view(300, q_heads, dim)
-            plain = want.float().view(300, q_heads, dim)
+            plain = want.float().view(300, q_heads, dim).clone()
+            if earlier:
+                assert not torch.isfinite(out[:, :, 9]).any()
+                out[:, :, 9] = plain[:, :, 9] = 0.0
             torch.testing.assert_close(out[clear], plain[clear], **attention_tol(torch.bfloat16))
             if of_values:
                 assert not torch.isfinite(out[hit][:, :, poisoned]).any()
