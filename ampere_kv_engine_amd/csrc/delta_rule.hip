@@ -114,6 +114,7 @@ __global__ __launch_bounds__(256) void delta_prepare_fours_kernel(const T* __res
 }
 
 // ---- many tokens of a request: the walk in chunks of 16 tokens on the matrix cores ------------------------------------------
+// The chunkwise form of Yang et al., "Parallelizing Linear Transformers with the Delta Rule over Sequence Length" (2024).
 // Over a chunk the recurrence is a linear system.  With S0 the state before it, cum_t the product of the decays of its tokens
 // up to t and fall_st that of the decays behind token s up to t (all products of decays forward in time: nothing is divided,
 // and what underflows is what has decayed away):
@@ -140,13 +141,14 @@ __host__ __device__ inline long chunk_floats(int dim) { return 3L * kChunk * dim
 // The fewest tokens of a request that goes in chunks.  Which form a request takes hangs on its own tokens and the head's size
 // alone, so that its bits do not change with what else is in the step (fewer than kTilesFrom walk in small tiles, others in
 // large ones: a step of all three kinds has three launches).  32 single tokens beside 171, 16 heads of 128 x 128: 60 us, where
-// the single ones went in chunks too 113, where all walked in large tiles 162.  The lines lie
-// where one request alone breaks even; batches would from fewer on.  Whole rule, walk / chunks us, decays per channel: 16 heads of 64
-// x 64 64 tokens 14.9 / 15.5, 80 18.1 / 16.1; 16 heads of 128 x 128 96 tokens 21.6 / 24.2, 128 25.8 / 25.9, 160 30.4 / 28.4 (four
-// requests 80 tokens 43.0 / 36.6; a decay per head 96 21.2 / 21.5, 128 25.0 / 23.5); 8 heads of 256 x 256 32 tokens 21.8 / 27.5, 48
-// 32.2 / 29.6; 6 of 192 x 192 32 22.2 / 24.2, 48 32.2 / 26.0.
+// the single ones went in chunks too 113, where all walked in large tiles 162.  Of 64 and 128 the lines lie where one request
+// alone breaks even (batches would from fewer on), of 192 and 256, whose large tiles take most of a unit's LDS, at the large
+// tiles' own: a request alone loses a little there and several gain much.  Whole rule, walk / chunks us, decays per channel: 16
+// heads of 64 x 64 64 tokens 14.9 / 15.5, 80 18.1 / 16.1; 16 of 128 x 128 96 tokens 21.6 / 24.2, 128 25.8 / 25.9, 160 30.4 / 28.4
+// (four requests of 80 43.0 / 36.6; a decay per head 96 21.2 / 21.5, 128 25.0 / 23.5); 8 of 256 x 256 24 tokens 21.3 / 27.2, 48
+// 32.2 / 29.6, four requests of 24 60.7 / 35.6; 6 of 192 x 192 24 tokens 22.1 / 23.9, four requests 41.9 / 29.8.
 __host__ __device__ inline int chunks_from(int dim) {
-  return dim == 64 ? 65 : dim == 128 ? 128 : dim == 192 || dim == 256 ? 33 : 0x7fffffff;
+  return dim == 64 ? 65 : dim == 128 ? 128 : dim == 192 || dim == 256 ? kTilesFrom : 0x7fffffff;
 }
 
 // Products over the 16 lanes of a row: of lanes up to this one (SHR), of this one and those behind it (SHL).
