@@ -761,7 +761,8 @@ __global__ __launch_bounds__(64 * kItemWaves, D <= 128 ? 2 : 1) void attention_i
 // per tile this takes three quarters of the traffic off the vector memory pipe and the address arithmetic off the
 // waves.  With 16 columns per wave (NQ = 1) three blocks fit a compute unit; with 32 (NQ = 2) two, which do a step for
 // twice the columns with the same loads, barriers and bookkeeping - the host takes them where they still fill the
-// device.  (Heads of 64 and 128 on pages of 16 and more have a kernel of their own for 32 columns, below.)  In LDS a key row is stored at the MFMA row it feeds (tile j, row rho); a value row is one dim's 32 keys.
+// device.  (Heads of 64 and 128 on pages of 16 and more have a kernel of their own for 32 columns, below.)  In LDS a key row is
+// stored at the MFMA row it feeds (tile j, row rho); a value row is one dim's 32 keys.
 // Pages must hold at least 8 tokens (an aligned run of 8 keys of a value row is one 16-byte piece).
 constexpr int kSharedWaves = 4;
 // Rows in LDS, in bfloat16.  16 lanes read 16 bytes each from 16 consecutive rows; such a read runs at full rate when
@@ -1247,8 +1248,11 @@ __global__ __launch_bounds__(64 * kSharedWaves, D <= 128 ? (NQ == 1 ? 3 : 2) : 1
 // 3 of them are the weighted sum's, a third the second part of the weights), the vector unit 50 %; in the same run the
 // order of a turn, the distance of the loads and what stands between the matrix instructions move it by 1 to 3 % only.
 // Where the device has one block a unit (short prompts) a wave alone issues an instruction every 5 cycles, 195 a turn.
-// 32 heads of 8 key heads, against the kernel above at its better width: 2,048 tokens 87 -> 72 us, 1,000 tokens of 40 heads
-// 41 -> 37; 64 heads, 2,048 tokens after 6,144 768 -> 600 us (0.80 PFLOP/s, the weights' second part not counted).
+// 32 heads of 8 key heads, against the kernel above at its better width, launches in a recorded graph: 2,048 tokens 78 -> 64 us,
+// 1,000 tokens of 40 heads 38 -> 34; 64 heads, 2,048 tokens after 6,144 762 -> 595 us (0.81 PFLOP/s, the weights' second part not
+// counted).  The denominator is the float32 weights' own sum - above it is summed from the two parts, as the numerator is: what the
+// second part's rounding leaves (2^-17 of a weight) no longer cancels, and lies far below an output's own (errors against 64 bits
+// are the same to three digits: 64 heads, 2,048 after 6,144 1.58e-3 either way).
 // Every address of a step is a page's address (scalar) plus a constant of the thread: pages are looked up at indices held
 // inside the range, keys beyond it (their slots hold anything) are hidden from the scores by position, values outside it are
 // blanked as they are read from LDS.
@@ -2040,7 +2044,7 @@ extern "C" int AKV_CONCAT(akv_attention_pair_d, AKV_HEAD_DIM)(
   single.num_splits = 1;
   single.plan = plan;
   single.items_grid = items_grid;
-    single.qkv = static_cast<const bf16_t*>(qkv);
+  single.qkv = static_cast<const bf16_t*>(qkv);
   single.q_weight = q_weight;
   single.k_weight = k_weight;
   single.rope_table = rope_table;
