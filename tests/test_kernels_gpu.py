@@ -1071,6 +1071,37 @@ def test_float32_products_on_the_matrix_cores(hip, outs, k):
         assert torch.equal(y[0], alone[0]), rows
 
 
+@pytest.mark.parametrize("rows", [2, 12, 30, 50, 333, 1000])     # (a kernel and a cut of k each)
+def test_float32_products_of_operands_without_parts(hip, rows):
+    """The products multiply operands as three bfloat16 numbers; what has none - infinities, numbers that bfloat16 rounds to
+    infinity - and sums beyond 2^80 take the float32 instruction, output by output: not a number and infinite where float64 says
+    so, finite elsewhere, and other outputs' bits as without them.  Tiny operands keep their last bits: the bound of the test above."""
+    outs, k = 200, 1100
+    w, x = rand(outs, k, seed=41).cuda(), rand(rows, k, seed=42).cuda()
+    clean = torch.empty(rows, outs, device="cuda")
+    hip.linear(x, w, clean)
+    reach = lambda x, w: (128 + 9 + 1) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+    for scale_x, scale_w in ((2.0 ** -110, 2.0 ** 90), (2.0 ** 95, 2.0 ** -120), (2.0 ** 60, 2.0 ** 50)):
+        a, b, y = x * scale_x, w * scale_w, torch.empty(rows, outs, device="cuda")
+        hip.linear(a, b, y)
+        assert ((y.double() - a.double() @ b.double().T).abs() <= reach(a, b)).all(), (scale_x, scale_w)
+    a, b = x.clone(), w.clone()
+    a[1, 7], a[0, 1030] = float("inf"), 3.4e38
+    b[5, 9], b[6, 7], b[7, 3], b[150, 1099] = -float("inf"), 0.0, float("nan"), -3.4028e38
+    a[0, 1099] = a[1, 1099] = b[150, 1030] = 0.0               # (no two products of either sign beyond float32 in one sum)
+    y = torch.empty(rows, outs, device="cuda")
+    hip.linear(a, b, y)
+    want = a.double() @ b.double().T
+    infinite = want.abs() > 3.4028235e38                       # (infinite, or beyond float32)
+    assert torch.equal(torch.isnan(y), torch.isnan(want)) and torch.equal(torch.isinf(y), infinite)
+    assert torch.equal(y[infinite].sign().double(), want[infinite].sign())
+    rest = torch.isfinite(want) & ~infinite
+    assert ((y.double() - want).abs() <= reach(a, b))[rest].all()
+    untouched = torch.ones(rows, outs, dtype=torch.bool, device="cuda")
+    untouched[:2], untouched[:, [5, 6, 7, 150]] = False, False
+    assert torch.equal(y[untouched], clean[untouched])
+
+
 def test_float32_product_of_rows_that_are_not_aligned(hip, ref):
     """A matrix that begins between 16-byte boundaries goes to the plain kernel."""
     x, w = rand(20, 64, seed=34).cuda(), rand(40 * 64 + 1, seed=35).cuda()[1:].view(40, 64)
