@@ -1265,21 +1265,38 @@ __device__ __forceinline__ floatx16 mfma32(uintx4 a, uintx4 b, floatx16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 
-// SP: pages per step of 32 keys (2: pages of 16, 1: of 32 or more)
-template <int SP>
-__device__ __forceinline__ void attention_prompt_body(const Args& a, const int block, const int tid) {
-  constexpr int KP = D / 8;        // 16-byte pieces of a key's row
-  constexpr int QT = D / 16;       // 16-dim steps of the score product
+// What a gated attention (`gated_attention.hip`) adds to it: a sink in the softmax's denominator (exp(0), or exp of a number per
+// query vector), a gate per head, outputs that are columns of wider rows and take a constant.
+// Against its own kernel of 64 columns a block (`gated_attention_shared`), 16 heads over 4, us: 2,000 tokens, 128 wide 76 -> 53, in two
+// maps of 64 beside values of 128, a window of 1,024, 59 -> 47; 1,024 tokens after 6,000 242 -> 157; four portions of 500 30 -> 22.  Below
+// some 500 keys that kernel's shorter start is faster (256 tokens 11.9 / 15.6): the host chooses (`prompt_tiles_time`).  What bounds it
+// is the plain kernel's (a block's step of 32 keys takes 0.68 us, with one block a unit or with two; eight waves a block, the steps
+// over two groups of them, took 52 to 55 us for the 2,000 tokens).
+struct Gated {
+  const float* sink_logits;   // [query vectors], or null
+  const bf16_t* gates;        // null, or [tokens, gate_stride]: head h's output times sigmoid(gates[t, gate_at + h])
+  long gate_stride, out_stride;
+  float out_scale;
+  int gate_at, sink;
+};
+
+// SP: pages per step of 32 keys (2: pages of 16, 1: of 32 or more).  MAPS: 0 plain attention; 1 gated; 2 gated, and a key's record
+// of D holds two vectors of D / 2, each with query vectors of its own (a head's two side by side): a block takes one of them.
+template <int SP, int MAPS>
+__device__ __forceinline__ void attention_prompt_body(const Args& a, const Gated& gated, const int block, const int tid) {
+  constexpr int KD = MAPS == 2 ? D / 2 : D;   // what a query vector and a key share
+  constexpr int KP = KD / 8;       // 16-byte pieces of a key's row
+  constexpr int QT = KD / 16;      // 16-dim steps of the score product
   constexpr int OT = D / 32;       // 32-dim tiles of the output
-  constexpr int kLoads = D / 64;   // pieces of a step's keys that a thread moves, and as many of its values
-  constexpr int kStep = 32 * D;    // elements of a step's keys, and of its values
-  __shared__ __align__(1024) bf16_t k_lds[4 * kStep];
-  __shared__ __align__(1024) bf16_t v_lds[4 * kStep];
+  constexpr int kKeyLoads = KD / 64, kValueLoads = D / 64;   // pieces of a step's keys and of its values that a thread moves
+  constexpr int kKeyStep = 32 * KD, kValueStep = 32 * D;     // elements of a step's keys, and of its values
+  __shared__ __align__(1024) bf16_t k_lds[4 * kKeyStep];
+  __shared__ __align__(1024) bf16_t v_lds[4 * kValueStep];
   const int page_shift = SP == 2 ? 4 : a.page_shift;
   const int lane = tid & 63, c32 = lane & 31, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   // the order of the blocks: as in attention_shared_body
-  const int heads = a.kv_heads * a.head_groups, round = 2 * a.units;
+  const int maps = MAPS == 2 ? 2 : 1, heads = a.kv_heads * a.head_groups * maps, round = 2 * a.units;
   const int turn = block / round, within = block % round;
   const int total = a.tiles * heads, in_round = min(round, total - turn * round);
   const int rank = turn * round + (within < a.units ? within : in_round - 1 - (within - a.units));
@@ -1289,7 +1306,8 @@ __device__ __forceinline__ void attention_prompt_body(const Args& a, const int b
   t.first_row = __builtin_amdgcn_readfirstlane(t.first_row);
   t.tokens = __builtin_amdgcn_readfirstlane(t.tokens);
   t.first_pos = __builtin_amdgcn_readfirstlane(t.first_pos);
-  const int kvh = (rank % heads) / a.head_groups, hg = (rank % heads) % a.head_groups;
+  const int pair = (rank % heads) / a.head_groups, hg = (rank % heads) % a.head_groups;
+  const int kvh = pair / maps, map = pair % maps;
   const uintx4 zero = uintx4{0u, 0u, 0u, 0u};
 
   // this lane's column
@@ -1298,7 +1316,8 @@ __device__ __forceinline__ void attention_prompt_body(const Args& a, const int b
   const bool col_valid = token < t.tokens && c32 / a.heads_per_tile < a.tokens_per_tile && head_in_group < a.group;
   const int col_pos = col_valid ? t.first_pos + token : -1;   // (a column that is no (token, head) pair sees nothing)
   const uint32_t span = a.window > 0 ? static_cast<uint32_t>(a.window) : 0x80000000u;   // keys a column sees: pos - key < span
-  const long col_at = (static_cast<long>(t.first_row + token) * a.q_heads + kvh * a.group + head_in_group) * D;
+  const int vector = (kvh * a.group + head_in_group) * maps + map;
+  const long col_at = (static_cast<long>(t.first_row + token) * a.q_heads + vector) * KD;
   uintx4 qreg[QT];
 #pragma unroll
   for (int kt = 0; kt < QT; ++kt) qreg[kt] = col_valid ? *reinterpret_cast<const uintx4*>(a.q + col_at + kt * 16 + h * 8) : zero;
@@ -1335,15 +1354,19 @@ __device__ __forceinline__ void attention_prompt_body(const Args& a, const int b
   const uint32_t page_bytes = static_cast<uint32_t>(a.kv_heads) * D * 2u << page_shift;
   const uint32_t head_bytes = static_cast<uint32_t>(kvh) * D * 2u << page_shift;
   const int page_mask = (1 << page_shift) - 1;
-  uint32_t k_from[kLoads], v_from[kLoads];   // byte offset inside the page, without what the step's first key adds
-  int k_sel[kLoads], v_sel[kLoads];          // which of the step's pages (the same in every lane of a wave)
+  uint32_t k_from[kKeyLoads], v_from[kValueLoads];   // byte offset inside the page, without what the step's first key adds
+  int k_sel[kKeyLoads], v_sel[kValueLoads];          // which of the step's pages (the same in every lane of a wave)
 #pragma unroll
-  for (int p = 0; p < kLoads; ++p) {
+  for (int p = 0; p < kKeyLoads; ++p) {
     const int c = p * 256 + tid, row = c / KP;
-    const int piece = (c % KP) ^ (D == 128 ? row & 15 : (row >> 1) & 7);
+    const int piece = (c % KP) ^ (KD == 128 ? row & 15 : (row >> 1) & 7);
     const int key = ((row >> 4) << 4) + (((row >> 2) & 1) << 3) + (((row >> 3) & 1) << 2) + (row & 3);
     k_sel[p] = SP == 1 ? 0 : __builtin_amdgcn_readfirstlane(row >> 4);
-    k_from[p] = head_bytes + piece * 16u + static_cast<uint32_t>(SP == 2 ? key & 15 : key) * (D * 2u);
+    k_from[p] = head_bytes + map * (KD * 2u) + piece * 16u + static_cast<uint32_t>(SP == 2 ? key & 15 : key) * (D * 2u);
+  }
+#pragma unroll
+  for (int p = 0; p < kValueLoads; ++p) {
+    const int c = p * 256 + tid;
     const int half = c / (2 * D), dim = (c % (2 * D)) >> 1, run = (c & 1) ^ ((dim >> 3) & 1);
     v_sel[p] = SP == 1 ? 0 : __builtin_amdgcn_readfirstlane(half);
     v_from[p] = head_bytes + (static_cast<uint32_t>(dim) << (page_shift + 1)) + (SP == 2 ? 0u : half * 32u) + run * 16u;
@@ -1374,14 +1397,14 @@ __device__ __forceinline__ void attention_prompt_body(const Args& a, const int b
   auto keys_of = [&](int step, int u) {   // (u: the step modulo 4)
     const uint32_t in = SP == 2 ? 0u : static_cast<uint32_t>((first_base + step * 32) & page_mask) * (D * 2u);
 #pragma unroll
-    for (int p = 0; p < kLoads; ++p)
-      into_lds(k_bytes + (k_sel[p] == 0 ? at[u][0] : at[u][SP - 1]) + in, k_from[p], k_base + u * (kStep * 2u) + p * 4096u);
+    for (int p = 0; p < kKeyLoads; ++p)
+      into_lds(k_bytes + (k_sel[p] == 0 ? at[u][0] : at[u][SP - 1]) + in, k_from[p], k_base + u * (kKeyStep * 2u) + p * 4096u);
   };
   auto values_of = [&](int step, int u) {
     const uint32_t in = SP == 2 ? 0u : static_cast<uint32_t>((first_base + step * 32) & page_mask) * 2u;
 #pragma unroll
-    for (int p = 0; p < kLoads; ++p)
-      into_lds(v_bytes + (v_sel[p] == 0 ? at[u][0] : at[u][SP - 1]) + in, v_from[p], v_base + u * (kStep * 2u) + p * 4096u);
+    for (int p = 0; p < kValueLoads; ++p)
+      into_lds(v_bytes + (v_sel[p] == 0 ? at[u][0] : at[u][SP - 1]) + in, v_from[p], v_base + u * (kValueStep * 2u) + p * 4096u);
   };
   auto resolve = [&](int u, int which) {
 #pragma unroll
@@ -1405,13 +1428,13 @@ __device__ __forceinline__ void attention_prompt_body(const Args& a, const int b
     }
   };
   // where a lane reads its operands: key row c32, dims kt * 16 + 8h .. + 7; value dim dt * 32 + c32, keys 16t + 8h .. + 7
-  const uint32_t k_row = c32 * (D * 2u) + ((h ^ (D == 128 ? c32 & 15 : (c32 >> 1) & 7)) << 4);
+  const uint32_t k_row = c32 * (KD * 2u) + ((h ^ (KD == 128 ? c32 & 15 : (c32 >> 1) & 7)) << 4);
   const uint32_t v_row = c32 * 32u + ((h ^ ((c32 >> 3) & 1)) << 4);
   auto key_piece = [&](int buffer, int kt) {
-    return *reinterpret_cast<const uintx4*>(reinterpret_cast<const char*>(k_lds) + (k_row ^ (kt * 32u)) + buffer * (kStep * 2u));
+    return *reinterpret_cast<const uintx4*>(reinterpret_cast<const char*>(k_lds) + (k_row ^ (kt * 32u)) + buffer * (kKeyStep * 2u));
   };
   auto value_piece = [&](int buffer, int half, int dt) {
-    return *reinterpret_cast<const uintx4*>(reinterpret_cast<const char*>(v_lds) + v_row + (buffer * (kStep * 2u) + half * (D * 32u) + dt * 1024u));
+    return *reinterpret_cast<const uintx4*>(reinterpret_cast<const char*>(v_lds) + v_row + (buffer * (kValueStep * 2u) + half * (D * 32u) + dt * 1024u));
   };
 
   // ---- the three pieces of work -------------------------------------------------------------------------------------------
@@ -1519,7 +1542,7 @@ __device__ __forceinline__ void attention_prompt_body(const Args& a, const int b
   // step j + 1 are asked for (the loads of two later turns may still be on their way when a turn begins) ---------------------
   auto begin = [&]() {
     __builtin_amdgcn_sched_barrier(0);
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"(4 * kLoads) : "memory");
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"(2 * (kKeyLoads + kValueLoads)) : "memory");
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
   };
@@ -1590,8 +1613,8 @@ __device__ __forceinline__ void attention_prompt_body(const Args& a, const int b
 #pragma unroll
       for (int x = 0; x < QT + 4 * OT; ++x) {
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x002, D == 128 ? 5 : 9, 0);
-        if (D == 64 || x % 3 != 2) __builtin_amdgcn_sched_group_barrier(0x400, D == 64 ? 2 : 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, KD < D ? 6 : D == 128 ? 5 : 9, 0);
+        if (D == 64 || x % (KD < D ? 5 : 3) != 2) __builtin_amdgcn_sched_group_barrier(0x400, D == 64 ? 2 : 1, 0);
         if (x < 2 * OT) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
       }
       if (__any(!(sum <= 256.f))) sum = follow(s[(u + 1) & 1], high[(u + 1) & 1], low[(u + 1) & 1]);
@@ -1608,12 +1631,12 @@ __device__ __forceinline__ void attention_prompt_body(const Args& a, const int b
     left &= left - 1u;
     for (int key = max(range_lo, first_base + step * 32); key <= min(range_hi, first_base + step * 32 + 31); ++key) {
       const long page = static_cast<long>(table[key >> page_shift]) * a.kv_heads + kvh;
-      const bf16_t* k = a.k_pages + (page * D << page_shift) + static_cast<long>(key & page_mask) * D + h * (D / 2);
+      const bf16_t* k = a.k_pages + (page * D << page_shift) + static_cast<long>(key & page_mask) * D + map * KD + h * (KD / 2);
       const bf16_t* v = a.v_pages + (page * D << page_shift) + (key & page_mask);
       const bool seen = static_cast<uint32_t>(col_pos - key) < span;
       float score = 0.f;
       if (seen)
-        for (int d = 0; d < D / 2; ++d) score = fmaf(to_float(a.q[col_at + h * (D / 2) + d]), to_float(k[d]), score);
+        for (int d = 0; d < KD / 2; ++d) score = fmaf(to_float(a.q[col_at + h * (KD / 2) + d]), to_float(k[d]), score);
       score += __shfl_xor(score, 32, 64);
       const float weight = __builtin_amdgcn_exp2f(fmaf(score, a.scale_log2, away));
 #pragma unroll
@@ -1629,8 +1652,21 @@ __device__ __forceinline__ void attention_prompt_body(const Args& a, const int b
   // ---- results: a lane holds, of its column, dims dt * 32 + 8 i + 4h .. + 3 ------------------------------------------------
   const auto halves = __builtin_amdgcn_permlane32_swap(__float_as_uint(l), __float_as_uint(l), false, false);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (the last turns' loads still write this block's LDS)
-  const float inv = bad ? __uint_as_float(0x7fc00000u) : 1.f / (__uint_as_float(halves[0]) + __uint_as_float(halves[1]));
+  float sum = __uint_as_float(halves[0]) + __uint_as_float(halves[1]), factor = 1.f;
   if (!col_valid) return;
+  bf16_t* to = a.out + col_at;
+  if constexpr (MAPS > 0) {
+    const int row = t.first_row + token;
+    // (the sink's term against the column's reference point, as the weights are formed; a sink of -inf is none)
+    if (gated.sink) sum += __builtin_amdgcn_exp2f(fmaf(gated.sink_logits != nullptr ? gated.sink_logits[vector] : 0.f, kLog2e, away));
+    factor = gated.out_scale;
+    if (gated.gates != nullptr) {
+      const float gate = to_float(gated.gates[static_cast<long>(row) * gated.gate_stride + gated.gate_at + vector]);
+      factor *= 1.f / (1.f + __expf(-gate));
+    }
+    to = a.out + static_cast<long>(row) * gated.out_stride + static_cast<long>(vector) * D;
+  }
+  const float inv = bad ? __uint_as_float(0x7fc00000u) : factor / sum;
 #pragma unroll
   for (int dt = 0; dt < OT; ++dt)
 #pragma unroll
@@ -1638,13 +1674,17 @@ __device__ __forceinline__ void attention_prompt_body(const Args& a, const int b
       uintx2 packed;
       packed.x = bf16_pair(o[dt][4 * i] * inv, o[dt][4 * i + 1] * inv);
       packed.y = bf16_pair(o[dt][4 * i + 2] * inv, o[dt][4 * i + 3] * inv);
-      *reinterpret_cast<uintx2*>(a.out + col_at + dt * 32 + i * 8 + h * 4) = packed;
+      *reinterpret_cast<uintx2*>(to + dt * 32 + i * 8 + h * 4) = packed;
     }
 }
 
 template <int SP>
 __global__ __launch_bounds__(64 * kSharedWaves, 2) void attention_prompt_kernel(const Args a) {
-  attention_prompt_body<SP>(a, static_cast<int>(blockIdx.x), static_cast<int>(threadIdx.x));
+  attention_prompt_body<SP, 0>(a, Gated{}, static_cast<int>(blockIdx.x), static_cast<int>(threadIdx.x));
+}
+template <int SP, int MAPS>
+__global__ __launch_bounds__(64 * kSharedWaves, 2) void attention_prompt_gated_kernel(const Args a, const Gated gated) {
+  attention_prompt_body<SP, MAPS>(a, gated, static_cast<int>(blockIdx.x), static_cast<int>(threadIdx.x));
 }
 #endif
 
@@ -2072,3 +2112,52 @@ extern "C" int AKV_CONCAT(akv_attention_pair_d, AKV_HEAD_DIM)(
   if (portion.units == 0) return -3;
   return launch_pair(single, portion, portion_tiles, stream);
 }
+
+#ifdef AKV_PROMPT_TILES
+// Gated attention of prompt portions (see `Gated`): requests seq_first .. seq_first + seq_count - 1 of the step in blocks of four
+// tiles of 32 columns, `tiles` of them over those requests (sum of ceil(tokens / (4 * tokens_per_tile))).  `maps` 1: keys and values
+// D wide; 2: values D wide, a key's record two vectors of D / 2, `q_heads` counts query vectors.  `q` [tokens, q_heads * D / maps];
+// `out`: column 0 of the first token's output, rows out_stride apart, 8-byte aligned; `q` and the pages 16-byte aligned.
+extern "C" int AKV_CONCAT(akv_attention_gated_d, AKV_HEAD_DIM)(
+    const void* q, const void* k_pages, const void* v_pages, const void* gates, long gate_stride, int gate_at, const int* q_start,
+    const int* seq_lens, const int* block_table, const int* table_rows, int table_width, void* out, int seq_first, int seq_count,
+    int tiles, int q_heads, int kv_heads, int maps, int heads_per_tile, int head_groups, int tokens_per_tile, int page_size,
+    long num_pages, float scale, int window, int sink, const float* sink_logits, long out_stride, float out_scale,
+    hipStream_t stream) {
+  if (tiles <= 0 || seq_count <= 0) return 0;
+  if (maps < 1 || maps > 2 || (maps == 2 && D != 128) || kv_heads <= 0 || q_heads % (kv_heads * maps) != 0 || page_size < 16 ||
+      heads_per_tile * tokens_per_tile > 32 || out_stride % 4 != 0 || reinterpret_cast<uintptr_t>(out) % 8 != 0 ||
+      ((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k_pages) | reinterpret_cast<uintptr_t>(v_pages)) % 16) != 0)
+    return -2;
+  Args a{};
+  const int status = common_args(a, q, k_pages, v_pages, out, q_start, seq_lens, block_table, table_rows, table_width,
+                                 q_heads, kv_heads, page_size, num_pages, scale, window);
+  if (status != 0) return status;
+  a.group = q_heads / (kv_heads * maps);
+  if (heads_per_tile * head_groups < a.group) return -2;
+  a.seq_first = seq_first;
+  a.seq_count = seq_count;
+  a.tiles = tiles;
+  a.heads_per_tile = heads_per_tile;
+  a.head_groups = head_groups;
+  a.tokens_per_tile = tokens_per_tile;
+  a.num_splits = 1;
+  a.units = units_of_device();
+  if (a.units == 0) return -3;
+  const long blocks = static_cast<long>(tiles) * kv_heads * head_groups * maps;
+  if (blocks > 0x7fffffffL) return -2;
+  const Gated gated{sink_logits, static_cast<const bf16_t*>(gates), gate_stride, out_stride, out_scale, gate_at, sink};
+  const dim3 grid(static_cast<unsigned>(blocks));
+  const bool large = a.page_shift >= 5;
+  if (maps == 1) {
+    if (large) attention_prompt_gated_kernel<1, 1><<<grid, 64 * kSharedWaves, 0, stream>>>(a, gated);
+    else attention_prompt_gated_kernel<2, 1><<<grid, 64 * kSharedWaves, 0, stream>>>(a, gated);
+  } else {
+#if AKV_HEAD_DIM == 128
+    if (large) attention_prompt_gated_kernel<1, 2><<<grid, 64 * kSharedWaves, 0, stream>>>(a, gated);
+    else attention_prompt_gated_kernel<2, 2><<<grid, 64 * kSharedWaves, 0, stream>>>(a, gated);
+#endif
+  }
+  return AKV_LAUNCH_STATUS();
+}
+#endif

@@ -84,11 +84,11 @@ int launch_tiled(const void* x, const void* w, void* y, int rows, int outs, int 
 // A lane's operand of an instruction is 32 bytes of a matrix row: lane (r, g) holds elements 4 g .. + 3 and 16 + 4 g .. + 3 of 32
 // of row r.  All kernels sum every output the same way, so that a row's result depends neither on how many rows a call carries nor
 // on which kernel takes it: k is cut into segments of 128, a segment is one chain of instructions (32 elements after 32, the six
-// products of each in their order), // every fourth segment's sums are added in their order, from the first, second, third and fourth
+// products of each in their order), every fourth segment's sums are added in their order, from the first, second, third and fourth
 // on, and then those four, the even ones and the odd ones first.  The instruction cuts a sum's low bits off towards minus infinity:
 // every result would be 0.02 x 2^-24 sum |x w| too low, which a model's residual sum collects layer by layer; so the rows' elements
-// of odd segments are negated, and what their sums make is subtracted.  (Rows and outputs beyond the matrices repeat the last one and are not stored; elements beyond k are
-// zeros and change no sum.)
+// of odd segments are negated, and what their sums make is subtracted.  (Rows and outputs beyond the matrices repeat the last one
+// and are not stored; elements beyond k are zeros and change no sum.)
 typedef float floats4 __attribute__((ext_vector_type(4)));
 typedef uint32_t uints4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));

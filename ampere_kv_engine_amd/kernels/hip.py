@@ -937,6 +937,15 @@ class HipKernels(PartsKernels, KernelSet):
             self._attention_entry[key] = entry
         return self._attention_entry[key]
 
+    def _attention_gated_entry(self, head_dim: int):
+        key = ("gated", head_dim)
+        if key not in self._attention_entry:
+            self._attention_mfma_entry(head_dim)            # (loads the head size's library)
+            entry = getattr(ctypes.CDLL(ensure_attention(head_dim)), f"akv_attention_gated_d{head_dim}")
+            entry.restype = ctypes.c_int
+            self._attention_entry[key] = entry
+        return self._attention_entry[key]
+
     def _pair_fits(self, ctx, decodes, q_heads, kv_heads, head_dim, page_size, fresh) -> bool:
         """Whether a step's single tokens and prompt portions can go into one launch: the single tokens' kernel takes
         raw projections and cuts the keys on the device (at most 64 requests, some history beyond one segment), the

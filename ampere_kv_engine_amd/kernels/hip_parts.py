@@ -45,6 +45,12 @@ def shares_keys(units: int, portions, vectors: int, kv_heads: int, maps: int, di
       64 / 64: 16 over 16, 1,024 31 / 28, after 3,000 109 / 117; 16 over 4, 1,280 38 / 32, 2,048 59 / 68, 1,024 after 4,000 134 / 142;
       64 / 128 in two maps, 16 over 8, a window of 1,024: 512 21 / 19, 512 after 6,000 40 / 50;
       32 / 32: 16 over 4, 1,024 30 / 17, 1,280 36 / 25, 2,048 55 / 49, 1,024 after 4,000 129 / 111; 32 over 8, 2,048 55 / 95."""
+    shared, tiles = key_times(units, portions, vectors, kv_heads, maps, dim, vdim, window, chunk)
+    return shared < tiles
+
+
+def key_times(units: int, portions, vectors: int, kv_heads: int, maps: int, dim: int, vdim: int, window, chunk) -> tuple[float, float]:
+    """What the two kernels of `shares_keys` are expected to take, us."""
     reach = min((x for x in (window, chunk) if x is not None), default=1 << 30)
     share = vectors // kv_heads // maps
     tile, step = 0.21 + 0.0024 * dim + 0.0022 * vdim, 0.72 + 0.0018 * dim + 0.0017 * vdim
@@ -61,7 +67,33 @@ def shares_keys(units: int, portions, vectors: int, kv_heads: int, maps: int, di
         tile_steps += of_tile * (keys / 16 + 1)
         steps += (count * share + 63) // 64 * kv_heads * maps * (keys / 32 + 1)
     by_tiles = 6 + max((6 * tiles + tile_steps) * tile / 1000 * 256 / units, longest / 64 * 2.2 * tile)
-    return 5 + step * max(longest / 32, steps / (2 * units)) < by_tiles
+    return 5 + step * max(longest / 32, steps / (2 * units)), by_tiles
+
+
+def prompt_tiles_time(units: int, portions, vectors: int, kv_heads: int, maps: int, dim: int, vdim: int, window) -> float:
+    """What prompt portions are expected to take on the plain prompt attention's tiles of 32 columns (`attention_prompt_gated_kernel`),
+    us: a start, and steps of 32 keys - the longest block's, or what all blocks make for a unit, each with four more for its own
+    start.  Fitted to, best of the other two / on these tiles, 256 units:
+      128 / 128: 16 heads over 4, 64 tokens 6.5 / 10.5, 256 11.9 / 15.6, 512 20.5 / 20.8, 1,024 41 / 32, 2,000 76 / 53, 512 after 2,048 83 / 61,
+        1,024 after 6,000 242 / 157, 4 x 500 30 / 22, 8 x 128 11.1 / 13.3, 2,000 in a window of 512 34 / 28, 1,024 26.0 / 25.8; 32 over 8,
+        2,000 84 / 63, 4 x 500 40 / 29;
+      64 / 128 in two maps, 16 over 4, a window of 1,024: 512 22.3 / 19.4, 1,024 40 / 31, 2,000 59 / 47, 1,024 after 6,000 51 / 37;
+      64 / 64: 16 over 4, 512 14.4 / 15.0, 1,024 27 / 23, 2,000 60 / 39, 1,024 after 6,000 189 / 112; 16 over 16, 2,000 60 / 39."""
+    reach = window if window is not None else 1 << 30
+    share = vectors // kv_heads // maps
+    heads_per_tile = min(share, 32)
+    per_block, head_groups = 4 * (32 // heads_per_tile), (share + heads_per_tile - 1) // heads_per_tile
+    longest = steps = 0.0
+    for count, length in portions:
+        if count == 0:
+            continue
+        before = length - count
+        growing = min(max(reach - before, 0), count)
+        keys = (growing * (before + growing / 2) + (count - growing) * reach) / count
+        longest = max(longest, min(length, reach + per_block))
+        steps += (count + per_block - 1) // per_block * head_groups * kv_heads * maps * ((keys + per_block / 2) / 32 + 4)
+    wide = dim + vdim
+    return 4.2 + 0.0207 * wide + (0.3 + 0.0015 * wide) * max(longest / 32, steps / units)
 
 
 class PartsKernels:
@@ -852,6 +884,40 @@ class PartsKernels:
     shared_attention_blocks = None      # prompt portions of this many blocks share their keys through LDS; None: by `shares_keys`
     FEW_TOKENS = 512                    # (what `EngineConfig.record_max_tokens` allows a recorded step by default; more where it does)
 
+    gated_prompt_tiles = None           # None: as `_takes_prompt_tiles` says; True or False (for tests and measurements)
+
+    def _takes_prompt_tiles(self, ctx, first: int, heads: tuple[int, int, int, int, int], window, page_size: int) -> bool:
+        """Whether the portions of a step, requests `first` on, go to the plain prompt attention's kernel on tiles of 32 columns.  It
+        takes keys and values of one width, 64 or 128, or two maps of 64 beside values of 128, on pages of 16, 32, 64 ...; it is taken
+        where some portion sees 448 keys and more and `prompt_tiles_time` lies below what the other two kernels are expected to take -
+        by a tenth in steps of few tokens, whose portions count as having as much before them as they bring (see
+        `_shares_attention_keys`)."""
+        vectors, kv_heads, maps, dim, vdim = heads
+        fits = (vdim in (64, 128) and dim == vdim and maps == 1) or (vdim == 128 and dim == 64 and maps == 2)
+        if (not fits or page_size < 16 or page_size & (page_size - 1) or self.shared_attention_blocks is not None
+                or getattr(ctx, "seq_lens", None) is None):        # (a step that names its requests' lengths on the host alone)
+            return False
+        if self.gated_prompt_tiles is not None:
+            return self.gated_prompt_tiles
+        starts, lengths = ctx.host_q_start[first:ctx.num_seqs + 1], ctx.host_seq_lens[first:ctx.num_seqs]
+        choices = ctx.__dict__.setdefault("prompt_tiles", {})
+        key = (tuple(starts), tuple(lengths), heads, window)
+        if key not in choices:
+            portions, few = self._portions(ctx, starts, lengths)
+            longest = max((length for count, length in portions if count), default=0)
+            shared, tiles = key_times(self.compute_units, portions, *heads, window, None)
+            if shared_blocks(portions, *heads[:3]) < self.compute_units:
+                shared = tiles
+            choices[key] = (min(longest, window or longest) >= 448 and
+                            prompt_tiles_time(self.compute_units, portions, *heads, window) * (1.1 if few else 1.0) < min(shared, tiles))
+        return choices[key]
+
+    def _portions(self, ctx, starts, lengths) -> tuple[list[tuple[int, int]], bool]:
+        """(tokens, tokens held after the step) of requests, and whether the step is one of few tokens: one that may be recorded,
+        where a length is only a bound and counts as twice the tokens, recorded or not."""
+        few = starts[-1] <= max(self.FEW_TOKENS, getattr(ctx, "recordable_tokens", 0))
+        return [(end - start, 2 * (end - start) if few else length) for start, end, length in zip(starts, starts[1:], lengths)], few
+
     def _shares_attention_keys(self, ctx, first: int, heads: tuple[int, int, int, int, int], window, chunk) -> tuple[int, bool]:
         """The blocks that the portions of a step, requests `first` on, make in the kernel that shares keys, and whether they go
         there.  It takes enough blocks for every unit, and then what `shares_keys` says.  In steps of few tokens - those that may be
@@ -861,9 +927,7 @@ class PartsKernels:
         choices = ctx.__dict__.setdefault("shared_attention", {})
         key = (tuple(starts), tuple(lengths), heads, window, chunk, self.shared_attention_blocks)
         if key not in choices:
-            few = starts[-1] <= max(self.FEW_TOKENS, getattr(ctx, "recordable_tokens", 0))
-            portions = [(end - start, 2 * (end - start) if few else length)
-                        for start, end, length in zip(starts, starts[1:], lengths)]
+            portions, _ = self._portions(ctx, starts, lengths)
             blocks = shared_blocks(portions, *heads[:3])
             if self.shared_attention_blocks is not None:
                 shared = blocks >= self.shared_attention_blocks
@@ -1014,8 +1078,9 @@ class PartsKernels:
             portions = singles < ctx.num_seqs
             singles = singles if plain else 0
             if portions:
+                plain_scores = not softcap and chunk is None and not keep_first and distance_bias is None and scale > 0
                 self._attend_portions(ctx, meta, (q, k_pages, v_pages, gates), gate_stride, gate_at, out, out_at, tail,
-                                      (q_heads, kv_heads, maps, dim, vdim), window, chunk, page_size, num_pages)
+                                      (q_heads, kv_heads, maps, dim, vdim), window, chunk, page_size, num_pages, plain_scores)
         if not singles:
             return
         # waves that share a token's head: by the most keys a row can see, fewer where the rows alone fill the device
@@ -1026,10 +1091,25 @@ class PartsKernels:
             self._code_of(q), _long(singles), q_heads, kv_heads, dim, vdim, page_size, _long(num_pages), *tail[:-5], row_waves,
             *tail[-5:]), "gated_attention")
 
-    def _attend_portions(self, ctx, meta, operands, gate_stride, gate_at, out, out_at, tail, heads, window, chunk, page_size, num_pages):
+    def _attend_portions(self, ctx, meta, operands, gate_stride, gate_at, out, out_at, tail, heads, window, chunk, page_size, num_pages,
+                         plain_scores=False):
         """The prompt portions of a step, which follow its single tokens, on the matrix cores."""
         first, (vectors, kv_heads, maps, dim, vdim) = ctx.num_decode_seqs, heads
         q, k_pages, v_pages, gates = map(_ptr, operands)
+        if plain_scores and self._takes_prompt_tiles(ctx, first, heads, window, page_size):
+            group = vectors // (kv_heads * maps)
+            heads_per_tile = min(group, 32)
+            head_groups, tokens_per_tile = (group + heads_per_tile - 1) // heads_per_tile, 32 // heads_per_tile
+            starts = ctx.host_q_start
+            tiles = sum((starts[r + 1] - starts[r] + 4 * tokens_per_tile - 1) // (4 * tokens_per_tile) for r in range(first, ctx.num_seqs))
+            self._dense(ctx.seq_lens, "seq_lens", torch.int32, (ctx.num_seqs,))
+            scale, _, _, window_or_none, sink, out_stride, out_scale, sink_logits = tail[:8]
+            self._check(self._attention_gated_entry(vdim)(
+                q, k_pages, v_pages, gates, _long(gate_stride), gate_at, _ptr(ctx.q_start), _ptr(ctx.seq_lens), _ptr(meta.block_table),
+                _ptr(meta.rows), meta.width, _ptr_at(out, out_at), first, ctx.num_seqs - first, tiles, vectors, kv_heads, maps,
+                heads_per_tile, head_groups, tokens_per_tile, page_size, _long(num_pages), scale, window_or_none, sink, sink_logits,
+                out_stride, out_scale, self._stream()), "gated_attention on prompt tiles")
+            return
         blocks, shared = self._shares_attention_keys(ctx, first, heads, window, chunk)
         if shared and dim <= 128 and vdim <= 128:
             self._dense(ctx.seq_lens, "seq_lens", torch.int32, (ctx.num_seqs,))

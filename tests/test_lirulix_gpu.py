@@ -296,6 +296,40 @@ def test_differential_attention_alone(hip, dtype, heads, kv_heads, dim, vdim, di
         assert error < (5e-5 if dtype == torch.float32 else 0.05), f"request {r}: {error:.2e}"
 
 
+@pytest.mark.parametrize("heads,kv_heads,dim,vdim,maps,page,window,sink,gated", [
+    (8, 2, 64, 64, 1, 16, None, "learned", False), (4, 4, 128, 128, 1, 32, 100, None, True), (3, 1, 128, 128, 1, 64, None, "zero", True),
+    (40, 1, 64, 64, 1, 16, 33, "learned", True), (4, 2, 64, 128, 2, 16, 130, None, False), (3, 3, 64, 128, 2, 32, None, "learned", False),
+    (36, 1, 64, 128, 2, 64, 40, "zero", False)])
+def test_gated_attention_on_prompt_tiles(hip, monkeypatch, heads, kv_heads, dim, vdim, maps, page, window, sink, gated):
+    """Portions of 1 to 300 tokens with and without a history on the plain prompt attention's tiles of 32 columns, their outputs columns
+    of wider rows, against the plain kernel on the same numbers in float32: an output is rounded once (2^-9 of it), a weight to two
+    bfloat16 numbers (2^-17 of it, of values of some units)."""
+    torch.manual_seed(heads + dim + maps)
+    befores, counts = [0, 70, 0, 513, 31], [129, 33, 2, 300, 97]
+    ctx = _ctx(befores, counts)
+    ctx.num_decode_seqs = 0
+    lengths = [b + c for b, c in zip(befores, counts)]
+    ctx.seq_lens = torch.tensor(lengths, dtype=torch.int32, device=DEVICE)
+    k_pages, v_pages, table = _pages_for(lengths, page, kv_heads, maps * dim, vdim, torch.bfloat16)
+    k_pages.normal_(), v_pages.normal_()
+    meta = SimpleNamespace(block_table=table.to(DEVICE), rows=None, width=table.shape[1])
+    q = (torch.randn(ctx.num_tokens, heads * maps * dim, device=DEVICE) * 2).bfloat16()
+    gates = torch.randn(ctx.num_tokens, heads + 5, device=DEVICE).bfloat16() if gated else None
+    sinks = torch.randn(heads * maps, device=DEVICE) * 3 if sink == "learned" else None
+    results = []
+    for dtype, tiles in ((torch.float32, False), (torch.bfloat16, True), (torch.bfloat16, False)):
+        monkeypatch.setattr(hip, "gated_prompt_tiles", tiles, raising=False)
+        out = torch.full((ctx.num_tokens, heads * maps * vdim + 12), 7.0, dtype=dtype, device=DEVICE)
+        hip.gated_attention(q.to(dtype), k_pages.to(dtype), v_pages.to(dtype), None if gates is None else gates.to(dtype), 5, ctx, meta, heads,
+                            kv_heads, dim, vdim, 1.3 / math.sqrt(dim), None, None, window, sink is not None, out, out_at=8, out_scale=0.7,
+                            sink_logits=sinks, maps=maps)
+        assert (out[:, :8] == 7.0).all() and (out[:, 8 + heads * maps * vdim:] == 7.0).all()
+        results.append(out[:, 8:8 + heads * maps * vdim].float())
+    want, got, other = results
+    assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -14 * 5).all()
+    assert not torch.equal(got, other)         # (else one kernel was compared with itself)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("heads,groups,dim,vdim,taps", [(4, 2, 24, 20, 4), (1, 1, 40, 8, 1), (6, 3, 8, 16, 2), (4, 4, 64, 64, 3),
                                                         (2, 1, 128, 128, 4), (2, 2, 300, 72, 2), (16, 16, 128, 128, 4)])
