@@ -372,6 +372,11 @@ class KernelSet:
         of `sums.rows`, every row divided by sqrt(its mean of squares + eps), the mean taken from `sums.sums`."""
         return False
 
+    def stacked_gate(self, matrix, rows: int, dtype):
+        """A stacked matrix [2 inter, k], gate before up, that was not packed as a gated pair, as what `gated_rows(x, weight, out)` and
+        `UnnormedRows.product` multiply and gate (silu) in one kernel, for a step of `rows` rows; or None."""
+        return None
+
     def norms_rows_in_product(self, rows: int, weight, dtype) -> bool:
         """`linear_scaled(stream, sums, norm_weight, eps, weight, out, bias=)` exists for this product."""
         return False
