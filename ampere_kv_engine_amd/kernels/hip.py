@@ -140,7 +140,7 @@ class HipKernels(PartsKernels, KernelSet):
         except OSError as error:
             raise KernelError(f"the kernel library {path} could not be loaded: {error}") from error
         self.library_path = path
-        self._attention_entry = {}      # head size -> entry point of that head size's attention library
+        self._attention_entry = {}      # ("library", head size) -> its attention library; (kind, head size) -> an entry point of it
         self._exchange_tiles, self._exchange_pieces, self._exchange_arrivals = 0, None, None
         self.decode_wave_target = 2048  # decode attention cuts the keys until about this many waves are at work,
         self.decode_min_segment = 128   # but into segments no shorter than this many keys (measured: 64 and 256 are slower)
@@ -970,36 +970,33 @@ class HipKernels(PartsKernels, KernelSet):
             ctypes.c_long(tokens), q_heads, kv_heads, head_dim, page_size, ctypes.c_long(num_pages), self._stream()),
             "qk_norm_rope_write")
 
-    def _attention_mfma_entry(self, head_dim: int):
-        if head_dim not in self._attention_entry:
+    def _attention_library(self, head_dim: int):
+        """The head size's library, looked for once (its sources are read to find the build that matches them)."""
+        key = ("library", head_dim)
+        if key not in self._attention_entry:
             path = ensure_attention(head_dim)
             try:
-                lib = ctypes.CDLL(path)
+                self._attention_entry[key] = ctypes.CDLL(path)
             except OSError as error:
                 raise KernelError(f"the attention library {path} could not be loaded: {error}") from error
-            entry = getattr(lib, f"akv_attention_mfma_d{head_dim}")
+        return self._attention_entry[key]
+
+    def _attention_function(self, kind: str, head_dim: int):
+        key = (kind, head_dim)
+        if key not in self._attention_entry:
+            entry = getattr(self._attention_library(head_dim), f"akv_attention_{kind}_d{head_dim}")
             entry.restype = ctypes.c_int
-            self._attention_entry[head_dim] = entry
-        return self._attention_entry[head_dim]
+            self._attention_entry[key] = entry
+        return self._attention_entry[key]
+
+    def _attention_mfma_entry(self, head_dim: int):
+        return self._attention_function("mfma", head_dim)
 
     def _attention_pair_entry(self, head_dim: int):
-        key = ("pair", head_dim)
-        if key not in self._attention_entry:
-            self._attention_mfma_entry(head_dim)            # (loads the head size's library)
-            lib = ctypes.CDLL(ensure_attention(head_dim))
-            entry = getattr(lib, f"akv_attention_pair_d{head_dim}")
-            entry.restype = ctypes.c_int
-            self._attention_entry[key] = entry
-        return self._attention_entry[key]
+        return self._attention_function("pair", head_dim)
 
     def _attention_gated_entry(self, head_dim: int):
-        key = ("gated", head_dim)
-        if key not in self._attention_entry:
-            self._attention_mfma_entry(head_dim)            # (loads the head size's library)
-            entry = getattr(ctypes.CDLL(ensure_attention(head_dim)), f"akv_attention_gated_d{head_dim}")
-            entry.restype = ctypes.c_int
-            self._attention_entry[key] = entry
-        return self._attention_entry[key]
+        return self._attention_function("gated", head_dim)
 
     def _pair_fits(self, ctx, decodes, q_heads, kv_heads, head_dim, page_size, fresh) -> bool:
         """Whether a step's single tokens and prompt portions can go into one launch: the single tokens' kernel takes

@@ -888,13 +888,11 @@ class PartsKernels:
 
     def _takes_prompt_tiles(self, ctx, first: int, heads: tuple[int, int, int, int, int], window, page_size: int) -> bool:
         """Whether the portions of a step, requests `first` on, go to the plain prompt attention's kernel on tiles of 32 columns.  It
-        takes keys and values of one width, 64 or 128, or two maps of 64 beside values of 128, on pages of 16, 32, 64 ...; it is taken
-        where some portion sees 448 keys and more and `prompt_tiles_time` lies below what the other two kernels are expected to take -
-        by a tenth in steps of few tokens, whose portions count as having as much before them as they bring (see
-        `_shares_attention_keys`)."""
+        takes what `_fits_prompt_tiles` says, and is taken where some portion sees 448 keys and more and `prompt_tiles_time` lies below
+        what the other two kernels are expected to take - by a tenth in steps of few tokens, whose portions count as having as much
+        before them as they bring (see `_shares_attention_keys`)."""
         vectors, kv_heads, maps, dim, vdim = heads
-        fits = (vdim in (64, 128) and dim == vdim and maps == 1) or (vdim == 128 and dim == 64 and maps == 2)
-        if (not fits or page_size < 16 or page_size & (page_size - 1) or self.shared_attention_blocks is not None
+        if (not self._fits_prompt_tiles(maps, dim, vdim, page_size) or self.shared_attention_blocks is not None
                 or getattr(ctx, "seq_lens", None) is None):        # (a step that names its requests' lengths on the host alone)
             return False
         if self.gated_prompt_tiles is not None:
@@ -941,6 +939,15 @@ class PartsKernels:
             self._refuse(f"q_heads {q_heads} is not a multiple of kv_heads {kv_heads}")
         if not 0 < vdim <= self.MAX_VALUE_DIM or not 0 < dim <= 2048:
             self._refuse(f"the attention takes values up to {self.MAX_VALUE_DIM} wide and keys up to 2048, not {vdim} and {dim}")
+        if any(self._fits_prompt_tiles(maps, dim, vdim, page_size) for maps in (1, 2)):
+            self._attention_gated_entry(vdim)       # (the library is found and loaded with the model, not by its first prompt)
+
+    @staticmethod
+    def _fits_prompt_tiles(maps: int, dim: int, vdim: int, page_size: int) -> bool:
+        """Whether the plain prompt attention's tiles take these heads: keys and values of 64 or 128, or two maps of 64 beside values of
+        128, on pages of 16, 32, 64 ..."""
+        fits = (vdim in (64, 128) and dim == vdim) if maps == 1 else (maps == 2 and vdim == 128 and dim == 64)
+        return fits and page_size >= 16 and page_size & (page_size - 1) == 0
 
     def _gated_pages(self, k_pages, v_pages, kv_heads, dim, vdim, dtype):
         self._dense(k_pages, "k_pages", dtype)
