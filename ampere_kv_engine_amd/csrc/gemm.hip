@@ -691,12 +691,12 @@ int launch_f32(const float* x, const float* w, float* y, int rows, int outs, int
     if (rows <= 16) return launch_f32_few_rows(x, w, y, rows, outs, k, bias, stream, Folded{});
     if (rows <= 32 && tiles <= units) return launch_f32_few<2>(x, w, y, rows, outs, k, bias, wide_stores, stream);
   }
-  // (The caller counts the grid's limit in tiles of 64 rows.  Where tiles of 32 would pass it they are not taken: by then tiles of 64
-  // are hundreds of rounds.)
+  // (The caller counts the grid's limit in tiles of 64 rows: where tiles of 32 would pass it they are not taken.)
+  const bool many = (rows + 31) / 32 > 65535;
   const long a = rounds(128, 64), b = rounds(64, 64), c = rounds(64, 32), d = rounds(32, 32);
   const long cost_a = 530 * a, cost_b = 295 * b, cost_c = c == 1 ? 210 : 182 * c + 10, cost_d = d == 1 ? 175 : 112 * d + 30;
-  if (cost_a <= cost_b && cost_a <= cost_c && cost_a <= cost_d) return launch_f32_wide<2, 4, 4, 2>(x, w, y, rows, outs, k, bias, wide_stores, stream);
-  if (cost_b <= cost_c && cost_b <= cost_d) return launch_f32_wide<1, 4, 4, 4>(x, w, y, rows, outs, k, bias, wide_stores, stream);
+  if (cost_a <= cost_b && (many || (cost_a <= cost_c && cost_a <= cost_d))) return launch_f32_wide<2, 4, 4, 2>(x, w, y, rows, outs, k, bias, wide_stores, stream);
+  if (many || (cost_b <= cost_c && cost_b <= cost_d)) return launch_f32_wide<1, 4, 4, 4>(x, w, y, rows, outs, k, bias, wide_stores, stream);
   if (cost_c <= cost_d) {
     if (c == 1) return launch_f32_wide<1, 2, 4, 4>(x, w, y, rows, outs, k, bias, wide_stores, stream);
     return launch_f32_wide<1, 2, 4, 2>(x, w, y, rows, outs, k, bias, wide_stores, stream);
