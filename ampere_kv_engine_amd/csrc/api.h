@@ -51,11 +51,8 @@ int akv_attention_f32(const float* q, const float* k_pages, const float* v_pages
 // Products y = x W^T (+ bias): `bias` [outs] float32 or null, added to the float32 sums before they are rounded.
 int akv_linear_tiled(const void* x, int x_dtype, const void* w, int w_dtype, void* y, int y_dtype, int rows, int outs,
                      int k, const float* bias, hipStream_t stream);
-// float32 products of up to 16 rows with the norm before them, the residual sum or the gate after them (see gemm.hip)
-int akv_linear_f32_folded(const float* x, const float* w, float* y, int rows, int outs, int k, const float* bias, int epilogue,
-                          const float* gain, float* left, float* squares, const float* scales, int groups, float eps,
-                          hipStream_t stream);
-int akv_linear_f32_groups(int rows, int outs, int k);
+// the gated float32 product of up to 16 rows (see gemm.hip)
+int akv_linear_f32_gated(const float* x, const float* w, float* y, int rows, int inter, int k, hipStream_t stream);
 int akv_linear_packed(const void* x, const void* wp, void* y, int y_dtype, int rows, int outs, int k, int n_tiles,
                       int k_tiles, int x_packed, const float* bias, hipStream_t stream);
 int akv_linear_packed_swiglu(const void* x, const void* wp, void* y, int y_dtype, int rows, int inter, int k,

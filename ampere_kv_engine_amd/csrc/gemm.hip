@@ -189,33 +189,21 @@ __device__ __forceinline__ floats4 settled(floats4 sums, const float* __restrict
   return sums;
 }
 
-// The sums of 16 outputs (4 g .. 4 g + 3 of them in this lane) for row `row`, with their bias, to y, or added to it - then also times
-// `gain` to `left`, where there is one; returns the sum of the squares of what y holds.
-template <bool ADDS = false>
-__device__ __forceinline__ float store_f32(float* __restrict__ y, long row, int out, int outs, floats4 sums,
-                                           const float* __restrict__ bias, bool wide_stores, const float* __restrict__ gain = nullptr,
-                                           float* __restrict__ left = nullptr) {
+// The sums of 16 outputs (4 g .. 4 g + 3 of them in this lane) for row `row`, with their bias, to y.
+__device__ __forceinline__ void store_f32(float* __restrict__ y, long row, int out, int outs, floats4 sums,
+                                          const float* __restrict__ bias, bool wide_stores) {
   if (bias != nullptr) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) sums[j] += bias[min(out + j, outs - 1)];
   }
   float* at = y + row * outs + out;
   if (wide_stores && out + 4 <= outs) {
-    if (ADDS) sums += *reinterpret_cast<floats4*>(at);
     *reinterpret_cast<floats4*>(at) = sums;
-    if (ADDS && left != nullptr) *reinterpret_cast<floats4*>(left + row * outs + out) = sums * *reinterpret_cast<const floats4*>(gain + out);
-    return ADDS ? sums[0] * sums[0] + sums[1] * sums[1] + sums[2] * sums[2] + sums[3] * sums[3] : 0.f;
+    return;
   }
-  float squares = 0.f;
 #pragma unroll
   for (int j = 0; j < 4; ++j)
-    if (out + j < outs) {
-      const float v = ADDS ? at[j] + sums[j] : sums[j];
-      at[j] = v;
-      if (ADDS) squares += v * v;
-      if (ADDS && left != nullptr) left[row * outs + out + j] = v * gain[out + j];
-    }
-  return squares;
+    if (out + j < outs) at[j] = sums[j];
 }
 
 __device__ __forceinline__ floats4 load_at(const char* from, uint32_t offset) {
@@ -223,31 +211,9 @@ __device__ __forceinline__ floats4 load_at(const char* from, uint32_t offset) {
   return *reinterpret_cast<const floats4*>(from + offset);
 }
 
-// What the kernels of few rows do beside the product (steps of up to 16 rows, where a launch costs as much as it does):
-//   kPlain    y = x W^T + bias
-//   kAdds     y += x W^T + bias: a branch's last product into the residual sum, every sum with one owner; where the weight of the
-//             norm that follows is known (`gain`), the new rows times it go to `left`, and the squares of a block's outputs, added
-//             up per row, to `squares` [blocks, 16]
-//   kSwiglu   y = silu(x Wgate^T) * (x Wup^T) of a matrix whose first half is the gate's: a block owns as many outputs of either half
-// and a product that reads rows left so (SCALES) divides its sums by the rows' root mean square, which follows from `squares` (the
-// division commutes with the product).  3 single tokens of a model of 8 layers, 2,048 wide: 87 launches 621 us, 64 launches 589;
-// 3 rows, us: 2048 x 2048 plain 7.2, added 7.4, 6144 x 2048 plain 12.3 and 4.6 for the gate's kernel, gated 13.2, a norm's kernel 4.3.
-// (A reader that meets the norm's weight and adds up the squares itself was slower than the norm's
-// kernel it saves: 3 rows of 6144 x 2048 12.3 -> 23 us, its waves' loads half as many again.)
-enum Epilogue { kPlain, kAdds, kSwiglu };
-
-// What a product of few rows does beside its sums.
-struct Folded {
-  Epilogue epilogue = kPlain;
-  const float* gain = nullptr;      // kAdds: the weight of the norm that follows, `left` [rows, outs], `squares` [blocks, 16]
-  float* left = nullptr;
-  float* squares = nullptr;
-  const float* scales = nullptr;    // the rows were left by such a product: its `squares`, `groups` blocks of them
-  int groups = 0;
-  float eps = 0.f;
-};
-constexpr int kAsked = 4;           // partial sums of squares that a lane asks for before anything else
-
+// GATED: y = silu(x Wgate^T) * (x Wup^T) of a matrix whose first half is the gate's, in steps of up to 16 rows, where a launch costs as
+// much as it does: a block owns as many outputs of either half and forms what the activation's kernel forms from the stored
+// product, the same bits (3 rows, us: 6144 x 2048 and the activation's kernel 12.3 + 4.6, gated 13.2).
 __device__ __forceinline__ float silu(float v) { return v / (1.f + expf(-v)); }
 
 // Up to 32 rows: the matrix is read once and its reads are what the product waits for.  A block owns 16 outputs and all of
@@ -255,24 +221,18 @@ __device__ __forceinline__ float silu(float v) { return v / (1.f + expf(-v)); }
 // a wave, 128 KB a block -, and leave their sums in LDS, where the first waves add them in order.  Rows lie in cache and
 // are read by every wave in operand order, without LDS, NT tiles of 16 rows - a single one before the weights (loads return in
 // order), so that it is split while those are on their way (1 row of 6144 x 2048: 13.8 -> 11.8 us).
-template <int NT, Epilogue E, bool SCALES>
+template <int NT, bool GATED>
 __global__ __launch_bounds__(1024) void linear_f32_few_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                              float* __restrict__ y, int rows, int outs, int k, int segments,
-                                                             const float* __restrict__ bias, bool wide_stores,
-                                                             const Folded folded) {
-  static_assert(NT == 1 || (E == kPlain && !SCALES), "");
-  extern __shared__ floats4 pieces[];                      // [waves][NT][64], then the sums of every fourth, then [waves][16] squares
+                                                             const float* __restrict__ bias, bool wide_stores) {
+  static_assert(NT == 1 || !GATED, "");
+  extern __shared__ floats4 pieces[];                      // [waves][NT][64], then the sums of every fourth
   floats4* total = pieces + (blockDim.x >> 6) * NT * 64;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
   const int r = lane & 15, g = lane >> 4;
-  constexpr int kOuts = E == kSwiglu ? 8 : 16;             // (of the result; with the gate's half of the matrix eight and eight)
+  constexpr int kOuts = GATED ? 8 : 16;                    // (of the result; with the gate's half of the matrix eight and eight)
   const int out0 = blockIdx.x * kOuts;
-  const float* wp = w + static_cast<long>(E == kSwiglu && r >= 8 ? outs + min(out0 + r - 8, outs - 1) : min(out0 + (E == kSwiglu ? r & 7 : r), outs - 1)) * k;
-  float asked[SCALES ? kAsked : 1];
-  if constexpr (SCALES) {
-#pragma unroll
-    for (int u = 0; u < kAsked; ++u) asked[u] = folded.scales[min((u * waves + wave) * 4 + g, folded.groups - 1) * 16 + r];
-  }
+  const float* wp = w + static_cast<long>(GATED && r >= 8 ? outs + min(out0 + r - 8, outs - 1) : min(out0 + (GATED ? r & 7 : r), outs - 1)) * k;
   const float* xp[NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t) xp[t] = x + static_cast<long>(min(16 * t + r, rows - 1)) * k;
@@ -325,26 +285,10 @@ __global__ __launch_bounds__(1024) void linear_f32_few_kernel(const float* __res
     if (wave < NT) add_fourths(total + wave * 64 + lane, pieces + wave * 64 + lane, waves, NT * 64, first == 0);
     __syncthreads();
   }
-  float* row_squares = reinterpret_cast<float*>(total + 4 * NT * 64);
-  if constexpr (SCALES) {
-    float squares = 0.f;
-#pragma unroll
-    for (int u = 0; u < kAsked; ++u) squares += (u * waves + wave) * 4 + g < folded.groups ? asked[u] : 0.f;
-    for (int n = (kAsked * waves + wave) * 4 + g; n < folded.groups; n += 4 * waves) squares += folded.scales[n * 16 + r];
-    squares += __shfl_xor(squares, 16, 64);
-    squares += __shfl_xor(squares, 32, 64);
-    if (lane < 16) row_squares[wave * 16 + r] = squares;
-    __syncthreads();
-  }
   // (a block has a multiple of four waves: the launch sees to it)
   if (wave >= NT) return;
   floats4 sums = settled(all_fourths(total + wave * 64 + lane, NT * 64), wp, x + static_cast<long>(min(16 * wave + r, rows - 1)) * k, k, g);
-  if constexpr (SCALES) {
-    float all = 0.f;
-    for (int n = 0; n < waves; ++n) all += row_squares[n * 16 + r];
-    sums *= rsqrtf(all / static_cast<float>(k) + folded.eps);
-  }
-  if constexpr (E == kSwiglu) {
+  if constexpr (GATED) {
     floats4 up;
 #pragma unroll
     for (int n = 0; n < 4; ++n) up[n] = __shfl_xor(sums[n], 32, 64);       // lane (row, g + 2)
@@ -352,13 +296,7 @@ __global__ __launch_bounds__(1024) void linear_f32_few_kernel(const float* __res
     for (int n = 0; n < 4; ++n) sums[n] = silu(sums[n]) * up[n];
     if (g >= 2) return;
   }
-  float of_block = 0.f;
-  if (16 * wave + r < rows) of_block = store_f32<E == kAdds>(y, 16 * wave + r, out0 + 4 * g, outs, sums, bias, wide_stores, folded.gain, folded.left);
-  if (E == kAdds && folded.squares != nullptr) {
-    of_block += __shfl_xor(of_block, 16, 64);
-    of_block += __shfl_xor(of_block, 32, 64);
-    if (lane < 16) folded.squares[blockIdx.x * 16 + r] = of_block;
-  }
+  if (16 * wave + r < rows) store_f32(y, 16 * wave + r, out0 + 4 * g, outs, sums, bias, wide_stores);
 }
 
 // Up to 8 rows: bound by what the units have on their way from memory; a block a tile of 16 outputs leaves half of them without
@@ -366,22 +304,17 @@ __global__ __launch_bounds__(1024) void linear_f32_few_kernel(const float* __res
 // and an instruction carries two segments of k - its rows 0 .. 7 the outputs' first and its rows 8 .. 15 their second, its
 // columns likewise the rows of x, so that two quarters of its sums are the two segments' and the others mean nothing (the matrix
 // cores have nothing else to do).  Each sum is the chain that the other kernels form, and the segments are added in their order.
-template <Epilogue E, bool SCALES>
+template <bool GATED>
 __global__ __launch_bounds__(1024) void linear_f32_pairs_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                                float* __restrict__ y, int rows, int outs, int k, int segments,
-                                                               const float* __restrict__ bias, bool wide_stores, const Folded folded) {
-  extern __shared__ floats4 pieces[];                      // [2 waves][16], then the sums of every fourth, then [waves][8] squares
+                                                               const float* __restrict__ bias, bool wide_stores) {
+  extern __shared__ floats4 pieces[];                      // [2 waves][16], then the sums of every fourth
   floats4* total = pieces + (blockDim.x >> 6) * 32;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
   const int r = lane & 7, second = lane >> 3 & 1, g = lane >> 4;
-  constexpr int kOuts = E == kSwiglu ? 4 : 8;              // (of the result; with the gate's half of the matrix four and four)
+  constexpr int kOuts = GATED ? 4 : 8;                     // (of the result; with the gate's half of the matrix four and four)
   const int out0 = blockIdx.x * kOuts;
-  const float* wp = w + static_cast<long>(E == kSwiglu && r >= 4 ? outs + min(out0 + r - 4, outs - 1) : min(out0 + (E == kSwiglu ? r & 3 : r), outs - 1)) * k;
-  float asked[SCALES ? kAsked : 1];
-  if constexpr (SCALES) {
-#pragma unroll
-    for (int u = 0; u < kAsked; ++u) asked[u] = folded.scales[min((u * waves + wave) * 8 + (lane >> 3), folded.groups - 1) * 16 + r];
-  }
+  const float* wp = w + static_cast<long>(GATED && r >= 4 ? outs + min(out0 + r - 4, outs - 1) : min(out0 + (GATED ? r & 3 : r), outs - 1)) * k;
   const float* xp = x + static_cast<long>(min(r, rows - 1)) * k;
   const floats4 zero = {0.f, 0.f, 0.f, 0.f};
   for (int first = 0; first < segments; first += 2 * waves) {
@@ -409,18 +342,6 @@ __global__ __launch_bounds__(1024) void linear_f32_pairs_kernel(const float* __r
     if (threadIdx.x < 16) add_fourths(total + threadIdx.x, pieces + threadIdx.x, 2 * waves, 16, first == 0);
     __syncthreads();
   }
-  float* row_squares = reinterpret_cast<float*>(total + 4 * 16);
-  if constexpr (SCALES) {
-    float squares = 0.f;
-#pragma unroll
-    for (int u = 0; u < kAsked; ++u) squares += (u * waves + wave) * 8 + (lane >> 3) < folded.groups ? asked[u] : 0.f;
-    for (int n = (kAsked * waves + wave) * 8 + (lane >> 3); n < folded.groups; n += 8 * waves) squares += folded.scales[n * 16 + r];
-    squares += __shfl_xor(squares, 8, 64);
-    squares += __shfl_xor(squares, 16, 64);
-    squares += __shfl_xor(squares, 32, 64);
-    if (lane < 8) row_squares[wave * 8 + r] = squares;
-    __syncthreads();
-  }
   if (wave > 0) return;
   floats4 sums = zero;                                     // (lanes 16 and more: zeros)
   if (lane < 16) sums = all_fourths(total + lane, 16) * kLowered;
@@ -432,24 +353,13 @@ __global__ __launch_bounds__(1024) void linear_f32_pairs_kernel(const float* __r
       sums[j] = finite(sums[j]) ? sums[j] : other;
     }
   }
-  if constexpr (SCALES) {
-    float all = 0.f;
-    for (int n = 0; n < waves; ++n) all += row_squares[n * 8 + r];
-    sums *= rsqrtf(all / static_cast<float>(k) + folded.eps);
-  }
-  if constexpr (E == kSwiglu) {
+  if constexpr (GATED) {
 #pragma unroll
     for (int n = 0; n < 4; ++n) sums[n] = silu(sums[n]) * __shfl_xor(sums[n], 8, 64);      // lane (row, second): the up's four
-    if (lane < 8 && r < rows) store_f32<false>(y, r, out0, outs, sums, bias, wide_stores);
+    if (lane < 8 && r < rows) store_f32(y, r, out0, outs, sums, bias, wide_stores);
     return;
   }
-  float of_block = 0.f;
-  if (lane < 16 && r < rows)
-    of_block = store_f32<E == kAdds>(y, r, out0 + 4 * second, outs, sums, bias, wide_stores && out0 + 8 <= outs, folded.gain, folded.left);
-  if (E == kAdds && folded.squares != nullptr) {
-    of_block += __shfl_xor(of_block, 8, 64);
-    if (lane < 8) folded.squares[blockIdx.x * 16 + r] = of_block;
-  }
+  if (lane < 16 && r < rows) store_f32(y, r, out0 + 4 * second, outs, sums, bias, wide_stores && out0 + 8 <= outs);
 }
 
 // More rows: a block has G groups of OW waves.  A wave owns 16 TM outputs by the block's 16 TN rows; a group takes every G-th
@@ -590,52 +500,25 @@ __global__ __launch_bounds__(64 * G * OW, TM * TN * OW > 16 ? 2 : 4) void linear
   }
 }
 
-template <int NT>
+template <int NT, bool GATED = false>
 int launch_f32_few(const float* x, const float* w, float* y, int rows, int outs, int k, const float* bias, bool wide_stores,
-                   hipStream_t stream, const Folded& folded = Folded{}) {
+                   hipStream_t stream) {
+  constexpr int kOuts = GATED ? 8 : 16;
   const int segments = (k + kSegment - 1) / kSegment, rounds = (segments + 15) / 16;
   const int waves = ((segments + rounds - 1) / rounds + 3) / 4 * 4;
-  const size_t lds = static_cast<size_t>(waves + 4) * NT * 64 * sizeof(floats4) + waves * 64;     // 41 KB at most
-#define AKV_FEW(E_, SCALES_) \
-  linear_f32_few_kernel<NT, E_, SCALES_><<<(outs + (E_ == kSwiglu ? 7 : 15)) / (E_ == kSwiglu ? 8 : 16), waves * 64, lds, stream>>>( \
-      x, w, y, rows, outs, k, segments, bias, wide_stores, folded)
-  if constexpr (NT == 1) {
-    if (folded.scales != nullptr) {
-      if (folded.epilogue == kSwiglu) AKV_FEW(kSwiglu, true);
-      else if (folded.epilogue == kAdds) return -2;
-      else AKV_FEW(kPlain, true);
-      return AKV_LAUNCH_STATUS();
-    }
-    if (folded.epilogue == kSwiglu) AKV_FEW(kSwiglu, false);
-    else if (folded.epilogue == kAdds) AKV_FEW(kAdds, false);
-    else AKV_FEW(kPlain, false);
-  } else {
-    AKV_FEW(kPlain, false);
-  }
-#undef AKV_FEW
+  const size_t lds = static_cast<size_t>(waves + 4) * NT * 64 * sizeof(floats4);     // 40 KB at most
+  linear_f32_few_kernel<NT, GATED><<<(outs + kOuts - 1) / kOuts, waves * 64, lds, stream>>>(x, w, y, rows, outs, k, segments, bias, wide_stores);
   return AKV_LAUNCH_STATUS();
 }
 
+template <bool GATED>
 int launch_f32_pairs(const float* x, const float* w, float* y, int rows, int outs, int k, const float* bias, bool wide_stores,
-                     hipStream_t stream, const Folded& folded = Folded{}) {
+                     hipStream_t stream) {
+  constexpr int kOuts = GATED ? 4 : 8;
   const int segments = (k + kSegment - 1) / kSegment, pairs = (segments + 1) / 2, rounds = (pairs + 15) / 16;
   const int waves = ((pairs + rounds - 1) / rounds + 1) / 2 * 2;
-#define AKV_PAIRS(E_, SCALES_) \
-  linear_f32_pairs_kernel<E_, SCALES_><<<(outs + (E_ == kSwiglu ? 3 : 7)) / (E_ == kSwiglu ? 4 : 8), waves * 64, \
-                                        (2 * waves + 4) * 16 * sizeof(floats4) + waves * 32, stream>>>( \
-      x, w, y, rows, outs, k, segments, bias, wide_stores, folded)
-  if (folded.scales != nullptr) {
-    if (folded.epilogue == kSwiglu) AKV_PAIRS(kSwiglu, true);
-    else if (folded.epilogue == kAdds) return -2;
-    else AKV_PAIRS(kPlain, true);
-  } else if (folded.epilogue == kSwiglu) {
-    AKV_PAIRS(kSwiglu, false);
-  } else if (folded.epilogue == kAdds) {
-    AKV_PAIRS(kAdds, false);
-  } else {
-    AKV_PAIRS(kPlain, false);
-  }
-#undef AKV_PAIRS
+  linear_f32_pairs_kernel<GATED><<<(outs + kOuts - 1) / kOuts, waves * 64, (2 * waves + 4) * 16 * sizeof(floats4), stream>>>(
+      x, w, y, rows, outs, k, segments, bias, wide_stores);
   return AKV_LAUNCH_STATUS();
 }
 
@@ -645,6 +528,20 @@ int launch_f32_wide(const float* x, const float* w, float* y, int rows, int outs
   dim3 grid((outs + 16 * TM * OW - 1) / (16 * TM * OW), (rows + 16 * TN - 1) / (16 * TN));
   linear_f32_wide_kernel<TM, TN, OW, G><<<grid, 64 * G * OW, 0, stream>>>(x, w, y, rows, outs, k, bias, wide_stores);
   return AKV_LAUNCH_STATUS();
+}
+
+// Whether up to 16 rows go to blocks of 8 outputs (pairs) rather than 16 (few): see `launch_f32`.
+bool takes_pairs(int rows, long outs, int k) {
+  const long units = device_facts().compute_units, tiles = (outs + 15) / 16;
+  return k > kSegment && (rows <= 4 || (rows <= 8 && ((outs + 7) / 8 <= units || tiles > units)));
+}
+
+// Up to 16 rows by blocks of few outputs; gated: `outs` of the result.
+template <bool GATED>
+int launch_f32_few_rows(const float* x, const float* w, float* y, int rows, int outs, int k, const float* bias, hipStream_t stream) {
+  const bool wide_stores = outs % 4 == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0;
+  if (takes_pairs(rows, GATED ? 2l * outs : outs, k)) return launch_f32_pairs<GATED>(x, w, y, rows, outs, k, bias, wide_stores, stream);
+  return launch_f32_few<1, GATED>(x, w, y, rows, outs, k, bias, wide_stores, stream);
 }
 
 // float32 operands whose rows are 16-byte aligned, k less than 2^24.  Which kernel takes a product is a matter of time alone (the bits
@@ -664,21 +561,6 @@ int launch_f32_wide(const float* x, const float* w, float* y, int rows, int outs
 // Up to 8 rows, blocks of 8 outputs (pairs) against blocks of 16 (few): 1 to 4 rows pairs (3 rows of 2048 x 3072: 8.3 / 12.2); from 5
 // on where they are one block a unit, or where blocks of 16 are several a unit (8 rows of 4096 x 12288 56 / 50, 3072 x 2048 10.4 /
 // 9.8).  Never where k is one segment: an instruction's second would be empty.
-// Whether up to 16 rows go to blocks of 8 outputs (pairs) rather than 16 (few): see `launch_f32`.
-bool takes_pairs(int rows, long outs, int k) {
-  const long units = device_facts().compute_units, tiles = (outs + 15) / 16;
-  return k > kSegment && (rows <= 4 || (rows <= 8 && ((outs + 7) / 8 <= units || tiles > units)));
-}
-
-int launch_f32_few_rows(const float* x, const float* w, float* y, int rows, int outs, int k, const float* bias, hipStream_t stream,
-                        const Folded& folded) {
-  const uintptr_t addresses = reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(folded.left) | reinterpret_cast<uintptr_t>(folded.gain);
-  const bool wide_stores = outs % 4 == 0 && addresses % 16 == 0;
-  if (takes_pairs(rows, folded.epilogue == kSwiglu ? 2l * outs : outs, k))
-    return launch_f32_pairs(x, w, y, rows, outs, k, bias, wide_stores, stream, folded);
-  return launch_f32_few<1>(x, w, y, rows, outs, k, bias, wide_stores, stream, folded);
-}
-
 int launch_f32(const float* x, const float* w, float* y, int rows, int outs, int k, const float* bias, hipStream_t stream) {
   const bool wide_stores = outs % 4 == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0;
   const long units = device_facts().compute_units;
@@ -688,7 +570,7 @@ int launch_f32(const float* x, const float* w, float* y, int rows, int outs, int
   };
   const long tiles = (outs + 15) / 16;
   if (rows <= 4 || tiles <= 4 * units) {
-    if (rows <= 16) return launch_f32_few_rows(x, w, y, rows, outs, k, bias, stream, Folded{});
+    if (rows <= 16) return launch_f32_few_rows<false>(x, w, y, rows, outs, k, bias, stream);
     if (rows <= 32 && tiles <= units) return launch_f32_few<2>(x, w, y, rows, outs, k, bias, wide_stores, stream);
   }
   // (The caller counts the grid's limit in tiles of 64 rows: where tiles of 32 would pass it they are not taken.)
@@ -727,31 +609,12 @@ extern "C" int akv_linear_tiled(const void* x, int x_dtype, const void* w, int w
   }
 }
 
-// float32 throughout, up to 16 rows, k a multiple of 4 below 2^24, x and w on 16-byte boundaries (else -2).  `epilogue` 0: y = x W^T +
-// bias; 1: y += that, and with `gain` [outs]: left [rows, outs] = y * gain, squares [akv_linear_f32_groups, 16] the sums of the squares
-// of y's new values per group of outputs and row; 2 (no bias): w [2 outs, k], y = silu(x W[:outs]^T) * (x W[outs:]^T).  `scales`
-// (epilogues 0 and 2): x are rows left so and `scales` [groups, 16] their squares: products are divided by sqrt(squares / k + eps).
-extern "C" int akv_linear_f32_folded(const float* x, const float* w, float* y, int rows, int outs, int k, const float* bias, int epilogue,
-                                     const float* gain, float* left, float* squares, const float* scales, int groups, float eps,
-                                     hipStream_t stream) {
-  if (rows <= 0 || outs <= 0) return 0;
-  if (rows > 16 || k <= 0 || k % 4 != 0 || k >= (1 << 24) || epilogue < kPlain || epilogue > kSwiglu ||
-      (epilogue == kAdds && scales != nullptr) || (epilogue == kSwiglu && bias != nullptr) || (scales != nullptr && groups <= 0) ||
-      (gain != nullptr && (epilogue != kAdds || left == nullptr || squares == nullptr)) ||
+// y [rows, inter] = silu(x W[:inter]^T) * (x W[inter:]^T), w [2 inter, k]: float32 throughout, up to 16 rows, k a multiple of 4 below
+// 2^24, x and w on 16-byte boundaries (else -2).
+extern "C" int akv_linear_f32_gated(const float* x, const float* w, float* y, int rows, int inter, int k, hipStream_t stream) {
+  if (rows <= 0 || inter <= 0) return 0;
+  if (rows > 16 || k <= 0 || k % 4 != 0 || k >= (1 << 24) || inter >= (1 << 30) ||
       (reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w)) % 16 != 0)
     return -2;
-  Folded folded;
-  folded.epilogue = static_cast<Epilogue>(epilogue);
-  if (gain != nullptr) {
-    folded.gain = gain;
-    folded.left = left;
-    folded.squares = squares;
-  }
-  folded.scales = scales;
-  folded.groups = groups;
-  folded.eps = eps;
-  return launch_f32_few_rows(x, w, y, rows, outs, k, bias, stream, folded);
+  return launch_f32_few_rows<true>(x, w, y, rows, inter, k, nullptr, stream);
 }
-
-// The groups of outputs whose squares `akv_linear_f32_folded` leaves.
-extern "C" int akv_linear_f32_groups(int rows, int outs, int k) { return takes_pairs(rows, outs, k) ? (outs + 7) / 8 : (outs + 15) / 16; }

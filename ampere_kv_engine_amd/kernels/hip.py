@@ -160,7 +160,7 @@ class HipKernels(PartsKernels, KernelSet):
         self.compute_units = torch.cuda.get_device_properties(self.device).multi_processor_count
         for name in ("akv_embed", "akv_add_rmsnorm", "akv_rmsnorm_rows", "akv_copy_rows", "akv_gather_rows",
                      "akv_swiglu", "akv_rope_table", "akv_rope", "akv_kv_write", "akv_qk_norm_rope_write",
-                     "akv_linear_tiled", "akv_linear_f32_folded", "akv_linear_f32_groups", "akv_linear_packed", "akv_linear_packed_swiglu", "akv_linear_packed_normed",
+                     "akv_linear_tiled", "akv_linear_f32_gated", "akv_linear_packed", "akv_linear_packed_swiglu", "akv_linear_packed_normed",
                      "akv_pack_rows", "akv_linear_packed_static", "akv_linear_mid", "akv_linear_mid_workspace",
                      "akv_linear_mid_adds", "akv_linear_mid_rowscaled", "akv_linear_mid_bands", "akv_linear_mid_most_groups",
                      "akv_linear_adds", "akv_linear_scaled", "akv_linear_adds_rows", "akv_linear_rowscaled",
@@ -572,8 +572,6 @@ class HipKernels(PartsKernels, KernelSet):
         (`add_to_stream`) and the next product take the norm upon itself: up to 16 rows it norms the rows from the
         sums left there (`linear_scaled`); up to 512 it reads rows that the adding product left multiplied by the
         norm's weight and divides its results by the rows' root mean square (`linear_rowscaled`)."""
-        if dtype == torch.float32:
-            return self.fold_norms and 0 < rows <= self.FOLD_NORM_ROWS and hidden % 4 == 0
         if dtype != torch.bfloat16 or hidden % 8 != 0:
             return False
         if 0 < rows <= self.FOLD_NORM_ROWS:     # (a product that norms its rows itself keeps them in LDS)
@@ -608,40 +606,26 @@ class HipKernels(PartsKernels, KernelSet):
         self.lib.akv_linear_decode_plan(row_tiles_per_wave, packed.n_tiles, packed.k_tiles, packed.k, normed_rows, may, out)
         return dict(k_split=out[0], waves=out[1], blocks=out[2], straddles=bool(out[3]), work_kb=out[4])
 
-    def _folds_float32(self, rows: int, weight, dtype) -> bool:
-        """Whether `akv_linear_f32_folded`'s kernels take this product: up to 16 float32 rows, a matrix that is read 16 bytes at a time."""
-        matrix = weight.stacked if isinstance(weight, StackedGate) else weight
-        return (isinstance(matrix, torch.Tensor) and matrix.dtype == dtype == torch.float32 and matrix.dim() == 2
-                and self.folds_norm(rows, matrix.shape[1], dtype) and matrix.shape[1] < 1 << 24 and matrix.data_ptr() % 16 == 0)
-
-    def _linear_folded(self, x, weight, out, epilogue: int, what: str, bias=None, leaves=(None, None, None), scales=None, eps=0.0) -> None:
-        matrix = weight.stacked if isinstance(weight, StackedGate) else weight
-        rows, k = x.shape
-        outs = out.shape[1]
-        self._dense(x, "x", torch.float32)
-        self._dense(matrix, "weight", torch.float32, ((2 if epilogue == 2 else 1) * outs, k))
-        self._dense(out, "out", torch.float32, (rows, outs))
-        gain, left, squares = leaves
-        if gain is not None:
-            self._dense(gain, "norm weight", torch.float32, (outs,))
-        if scales is not None:
-            self._dense(scales, "sums", torch.float32, (scales.shape[0], 16))
-        self._check(self.lib.akv_linear_f32_folded(
-            _ptr(x), _ptr(matrix), _ptr(out), rows, outs, k, _ptr(self._bias(bias, outs)), epilogue, _ptr(gain), _ptr(left), _ptr(squares),
-            _ptr(scales), scales.shape[0] if scales is not None else 0, ctypes.c_float(eps), self._stream()), what)
+    STACKED_GATE_ROWS = 16          # the most rows that `gated_rows` takes
 
     def stacked_gate(self, matrix, rows: int, dtype) -> "StackedGate | None":
-        """A stacked float32 matrix [2 inter, k] as what `gated_rows` and `linear_rowscaled` multiply and gate in one kernel, for a step
-        of so many rows, or None."""
-        return StackedGate(matrix) if self._folds_float32(rows, matrix, dtype) and matrix.shape[0] % 2 == 0 else None
+        """A stacked float32 matrix [2 inter, k] as what `gated_rows` multiplies and gates in one kernel, for a step of so many rows, or
+        None.  (Residual sum and norm stay with their own kernel: a float32 row has the same bits whatever stands beside it, and a
+        norm whose division came after the product would not have those of a larger step's.)"""
+        takes = (isinstance(matrix, torch.Tensor) and matrix.dtype == dtype == torch.float32 and matrix.dim() == 2 and matrix.is_contiguous()
+                 and 0 < rows <= self.STACKED_GATE_ROWS and matrix.shape[0] % 2 == 0 and matrix.shape[1] % 4 == 0
+                 and 0 < matrix.shape[1] < 1 << 24 and matrix.data_ptr() % 16 == 0)
+        return StackedGate(matrix) if takes else None
 
     def gated_rows(self, x, weight: "StackedGate", out) -> None:
         """out [rows, inter] = silu(x Wgate^T) * (x Wup^T): the product and the activation kernel's arithmetic in one launch."""
-        self._linear_folded(x, weight, out, 2, "gated_rows")
+        (rows, k), inter = x.shape, out.shape[1]
+        self._dense(x, "x", torch.float32)
+        self._dense(weight.stacked, "weight", torch.float32, (2 * inter, k))
+        self._dense(out, "out", torch.float32, (rows, inter))
+        self._check(self.lib.akv_linear_f32_gated(_ptr(x), _ptr(weight.stacked), _ptr(out), rows, inter, k, self._stream()), "gated_rows")
 
     def adds_to_stream(self, rows: int, weight, dtype, gain=None) -> bool:
-        if isinstance(weight, torch.Tensor):
-            return self._folds_float32(rows, weight, dtype)
         if not isinstance(weight, PackedWeight) or not self.folds_norm(rows, weight.outs, dtype):
             return False
         if rows <= self.FOLD_NORM_ROWS:
@@ -656,14 +640,6 @@ class HipKernels(PartsKernels, KernelSet):
         new rows times `gain` as well."""
         from ..parts.base import StreamSums
         rows = x.shape[0]
-        if isinstance(weight, torch.Tensor):    # float32
-            if gain is None:                    # (the model's end: its norm reads the residual sum)
-                self._linear_folded(x, weight, stream, 1, "add_to_stream", bias=bias)
-                return StreamSums(None)
-            sums = arena.take((self.lib.akv_linear_f32_groups(rows, weight.shape[0], weight.shape[1]), 16), torch.float32)
-            left = arena.take((rows, weight.shape[0]), torch.float32)
-            self._linear_folded(x, weight, stream, 1, "add_to_stream", bias=bias, leaves=(gain, left, sums))
-            return StreamSums(sums, rows=left, gain=gain)
         if rows <= self.FOLD_NORM_ROWS:
             sums = arena.take(((weight.outs + 15) // 16, 16), torch.float32)
             if gain is None or not self.fold_rows_left:
@@ -684,8 +660,6 @@ class HipKernels(PartsKernels, KernelSet):
         return StreamSums(sums, rows=left, gain=gain)
 
     def scales_rows_in_product(self, rows: int, weight, dtype, sums) -> bool:
-        if isinstance(weight, (torch.Tensor, StackedGate)):
-            return sums.rows is not None and sums.rows.dtype == torch.float32 and self._folds_float32(rows, weight, dtype)
         gated = isinstance(weight, GatedWeight)
         packed = weight.packed if gated else weight
         if not isinstance(packed, PackedWeight) or sums.rows is None or dtype != torch.bfloat16:
@@ -702,9 +676,6 @@ class HipKernels(PartsKernels, KernelSet):
         """out = (x W^T) with every row divided by sqrt(mean of squares + eps), plus `bias` (a `GatedWeight`: its
         gate of the scaled gate and up): x [rows, k] are rows that `add_to_stream` left - the residual sum times
         the norm's weight -, sums [groups, rows rounded up to 16] the partial sums of squares of the residual rows."""
-        if isinstance(weight, (torch.Tensor, StackedGate)):
-            self._linear_folded(x, weight, out, 2 if isinstance(weight, StackedGate) else 0, "linear_rowscaled", bias=bias, scales=sums, eps=eps)
-            return
         gated = isinstance(weight, GatedWeight)
         packed = weight.packed if gated else weight
         rows = x.shape[0]

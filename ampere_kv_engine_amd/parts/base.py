@@ -373,8 +373,8 @@ class KernelSet:
         return False
 
     def stacked_gate(self, matrix, rows: int, dtype):
-        """A stacked matrix [2 inter, k], gate before up, that was not packed as a gated pair, as what `gated_rows(x, weight, out)` and
-        `UnnormedRows.product` multiply and gate (silu) in one kernel, for a step of `rows` rows; or None."""
+        """A stacked matrix [2 inter, k], gate before up, that was not packed as a gated pair, as what `gated_rows(x, weight, out)`
+        multiplies and gates (silu) in one kernel, for a step of `rows` rows; or None."""
         return None
 
     def norms_rows_in_product(self, rows: int, weight, dtype) -> bool:

@@ -74,8 +74,7 @@ class SwiGLU(Part):
             self.rt.kernels.gated_linear(x, self.gated, act, scratch)
         elif self.activation == "silu" and (gate := self.rt.kernels.stacked_gate(self.gate_up.weight, tokens, self.rt.dtype)) is not None:
             # a few float32 rows: the stacked product gates its sums itself
-            if not (isinstance(x, UnnormedRows) and x.product(gate, act)):
-                self.rt.kernels.gated_rows(x.rows() if isinstance(x, UnnormedRows) else x, gate, act)
+            self.rt.kernels.gated_rows(x.rows() if isinstance(x, UnnormedRows) else x, gate, act)
         else:
             gate_up = ctx.arena.take((tokens, 2 * self.inter), self.rt.dtype)
             self.gate_up.forward(x, gate_up)

@@ -45,6 +45,39 @@ def test_cutting_with_the_norm_kernels_of_their_own(case, cutting):
     getattr(cases, "case_" + cutting)(engine, case)
 
 
+def test_float32_rows_have_the_same_bits_whatever_stands_beside_them():
+    """A request's float32 logits, bit for bit, as it decodes alone and among 3, 4, 7, 8, 15, 16 and 32 others - over the row counts where
+    the products change kernels and the gate leaves them (counted: a layer's gate is formed in its product up to 16 rows)."""
+    from ampere_kv_engine_amd.config import EngineConfig, Qwen3Config
+    from ampere_kv_engine_amd.engine import Engine, StepEntry
+    layers = 2
+    config = Qwen3Config.from_dict(dict(
+        architectures=["Qwen3ForCausalLM"], vocab_size=320, hidden_size=512, num_hidden_layers=layers, num_attention_heads=8,
+        num_key_value_heads=2, head_dim=64, intermediate_size=640, rope_theta=1000000.0, rms_norm_eps=1e-6, tie_word_embeddings=False))
+    engine = Engine.from_random(config, seed=3, engine_config=EngineConfig(
+        dtype="float32", page_size=16, num_pages=33 * 3, max_seqs=33, max_batched_tokens=256, max_seq_len=48, device="cuda:0"))
+    engine._recordable = False           # (a replayed step calls no Python)
+    gated, calls = engine.kernels.gated_rows, []
+    engine.kernels.gated_rows = lambda x, *args: (calls.append(x.shape[0]), gated(x, *args))
+    ids = torch.randint(0, 320, (33, 24), generator=torch.Generator().manual_seed(5)).tolist()
+    seen = []
+    for others in (0, 3, 4, 7, 8, 15, 16, 32):
+        seqs = [engine.open(f"r{i}") for i in range(others + 1)]
+        for seq, tokens in zip(seqs, ids):
+            engine.step([StepEntry(seq, tokens[:20 + (seq is not seqs[0])], [])])
+        rows = []
+        for place in (20, 21):
+            calls.clear()
+            logits = engine.step([StepEntry(seq, [tokens[place + (seq is not seqs[0])]], [0]) for seq, tokens in zip(seqs, ids)])
+            rows.append(logits[0].clone())
+            assert calls == ([others + 1] * layers if others < 16 else []), others
+        seen.append(torch.stack(rows))
+        for seq in seqs:
+            engine.close(seq)
+    for others, got in zip((3, 4, 7, 8, 15, 16, 32), seen[1:]):
+        assert torch.equal(got, seen[0]), f"{others} others: {int((got != seen[0]).sum())} logits differ"
+
+
 @pytest.mark.parametrize("cutting", ["whole", "mixed_with_pages_used_again"])
 def test_steps_of_many_rows_without_norm_kernels_and_with_them(case, cutting):
     """Steps of 17 to 512 bfloat16 rows run without norm kernels inside the layers too: a branch's last product (the

@@ -1103,53 +1103,24 @@ def test_float32_products_of_operands_without_parts(hip, rows):
 
 
 @pytest.mark.parametrize("outs,k", [(16, 4), (20, 132), (2048, 260), (102, 2048), (4104, 4300)])
-def test_float32_products_with_what_stands_beside_them(hip, outs, k):
-    """Up to 16 rows: the product added to the residual sum (which leaves its rows times the next norm's weight and their squares), the
-    gated one, and both readers of such rows - one and several rounds of segments, both kernels of few rows, outputs that end inside a
-    block, more partial sums of squares than a lane asks for at once - against the separate steps in float64.  A result passes
-    (min(k, 128) + chains + 1) roundings of 2^-24 sum |x w|, a scaled one eight more of it (weight, squares, root, division), and
-    silu's argument moves it by at most 1.1 of its own error."""
-    from types import SimpleNamespace
-    from ampere_kv_engine_amd.kernels.hip import StackedGate
-    w, both, gain, bias = (rand(*shape, seed=61 + i).cuda() for i, shape in enumerate(((outs, k), (2 * outs, k), (k,), (outs,))))
-    into = rand(k, 36, seed=66).cuda()                         # the product that leaves the rows
-    both *= 2.0 / k ** 0.5
-    arena = SimpleNamespace(take=lambda shape, dtype: torch.full(shape, float("nan"), dtype=dtype, device="cuda"))
+def test_float32_gated_products_of_few_rows(hip, outs, k):
+    """Up to 16 rows the product gates its own sums - one and several rounds of segments, both kernels of few rows, outputs that end inside
+    a block - against float64, and the same bits as the product followed by the activation kernel.  A sum passes
+    (min(k, 128) + chains + 1) roundings of 2^-24 sum |x w|, and silu's argument moves a result by at most 1.1 of its own error."""
+    both = rand(2 * outs, k, seed=62).cuda() * (2.0 / k ** 0.5)
+    steps = (min(k, 128) + (k + 127) // 128 + 1) * 2.0 ** -24
+    assert hip.stacked_gate(both, 17, torch.float32) is None
     for rows in (1, 3, 4, 5, 8, 9, 16):
-        steps = lambda k: (min(k, 128) + (k + 127) // 128 + 1) * 2.0 ** -24
-        reach = lambda a, m, more=0.0: (steps(a.shape[1]) + more) * (a.double().abs() @ m.double().abs().T)
-        assert hip.adds_to_stream(rows, into, torch.float32, gain) and not hip.adds_to_stream(17, into, torch.float32, gain)
-        a, x = rand(rows, 36, seed=67).cuda(), rand(rows, k, seed=68).cuda()
-        want = x.double() + a.double() @ into.double().T
-        end = x.clone()
-        left = hip.add_to_stream(a, into, x, arena, gain=gain)
-        assert ((x - want).abs() <= reach(a, into) + 2.0 ** -23 * want.abs()).all(), rows
-        assert torch.equal(left.rows, x * gain) and torch.allclose(left.sums[:, :rows].sum(0), x.square().sum(1), rtol=1e-5)
-        assert hip.add_to_stream(a, into, end, arena).sums is None and torch.equal(end, x)
-        y, before = rand(rows, outs, seed=69).cuda(), rand(rows, outs, seed=69).cuda()
-        hip.add_to_stream(x, w, y, arena, bias=bias)
-        want = before.double() + x.double() @ w.double().T + bias
-        assert ((y - want).abs() <= reach(x, w) + 2.0 ** -22 * (want.abs() + before.abs() + bias.abs())).all(), rows
-        normed = x.double() / (x.double().square().mean(1, keepdim=True) + 1e-5).sqrt() * gain.double()
-        out = torch.full((rows, outs), float("nan"), device="cuda")
-        assert hip.scales_rows_in_product(rows, w, torch.float32, left)
-        hip.linear_rowscaled(left.rows, left.sums, 1e-5, w, out, bias=bias)
-        want = normed @ w.double().T + bias
-        assert ((out - want).abs() <= reach(normed, w, 2.0 ** -21) + 2.0 ** -23 * (want.abs() + bias.abs())).all(), rows
-        for source, reader in ((x.double(), lambda: hip.gated_rows(x, StackedGate(both), out)),
-                               (normed, lambda: hip.linear_rowscaled(left.rows, left.sums, 1e-5, StackedGate(both), out))):
-            out.fill_(float("nan"))
-            reader()
-            gate, up = source @ both[:outs].double().T, source @ both[outs:].double().T
-            errors = reach(source, both, 2.0 ** -21)
-            want = gate * torch.sigmoid(gate) * up
-            allowed = 1.1 * errors[:, :outs] * up.abs() + errors[:, outs:] * gate.abs() + 2 * errors[:, :outs] * errors[:, outs:] + 2.0 ** -20 * want.abs()
-            assert ((out - want).abs() <= allowed).all(), rows
-        # (the same bits as the product followed by the activation kernel)
+        x, out = rand(rows, k, seed=68).cuda(), torch.full((rows, outs), float("nan"), device="cuda")
+        hip.gated_rows(x, hip.stacked_gate(both, rows, torch.float32), out)
+        gate, up = x.double() @ both[:outs].double().T, x.double() @ both[outs:].double().T
+        errors = steps * (x.double().abs() @ both.double().abs().T)
+        want = gate * torch.sigmoid(gate) * up
+        allowed = 1.1 * errors[:, :outs] * up.abs() + errors[:, outs:] * gate.abs() + 2 * errors[:, :outs] * errors[:, outs:] + 2.0 ** -20 * want.abs()
+        assert ((out - want).abs() <= allowed).all(), rows
         stacked, apart = torch.empty(rows, 2 * outs, device="cuda"), torch.empty(rows, outs, device="cuda")
         hip.linear(x, both, stacked)
         hip.swiglu(stacked, apart)
-        hip.gated_rows(x, StackedGate(both), out)
         assert torch.equal(out, apart), rows
 
 
