@@ -614,7 +614,7 @@ class HipKernels(PartsKernels, KernelSet):
         norm whose division came after the product would not have those of a larger step's.)"""
         takes = (isinstance(matrix, torch.Tensor) and matrix.dtype == dtype == torch.float32 and matrix.dim() == 2 and matrix.is_contiguous()
                  and 0 < rows <= self.STACKED_GATE_ROWS and matrix.shape[0] % 2 == 0 and matrix.shape[1] % 4 == 0
-                 and 0 < matrix.shape[1] < 1 << 24 and matrix.data_ptr() % 16 == 0)
+                 and matrix.shape[1] > 0 and matrix.data_ptr() % 16 == 0)
         return StackedGate(matrix) if takes else None
 
     def gated_rows(self, x, weight: "StackedGate", out) -> None:

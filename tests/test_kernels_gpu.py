@@ -1072,10 +1072,9 @@ def test_float32_products_on_the_matrix_cores(hip, outs, k):
 
 
 @pytest.mark.parametrize("rows", [2, 12, 30, 50, 333, 1000])     # (a kernel and a cut of k each)
-def test_float32_products_of_operands_without_parts(hip, rows):
-    """The products multiply operands as three bfloat16 numbers; what has none - infinities, numbers that bfloat16 rounds to
-    infinity - and sums beyond 2^80 take the float32 instruction, output by output: not a number and infinite where float64 says
-    so, finite elsewhere, and other outputs' bits as without them.  Tiny operands keep their last bits: the bound of the test above."""
+def test_float32_products_at_the_ends_of_the_range(hip, rows):
+    """Infinities, numbers near float32's largest and sums beyond it: not a number and infinite where float64 says so, finite elsewhere, and
+    other outputs' bits as without them.  Tiny and huge operands keep the bound of the test above."""
     outs, k = 200, 1100
     w, x = rand(outs, k, seed=41).cuda(), rand(rows, k, seed=42).cuda()
     clean = torch.empty(rows, outs, device="cuda")
@@ -1100,6 +1099,23 @@ def test_float32_products_of_operands_without_parts(hip, rows):
     untouched = torch.ones(rows, outs, dtype=torch.bool, device="cuda")
     untouched[:2], untouched[:, [5, 6, 7, 150]] = False, False
     assert torch.equal(y[untouched], clean[untouched])
+
+
+@pytest.mark.parametrize("rows", [2, 12, 30, 50, 333])           # (a kernel each)
+@pytest.mark.parametrize("terms", [1, 2, 3])
+def test_float32_products_of_a_few_terms(hip, rows, terms):
+    """Rows of one to three numbers that are not zero: a product is rounded once and every sum of them once, to nearest - no more than
+    `terms` times 2^-24 of sum |x w| in all - as a sum of float32 products is."""
+    outs, k = 1030, 2048
+    generator = torch.Generator().manual_seed(71 + terms)
+    w, x = rand(outs, k, seed=72).cuda(), torch.zeros(rows, k)
+    places = torch.rand(rows, k, generator=generator).argsort(1)[:, :terms]
+    x.scatter_(1, places, torch.randn(rows, terms, generator=generator))
+    x, y = x.cuda(), torch.empty(rows, outs, device="cuda")
+    hip.linear(x, w, y)
+    reach = terms * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+    error = (y.double() - x.double() @ w.double().T).abs()
+    assert (error <= reach).all(), float((error / reach).max()) * terms
 
 
 @pytest.mark.parametrize("outs,k", [(16, 4), (20, 132), (2048, 260), (102, 2048), (4104, 4300)])
