@@ -1140,6 +1140,19 @@ def test_float32_gated_products_of_few_rows(hip, outs, k):
         assert torch.equal(out, apart), rows
 
 
+def test_float32_gated_products_where_they_are_taken(hip):
+    """Up to four rows of wide matrices keep the activation's kernel; rows off a 16-byte boundary go to the plain product."""
+    most = 32 * hip.compute_units
+    for outs, rows, taken in ((most, 1, True), (most, 4, True), (most + 2, 4, False), (most + 2, 5, True), (most + 2, 16, True), (64, 0, False)):
+        assert (hip.stacked_gate(torch.empty(outs, 4, device="cuda"), rows, torch.float32) is not None) == taken, (outs, rows)
+    both, held = rand(40, 64, seed=73).cuda(), rand(3 * 64 + 1, seed=74).cuda()
+    x, out, stacked, apart = held[1:].view(3, 64), torch.empty(3, 20, device="cuda"), torch.empty(3, 40, device="cuda"), torch.empty(3, 20, device="cuda")
+    hip.gated_rows(x, hip.stacked_gate(both, 3, torch.float32), out)
+    hip.linear(x, both, stacked)
+    hip.swiglu(stacked, apart)
+    assert torch.equal(out, apart)
+
+
 def test_float32_product_of_rows_that_are_not_aligned(hip, ref):
     """A matrix that begins between 16-byte boundaries goes to the plain kernel."""
     x, w = rand(20, 64, seed=34).cuda(), rand(40 * 64 + 1, seed=35).cuda()[1:].view(40, 64)
