@@ -6,6 +6,7 @@ devices are checked on the host before a launch."""
 from __future__ import annotations
 
 import ctypes
+import warnings
 
 import torch
 
@@ -893,7 +894,8 @@ class PartsKernels:
         before them as they bring (see `_shares_attention_keys`)."""
         vectors, kv_heads, maps, dim, vdim = heads
         if (not self._fits_prompt_tiles(maps, dim, vdim, page_size) or self.shared_attention_blocks is not None
-                or getattr(ctx, "seq_lens", None) is None):        # (a step that names its requests' lengths on the host alone)
+                or getattr(ctx, "seq_lens", None) is None          # (a step that names its requests' lengths on the host alone)
+                or not self._has_prompt_tiles(vdim)):
             return False
         if self.gated_prompt_tiles is not None:
             return self.gated_prompt_tiles
@@ -939,8 +941,23 @@ class PartsKernels:
             self._refuse(f"q_heads {q_heads} is not a multiple of kv_heads {kv_heads}")
         if not 0 < vdim <= self.MAX_VALUE_DIM or not 0 < dim <= 2048:
             self._refuse(f"the attention takes values up to {self.MAX_VALUE_DIM} wide and keys up to 2048, not {vdim} and {dim}")
-        if any(self._fits_prompt_tiles(maps, dim, vdim, page_size) for maps in (1, 2)):
-            self._attention_gated_entry(vdim)       # (the library is found and loaded with the model, not by its first prompt)
+
+    def find_gated_attention(self, maps: int, dim: int, vdim: int, page_size: int, dtype) -> None:
+        if dtype == torch.bfloat16 and self._fits_prompt_tiles(maps, dim, vdim, page_size):
+            self._has_prompt_tiles(vdim)
+
+    def _has_prompt_tiles(self, vdim: int) -> bool:
+        """Whether the prompt tiles' library of this head size is there (or can be built here).  Where it is not, portions stay with the
+        kernels of the library that holds all other gated attention, and a warning says so."""
+        key = ("prompt tiles", vdim)
+        if key not in self._attention_entry:
+            try:
+                self._attention_gated_entry(vdim)
+                self._attention_entry[key] = True
+            except (RuntimeError, OSError) as error:
+                warnings.warn(f"gated attention goes without the prompt tiles of head size {vdim}: {error}")
+                self._attention_entry[key] = False
+        return self._attention_entry[key]
 
     @staticmethod
     def _fits_prompt_tiles(maps: int, dim: int, vdim: int, page_size: int) -> bool:

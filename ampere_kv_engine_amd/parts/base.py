@@ -377,6 +377,9 @@ class KernelSet:
         multiplies and gates (silu) in one kernel, for a step of `rows` rows; or None."""
         return None
 
+    def find_gated_attention(self, maps: int, dim: int, vdim: int, page_size: int, dtype) -> None:
+        """Called as a part with gated attention is built: what its kernels load is found then and not by the first prompt."""
+
     def norms_rows_in_product(self, rows: int, weight, dtype) -> bool:
         """`linear_scaled(stream, sums, norm_weight, eps, weight, out, bias=)` exists for this product."""
         return False

@@ -49,6 +49,7 @@ class DifferentialAttention(Part):
         self.out = Linear(runtime, self.o_size, [self.hidden], ["o"])
         self.lam = None
         runtime.kernels.check_gated_attention_sizes(self.q_heads * MAPS, self.kv_heads, self.dim, self.vdim, runtime.page_size)
+        runtime.kernels.find_gated_attention(MAPS, self.dim, self.vdim, runtime.page_size, runtime.dtype)
 
     def _prefix(self, prefix):
         return f"{prefix}{self.name}."

@@ -112,6 +112,7 @@ class GatedAttention(Part, SharesProducts):
         if self.learned_sink or self.has_bias or out_bias:
             self.inputs = None      # (a tensor of its own beside the products: side by side with others it runs by itself)
         runtime.kernels.check_gated_attention_sizes(self.q_heads, self.kv_heads, self.dim, self.vdim, runtime.page_size)
+        runtime.kernels.find_gated_attention(1, self.dim, self.vdim, runtime.page_size, runtime.dtype)
 
     def _prefix(self, prefix):
         return f"{prefix}{self.name}."

@@ -262,6 +262,34 @@ def test_an_engine_that_records_longer_portions_sends_them_the_same_way(allowed)
     assert turned == (allowed < 1025)
 
 
+def test_the_prompt_tiles_library_is_looked_for_by_bfloat16_engines_alone(monkeypatch):
+    """A gated attention of float32, or of heads that the tiles do not take, asks for no library of a head size; where a bfloat16 one has
+    none and none can be built, it says so once and its portions go to the other kernels."""
+    from types import SimpleNamespace
+    from ampere_kv_engine_amd.kernels import hip as module
+    asked = []
+
+    def absent(head_dim):
+        asked.append(head_dim)
+        raise RuntimeError("no compiler here")
+
+    monkeypatch.setattr(module, "ensure_attention", absent)
+    kernels = module.HipKernels.__new__(module.HipKernels)
+    kernels._attention_entry, kernels.compute_units = {}, 256
+    for dtype in (torch.float32, torch.bfloat16):
+        kernels.check_gated_attention_sizes(16, 4, 128, 128, 16)
+        kernels.find_gated_attention(1, 128, 128, 16, torch.float32)
+        kernels.find_gated_attention(1, 128, 64, 16, dtype)
+        kernels.find_gated_attention(1, 128, 128, 8, dtype)
+    assert not asked
+    with pytest.warns(UserWarning, match="no compiler here"):
+        kernels.find_gated_attention(1, 128, 128, 16, torch.bfloat16)
+    ctx = SimpleNamespace(num_seqs=1, host_q_start=[0, 2000], host_seq_lens=[2000], seq_lens=object())
+    assert not kernels._takes_prompt_tiles(ctx, 0, (16, 4, 1, 128, 128), None, 16) and asked == [128]
+    kernels._attention_entry[("prompt tiles", 128)] = True
+    assert kernels._takes_prompt_tiles(ctx, 0, (16, 4, 1, 128, 128), None, 16)
+
+
 def test_every_step_says_what_its_engine_may_record(engine, case):
     T.case_whole(engine, case)
     assert engine._last_step.recordable_tokens == engine.config.record_max_tokens
