@@ -77,7 +77,7 @@ def prompt_tiles_time(units: int, portions, vectors: int, kv_heads: int, maps: i
     start.  Fitted to, best of the other two / on these tiles, 256 units:
       128 / 128: 16 heads over 4, 64 tokens 6.5 / 10.5, 256 11.9 / 15.6, 512 20.5 / 20.8, 1,024 41 / 32, 2,000 76 / 53, 512 after 2,048 83 / 61,
         1,024 after 6,000 242 / 157, 4 x 500 30 / 22, 8 x 128 11.1 / 13.3, 2,000 in a window of 512 34 / 28, 1,024 26.0 / 25.8; 32 over 8,
-        2,000 84 / 63, 4 x 500 40 / 29;
+        2,000 84 / 63, 4 x 500 40 / 29 (expected to be slower here: the others keep it);
       64 / 128 in two maps, 16 over 4, a window of 1,024: 512 22.3 / 19.4, 1,024 40 / 31, 2,000 59 / 47, 1,024 after 6,000 51 / 37;
       64 / 64: 16 over 4, 512 14.4 / 15.0, 1,024 27 / 23, 2,000 60 / 39, 1,024 after 6,000 189 / 112; 16 over 16, 2,000 60 / 39."""
     reach = window if window is not None else 1 << 30

@@ -1123,12 +1123,13 @@ def test_float32_gated_products_of_few_rows(hip, outs, k):
     """Up to 16 rows the product gates its own sums - one and several rounds of segments, both kernels of few rows, outputs that end inside
     a block - against float64, and the same bits as the product followed by the activation kernel.  A sum passes
     (min(k, 128) + chains + 1) roundings of 2^-24 sum |x w|, and silu's argument moves a result by at most 1.1 of its own error."""
+    from ampere_kv_engine_amd.kernels.hip import StackedGate
     both = rand(2 * outs, k, seed=62).cuda() * (2.0 / k ** 0.5)
     steps = (min(k, 128) + (k + 127) // 128 + 1) * 2.0 ** -24
     assert hip.stacked_gate(both, 17, torch.float32) is None
     for rows in (1, 3, 4, 5, 8, 9, 16):
         x, out = rand(rows, k, seed=68).cuda(), torch.full((rows, outs), float("nan"), device="cuda")
-        hip.gated_rows(x, hip.stacked_gate(both, rows, torch.float32), out)
+        hip.gated_rows(x, StackedGate(both), out)                # (also where `stacked_gate` keeps the two kernels)
         gate, up = x.double() @ both[:outs].double().T, x.double() @ both[outs:].double().T
         errors = steps * (x.double().abs() @ both.double().abs().T)
         want = gate * torch.sigmoid(gate) * up

@@ -50,6 +50,38 @@ def test_cutting(engine, case, cutting):
 
 
 @pytest.mark.filterwarnings("ignore:a bfloat16 matrix")
+@pytest.mark.parametrize("page", [16, 32])
+def test_recorded_portions_on_prompt_tiles(page):
+    """Portions of 50 tokens, five in a row of one request beside another's single tokens, on the plain prompt attention's tiles: run as
+    they are, recorded and replayed - with eager steps of another engine in between - they have the bits of an engine that
+    records nothing (counted: three layers of five steps, and of the two that a recording engine's launches are called in)."""
+    from ampere_kv_engine_amd.config import EngineConfig, LirulixConfig
+    from ampere_kv_engine_amd.engine import Engine, StepEntry
+    raw = dict(architecture="Lirulix", vocab=200, width=64, norm=dict(eps=1e-6), layers=[
+        dict(type="attention", mixer=L.SINK(4, 2, 128, 128, 0.09, L.ROT(32, 1e4)), mlp=L.DENSE(64)),
+        dict(type="attention", mixer=L.SINK(6, 1, 64, 64, 0.125, L.ROT(64, 1e4), window=70), mlp=None),
+        dict(type="attention_2", mixer=L.DIFF(2, 1, 64, 128, 0.15, L.ROT(16, 1e4), 120, 0.25), mlp=L.DENSE(64))])
+    ids = torch.randint(0, 200, (2, 256), generator=torch.Generator().manual_seed(8)).tolist()
+    runs, calls = {}, {}
+    for graphs in (True, False):
+        engine = Engine.from_random(LirulixConfig.from_dict(raw), seed=4, engine_config=EngineConfig(
+            dtype="bfloat16", page_size=page, num_pages=2 * (288 // page), max_seqs=2, max_batched_tokens=128, max_seq_len=288, device=DEVICE,
+            decode_graphs=graphs))
+        kernels, calls[graphs] = engine.kernels, []
+        kernels.gated_prompt_tiles, entry = True, kernels._attention_gated_entry
+        kernels._attention_gated_entry = lambda vdim, entry=entry, met=calls[graphs]: (met.append(vdim), entry(vdim))[1]
+        runs[graphs] = engine, engine.open("long"), engine.open("single"), []
+    for step in range(5):
+        for engine, long, single, rows in runs.values():
+            logits = engine.step([StepEntry(long, ids[0][50 * step:50 * step + 50], [49]), StepEntry(single, [ids[1][step]], [0])])
+            rows.append(logits.clone())
+    assert any(graph is not None for graph in runs[True][0]._graphs.values()), "nothing was recorded"
+    assert calls == {True: [128, 64, 128] * 2, False: [128, 64, 128] * 5}
+    for step, (recorded, eager) in enumerate(zip(runs[True][-1], runs[False][-1])):
+        assert torch.equal(recorded, eager), step
+
+
+@pytest.mark.filterwarnings("ignore:a bfloat16 matrix")
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("mechanism", L.MECHANISMS)
 def test_one_mechanism_alone(mechanism, dtype, tmp_path):

@@ -619,6 +619,64 @@ def test_portions_that_share_their_keys_keep_clear_of_values_they_do_not_see(hip
         assert ((got - want).abs() <= reach).all(), (request, at)
 
 
+@pytest.mark.parametrize("poison", [float("inf"), float("-inf"), float("nan")])
+@pytest.mark.parametrize("heads,kv_heads,dim,vdim,maps,page,options", [
+    (4, 4, 64, 64, 1, 16, {}), (16, 4, 128, 128, 1, 32, dict(sink=True)), (40, 1, 64, 64, 1, 64, dict(window=40)),
+    (6, 2, 128, 128, 1, 16, dict(window=33, sink=True)), (4, 2, 64, 128, 2, 16, dict(window=40)), (3, 1, 64, 128, 2, 32, {}),
+    (2, 2, 64, 128, 2, 64, dict(window=70))])
+def test_portions_on_prompt_tiles_keep_clear_of_what_they_do_not_see(hip, monkeypatch, poison, heads, kv_heads, dim, vdim, maps, page, options):
+    """As above on the plain prompt attention's tiles: one dimension of a position's value is not finite - inside a portion, in its history,
+    the last position of a request -, and in every case keys and values of slots that no token sees are not finite at all: those
+    behind a request's last token in its last page, and those that lie behind every token's window."""
+    from torch_kernels import TorchKernels
+    torch.manual_seed(dim + heads)
+    befores, counts = [0, 170], [131, 90]
+    ctx = _ctx(befores, counts)
+    ctx.seq_lens = torch.tensor(ctx.host_seq_lens, dtype=torch.int32, device=DEVICE)
+    need = [(n + page - 1) // page for n in ctx.host_seq_lens]
+    order, table = torch.randperm(sum(need)).tolist(), torch.full((2, max(need)), -1, dtype=torch.int32)
+    for r, pages in enumerate(need):
+        table[r, :pages] = torch.tensor([order.pop() for _ in range(pages)])
+    k_pages = torch.randn(sum(need), kv_heads, page, maps * dim).bfloat16()
+    v_pages = torch.randn(sum(need), kv_heads, vdim, page).bfloat16()
+    vectors, tokens, window = heads * maps, ctx.num_tokens, options.get("window")
+    q = torch.randn(tokens, vectors * dim).bfloat16()
+
+    def through(kernels, device, keys, values, c):
+        out = torch.zeros(tokens, vectors * vdim, dtype=torch.bfloat16, device=device)
+        meta = SimpleNamespace(block_table=table.to(device), rows=None, width=table.shape[1])
+        kernels.gated_attention(q.to(device), keys.to(device), values.to(device), None, 0, c, meta, heads, kv_heads, dim, vdim, dim ** -0.5,
+                                None, None, window, options.get("sink", False), out, maps=maps)
+        return out.float().cpu().view(tokens, vectors, vdim)
+
+    host = SimpleNamespace(**{k: (v.cpu() if isinstance(v, torch.Tensor) else v) for k, v in vars(ctx).items()})
+    want = through(TorchKernels(), "cpu", k_pages, v_pages, host)
+    reach = want.abs() * 2.0 ** -7 + 2e-3
+    ctx.num_decode_seqs = 0
+    monkeypatch.setattr(hip, "gated_prompt_tiles", True, raising=False)
+    for r, length in enumerate(ctx.host_seq_lens):
+        unseen = list(range(length, need[r] * page))
+        if window is not None:
+            unseen += range(max(befores[r] - window + 1, 0))
+        for at in unseen:
+            k_pages[int(table[r, at // page]), :, at % page] = poison
+            v_pages[int(table[r, at // page]), :, :, at % page] = poison
+    for request, at in ((None, None), (0, 37), (0, 100), (0, 130), (1, 150), (1, 200), (1, 259)):
+        values, got = v_pages.clone(), None
+        sees = torch.zeros(tokens, dtype=torch.bool)
+        if request is not None:
+            values[int(table[request, at // page]), :, 3, at % page] = poison
+            pos = ctx.positions.cpu()
+            sees = (ctx.seq_of_token.cpu() == request) & (pos >= at)
+            if window is not None:
+                sees &= pos - at < window
+        got = through(hip, DEVICE, k_pages, values, ctx)
+        assert not torch.isfinite(got[sees][:, :, 3]).any(), (request, at)
+        got[sees, :, 3] = want[sees, :, 3]
+        assert torch.isfinite(got).all(), (request, at)
+        assert ((got - want).abs() <= reach).all(), (request, at)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("heads,dim,vdim,rot", [(2, 16, 12, 8), (1, 64, 32, 64), (3, 24, 40, 0), (2, 128, 128, 32), (1, 256, 256, 2)])
 def test_retention_kernel_alone(hip, dtype, heads, dim, vdim, rot):

@@ -262,6 +262,63 @@ def test_an_engine_that_records_longer_portions_sends_them_the_same_way(allowed)
     assert turned == (allowed < 1025)
 
 
+# us in the faster of those two kernels and on the plain prompt attention's tiles, and whether the tiles are taken: steps that may be
+# recorded (up to 512 tokens) are chosen as if as much lay before their portions as they bring, whatever does
+PROMPT_TILES_MEASURED = [
+    ((16, 4, 1, 128, 128, None), [(64, 0)], 6.5, 10.5, False), ((16, 4, 1, 128, 128, None), [(256, 0)], 11.9, 15.6, False),
+    ((16, 4, 1, 128, 128, None), [(512, 0)], 20.5, 20.8, False), ((16, 4, 1, 128, 128, None), [(1024, 0)], 41, 32, True),
+    ((16, 4, 1, 128, 128, None), [(2000, 0)], 76, 53, True), ((16, 4, 1, 128, 128, None), [(512, 2048)], 83, 61, False),
+    ((16, 4, 1, 128, 128, None), [(1024, 6000)], 242, 157, True), ((16, 4, 1, 128, 128, None), [(500, 0)] * 4, 30, 22, True),
+    ((16, 4, 1, 128, 128, None), [(128, 0)] * 8, 11.1, 13.3, False), ((16, 4, 1, 128, 128, 512), [(2000, 0)], 34, 28, True),
+    ((16, 4, 1, 128, 128, 512), [(1024, 0)], 26.0, 25.8, True), ((32, 8, 1, 128, 128, None), [(2000, 0)], 84, 63, True),
+    ((32, 8, 1, 128, 128, None), [(500, 0)] * 4, 40, 29, False), ((16, 4, 2, 64, 128, 1024), [(512, 0)], 22.3, 19.4, True),
+    ((16, 4, 2, 64, 128, 1024), [(1024, 0)], 40, 31, True), ((16, 4, 2, 64, 128, 1024), [(2000, 0)], 59, 47, True),
+    ((16, 4, 2, 64, 128, 1024), [(1024, 6000)], 51, 37, True), ((16, 4, 1, 64, 64, None), [(512, 0)], 14.4, 15.0, False),
+    ((16, 4, 1, 64, 64, None), [(1024, 0)], 27, 23, True), ((16, 4, 1, 64, 64, None), [(2000, 0)], 60, 39, True),
+    ((16, 4, 1, 64, 64, None), [(1024, 6000)], 189, 112, True), ((16, 16, 1, 64, 64, None), [(2000, 0)], 60, 39, True)]
+
+
+def _prompt_tiles_chosen(sizes, portions, lengths=None, allowed=0, singles=0):
+    from types import SimpleNamespace
+    from ampere_kv_engine_amd.kernels.hip import HipKernels
+    kernels = HipKernels.__new__(HipKernels)
+    kernels.compute_units, kernels._attention_entry = 256, {("prompt tiles", 64): True, ("prompt tiles", 128): True}
+    heads, kv_heads, maps, dim, vdim, window = sizes
+    starts = [0]
+    for count in [1] * singles + [count for count, _ in portions]:
+        starts.append(starts[-1] + count)
+    held = [9000] * singles + [before + count for count, before in portions] if lengths is None else lengths
+    ctx = SimpleNamespace(num_seqs=len(held), host_q_start=starts, host_seq_lens=held, seq_lens=object(), recordable_tokens=allowed)
+    chosen = kernels._takes_prompt_tiles(ctx, singles, (heads * maps, kv_heads, maps, dim, vdim), window, 16)
+    assert kernels._takes_prompt_tiles(ctx, singles, (heads * maps, kv_heads, maps, dim, vdim), window, 16) == chosen
+    return chosen
+
+
+@pytest.mark.parametrize("sizes,portions,others,tiles,taken", PROMPT_TILES_MEASURED)
+def test_portions_go_to_prompt_tiles_where_they_are_faster(sizes, portions, others, tiles, taken):
+    """The choice as it stands, never for the slower kernel of the two where the tiles are it; the order of requests, requests without
+    tokens and single tokens in front do not turn it."""
+    assert not taken or tiles <= others
+    for order in (portions, portions[::-1], portions + [(0, 0)], [(0, 5000)] + portions):
+        assert _prompt_tiles_chosen(sizes, order) == taken
+    if sum(count for count, _ in portions) > 512:
+        assert _prompt_tiles_chosen(sizes, portions, singles=3) == taken
+
+
+@pytest.mark.parametrize("allowed", [64, 512, 1024, 4096])
+def test_recorded_steps_go_to_prompt_tiles_as_they_go_unrecorded(allowed):
+    """Lengths - as they are, or bounds - do not turn the choice for a step that its engine may record; larger ones go by them."""
+    turned, seen = False, set()
+    for sizes in ((16, 4, 1, 128, 128, None), (16, 4, 2, 64, 128, 1024), (32, 8, 1, 64, 64, None)):
+        for tokens in (200, 511, 512, 513, 1000, 1025):
+            choices = {_prompt_tiles_chosen(sizes, [(tokens, 0)], lengths=[length], allowed=allowed)
+                       for length in (tokens, tokens + 300, 2048, 7000, 65536)}
+            seen |= choices
+            turned |= len(choices) > 1
+            assert len(choices) == 1 or tokens > max(allowed, 512)
+    assert seen == {False, True} and (turned or allowed > 64)
+
+
 def test_the_prompt_tiles_library_is_looked_for_by_bfloat16_engines_alone(monkeypatch):
     """A gated attention of float32, or of heads that the tiles do not take, asks for no library of a head size; where a bfloat16 one has
     none and none can be built, it says so once and its portions go to the other kernels."""
