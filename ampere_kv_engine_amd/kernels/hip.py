@@ -569,9 +569,10 @@ class HipKernels(PartsKernels, KernelSet):
 
     def folds_norm(self, rows: int, hidden: int, dtype) -> bool:
         """Whether a step of `rows` rows may let a branch's last product add itself to the residual sum
-        (`add_to_stream`) and the next product take the norm upon itself: up to 16 rows it norms the rows from the
-        sums left there (`linear_scaled`); up to 512 it reads rows that the adding product left multiplied by the
-        norm's weight and divides its results by the rows' root mean square (`linear_rowscaled`)."""
+        (`add_to_stream`) and the next product take the norm upon itself: it reads rows that the adding product left
+        multiplied by the norm's weight and divides its results by the rows' root mean square (`linear_rowscaled`); up to
+        16 rows, where that weight was not known or `fold_rows_left` is off, it norms the rows from the sums left there
+        (`linear_scaled`).  bfloat16 steps alone: in float32 a row has the same bits whatever stands beside it."""
         if dtype != torch.bfloat16 or hidden % 8 != 0:
             return False
         if 0 < rows <= self.FOLD_NORM_ROWS:     # (a product that norms its rows itself keeps them in LDS)
@@ -647,8 +648,8 @@ class HipKernels(PartsKernels, KernelSet):
 
     def add_to_stream(self, x, weight: PackedWeight, stream, arena, bias=None, gain=None):
         """stream [rows, outs] (float32) += bfloat16(x W^T (+ bias)) in place; returns what the product left for the
-        norm that follows (`StreamSums`): the rows' partial sums of squares, and in steps of more than 16 rows the
-        new rows times `gain` as well."""
+        norm that follows (`StreamSums`): the rows' partial sums of squares, and with `gain` - which steps of more than 16
+        rows need - the new rows times it as well."""
         from ..parts.base import StreamSums
         rows = x.shape[0]
         if rows <= self.FOLD_NORM_ROWS:

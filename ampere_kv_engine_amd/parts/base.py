@@ -321,8 +321,9 @@ class StreamSums:
     """What a branch hands on instead of its output when its last product has already added that output to the
     residual sum (`Linear.add_to_stream`): the partial sums of squares of the new residual rows, float32, from which
     the next norm's scale follows without a pass over the rows - `[ceil(width / 16), 16]` in steps of up to 16 rows,
-    `[groups, rows rounded up to 16]` in larger ones.  There the product leaves `rows` as well: the new residual
-    rows times `gain`, the weight of the norm that reads them, in the activation dtype - what is still missing
+    `[groups, rows rounded up to 16]` in larger ones.  Where it knows `gain`, the weight of the norm that reads them, the
+    product leaves `rows` as well (always in steps of more than 16 rows): the new residual
+    rows times `gain`, in the activation dtype - what is still missing
     from the normed rows is the division by each row's root mean square, which the reading product applies to its
     results (`KernelSet.scales_rows_in_product`)."""
 

@@ -132,7 +132,7 @@ class ScaledNorm(UnnormedRows):
 
     def product(self, weight, out: torch.Tensor, bias: torch.Tensor | None = None) -> bool:
         kernels = self.norm.rt.kernels
-        if self.sums.rows is not None:      # a step of many rows: the rows times this norm's weight are at hand
+        if self.sums.rows is not None:      # the rows times this norm's weight are at hand
             if self.sums.gain is not self.norm.weight or not kernels.scales_rows_in_product(self.shape[0], weight, out.dtype, self.sums):
                 return False
             self._once()
