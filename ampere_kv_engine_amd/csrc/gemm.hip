@@ -241,11 +241,16 @@ __global__ __launch_bounds__(1024) void linear_f32_pairs_kernel(const float* __r
 // More rows: tiles of 32 TM outputs by 32 TN rows, four waves of TM x TN tiles of 16 each, operands through two LDS buffers
 // of 32 k (row stride 36 floats: 16-byte reads of eight rows meet no bank twice), the next AHEAD steps of 32 k on their way in
 // registers.  Bound by the matrix cores where tiles fill the chip (8 TM TN instructions of 32 cycles a step and wave for
-// 2 (TM + TN) reads of 1 KB), and by the time a read takes where a unit holds one or two blocks, which is longer than a step:
-// 2048 outputs, k 2048 with 128 rows take 36.5 / 22.0 / 20.1 us with 1 / 2 / 4 steps on their way, k 6144 136 / 73 / 54, and
-// with 999 rows (tiles of 64 x 64) 85.5 / 85.1 / 83.9 and 251 / 244 / 242; 2048 rows of 12288 x 2048 949 / 916 / 918 (113
-// TFLOP/s).  Steps are a multiple of AHEAD, so that no register is copied at a loop's end: steps beyond k add zeros.
-template <int TM, int TN, int AHEAD>
+// 2 (TM + TN) reads of 1 KB), so a step is written in the order in which they never wait: either half of a step's 32 k is
+// read from LDS while the half before it is multiplied, the next step is filed between a half's instructions, and the one
+// barrier of a step stands between its halves - the reads behind it have the second half's time, those before it are long
+// there.  (Read where they are used and filed at the end, with the barrier after it, 999 rows of 2048 x 2048 / 6144 x 2048 /
+// 2048 x 3072 took 89 / 249 / 130 us instead of 73 / 217 / 109 with tiles of 64 x 64, 333 rows of 2048 x 2048 / 6144 x 2048 43 /
+// 117 instead of 33 / 93 with tiles of 32 x 32, 2048 rows of 6144 x 2048 488 instead of 416, 124 TFLOP/s.)  Where a unit holds one or
+// two blocks a read from memory takes longer than a step: 2048 outputs, k 2048 with 333 rows (64 x 64) take 61 / 43 / 41 us
+// with 1 / 2 / 4 steps on their way, with 999 rows 87 / 73 / 84.  Steps are a multiple of AHEAD, so that no register is copied
+// at a loop's end: steps beyond k add zeros.  ZEROS: k is no multiple of AHEAD steps, so some of what is filed counts as zeros.
+template <int TM, int TN, int AHEAD, bool ZEROS>
 __global__ __launch_bounds__(256) void linear_f32_wide_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                               float* __restrict__ y, int rows, int outs, int k,
                                                               const float* __restrict__ bias, bool wide_stores) {
@@ -276,7 +281,7 @@ __global__ __launch_bounds__(256) void linear_f32_wide_kernel(const float* __res
     for (int i = 0; i < TN; ++i) next_x[slot][i] = *reinterpret_cast<const floats4*>(xp[i] + at);
   };
   auto file = [&](int slot, int buffer, int k0) {
-    const bool inside = k0 + file_k < k;
+    const bool inside = !ZEROS || k0 + file_k < k;
 #pragma unroll
     for (int i = 0; i < TM; ++i)
       *reinterpret_cast<floats4*>(&ws[buffer][(file_row + 32 * i) * kStride + file_k]) = inside ? next_w[slot][i] : zero;
@@ -285,34 +290,49 @@ __global__ __launch_bounds__(256) void linear_f32_wide_kernel(const float* __res
       *reinterpret_cast<floats4*>(&xs[buffer][(file_row + 32 * i) * kStride + file_k]) = inside ? next_x[slot][i] : zero;
   };
   const int w_at = ((wave >> 1) * 16 * TM + r) * kStride + 4 * g, x_at = ((wave & 1) * 16 * TN + r) * kStride + 4 * g;
+  floats4 a[2][TM], v[2][TN];                              // the operands of either half of a step
+  auto read = [&](int half, int buffer) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i) a[half][i] = *reinterpret_cast<const floats4*>(&ws[buffer][w_at + 16 * i * kStride + 16 * half]);
+#pragma unroll
+    for (int j = 0; j < TN; ++j) v[half][j] = *reinterpret_cast<const floats4*>(&xs[buffer][x_at + 16 * j * kStride + 16 * half]);
+  };
+  auto multiply = [&](int half, int first, int last) {
+#pragma unroll
+    for (int e = first; e < last; ++e)
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+          sums[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[half][i][e], v[half][j][e], sums[i][j], 0, 0, 0);
+  };
   const int steps = (k + AHEAD * kDeep - 1) / (AHEAD * kDeep) * AHEAD;
   fetch(0, 0);
 #pragma unroll
   for (int i = 1; i < AHEAD; ++i) fetch(i, i * kDeep);
   file(0, 0, 0);
   __syncthreads();
+  read(0, 0);
   for (int first = 0; first < steps; first += AHEAD) {
 #pragma unroll
     for (int turn = 0; turn < AHEAD; ++turn) {
       const int step = first + turn;
       const int buffer = step & 1;
-      fetch(turn, (step + AHEAD) * kDeep);                 // (beyond k the last elements once more; they are filed as zeros)
-      __builtin_amdgcn_sched_barrier(0);                   // (else the loads are moved down to where they are filed)
-#pragma unroll
-      for (int b = 0; b < 2; ++b) {
-        floats4 a[TM], v[TN];
-#pragma unroll
-        for (int i = 0; i < TM; ++i) a[i] = *reinterpret_cast<const floats4*>(&ws[buffer][w_at + 16 * i * kStride + 16 * b]);
-#pragma unroll
-        for (int j = 0; j < TN; ++j) v[j] = *reinterpret_cast<const floats4*>(&xs[buffer][x_at + 16 * j * kStride + 16 * b]);
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-#pragma unroll
-          for (int i = 0; i < TM; ++i)
-#pragma unroll
-            for (int j = 0; j < TN; ++j)
-              sums[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i][e], v[j][e], sums[i][j], 0, 0, 0);
-      }
+      fetch(turn, (step + AHEAD) * kDeep);                 // (beyond k the last elements once more; they are filed as zeros or not multiplied)
+      __builtin_amdgcn_sched_barrier(0);                   // (left alone the compiler moves all of these to where they are used)
+      read(1, buffer);
+      __builtin_amdgcn_sched_barrier(0);
+      multiply(0, 0, 2);
+      __builtin_amdgcn_sched_barrier(0);
+      file((turn + 1) % AHEAD, buffer ^ 1, (step + 1) * kDeep);   // (read last before the barrier of the step before)
+      __builtin_amdgcn_sched_barrier(0);
+      multiply(0, 2, 4);
+      __builtin_amdgcn_sched_barrier(0);
+      __syncthreads();
+      read(0, buffer ^ 1);
+      __builtin_amdgcn_sched_barrier(0);
+      multiply(1, 0, 4);
+      __builtin_amdgcn_sched_barrier(0);
       if ((step & 3) == 3 || step + 1 == steps) {          // the end of a segment of 128
 #pragma unroll
         for (int i = 0; i < TM; ++i)
@@ -322,8 +342,6 @@ __global__ __launch_bounds__(256) void linear_f32_wide_kernel(const float* __res
             sums[i][j] = zero;
           }
       }
-      file((turn + 1) % AHEAD, buffer ^ 1, (step + 1) * kDeep);   // (read last before the barrier of the step before)
-      __syncthreads();
     }
   }
 #pragma unroll
@@ -362,10 +380,13 @@ template <int TM, int TN>
 int launch_f32_wide(const float* x, const float* w, float* y, int rows, int outs, int k, const float* bias, bool wide_stores,
                     hipStream_t stream) {
   dim3 grid((outs + 32 * TM - 1) / (32 * TM), (rows + 32 * TN - 1) / (32 * TN));
+  constexpr int kAhead = TM * TN == 4 ? 2 : 4;
   if (k <= 32)       // (one step: those that are asked for ahead would add zeros)
-    linear_f32_wide_kernel<TM, TN, 1><<<grid, 256, 0, stream>>>(x, w, y, rows, outs, k, bias, wide_stores);
+    linear_f32_wide_kernel<TM, TN, 1, true><<<grid, 256, 0, stream>>>(x, w, y, rows, outs, k, bias, wide_stores);
+  else if (k % (32 * kAhead) != 0)
+    linear_f32_wide_kernel<TM, TN, kAhead, true><<<grid, 256, 0, stream>>>(x, w, y, rows, outs, k, bias, wide_stores);
   else
-    linear_f32_wide_kernel<TM, TN, TM * TN == 4 ? 2 : 4><<<grid, 256, 0, stream>>>(x, w, y, rows, outs, k, bias, wide_stores);
+    linear_f32_wide_kernel<TM, TN, kAhead, false><<<grid, 256, 0, stream>>>(x, w, y, rows, outs, k, bias, wide_stores);
   return AKV_LAUNCH_STATUS();
 }
 
@@ -382,13 +403,13 @@ int launch_f32_few_rows(const float* x, const float* w, float* y, int rows, int 
 // float32 operands whose rows are 16-byte aligned.  Which kernel takes a product is a matter of time alone (the bits are the
 // same).  Measured, us, on weights that no cache holds (outs x k = 2048 x 2048 / 6144 x 2048 / 4096 x 12288 / 32768 x 2048;
 // tiles of outputs x rows):
-//     16 rows: few 9.8 / 20 / 59 / 74     32 x 32 19 / 20 / 102 / 90
-//     17 rows: few 12.4 / 26 / 73 / 86    32 x 32 19 / 20 / 101 / 87   (64 x 64 at 32768)
-//     64 rows: few 22 / 45 / 129 / -      32 x 32 20 / 28 / 101 / 114  32 x 64 30 / 30 / 160 / 92    64 x 64 48 / 48 / 273 / 92
-//    300 rows:                            32 x 32 39 / 90 / 338 / 498  32 x 64 47 / 84 / 362 / 409   64 x 64 48 / 84 / 478 / 390
-//    700 rows:                            32 x 32 68 / 184 / 708 / 1046  32 x 64 64 / 178 / 709 / 892  64 x 64 82 / 196 / 698 / 849
-//    999 rows:                            32 x 32 89 / 264 / 1025 / 1496 32 x 64 86 / 244 / 932 / 1291 64 x 64 85 / 237 / 920 / 1224
-// (110 TFLOP/s at best; the vector kernel above: 511 us on average over 999 rows of 2048 x 2048 and 2048 x 3072).  So: few
+//     16 rows: few 9.8 / 20 / 59 / 74     32 x 32 as with 17 rows
+//     17 rows: few 12.4 / 26 / 73 / 86    32 x 32 16 / 18 / 87 / 62       32 x 64 23 / 24 / 125 / 86     64 x 64 41 / 41 / 233 / 84
+//     64 rows: few 22 / 45 / 129 / -      32 x 32 16 / 25 / 91 / 115      32 x 64 23 / 25 / 125 / 92     64 x 64 41 / 42 / 233 / 89
+//    300 rows:                            32 x 32 33 / 84 / 314 / 519     32 x 64 40 / 86 / 321 / 400    64 x 64 41 / 84 / 422 / 364
+//    700 rows:                            32 x 32 62 / 191 / 675 / 1049   32 x 64 60 / 184 / 642 / 845   64 x 64 74 / 183 / 613 / 781
+//    999 rows:                            32 x 32 83 / 253 / 977 / 1483   32 x 64 86 / 239 / 862 / 1219  64 x 64 81 / 225 / 823 / 1122
+// (122 TFLOP/s at best; the vector kernel above: 511 us on average over 999 rows of 2048 x 2048 and 2048 x 3072).  So: few
 // rows stay with the kernels that read the matrix once, from 17 on only where blocks of 16 outputs are one a unit; tiles
 // are the kind whose busiest unit has the least to do - the blocks it gets times their area, a block of 32 x 64 taking 5 % and
 // one of 32 x 32 15 % longer for its area than one of 64 x 64.  (Tiles of 128 are slower everywhere: the matrix cores wait for

@@ -1071,6 +1071,21 @@ def test_float32_products_on_the_matrix_cores(hip, outs, k):
         assert torch.equal(y[0], alone[0]), rows
 
 
+@pytest.mark.parametrize("rows,outs", [(40, 130), (130, 6100), (70, 16500)])     # (tiles of 32 x 32, 32 x 64, 64 x 64)
+@pytest.mark.parametrize("k", [4, 32, 36, 64, 68, 96, 128, 192, 224, 256, 2112])
+def test_float32_tiles_where_their_steps_end(hip, rows, outs, k):
+    """Widths that are whole rings of steps (nothing is filed as zeros there), a step short of one, a step or four numbers beyond
+    one: every output's bits are those of the kernel that takes up to 16 rows, also where the last numbers are huge - what is
+    asked for beyond k counts for nothing."""
+    w, x = rand(outs, k, seed=51).cuda(), rand(rows, k, seed=52).cuda()
+    x[:, -4:] *= 2.0 ** 60
+    y, few = torch.full((rows, outs), float("nan"), device="cuda"), torch.empty(rows, outs, device="cuda")
+    hip.linear(x, w, y)
+    for start in range(0, rows, 16):
+        hip.linear(x[start:start + 16].contiguous(), w, few[start:start + 16])
+    assert torch.equal(y, few)
+
+
 @pytest.mark.parametrize("rows", [2, 12, 30, 50, 333, 1000])     # (a kernel and a cut of k each)
 def test_float32_products_at_the_ends_of_the_range(hip, rows):
     """Infinities, numbers near float32's largest and sums beyond it: not a number and infinite where float64 says so, finite elsewhere, and
