@@ -276,9 +276,10 @@ struct ItemLds {
 };
 
 enum Items : int { kNoItems, kPlanned, kWhole };     // (kWhole: a request is an item, whose result is the output)
-template <int NQ, bool SPLIT, bool PIPE, bool FRESH, bool ONCE, Items ITEMS>
+template <int NQ, bool SPLIT, bool PIPE, bool FRESH, bool ONCE, Items ITEMS, bool AHEAD>
 __device__ __forceinline__ void attention_mfma_body(const Args& a, const Where at, ItemLds* item_lds) {
   static_assert(ITEMS == kNoItems || (SPLIT && NQ == 1), "items are single tokens");
+  static_assert(!AHEAD || ITEMS != kNoItems, "");
   const int lane = at.lane, r16 = lane & 15, g = lane >> 4;
   auto from_pages = [](const char* at) {
     const uintx4* p = reinterpret_cast<const uintx4*>(at);
@@ -296,17 +297,17 @@ __device__ __forceinline__ void attention_mfma_body(const Args& a, const Where a
   int seg_lo = 0, seg_hi = 0x7fffffff;     // SPLIT: the keys of this block's segment
   long part = 0;                           // SPLIT: index of its partial result's tile
   if (SPLIT && (ITEMS == kWhole || a.plan != nullptr)) {   // item `by` of the plan: a request and a segment of its keys
-    const int item = at.by;
+    const int item = at.by, first_row = a.q_start[a.seq_first];
     int4 record;
     if constexpr (ITEMS == kWhole) {       // request `by`, all of its keys
       const int pos = a.seq_lens[a.seq_first + item] - 1;
       record = make_int4(item, a.window > 0 ? max(0, pos - a.window + 1) & ~31 : 0, pos, pos);
     } else {
+      record = *reinterpret_cast<const int4*>(a.plan + 132 + 4 * item);   // (asked for together with the number of items)
       if (item >= a.plan[0]) return;
-      record = *reinterpret_cast<const int4*>(a.plan + 132 + 4 * item);
     }
     t.request = a.seq_first + record.x;
-    t.first_row = a.q_start[a.seq_first] + record.x;   // one row per request
+    t.first_row = first_row + record.x;    // one row per request
     t.tokens = 1;
     t.first_pos = record.z;
     t.found = true;
@@ -328,9 +329,47 @@ __device__ __forceinline__ void attention_mfma_body(const Args& a, const Where a
     }
   }
   const int head_block = (SPLIT && (ITEMS == kWhole || a.plan != nullptr)) ? at.bx : at.by;  // (kv head, group of its query heads)
-  const int kvh = head_block / a.head_groups, hg = head_block % a.head_groups;
+  const int kvh = a.head_groups == 1 ? head_block : head_block / a.head_groups, hg = head_block - kvh * a.head_groups;
   const uintx4 zero = uintx4{0u, 0u, 0u, 0u};
   const int page_size = 1 << a.page_shift, page_mask = page_size - 1;
+
+  // keys this block looks at: every key any of its tokens may see, cut to its segment
+  const int last_pos = t.first_pos + t.tokens - 1;
+  int range_lo = a.window > 0 ? max(0, t.first_pos - a.window + 1) : 0;
+  int range_hi = last_pos;
+  if (SPLIT) {
+    range_lo = max(range_lo, seg_lo);
+    range_hi = min(range_hi, seg_hi);
+  }
+
+  const int* table = a.block_table + static_cast<long>(a.table_rows != nullptr ? a.table_rows[t.request] : t.request) * a.table_width;
+
+  // AHEAD (items; pages of 8 tokens and more): a wave has a step or a few, so what it waits for is one trip to memory after
+  // the other, and loads come back in the order they were asked for: an entry of the table asked for behind keys is
+  // there when they are.  So the entries of the 64 pages from the first step's on are asked for before anything else, one a
+  // lane, and handed round by shuffles; the first step's keys and values are asked for at once, before the queries are
+  // encoded, and every next step's before the products of the one before.  None of these loads stands behind a test
+  // (with one the compiler cannot count them and waits for all before the encoding): places outside the range
+  // are asked for at the nearest one inside, and what must count as zero is zeroed where it is used.  (A step of one
+  // request, 8 layers: 210 keys of 16 / 4 heads 363 -> 340 us, 2,048 keys of 32 / 8 heads 924 -> 895; the shuffles and the early
+  // loads with the tests left in gave nothing.)
+  int entries_first = 0, entries = 0;
+  auto ask_entries = [&](int base) {
+    entries_first = base >> a.page_shift;
+    entries = table[min(entries_first + lane, max(last_pos, 0) >> a.page_shift)];
+  };
+  const bool any_key = range_lo <= range_hi;       // (AHEAD: else the token's own position is asked for and not used)
+  const int near_lo = any_key ? range_lo : max(last_pos, 0), near_hi = any_key ? range_hi : max(last_pos, 0);
+  int new_entry = 0;                               // AHEAD: the entry of the token's own page
+  if constexpr (AHEAD) {
+    ask_entries(near_lo & ~31);
+    if constexpr (FRESH) new_entry = table[max(last_pos, 0) >> a.page_shift];
+  }
+  // the table's entry for a key of a step; AHEAD: all lanes call it together
+  auto page_of = [&](int key) {
+    if constexpr (AHEAD) return __shfl(entries, (key >> a.page_shift) - entries_first, 64);
+    else return table[key >> a.page_shift];
+  };
 
   // this lane's columns: one per NQ tile
   bool col_valid[NQ];
@@ -340,8 +379,10 @@ __device__ __forceinline__ void attention_mfma_body(const Args& a, const Where a
 #pragma unroll
   for (int nq = 0; nq < NQ; ++nq) {
     const int c = nq * 16 + r16;
-    const int token = c / a.heads_per_tile, head_in_group = hg * a.heads_per_tile + c % a.heads_per_tile;
-    col_valid[nq] = token < t.tokens && head_in_group < a.group;
+    // (items have one token: columns beyond its heads are nobody's)
+    const int token = ITEMS != kNoItems ? 0 : c / a.heads_per_tile;
+    const int head_in_group = hg * a.heads_per_tile + (ITEMS != kNoItems ? c : c % a.heads_per_tile);
+    col_valid[nq] = (ITEMS != kNoItems ? c < a.heads_per_tile : token < t.tokens) && head_in_group < a.group;
     col_pos[nq] = t.first_pos + token;
     col_low[nq] = a.window > 0 ? max(0, col_pos[nq] - a.window + 1) : 0;
     col_at[nq] = (static_cast<long>(t.first_row + token) * a.q_heads + kvh * a.group + head_in_group) * D;
@@ -368,15 +409,6 @@ __device__ __forceinline__ void attention_mfma_body(const Args& a, const Where a
     }
   }
 
-  // keys this block looks at: every key any of its tokens may see, cut to its segment
-  const int last_pos = t.first_pos + t.tokens - 1;
-  int range_lo = a.window > 0 ? max(0, t.first_pos - a.window + 1) : 0;
-  int range_hi = last_pos;
-  if (SPLIT) {
-    range_lo = max(range_lo, seg_lo);
-    range_hi = min(range_hi, seg_hi);
-  }
-
   float m[NQ], l[NQ];
   floatx4 o[NQ][DT];
 #pragma unroll
@@ -387,7 +419,6 @@ __device__ __forceinline__ void attention_mfma_body(const Args& a, const Where a
     for (int dt = 0; dt < DT; ++dt) o[nq][dt] = floatx4{0.f, 0.f, 0.f, 0.f};
   }
   bool poisoned = false;  // a key inside the range lies in a page that is not the request's
-  const int* table = a.block_table + static_cast<long>(a.table_rows != nullptr ? a.table_rows[t.request] : t.request) * a.table_width;
   const int key_in_step = (r16 >> 2) * 8 + (r16 & 3);  // + j * 4: this lane's key row of tile j
 
   // A page's byte offset is 64-bit (pools of many gigabytes); what is added inside a page fits 32 bits and is
@@ -430,7 +461,7 @@ __device__ __forceinline__ void attention_mfma_body(const Args& a, const Where a
     if (!owns_new) return;
     encode_head(knew, normed, a.eps, k_weights, rotated, head_angles);
     if (hg != 0) return;
-    const int page = table[new_pos >> a.page_shift];
+    const int page = AHEAD ? new_entry : table[new_pos >> a.page_shift];
     if (page < 0 || page >= a.num_pages) {
       poisoned = true;
       return;
@@ -458,7 +489,7 @@ __device__ __forceinline__ void attention_mfma_body(const Args& a, const Where a
       const bool wanted = !decltype(check)::value || (key >= range_lo && key <= range_hi);
       int page = 0;
       if (wanted) {
-        page = table[key >> a.page_shift];
+        page = page_of(key);
         if (page < 0 || page >= a.num_pages) {
           poisoned = true;
           page = 0;
@@ -477,7 +508,7 @@ __device__ __forceinline__ void attention_mfma_body(const Args& a, const Where a
   auto load_values = [&](int base, uintx4 (&dst)[DT], auto check) {
     const int key = base + g * 8;
     if (!decltype(check)::value && page_size >= 8) {
-      int page = table[key >> a.page_shift];
+      int page = page_of(key);
       if (page < 0 || page >= a.num_pages) {
         poisoned = true;
         page = 0;
@@ -497,7 +528,7 @@ __device__ __forceinline__ void attention_mfma_body(const Args& a, const Where a
         const int first = key + half * 4;
         if (half == 1 && (page_size >= 8 || live <= 4)) break;
         if (half == 0 && page_size < 8 && key + 3 < range_lo) continue;
-        const int page = table[first >> a.page_shift];
+        const int page = page_of(first);
         if (page < 0 || page >= a.num_pages) poisoned = true;
         else {
           have[half] = true;
@@ -529,13 +560,13 @@ __device__ __forceinline__ void attention_mfma_body(const Args& a, const Where a
     }
   };
 
-  uintx4 kreg[2][KT], knext[PIPE ? 2 : 1][PIPE ? KT : 1], vreg[DT];
+  uintx4 kreg[2][KT], knext[PIPE ? 2 : 1][PIPE ? KT : 1], vreg[DT], vnext[AHEAD ? DT : 1];
   const std::true_type checked{};
   const std::false_type unchecked{};
   auto inside = [&](int base) { return base >= range_lo && base + 31 <= range_hi; };
 
   // One step of 32 keys.  MASK: some column does not see the whole step (diagonal, window, segment edge).
-  auto step = [&](int base, const uintx4 (&kreg)[2][KT], auto mask) {
+  auto step = [&](int base, const uintx4 (&kreg)[2][KT], const uintx4 (&values)[DT], auto mask) {
     // ---- S^T = K . Q^T for two tiles of 16 keys --------------------------------------------------------------
     floatx4 s[NQ][2];
 #pragma unroll
@@ -602,7 +633,70 @@ __device__ __forceinline__ void attention_mfma_body(const Args& a, const Where a
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-      for (int nq = 0; nq < NQ; ++nq) o[nq][dt] = mfma16(vreg[dt], plow[nq], mfma16(vreg[dt], preg[nq], o[nq][dt]));
+      for (int nq = 0; nq < NQ; ++nq) o[nq][dt] = mfma16(values[dt], plow[nq], mfma16(values[dt], preg[nq], o[nq][dt]));
+  };
+
+  // AHEAD: keys and values of the step at `base`, and what of them counts as zero (before they are used).
+  auto load_step = [&](int base, uintx4 (&keys)[2][KT], uintx4 (&values)[DT]) {
+    auto page_at = [&](int key) {
+      const int page = page_of(key);
+      const bool known = page >= 0 && page < a.num_pages;
+      poisoned = poisoned || !known;
+      return static_cast<size_t>(known ? page : 0) * page_bytes;
+    };
+    size_t k_at[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int key = min(max(base + key_in_step + j * 4, near_lo), near_hi);
+      k_at[j] = page_at(key) + (k_lane + static_cast<uint32_t>(key & page_mask) * (D * 2u));
+    }
+    const int run = min(max(base + g * 8, near_lo & ~7), near_hi & ~7);
+    const size_t v_at = page_at(run) + (v_lane + static_cast<uint32_t>(run & page_mask) * 2u);
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int kt = 0; kt < KT; ++kt)      // (beyond the head: its first dims, zeroed below)
+        keys[j][kt] = from_pages(k_bytes + (k_at[j] + kt * 64u - ((D % 32 == 0 || kt * 32 + g * 8 < D) ? 0u : kt * 64u + g * 16u)));
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) values[dt] = from_pages(v_bytes + v_at + dt * v_tile);
+  };
+  auto zero_outside = [&](int base, uintx4 (&keys)[2][KT], uintx4 (&values)[DT]) {
+    if constexpr (D % 32 != 0) {
+      if ((KT - 1) * 32 + g * 8 >= D) keys[0][KT - 1] = keys[1][KT - 1] = zero;
+    }
+    if (inside(base)) return;              // (scores of keys outside the range are set, whatever the keys hold)
+    const int key = base + g * 8, live = key + 7 >= range_lo ? min(8, range_hi - key + 1) : 0;
+    uint32_t keep[4];
+#pragma unroll
+    for (int w = 0; w < 4; ++w) keep[w] = live >= 2 * w + 2 ? 0xffffffffu : (live == 2 * w + 1 ? 0x0000ffffu : 0u);
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) values[dt] = uintx4{values[dt].x & keep[0], values[dt].y & keep[1], values[dt].z & keep[2], values[dt].w & keep[3]};
+  };
+  // the new key and value take the place of what the page holds
+  auto place_new = [&](int base, uintx4 (&cur)[2][KT], uintx4 (&values)[DT]) {
+    if (owns_new && base == (new_pos & ~31)) {
+      const int at = new_pos - base;
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        if (key_in_step + j * 4 == at) {
+#pragma unroll
+          for (int kt = 0; kt < KT; ++kt) cur[j][kt] = knew[kt];
+        }
+      if (g == (at >> 3)) {
+        const int word = (at & 7) >> 1, shift = (at & 1) * 16;
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+          for (int w = 0; w < 4; ++w)
+            if (w == word) values[dt][w] = (values[dt][w] & ~(0xffffu << shift)) | (vnew[dt] << shift);
+      }
+    }
+  };
+  auto compute = [&](int base, bool here, const uintx4 (&cur)[2][KT], const uintx4 (&values)[DT]) {
+    // every valid column sees the whole step: below the diagonal, inside window and segment
+    const bool whole = here && base + 31 <= t.first_pos && (a.window == 0 || base >= last_pos - a.window + 1);
+    if (whole) step(base, cur, values, unchecked);
+    else step(base, cur, values, checked);
   };
 
   // One turn: fetch this step's values and (PIPE) the next step's keys, then compute the step on `cur`.
@@ -621,32 +715,29 @@ __device__ __forceinline__ void attention_mfma_body(const Args& a, const Where a
         else load_keys(base + 32, next, checked);
       }
     }
-    if constexpr (FRESH) {
-      if (owns_new && base == (new_pos & ~31)) {  // the new key and value take the place of what the page holds
-        const int at = new_pos - base;
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-          if (key_in_step + j * 4 == at) {
-#pragma unroll
-            for (int kt = 0; kt < KT; ++kt) cur[j][kt] = knew[kt];
-          }
-        if (g == (at >> 3)) {
-          const int word = (at & 7) >> 1, shift = (at & 1) * 16;
-#pragma unroll
-          for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-            for (int w = 0; w < 4; ++w)
-              if (w == word) vreg[dt][w] = (vreg[dt][w] & ~(0xffffu << shift)) | (vnew[dt] << shift);
-        }
-      }
-    }
-    // every valid column sees the whole step: below the diagonal, inside window and segment
-    const bool whole = here && base + 31 <= t.first_pos && (a.window == 0 || base >= last_pos - a.window + 1);
-    if (whole) step(base, cur, unchecked);
-    else step(base, cur, checked);
+    if constexpr (FRESH) place_new(base, cur, vreg);
+    compute(base, here, cur, vreg);
+  };
+  // AHEAD: keys and values of the next step, then this one
+  auto turn_ahead = [&](int base, uintx4 (&cur)[2][KT], uintx4 (&values)[DT], uintx4 (&next)[2][KT], uintx4 (&next_values)[DT]) {
+    if ((min(base + 63, near_hi) >> a.page_shift) - entries_first > 63) ask_entries(base + 32);
+    load_step(base + 32, next, next_values);
+    __builtin_amdgcn_sched_barrier(0);
+    zero_outside(base, cur, values);
+    if constexpr (FRESH) place_new(base, cur, values);
+    compute(base, inside(base), cur, values);
   };
   const int first_base = range_lo & ~31;
-  if constexpr (PIPE) {
+  if constexpr (AHEAD) {
+    load_step(first_base, kreg, vreg);
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (FRESH) encode_fresh();  // while the first keys and values are on their way
+    for (int base = first_base; base <= range_hi; base += 64) {  // two turns: the registers swap roles
+      turn_ahead(base, kreg, vreg, knext, vnext);
+      if (base + 32 > range_hi) break;
+      turn_ahead(base + 32, knext, vnext, kreg, vreg);
+    }
+  } else if constexpr (PIPE) {
     if (first_base <= range_hi) {
       if (inside(first_base)) load_keys(first_base, kreg, unchecked);
       else load_keys(first_base, kreg, checked);
@@ -739,17 +830,17 @@ __device__ __forceinline__ void attention_mfma_body(const Args& a, const Where a
 
 template <int NQ, bool SPLIT, bool PIPE, bool FRESH, bool ONCE>
 __global__ __launch_bounds__(64, (SPLIT && NQ == 1 && D <= 128) ? 2 : 1) void attention_mfma_kernel(const Args a) {
-  attention_mfma_body<NQ, SPLIT, PIPE, FRESH, ONCE, kNoItems>(
+  attention_mfma_body<NQ, SPLIT, PIPE, FRESH, ONCE, kNoItems, false>(
       a, Where{static_cast<int>(blockIdx.x), static_cast<int>(blockIdx.y), static_cast<int>(blockIdx.z),
                static_cast<int>(gridDim.x), static_cast<int>(gridDim.y), static_cast<int>(threadIdx.x), 0}, nullptr);
 }
 
 // Items of a plan, or requests: block (head block, item).
-template <bool FRESH, bool ONCE, Items ITEMS>
-__global__ __launch_bounds__(64 * kItemWaves, D <= 128 ? 2 : 1) void attention_items_kernel(const Args a) {
+template <bool FRESH, bool ONCE, Items ITEMS, bool AHEAD>
+__global__ __launch_bounds__(64 * kItemWaves, D <= 128 && ITEMS != kWhole ? 2 : 1) void attention_items_kernel(const Args a) {
   __shared__ __align__(16) ItemLds lds;
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
-  attention_mfma_body<1, true, true, FRESH, ONCE, ITEMS>(
+  attention_mfma_body<1, true, true, FRESH, ONCE, ITEMS, AHEAD>(
       a, Where{static_cast<int>(blockIdx.x), static_cast<int>(blockIdx.y), 0, static_cast<int>(gridDim.x),
                static_cast<int>(gridDim.y), static_cast<int>(threadIdx.x) & 63, wave}, &lds);
 }
@@ -1710,7 +1801,7 @@ __global__ __launch_bounds__(64 * kSharedWaves, 2) void attention_pair_kernel(co
       const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
       const int unit = (static_cast<int>(blockIdx.x) - portion_blocks) * kSharedWaves + wave;
       if (unit >= gx * gy) return;
-      attention_mfma_body<1, true, true, true, ONCE, kNoItems>(
+      attention_mfma_body<1, true, true, true, ONCE, kNoItems, false>(
           single, Where{unit % gx, unit / gx, 0, gx, gy, static_cast<int>(threadIdx.x) & 63, 0}, nullptr);
     }
   }
@@ -1834,11 +1925,17 @@ __global__ __launch_bounds__(64 * kMergeWaves) void attention_merge_kernel(const
     if (lane + e * 64 < D) dst[lane + e * 64] = from_float<bf16_t>(acc[e] * inv);
 }
 
+template <bool FRESH, bool AHEAD>
+void launch_items(const Args& a, dim3 grid, bool once, bool whole, hipStream_t stream) {
+  if (whole) attention_items_kernel<FRESH, false, kWhole, AHEAD><<<grid, 64 * kItemWaves, 0, stream>>>(a);   // (few keys: not marked)
+  else if (once) attention_items_kernel<FRESH, true, kPlanned, AHEAD><<<grid, 64 * kItemWaves, 0, stream>>>(a);
+  else attention_items_kernel<FRESH, false, kPlanned, AHEAD><<<grid, 64 * kItemWaves, 0, stream>>>(a);
+}
+
 template <bool FRESH>
 void launch_items(const Args& a, dim3 grid, bool once, bool whole, hipStream_t stream) {
-  if (whole) attention_items_kernel<FRESH, false, kWhole><<<grid, 64 * kItemWaves, 0, stream>>>(a);   // (few keys: not marked)
-  else if (once) attention_items_kernel<FRESH, true, kPlanned><<<grid, 64 * kItemWaves, 0, stream>>>(a);
-  else attention_items_kernel<FRESH, false, kPlanned><<<grid, 64 * kItemWaves, 0, stream>>>(a);
+  if (a.page_shift >= 3) launch_items<FRESH, true>(a, grid, once, whole, stream);
+  else launch_items<FRESH, false>(a, grid, once, whole, stream);       // (pages of 4: eight keys of a value row in two pieces)
 }
 
 template <int NQ>
