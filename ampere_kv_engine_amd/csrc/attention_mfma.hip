@@ -279,7 +279,8 @@ enum Items : int { kNoItems, kPlanned, kWhole };     // (kWhole: a request is an
 template <int NQ, bool SPLIT, bool PIPE, bool FRESH, bool ONCE, Items ITEMS, bool AHEAD>
 __device__ __forceinline__ void attention_mfma_body(const Args& a, const Where at, ItemLds* item_lds) {
   static_assert(ITEMS == kNoItems || (SPLIT && NQ == 1), "items are single tokens");
-  static_assert(!AHEAD || ITEMS != kNoItems, "");
+  constexpr bool kSingle = ITEMS != kNoItems || FRESH;   // every request brings one token
+  static_assert(!AHEAD || (SPLIT && kSingle && NQ == 1), "");
   const int lane = at.lane, r16 = lane & 15, g = lane >> 4;
   auto from_pages = [](const char* at) {
     const uintx4* p = reinterpret_cast<const uintx4*>(at);
@@ -344,7 +345,7 @@ __device__ __forceinline__ void attention_mfma_body(const Args& a, const Where a
 
   const int* table = a.block_table + static_cast<long>(a.table_rows != nullptr ? a.table_rows[t.request] : t.request) * a.table_width;
 
-  // AHEAD (items; pages of 8 tokens and more): a wave has a step or a few, so what it waits for is one trip to memory after
+  // AHEAD (items and raw single tokens; pages of 8 tokens and more): a wave has a step or a few, so what it waits for is one trip to memory after
   // the other, and loads come back in the order they were asked for: an entry of the table asked for behind keys is
   // there when they are.  So the entries of the 64 pages from the first step's on are asked for before anything else, one a
   // lane, and handed round by shuffles; the first step's keys and values are asked for at once, before the queries are
@@ -352,7 +353,8 @@ __device__ __forceinline__ void attention_mfma_body(const Args& a, const Where a
   // (with one the compiler cannot count them and waits for all before the encoding): places outside the range
   // are asked for at the nearest one inside, and what must count as zero is zeroed where it is used.  (A step of one
   // request, 8 layers: 210 keys of 16 / 4 heads 363 -> 340 us, 2,048 keys of 32 / 8 heads 924 -> 895; the shuffles and the early
-  // loads with the tests left in gave nothing.)
+  // loads with the tests left in gave nothing.  Waves alone on their segments, 8, 64 and 27 uneven requests: 1,261 -> 1,251, 1,978 ->
+  // 1,961, 1,655 -> 1,605; 171 tokens beside 8 requests 2,361 -> 2,315.)
   int entries_first = 0, entries = 0;
   auto ask_entries = [&](int base) {
     entries_first = base >> a.page_shift;
@@ -379,10 +381,10 @@ __device__ __forceinline__ void attention_mfma_body(const Args& a, const Where a
 #pragma unroll
   for (int nq = 0; nq < NQ; ++nq) {
     const int c = nq * 16 + r16;
-    // (items have one token: columns beyond its heads are nobody's)
-    const int token = ITEMS != kNoItems ? 0 : c / a.heads_per_tile;
-    const int head_in_group = hg * a.heads_per_tile + (ITEMS != kNoItems ? c : c % a.heads_per_tile);
-    col_valid[nq] = (ITEMS != kNoItems ? c < a.heads_per_tile : token < t.tokens) && head_in_group < a.group;
+    // (a single token: columns beyond its heads are nobody's)
+    const int token = kSingle ? 0 : c / a.heads_per_tile;
+    const int head_in_group = hg * a.heads_per_tile + (kSingle ? c : c % a.heads_per_tile);
+    col_valid[nq] = (kSingle ? c < a.heads_per_tile : token < t.tokens) && head_in_group < a.group;
     col_pos[nq] = t.first_pos + token;
     col_low[nq] = a.window > 0 ? max(0, col_pos[nq] - a.window + 1) : 0;
     col_at[nq] = (static_cast<long>(t.first_row + token) * a.q_heads + kvh * a.group + head_in_group) * D;
@@ -828,9 +830,9 @@ __device__ __forceinline__ void attention_mfma_body(const Args& a, const Where a
   }  // pass
 }
 
-template <int NQ, bool SPLIT, bool PIPE, bool FRESH, bool ONCE>
+template <int NQ, bool SPLIT, bool PIPE, bool FRESH, bool ONCE, bool AHEAD>
 __global__ __launch_bounds__(64, (SPLIT && NQ == 1 && D <= 128) ? 2 : 1) void attention_mfma_kernel(const Args a) {
-  attention_mfma_body<NQ, SPLIT, PIPE, FRESH, ONCE, kNoItems, false>(
+  attention_mfma_body<NQ, SPLIT, PIPE, FRESH, ONCE, kNoItems, AHEAD>(
       a, Where{static_cast<int>(blockIdx.x), static_cast<int>(blockIdx.y), static_cast<int>(blockIdx.z),
                static_cast<int>(gridDim.x), static_cast<int>(gridDim.y), static_cast<int>(threadIdx.x), 0}, nullptr);
 }
@@ -1801,7 +1803,7 @@ __global__ __launch_bounds__(64 * kSharedWaves, 2) void attention_pair_kernel(co
       const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
       const int unit = (static_cast<int>(blockIdx.x) - portion_blocks) * kSharedWaves + wave;
       if (unit >= gx * gy) return;
-      attention_mfma_body<1, true, true, true, ONCE, kNoItems, false>(
+      attention_mfma_body<1, true, true, true, ONCE, kNoItems, true>(
           single, Where{unit % gx, unit / gx, 0, gx, gy, static_cast<int>(threadIdx.x) & 63, 0}, nullptr);
     }
   }
@@ -1974,11 +1976,16 @@ int launch(const Args& a, int tiles, bool shared, int waves_per_item, hipStream_
         launch_items<true>(a, grid, once, whole, stream);
         if (!whole) merge();
       } else if (items || a.num_splits > 1) {
-        if (once) attention_mfma_kernel<NQ, true, true, true, true><<<grid, 64, 0, stream>>>(a);
-        else attention_mfma_kernel<NQ, true, true, true, false><<<grid, 64, 0, stream>>>(a);
+        if (a.page_shift >= 3) {
+          if (once) attention_mfma_kernel<NQ, true, true, true, true, true><<<grid, 64, 0, stream>>>(a);
+          else attention_mfma_kernel<NQ, true, true, true, false, true><<<grid, 64, 0, stream>>>(a);
+        } else {                             // (pages of 4: eight keys of a value row in two pieces)
+          if (once) attention_mfma_kernel<NQ, true, true, true, true, false><<<grid, 64, 0, stream>>>(a);
+          else attention_mfma_kernel<NQ, true, true, true, false, false><<<grid, 64, 0, stream>>>(a);
+        }
         merge();
       } else {
-        attention_mfma_kernel<NQ, false, true, true, false><<<grid, 64, 0, stream>>>(a);
+        attention_mfma_kernel<NQ, false, true, true, false, false><<<grid, 64, 0, stream>>>(a);
       }
       return AKV_LAUNCH_STATUS();
     } else {
@@ -1993,11 +2000,11 @@ int launch(const Args& a, int tiles, bool shared, int waves_per_item, hipStream_
       return -2;
     }
   } else if (items || a.num_splits > 1) {
-    if (once) attention_mfma_kernel<NQ, true, true, false, true><<<grid, 64, 0, stream>>>(a);
-    else attention_mfma_kernel<NQ, true, true, false, false><<<grid, 64, 0, stream>>>(a);
+    if (once) attention_mfma_kernel<NQ, true, true, false, true, false><<<grid, 64, 0, stream>>>(a);
+    else attention_mfma_kernel<NQ, true, true, false, false, false><<<grid, 64, 0, stream>>>(a);
     merge();
   } else {
-    attention_mfma_kernel<NQ, false, true, false, false><<<grid, 64, 0, stream>>>(a);
+    attention_mfma_kernel<NQ, false, true, false, false, false><<<grid, 64, 0, stream>>>(a);
   }
   return AKV_LAUNCH_STATUS();
 }

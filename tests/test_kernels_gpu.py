@@ -1872,10 +1872,13 @@ def test_encode_and_attend_single_tokens(hip, ref, q_heads, kv_heads, dim, page_
 @pytest.mark.parametrize("dim,page_size", [(128, 8), (64, 16), (128, 4)])
 @pytest.mark.parametrize("histories", [[4090], [2047, 2048, 2049, 0], [9000, 33, 5]])
 @pytest.mark.parametrize("window", [None, 3000])
-def test_encode_and_attend_where_a_wave_walks_many_pages(hip, ref, monkeypatch, dim, page_size, histories, window):
+@pytest.mark.parametrize("alone", [False, True])
+def test_encode_and_attend_where_a_wave_walks_many_pages(hip, ref, monkeypatch, dim, page_size, histories, window, alone):
     """A request is one item, so a wave's keys lie in more pages than it has lanes to hold their table entries: the entries are
     asked for again on the way; the token's own page is beyond the first of them."""
     monkeypatch.setattr(hip, "decode_wave_target", 1)
+    if alone:
+        monkeypatch.setattr(type(hip), "_share_segments", staticmethod(lambda seq_count, head_blocks: False))
     _check_encode_and_attend(hip, ref, 8, 2, dim, page_size, [(h, 1) for h in histories], window, len(histories))
 
 
