@@ -108,6 +108,24 @@ __device__ __forceinline__ unsigned arrive(unsigned* counter) {
   return before;
 }
 
+// Division of 0 <= x < 2^31 by a number that the host knows: one product and a shift where the compiler's own division is some
+// forty instructions one after the other.  With s the smallest number for which 2^s >= by and magic = ceil(2^(31 + s) / by) - at
+// most 2^32 - 1 for by > 1 - magic * by exceeds 2^(31 + s) by less than by <= 2^s, so x * magic / 2^(31 + s) exceeds x / by by less than
+// x / (2^31 by) < 1 / by and its whole part is the quotient.  (by = 1: magic 2^31, shift 31.)
+struct Divider {
+  uint32_t by, magic;
+  int shift;
+  static Divider of(int by) {
+    int s = 0;
+    while ((1LL << s) < by) ++s;
+    return Divider{static_cast<uint32_t>(by), static_cast<uint32_t>(((1ULL << (31 + s)) + by - 1) / by), 31 + s};
+  }
+  __host__ __device__ __forceinline__ int quotient(int x) const {
+    return static_cast<int>((static_cast<uint64_t>(static_cast<uint32_t>(x)) * magic) >> shift);
+  }
+  __host__ __device__ __forceinline__ int rest(int x, int quotient) const { return x - quotient * static_cast<int>(by); }
+};
+
 }  // namespace akv
 
 // Expands `body` with `T` bound to the storage type named by `code`; unknown codes return -1.

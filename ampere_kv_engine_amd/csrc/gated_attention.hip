@@ -913,6 +913,8 @@ struct SingleArgs {
   long gate_stride, num_pages, out_stride;
   float scale, softcap, out_scale;
   int gate_at, table_width, q_heads, kv_heads, page_size, chunk, window, sink, maps, keep_first, segments;
+  int share, groups;                 // query vectors of a key vector, tiles of 16 of them
+  Divider by_segments, by_page, by_maps_and_groups, by_groups, by_heads;   // (a block's divisions stand before its first load)
 };
 
 __device__ __forceinline__ float gate_of(const SingleArgs& a, long n, int vector) {
@@ -935,10 +937,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 4))) voi
   __shared__ float top_of[4][16], weight_of[4][16];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x & (kWave - 1);
   const int col = lane & 15, grp = lane >> 4;
-  const long n = blockIdx.x / a.segments;
-  const int segment = blockIdx.x % a.segments;
-  const int share = a.q_heads / a.kv_heads / a.maps, groups = (share + 15) / 16;      // query vectors of a key vector
-  const int kvh = blockIdx.y / (a.maps * groups), map = blockIdx.y / groups % a.maps, of_group = blockIdx.y % groups * 16 + col;
+  const long n = a.by_segments.quotient(blockIdx.x);
+  const int segment = a.by_segments.rest(blockIdx.x, static_cast<int>(n));
+  const int share = a.share, kvh = a.by_maps_and_groups.quotient(blockIdx.y), of_key = a.by_maps_and_groups.rest(blockIdx.y, kvh);
+  const int map = a.by_groups.quotient(of_key), of_group = a.by_groups.rest(of_key, map) * 16 + col;
   const int vector = (kvh * share + min(of_group, share - 1)) * a.maps + map;
   const int r = a.table_rows != nullptr ? a.table_rows[a.seq_of_token[n]] : a.seq_of_token[n];
   const int pos = a.positions[n];
@@ -964,8 +966,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 4))) voi
     for (int i = 0; i < STEPS; ++i) {
       const int turn = first + wave + 4 * i;
       const int key = steps.key(min(turn, steps.all - 1));
-      page[i] = table[key / a.page_size];
-      offset[i] = key % a.page_size;
+      const int nth = a.by_page.quotient(key);
+      page[i] = table[nth];
+      offset[i] = a.by_page.rest(key, nth);
       at_key[i] = turn < steps.all ? key : pos + 1;                  // (none of a step beyond the last counts)
     }
     const bf16_t* qp = a.q + (n * a.q_heads + vector) * DIM + grp * 8;
@@ -1156,8 +1159,8 @@ __global__ __launch_bounds__(256) void gated_attention_fold_kernel(const SingleA
   const int lane = threadIdx.x & (kWave - 1);
   const long row = static_cast<long>(blockIdx.x) * 4 + threadIdx.x / kWave;
   if (row >= rows) return;
-  const long n = row / a.q_heads;
-  const int vector = static_cast<int>(row % a.q_heads);
+  const long n = a.by_heads.quotient(static_cast<int>(row));
+  const int vector = a.by_heads.rest(static_cast<int>(row), static_cast<int>(n));
   const Steps steps(a.positions[n], a.window, a.chunk, a.keep_first);
   if (steps.all <= kSegmentSteps || 4 * lane >= vdim) return;
   const int count = min((steps.all + kSegmentSteps - 1) / kSegmentSteps, a.segments);
@@ -1193,13 +1196,18 @@ int akv_gated_attention_singles(const void* q, const void* k_pages, const void* 
                                 hipStream_t stream) {
   if (tokens <= 0) return 0;
   if (page_size % 16 != 0 || maps < 1 || kv_heads <= 0 || q_heads % (kv_heads * maps) != 0 || segments < 1 || at_once < 1 ||
-      static_cast<long>(at_once) * segments > 0x7fffffffL || (segments > 1 && partial == nullptr))
+      static_cast<long>(at_once) * segments > 0x7fffffffL || static_cast<long>(min(at_once, tokens)) * q_heads > 0x7fffffffL ||
+      (segments > 1 && partial == nullptr))
     return -2;
   SingleArgs a{static_cast<const bf16_t*>(q), static_cast<const bf16_t*>(k_pages), static_cast<const bf16_t*>(v_pages),
                      static_cast<const bf16_t*>(gates), seq_of_token, positions, block_table, table_rows, sink_logits,
                      distance_bias, static_cast<bf16_t*>(out), partial, gate_stride, num_pages, out_stride, scale, softcap,
                      out_scale, gate_at, table_width, q_heads, kv_heads, page_size, chunk, window, sink, maps, keep_first, segments};
-  const long columns = static_cast<long>(kv_heads) * maps * ((q_heads / kv_heads / maps + 15) / 16);
+  a.share = q_heads / kv_heads / maps, a.groups = (a.share + 15) / 16;
+  if (a.share < 1 || page_size < 1) return -2;
+  a.by_segments = Divider::of(segments), a.by_page = Divider::of(page_size), a.by_groups = Divider::of(a.groups);
+  a.by_maps_and_groups = Divider::of(maps * a.groups), a.by_heads = Divider::of(q_heads);
+  const long columns = static_cast<long>(kv_heads) * maps * a.groups;
   if (!aligned_for_tiles(q, k_pages, v_pages, out, out_stride)) return -2;
   if (columns > 65535) return -2;
   // (a launch's partial sums are folded before the next one, on the same stream, writes its own)

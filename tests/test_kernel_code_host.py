@@ -55,3 +55,37 @@ def test_calm_turns_of_the_prompt_attention_wait_for_counted_loads_alone(dim, pa
     assert len(loops) == 1
     waits = [re.search(r"vmcnt\((\d+)\)", t) for t in loops[0] if t.startswith("s_waitcnt")]
     assert [int(w[1]) for w in waits if w] == [4 * dim // 64] * 4
+
+
+def test_divider_is_exact(tmp_path):
+    """`Divider` (common.h) against the language's division: every small divisor, those beside powers of two and large ones, at the
+    multiples where a quotient changes and at the ends of its range."""
+    source = tmp_path / "divider.hip"
+    source.write_text("""
+#include "common.h"
+#include <cstdio>
+int main() {
+  long wrong = 0;
+  auto check = [&](long by) {
+    const akv::Divider d = akv::Divider::of(static_cast<int>(by));
+    const long last = 0x7fffffffL / by;
+    for (long q : {0L, 1L, 2L, 3L, last / 3, last / 2, last - 1, last})
+      for (long x = q * by - 1; x <= q * by + 1; ++x)
+        if (x >= 0 && x <= 0x7fffffffL) {
+          const int got = d.quotient(static_cast<int>(x));
+          wrong += got != x / by || d.rest(static_cast<int>(x), got) != x % by;
+        }
+    wrong += d.quotient(0x7fffffff) != 0x7fffffffL / by;
+  };
+  for (long by = 1; by <= 5000; ++by) check(by);
+  for (int bit = 2; bit < 31; ++bit)
+    for (long by = (1L << bit) - 1; by <= (1L << bit) + 1; ++by) check(by);
+  for (long by = 0x7fffffffL; by > 5000; by -= 1 + by / 977) check(by);
+  std::printf("%ld\\n", wrong);
+  return 0;
+}
+""")
+    program = tmp_path / "divider"
+    subprocess.run([build._hipcc(), "-O1", "-std=c++17", f"--offload-arch={build.ARCH}", f"-I{build.HERE}", str(source), "-o", str(program)],
+                   check=True, capture_output=True)
+    assert subprocess.run([str(program)], check=True, capture_output=True, text=True).stdout.strip() == "0"
