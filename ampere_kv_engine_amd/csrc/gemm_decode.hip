@@ -50,6 +50,9 @@ struct DecodeArgs {
   const float* bias;        // [outs] or null: added to the sums over k before anything else is done with them; GATED: `clamp` of `gate_times`
   float eps;
   int sum_tiles, rows, outs, k, k_tiles, n_tiles, k_split, red_floats;
+  int per_part;             // k-tiles of a part
+  int sums_per_wave;        // SCALED, ROWSCALED: quads of partial sums that a wave adds up, a multiple of 64
+  Divider by_split;         // (divisions would stand before the first weights)
   float* pieces;            // [wave-row][2][RT][4][64]: the sums of a wave-row whose parts of k lie in two blocks
   unsigned int* arrivals;   // [wave-row], zero between launches: how many of the two have left their sums
 };
@@ -68,10 +71,9 @@ __global__ __launch_bounds__(768) void linear_decode_kernel(const DecodeArgs a) 
   // The product's work is cut into units - (wave-row of RT row tiles, part of k) - numbered wave-row by wave-row; a
   // block's waves take consecutive units, whole wave-rows or not.
   const int first_unit = blockIdx.x * waves, unit = first_unit + wave;
-  const int wave_row = unit / a.k_split, part = unit % a.k_split;
+  const int wave_row = a.by_split.quotient(unit), part = a.by_split.rest(unit, wave_row);
   const int row_tile = wave_row * RT;
-  const int per_part = (a.k_tiles + a.k_split - 1) / a.k_split;
-  const int kt0 = part * per_part, kt1 = min(a.k_tiles, kt0 + per_part);
+  const int kt0 = part * a.per_part, kt1 = min(a.k_tiles, kt0 + a.per_part);
   const bool works = row_tile < a.n_tiles && kt0 < kt1;
   const bool ragged = (a.k & 31) != 0;
   const uintx4 zero = {0u, 0u, 0u, 0u};
@@ -95,8 +97,37 @@ __global__ __launch_bounds__(768) void linear_decode_kernel(const DecodeArgs a) 
   // SCALED: the rows as the operand wants them, [k tile][k chunk of 8][row] x 16 bytes: lane (r, g) reads chunk g, row r
   constexpr int kScaleFloats = 12 * 16 + 16;   // SCALED: every wave's share of the rows' sums of squares, then the scales
   uintx4* rows_lds = reinterpret_cast<uintx4*>(red + (SCALED ? kScaleFloats : 0));
+  // the operand of the rows: lane (r, g) brings row r, 8 values at k = g * 8 of the k-tile.  Rows beyond `rows` read
+  // the last row again (their results are never stored); the chunks of a ragged last k-tile beyond k count as zero.
+  const int row_read = min(r, a.rows - 1);
+  const bool lane_outside = ragged && (a.k_tiles - 1) * 32 + g * 8 >= a.k;
+  uintx4 x0[U], x1[U];
+  auto fetch_rows = [&](int kt, uintx4 (&x)[U]) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int tile = min(kt + u, last_tile);
+      const int chunk = (lane_outside && tile == a.k_tiles - 1) ? 0 : g;
+      if constexpr (SCALED) x[u] = rows_lds[(tile * 4 + chunk) * a.rows + row_read];
+      else x[u] = *reinterpret_cast<const uintx4*>(a.x + static_cast<size_t>(row_read) * a.k + tile * 32 + chunk * 8);
+    }
+  };
+  // ROWSCALED: the partial sums are asked for before the weights, the rows behind them, all without a test: the sums are added
+  // up while both are on their way.  (Sums behind the weights and rows behind the sums, a step of one request, 8 layers of width
+  // 2048: 339 -> 333 us, the divisions at a block's start among them; at width 4096 the same within 0.3 %.)
+  constexpr int kSumsHeld = 4;  // quads of sums that a lane asks for so; further ones (wide models, few waves) follow in a loop
+  const int sum_quads = a.sum_tiles * 4, sum0 = wave * a.sums_per_wave, sum1 = min(sum_quads, sum0 + a.sums_per_wave);
+  float4 sums_held[ROWSCALED ? kSumsHeld : 1];
+  if constexpr (ROWSCALED) {
+#pragma unroll
+    for (int i = 0; i < kSumsHeld; ++i) sums_held[i] = reinterpret_cast<const float4*>(a.sums)[min(sum0 + lane + 64 * i, sum_quads - 1)];
+  }
   fetch_weights(kt0, w0);       // two groups on their way while the rows are normed
   fetch_weights(kt0 + U, w1);
+  if constexpr (ROWSCALED) {
+    fetch_rows(kt0, x0);
+    fetch_rows(kt0 + U, x1);
+    __builtin_amdgcn_sched_barrier(0);
+  }
   // ADDS: what the sums will be added to, and the next norm's weight there, are asked for now - in the epilogue they
   // would cost the block's last wave a trip to memory.  (Every output has one owner: nobody changes them meanwhile.)
   float4 held[ADDS ? RT : 1], gain_held[ADDS ? RT : 1];
@@ -121,11 +152,17 @@ __global__ __launch_bounds__(768) void linear_decode_kernel(const DecodeArgs a) 
     float* shares = red;
     float* scales = red + 12 * 16;
     {
-      const int quads = a.sum_tiles * 4, per_wave = ((quads + waves - 1) / waves + 63) / 64 * 64;
-      const int q0 = wave * per_wave, q1 = min(quads, q0 + per_wave);
       float4 part = make_float4(0.f, 0.f, 0.f, 0.f);
+      if constexpr (ROWSCALED) {
+#pragma unroll
+        for (int i = 0; i < kSumsHeld; ++i)
+          if (sum0 + lane + 64 * i < sum1) {
+            const float4 v = sums_held[i];
+            part.x += v.x, part.y += v.y, part.z += v.z, part.w += v.w;
+          }
+      }
 #pragma unroll 4
-      for (int q = q0 + lane; q < q1; q += 64) {
+      for (int q = sum0 + lane + (ROWSCALED ? 64 * kSumsHeld : 0); q < sum1; q += 64) {
         const float4 v = reinterpret_cast<const float4*>(a.sums)[q];
         part.x += v.x, part.y += v.y, part.z += v.z, part.w += v.w;
       }
@@ -182,20 +219,6 @@ __global__ __launch_bounds__(768) void linear_decode_kernel(const DecodeArgs a) 
     __syncthreads();
   }
 
-  // the operand of the rows: lane (r, g) brings row r, 8 values at k = g * 8 of the k-tile.  Rows beyond `rows` read
-  // the last row again (their results are never stored); the chunks of a ragged last k-tile beyond k count as zero.
-  const int row_read = min(r, a.rows - 1);
-  const bool lane_outside = ragged && (a.k_tiles - 1) * 32 + g * 8 >= a.k;
-  uintx4 x0[U], x1[U];
-  auto fetch_rows = [&](int kt, uintx4 (&x)[U]) {
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int tile = min(kt + u, last_tile);
-      const int chunk = (lane_outside && tile == a.k_tiles - 1) ? 0 : g;
-      if constexpr (SCALED) x[u] = rows_lds[(tile * 4 + chunk) * a.rows + row_read];
-      else x[u] = *reinterpret_cast<const uintx4*>(a.x + static_cast<size_t>(row_read) * a.k + tile * 32 + chunk * 8);
-    }
-  };
   auto multiply = [&](int kt, const uintx4 (&w)[RT][U], const uintx4 (&x)[U]) {
     if (kt + U <= kt1 && !(ragged && kt + U == a.k_tiles)) {
 #pragma unroll
@@ -213,8 +236,10 @@ __global__ __launch_bounds__(768) void linear_decode_kernel(const DecodeArgs a) 
     }
   };
   if (works) {
-    fetch_rows(kt0, x0);
-    fetch_rows(kt0 + U, x1);
+    if constexpr (!ROWSCALED) {
+      fetch_rows(kt0, x0);
+      fetch_rows(kt0 + U, x1);
+    }
     int kt = kt0;
     for (; kt + 2 * U < kt1; kt += 2 * U) {   // two groups are in flight; the one after them holds tiles of the part
       multiply(kt, w0, x0);
@@ -396,6 +421,9 @@ int launch_decode(DecodeArgs a, hipStream_t stream) {
   const DecodePlan plan = plan_decode(RT, a.n_tiles, a.k_tiles, a.k, SCALED ? a.rows : 0, a.pieces != nullptr);
   const int k_split = plan.k_split, waves = plan.waves, blocks = plan.blocks;
   a.k_split = k_split;
+  a.per_part = (a.k_tiles + k_split - 1) / k_split;
+  a.by_split = Divider::of(k_split);
+  a.sums_per_wave = ((a.sum_tiles * 4 + waves - 1) / waves + 63) / 64 * 64;
   a.red_floats = k_split > 1 ? waves * RT * 4 * 64 : 0;
   const size_t lds = max(static_cast<size_t>(a.red_floats) * 4,
                          SCALED ? (12 * 16 + 16) * 4 + static_cast<size_t>(a.rows) * a.k * 2 : (ROWSCALED ? (12 * 16 + 16) * 4 : 0));
@@ -483,7 +511,7 @@ extern "C" int akv_linear_rowscaled(const void* x, const float* sums, int sum_ti
                                     int n_tiles, int k_tiles, int gated, int row_tiles, const float* bias,
                                     hipStream_t stream) {
   if (rows <= 0 || outs <= 0) return 0;
-  if (rows > 16 || (k & 7) != 0 || k_tiles * 32 < k || sum_tiles != (k + 15) / 16) return -2;
+  if (rows > 16 || k <= 0 || (k & 7) != 0 || k_tiles * 32 < k || sum_tiles != (k + 15) / 16) return -2;
   if (row_tiles < 0 || row_tiles > 2 || (gated && row_tiles == 1)) return -2;
   if (gated ? ((outs & 15) != 0 || n_tiles * 8 != outs) : n_tiles * 16 < outs) return -2;
   DecodeArgs a{};
