@@ -75,8 +75,8 @@ __global__ __launch_bounds__((A * kHalves + kFetchers) * 64) void linear_mid_ker
                                                               TY* __restrict__ y, float* __restrict__ partial,
                                                               unsigned* __restrict__ counters, int rows, int outs, int k,
                                                               int k_tiles, int n_tiles, int bands, int parts,
-                                                              int part_tiles, int m_blocks, const float* __restrict__ bias,
-                                                              const MidFold fold) {
+                                                              int part_tiles, int m_blocks, Divider by_parts, Divider by_m_blocks,
+                                                              const float* __restrict__ bias, const MidFold fold) {
   constexpr int S = kStage<MT>;
   constexpr int kBlockRows = MT * 16, kChunks = kSumChunks<MT>;
   const bool rowscaled = fold.sums_in != nullptr;
@@ -90,9 +90,9 @@ __global__ __launch_bounds__((A * kHalves + kFetchers) * 64) void linear_mid_ker
 
   // which work: blocks that share weights (same band and part of k, other rows) are neighbours on one XCD
   const int xcd = blockIdx.x % kXcds, slot = blockIdx.x / kXcds;
-  const int item = (slot / m_blocks) * kXcds + xcd, m_block = slot % m_blocks;
+  const int of_xcd = by_m_blocks.quotient(slot), item = of_xcd * kXcds + xcd, m_block = by_m_blocks.rest(slot, of_xcd);
   if (item >= bands * parts) return;
-  const int band = item / parts, part = item % parts;
+  const int band = by_parts.quotient(item), part = by_parts.rest(item, band);
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -508,7 +508,7 @@ int launch_mid(const MidPlan& p, const void* x, const void* wp, void* y, float* 
   if (blocks > 0x7fffffffL) return -2;
   linear_mid_kernel<A, MT, RT, G, GATED, TY><<<static_cast<unsigned>(blocks), (A * kHalves + kFetchers) * 64, lds, stream>>>(
       static_cast<const bf16_t*>(x), static_cast<const uintx4*>(wp), static_cast<TY*>(y), partial, counters, rows, outs,
-      k, k_tiles, n_tiles, p.bands, p.parts, p.part_tiles, p.m_blocks, bias, fold);
+      k, k_tiles, n_tiles, p.bands, p.parts, p.part_tiles, p.m_blocks, Divider::of(p.parts), Divider::of(p.m_blocks), bias, fold);
   return AKV_LAUNCH_STATUS();
 }
 
