@@ -21,7 +21,7 @@
 // What bounds it: single tokens wait for their keys - a trip to the block table, one to the records, one to the values, then
 // the fold's launch; prompts run at the matrix cores' rate (64 instructions of 32 cycles per 16 x 16 scores at dim 128) where
 // their tiles fill the device.  Measured, us a layer, 16 heads over 4 of 128, against one wave per (token, head) in plain
-// float32 (`attention_rows`): 3 single tokens after 64 to 700 keys 298 -> 16.1 + 4.6 for the fold; 3 prompts of 333 tokens
+// float32 (`attention_rows`): 3 single tokens after 64 to 700 keys 298 -> 13.4 + 4.6 for the fold; 3 prompts of 333 tokens
 // 811 -> 62.
 
 #include <type_traits>
