@@ -251,7 +251,9 @@ __device__ __forceinline__ void encode_head(uintx4 (&reg)[KT], bool normed, floa
 // FRESH (single tokens, D a multiple of 64): query, key and value of the token come raw from the stacked projection
 // `a.qkv`.  Every block norms and rotates its own query heads in registers; the block whose keys include the token's
 // own position does the same for the new key, puts it and the new value into its operands in place of what the page
-// holds there, and writes both to the page for later steps.  No other block reads that slot in this launch.
+// holds there, and writes both to the page for later steps.  No other block of the launch uses what that slot holds:
+// blocks whose keys do not include the position do not ask for it, and those of further groups of the same kv head's query
+// heads, which ask for the whole step, encode the new key for themselves as well and put it in place of what they read.
 // (Split launches of head sizes up to 128 are held to the registers of two waves per SIMD: decoding lives on the
 // number of waves that wait for memory at the same time.)
 // ONCE: no other block of the launch reads these keys and values (single tokens, one block per kv head and segment):
@@ -351,7 +353,8 @@ __device__ __forceinline__ void attention_mfma_body(const Args& a, const Where a
   // lane, and handed round by shuffles; the first step's keys and values are asked for at once, before the queries are
   // encoded, and every next step's before the products of the one before.  None of these loads stands behind a test
   // (with one the compiler cannot count them and waits for all before the encoding): places outside the range
-  // are asked for at the nearest one inside, and what must count as zero is zeroed where it is used.  (A step of one
+  // are asked for at the nearest one inside, and what must count as zero is zeroed where it is used.  A wave without keys - the
+  // fourth of an item of three steps, a segment beyond a short request's end - steps over all of it, as a whole.  (A step of one
   // request, 8 layers: 210 keys of 16 / 4 heads 363 -> 340 us, 2,048 keys of 32 / 8 heads 924 -> 895; the shuffles and the early
   // loads with the tests left in gave nothing.  Waves alone on their segments, 8, 64 and 27 uneven requests: 1,261 -> 1,251, 1,978 ->
   // 1,961, 1,655 -> 1,605; 171 tokens beside 8 requests 2,361 -> 2,315.)
@@ -360,11 +363,9 @@ __device__ __forceinline__ void attention_mfma_body(const Args& a, const Where a
     entries_first = base >> a.page_shift;
     entries = table[min(entries_first + lane, max(last_pos, 0) >> a.page_shift)];
   };
-  const bool any_key = range_lo <= range_hi;       // (AHEAD: else the token's own position is asked for and not used)
-  const int near_lo = any_key ? range_lo : max(last_pos, 0), near_hi = any_key ? range_hi : max(last_pos, 0);
   int new_entry = 0;                               // AHEAD: the entry of the token's own page
   if constexpr (AHEAD) {
-    ask_entries(near_lo & ~31);
+    ask_entries(range_lo & ~31);
     if constexpr (FRESH) new_entry = table[max(last_pos, 0) >> a.page_shift];
   }
   // the table's entry for a key of a step; AHEAD: all lanes call it together
@@ -649,10 +650,10 @@ __device__ __forceinline__ void attention_mfma_body(const Args& a, const Where a
     size_t k_at[2];
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-      const int key = min(max(base + key_in_step + j * 4, near_lo), near_hi);
+      const int key = min(max(base + key_in_step + j * 4, range_lo), range_hi);
       k_at[j] = page_at(key) + (k_lane + static_cast<uint32_t>(key & page_mask) * (D * 2u));
     }
-    const int run = min(max(base + g * 8, near_lo & ~7), near_hi & ~7);
+    const int run = min(max(base + g * 8, range_lo & ~7), range_hi & ~7);
     const size_t v_at = page_at(run) + (v_lane + static_cast<uint32_t>(run & page_mask) * 2u);
 #pragma unroll
     for (int j = 0; j < 2; ++j)
@@ -722,7 +723,7 @@ __device__ __forceinline__ void attention_mfma_body(const Args& a, const Where a
   };
   // AHEAD: keys and values of the next step, then this one
   auto turn_ahead = [&](int base, uintx4 (&cur)[2][KT], uintx4 (&values)[DT], uintx4 (&next)[2][KT], uintx4 (&next_values)[DT]) {
-    if ((min(base + 63, near_hi) >> a.page_shift) - entries_first > 63) ask_entries(base + 32);
+    if ((min(base + 63, range_hi) >> a.page_shift) - entries_first > 63) ask_entries(base + 32);
     load_step(base + 32, next, next_values);
     __builtin_amdgcn_sched_barrier(0);
     zero_outside(base, cur, values);
@@ -731,13 +732,15 @@ __device__ __forceinline__ void attention_mfma_body(const Args& a, const Where a
   };
   const int first_base = range_lo & ~31;
   if constexpr (AHEAD) {
-    load_step(first_base, kreg, vreg);
-    __builtin_amdgcn_sched_barrier(0);
-    if constexpr (FRESH) encode_fresh();  // while the first keys and values are on their way
-    for (int base = first_base; base <= range_hi; base += 64) {  // two turns: the registers swap roles
-      turn_ahead(base, kreg, vreg, knext, vnext);
-      if (base + 32 > range_hi) break;
-      turn_ahead(base + 32, knext, vnext, kreg, vreg);
+    if (__builtin_amdgcn_readfirstlane(range_lo <= range_hi)) {   // (a wave without keys asks for none; the new key is then another's)
+      load_step(first_base, kreg, vreg);
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (FRESH) encode_fresh();  // while the first keys and values are on their way
+      for (int base = first_base; base <= range_hi; base += 64) {  // two turns: the registers swap roles
+        turn_ahead(base, kreg, vreg, knext, vnext);
+        if (base + 32 > range_hi) break;
+        turn_ahead(base + 32, knext, vnext, kreg, vreg);
+      }
     }
   } else if constexpr (PIPE) {
     if (first_base <= range_hi) {

@@ -25,18 +25,42 @@ def test_inline_assembly_that_writes_m0_says_so():
         assert block.count(":") == 3 and '"m0"' in block.split(":")[3], f"{name}: {block}"
 
 
-def _prompt_kernel(dim, pages_per_step, folder):
-    """(address, instruction) of `attention_prompt_kernel` in the built library."""
+def _device_code(dim, folder):
+    """The built attention library's code for the device, as a file of its own."""
     library = build.attention_library_path(dim)
     if library is None or OBJDUMP is None:
         pytest.skip("the attention library is not built, or there is nothing to list it with")
     copied = shutil.copy(library, folder)
     subprocess.run([OBJDUMP, "--offloading", copied], cwd=folder, check=True, capture_output=True)
     code, = glob.glob(os.path.join(folder, "*gfx950"))
-    listing = subprocess.run([OBJDUMP, "-d", "--no-show-raw-insn", code], cwd=folder, check=True, capture_output=True, text=True).stdout
-    kernel = re.split(r"\n\n", listing[listing.index(f"attention_prompt_kernelILi{pages_per_step}E"):])[0]
+    return code
+
+
+def _kernel(code, name):
+    """(address, instruction, target) of the first kernel whose mangled name holds `name`."""
+    listing = subprocess.run([OBJDUMP, "-d", "--no-show-raw-insn", code], check=True, capture_output=True, text=True).stdout
+    kernel = re.split(r"\n\n", listing[listing.index(name):])[0]
     lines = [re.match(r"\s+(\S.*?)\s*// ([0-9A-F]+):(?:.*<.*\+0x([0-9a-f]+)>)?", line) for line in kernel.splitlines()]
     return [(int(m[2], 16), m[1], int(m[3], 16) if m[3] else None) for m in lines if m]
+
+
+def _prompt_kernel(dim, pages_per_step, folder):
+    return _kernel(_device_code(dim, folder), f"attention_prompt_kernelILi{pages_per_step}E")
+
+
+@pytest.mark.parametrize("dim", [64, 128, 192, 256])
+def test_waves_without_keys_ask_for_none(dim, tmp_path):
+    """The kernel whose four waves share an item, asking ahead: before its first load of keys (the first that is marked read-once)
+    stands a branch over all of the matrix instructions to where the wave's empty result is left in LDS."""
+    code = _kernel(_device_code(dim, str(tmp_path)), "attention_items_kernelILb1ELb1ELNS_5ItemsE1ELb1EEEv")
+    start = code[0][0]
+    first_load = next(i for i, (_, text, _) in enumerate(code) if text.startswith("global_load") and text.endswith(" nt"))
+    last_product = max(i for i, (_, text, _) in enumerate(code) if "v_mfma" in text)
+    landings = [next((i for i, (at, _, _) in enumerate(code) if at == start + target), None)
+                for _, text, target in code[:first_load] if text.startswith(("s_cbranch", "s_branch")) and target is not None]
+    results = [i for i in landings if i is not None and i > last_product
+               and any(text.startswith("ds_write") for _, text, _ in code[i:]) and not code[i][1].startswith("s_endpgm")]
+    assert results
 
 
 @pytest.mark.parametrize("pages_per_step", [1, 2])
