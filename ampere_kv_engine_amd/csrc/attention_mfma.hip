@@ -255,7 +255,7 @@ __device__ __forceinline__ void encode_head(uintx4 (&reg)[KT], bool normed, floa
 // blocks whose keys do not include the position do not ask for it, and those of further groups of the same kv head's query
 // heads, which ask for the whole step, encode the new key for themselves as well and put it in place of what they read.
 // (Split launches of head sizes up to 128 are held to the registers of two waves per SIMD: decoding lives on the
-// number of waves that wait for memory at the same time.)
+// number of waves that wait for memory at the same time.  Whole requests as items are few: their waves have all registers.)
 // ONCE: no other block of the launch reads these keys and values (single tokens, one block per kv head and segment):
 // the loads are marked read-once.  A bare reader with this kernel's lanes and depth draws 7.1 TB/s from 2 GB of
 // pages with the mark and 6.5 TB/s without.
@@ -344,6 +344,10 @@ __device__ __forceinline__ void attention_mfma_body(const Args& a, const Where a
     range_lo = max(range_lo, seg_lo);
     range_hi = min(range_hi, seg_hi);
   }
+  if constexpr (AHEAD && D > 192) {        // (the same in every lane: kept out of the vector registers, which are all taken)
+    range_lo = __builtin_amdgcn_readfirstlane(range_lo);
+    range_hi = __builtin_amdgcn_readfirstlane(range_hi);
+  }
 
   const int* table = a.block_table + static_cast<long>(a.table_rows != nullptr ? a.table_rows[t.request] : t.request) * a.table_width;
 
@@ -358,6 +362,15 @@ __device__ __forceinline__ void attention_mfma_body(const Args& a, const Where a
   // request, 8 layers: 210 keys of 16 / 4 heads 363 -> 340 us, 2,048 keys of 32 / 8 heads 924 -> 895; the shuffles and the early
   // loads with the tests left in gave nothing.  Waves alone on their segments, 8, 64 and 27 uneven requests: 1,261 -> 1,251, 1,978 ->
   // 1,961, 1,655 -> 1,605; 171 tokens beside 8 requests 2,361 -> 2,315.)
+  // It holds two steps' values as well as two steps' keys, D / 4 registers more, and is taken where the kernel has them - everywhere but in
+  // the launch with portions at heads of 192 and for whole requests of heads beyond 224.  The kernel and its merge, us without / with, raw
+  // projections: 16 / 4 heads of 192, one request of 210 and of 2,048 keys 14.9 / 13.1, 15.4 / 14.3, 27 of 64 to 16,000 71.7 / 63.1;
+  // of 256 17.5 / 15.5, 17.4 / 17.0, 83.6 / 81.4 (with the range's ends in vector registers, and 28 bytes a lane in memory, 16.2, 18.5
+  // and 83.5).  Encoded queries: one request of 100 keys 5.8 / 5.3 (heads of 128), 6.9 / 6.4 (192), 8.1 / 11.1 (256, not taken so);
+  // of 6,000 14.5 / 11.1, 17.7 / 13.5, 21.5 / 15.5.  Where a wave has exactly one step, the unused step that it asks for last can cost what the
+  // early loads give: encoded queries, 4 x 2,048 keys of 32 / 8 heads of 128 13.5 / 14.5, one request of 16,000 of 16 / 4 15.3 / 16.2.  (The last turn
+  // written out without loads takes 72 to 300 bytes a lane of memory at heads of 128; all its lanes at one address gained 1 to 2 % of
+  // long contexts and lost as much of short ones.)
   int entries_first = 0, entries = 0;
   auto ask_entries = [&](int base) {
     entries_first = base >> a.page_shift;
@@ -1793,7 +1806,13 @@ __global__ __launch_bounds__(64 * kSharedWaves, 2) void attention_prompt_gated_k
 // after them is four independent waves of the single tokens' kernel, wave w of block b standing where block
 // 4 b + w of that kernel's own grid (kv heads x items of the plan) would.  The text of either kernel is the same as in
 // its own launch, so the bits are.  Registers are the larger of the two (two waves a SIMD, which the single tokens'
-// kernel has anyway); every block holds the portion kernel's LDS.
+// kernel has anyway up to heads of 128); every block holds the portion kernel's LDS.
+// The single tokens ask ahead where the registers hold it: two blocks on a unit leave a wave 256, which heads of 192 exceed by
+// 188 to 212 bytes a lane as it is and by 480 with two steps' values (8 x 4,000 keys beside 171 tokens, 16 / 4 heads of 192: 46
+// us without, 60 with; 27 uneven requests beside 64 tokens 98 and 120); the LDS of heads of 256 lets a unit hold one block,
+// whose waves have 512 (55 and 52; 97 and 90).
+constexpr bool kPairAhead = D <= 128 || 2 * sizeof(SharedLds) > 160 * 1024;
+
 template <bool ONCE, int SP>
 __global__ __launch_bounds__(64 * kSharedWaves, 2) void attention_pair_kernel(const Args single, const Args portion,
                                                                               const int portion_blocks) {
@@ -1806,7 +1825,7 @@ __global__ __launch_bounds__(64 * kSharedWaves, 2) void attention_pair_kernel(co
       const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
       const int unit = (static_cast<int>(blockIdx.x) - portion_blocks) * kSharedWaves + wave;
       if (unit >= gx * gy) return;
-      attention_mfma_body<1, true, true, true, ONCE, kNoItems, true>(
+      attention_mfma_body<1, true, true, true, ONCE, kNoItems, kPairAhead>(
           single, Where{unit % gx, unit / gx, 0, gx, gy, static_cast<int>(threadIdx.x) & 63, 0}, nullptr);
     }
   }
@@ -1932,7 +1951,8 @@ __global__ __launch_bounds__(64 * kMergeWaves) void attention_merge_kernel(const
 
 template <bool FRESH, bool AHEAD>
 void launch_items(const Args& a, dim3 grid, bool once, bool whole, hipStream_t stream) {
-  if (whole) attention_items_kernel<FRESH, false, kWhole, AHEAD><<<grid, 64 * kItemWaves, 0, stream>>>(a);   // (few keys: not marked)
+  // (few keys: not marked; asking ahead, heads beyond 224 would keep some 380 bytes a lane in memory: see AHEAD)
+  if (whole) attention_items_kernel<FRESH, false, kWhole, AHEAD && D <= 224><<<grid, 64 * kItemWaves, 0, stream>>>(a);
   else if (once) attention_items_kernel<FRESH, true, kPlanned, AHEAD><<<grid, 64 * kItemWaves, 0, stream>>>(a);
   else attention_items_kernel<FRESH, false, kPlanned, AHEAD><<<grid, 64 * kItemWaves, 0, stream>>>(a);
 }

@@ -48,6 +48,23 @@ def _prompt_kernel(dim, pages_per_step, folder):
     return _kernel(_device_code(dim, folder), f"attention_prompt_kernelILi{pages_per_step}E")
 
 
+@pytest.mark.parametrize("dim", build.DEFAULT_HEAD_DIMS)
+def test_single_tokens_ask_ahead_only_where_registers_hold_it(dim, tmp_path):
+    """Kernels of single tokens that ask for a step's keys and values while the step before is computed hold two steps' values: none
+    of them keeps registers in memory (the compiler's own count), and the launch that holds prompt portions too, which the portions'
+    registers bound to two waves a SIMD at heads of 192, keeps no more than without (188 to 212 bytes a lane; asking ahead 480)."""
+    readelf = os.path.join(os.path.dirname(OBJDUMP or ""), "llvm-readelf")
+    code = _device_code(dim, str(tmp_path))
+    notes = subprocess.run([readelf, "--notes", code], check=True, capture_output=True, text=True).stdout
+    kernels = re.findall(r"\.name: +(\S+)\n +\.private_segment_fixed_size: (\d+)", notes)
+    ahead = [(name, int(scratch)) for name, scratch in kernels if re.search(r"attention_(items|mfma)_kernelI\S*Lb1EEEv", name)
+             and ("items" in name or re.search(r"kernelILi1E(Lb[01]E){4}Lb1EEEv", name))]
+    pair = [(name, int(scratch)) for name, scratch in kernels if "attention_pair_kernel" in name]
+    assert len(ahead) >= 2 and (len(pair) == 6 or dim % 64 != 0)
+    assert [(name, scratch) for name, scratch in ahead if scratch != 0] == []
+    assert [(name, scratch) for name, scratch in pair if scratch > (216 if dim == 192 else 0)] == []
+
+
 @pytest.mark.parametrize("dim", [64, 128, 192, 256])
 def test_waves_without_keys_ask_for_none(dim, tmp_path):
     """The kernel whose four waves share an item, asking ahead: before its first load of keys (the first that is marked read-once)
