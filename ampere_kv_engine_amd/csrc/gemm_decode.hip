@@ -111,10 +111,16 @@ __global__ __launch_bounds__(768) void linear_decode_kernel(const DecodeArgs a) 
       else x[u] = *reinterpret_cast<const uintx4*>(a.x + static_cast<size_t>(row_read) * a.k + tile * 32 + chunk * 8);
     }
   };
-  // ROWSCALED: the partial sums are asked for before the weights, the rows behind them, all without a test: the sums are added
-  // up while both are on their way.  (Sums behind the weights and rows behind the sums, a step of one request, 8 layers of width
-  // 2048: 339 -> 333 us, the divisions at a block's start among them; at width 4096 the same within 0.3 %.)
-  constexpr int kSumsHeld = 4;  // quads of sums that a lane asks for so; further ones (wide models, few waves) follow in a loop
+  // ROWSCALED: the first partial sums are asked for before the weights - loads come back in the order they were asked for, so
+  // they are added up while the weights are on their way -, the rows after the scales are there.  How many quads a lane asks for so is
+  // what costs no wave: with four, two row tiles a wave take 132 registers instead of 128, 12 waves a unit instead of 16, and
+  // rows asked for early take one row tile a wave from 86 to 100.  Further quads (two row tiles: widths beyond 2,048 with
+  // eight waves a block; one: beyond 8,192) follow in a loop.  us, sums behind the weights / four quads and the rows early
+  // everywhere / so: q/k/v of 3,072 x 2,048, 1 and 8 rows 5.7 6.4 / 5.4 5.6 / 5.2 5.8; gate and up of 3,072 x 2,048 8.0 8.6 / 7.6 7.8 / 7.1 7.7;
+  // q/k/v of 6,144 x 4,096 12.5 13.1 / 12.7 13.6 / 12.5 13.2; of 7,168 x 5,120 17.7 18.8 / 17.0 18.3 / 16.9 18.3; gate and up of 3,072 x 1,024 6.3
+  // 6.9 / 6.7 6.9 / 6.2 6.8, of 9,728 x 2,560 21.2 22.1 / 21.6 22.7 / 20.7 21.4, of 12,288 x 4,096 35.8 35.2 / 35.6 35.1 / 35.5 34.8, of 17,408 x 5,120
+  // (four waves a block, 320 quads each) 66.7 67.5 / 66.6 66.6 / 67.0 66.9.
+  constexpr int kSumsHeld = RT == 1 ? 4 : 1;
   const int sum_quads = a.sum_tiles * 4, sum0 = wave * a.sums_per_wave, sum1 = min(sum_quads, sum0 + a.sums_per_wave);
   float4 sums_held[ROWSCALED ? kSumsHeld : 1];
   if constexpr (ROWSCALED) {
@@ -123,11 +129,7 @@ __global__ __launch_bounds__(768) void linear_decode_kernel(const DecodeArgs a) 
   }
   fetch_weights(kt0, w0);       // two groups on their way while the rows are normed
   fetch_weights(kt0 + U, w1);
-  if constexpr (ROWSCALED) {
-    fetch_rows(kt0, x0);
-    fetch_rows(kt0 + U, x1);
-    __builtin_amdgcn_sched_barrier(0);
-  }
+  if constexpr (ROWSCALED) __builtin_amdgcn_sched_barrier(0);
   // ADDS: what the sums will be added to, and the next norm's weight there, are asked for now - in the epilogue they
   // would cost the block's last wave a trip to memory.  (Every output has one owner: nobody changes them meanwhile.)
   float4 held[ADDS ? RT : 1], gain_held[ADDS ? RT : 1];
@@ -144,8 +146,8 @@ __global__ __launch_bounds__(768) void linear_decode_kernel(const DecodeArgs a) 
   }
   float my_scale = 1.f;         // ROWSCALED: 1 / rms of this lane's row
   if constexpr (SCALED || ROWSCALED) {
-    // (Asking for what the norm needs BEFORE the first weights - a wave's loads come back in the order in which they
-    // were asked for - was measured and is no gain: 15.0 -> 16.0 us at one row, 23.1 -> 22.8 at eight, q/k/v.)
+    // (SCALED: asking for what the norm needs, sums and rows, before the first weights was measured and is no gain: 15.0 ->
+    // 16.0 us at one row, 23.1 -> 22.8 at eight, q/k/v.)
     // The rows' sums of squares: sum_tiles x 16 partial sums.  The waves share the tiles; a lane adds up quads of
     // rows (lane % 4 fixes which four), the lanes of a wave are folded in a fixed order, then the waves' shares - the
     // same order in every block.
@@ -236,10 +238,8 @@ __global__ __launch_bounds__(768) void linear_decode_kernel(const DecodeArgs a) 
     }
   };
   if (works) {
-    if constexpr (!ROWSCALED) {
-      fetch_rows(kt0, x0);
-      fetch_rows(kt0 + U, x1);
-    }
+    fetch_rows(kt0, x0);
+    fetch_rows(kt0 + U, x1);
     int kt = kt0;
     for (; kt + 2 * U < kt1; kt += 2 * U) {   // two groups are in flight; the one after them holds tiles of the part
       multiply(kt, w0, x0);
@@ -384,7 +384,8 @@ DecodePlan plan_decode(int rt, int n_tiles, int k_tiles, int k, int normed_rows,
   // units (768 wave-rows of 4 parts: 12 waves a block make 256 blocks, one a unit; 8 waves, 384 blocks, would leave
   // half the units with two) and, where blocks norm rows, those rows (counted at 1.5 times their bytes: measured,
   // norming 64 KB of rows costs a block what streaming 90 KB of weights does).  A unit holds as many blocks at once as
-  // its 160 KB of LDS and its 32 waves allow; blocks beyond that wait for a further round.  Blocks need not hold
+  // its 160 KB of LDS and 32 waves allow (the registers of most of these kernels leave 12 to 20; the count that the choice was
+  // measured with); blocks beyond that wait for a further round.  Blocks need not hold
   // whole wave-rows: 320 wave-rows of 8 parts are 256 blocks of 10 waves, one and a quarter wave-rows each - the price
   // is the exchange of one wave-row's sums between two blocks, counted as 96 KB (measured: q/k/v of 6,144 x 4,096 gains
   // nothing from it, o of 5,120 x 8,192 goes from 26 to 20 us, down of 5,120 x 25,600 from 62 to 48).

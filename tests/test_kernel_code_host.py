@@ -25,15 +25,31 @@ def test_inline_assembly_that_writes_m0_says_so():
         assert block.count(":") == 3 and '"m0"' in block.split(":")[3], f"{name}: {block}"
 
 
-def _device_code(dim, folder):
-    """The built attention library's code for the device, as a file of its own."""
-    library = build.attention_library_path(dim)
+def _device_codes(library, folder):
+    """A built library's code for the device, a file per source."""
     if library is None or OBJDUMP is None:
-        pytest.skip("the attention library is not built, or there is nothing to list it with")
+        pytest.skip("the library is not built, or there is nothing to list it with")
     copied = shutil.copy(library, folder)
     subprocess.run([OBJDUMP, "--offloading", copied], cwd=folder, check=True, capture_output=True)
-    code, = glob.glob(os.path.join(folder, "*gfx950"))
+    return glob.glob(os.path.join(folder, "*gfx950"))
+
+
+def _device_code(dim, folder):
+    code, = _device_codes(build.attention_library_path(dim), folder)
     return code
+
+
+def _kernel_facts(codes):
+    """Per kernel what the compiler says of it: mangled name -> dict of numbers."""
+    readelf = os.path.join(os.path.dirname(OBJDUMP), "llvm-readelf")
+    facts = {}
+    for code in codes:
+        notes = subprocess.run([readelf, "--notes", code], check=True, capture_output=True, text=True).stdout
+        for kernel in re.split(r"\n  - ", notes)[1:]:
+            name = re.search(r"^ *\.name: +(_Z\S+)$", kernel, re.M)
+            if name:
+                facts[name[1]] = {key: int(value) for key, value in re.findall(r"^ *\.(\w+): +(\d+)$", kernel, re.M)}
+    return facts
 
 
 def _kernel(code, name):
@@ -53,13 +69,10 @@ def test_single_tokens_ask_ahead_only_where_registers_hold_it(dim, tmp_path):
     """Kernels of single tokens that ask for a step's keys and values while the step before is computed hold two steps' values: none
     of them keeps registers in memory (the compiler's own count), and the launch that holds prompt portions too, which the portions'
     registers bound to two waves a SIMD at heads of 192, keeps no more than without (188 to 212 bytes a lane; asking ahead 480)."""
-    readelf = os.path.join(os.path.dirname(OBJDUMP or ""), "llvm-readelf")
-    code = _device_code(dim, str(tmp_path))
-    notes = subprocess.run([readelf, "--notes", code], check=True, capture_output=True, text=True).stdout
-    kernels = re.findall(r"\.name: +(\S+)\n +\.private_segment_fixed_size: (\d+)", notes)
-    ahead = [(name, int(scratch)) for name, scratch in kernels if re.search(r"attention_(items|mfma)_kernelI\S*Lb1EEEv", name)
+    kernels = [(name, facts["private_segment_fixed_size"]) for name, facts in _kernel_facts([_device_code(dim, str(tmp_path))]).items()]
+    ahead = [(name, scratch) for name, scratch in kernels if re.search(r"attention_(items|mfma)_kernelI\S*Lb1EEEv", name)
              and ("items" in name or re.search(r"kernelILi1E(Lb[01]E){4}Lb1EEEv", name))]
-    pair = [(name, int(scratch)) for name, scratch in kernels if "attention_pair_kernel" in name]
+    pair = [(name, scratch) for name, scratch in kernels if "attention_pair_kernel" in name]
     assert len(ahead) >= 2 and (len(pair) == 6 or dim % 64 != 0)
     assert [(name, scratch) for name, scratch in ahead if scratch != 0] == []
     assert [(name, scratch) for name, scratch in pair if scratch > (216 if dim == 192 else 0)] == []
@@ -96,6 +109,15 @@ def test_calm_turns_of_the_prompt_attention_wait_for_counted_loads_alone(dim, pa
     assert len(loops) == 1
     waits = [re.search(r"vmcnt\((\d+)\)", t) for t in loops[0] if t.startswith("s_waitcnt")]
     assert [int(w[1]) for w in waits if w] == [4 * dim // 64] * 4
+
+
+@pytest.mark.parametrize("kernel,waves", [("ILi1ELb0ELb0ELb0ELb1EE", 20), ("ILi2ELb0ELb0ELb0ELb1EE", 16), ("ILi2ELb1ELb0ELb0ELb1EE", 12)])
+def test_decode_products_that_scale_their_sums_leave_a_unit_its_waves(kernel, waves, tmp_path):
+    """One row tile a wave, two, and gated: what the product asks for early must not cost a unit a wave (512 registers a lane and
+    SIMD, handed out in eights)."""
+    facts = _kernel_facts(_device_codes(build.library_path(), str(tmp_path)))
+    registers, = [f["vgpr_count"] for name, f in facts.items() if "linear_decode_kernel" + kernel in name]
+    assert 4 * (512 // (-(-registers // 8) * 8)) >= waves, registers
 
 
 def test_divider_is_exact(tmp_path):
