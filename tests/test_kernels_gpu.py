@@ -857,7 +857,9 @@ def test_adding_products_at_widths_that_are_no_multiple_of_four(hip_own, rows, o
 
 
 @pytest.mark.parametrize("rows,hidden,k,inter", [(1, 96, 72, 64), (3, 304, 520, 208), (8, 4096, 4096, 1024), (16, 4096, 512, 512),
-                                                 (5, 1000, 2048, 256), (16, 5120, 256, 64), (8, 104, 64, 32), (2, 8192, 1024, 128)])
+                                                 (5, 1000, 2048, 256), (16, 5120, 256, 64), (8, 104, 64, 32), (2, 8192, 1024, 128),
+                                                 # (more partial sums than a wave's lanes ask for at once, with one row tile a wave too)
+                                                 (3, 8208, 64, 48), (1, 16384, 64, 128), (16, 12296, 64, 144), (2, 5120, 64, 17408)])
 def test_decode_products_leave_rows_for_a_product_that_scales_its_sums(hip, ref, rows, hidden, k, inter, monkeypatch):
     """Steps of up to 16 rows: `linear_adds(..., rows_out=, gain=)` adds to the residual sum exactly as without the
     two (the same bits, sums of squares included) and leaves the new rows times the next norm's weight;
