@@ -1196,8 +1196,7 @@ int akv_gated_attention_singles(const void* q, const void* k_pages, const void* 
                                 hipStream_t stream) {
   if (tokens <= 0) return 0;
   if (page_size % 16 != 0 || maps < 1 || kv_heads <= 0 || q_heads % (kv_heads * maps) != 0 || segments < 1 || at_once < 1 ||
-      static_cast<long>(at_once) * segments > 0x7fffffffL || static_cast<long>(min(at_once, tokens)) * q_heads > 0x7fffffffL ||
-      (segments > 1 && partial == nullptr))
+      static_cast<long>(at_once) * segments > 0x7fffffffL || (segments > 1 && partial == nullptr))
     return -2;
   SingleArgs a{static_cast<const bf16_t*>(q), static_cast<const bf16_t*>(k_pages), static_cast<const bf16_t*>(v_pages),
                      static_cast<const bf16_t*>(gates), seq_of_token, positions, block_table, table_rows, sink_logits,
@@ -1205,6 +1204,7 @@ int akv_gated_attention_singles(const void* q, const void* k_pages, const void* 
                      out_scale, gate_at, table_width, q_heads, kv_heads, page_size, chunk, window, sink, maps, keep_first, segments};
   a.share = q_heads / kv_heads / maps, a.groups = (a.share + 15) / 16;
   if (a.share < 1 || page_size < 1) return -2;
+  at_once = min(at_once, 0x7fffffff / q_heads);      // (a launch's rows of the fold are counted in 31 bits)
   a.by_segments = Divider::of(segments), a.by_page = Divider::of(page_size), a.by_groups = Divider::of(a.groups);
   a.by_maps_and_groups = Divider::of(maps * a.groups), a.by_heads = Divider::of(q_heads);
   const long columns = static_cast<long>(kv_heads) * maps * a.groups;

@@ -506,7 +506,7 @@ extern "C" int akv_linear_adds_rows(const void* x, const void* wp, float* stream
 // `gate_times` makes of the scaled gate and the scaled up, `bias` being its `clamp`): x [rows, k] bfloat16 are the rows akv_linear_adds_rows left - the residual
 // sum times the norm's weight -, `sums` [sum_tiles][16] the partial sums of squares of the residual rows it left
 // (sum_tiles = ceil(k / 16)).  Sizes, `pieces`, `arrivals`, `row_tiles`: as for akv_linear_scaled, without its limit
-// on the rows' bytes.
+// on the rows' bytes; k > 0 (the first tile and the first sums are read whatever the sizes).
 extern "C" int akv_linear_rowscaled(const void* x, const float* sums, int sum_tiles, float eps, const void* wp, void* y,
                                     float* pieces, unsigned int* arrivals, int exchange_tiles, int rows, int outs, int k,
                                     int n_tiles, int k_tiles, int gated, int row_tiles, const float* bias,

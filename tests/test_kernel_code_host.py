@@ -1,6 +1,7 @@
 """What the compiler is told, and what it makes of it, where results cannot show a mistake: inline assembly that writes a register
 must say so, and loads that are meant to stay on their way must not be waited for."""
 
+import ctypes
 import glob
 import os
 import re
@@ -8,6 +9,7 @@ import shutil
 import subprocess
 
 import pytest
+import torch
 
 from ampere_kv_engine_amd.csrc import build
 
@@ -118,6 +120,21 @@ def test_decode_products_that_scale_their_sums_leave_a_unit_its_waves(kernel, wa
     facts = _kernel_facts(_device_codes(build.library_path(), str(tmp_path)))
     registers, = [f["vgpr_count"] for name, f in facts.items() if "linear_decode_kernel" + kernel in name]
     assert 4 * (512 // (-(-registers // 8) * 8)) >= waves, registers
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="the operands are no memory: nothing may be launched")
+def test_gated_single_tokens_of_any_number_are_taken():
+    """4,096 tokens of a million heads are more (token, head) rows than 31 bits count: they are taken in several launches, not refused."""
+    library = ctypes.CDLL(build.ensure_parts())
+    entry, operand, nothing = library.akv_gated_attention_singles, ctypes.c_void_p(4096), ctypes.c_void_p(0)
+    entry.restype = ctypes.c_int
+    long, real = ctypes.c_long, ctypes.c_float
+    status = lambda q_heads, segments: entry(
+        operand, operand, operand, nothing, long(0), 0, operand, operand, operand, nothing, 1, operand, operand, segments, 4096, 4096,
+        q_heads, 1, 64, 64, 16, long(1), real(1.0), real(0.0), 0, 0, 0, long(q_heads * 64), real(1.0), nothing, 1, 0, nothing, nothing)
+    assert status(1 << 20, 1) == -2                 # (its tiles of 16 heads do not fit the grid)
+    assert status(1 << 19, 1 << 20) == -2           # (nor tokens x segments)
+    assert status(1 << 19, 2) not in (0, -1, -2)    # (taken: what fails is the launch, for want of a device)
 
 
 def test_divider_is_exact(tmp_path):
