@@ -1741,6 +1741,26 @@ def test_single_tokens_whose_items_are_shared_by_four_waves(hip, ref, monkeypatc
         torch.testing.assert_close(got.cpu().float(), want.float(), **attention_tol(torch.bfloat16))
 
 
+@pytest.mark.parametrize("q_heads,kv_heads,dim,page_size", [(6, 1, 32, 8), (5, 5, 80, 16), (5, 5, 80, 8), (8, 2, 128, 8), (6, 2, 192, 16),
+                                                            (3, 1, 256, 8)])
+@pytest.mark.parametrize("histories", [[4090], [2047, 2048, 2049, 0], [9000, 33, 5]])
+@pytest.mark.parametrize("window", [None, 3001])
+def test_single_tokens_whose_waves_walk_many_pages(hip, ref, monkeypatch, q_heads, kv_heads, dim, page_size, histories, window):
+    """Encoded queries, a request one item: a wave's keys lie in more pages than it has lanes to hold their table entries, with heads
+    that fill their last 32 dims or not and a window that begins inside a step, a page and a run of eight keys."""
+    monkeypatch.setattr(hip, "decode_wave_target", 1)
+    portions = [(h, 1) for h in histories]
+    q, k_pages, v_pages, ctx, meta, _, _ = _attention_case(torch.bfloat16, q_heads, kv_heads, dim, page_size, portions, window, 65)
+    ctx.num_decode_seqs = len(portions)
+    assert type(hip)._share_segments(len(portions), kv_heads)
+    want = torch.empty_like(q)
+    ref.attention(q, k_pages, v_pages, ctx, meta, q_heads, kv_heads, dim, dim ** -0.5, window, want)
+    cctx, cmeta = _to_cuda(ctx, meta)
+    got = torch.full_like(q, float("nan"), device="cuda")
+    hip.attention(q.cuda(), k_pages.cuda(), v_pages.cuda(), cctx, cmeta, q_heads, kv_heads, dim, dim ** -0.5, window, got)
+    torch.testing.assert_close(got.cpu().float(), want.float(), **attention_tol(torch.bfloat16))
+
+
 @pytest.mark.parametrize("q_heads,kv_heads,dim,page_size", [(8, 2, 128, 16), (16, 4, 64, 32), (3, 1, 256, 32), (40, 2, 64, 8), (6, 1, 32, 4), (5, 5, 80, 16)])
 @pytest.mark.parametrize("window", [None, 1, 100])
 @pytest.mark.parametrize("histories", [[0], [127], [0, 31, 32, 126], [64, 100, 5]])
@@ -1871,7 +1891,7 @@ def test_encode_and_attend_single_tokens(hip, ref, q_heads, kv_heads, dim, page_
                              len(histories))
 
 
-@pytest.mark.parametrize("dim,page_size", [(128, 8), (64, 16), (128, 4)])
+@pytest.mark.parametrize("dim,page_size", [(128, 8), (64, 16), (128, 4), (192, 16), (256, 8)])
 @pytest.mark.parametrize("histories", [[4090], [2047, 2048, 2049, 0], [9000, 33, 5]])
 @pytest.mark.parametrize("window", [None, 3000])
 @pytest.mark.parametrize("alone", [False, True])
@@ -1882,6 +1902,17 @@ def test_encode_and_attend_where_a_wave_walks_many_pages(hip, ref, monkeypatch, 
     if alone:
         monkeypatch.setattr(type(hip), "_share_segments", staticmethod(lambda seq_count, head_blocks: False))
     _check_encode_and_attend(hip, ref, 8, 2, dim, page_size, [(h, 1) for h in histories], window, len(histories))
+
+
+@pytest.mark.parametrize("dim,page_size", [(64, 16), (128, 8), (128, 16), (192, 16), (256, 8)])
+@pytest.mark.parametrize("window", [None, 3000])
+def test_encode_and_attend_beside_a_portion_where_a_wave_walks_many_pages(hip, ref, monkeypatch, dim, page_size, window):
+    """The same in the launch that holds a prompt portion's blocks too, whose single tokens are taken by waves alone."""
+    monkeypatch.setattr(hip, "decode_wave_target", 1)
+    pairs, pair = [], hip._attention_pair
+    monkeypatch.setattr(hip, "_attention_pair", lambda *a: pairs.append(1) or pair(*a))
+    _check_encode_and_attend(hip, ref, 8, 2, dim, page_size, [(4090, 1), (2047, 1), (0, 1), (40, 37)], window, 3)
+    assert pairs
 
 
 @pytest.mark.parametrize("normed,rotated", [(False, True), (True, False), (False, False)])
