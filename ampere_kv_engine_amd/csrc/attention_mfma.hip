@@ -360,8 +360,8 @@ __device__ __forceinline__ void attention_mfma_body(const Args& a, const Where a
   // are asked for at the nearest one inside, and what must count as zero is zeroed where it is used.  A wave without keys - the
   // fourth of an item of three steps, a segment beyond a short request's end - steps over all of it, as a whole.  (A step of one
   // request, 8 layers: 210 keys of 16 / 4 heads 363 -> 340 us, 2,048 keys of 32 / 8 heads 924 -> 895; the shuffles and the early
-  // loads with the tests left in gave nothing.  Waves alone on their segments, 8, 64 and 27 uneven requests: 1,261 -> 1,251, 1,978 ->
-  // 1,961, 1,655 -> 1,605; 171 tokens beside 8 requests 2,361 -> 2,315.)
+  // loads with the tests left in gave nothing.  Waves alone on their segments, the kernel and its merge: 64 x 2,048 keys of 32 / 8 heads
+  // 107 -> 105, 27 uneven requests of 16 / 4 43 -> 39, 8 x 4,000 beside 171 tokens 44 -> 42.)
   // It holds two steps' values as well as two steps' keys, D / 4 registers more, and is taken where the kernel has them - everywhere but in
   // the launch with portions at heads of 192 and for whole requests of heads beyond 224.  The kernel and its merge, us without / with, raw
   // projections: 16 / 4 heads of 192, one request of 210 and of 2,048 keys 14.9 / 13.1, 15.4 / 14.3, 27 of 64 to 16,000 71.7 / 63.1;
@@ -369,7 +369,7 @@ __device__ __forceinline__ void attention_mfma_body(const Args& a, const Where a
   // and 83.5).  Encoded queries: one request of 100 keys 5.8 / 5.3 (heads of 128), 6.9 / 6.4 (192), 8.1 / 11.1 (256, not taken so);
   // of 6,000 14.5 / 11.1, 17.7 / 13.5, 21.5 / 15.5.  Where a wave has exactly one step, the unused step that it asks for last can cost what the
   // early loads give: encoded queries, 4 x 2,048 keys of 32 / 8 heads of 128 13.5 / 14.5, one request of 16,000 of 16 / 4 15.3 / 16.2.  (The last turn
-  // written out without loads takes 72 to 300 bytes a lane of memory at heads of 128; all its lanes at one address gained 1 to 2 % of
+  // written out without loads takes 72 to 376 bytes a lane of memory at heads of 128; all its lanes at one address gained 1 to 2 % of
   // long contexts and lost as much of short ones.)
   int entries_first = 0, entries = 0;
   auto ask_entries = [&](int base) {

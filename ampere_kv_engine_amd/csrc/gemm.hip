@@ -245,10 +245,10 @@ __global__ __launch_bounds__(1024) void linear_f32_pairs_kernel(const float* __r
 // read from LDS while the half before it is multiplied, the next step is filed between a half's instructions, and the one
 // barrier of a step stands between its halves - the reads behind it have the second half's time, those before it are long
 // there.  (Read where they are used and filed at the end, with the barrier after it, 999 rows of 2048 x 2048 / 6144 x 2048 /
-// 2048 x 3072 took 89 / 249 / 130 us instead of 73 / 217 / 109 with tiles of 64 x 64, 333 rows of 2048 x 2048 / 6144 x 2048 43 /
-// 117 instead of 33 / 93 with tiles of 32 x 32, 2048 rows of 6144 x 2048 488 instead of 416, 124 TFLOP/s.)  Where a unit holds one or
-// two blocks a read from memory takes longer than a step: 2048 outputs, k 2048 with 333 rows (64 x 64) take 61 / 43 / 41 us
-// with 1 / 2 / 4 steps on their way, with 999 rows 87 / 73 / 84.  Steps are a multiple of AHEAD, so that no register is copied
+// 2048 x 3072 took 85 / 237 / 125 us instead of 75 / 214 / 110 with tiles of 64 x 64, 333 rows of 2048 x 2048 / 6144 x 2048 38 /
+// 101 instead of 33 / 95 with tiles of 32 x 32, 2048 rows of 6144 x 2048 462 instead of 419, 123 TFLOP/s; weights that no cache
+// holds, as in the table at `launch_f32`.)  Where a unit holds one or two blocks a read from memory takes longer than a step:
+// 2048 outputs, k 2048 with 333 rows (64 x 64) take 69 / 43 / 42 us with 1 / 2 / 4 steps on their way, with 999 rows 79 / 75 / 74.  Steps are a multiple of AHEAD, so that no register is copied
 // at a loop's end: steps beyond k add zeros.  ZEROS: k is no multiple of AHEAD steps, so some of what is filed counts as zeros.
 template <int TM, int TN, int AHEAD, bool ZEROS>
 __global__ __launch_bounds__(256) void linear_f32_wide_kernel(const float* __restrict__ x, const float* __restrict__ w,
@@ -404,12 +404,12 @@ int launch_f32_few_rows(const float* x, const float* w, float* y, int rows, int 
 // same).  Measured, us, on weights that no cache holds (outs x k = 2048 x 2048 / 6144 x 2048 / 4096 x 12288 / 32768 x 2048;
 // tiles of outputs x rows):
 //     16 rows: few 9.8 / 20 / 59 / 74     32 x 32 as with 17 rows
-//     17 rows: few 12.4 / 26 / 73 / 86    32 x 32 16 / 18 / 87 / 62       32 x 64 23 / 24 / 125 / 86     64 x 64 41 / 41 / 233 / 84
-//     64 rows: few 22 / 45 / 129 / -      32 x 32 16 / 25 / 91 / 115      32 x 64 23 / 25 / 125 / 92     64 x 64 41 / 42 / 233 / 89
-//    300 rows:                            32 x 32 33 / 84 / 314 / 519     32 x 64 40 / 86 / 321 / 400    64 x 64 41 / 84 / 422 / 364
-//    700 rows:                            32 x 32 62 / 191 / 675 / 1049   32 x 64 60 / 184 / 642 / 845   64 x 64 74 / 183 / 613 / 781
-//    999 rows:                            32 x 32 83 / 253 / 977 / 1483   32 x 64 86 / 239 / 862 / 1219  64 x 64 81 / 225 / 823 / 1122
-// (122 TFLOP/s at best; the vector kernel above: 511 us on average over 999 rows of 2048 x 2048 and 2048 x 3072).  So: few
+//     17 rows: few 13.3 / 26 / 74 / 86    32 x 32 16 / 18 / 87 / 58       32 x 64 23 / 25 / 125 / 90     64 x 64 41 / 42 / 233 / 84
+//     64 rows: few 22 / 45 / 129 / -      32 x 32 17 / 25 / 92 / 106      32 x 64 24 / 25 / 134 / 90     64 x 64 42 / 43 / 238 / 85
+//    300 rows:                            32 x 32 33 / 86 / 336 / 483     32 x 64 40 / 79 / 350 / 414    64 x 64 42 / 75 / 427 / 367
+//    700 rows:                            32 x 32 62 / 184 / 718 / 1036   32 x 64 58 / 173 / 669 / 899   64 x 64 74 / 177 / 618 / 801
+//    999 rows:                            32 x 32 82 / 265 / 1026 / 1477  32 x 64 77 / 233 / 894 / 1288  64 x 64 75 / 214 / 834 / 1160
+// (123 TFLOP/s at best; the vector kernel above: 511 us on average over 999 rows of 2048 x 2048 and 2048 x 3072).  So: few
 // rows stay with the kernels that read the matrix once, from 17 on only where blocks of 16 outputs are one a unit; tiles
 // are the kind whose busiest unit has the least to do - the blocks it gets times their area, a block of 32 x 64 taking 5 % and
 // one of 32 x 32 15 % longer for its area than one of 64 x 64.  (Tiles of 128 are slower everywhere: the matrix cores wait for
