@@ -288,8 +288,9 @@ __global__ __launch_bounds__((A * kHalves + kFetchers) * 64) void linear_mid_ker
         for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
           for (int i = 0; i < 4; ++i) publish(mine + ((rt * MT + mt) * 4 + i) * 64 + lane, acc[rt][mt][i]);
+      settle();                        // (the tick answers for all waves' stores and waits for its own wave's alone)
     }
-    __syncthreads();                   // (the fetching waves have gone; all multiplying waves have stored)
+    __syncthreads();                   // (the fetching waves have gone; all multiplying waves' stores have arrived)
     if (threadIdx.x == 0) {
       unsigned* counter = counters + m_block * bands + band;
       const bool last = arrive(counter) == static_cast<unsigned>(parts - 1);

@@ -137,6 +137,27 @@ def test_gated_single_tokens_of_any_number_are_taken():
     assert status(1 << 19, 2) not in (0, -1, -2)    # (taken: what fails is the launch, for want of a device)
 
 
+@pytest.mark.parametrize("kernel", ["linear_mid_kernel", "linear_decode_kernel", "sample_parts_kernel"])
+def test_sums_for_other_blocks_have_arrived_before_the_tick(kernel, tmp_path):
+    """Blocks that hand sums to each other store them with device scope and tick a counter.  Whoever stores waits until its stores
+    have been acknowledged: the wave that ticks before its tick, every other wave before the barrier that lets the first one tick."""
+    checked = 0
+    for code in _device_codes(build.library_path(), str(tmp_path)):
+        listing = subprocess.run([OBJDUMP, "-d", "--no-show-raw-insn", code], check=True, capture_output=True, text=True).stdout
+        for body in re.split(r"\n\n", listing):
+            if not re.match(rf"\s*[0-9a-f]+ <_Z\S*{kernel}", body):
+                continue
+            instructions = [re.sub(r"\s*//.*", "", line).strip() for line in body.splitlines()[1:]]
+            waiting = False                  # device-scope stores that nothing has waited for
+            for text in instructions:
+                if text.startswith("global_store") and "sc1" in text.split():
+                    waiting, checked = True, checked + 1
+                elif re.match(r"s_waitcnt .*vmcnt\(0\)", text):
+                    waiting = False
+                assert not (waiting and text.startswith(("s_barrier", "global_atomic_add"))), body.splitlines()[0]
+    assert checked
+
+
 def test_divider_is_exact(tmp_path):
     """`Divider` (common.h) against the language's division: every small divisor, those beside powers of two and large ones, at the
     multiples where a quotient changes and at the ends of its range."""

@@ -596,6 +596,25 @@ def test_exchanging_products_give_the_same_bits_two_hundred_times(hip, hip_own, 
     assert int(hip._exchange_arrivals.abs().sum()) == 0 and int(hip_own._mid_counters.abs().sum()) == 0
 
 
+@pytest.mark.parametrize("rows,outs,k", [(210, 3072, 2048), (64, 6144, 4096), (40, 4096, 12288), (179, 4096, 4096), (27, 5120, 5120)])
+def test_products_that_hand_sums_over_never_read_what_an_earlier_one_left(hip_own, rows, outs, k):
+    """A product whose k is cut over blocks, 300 times back to back on two inputs in turn: the workspace holds the other input's sums
+    whenever a block reads its neighbours', so a sum that has not arrived shows as a difference from the first results."""
+    import ctypes
+    weight = hip_own.prepare_linear(rand(outs, k, dtype=torch.bfloat16, seed=78, scale=0.05).cuda())
+    need, words = ctypes.c_long(0), ctypes.c_long(0)
+    hip_own.lib.akv_linear_mid_workspace(rows, weight.n_tiles, weight.k_tiles, 0, 0, 0, 0, 0, ctypes.byref(need), ctypes.byref(words))
+    assert need.value > 0, "this product's k is not cut over blocks"
+    inputs = [rand(rows, k, dtype=torch.bfloat16, seed=79 + i).cuda() for i in range(2)]
+    results = torch.empty(300, rows, outs, dtype=torch.bfloat16, device="cuda")
+    for turn in range(300):
+        hip_own._mid(inputs[turn % 2], weight, results[turn], rows, outs, False)
+    for turn in range(2, 300):
+        assert torch.equal(results[turn], results[turn % 2]), f"call {turn}"
+    torch.testing.assert_close(results[0].float(), (inputs[0].float() @ rand(outs, k, dtype=torch.bfloat16, seed=78, scale=0.05).cuda().float().T)
+                               .bfloat16().float(), **tol(torch.bfloat16))
+
+
 def test_decode_products_at_random_sizes(hip, ref, monkeypatch):
     """The products that add themselves to the residual sum and norm their rows, at sixty random sizes - outputs and k
     that are no multiples of the tiles, every number of rows, small matrices (one block) and large ones (blocks that
